@@ -11,43 +11,19 @@
 //    bytes per instruction and accumulated with v_dot2 (bf16 / fp16) or v_fma (fp32) in fp32 per
 //    128-wide scale block; a row pair's sums are reduced together across the wavefront.
 //  * M == 1, other K or misaligned rows (gemv_kernel): the same shape with bounds tests, fp32 math.
-//  * 5 <= M <= 16 bf16 activations (any M >= 5 for fp16, in passes of 16), K a multiple of 128
-//    (skinny_rows_kernel): a workgroup owns up to
-//    32 weight rows for the whole K; weights converted to bf16 in registers, v_mfma_f32_16x16x32_bf16 on
+//  * 5 <= M <= 16 bf16 / fp16 activations, K a multiple of 128 (skinny_rows_kernel): a workgroup owns up to
+//    32 weight rows for the whole K; weights converted to bf16 / fp16 in registers, v_mfma_f32_16x16x32 on
 //    the activations as they are; one kernel, no workspace.
-//  * 17 <= M <= 32, bf16 activations (skinny_mfma_kernel): split-K over 8 workgroup columns with
-//    v_mfma_scale_f32_16x16x128_f8f6f4.  The weights feed the matrix cores as the e4m3 bytes
-//    they are; the activations are split once per workgroup into two e4m3 planes in LDS.  The
-//    per-split partial sums go to a workspace and a second kernel adds them in split order.
+//  * M >= 17, K a multiple of 128: the tiled GEMM of fp8_gemm.hip.
 //  * anything else (odd K, misaligned rows): rowwise_kernel, one wavefront per
 //    output row, scalar byte loads.
 
 #include <type_traits>
 
-#include "common.h"
+#include "fp8_vecmat.h"
 
 namespace cm {
 namespace {
-
-struct VecmatParams {
-  const void* x;
-  const float* scale_x;
-  const unsigned char* w;
-  const float* scale_w;
-  void* out;
-  float* partial;          // [splits][M][N] fp32 (skinny kernel)
-  int m, n, k;
-  int x_dtype, out_dtype;
-  int srow_shift;          // scale row index = n >> srow_shift
-  int srow_stride;         // floats between scale rows
-  int scol_stride;         // floats between 128-wide K blocks (0 or 1)
-  int rows_per_wg;
-  int k_splits;
-};
-
-__device__ __forceinline__ float wscale(const VecmatParams& p, int n, int kb) {
-  return p.scale_w[(size_t)(n >> p.srow_shift) * p.srow_stride + (size_t)kb * p.scol_stride];
-}
 
 // 16 consecutive activation values starting at element k -> fp32
 __device__ __forceinline__ void load_x16(const VecmatParams& p, size_t off, float (&o)[16]) {
@@ -393,220 +369,8 @@ __global__ __launch_bounds__(W * 64) void gemv_stream_kernel(const VecmatParams 
   }
 }
 
-// 5 <= M <= 32 with bf16 activations, K a multiple of 1024: the split-K matrix-core kernel.
-//
-// The weights never leave e4m3: they are the B operand of v_mfma_scale_f32_16x16x128_f8f6f4
-// as they come from memory (32 contiguous bytes per lane, a whole 128-byte line per weight row
-// and 128-channel block).  The activations are the A operand.  A workgroup first writes its K
-// slice of them to LDS as two e4m3 planes hi + lo with x = hi 2^(e-127) + lo 2^(e-131), e one
-// exponent per activation row and 128-channel block, which the instruction applies as the
-// operand scales: hi carries the upper four significant bits of a bf16 value and lo the lower
-// four, so the pair is exact for every element within 2^-14 of the largest of its 128 and off
-// by less than 2^-22 of that largest one otherwise.  One block is two MFMAs (hi, lo) into a
-// zeroed tile whose lanes all belong to one weight row, so the block's fp32 weight scale (any
-// value, not only powers of two) is applied exactly as acc += scale * tile.
-constexpr int kSkinnySplits = 8;         // K is cut into eighths, one per workgroup column
-constexpr int kSkinnyWaves = 14;         // 448 row tiles x 8 splits = 256 workgroups x 14 wavefronts at N = 7168
-constexpr int kSkinnyDepth = 4;          // 128-channel weight blocks in flight per wavefront
-constexpr int kSkinnyMaxKw = 2048;       // channels per split the LDS activation slice can hold
-constexpr int kXPitch = kSkinnyMaxKw + 16;            // bytes per row of an e4m3 plane: 16 rows fall on distinct banks
-constexpr int kXBlocks = kSkinnyMaxKw / 128;
-
-typedef int i32x8 __attribute__((ext_vector_type(8)));
-typedef short i16x2 __attribute__((ext_vector_type(2)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-
-constexpr int skinny_lds_bytes(int mt) { return 2 * 16 * mt * kXPitch + 16 * mt * kXBlocks * 4; }
-
-// 32 bf16 channels of one lane (four 16-byte pieces) -> 32 e4m3 hi + 32 e4m3 lo bytes in channel
-// order.  The exponent is shared by the four lanes of a quad (one activation row's 128 channels).
-__device__ __forceinline__ int split_bf16_quad(const uint4 (&x)[4], i32x8& hi, i32x8& lo) {
-  u16x2 top = {0, 0};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const unsigned w[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
-#pragma unroll
-    for (int d = 0; d < 4; ++d) top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, w[d] & 0x7fff7fffu));
-  }
-  int amax_bits = max((int)top[0], (int)top[1]);             // bf16 bits of the largest magnitude
-  amax_bits = max(amax_bits, __builtin_amdgcn_update_dpp(0, amax_bits, 0xB1, 0xf, 0xf, true));   // quad_perm [1,0,3,2]
-  amax_bits = max(amax_bits, __builtin_amdgcn_update_dpp(0, amax_bits, 0x4E, 0xf, 0xf, true));   // quad_perm [2,3,0,1]
-  const int e = max((amax_bits >> 7) - 7, 5);                 // |x| / 2^(e-127) < 256
-  const float unit = __uint_as_float((unsigned)e << 23);
-  const float unit_lo = __uint_as_float((unsigned)(e - 4) << 23);   // the remainder is below 2^-4 of the element
-  const i16x2 zero = {0, 0};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const unsigned w[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
-#pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      const unsigned w0 = w[2 * d], w1 = w[2 * d + 1];
-      i16x2 h = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(zero, __builtin_bit_cast(bf16x2, w0), unit, false);
-      h = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(h, __builtin_bit_cast(bf16x2, w1), unit, true);
-      const unsigned hw = __builtin_bit_cast(unsigned, h);
-      const f32x2 d0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hw, unit, false);
-      const f32x2 d1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hw, unit, true);
-      i16x2 l = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(zero, __uint_as_float(w0 << 16) - d0[0],
-                                                         __uint_as_float(w0 & 0xffff0000u) - d0[1], unit_lo, false);
-      l = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(l, __uint_as_float(w1 << 16) - d1[0],
-                                                   __uint_as_float(w1 & 0xffff0000u) - d1[1], unit_lo, true);
-      hi[2 * j + d] = (int)hw;
-      lo[2 * j + d] = __builtin_bit_cast(int, l);
-    }
-  }
-  return e;
-}
-
-// MT: groups of 16 activation rows
-template <int MT>
-__global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_mfma_kernel(const VecmatParams p) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  unsigned char* xh = smem;                                            // [16 MT][kXPitch] e4m3 hi
-  unsigned char* xl = smem + 16 * MT * kXPitch;                        // [16 MT][kXPitch] e4m3 lo
-  int* xe = reinterpret_cast<int*>(smem + 2 * 16 * MT * kXPitch);      // [16 MT][kXBlocks] exponents of the two planes
-  const int lane = lane_id();
-  const int wave = (int)(threadIdx.x >> 6);
-  const int K = p.k;
-  const int kw = K / kSkinnySplits;                      // channels of this split (multiple of 128)
-  const int split = (int)blockIdx.y;
-  const int k0 = split * kw;
-  const int blocks = kw / 128;
-  // lane (r16, g): B operand = weight row r16 of the tile, channels 32 g .. 32 g + 31 of a block;
-  // A operand = activation row r16 (+ 16 mt), the same channels.  The result tile has weight row
-  // r16 in every register of the lane: register i is activation row 4 g + i.
-  const int r16 = lane & 15, g = lane >> 4;
-  const int perm_addr = 4 * (8 * (r16 & 7) + g + (r16 >= 8 ? 4 : 0));   // source lane of this lane's weight bytes
-  const unsigned char* ah = xh + r16 * kXPitch + 16 * g;
-  const unsigned char* al = xl + r16 * kXPitch + 16 * g;
-  const int* ae = xe + r16 * kXBlocks;
-  const int tiles = (p.n + 15) / 16;
-  // this wavefront's tiles: first, first + kSkinnyWaves, ...; their blocks form one continuous
-  // stream so the weight prefetch never drains between tiles
-  const int first = (int)blockIdx.x * p.rows_per_wg + wave;
-  const int tile_end = min(tiles, ((int)blockIdx.x + 1) * p.rows_per_wg);
-  const int my_tiles = first < tile_end ? (tile_end - first + kSkinnyWaves - 1) / kSkinnyWaves : 0;
-  const int total = my_tiles * blocks;
-  // prefetch cursor: next weight bytes / scale of this lane, advanced block by block
-  int pf_tile = first, pf_b = 0;
-  const unsigned char* pf_w = nullptr;
-  const unsigned char* pf_w2 = nullptr;
-  const float* pf_s = nullptr;
-  auto pf_seek = [&]() {                                 // (per tile) row of this lane in tile pf_tile
-    const int n = min(pf_tile * 16 + r16, p.n - 1);
-    // (weights are fetched by lane 8 r + q = bytes 16 q of the block's 128-byte line of row r
-    // (first load) and row 8 + r (second load): eight neighbouring lanes read a whole line, which
-    // the memory pipeline requests in one piece; two DPP moves and a lane permutation per
-    // register then hand the bytes to the matrix core's row-major lanes)
-    const int nl = min(pf_tile * 16 + (lane >> 3), p.n - 1);
-    const int nl2 = min(pf_tile * 16 + 8 + (lane >> 3), p.n - 1);
-    pf_w = p.w + (size_t)nl * K + k0 + 16 * (lane & 7);
-    pf_w2 = p.w + (size_t)nl2 * K + k0 + 16 * (lane & 7);
-    pf_s = p.scale_w + (size_t)(n >> p.srow_shift) * p.srow_stride + (size_t)(k0 >> 7) * p.scol_stride;
-  };
-  auto pf_next = [&](uint4& w0, uint4& w1, float& sc) {
-    w0 = load_w16(pf_w + 128 * pf_b);
-    w1 = load_w16(pf_w2 + 128 * pf_b);
-    sc = pf_s[(size_t)pf_b * p.scol_stride];
-    if (++pf_b == blocks) {                              // (uniform)
-      pf_b = 0;
-      pf_tile += kSkinnyWaves;
-      if (pf_tile < tile_end) pf_seek();
-    }
-  };
-  uint4 wq0[kSkinnyDepth], wq1[kSkinnyDepth];
-  float sq[kSkinnyDepth];
-  if (total > 0) {
-    pf_seek();
-#pragma unroll
-    for (int d = 0; d < kSkinnyDepth; ++d) {
-      if (d < total) pf_next(wq0[d], wq1[d], sq[d]);
-      else { wq0[d] = make_uint4(0, 0, 0, 0); wq1[d] = wq0[d]; sq[d] = 0.0f; }
-    }
-  }
-  // (the first weight blocks are already on their way: the conversion below runs in their shadow)
-  // activation slice -> LDS: a quad of lanes per (row, block), 32 channels per lane (rows >= M are zero)
-  for (int t = (int)threadIdx.x; t < 16 * MT * blocks * 4; t += kSkinnyWaves * 64) {
-    const int q = t & 3, item = t >> 2;
-    const int m = item / blocks, b = item % blocks;
-    uint4 x[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) x[j] = make_uint4(0, 0, 0, 0);
-    if (m < p.m) {
-      const uint4* src = reinterpret_cast<const uint4*>((const unsigned short*)p.x + (size_t)m * K + k0 + 128 * b + 32 * q);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) x[j] = src[j];
-    }
-    i32x8 hi, lo;
-    const int e = split_bf16_quad(x, hi, lo);
-    uint4* dh = reinterpret_cast<uint4*>(xh + m * kXPitch + 128 * b + 32 * q);
-    uint4* dl = reinterpret_cast<uint4*>(xl + m * kXPitch + 128 * b + 32 * q);
-    dh[0] = make_uint4((unsigned)hi[0], (unsigned)hi[1], (unsigned)hi[2], (unsigned)hi[3]);
-    dh[1] = make_uint4((unsigned)hi[4], (unsigned)hi[5], (unsigned)hi[6], (unsigned)hi[7]);
-    dl[0] = make_uint4((unsigned)lo[0], (unsigned)lo[1], (unsigned)lo[2], (unsigned)lo[3]);
-    dl[1] = make_uint4((unsigned)lo[4], (unsigned)lo[5], (unsigned)lo[6], (unsigned)lo[7]);
-    if (q == 0) xe[m * kXBlocks + b] = e | ((e - 4) << 8);          // byte 0: hi plane, byte 1: lo plane
-  }
-  __syncthreads();
-
-  f32x4 acc[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  int b = 0, tile = first;                               // position of flat block f0 + d, tracked incrementally
-  for (int f0 = 0; f0 < total; f0 += kSkinnyDepth) {
-#pragma unroll
-    for (int d = 0; d < kSkinnyDepth; ++d) {
-      const int f = f0 + d;
-      const uint4 w0 = wq0[d], w1 = wq1[d];
-      const float sc = sq[d];
-      if (f + kSkinnyDepth < total) pf_next(wq0[d], wq1[d], sq[d]);
-      if (f < total) {                                   // (uniform)
-        // x0: pieces 0..3 of all 16 rows (the second load's, moved up four lanes, fill lanes 4..7 of
-        // every eight); x1: pieces 4..7 (the first load's, moved down four lanes, fill lanes 0..3)
-        const int a_[4] = {(int)w0.x, (int)w0.y, (int)w0.z, (int)w0.w}, b_[4] = {(int)w1.x, (int)w1.y, (int)w1.z, (int)w1.w};
-        i32x8 bw;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          const int x0 = __builtin_amdgcn_update_dpp(a_[d], b_[d], 0x114, 0xf, 0xa, false);   // row_shr:4 into banks 1, 3
-          const int x1 = __builtin_amdgcn_update_dpp(b_[d], a_[d], 0x104, 0xf, 0x5, false);   // row_shl:4 into banks 0, 2
-          bw[d] = __builtin_amdgcn_ds_bpermute(perm_addr, x0);
-          bw[4 + d] = __builtin_amdgcn_ds_bpermute(perm_addr, x1);
-        }
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const uint4 h0 = *reinterpret_cast<const uint4*>(ah + mt * 16 * kXPitch + 128 * b);
-          const uint4 h1 = *reinterpret_cast<const uint4*>(ah + mt * 16 * kXPitch + 128 * b + 64);
-          const uint4 l0 = *reinterpret_cast<const uint4*>(al + mt * 16 * kXPitch + 128 * b);
-          const uint4 l1 = *reinterpret_cast<const uint4*>(al + mt * 16 * kXPitch + 128 * b + 64);
-          const int e = ae[mt * 16 * kXBlocks + b];
-          const i32x8 ahi = {(int)h0.x, (int)h0.y, (int)h0.z, (int)h0.w, (int)h1.x, (int)h1.y, (int)h1.z, (int)h1.w};
-          const i32x8 alo = {(int)l0.x, (int)l0.y, (int)l0.z, (int)l0.w, (int)l1.x, (int)l1.y, (int)l1.z, (int)l1.w};
-          f32x4 t = {0.f, 0.f, 0.f, 0.f};
-          t = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ahi, bw, t, 0, 0, 0, e, 0, 0x7f7f7f7f);
-          t = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(alo, bw, t, 0, 0, 1, e, 0, 0x7f7f7f7f);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[mt][i] = fmaf(sc, t[i], acc[mt][i]);
-        }
-        if (++b == blocks) {                             // (uniform) tile finished: partial[split][m][row]
-          const int row = tile * 16 + r16;
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int m = 16 * mt + 4 * g + i;
-              if (m < p.m && row < p.n) p.partial[((size_t)split * p.m + m) * p.n + row] = acc[mt][i];
-            }
-            acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-          }
-          b = 0;
-          tile += kSkinnyWaves;
-        }
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// 5 <= M <= 32 without a K split: a workgroup owns up to 32 weight rows for the whole K.
+// 5 <= M <= 16: a workgroup owns up to 32 weight rows for the whole K.
 //
 // Each of its 8 wavefronts takes a contiguous eighth of the 128-channel blocks, so a weight row
 // is streamed as 8 sequential runs.  Per block a wavefront fetches the 32 x 128 weight bytes and
@@ -805,17 +569,6 @@ __global__ __launch_bounds__(rows_waves(MT) * 64) void skinny_rows_kernel(const 
   }
 }
 
-// out[m][n] = sum over the K splits of partial[split][m][n], in split order
-__global__ __launch_bounds__(256) void skinny_reduce_kernel(const VecmatParams p) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  const size_t total = (size_t)p.m * p.n;
-  if (i >= total) return;
-  float s = 0.0f;
-#pragma unroll
-  for (int z = 0; z < kSkinnySplits; ++z) s += p.partial[(size_t)z * total + i];
-  store_as(p.out, i, p.out_dtype, s);
-}
-
 // Any shape: one wavefront per output row, all M activations in turn.
 __global__ __launch_bounds__(256) void rowwise_kernel(const VecmatParams p) {
   const int lane = lane_id();
@@ -874,33 +627,24 @@ static bool stream_k(const cppmega_mi355_vecmat_args_t& a) {
   return stream_row_cap(a.x_dtype) > 0 && (a.k % 16 == 0) && a.k <= kStreamMaxK;
 }
 static bool stream_shape(const cppmega_mi355_vecmat_args_t& a) { return stream_k(a) && a.m <= stream_row_cap(a.x_dtype); }
-// the split-K MFMA kernel: bf16 activations, M >= 5 (in passes of 32 rows), K in eighths of whole scale blocks that fit the LDS slice
-constexpr int kSkinnyMaxRows = 32;
-constexpr int kRowsMaxM = 16;             // activation rows the kernel without a K split takes (17..32 measured no faster than the split-K kernel)
-static bool skinny_shape(const cppmega_mi355_vecmat_args_t& a) {
-  return a.x_dtype == CPPMEGA_MI355_BF16 && a.m >= 5 &&
-         (a.k % (kSkinnySplits * 128) == 0) && a.k / kSkinnySplits <= kSkinnyMaxKw;
-}
-static bool skinny_ok(const cppmega_mi355_vecmat_args_t& a) { return vecmat_aligned(a) && skinny_shape(a); }
-// the kernel without a K split: bf16 activations, M >= 5 (in passes of 32 rows), whole 128-channel blocks,
+// the kernel without a K split: bf16 / fp16 activations, 5 <= M <= 16, whole 128-channel blocks,
 // scales of 32 rows and partial tiles within the LDS
+constexpr int kRowsMaxM = 16;             // more activation rows: the tiled GEMM (M = 32: 31 us against 37 us at 7168 x 16384)
 static size_t rows_lds_bytes(int k, int mt) { return (size_t)rows_waves(mt) * (32 * 128 + mt * 16 * 256) + (size_t)(k / 128) * 32 * sizeof(float); }
 static bool rows_shape(const cppmega_mi355_vecmat_args_t& a) {
-  const bool bf16 = a.x_dtype == CPPMEGA_MI355_BF16;
-  // float16 rows have no split-K kernel behind them (they would run in passes of 4 on the streaming kernel): any M >= 5
-  if (a.x_dtype == CPPMEGA_MI355_F16) return a.m >= 5 && a.k % 128 == 0 && rows_lds_bytes(a.k, 1) <= 160 * 1024;
-  return bf16 && a.m >= 5 && a.m <= kRowsMaxM && a.k % 128 == 0 && rows_lds_bytes(a.k, a.m <= 16 ? 1 : 2) <= 160 * 1024;
+  return (a.x_dtype == CPPMEGA_MI355_BF16 || a.x_dtype == CPPMEGA_MI355_F16) && a.m >= 5 && a.m <= kRowsMaxM && a.k % 128 == 0 &&
+         rows_lds_bytes(a.k, 1) <= 160 * 1024;
 }
 
 int fp8_vecmat_workspace_bytes(const cppmega_mi355_vecmat_args_t& a, size_t* bytes) {
   if (!bytes) return fail(CPPMEGA_MI355_ERR_NULL, "vecmat: bytes is NULL");
   // pointers may be absent in a sizing call: decided from the shape alone (a misaligned call then
   // simply does not use the workspace)
-  *bytes = (skinny_shape(a) && !rows_shape(a)) ? (size_t)kSkinnySplits * (a.m < kSkinnyMaxRows ? a.m : kSkinnyMaxRows) * a.n * sizeof(float) : 0;
+  *bytes = fp8_gemm_shape(a) ? fp8_gemm_workspace_bytes(a) : 0;
   return 0;
 }
 
-static int device_cus() {
+int device_cus() {
   static int cus = 0;
   if (cus == 0) {
     int dev = 0, v = 0;
@@ -1012,6 +756,12 @@ int fp8_vecmat_launch(const cppmega_mi355_vecmat_args_t& a, hipStream_t stream) 
   if (aligned && stream_shape(a)) {
     rc = stream_pass(p, 0, a.m);
     if (rc) return rc;
+  } else if (aligned && fp8_gemm_shape(a)) {
+    const size_t need = fp8_gemm_workspace_bytes(a);
+    if (need > 0 && (!a.workspace || a.workspace_bytes < need))
+      return fail(CPPMEGA_MI355_ERR_WORKSPACE, "vecmat: workspace of %zu bytes needed, %zu given", need, a.workspace ? (size_t)a.workspace_bytes : (size_t)0);
+    p.partial = (float*)a.workspace;
+    return fp8_gemm_launch(p, stream);
   } else if (aligned && rows_shape(a)) {
     // about one workgroup per CU, whole MFMA row tiles where that is possible
     int rows = (a.n + device_cus() - 1) / device_cus();
@@ -1022,44 +772,8 @@ int fp8_vecmat_launch(const cppmega_mi355_vecmat_args_t& a, hipStream_t stream) 
     const bool f16 = a.x_dtype == CPPMEGA_MI355_F16;
     const void* fn = f16 ? (const void*)skinny_rows_kernel<1, true> : (const void*)skinny_rows_kernel<1, false>;
     if (smem > 64 * 1024) CM_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-    for (int m0 = 0; m0 < a.m; m0 += 16) {             // (more than 16 rows: float16 only, in passes)
-      VecmatParams q = p;
-      q.m = a.m - m0 < 16 ? a.m - m0 : 16;
-      q.x = (const char*)a.x + (size_t)m0 * a.k * dtype_size(a.x_dtype);
-      q.out = (char*)a.out + (size_t)m0 * a.n * dtype_size(a.out_dtype);
-      void* kargs[] = {(void*)&q};
-      CM_HIP_CHECK(hipLaunchKernel(fn, grid, dim3(rows_waves(1) * 64), kargs, smem, stream));
-    }
-  } else if (skinny_ok(a)) {
-    // more than 32 activation rows: passes of 32 over the same workspace (stream order keeps them apart)
-    const int cap = a.m < kSkinnyMaxRows ? a.m : kSkinnyMaxRows;
-    const size_t need = (size_t)kSkinnySplits * cap * a.n * sizeof(float);
-    if (!a.workspace || a.workspace_bytes < need)
-      return fail(CPPMEGA_MI355_ERR_WORKSPACE, "vecmat: workspace of %zu bytes needed, %zu given", need, (size_t)a.workspace_bytes);
-    p.partial = (float*)a.workspace;
-    // row tiles per workgroup: about one workgroup per CU and split, a multiple of the wavefront count
-    const int tiles = (a.n + 15) / 16;
-    int per_wave = (tiles * kSkinnySplits + 256 * kSkinnyWaves - 1) / (256 * kSkinnyWaves);
-    if (per_wave < 1) per_wave = 1;
-    p.rows_per_wg = per_wave * kSkinnyWaves;
-    const dim3 grid((unsigned)((tiles + p.rows_per_wg - 1) / p.rows_per_wg), kSkinnySplits), block(kSkinnyWaves * 64);
-    for (int m0 = 0; m0 < a.m; m0 += kSkinnyMaxRows) {
-      VecmatParams q = p;
-      q.m = a.m - m0 < kSkinnyMaxRows ? a.m - m0 : kSkinnyMaxRows;
-      q.x = (const char*)a.x + (size_t)m0 * a.k * dtype_size(a.x_dtype);
-      q.out = (char*)a.out + (size_t)m0 * a.n * dtype_size(a.out_dtype);
-      if (q.m <= 16) {
-        const int smem = skinny_lds_bytes(1);
-        CM_HIP_CHECK(hipFuncSetAttribute((const void*)skinny_mfma_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-        hipLaunchKernelGGL(skinny_mfma_kernel<1>, grid, block, smem, stream, q);
-      } else {
-        const int smem = skinny_lds_bytes(2);
-        CM_HIP_CHECK(hipFuncSetAttribute((const void*)skinny_mfma_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-        hipLaunchKernelGGL(skinny_mfma_kernel<2>, grid, block, smem, stream, q);
-      }
-      CM_HIP_CHECK(hipGetLastError());
-      hipLaunchKernelGGL(skinny_reduce_kernel, dim3((unsigned)(((size_t)q.m * a.n + 255) / 256)), dim3(256), 0, stream, q);
-    }
+    void* kargs[] = {(void*)&p};
+    CM_HIP_CHECK(hipLaunchKernel(fn, grid, dim3(rows_waves(1) * 64), kargs, smem, stream));
   } else if (aligned && stream_k(a)) {
     // more rows than one launch takes: passes over the weights (which the last-level cache may keep)
     const int cap = stream_row_cap(a.x_dtype);

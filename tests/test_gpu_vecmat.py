@@ -195,3 +195,21 @@ def test_headline_config_full_size(device, M):
     torch.cuda.synchronize()
     scale_out = max(o1.abs().max().item(), o2.abs().max().item())
     assert (o3 - (2 * o1 - o2)).abs().max().item() <= 1e-4 * scale_out
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(17, 1, 128), (32, 129, 384), (33, 127, 256), (64, 300, 2176), (65, 128, 128), (129, 257, 1152),
+                                   (300, 1434, 896), (1025, 8200, 256), (260, 8192, 512)])
+def test_tiled_gemm_edges(device, M, N, K, dtype):
+    """From 17 activation rows on, tiles of 32, 64 and 128 rows with and without a K split: ragged rows, columns
+    that are not whole 16-byte stores, one scale block, both half types, 16- and 32-bit results."""
+    gen = torch.Generator(device="cpu").manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=gen).to(dtype)
+    codes = torch.randn((N, K), generator=gen).mul(2).to(torch.float8_e4m3fn)
+    scale = torch.rand((N, K // 128), generator=gen) + 0.5
+    want = x.double() @ (codes.double() * scale.double().repeat_interleave(128, dim=1)).T
+    for out_dtype, tol in ((torch.float32, 2e-6), (dtype, 5e-3)):
+        out = torch.full((M, N), 7.0, dtype=out_dtype, device=device)
+        vm.fp8_scaled_vecmat_path_c(x.to(device), codes.view(torch.uint8).to(device), scale_x=None, scale_w=scale.to(device), out=out)
+        err = (out.double().cpu() - want).abs().max() / want.abs().max()
+        assert err <= tol, err
