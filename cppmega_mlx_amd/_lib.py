@@ -50,6 +50,7 @@ EXPORTED_SYMBOLS = (
     "cppmega_mi355_fp8_vecmat",
     "cppmega_mi355_fp8_quantize",
     "cppmega_mi355_head_gemm",
+    "cppmega_mi355_dsa_indexer_loss_workspace_bytes",
     "cppmega_mi355_dsa_indexer_loss",
     "cppmega_mi355_sparse_mla_bwd",
     "cppmega_mi355_dequant_block_fp8",
@@ -182,6 +183,10 @@ class DsaLossArgs(C.Structure):
         ("topk_indices", C.c_void_p),
         ("topk", C.c_int32),
         ("index_dtype", C.c_int32),
+        ("workspace", C.c_void_p),
+        ("workspace_bytes", C.c_size_t),
+        ("range_flag", C.c_void_p),
+        ("range_event", C.c_void_p),
     ]
 
 
@@ -418,6 +423,8 @@ def load() -> C.CDLL:
         lib.cppmega_mi355_sparse_mla_bwd.restype = C.c_int
         lib.cppmega_mi355_dsa_indexer_loss.argtypes = [C.POINTER(DsaLossArgs), C.c_size_t, C.c_void_p]
         lib.cppmega_mi355_dsa_indexer_loss.restype = C.c_int
+        lib.cppmega_mi355_dsa_indexer_loss_workspace_bytes.argtypes = [C.POINTER(DsaLossArgs), C.c_size_t, C.POINTER(C.c_size_t)]
+        lib.cppmega_mi355_dsa_indexer_loss_workspace_bytes.restype = C.c_int
         lib.cppmega_mi355_head_gemm.argtypes = [C.POINTER(HeadGemmArgs), C.c_size_t, C.c_void_p]
         lib.cppmega_mi355_head_gemm.restype = C.c_int
         lib.cppmega_mi355_dequant_block_fp8.argtypes = [C.POINTER(DequantBlockArgs), C.c_size_t, C.c_void_p]

@@ -38,6 +38,7 @@ int causal_indices_launch(const cppmega_mi355_causal_indices_args_t& a, hipStrea
 int mask_indices_launch(const cppmega_mi355_mask_indices_args_t& a, hipStream_t stream);
 int sparse_mla_bwd_launch(const cppmega_mi355_sparse_mla_bwd_args_t& a, hipStream_t stream);
 int dsa_indexer_loss_launch(const cppmega_mi355_dsa_loss_args_t& a, hipStream_t stream);
+int dsa_indexer_loss_workspace_bytes(const cppmega_mi355_dsa_loss_args_t& a, size_t* bytes);
 int head_gemm_launch(const cppmega_mi355_head_gemm_args_t& a, hipStream_t stream);
 int dequant_block_fp8_launch(const cppmega_mi355_dequant_block_args_t& a, hipStream_t stream);
 int indexer_topk_launch(const cppmega_mi355_indexer_args_t& a, hipStream_t stream);
@@ -99,17 +100,20 @@ static int build_mla_params(const cppmega_mi355_sparse_mla_args_t& a, MlaParams&
   return 0;
 }
 
-// Copies the caller's sparse-MLA struct into the current layout; a caller built against the first
-// ABI (struct_size ends at workspace_bytes) gets zeros for the fields appended since.
-static int widen_mla_args(const cppmega_mi355_sparse_mla_args_t* args, size_t args_size, cppmega_mi355_sparse_mla_args_t& a) {
+// Copies the caller's struct into the current layout; a caller built against an earlier layout (of at
+// least v1_size bytes) gets zeros for the fields appended since.
+template <class T>
+static int widen_args(const T* args, size_t args_size, size_t v1_size, T& a) {
   if (!args) return fail(CPPMEGA_MI355_ERR_NULL, "args is NULL");
   const size_t have = args_size < (size_t)args->struct_size ? args_size : (size_t)args->struct_size;
-  if (have < CPPMEGA_MI355_SPARSE_MLA_ARGS_V1_SIZE)
-    return fail(CPPMEGA_MI355_ERR_STRUCT_SIZE, "args struct is %zu/%u bytes, need %zu", args_size, args->struct_size,
-                (size_t)CPPMEGA_MI355_SPARSE_MLA_ARGS_V1_SIZE);
+  if (have < v1_size)
+    return fail(CPPMEGA_MI355_ERR_STRUCT_SIZE, "args struct is %zu/%u bytes, need %zu", args_size, args->struct_size, v1_size);
   memset(&a, 0, sizeof(a));
   memcpy(&a, args, have < sizeof(a) ? have : sizeof(a));
   return 0;
+}
+static int widen_mla_args(const cppmega_mi355_sparse_mla_args_t* args, size_t args_size, cppmega_mi355_sparse_mla_args_t& a) {
+  return widen_args(args, args_size, CPPMEGA_MI355_SPARSE_MLA_ARGS_V1_SIZE, a);
 }
 
 static int pick_mla_kernel(const cppmega_mi355_sparse_mla_args_t& a, const MlaParams& p) {
@@ -203,16 +207,8 @@ int cppmega_mi355_status(cppmega_mi355_status_t* out, size_t out_size) {
   return CPPMEGA_MI355_OK;
 }
 
-// Copies the caller's top-k struct into the current layout (zeros for fields appended after the first ABI).
 static int widen_topk_args(const cppmega_mi355_topk_args_t* args, size_t args_size, cppmega_mi355_topk_args_t& a) {
-  if (!args) return fail(CPPMEGA_MI355_ERR_NULL, "args is NULL");
-  const size_t have = args_size < (size_t)args->struct_size ? args_size : (size_t)args->struct_size;
-  if (have < CPPMEGA_MI355_TOPK_ARGS_V1_SIZE)
-    return fail(CPPMEGA_MI355_ERR_STRUCT_SIZE, "args struct is %zu/%u bytes, need %zu", args_size, args->struct_size,
-                (size_t)CPPMEGA_MI355_TOPK_ARGS_V1_SIZE);
-  memset(&a, 0, sizeof(a));
-  memcpy(&a, args, have < sizeof(a) ? have : sizeof(a));
-  return 0;
+  return widen_args(args, args_size, CPPMEGA_MI355_TOPK_ARGS_V1_SIZE, a);
 }
 
 int cppmega_mi355_topk_select(const cppmega_mi355_topk_args_t* args, size_t args_size, void* stream) {
@@ -335,8 +331,18 @@ int cppmega_mi355_sparse_mla_bwd(const cppmega_mi355_sparse_mla_bwd_args_t* args
 }
 
 int cppmega_mi355_dsa_indexer_loss(const cppmega_mi355_dsa_loss_args_t* args, size_t args_size, void* stream) {
-  CM_CHECK_ARGS(args, args_size, cppmega_mi355_dsa_loss_args_t);
-  return dsa_indexer_loss_launch(*args, (hipStream_t)stream);
+  cppmega_mi355_dsa_loss_args_t a;
+  const int rc = widen_args(args, args_size, CPPMEGA_MI355_DSA_LOSS_ARGS_V1_SIZE, a);
+  if (rc) return rc;
+  return dsa_indexer_loss_launch(a, (hipStream_t)stream);
+}
+
+int cppmega_mi355_dsa_indexer_loss_workspace_bytes(const cppmega_mi355_dsa_loss_args_t* args, size_t args_size, size_t* bytes) {
+  cppmega_mi355_dsa_loss_args_t a;
+  const int rc = widen_args(args, args_size, CPPMEGA_MI355_DSA_LOSS_ARGS_V1_SIZE, a);
+  if (rc) return rc;
+  if (!bytes) return fail(CPPMEGA_MI355_ERR_NULL, "bytes is NULL");
+  return dsa_indexer_loss_workspace_bytes(a, bytes);
 }
 
 int cppmega_mi355_head_gemm(const cppmega_mi355_head_gemm_args_t* args, size_t args_size, void* stream) {

@@ -168,18 +168,41 @@ __global__ __launch_bounds__(kThreads) void dsa_indexer_loss_kernel(const LossPa
 bool dsa_indexer_loss_mfma_supports(const cppmega_mi355_dsa_loss_args_t& a);                    // dsa_indexer_loss_mfma.hip
 int dsa_indexer_loss_mfma_launch(const cppmega_mi355_dsa_loss_args_t& a, hipStream_t stream);
 
-int dsa_indexer_loss_launch(const cppmega_mi355_dsa_loss_args_t& a, hipStream_t stream) {
-  if (!a.query || !a.key || !a.index_scores || !a.loss) return fail(CPPMEGA_MI355_ERR_NULL, "dsa_indexer_loss: a pointer is NULL");
+bool dsa_indexer_loss_tiled_supports(const cppmega_mi355_dsa_loss_args_t& a);                   // dsa_indexer_loss_tiled.hip
+size_t dsa_indexer_loss_tiled_workspace_bytes(const cppmega_mi355_dsa_loss_args_t& a);
+int dsa_indexer_loss_tiled_launch(const cppmega_mi355_dsa_loss_args_t& a, hipStream_t stream);
+
+static int check_shape(const cppmega_mi355_dsa_loss_args_t& a) {
   if (a.seq_q < 0 || a.batch < 0 || a.heads < 0 || a.head_dim < 0 || a.seq_k < 0)
     return fail(CPPMEGA_MI355_ERR_SHAPE, "dsa_indexer_loss: negative dimension");
   if (a.heads > 128) return fail(CPPMEGA_MI355_ERR_SHAPE, "dsa_indexer_loss: AH > 128 is numerically unsafe (got AH=%d)", a.heads);
   if (a.in_dtype != CPPMEGA_MI355_F32 && a.in_dtype != CPPMEGA_MI355_F16 && a.in_dtype != CPPMEGA_MI355_BF16)
     return fail(CPPMEGA_MI355_ERR_DTYPE, "dsa_indexer_loss: query / key must be float32, float16 or bfloat16");
+  return 0;
+}
+
+int dsa_indexer_loss_workspace_bytes(const cppmega_mi355_dsa_loss_args_t& a, size_t* bytes) {
+  const int rc = check_shape(a);
+  if (rc) return rc;
+  *bytes = dsa_indexer_loss_tiled_supports(a) ? dsa_indexer_loss_tiled_workspace_bytes(a) : 0;
+  return 0;
+}
+
+int dsa_indexer_loss_launch(const cppmega_mi355_dsa_loss_args_t& a, hipStream_t stream) {
+  if (!a.query || !a.key || !a.index_scores || !a.loss) return fail(CPPMEGA_MI355_ERR_NULL, "dsa_indexer_loss: a pointer is NULL");
+  const int rc = check_shape(a);
+  if (rc) return rc;
   if ((size_t)a.seq_q * a.batch == 0 || a.heads == 0 || a.head_dim == 0 || a.seq_k == 0) return 0;
   if (a.topk_indices) {
     if (a.topk < 1) return fail(CPPMEGA_MI355_ERR_SHAPE, "dsa_indexer_loss: an index list needs topk >= 1 (an empty list masks every key)");
     if (a.index_dtype != CPPMEGA_MI355_I32 && a.index_dtype != CPPMEGA_MI355_I64)
       return fail(CPPMEGA_MI355_ERR_DTYPE, "dsa_indexer_loss: topk_indices must be int32 or int64");
+  }
+  if (a.workspace && dsa_indexer_loss_tiled_supports(a)) {
+    const size_t need = dsa_indexer_loss_tiled_workspace_bytes(a);
+    if (a.workspace_bytes < need)
+      return fail(CPPMEGA_MI355_ERR_WORKSPACE, "dsa_indexer_loss: workspace of %zu bytes needed, %zu given", need, (size_t)a.workspace_bytes);
+    return dsa_indexer_loss_tiled_launch(a, stream);
   }
   if (dsa_indexer_loss_mfma_supports(a)) return dsa_indexer_loss_mfma_launch(a, stream);    // bfloat16 / float16 rows
   const size_t lds = ((size_t)2 * a.seq_k + a.head_dim + 8 + (a.seq_k + 31) / 32) * sizeof(float);

@@ -1,4 +1,5 @@
-// DSA indexer KL loss on the matrix cores, bfloat16 / float16 query and key (gfx950).
+// DSA indexer KL loss on the matrix cores, bfloat16 / float16 query and key, for callers without a
+// workspace (dsa_indexer_loss_tiled.hip is the faster one) (gfx950).
 //
 // Same result as dsa_indexer_loss.hip (the reference's two stages,
 // cppmega_mlx/nn/_tilelang/dsa_splitk_indexer_loss.py:398-656 and :855-1165) with the attention

@@ -76,9 +76,6 @@ def _validated_topk(topk_indices: torch.Tensor, query: torch.Tensor, AB: int, AS
     if topk_indices.dtype not in (torch.int32, torch.int64):
         raise TypeError(f"{_NAME}: topk_indices.dtype must be int32 or int64; got {topk_indices.dtype}")
     idx = topk_indices if topk_indices.is_contiguous() else topk_indices.contiguous()
-    # One fused reduction and one host read, as the reference does on every call (:1404-1415).
-    if bool(((idx < 0) | (idx >= Sk)).any().item()):
-        raise ValueError(f"{_NAME}: topk_indices out of range [0, {Sk}); got [{int(idx.min().item())}, {int(idx.max().item())}].")
     return idx
 
 
@@ -102,8 +99,11 @@ def dsa_splitk_indexer_loss_per_position(index_scores: torch.Tensor, topk_indice
         raise ValueError(f"{_NAME}: unsupported device type {query.device.type!r}")
     idx = _validated_topk(topk_indices, query, AB, ASq, Sk) if sparse_loss else None
     scores = index_scores if index_scores.dtype == torch.float32 and index_scores.is_contiguous() else index_scores.to(torch.float32).contiguous()
-    return ops.dsa_indexer_loss(query if query.is_contiguous() else query.contiguous(), key if key.is_contiguous() else key.contiguous(),
-                                scores, softmax_scale=float(softmax_scale), out=out, topk_indices=idx)
+    try:                                                   # (out-of-range lists raise, as the reference's host read does on every call, :1404-1415)
+        return ops.dsa_indexer_loss(query if query.is_contiguous() else query.contiguous(), key if key.is_contiguous() else key.contiguous(),
+                                    scores, softmax_scale=float(softmax_scale), out=out, topk_indices=idx, check_range=True)
+    except ops.IndexRangeError:
+        raise ValueError(f"{_NAME}: topk_indices out of range [0, {Sk}); got [{int(idx.min().item())}, {int(idx.max().item())}].") from None
 
 
 def dsa_splitk_indexer_loss_tilelang(index_scores: torch.Tensor, topk_indices: torch.Tensor, query: torch.Tensor, key: torch.Tensor,

@@ -264,10 +264,12 @@ def dequant_block_fp8(weight: torch.Tensor, scale_inv: torch.Tensor, *, out: tor
 # ---------------------------------------------------------------------------
 def dsa_indexer_loss(query: torch.Tensor, key: torch.Tensor, index_scores: torch.Tensor, *, softmax_scale: float,
                      out: torch.Tensor, index_mask: torch.Tensor | None = None,
-                     topk_indices: torch.Tensor | None = None) -> torch.Tensor:
+                     topk_indices: torch.Tensor | None = None, check_range: bool = False) -> torch.Tensor:
     """Per-position KL(attention || index) into caller-owned float32 ``out`` [AB, ASq];
     ``query`` [ASq, AB, AH, AD], ``key`` [Sk, AB, AH, AD], ``index_scores`` / ``index_mask`` float32 [AB, ASq, Sk];
-    ``topk_indices`` int32 / int64 [AB, ASq, topk] restricts both distributions to the listed keys."""
+    ``topk_indices`` int32 / int64 [AB, ASq, topk] restricts both distributions to the listed keys.
+    ``check_range`` raises :class:`IndexRangeError` when a list holds an index outside [0, Sk): the host waits for the
+    kernel that reads the lists, not for the loss."""
     for name, t in (("query", query), ("key", key), ("index_scores", index_scores), ("out", out), ("index_mask", index_mask),
                     ("topk_indices", topk_indices)):
         if t is not None:
@@ -295,10 +297,54 @@ def dsa_indexer_loss(query: torch.Tensor, key: torch.Tensor, index_scores: torch
             raise ValueError(f"topk_indices must have shape (AB={AB}, ASq={ASq}, TOPK); got {tuple(topk_indices.shape)}")
         a.topk_indices, a.topk = topk_indices.data_ptr(), int(topk_indices.shape[2])
         a.index_dtype = _dtype_or_raise(topk_indices, "topk_indices", (_lib.I32, _lib.I64))
+    lib = _lib.load()
+    stream = _lib.current_stream(query.device)
+    need = C.c_size_t(0)
+    _lib.check(lib.cppmega_mi355_dsa_indexer_loss_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)), "dsa_indexer_loss")
+    watch = None
+    if need.value:
+        workspace = _workspace(query.device, need.value, stream)
+        a.workspace = workspace.data_ptr()
+        a.workspace_bytes = workspace.numel()
+        if check_range and topk_indices is not None:
+            watch = _range_watch(query.device)
+            watch.flag[0] = 0
+            a.range_flag, a.range_event = watch.flag.data_ptr(), watch.event.cuda_event
+    elif check_range and topk_indices is not None and bool(((topk_indices < 0) | (topk_indices >= Sk)).any().item()):
+        raise IndexRangeError("topk_indices out of range")
     with torch.cuda.device(query.device):
-        rc = _lib.load().cppmega_mi355_dsa_indexer_loss(C.byref(a), C.sizeof(a), _lib.current_stream(query.device))
+        rc = lib.cppmega_mi355_dsa_indexer_loss(C.byref(a), C.sizeof(a), stream)
     _lib.check(rc, "dsa_indexer_loss")
+    if watch is not None:
+        watch.event.synchronize()
+        if watch.flag[0]:
+            raise IndexRangeError("topk_indices out of range")
     return out
+
+
+class IndexRangeError(ValueError):
+    """An index list names a key that does not exist."""
+
+
+class _RangeWatch:
+    """Where the list kernel reports to the host: a word of pinned memory, and the event behind the kernel."""
+
+    def __init__(self, device: torch.device):
+        self.flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        with torch.cuda.device(device):
+            self.event = torch.cuda.Event()
+            self.event.record()          # creates the handle
+
+
+_range_watches = threading.local()       # a call waits for its own report, so one per thread and device is enough
+
+
+def _range_watch(device: torch.device) -> _RangeWatch:
+    key = device.index if device.index is not None else torch.cuda.current_device()
+    cached = _range_watches.__dict__.setdefault("by_device", {})
+    if key not in cached:
+        cached[key] = _RangeWatch(device)
+    return cached[key]
 
 
 # ---------------------------------------------------------------------------

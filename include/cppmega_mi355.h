@@ -366,8 +366,20 @@ typedef struct cppmega_mi355_dsa_loss_args {
   const void* topk_indices;
   int32_t topk;
   int32_t index_dtype;
+  /* Optional (callers built against the first layout end here): *_workspace_bytes of scratch switches
+   * 16-bit rows to the tiled kernels, the same result several times faster.  With it, an entry of
+   * topk_indices outside [0, Sk) also sets *range_flag (device or pinned host memory the caller has
+   * cleared) to 1, and range_event (a hipEvent_t) is recorded on the stream behind the kernel that
+   * reads the lists, in front of the others. */
+  void* workspace;
+  size_t workspace_bytes;
+  int32_t* range_flag;
+  void* range_event;
 } cppmega_mi355_dsa_loss_args_t;
+#define CPPMEGA_MI355_DSA_LOSS_ARGS_V1_SIZE (offsetof(cppmega_mi355_dsa_loss_args_t, workspace))
 
+/* 0: no kernel takes a workspace for this request */
+int cppmega_mi355_dsa_indexer_loss_workspace_bytes(const cppmega_mi355_dsa_loss_args_t* args, size_t args_size, size_t* bytes);
 int cppmega_mi355_dsa_indexer_loss(const cppmega_mi355_dsa_loss_args_t* args, size_t args_size, void* stream);
 
 /* ---- FP8 vecmat / skinny GEMM ----------------------------------------------

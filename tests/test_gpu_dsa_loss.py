@@ -156,3 +156,41 @@ def test_bench_size_properties():
                         AD ** -0.5, mask)
         d = float(dsa_splitk_indexer_loss_per_position(idx, top, q, k, AD ** -0.5, False)[0, sq])
         assert abs(d - w) <= 2e-5 + 2e-4 * abs(w), (sq, d, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(130, 1, 3, 96, 203, 40), (200, 2, 5, 64, 97, 33), (64, 1, 1, 128, 64, 64), (65, 1, 2, 32, 129, 1), (1, 3, 2, 64, 1, 1)])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("sparse", [False, True])
+def test_tile_edges(shape, dt, sparse):
+    """Positions and keys that are not whole tiles of 64 x 128, more positions than keys and the other way round, rows of
+    index scores that are not whole 16-byte loads."""
+    ASq, AB, AH, AD, Sk, topk = shape
+    q, k, idx, top = _case(ASq + Sk, ASq, AB, AH, AD, Sk, topk, DTYPES[dt])
+    got = dsa_splitk_indexer_loss_per_position(idx.cuda(), top.cuda(), q.cuda(), k.cuda(), AD ** -0.5, sparse).cpu().numpy()
+    np.testing.assert_allclose(got, _want(q, k, idx, top, AD ** -0.5, sparse), atol=2e-5, rtol=2e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(4096, 1, 64, 32, 4096, 0), (300, 2, 4, 64, 300, 50)])
+def test_tiled_kernels_agree_with_the_kernel_without_a_workspace(shape):
+    """Several slabs of positions (64 heads x 4096 positions), and an additive mask with masked rows."""
+    import ctypes as C
+
+    from cppmega_mlx_amd import _lib, ops
+    ASq, AB, AH, AD, Sk, topk = shape
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, k = (torch.randn((n, AB, AH, AD), generator=g, device="cuda").to(torch.bfloat16) for n in (ASq, Sk))
+    idx = torch.randn((AB, ASq, Sk), generator=g, device="cuda")
+    mask = None
+    if topk:
+        mask = torch.where(torch.rand((AB, ASq, Sk), generator=g, device="cuda") < 0.3, float("-inf"), torch.randn((AB, ASq, Sk), generator=g, device="cuda"))
+        mask[:, 7] = float("-inf")
+    got, want = (torch.empty((AB, ASq), device="cuda") for _ in range(2))
+    ops.dsa_indexer_loss(q, k, idx, softmax_scale=AD ** -0.5, out=got, index_mask=mask)
+    a = _lib.DsaLossArgs()
+    a.struct_size, a.in_dtype, a.softmax_scale = _lib.DsaLossArgs.workspace.offset, _lib.BF16, AD ** -0.5
+    a.query, a.key, a.index_scores, a.index_mask, a.loss = q.data_ptr(), k.data_ptr(), idx.data_ptr(), _lib.ptr(mask), want.data_ptr()
+    a.seq_q, a.batch, a.heads, a.head_dim, a.seq_k = ASq, AB, AH, AD, Sk
+    assert _lib.load().cppmega_mi355_dsa_indexer_loss(C.byref(a), a.struct_size, _lib.current_stream(q.device)) == 0
+    torch.testing.assert_close(got, want, atol=2e-5, rtol=2e-4)
