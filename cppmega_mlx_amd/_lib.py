@@ -441,6 +441,18 @@ def load() -> C.CDLL:
         return lib
 
 
+def load_host():
+    """The launch path of the per-step calls (csrc/host_calls.cpp); its functions return None for a call that is not
+    the plain case, which then takes the checks and the struct of the Python helpers."""
+    try:
+        from . import _host
+    except ImportError as exc:
+        raise NativeLibraryError(
+            f"cannot load the extension beside {LIB_PATH}: {exc}; build it with `python -m cppmega_mlx_amd.build`. "
+            "There is no fallback path.") from exc
+    return _host
+
+
 _status_cache: dict[str, Any] | None = None
 
 

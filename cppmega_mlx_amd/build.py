@@ -2,7 +2,8 @@
 
 ``python -m cppmega_mlx_amd.build`` compiles every ``csrc/*.hip`` translation
 unit and links the shared library next to this package, where the loader in
-``_lib.py`` looks for it.  hipcc cross-compiles without a GPU.
+``_lib.py`` looks for it, and then the CPython extension that launches the
+per-step calls.  hipcc cross-compiles without a GPU.
 """
 
 from __future__ import annotations
@@ -18,6 +19,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_NAME = "libcppmega_mi355.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+HOST_PATH = PKG_DIR / "_host.so"          # the CPython extension in front of it (csrc/host_calls.cpp)
 OBJ_DIR = PKG_DIR / "csrc" / "build"
 
 OFFLOAD_ARCH = "gfx950"
@@ -102,7 +104,31 @@ def build(verbose: bool = True, jobs: int | None = None) -> Path:
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, LIB_PATH)
+    _build_host(verbose)
     return LIB_PATH
+
+
+def _build_host(verbose: bool) -> None:
+    """Compile csrc/host_calls.cpp against torch's headers and link it to the library beside it."""
+    import sysconfig
+
+    import torch
+
+    torch_dir = Path(torch.__file__).resolve().parent
+    rocm = Path(_hipcc()).resolve().parent.parent
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{torch_dir}/include", f"-I{torch_dir}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}", f"-I{rocm}/include",
+           str(CSRC / "host_calls.cpp"), "-o", str(tmp),
+           f"-L{torch_dir}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           f"-L{PKG_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for host_calls.cpp:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, HOST_PATH)
 
 
 if __name__ == "__main__":

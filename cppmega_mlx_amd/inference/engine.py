@@ -101,6 +101,11 @@ class SparseFP8KVCache:
         as views of the cache (reference: ``engine.py:76-98``)."""
         layer = self._sparse_fp8_layer(layer_idx)
         cfg = self.config
+        if getattr(kv_fp8, "dtype", None) == torch.uint8:
+            views = ops.host.cache_append(kv_fp8, kv_scale, None, layer.kv, layer.scale, None, layer.offset, cfg.scale_block, False)
+            if views is not None:
+                layer.offset = views[0].shape[1]
+                return views[:2]
         if not isinstance(kv_fp8, torch.Tensor) or not isinstance(kv_scale, torch.Tensor):
             raise TypeError("kv_fp8 and kv_scale must be torch.Tensor instances")
         if kv_fp8.ndim != 4:
@@ -134,6 +139,11 @@ class SparseFP8KVCache:
         beside it; returns ``(kv, scale, rope)`` views up to the new position."""
         layer = self._sparse_fp8_layer(layer_idx)
         cfg = self.config
+        if (rope is None) == (layer.rope is None) and latent.dtype != torch.uint8:
+            views = ops.host.cache_append(latent, None, rope, layer.kv, layer.scale, layer.rope, layer.offset, cfg.scale_block, cfg.pow2_scales)
+            if views is not None:
+                layer.offset = views[0].shape[1]
+                return views
         if latent.ndim != 4 or tuple(latent.shape[0:1] + latent.shape[2:]) != (cfg.batch_size, cfg.num_kv_heads, cfg.head_dim):
             raise ValueError("latent must have shape (batch, sequence, kv_heads, head_dim) matching the cache config")
         sequence = int(latent.shape[1])

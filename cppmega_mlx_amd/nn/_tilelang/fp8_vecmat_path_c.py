@@ -112,6 +112,8 @@ def fp8_scaled_vecmat_path_c_direct(
     kernel's tuning knobs; the HIP kernels pick their own tiling and ignore them.
     """
     del outputs_per_block, reduce_threads, vec
+    if ops.host.vecmat(x_fp8, W_fp8, scale_x, scale_w, out) is not None:
+        return out
     if not fp8_vecmat_path_c_status().available:
         raise FP8VecmatPathCDirectError(fp8_vecmat_path_c_status().reason)
     if W_fp8.ndim != 2 or x_fp8.ndim not in (1, 2):

@@ -81,6 +81,10 @@ def sparse_mla_blockscaled_path_c_apply_direct(
     kernel: str = "auto",
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """Forward into caller-owned ``out``/``lse``; returns those same objects."""
+    if out is not None and lse is not None and kernel in ops.KERNELS:
+        if ops.host.sparse_mla(q_fp8, q_scale, kv_fp8, kv_scale, kv_rope, indices, None, out, lse, d_v, float(sm_scale), ops.RULES_BLOCKSCALED,
+                               ops.KERNELS[kernel], False) is not None:
+            return out, lse
     status = sparse_mla_blockscaled_path_c_status()
     if not status.available:
         raise SparseMLABlockScaledPathCDirectError(status.reason)

@@ -102,6 +102,10 @@ def sparse_mla_fp8_path_c_apply_direct(
     kernel: str = "auto",
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """Forward into caller-owned ``out``/``lse``; returns those same objects."""
+    if out is not None and lse is not None and output_dtype is None and kernel in ops.KERNELS:
+        if ops.host.sparse_mla(q_fp8, q_scale, kv_fp8, kv_scale, kv_rope, indices, sinks, out, lse, d_v, float(sm_scale), ops.RULES_PER_TOKEN,
+                               ops.KERNELS[kernel], False) is not None:
+            return out, lse
     status = sparse_mla_fp8_path_c_status()
     if not status.available:
         raise SparseMLAFp8PathCDirectError(status.reason)

@@ -45,6 +45,8 @@ __all__ = [
     "topk_selector_tilelang_direct",
 ]
 
+_HIP_BACKENDS = frozenset(("auto", "mlx", "tilelang", "path_c", "hip"))
+_ORDERS = ("index", "value")
 MAX_WIDTH = 65536  # columns one workgroup keeps in registers
 _SCORE_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
@@ -121,6 +123,10 @@ def topk_selector_tilelang_direct(
     current stream; no host synchronisation happens here.  The default order
     is value-descending, the order of the reference kernel this entry replaces.
     """
+    if out is not None and order in _ORDERS:
+        done = ops.host.topk(scores, k, starts, ends, out, order == "value", bool(neg_inf_is_masked))
+        if done is not None:
+            return done
     batch, _ = _check_scores(scores, k)
     if batch <= 0 or scores.numel() == 0:
         raise TopKPathCDirectError("empty topk inputs are not dispatchable")
@@ -226,6 +232,10 @@ def topk_selector(
     or ``(B, S, T)`` (then ``starts``/``ends`` are ``(B*S,)`` and the result is
     ``(B, S, k)``).
     """
+    if backend in _HIP_BACKENDS and order in _ORDERS:
+        done = ops.host.topk(scores, k, starts, ends, None, order == "value", bool(neg_inf_is_masked))
+        if done is not None:
+            return done
     if backend not in {"auto", "mlx", "metal", "tilelang", "path_c", "hip"}:
         raise ValueError(f"unknown backend {backend!r}")
     if backend == "metal":

@@ -79,6 +79,9 @@ def indexer_scores_topk(q: torch.Tensor, k: torch.Tensor, weights: torch.Tensor,
     """``argpartition(-(einsum("bqhd,bkd,bqh->bqk") * sm_scale + mask))[..., :topk]`` as int32
     [B, T, min(index_topk, T_kv)], ascending by index; ``ends`` ([B*T] int32) bounds each row's
     selectable keys without a mask read."""
+    done = ops.host.indexer(q, k, weights, float(sm_scale), int(index_topk), mask, ends, out)
+    if done is not None:
+        return done
     B, T = q.shape[0], q.shape[1]
     topk = min(int(index_topk), int(k.shape[1]))
     if out is None:

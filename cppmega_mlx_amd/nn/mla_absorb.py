@@ -49,6 +49,8 @@ def _dense(t: torch.Tensor) -> torch.Tensor:
 def absorb_query(q: torch.Tensor, w_uk_abs: torch.Tensor, *, out: torch.Tensor | None = None) -> torch.Tensor:
     """q_abs[b,t,h,:] = q[b,t,h,:] @ w_uk_abs[h] ("bthk,hkv->bthv"); ``out`` may be the leading D_kv
     channels of wider query rows (a view with its own strides)."""
+    if out is not None and ops.host.absorb_query(q, w_uk_abs, out) is not None:
+        return out
     b, t, h, d_k = q.shape
     d_kv = w_uk_abs.shape[2]
     if out is None:

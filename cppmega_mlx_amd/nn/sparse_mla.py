@@ -158,6 +158,14 @@ def sparse_mla_attention(
                                           kernel="mfma")
         except ops._lib.NativeCallError as exc:
             raise RuntimeError(f"sparse_mla_attention: Path C unavailable: {exc}") from exc
+    done = None
+    if sm_scale is None or isinstance(sm_scale, (int, float)):
+        scale = (q.shape[-1] ** -0.5 if q.ndim == 4 else 1.0) if sm_scale is None else float(sm_scale)
+        done = ops.host.sparse_mla(q, None, kv, None, None, indices, None, None, None, d_v, scale, ops.RULES_FLOAT,
+                                   ops.KERNELS["auto"], bool(return_lse))
+    if done is not None:
+        record_dispatch("sparse_mla", path, "hip_mfma_gfx950" if done[2] == ops.KERNELS["mfma"] else "hip_scalar_fp32")
+        return done[:2] if return_lse else done[0]
     shapes = _resolve_shapes(q, kv, indices, d_v=d_v)
     _check_carriers(q, kv, indices)
     chosen = ops.sparse_mla_selected_kernel(q, kv, indices, d_v=shapes.d_v)

@@ -5,8 +5,9 @@ dense device tensors and enqueue the kernel on torch's current HIP stream.
 They validate what the C side cannot see (tensor ranks, devices, contiguity)
 and leave value/shape contracts to the library, whose status codes come back as
 ``ValueError`` / ``TypeError`` / ``NativeCallError``.  Outputs are caller-owned;
-the only tensor this module ever creates is the split-KV / split-K workspace,
-kept per device and reused, unless the caller passes ``workspace=``.
+the only tensor this module ever creates is the workspace, kept per device and
+stream and reused, unless the caller passes ``workspace=``.  The calls of every
+step have a native launch path in front of these helpers (``host``).
 """
 
 from __future__ import annotations
@@ -19,24 +20,18 @@ import torch
 
 from . import _lib
 
-_ws_lock = threading.Lock()
-_workspaces: dict[tuple[int, int], torch.Tensor] = {}
-
+host = _lib.load_host()
 
 def _workspace(device: torch.device, nbytes: int, stream: int) -> torch.Tensor | None:
-    """Per-(device, stream) scratch, grown geometrically, never shrunk."""
+    """Per-(device, stream) scratch, grown geometrically up to 1 GiB; a larger request gets a tensor of its own."""
     if nbytes <= 0:
         return None
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
-    with _ws_lock:
-        buf = _workspaces.get(key)
-        if buf is None or buf.numel() < nbytes:
-            size = max(nbytes, 1 << 20)
-            if buf is not None:
-                size = max(size, 2 * buf.numel())
-            buf = torch.zeros(size, dtype=torch.uint8, device=device)
-            _workspaces[key] = buf
-        return buf
+    return host.workspace(device.index if device.index is not None else torch.cuda.current_device(), nbytes, stream)
+
+
+def release_workspaces() -> None:
+    """Give the scratch kept between calls back to torch's allocator (the next calls allocate it again)."""
+    host.release_workspaces()
 
 
 def _dtype_or_raise(t: torch.Tensor, name: str, allowed: tuple[int, ...]) -> int:
@@ -64,6 +59,10 @@ def topk_select(
 ) -> torch.Tensor:
     """Write the per-row top-k indices of ``scores`` (rows, width) into ``out`` (rows, k).  Rows wider
     than 16384 columns go through a workspace in two stages unless ``two_stage`` is off."""
+    if workspace is None and two_stage and order in ("index", "value"):
+        done = host.topk(scores, k, starts, ends, out, order == "value", bool(neg_inf_is_masked))
+        if done is not None:
+            return done
     _lib.require_device_tensor(scores, "scores")
     _lib.require_device_tensor(out, "out", scores)
     if scores.ndim != 2:
@@ -205,6 +204,8 @@ def head_gemm(x: torch.Tensor, w: torch.Tensor, *, out: torch.Tensor) -> torch.T
 
     ``x`` [M, G, K] and ``out`` [M, G, N] may be views with their own row and group strides (the
     last axis contiguous); ``w`` [G, N, K] is dense.  float32 / bfloat16 operands, fp32 accumulation."""
+    if host.head_gemm(x, w, out) is not None:
+        return out
     for name, t in (("x", x), ("w", w), ("out", out)):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{name} must be a torch.Tensor")
@@ -360,7 +361,10 @@ class QuantSpec:
     block: int = 0
 
 
-_KERNELS = {"auto": _lib.MLA_KERNEL_AUTO, "scalar": _lib.MLA_KERNEL_SCALAR, "mfma": _lib.MLA_KERNEL_MFMA}
+# which wrapper's rules the native launch path applies to the operands
+RULES_BLOCKSCALED, RULES_PER_TOKEN, RULES_FLOAT = range(3)
+
+KERNELS = {"auto": _lib.MLA_KERNEL_AUTO, "scalar": _lib.MLA_KERNEL_SCALAR, "mfma": _lib.MLA_KERNEL_MFMA}
 
 
 def _cache_pitch(kv, kv_scale, kv_rope) -> int:
@@ -378,7 +382,7 @@ def _fill_mla_args(q, q_spec, kv, kv_spec, kv_rope, indices, sm_scale, d_v, sink
     rope_dim = 0 if kv_rope is None else kv_rope.shape[-1]
     a = _lib.SparseMlaArgs()
     a.struct_size = C.sizeof(a)
-    a.kernel = _KERNELS[kernel]
+    a.kernel = KERNELS[kernel]
     a.q = q.data_ptr()
     a.q_scale = _lib.ptr(q_spec.scale)
     a.q_dtype = _dtype_or_raise(q, "q", (_lib.F32, _lib.F16, _lib.BF16, _lib.E4M3))
@@ -446,7 +450,7 @@ def sparse_mla_forward(
     """
     q_spec = q_spec or QuantSpec()
     kv_spec = kv_spec or QuantSpec()
-    if kernel not in _KERNELS:
+    if kernel not in KERNELS:
         raise ValueError(f"unknown kernel {kernel!r}")
     named = [("q", q), ("kv", kv), ("indices", indices), ("out", out), ("lse", lse), ("kv_rope", kv_rope),
              ("sinks", sinks), ("q_scale", q_spec.scale), ("kv_scale", kv_spec.scale)]
@@ -591,7 +595,7 @@ def sparse_mla_selected_kernel(q, kv, indices, *, d_v, q_spec=None, kv_spec=None
     rc = _lib.load().cppmega_mi355_sparse_mla_select_kernel(C.byref(a), C.sizeof(a))
     if rc < 0:
         _lib.check(-rc, "sparse_mla_select_kernel")
-    return {v: k for k, v in _KERNELS.items()}[rc]
+    return {v: k for k, v in KERNELS.items()}[rc]
 
 
 # ---------------------------------------------------------------------------

@@ -159,7 +159,8 @@ def test_bench_size_properties():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape", [(130, 1, 3, 96, 203, 40), (200, 2, 5, 64, 97, 33), (64, 1, 1, 128, 64, 64), (65, 1, 2, 32, 129, 1), (1, 3, 2, 64, 1, 1)])
+@pytest.mark.parametrize("shape", [(130, 1, 3, 96, 203, 40), (200, 2, 5, 64, 97, 33), (64, 1, 1, 128, 64, 64), (65, 1, 2, 32, 129, 1), (1, 3, 2, 64, 1, 1),
+                                   (130, 1, 2, 32, 345, 20)])
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("sparse", [False, True])
 def test_tile_edges(shape, dt, sparse):
@@ -172,7 +173,7 @@ def test_tile_edges(shape, dt, sparse):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape", [(4096, 1, 64, 32, 4096, 0), (300, 2, 4, 64, 300, 50)])
+@pytest.mark.parametrize("shape", [(4096, 1, 64, 32, 4096, 0), (389, 2, 4, 64, 389, 50)])
 def test_tiled_kernels_agree_with_the_kernel_without_a_workspace(shape):
     """Several slabs of positions (64 heads x 4096 positions), and an additive mask with masked rows."""
     import ctypes as C
