@@ -52,6 +52,7 @@ EXPORTED_SYMBOLS = (
     "cppmega_mi355_head_gemm",
     "cppmega_mi355_dsa_indexer_loss_workspace_bytes",
     "cppmega_mi355_dsa_indexer_loss",
+    "cppmega_mi355_sparse_mla_bwd_workspace_bytes",
     "cppmega_mi355_sparse_mla_bwd",
     "cppmega_mi355_dequant_block_fp8",
     "cppmega_mi355_kv_cache_append",
@@ -162,6 +163,8 @@ class SparseMlaBwdArgs(C.Structure):
         ("dkv", C.c_void_p),
         ("q_scale", C.c_void_p),
         ("kv_scale", C.c_void_p),
+        ("workspace", C.c_void_p),
+        ("workspace_bytes", C.c_size_t),
     ]
 
 
@@ -421,6 +424,8 @@ def load() -> C.CDLL:
         lib.cppmega_mi355_fp8_quantize.restype = C.c_int
         lib.cppmega_mi355_sparse_mla_bwd.argtypes = [C.POINTER(SparseMlaBwdArgs), C.c_size_t, C.c_void_p]
         lib.cppmega_mi355_sparse_mla_bwd.restype = C.c_int
+        lib.cppmega_mi355_sparse_mla_bwd_workspace_bytes.argtypes = [C.POINTER(SparseMlaBwdArgs), C.c_size_t, C.POINTER(C.c_size_t)]
+        lib.cppmega_mi355_sparse_mla_bwd_workspace_bytes.restype = C.c_int
         lib.cppmega_mi355_dsa_indexer_loss.argtypes = [C.POINTER(DsaLossArgs), C.c_size_t, C.c_void_p]
         lib.cppmega_mi355_dsa_indexer_loss.restype = C.c_int
         lib.cppmega_mi355_dsa_indexer_loss_workspace_bytes.argtypes = [C.POINTER(DsaLossArgs), C.c_size_t, C.POINTER(C.c_size_t)]

@@ -37,6 +37,7 @@ int kv_cache_append_launch(const cppmega_mi355_cache_append_args_t& a, hipStream
 int causal_indices_launch(const cppmega_mi355_causal_indices_args_t& a, hipStream_t stream);
 int mask_indices_launch(const cppmega_mi355_mask_indices_args_t& a, hipStream_t stream);
 int sparse_mla_bwd_launch(const cppmega_mi355_sparse_mla_bwd_args_t& a, hipStream_t stream);
+int sparse_mla_bwd_workspace_bytes(const cppmega_mi355_sparse_mla_bwd_args_t& a, size_t* bytes);
 int dsa_indexer_loss_launch(const cppmega_mi355_dsa_loss_args_t& a, hipStream_t stream);
 int dsa_indexer_loss_workspace_bytes(const cppmega_mi355_dsa_loss_args_t& a, size_t* bytes);
 int head_gemm_launch(const cppmega_mi355_head_gemm_args_t& a, hipStream_t stream);
@@ -326,8 +327,18 @@ int cppmega_mi355_sparse_mla_scores(const cppmega_mi355_sparse_mla_args_t* args,
 }
 
 int cppmega_mi355_sparse_mla_bwd(const cppmega_mi355_sparse_mla_bwd_args_t* args, size_t args_size, void* stream) {
-  CM_CHECK_ARGS(args, args_size, cppmega_mi355_sparse_mla_bwd_args_t);
-  return sparse_mla_bwd_launch(*args, (hipStream_t)stream);
+  cppmega_mi355_sparse_mla_bwd_args_t a;
+  const int rc = widen_args(args, args_size, CPPMEGA_MI355_SPARSE_MLA_BWD_ARGS_V1_SIZE, a);
+  if (rc) return rc;
+  return sparse_mla_bwd_launch(a, (hipStream_t)stream);
+}
+
+int cppmega_mi355_sparse_mla_bwd_workspace_bytes(const cppmega_mi355_sparse_mla_bwd_args_t* args, size_t args_size, size_t* bytes) {
+  cppmega_mi355_sparse_mla_bwd_args_t a;
+  const int rc = widen_args(args, args_size, CPPMEGA_MI355_SPARSE_MLA_BWD_ARGS_V1_SIZE, a);
+  if (rc) return rc;
+  if (!bytes) return fail(CPPMEGA_MI355_ERR_NULL, "bytes is NULL");
+  return sparse_mla_bwd_workspace_bytes(a, bytes);
 }
 
 int cppmega_mi355_dsa_indexer_loss(const cppmega_mi355_dsa_loss_args_t* args, size_t args_size, void* stream) {

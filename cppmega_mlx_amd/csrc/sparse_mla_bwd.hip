@@ -168,18 +168,41 @@ bool operand_dtype(int dt) { return float_carrier(dt) || dt == CPPMEGA_MI355_E4M
 bool sparse_mla_bwd_mfma_supports(const cppmega_mi355_sparse_mla_bwd_args_t& a);                    // sparse_mla_bwd_mfma.hip
 int sparse_mla_bwd_mfma_launch(const cppmega_mi355_sparse_mla_bwd_args_t& a, hipStream_t stream);
 
-int sparse_mla_bwd_launch(const cppmega_mi355_sparse_mla_bwd_args_t& a, hipStream_t stream) {
-  if (!a.q || !a.kv || !a.d_out || !a.indices || !a.dq || !a.dkv) return fail(CPPMEGA_MI355_ERR_NULL, "sparse_mla_bwd: a pointer is NULL");
+bool sparse_mla_bwd_split_supports(const cppmega_mi355_sparse_mla_bwd_args_t& a);                   // sparse_mla_bwd_split.hip
+size_t sparse_mla_bwd_split_workspace_bytes(const cppmega_mi355_sparse_mla_bwd_args_t& a);
+int sparse_mla_bwd_split_launch(const cppmega_mi355_sparse_mla_bwd_args_t& a, hipStream_t stream);
+
+static int check_shape(const cppmega_mi355_sparse_mla_bwd_args_t& a) {
   if (a.batch < 0 || a.seq_q < 0 || a.heads < 1 || a.kv_groups < 1 || a.seq_kv < 0 || a.topk < 0 || a.d_qk < 1)
     return fail(CPPMEGA_MI355_ERR_SHAPE, "sparse_mla_bwd: negative or empty dimension");
   if (a.heads % a.kv_groups != 0) return fail(CPPMEGA_MI355_ERR_SHAPE, "heads %d not divisible by kv_group %d", a.heads, a.kv_groups);
   if (a.d_v <= 0 || a.d_v > a.d_qk) return fail(CPPMEGA_MI355_ERR_SHAPE, "d_v must be in (0, %d], got %d", a.d_qk, a.d_v);
   if (!operand_dtype(a.q_dtype) || !operand_dtype(a.kv_dtype) || !float_carrier(a.d_out_dtype) || !float_carrier(a.dq_dtype))
     return fail(CPPMEGA_MI355_ERR_DTYPE, "sparse_mla_bwd: q / kv must be float32, float16, bfloat16 or e4m3; d_out and dq a float carrier");
+  return 0;
+}
+
+int sparse_mla_bwd_workspace_bytes(const cppmega_mi355_sparse_mla_bwd_args_t& a, size_t* bytes) {
+  const int rc = check_shape(a);
+  if (rc) return rc;
+  *bytes = sparse_mla_bwd_split_supports(a) ? sparse_mla_bwd_split_workspace_bytes(a) : 0;
+  return 0;
+}
+
+int sparse_mla_bwd_launch(const cppmega_mi355_sparse_mla_bwd_args_t& a, hipStream_t stream) {
+  if (!a.q || !a.kv || !a.d_out || !a.indices || !a.dq || !a.dkv) return fail(CPPMEGA_MI355_ERR_NULL, "sparse_mla_bwd: a pointer is NULL");
+  const int rc = check_shape(a);
+  if (rc) return rc;
   if ((a.q_dtype == CPPMEGA_MI355_E4M3 && !a.q_scale) || (a.kv_dtype == CPPMEGA_MI355_E4M3 && !a.kv_scale))
     return fail(CPPMEGA_MI355_ERR_NULL, "sparse_mla_bwd: e4m3 operands need their per-token scales");
   if (a.index_dtype != CPPMEGA_MI355_I32 && a.index_dtype != CPPMEGA_MI355_I64)
     return fail(CPPMEGA_MI355_ERR_DTYPE, "sparse_mla_bwd: indices must be int32 or int64");
+  if (a.workspace && sparse_mla_bwd_split_supports(a)) {
+    const size_t need = sparse_mla_bwd_split_workspace_bytes(a);
+    if (a.workspace_bytes < need)
+      return fail(CPPMEGA_MI355_ERR_WORKSPACE, "sparse_mla_bwd: workspace of %zu bytes needed, %zu given", need, (size_t)a.workspace_bytes);
+    return sparse_mla_bwd_split_launch(a, stream);
+  }
   const bool on_matrix_cores = sparse_mla_bwd_mfma_supports(a);      // bfloat16 / float16 (or per-token e4m3) operands
   const size_t lds = ((size_t)3 * a.topk + a.d_qk + a.d_v + 8) * sizeof(float);
   if (!on_matrix_cores && lds > 160 * 1024) return fail(CPPMEGA_MI355_ERR_UNSUPPORTED, "sparse_mla_bwd: topk %d with d_qk %d needs %zu bytes of LDS (limit 160 KiB)", a.topk, a.d_qk, lds);

@@ -38,6 +38,7 @@
 
 #include "common.h"
 #include "mfma_util.h"
+#include "sparse_mla_bwd_util.h"
 
 namespace cm {
 namespace {
@@ -63,21 +64,6 @@ struct BwdMfmaParams {
   float sm_scale;
 };
 
-__device__ __forceinline__ bf16x8 lds_b128(const unsigned short* p) { return *reinterpret_cast<const bf16x8*>(p); }
-
-// Transposing read: within a group of 16 lanes, lane i points at 4 consecutive elements
-// (row i / 4, columns 4 * (i % 4) ..) of a 4 x 16 block and receives column i of rows 0..3.
-__device__ __forceinline__ bf16x4 lds_tr16(const unsigned short* p) {
-  typedef __attribute__((ext_vector_type(4))) short s16x4;
-  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
-  return __builtin_bit_cast(bf16x4, v);
-}
-__device__ __forceinline__ bf16x8 join(const bf16x4 a, const bf16x4 b) {
-  bf16x8 r;
-  r[0] = a[0]; r[1] = a[1]; r[2] = a[2]; r[3] = a[3];
-  r[4] = b[0]; r[5] = b[1]; r[6] = b[2]; r[7] = b[3];
-  return r;
-}
 // 8 e4m3 bytes -> 8 float16 / 8 bfloat16, exact
 __device__ __forceinline__ uint4 e4m3x8_to_f16(const uint2 v) {
   uint4 r;
@@ -95,25 +81,12 @@ __device__ __forceinline__ uint4 e4m3x8_to_bf16(const uint2 v) {
   r.w = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v.y, 1.0f, true));
   return r;
 }
-typedef _Float16 f16x8b __attribute__((ext_vector_type(8)));
-// one matrix instruction on operands held as 8 x 16 bits: bfloat16, or float16 when F16
-template <bool F16>
-__device__ __forceinline__ f32x4 mm(const bf16x8 a, const bf16x8 b, const f32x4 c) {
-  if (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8b, a), __builtin_bit_cast(f16x8b, b), c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ bf16x8 zero8() {
-  return __builtin_bit_cast(bf16x8, make_uint4(0u, 0u, 0u, 0u));
-}
-
 // EL: 0 bfloat16 operands, 1 per-token e4m3 operands with a bfloat16 cotangent, 2 float16 operands,
 //     3 per-token e4m3 operands with a float16 cotangent
 template <int HB, int EL>
 __global__ __launch_bounds__(kThreads, 1) void sparse_mla_bwd_mfma_kernel(const BwdMfmaParams p) {
   constexpr bool FP8 = EL == 1 || EL == 3, F16 = EL == 2 || EL == 3;
-  // float16 planes of P and dS are kept at 16 times their value: a float16 is flushed below 6e-8 and overflows above
-  // 65504, so entries down to 4e-9 survive and |dS| may reach 4000
-  constexpr float kPlaneScale = F16 ? 16.0f : 1.0f, kPlaneUnscale = F16 ? 1.0f / 16.0f : 1.0f;
+  constexpr float kPlaneScale = PlaneScale<F16>::up, kPlaneUnscale = PlaneScale<F16>::down;
   constexpr int HC = 16 * HB;            // heads per workgroup
   constexpr int KT = 64 / HB;            // keys per tile
   constexpr int KSUB = KT / 16;          // 16-key blocks per tile

@@ -1,0 +1,744 @@
+// Sparse MLA backward in separate steps over a workspace: bfloat16 or float16 operands (gfx950).
+//
+// sparse_mla_bwd_mfma.hip adds every (selected row, channel) of every query to dkv with a float32 atomic
+// at the L2, which takes one element per channel and clock: 151 M adds are 0.47 ms whatever else runs.
+// With a workspace the adds happen in LDS instead, and the steps that do not need each other's registers run
+// at their own occupancy:
+//
+//   lists    per (query, group): its valid keys in order, and where each band of keys begins;
+//   steps    per band: the pieces of up to 16 keys that the queries have in it, one after the other;
+//   scores   per (query, 16 heads): S = Q . K^T and dP = dO . K^T with the scores of all keys in registers,
+//            softmax statistics and delta across the workgroup, then P and dS = sm_scale P (dP - delta) as two
+//            16-bit planes each (hi = round(x), lo = round(x - hi), a term is good to 2^-17), and q and d_out by
+//            channel, both as dkv's matrix instructions take them: a load is 1 KB in a row;
+//   dq       per (query, 16 heads, 144 channels): dQ^T = K^T . dS^T over 32-key tiles staged in LDS;
+//   dkv      per (four bands, 64 channels, share of the steps): dS^T . Q + P^T . dO of every step, added to a
+//            float32 tile in LDS, written out once;
+//   sum      over the shares, when there are several.
+//
+// Nothing is added in an order that varies: the same input gives the same bits.
+//
+// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 172 us (561 us with the atomics): lists 8,
+// steps 7, scores 38, dq 31, dkv 89, sum 9.  dkv is bound by the vector cache (27 M accesses of 64 bytes, 51 us if
+// it never waited: 4 KB of q and d_out and about 1 KB of planes for a step's 9 keys of 16) and by the issue of its
+// one wavefront per SIMD; scores and dq by the gather of 302 MB of key rows each.
+
+#include <algorithm>
+
+#include "common.h"
+#include "mfma_util.h"
+#include "sparse_mla_bwd_util.h"
+
+namespace cm {
+namespace {
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kThreads = 256;
+constexpr int kBands = 4;              // bands of keys in a dkv tile
+constexpr int kBandKeys = 150;         // at most: 601 rows of 64 floats (one for nobody) are 154 KB of LDS
+constexpr int kAhead = 4;              // steps on their way in dkv
+constexpr int kAgain = 1 << 30;        // mark of a slot whose key occurs earlier in the same 16 slots
+constexpr int kHeads = 16;             // heads of an item
+constexpr int kRowBytes = 128;         // of planes per key
+constexpr size_t kSlabBytes = 192u << 20;
+
+struct SplitParams {
+  const unsigned short* q;      // [B, S, H, D]
+  const unsigned short* kv;     // [B, Skv, G, D]
+  const unsigned short* d_out;  // [B, S, H, d_v]
+  const void* indices;          // [B, S, G, topk]
+  const float* sm_scale_dev;
+  void* dq;                     // [B, S, H, D]
+  float* dkv;                   // [B, Skv, G, D]
+  int* keys;                    // [lists][stride] ascending, -1 behind the last
+  int* starts;                  // [lists][bands + 2]: first slot of each band, the number of keys, whether one is marked kAgain
+  int* step_starts;             // [lists][bands]: each band's first step among the list's
+  int* rows;                    // [lists][list_steps][16]: where in its tile of dkv a slot's key stands, band by band in whole steps
+  int* band_steps;              // the number of steps so far, then [B * G * bands][first, number]
+  i32x4* steps;                 // byte offsets of planes, rows (| keys | 32 if one may be marked), by_channel, keys
+  char* planes;                 // [lists][chunks][hi, lo][dS heads 0-7, 8-15, P heads 0-7, 8-15][stride][8]
+  unsigned short* by_channel;   // [lists][chunks][D / 64][channel % 4][q heads 0-7, 8-15, d_out heads 0-7, 8-15][16 channels][8]
+  float* part;                  // [shares][B, Skv, G, D]
+  int dq_dtype, index_dtype;
+  int B, S, H, G, Skv, topk, D, d_v;
+  int channels;                 // D in whole tiles of dkv
+  int s0, ns;                   // queries of this slab: s0 .. s0 + ns of every sequence; list = (b * ns + s - s0) * G + g
+  int chunks;                   // of 16 heads per group
+  int stride;                   // key slots per list: topk in whole tiles, and two tiles to read past
+  int tiles, bands, band_keys, shares;                  // bands = tiles * kBands of band_keys keys
+  int list_steps;               // at most, of 16 slots of one band
+  unsigned dead_step;           // byte offset in rows of a step of no keys
+  int accumulate;               // add to dkv
+  float sm_scale;
+};
+
+constexpr int kDeadRow = kBands * kBandKeys;           // of slots of no key
+
+// ---- lists -----------------------------------------------------------------------------------
+// The valid keys by band in LDS, then each to its rank within the band.
+__global__ __launch_bounds__(kThreads) void bwd_lists_kernel(const SplitParams p) {
+  extern __shared__ int smem_lists[];
+  int* begin = smem_lists;                             // [bands]
+  int* fill = begin + p.bands;                         // [bands]
+  int* loose = fill + p.bands;                         // [topk]
+  int* sorted = loose + p.topk;                        // [topk]
+  int* again = sorted + p.topk;                        // [1]
+  int* step_of = again + 1;                            // [bands + 1]: the band's first step
+  const int tid = (int)threadIdx.x, lane = tid & 63;
+  const size_t list = blockIdx.x;
+  const int g = (int)(list % p.G), s = (int)((list / p.G) % p.ns), b = (int)(list / ((size_t)p.G * p.ns));
+  const size_t src = (((size_t)b * p.S + p.s0 + s) * p.G + g) * (size_t)p.topk;
+  if (list == 0 && tid == 0) p.band_steps[0] = 0;
+  if (list == 0 && tid < 16) p.rows[p.dead_step / 4 + tid] = kDeadRow * 256;
+  for (int r = tid; r < p.bands; r += kThreads) fill[r] = 0;
+  if (tid == 0) *again = 0;
+  __syncthreads();
+  int key[8], band[8];                                 // topk <= 2048
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int k = tid + i * kThreads;
+    if (i * kThreads >= p.topk) {                      // (uniform)
+      key[i] = band[i] = -1;
+      continue;
+    }
+    long long v = -1;
+    if (k < p.topk)
+      v = p.index_dtype == CPPMEGA_MI355_I64 ? static_cast<const long long*>(p.indices)[src + k] : (long long)static_cast<const int*>(p.indices)[src + k];
+    key[i] = v >= 0 && v < p.Skv ? (int)v : -1;
+    band[i] = key[i] >= 0 ? key[i] / p.band_keys : -1;
+    if (band[i] >= 0) atomicAdd(fill + band[i], 1);
+  }
+  __syncthreads();
+  int* starts = p.starts + list * (p.bands + 2);
+  if (tid < 64) {                                      // exclusive prefix, 64 bands at a time
+    int base = 0, step_base = 0;
+    for (int r0 = 0; r0 < p.bands; r0 += 64) {
+      const int r = r0 + lane, n = r < p.bands ? fill[r] : 0, steps = (n + 15) / 16;
+      const int upto = (int)wave_inclusive_sum((unsigned)n), steps_upto = (int)wave_inclusive_sum((unsigned)steps);
+      if (r < p.bands) {
+        starts[r] = begin[r] = fill[r] = base + upto - n;
+        step_of[r] = step_base + steps_upto - steps;
+      }
+      base += __shfl(upto, 63, 64);
+      step_base += __shfl(steps_upto, 63, 64);
+    }
+    if (lane == 0) {
+      starts[p.bands] = base;
+      step_of[p.bands] = step_base;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (band[i] >= 0) loose[atomicAdd(fill + band[i], 1)] = key[i];
+  __syncthreads();
+  const int valid = fill[p.bands - 1];                 // (where its keys end now)
+  for (int e = tid; e < valid; e += kThreads) {
+    const int v = loose[e], first = begin[v / p.band_keys], last = fill[v / p.band_keys];
+    int at = first;
+    for (int o = first; o < last; ++o) at += loose[o] < v || (loose[o] == v && o < e);
+    sorted[at] = v;
+  }
+  __syncthreads();
+  // a key that its step of 16 (from the band's first slot on) holds already is marked, and has no row
+  int* out = p.keys + list * (size_t)p.stride;
+  int* rows = p.rows + list * (size_t)p.list_steps * 16;
+  for (int k = tid; k < p.stride; k += kThreads) {
+    int v = -1;
+    if (k < valid) {
+      v = sorted[k];
+      const int of = v / p.band_keys, nth = k - begin[of], row = v - of / kBands * (kBands * p.band_keys);
+      const bool marked = (nth & 15) != 0 && sorted[k - 1] == v;
+      int* at = rows + step_of[of] * 16 + nth;
+      *at = (marked ? kDeadRow : row) * 256;
+      if (k + 1 == fill[of])
+        for (int e = nth + 1; e & 15; ++e) *++at = kDeadRow * 256;
+      if (marked) {
+        v |= kAgain;
+        *again = 1;
+      }
+    }
+    out[k] = v;
+  }
+  __syncthreads();
+  if (tid == 0) starts[p.bands + 1] = *again;
+  for (int r = tid; r < p.bands; r += kThreads) p.step_starts[list * p.bands + r] = step_of[r];
+}
+
+// ---- steps -----------------------------------------------------------------------------------
+constexpr int kStepThreads = 1024;
+
+__global__ __launch_bounds__(kStepThreads) void bwd_steps_kernel(const SplitParams p) {
+  __shared__ int sums[kStepThreads / 64], base_of;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int band = (int)blockIdx.x % p.bands, bg = (int)blockIdx.x / p.bands, b = bg / p.G, g = bg - b * p.G;
+  const int per = (p.ns + kStepThreads - 1) / kStepThreads, s0 = min(tid * per, p.ns), s1 = min(s0 + per, p.ns);
+  auto row = [&](int s) { return p.starts + (((size_t)b * p.ns + s) * p.G + g) * (p.bands + 2); };
+  int mine = 0;
+  for (int s = s0; s < s1; ++s) mine += (row(s)[band + 1] - row(s)[band] + 15) / 16 * p.chunks;
+  const int upto = (int)wave_inclusive_sum((unsigned)mine);
+  if (lane == 63) sums[wave] = upto;
+  __syncthreads();
+  int at = upto - mine, all = 0;
+  for (int w = 0; w < kStepThreads / 64; ++w) {
+    if (w < wave) at += sums[w];
+    all += sums[w];
+  }
+  const int padded = (all + kAhead - 1) / kAhead * kAhead;            // with steps whose rows are all dead
+  if (tid == 0) {
+    base_of = atomicAdd(p.band_steps, padded);
+    p.band_steps[2 + 2 * blockIdx.x] = base_of;
+    p.band_steps[3 + 2 * blockIdx.x] = padded;
+  }
+  __syncthreads();
+  i32x4* out = p.steps + base_of;
+  for (int e = all + tid; e < padded; e += kStepThreads) out[e] = i32x4{0, (int)p.dead_step, 0, 0};
+  for (int s = s0; s < s1; ++s) {
+    const size_t list = ((size_t)b * p.ns + s) * p.G + g;
+    const int* st = row(s);
+    const int end = st[band + 1], marked = st[p.bands + 1];
+    unsigned row = ((unsigned)list * p.list_steps + p.step_starts[list * p.bands + band]) * 64;
+    for (int t = st[band]; t < end; t += 16, row += 64)
+      for (int c = 0; c < p.chunks; ++c) {
+        const unsigned item = (unsigned)(list * p.chunks + c);
+        out[at++] = i32x4{(int)(item * (unsigned)p.stride * kRowBytes + t * 16), (int)(row | min(end - t, 16) | (marked ? 32 : 0)),
+                          (int)(item * (unsigned)p.channels * 64), (int)(((unsigned)list * p.stride + t) * 4)};
+      }
+  }
+}
+
+// the key of a slot, -1 for none
+__device__ __forceinline__ int plain_key(int slot) { return slot < 0 ? -1 : slot & ~kAgain; }
+
+// sum / maximum over the 16 lanes of a row
+__device__ __forceinline__ float row_sum(float v) {
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+__device__ __forceinline__ float row_max(float v) {
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+  return v;
+}
+
+template <bool F16>
+__device__ __forceinline__ uint2 pack4(const float (&v)[4]) {
+  return F16 ? make_uint2(pack_f16(v[0], v[1]), pack_f16(v[2], v[3])) : make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+}
+// hi and lo planes of 4 values
+template <bool F16>
+__device__ __forceinline__ void put_planes(char* at, size_t to_lo, const float (&v)[4]) {
+  float hi[4], lo[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    hi[i] = v[i] * PlaneScale<F16>::up;
+    lo[i] = hi[i] - (F16 ? (float)(_Float16)hi[i] : (float)(__bf16)hi[i]);
+  }
+  *reinterpret_cast<uint2*>(at) = pack4<F16>(hi);
+  *reinterpret_cast<uint2*>(at + to_lo) = pack4<F16>(lo);
+}
+
+struct Item {
+  int g, b, chunk, h0, nh;
+  size_t list, bs;
+};
+__device__ __forceinline__ Item item_of(const SplitParams& p, size_t i) {
+  Item it;
+  it.chunk = (int)(i % p.chunks);
+  it.list = i / p.chunks;
+  it.g = (int)(it.list % p.G);
+  const int s = (int)((it.list / p.G) % p.ns);
+  it.b = (int)(it.list / ((size_t)p.G * p.ns));
+  it.bs = (size_t)it.b * p.S + p.s0 + s;
+  const int hg = p.H / p.G;
+  it.h0 = it.g * hg + it.chunk * kHeads;
+  it.nh = min(kHeads, hg - it.chunk * kHeads);
+  return it;
+}
+
+// ---- scores ------------------------------------------------------------------------------------
+// W wavefronts take the 16-key tiles in turn, up to T each.  A tile's rows come 32 channels at a time, four lanes
+// to a row (a load of 64 rows' pieces is served a lane at a time: 53 us for the form that read its operands
+// straight from memory), and go through 1 KB of LDS of the wavefront's own, so there is no barrier in the loop.
+// A lane ends up with 4 heads of one key.
+constexpr int kQueue = 6;                              // pieces of 32 channels on their way
+
+template <bool F16, int W, int T>
+__global__ __launch_bounds__(W * 64, 4) void bwd_scores_kernel(const SplitParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int D = p.D, dv = p.d_v, Dp = D + 8, Dvp = dv + 8;
+  unsigned short* Qs = reinterpret_cast<unsigned short*>(smem);       // [16][Dp]
+  unsigned short* Os = Qs + kHeads * Dp;                              // [16][Dvp]
+  float* met = reinterpret_cast<float*>(Os + kHeads * Dvp);           // [W][16][3]
+  unsigned short* pieces = reinterpret_cast<unsigned short*>(met + W * kHeads * 3);       // [W][16 keys][32]
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, kg = lane >> 4;
+  const Item it = item_of(p, blockIdx.x);
+  const float sm_scale = p.sm_scale_dev ? *p.sm_scale_dev : p.sm_scale;
+  const float scale2 = sm_scale * kLog2e;
+  const int* keys = p.keys + it.list * (size_t)p.stride;
+  const int valid = p.starts[it.list * (p.bands + 2) + p.bands], tiles = (valid + 15) / 16;
+
+  for (int e = tid; e < kHeads * (D / 8); e += W * 64) {
+    const int h = e / (D / 8), c = e - h * (D / 8);
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (h < it.nh) v = *reinterpret_cast<const u32x4*>(p.q + (it.bs * p.H + it.h0 + h) * (size_t)D + c * 8);
+    *reinterpret_cast<u32x4*>(Qs + h * Dp + c * 8) = v;
+  }
+  for (int e = tid; e < kHeads * (dv / 8); e += W * 64) {
+    const int h = e / (dv / 8), c = e - h * (dv / 8);
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (h < it.nh) v = *reinterpret_cast<const u32x4*>(p.d_out + (it.bs * p.H + it.h0 + h) * (size_t)dv + c * 8);
+    *reinterpret_cast<u32x4*>(Os + h * Dvp + c * 8) = v;
+  }
+  __syncthreads();
+
+  const unsigned short* qa = Qs + l16 * Dp + 8 * kg;
+  const unsigned short* oa = Os + l16 * Dvp + 8 * kg;
+  f32x4 s[T], dp[T];
+  float m[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  const int ks = D / 32, vs = dv / 32, groups = (ks + kQueue - 1) / kQueue;
+  const int row = lane >> 2, col = lane & 3;
+  unsigned short* put = pieces + wave * 512 + row * 32 + ((col ^ (-(row >> 2) & 3)) << 3);
+  const unsigned short* get = pieces + wave * 512 + l16 * 32 + ((kg ^ (-(l16 >> 2) & 3)) << 3);
+  const unsigned short* kv = p.kv + ((size_t)it.b * p.Skv * p.G + it.g) * (size_t)D + col * 8;
+  auto row_of = [&](int t) { return kv + (size_t)max(plain_key(keys[min(t, tiles - 1) * 16 + row]), 0) * p.G * (size_t)D; };
+  const unsigned short *cur = kv, *next = kv;
+  u32x4 queue[kQueue];
+  auto request = [&](int i, const unsigned short* at, int c) { queue[i] = *reinterpret_cast<const u32x4*>(at + min(c, ks - 1) * 32); };
+  if (wave < tiles) {
+    cur = row_of(wave);
+#pragma unroll
+    for (int i = 0; i < kQueue; ++i) request(i, cur, i);
+  }
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    const int t = wave + i * W;
+    if (t >= tiles) break;                             // (uniform)
+    const int key = plain_key(keys[t * 16 + l16]);
+    next = row_of(t + W);
+    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, da = {0.f, 0.f, 0.f, 0.f};
+    for (int c0 = 0; c0 < groups; ++c0) {
+      const bool last = c0 + 1 == groups;
+#pragma unroll
+      for (int q = 0; q < kQueue; ++q) {
+        const int c = c0 * kQueue + q;
+        *reinterpret_cast<u32x4*>(put) = queue[q];
+        request(q, last ? next : cur, last ? q : c + kQueue);
+        if (c < ks) {
+          const bf16x8 k = lds_b128(get);
+          sa = mm<F16>(lds_b128(qa + c * 32), k, sa);
+          if (c < vs) da = mm<F16>(lds_b128(oa + c * 32), k, da);
+        }
+      }
+    }
+    cur = next;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      s[i][v] = key >= 0 ? sa[v] * scale2 : -INFINITY;
+      m[v] = fmaxf(m[v], s[i][v]);
+    }
+    dp[i] = da;
+  }
+  // statistics of head 4 * kg + v: over the row of 16 lanes, then over the wavefronts
+#pragma unroll
+  for (int v = 0; v < 4; ++v) m[v] = row_max(m[v]);
+  if (l16 == 0)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) met[(wave * 16 + 4 * kg + v) * 3] = m[v];
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    m[v] = -INFINITY;
+    for (int w = 0; w < W; ++w) m[v] = fmaxf(m[v], met[(w * 16 + 4 * kg + v) * 3]);
+    m[v] = m[v] > -INFINITY ? m[v] : 0.0f;
+  }
+  float l[4] = {0.f, 0.f, 0.f, 0.f}, dot[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    if (wave + i * W >= tiles) break;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      s[i][v] = exp2f(s[i][v] - m[v]);
+      l[v] += s[i][v];
+      dot[v] = fmaf(s[i][v], dp[i][v], dot[v]);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    l[v] = row_sum(l[v]);
+    dot[v] = row_sum(dot[v]);
+  }
+  if (l16 == 0)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      met[(wave * 16 + 4 * kg + v) * 3 + 1] = l[v];
+      met[(wave * 16 + 4 * kg + v) * 3 + 2] = dot[v];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    float sum = 0.0f, d = 0.0f;
+    for (int w = 0; w < W; ++w) {
+      sum += met[(w * 16 + 4 * kg + v) * 3 + 1];
+      d += met[(w * 16 + 4 * kg + v) * 3 + 2];
+    }
+    l[v] = sum > 0.0f ? 1.0f / sum : 0.0f;
+    dot[v] = d * l[v];
+  }
+  char* out = p.planes + (it.list * p.chunks + it.chunk) * (size_t)p.stride * kRowBytes + (size_t)(kg >> 1) * p.stride * 16 + 8 * (kg & 1);
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    const int t = wave + i * W;
+    if (t >= tiles) break;
+    float pv[4], ds[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      pv[v] = s[i][v] * l[v];
+      ds[v] = pv[v] * (dp[i][v] - dot[v]) * sm_scale;
+    }
+    char* at = out + (size_t)(t * 16 + l16) * 16;
+    put_planes<F16>(at, (size_t)p.stride * 64, ds);
+    put_planes<F16>(at + (size_t)p.stride * 32, (size_t)p.stride * 64, pv);
+  }
+  // q and d_out by channel: lane (channel l16 of a block, kg): 8 heads of q (kg 0, 1) or of d_out (kg 2, 3)
+  const int tr_row = l16 >> 2, tr_col = (l16 & 3) * 4;
+  unsigned short* bc = p.by_channel + (it.list * p.chunks + it.chunk) * (size_t)p.channels * 32 + (l16 & 3) * 512 + kg * 128 + (l16 >> 2) * 8;
+  for (int cb = wave; cb < D / 16; cb += W) {
+    const bool has_v = cb * 16 < dv, from_q = kg < 2 || !has_v;      // (every lane issues the transposing read)
+    const unsigned short* src = from_q ? Qs + (8 * (kg & 1) + tr_row) * Dp + cb * 16 + tr_col : Os + (8 * (kg - 2) + tr_row) * Dvp + cb * 16 + tr_col;
+    bf16x8 v = join(lds_tr16(src), lds_tr16(src + 4 * (from_q ? Dp : Dvp)));
+    if (kg >= 2 && !has_v) v = zero8();
+    *reinterpret_cast<bf16x8*>(bc + (size_t)(cb >> 2) * 2048 + (cb & 3) * 32) = v;
+  }
+}
+
+// ---- dq ------------------------------------------------------------------------------------------
+// A workgroup is one wavefront with up to 144 channels of an item: the K tiles it stages in LDS are its own, so
+// nothing waits at a barrier (73 us for workgroups of four that shared 32 whole rows).
+constexpr int kStep = 32;                              // keys per tile
+constexpr int kBlocks = 9;                             // 16-channel blocks per wavefront
+constexpr int kPieces = kStep * kBlocks * 2 / 64;      // 16-byte pieces of a tile per lane
+// Bytes to a row: the rows that one transposing read takes together stand in different banks.
+__device__ __forceinline__ int k_row(int row) { return row * 320 + (row & 8) * 4; }
+constexpr int kKtile = kStep * 320 + 32;
+
+template <bool F16>
+__global__ __launch_bounds__(64, 3) void bwd_dq_kernel(const SplitParams p) {
+  __shared__ __align__(16) char Ks[kKtile];
+  __shared__ __align__(16) unsigned short Ss[2 * kStep * kHeads];     // [hi, lo][32 keys][16 heads]
+  const int D = p.D, nblk = D / 16, parts = (nblk + kBlocks - 1) / kBlocks;
+  const int lane = (int)threadIdx.x, l16 = lane & 15, kg = lane >> 4;
+  const int part = (int)(blockIdx.x % parts), b0 = part * kBlocks, blocks = min(kBlocks, nblk - b0);
+  const Item it = item_of(p, blockIdx.x / parts);
+  const int* keys = p.keys + it.list * (size_t)p.stride;
+  const int valid = p.starts[it.list * (p.bands + 2) + p.bands], steps = (valid + kStep - 1) / kStep;
+  const char* planes = p.planes + (it.list * p.chunks + it.chunk) * (size_t)p.stride * kRowBytes;
+  const unsigned short* kv = p.kv + ((size_t)it.b * p.Skv * p.G + it.g) * (size_t)D + b0 * 16;
+
+  int piece_row[kPieces], piece_col[kPieces];
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) {
+    const int e = lane + i * 64;
+    piece_row[i] = e / (kBlocks * 2);
+    piece_col[i] = e - piece_row[i] * (kBlocks * 2);
+  }
+  const int s_key = lane & 31, s_half = lane >> 5;
+  u32x4 pre[kPieces], pre_s[2];
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  int tile_keys = 0;
+  auto fetch_keys = [&](int step) { tile_keys = plain_key(keys[min(step * kStep + s_key, valid - 1)]); };
+  auto fetch = [&](int step) {                         // of the keys in tile_keys
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int key = __shfl(tile_keys, piece_row[i], 64);
+      pre[i] = *reinterpret_cast<const u32x4*>(kv + (size_t)key * p.G * (size_t)D + min(piece_col[i], blocks * 2 - 1) * 8);
+    }
+    const int pos = step * kStep + s_key;
+#pragma unroll
+    for (int pl = 0; pl < 2; ++pl) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(planes + ((size_t)(pl * 4 + s_half) * p.stride + min(pos, valid - 1)) * 16);
+      pre_s[pl] = pos < valid ? v : zero;
+    }
+  };
+  f32x4 acc[kBlocks];
+#pragma unroll
+  for (int j = 0; j < kBlocks; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int tr_row = l16 >> 2, tr_col = (l16 & 3) * 4;
+  if (steps) {
+    fetch_keys(0);
+    fetch(0);
+    fetch_keys(1);
+  }
+  for (int step = 0; step < steps; ++step) {
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) *reinterpret_cast<u32x4*>(Ks + k_row(piece_row[i]) + piece_col[i] * 16) = pre[i];
+#pragma unroll
+    for (int pl = 0; pl < 2; ++pl) *reinterpret_cast<u32x4*>(Ss + (pl * kStep + s_key) * kHeads + s_half * 8) = pre_s[pl];
+    __syncthreads();
+    fetch(step + 1);                                   // (behind the last: its keys again)
+    fetch_keys(step + 2);
+    bf16x8 ds[2];
+#pragma unroll
+    for (int pl = 0; pl < 2; ++pl) {
+      const unsigned short* src = Ss + (pl * kStep + 8 * kg + tr_row) * kHeads + tr_col;
+      ds[pl] = join(lds_tr16(src), lds_tr16(src + 4 * kHeads));
+    }
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j) {
+      const unsigned short* src = reinterpret_cast<const unsigned short*>(Ks + k_row(8 * kg + tr_row)) + j * 16 + tr_col;
+      const bf16x8 k = join(lds_tr16(src), lds_tr16(src + 4 * 160));
+      acc[j] = mm<F16>(k, ds[0], acc[j]);
+      acc[j] = mm<F16>(k, ds[1], acc[j]);
+    }
+    __syncthreads();
+  }
+  // acc[j][v]: channel 16 * j + 4 * kg + v of head l16
+#pragma unroll
+  for (int j = 0; j < kBlocks; ++j)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[j][v] *= PlaneScale<F16>::down;
+  const size_t base = (it.bs * p.H + it.h0) * (size_t)D + b0 * 16;
+  if (p.dq_dtype == CPPMEGA_MI355_F32) {
+    if (l16 >= it.nh) return;
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j)
+      if (j < blocks) *reinterpret_cast<f32x4*>((float*)p.dq + base + (size_t)l16 * D + j * 16 + 4 * kg) = acc[j];
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < kBlocks; ++j) {
+    const float v[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
+    *reinterpret_cast<uint2*>(Ks + l16 * 304 + j * 32 + kg * 8) = p.dq_dtype == CPPMEGA_MI355_F16 ? pack4<true>(v) : pack4<false>(v);
+  }
+  __syncthreads();
+  for (int e = lane; e < it.nh * (kBlocks * 2); e += 64) {
+    const int h = e / (kBlocks * 2), c = e - h * (kBlocks * 2);
+    if (c < blocks * 2)
+      *reinterpret_cast<u32x4*>((unsigned short*)p.dq + base + (size_t)h * D + c * 8) = *reinterpret_cast<const u32x4*>(Ks + h * 304 + c * 16);
+  }
+}
+
+// ---- dkv -----------------------------------------------------------------------------------------
+constexpr int kDkvThreads = 256;                       // a wavefront per band
+// A wavefront owns its band of the tile, so it adds with plain reads and writes: ds_add_f32 takes a lane at a time
+// (1160 us for a form of this kernel that took 280 with a plain write in its place).  16 bytes per lane of whole rows
+// meet in no bank.  Two wavefronts per band, 32 channels each, read the planes twice (110 us); one per 16 channels
+// of 600 keys, four times (315 us).
+template <bool F16>
+__global__ __launch_bounds__(kDkvThreads, 1) void bwd_dkv_kernel(const SplitParams p) {
+  extern __shared__ __align__(16) float tile[];        // [kDeadRow + 1][64], the last row for lanes of no key
+  const int tid = (int)threadIdx.x, lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // consecutive tiles read the same planes and rows: an XCD (launches go round them) takes a run of tiles
+  const int per_xcd = (int)gridDim.x / 8, work = (int)blockIdx.x % 8 * per_xcd + (int)blockIdx.x / 8;
+  const int cols = (p.D + 63) / 64, range = work % p.tiles, ch0 = work / p.tiles % cols * 64;
+  const int share = work / (p.tiles * cols) % p.shares, bg = work / (p.tiles * cols * p.shares);
+  if (bg >= p.B * p.G) return;
+  const int g = bg % p.G, b = bg / p.G;
+  const int k0 = range * kBands * p.band_keys, rows = min(kBands * p.band_keys, p.Skv - k0);
+  for (int e = tid; e < (kDeadRow + 1) * 16; e += kDkvThreads) reinterpret_cast<f32x4*>(tile)[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+
+  const int* all = p.band_steps + 2 + 2 * (bg * p.bands + range * kBands + wave);
+  const int groups = __builtin_amdgcn_readfirstlane(all[1]) / kAhead;
+  const int first = (int)((long long)groups * share / p.shares) * kAhead, n = (int)((long long)groups * (share + 1) / p.shares) * kAhead - first;
+  if (n > 0) {
+    const i32x4* steps = p.steps + __builtin_amdgcn_readfirstlane(all[0]) + first;
+    const unsigned plane_lane = ((unsigned)kg * p.stride + l16) * 16, lo_plane = (unsigned)p.stride * 64;
+    const unsigned qo_lane = lane * 16;
+    const char* rows_of = reinterpret_cast<const char*>(p.rows);
+    const char* by_channel = reinterpret_cast<const char*>(p.by_channel) + (size_t)ch0 * 64;
+    bf16x8 hi[kAhead], lo[kAhead], qo[kAhead][4];
+    i32x4 slot[kAhead];
+    int marked[kAhead], key_at[kAhead];
+    i32x4 cur = steps[min(lane, n - 1)], next = steps[min(64 + lane, n - 1)];
+    auto request = [&](int i, int at) {
+      const unsigned plane = __builtin_amdgcn_readlane(cur[0], at), row = __builtin_amdgcn_readlane(cur[1], at);
+      const unsigned operand = __builtin_amdgcn_readlane(cur[2], at);
+      marked[i] = row & 32;
+      key_at[i] = __builtin_amdgcn_readlane(cur[3], at);
+      const char *planes = p.planes + plane, *channels = by_channel + operand, *lo_planes = planes + lo_plane;
+      if (l16 < (int)(row & 31)) {                     // (the cache serves the lanes that ask)
+        hi[i] = *reinterpret_cast<const bf16x8*>(planes + plane_lane);
+        lo[i] = *reinterpret_cast<const bf16x8*>(lo_planes + plane_lane);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) qo[i][j] = *reinterpret_cast<const bf16x8*>(channels + qo_lane + j * 1024);
+      slot[i] = *reinterpret_cast<const i32x4*>(rows_of + (row & ~63u) + kg * 16);
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) request(i, i);
+    for (int step = 0; step < n; step += kAhead) {
+      const int ahead = step + kAhead;
+      if ((ahead & 63) == 0) {
+        cur = next;
+        next = steps[min(ahead + 64 + lane, n - 1)];
+      }
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        // keys 4 * kg + v, channels 4 * l16 + j
+        f32x4* at[4];
+        f32x4 was[4], add[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          at[v] = reinterpret_cast<f32x4*>(reinterpret_cast<char*>(tile) + slot[i][v] + l16 * 16);
+          was[v] = *at[v];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) add[j] = mm<F16>(hi[i], qo[i][j], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int j = 0; j < 4; ++j) add[j] = mm<F16>(lo[i], qo[i][j], add[j]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) *at[v] = was[v] + f32x4{add[0][v], add[1][v], add[2][v], add[3][v]};
+        if (marked[i]) {                               // (a list that names a key twice)
+          const int* keys = p.keys + key_at[i] / 4 + kg * 4;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int slot_of = keys[v], row = (slot_of & ~kAgain) - k0 - wave * p.band_keys;
+            const bool again = slot_of >= 0 && (slot_of & kAgain) && row >= 0 && row < p.band_keys;   // (not of a band behind)
+            for (int k = 0; k < 4; ++k)
+              if (again && kg == k) {
+                f32x4* once_more = reinterpret_cast<f32x4*>(tile + (row + wave * p.band_keys) * 64) + l16;
+                *once_more += f32x4{add[0][v], add[1][v], add[2][v], add[3][v]};
+              }
+          }
+        }
+        request(i, (ahead + i) & 63);
+      }
+    }
+  }
+  __syncthreads();
+  const bool whole = p.shares > 1;
+  float* out = (whole ? p.part + (size_t)share * p.B * p.Skv * p.G * p.D : p.dkv) + ((size_t)b * p.Skv + k0) * p.G * (size_t)p.D + (size_t)g * p.D + ch0;
+  const int quads = min(64, p.D - ch0) / 4;
+  for (int e = tid; e < rows * 16; e += kDkvThreads) {
+    const int row = e >> 4, c4 = e & 15;
+    if (c4 >= quads) continue;
+    f32x4 v = *reinterpret_cast<const f32x4*>(tile + row * 64 + c4 * 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] *= PlaneScale<F16>::down;
+    f32x4* dst = reinterpret_cast<f32x4*>(out + (size_t)row * p.G * p.D + c4 * 4);
+    if (!whole && p.accumulate) v += *dst;
+    *dst = v;
+  }
+}
+
+__global__ __launch_bounds__(kThreads) void bwd_sum_kernel(const SplitParams p) {
+  const size_t n = (size_t)p.B * p.Skv * p.G * p.D / 4, i = (size_t)blockIdx.x * kThreads + threadIdx.x;
+  if (i >= n) return;
+  f32x4* dst = reinterpret_cast<f32x4*>(p.dkv) + i;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  if (p.accumulate) v = *dst;
+  for (int z = 0; z < p.shares; ++z) v += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.part) + (size_t)z * n + i);
+  *dst = v;
+}
+
+struct Plan {
+  int chunks, stride, tiles, band_keys, shares, ns;
+  size_t keys, starts, step_starts, rows, band_steps, steps, list_steps, planes, by_channel, part, slab_bytes, bytes;
+};
+
+Plan make_plan(const cppmega_mi355_sparse_mla_bwd_args_t& a) {
+  Plan l;
+  l.chunks = (a.heads / a.kv_groups + kHeads - 1) / kHeads;
+  l.stride = (a.topk + 15) / 16 * 16 + 32;
+  l.tiles = (a.seq_kv + kBands * kBandKeys - 1) / (kBands * kBandKeys);
+  l.band_keys = (a.seq_kv + l.tiles * kBands - 1) / (l.tiles * kBands);
+  const size_t lists = (size_t)a.batch * a.kv_groups, bands = (size_t)l.tiles * kBands;      // lists per query position
+  l.list_steps = a.topk / 16 + std::min<size_t>((size_t)a.topk, bands) + 1;
+  const size_t per_s = lists * (l.stride * 4 + (2 * bands + 2) * 4 + l.list_steps * (64 + 16 * l.chunks) + l.chunks * ((size_t)l.stride * kRowBytes + (size_t)(a.d_qk + 63) / 64 * 4096));
+  l.ns = (int)std::min<size_t>((size_t)a.seq_q, std::max<size_t>(kSlabBytes / per_s, 1));
+  // a tile of dkv has a CU to itself: as many shares of the steps as bring the tiles to the number of CUs, of eight at least
+  const long long tiles = (long long)l.tiles * ((a.d_qk + 63) / 64) * lists;
+  l.shares = (int)std::max<long long>(1, std::min<long long>(256 / tiles, (long long)l.ns * l.chunks * (a.topk / (bands * 16) + 1) / 8));
+  size_t at = 0;
+  auto take = [&](size_t bytes) { const size_t here = at; at += (bytes + 255) & ~(size_t)255; return here; };
+  l.keys = take(lists * l.ns * l.stride * 4);
+  l.starts = take(lists * l.ns * (bands + 2) * 4);
+  l.band_steps = take((2 + lists * bands * 2) * 4);
+  l.step_starts = take(lists * l.ns * bands * 4);
+  l.rows = take((lists * l.ns * l.list_steps + 1) * 64);
+  l.steps = take((lists * l.ns * l.list_steps * l.chunks + lists * bands * kAhead) * 16);
+  l.planes = take(lists * l.ns * l.chunks * l.stride * kRowBytes);
+  l.by_channel = take(lists * l.ns * l.chunks * ((a.d_qk + 63) / 64) * 4096);
+  l.slab_bytes = at;
+  l.part = take(l.shares > 1 ? (size_t)l.shares * a.batch * a.seq_kv * a.kv_groups * a.d_qk * 4 : 0);
+  l.bytes = at;
+  return l;
+}
+
+template <bool F16>
+int run(SplitParams p, const Plan& l, bool clear, hipStream_t stream) {
+  auto scores_lds = [&](int waves) { return (size_t)2 * kHeads * (p.D + 8 + p.d_v + 8) + waves * (kHeads * 3 * 4 + 1024); };
+  const size_t dkv_lds = (size_t)(kDeadRow + 1) * 64 * 4;
+  const int dq_parts = (p.D / 16 + kBlocks - 1) / kBlocks;
+  CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_kernel<F16, 8, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scores_lds(8)));
+  CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_kernel<F16, 16, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scores_lds(16)));
+  CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_dkv_kernel<F16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dkv_lds));
+  for (p.s0 = 0; p.s0 < p.S; p.s0 += l.ns) {
+    p.ns = std::min(l.ns, p.S - p.s0);
+    p.shares = l.shares;
+    p.accumulate = p.s0 > 0 || !clear;
+    const size_t lists = (size_t)p.B * p.ns * p.G, items = lists * p.chunks;
+    hipLaunchKernelGGL(bwd_lists_kernel, dim3((unsigned)lists), dim3(kThreads), (size_t)(3 * p.bands + 2 * p.topk + 2) * 4, stream, p);
+    hipLaunchKernelGGL(bwd_steps_kernel, dim3((unsigned)(p.B * p.G * p.bands)), dim3(kStepThreads), 0, stream, p);
+    const dim3 of_items((unsigned)items);
+    if (p.topk <= 16 * 4 * 4) hipLaunchKernelGGL((bwd_scores_kernel<F16, 4, 4>), of_items, dim3(256), scores_lds(4), stream, p);
+    else if (p.topk <= 16 * 8 * 4) hipLaunchKernelGGL((bwd_scores_kernel<F16, 8, 4>), of_items, dim3(512), scores_lds(8), stream, p);
+    else hipLaunchKernelGGL((bwd_scores_kernel<F16, 16, 8>), of_items, dim3(1024), scores_lds(16), stream, p);
+    hipLaunchKernelGGL(bwd_dq_kernel<F16>, dim3((unsigned)(items * dq_parts)), dim3(64), 0, stream, p);
+    const dim3 tiles((unsigned)((p.tiles * ((p.D + 63) / 64) * p.shares * p.B * p.G + 7) / 8 * 8));
+    hipLaunchKernelGGL(bwd_dkv_kernel<F16>, tiles, dim3(kDkvThreads), dkv_lds, stream, p);
+    if (p.shares > 1) {
+      const size_t n = (size_t)p.B * p.Skv * p.G * p.D / 4;
+      hipLaunchKernelGGL(bwd_sum_kernel, dim3((unsigned)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, stream, p);
+    }
+    CM_HIP_CHECK(hipGetLastError());
+  }
+  return 0;
+}
+
+}  // namespace
+
+bool sparse_mla_bwd_split_supports(const cppmega_mi355_sparse_mla_bwd_args_t& a) {
+  const bool half = (a.q_dtype == CPPMEGA_MI355_BF16 || a.q_dtype == CPPMEGA_MI355_F16) && a.kv_dtype == a.q_dtype && a.d_out_dtype == a.q_dtype;
+  if (!half || a.d_qk % 32 != 0 || a.d_v % 32 != 0 || a.d_qk > kBlocks * 64 || a.topk < 1 || a.topk > 2048) return false;
+  if (a.batch < 1 || a.seq_q < 1 || a.seq_kv < 1 || a.seq_kv > 64 * 1024 || (long long)a.batch * a.kv_groups > 65535) return false;
+  // A step costs the same for one key of a band as for sixteen.  Measured at 64 .. 1024 queries against
+  // sparse_mla_bwd_mfma.hip: with 16 heads it is as fast at one key per band (1.1 .. 1.3x) and 3.5x faster at nine;
+  // with more heads, which that kernel adds up before its atomics, the line is at two to three (32 heads 0.8x at one
+  // key, 1.06x at two; 128 heads 0.9x at two, 1.3x at five).
+  const long long bands = ((long long)a.seq_kv + kBandKeys - 1) / kBandKeys;
+  if (bands * (a.heads / a.kv_groups > kHeads ? 3 : 1) > a.topk) return false;
+  if ((long long)a.batch * a.seq_q * a.heads * ((a.d_qk + 143) / 144) > 0x7fffffffLL) return false;
+  return make_plan(a).slab_bytes < 0x7fffffffu;        // (offsets into a slab are 32 bits)
+}
+
+size_t sparse_mla_bwd_split_workspace_bytes(const cppmega_mi355_sparse_mla_bwd_args_t& a) { return make_plan(a).bytes; }
+
+// dkv is written, or added to when clear_dkv is off: no clearing kernel in front.
+int sparse_mla_bwd_split_launch(const cppmega_mi355_sparse_mla_bwd_args_t& a, hipStream_t stream) {
+  const Plan l = make_plan(a);
+  char* ws = static_cast<char*>(a.workspace);
+  SplitParams p;
+  p.q = static_cast<const unsigned short*>(a.q); p.kv = static_cast<const unsigned short*>(a.kv);
+  p.d_out = static_cast<const unsigned short*>(a.d_out);
+  p.indices = a.indices; p.sm_scale_dev = a.sm_scale_dev; p.dq = a.dq; p.dkv = a.dkv;
+  p.keys = reinterpret_cast<int*>(ws + l.keys); p.starts = reinterpret_cast<int*>(ws + l.starts);
+  p.band_steps = reinterpret_cast<int*>(ws + l.band_steps); p.steps = reinterpret_cast<i32x4*>(ws + l.steps);
+  p.step_starts = reinterpret_cast<int*>(ws + l.step_starts); p.rows = reinterpret_cast<int*>(ws + l.rows);
+  p.list_steps = (int)l.list_steps; p.dead_step = (unsigned)((size_t)a.batch * a.kv_groups * l.ns * l.list_steps * 64);
+  p.planes = ws + l.planes; p.by_channel = reinterpret_cast<unsigned short*>(ws + l.by_channel);
+  p.part = reinterpret_cast<float*>(ws + l.part);
+  p.dq_dtype = a.dq_dtype; p.index_dtype = a.index_dtype;
+  p.B = a.batch; p.S = a.seq_q; p.H = a.heads; p.G = a.kv_groups; p.Skv = a.seq_kv; p.topk = a.topk; p.D = a.d_qk; p.d_v = a.d_v;
+  p.channels = (a.d_qk + 63) / 64 * 64;
+  p.chunks = l.chunks; p.stride = l.stride; p.tiles = l.tiles; p.bands = l.tiles * kBands; p.band_keys = l.band_keys;
+  p.sm_scale = a.sm_scale;
+  return a.q_dtype == CPPMEGA_MI355_F16 ? run<true>(p, l, a.clear_dkv != 0, stream) : run<false>(p, l, a.clear_dkv != 0, stream);
+}
+
+}  // namespace cm

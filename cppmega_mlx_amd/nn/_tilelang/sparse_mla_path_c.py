@@ -143,9 +143,14 @@ def sparse_mla_path_c_apply(
 
 def _sparse_mla_bwd_path_c_direct(q: torch.Tensor, kv: torch.Tensor, d_out: torch.Tensor, indices: torch.Tensor, *,
                                   sm_scale_buf: torch.Tensor, d_v: int | None = None) -> tuple[torch.Tensor, torch.Tensor]:
-    """Backward into fresh owner outputs: ``dq`` in q's dtype, ``dkv`` float32 (cleared, then
-    accumulated with atomic adds).  The reference requires fp16 carriers; any of float32 /
-    float16 / bfloat16 is taken here, all three operands alike."""
+    """Backward into fresh owner outputs: ``dq`` in q's dtype, ``dkv`` float32.  The reference
+    requires fp16 carriers; any of float32 / float16 / bfloat16 is taken here, all three operands
+    alike."""
+    return _backward(q, kv, d_out, indices, None if isinstance(sm_scale_buf, float) else sm_scale_buf, d_v)
+
+
+def _backward(q, kv, d_out, indices, sm_scale: torch.Tensor | float, d_v: int | None) -> tuple[torch.Tensor, torch.Tensor]:
+    # (a number goes with the call: a buffer made for it would be a copy that the host waits for)
     status = sparse_mla_path_c_status()
     if not status.available:
         raise SparseMLAPathCDirectError(status.reason)
@@ -154,12 +159,12 @@ def _sparse_mla_bwd_path_c_direct(q: torch.Tensor, kv: torch.Tensor, d_out: torc
     if d_out.dtype != q.dtype or kv.dtype != q.dtype:
         raise SparseMLAPathCDirectError("Sparse-MLA backward takes q, kv and d_out in one carrier dtype without hidden casts; got "
                                         f"q={q.dtype}, kv={kv.dtype}, d_out={d_out.dtype}")
-    if not isinstance(sm_scale_buf, torch.Tensor) or tuple(sm_scale_buf.shape) != (1,) or sm_scale_buf.dtype != torch.float32:
+    if not isinstance(sm_scale, float) and (not isinstance(sm_scale, torch.Tensor) or tuple(sm_scale.shape) != (1,) or sm_scale.dtype != torch.float32):
         raise SparseMLAPathCDirectError("Sparse-MLA backward requires sm_scale_buf with shape (1,) and dtype torch.float32")
     dq = torch.empty_like(q)
     dkv = torch.empty(tuple(kv.shape), dtype=torch.float32, device=kv.device)
     try:
-        ops.sparse_mla_backward(q.contiguous(), kv.contiguous(), d_out.contiguous(), indices.contiguous(), sm_scale=sm_scale_buf,
+        ops.sparse_mla_backward(q.contiguous(), kv.contiguous(), d_out.contiguous(), indices.contiguous(), sm_scale=sm_scale,
                                 d_v=shapes.d_v, dq=dq, dkv=dkv, clear_dkv=True)
     except (_lib.NativeCallError, _lib.NativeLibraryError) as exc:
         raise SparseMLAPathCDirectError(f"sparse-MLA backward dispatch failed: {type(exc).__name__}: {exc}") from exc
@@ -173,9 +178,8 @@ def sparse_mla_bwd_path_c(q: torch.Tensor, kv: torch.Tensor, d_out: torch.Tensor
         return None
     shapes = _resolve_shapes(q, kv, indices, d_v=d_v)
     scale = shapes.qk_dim ** -0.5 if sm_scale is None else float(sm_scale)
-    buf = torch.tensor([scale], dtype=torch.float32, device=q.device)
     try:
-        return _sparse_mla_bwd_path_c_direct(q, kv, d_out, indices, sm_scale_buf=buf, d_v=shapes.d_v)
+        return _backward(q, kv, d_out, indices, scale, shapes.d_v)
     except SparseMLAPathCDirectError:
         return None
 
@@ -192,8 +196,7 @@ class _SparseMLAPathCFunction(torch.autograd.Function):
         q, kv, indices = ctx.saved_tensors
         # (the direct form: a carrier or shape error surfaces as what it is instead of as "unavailable")
         shapes = _resolve_shapes(q, kv, indices, d_v=None)
-        buf = torch.tensor([shapes.qk_dim ** -0.5], dtype=torch.float32, device=q.device)
-        dq, dkv = _sparse_mla_bwd_path_c_direct(q, kv, cotangent.to(q.dtype).contiguous(), indices, sm_scale_buf=buf, d_v=shapes.d_v)
+        dq, dkv = _backward(q, kv, cotangent.to(q.dtype).contiguous(), indices, shapes.qk_dim ** -0.5, shapes.d_v)
         return dq, dkv.to(kv.dtype), None
 
 

@@ -540,8 +540,15 @@ def sparse_mla_backward(q: torch.Tensor, kv: torch.Tensor, d_out: torch.Tensor, 
     else:
         a.sm_scale = float(sm_scale)
     a.clear_dkv = 1 if clear_dkv else 0
+    lib = _lib.load()
+    stream = _lib.current_stream(q.device)
+    need = C.c_size_t(0)
+    _lib.check(lib.cppmega_mi355_sparse_mla_bwd_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)), "sparse_mla_bwd")
+    if need.value:
+        workspace = _workspace(q.device, need.value, stream)
+        a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel()
     with torch.cuda.device(q.device):
-        rc = _lib.load().cppmega_mi355_sparse_mla_bwd(C.byref(a), C.sizeof(a), _lib.current_stream(q.device))
+        rc = lib.cppmega_mi355_sparse_mla_bwd(C.byref(a), C.sizeof(a), stream)
     _lib.check(rc, "sparse_mla_bwd")
     return dq, dkv
 

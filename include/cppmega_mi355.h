@@ -335,8 +335,15 @@ typedef struct cppmega_mi355_sparse_mla_bwd_args {
   float* dkv;
   const float* q_scale;       /* e4m3 q only */
   const float* kv_scale;      /* e4m3 kv only */
+  /* Optional (callers built against the first layout end here): with *_workspace_bytes of scratch the additions
+   * into dkv happen on chip, the same result faster. */
+  void* workspace;
+  size_t workspace_bytes;
 } cppmega_mi355_sparse_mla_bwd_args_t;
+#define CPPMEGA_MI355_SPARSE_MLA_BWD_ARGS_V1_SIZE (offsetof(cppmega_mi355_sparse_mla_bwd_args_t, workspace))
 
+/* 0: no kernel takes a workspace for this request */
+int cppmega_mi355_sparse_mla_bwd_workspace_bytes(const cppmega_mi355_sparse_mla_bwd_args_t* args, size_t args_size, size_t* bytes);
 int cppmega_mi355_sparse_mla_bwd(const cppmega_mi355_sparse_mla_bwd_args_t* args, size_t args_size, void* stream);
 
 /* ---- DSA indexer KL loss, per position ---------------------------------------------

@@ -306,3 +306,47 @@ def test_training_entry_points_replay_from_a_hip_graph(device):
         assert err <= 1e-4 * ref
     want_loss = dsa_splitk_indexer_loss_per_position(lidx, ltop, lq, lk, 0.125, True)
     assert torch.equal(captured["loss"], want_loss)
+
+
+@pytest.mark.parametrize("shape", [
+    dict(B=1, S=5, H=16, G=1, Skv=600, topk=17, D=96, d_v=64),         # one full tile of dkv, half a tile of channels
+    dict(B=1, S=3, H=20, G=1, Skv=601, topk=257, D=576, d_v=512),      # two tiles, a chunk of 4 heads, eight wavefronts of scores
+    dict(B=2, S=3, H=16, G=2, Skv=16, topk=64, D=64, d_v=64),          # bands of one key, keys named again and again
+    dict(B=1, S=2, H=8, G=1, Skv=1300, topk=1030, D=160, d_v=32),      # sixteen wavefronts, three tiles
+], ids=lambda c: "B%dS%dH%dG%dT%dk%dD%ddv%d" % tuple(c.values()))
+@pytest.mark.parametrize("carrier", [torch.bfloat16, torch.float16])
+def test_backward_over_a_workspace(device, shape, carrier):
+    B, S, H, G, Skv, topk, D, d_v = shape.values()
+    rng = np.random.default_rng(topk)
+    q, kv, d_out = (to_dev(rng.standard_normal(s).astype(np.float32), device).to(carrier) for s in ((B, S, H, D), (B, Skv, G, D), (B, S, H, d_v)))
+    idx = sparse_indices(rng, B, S, G, Skv, topk, replace=True)
+    idx[rng.random(idx.shape) < 0.1] = -1
+    idx[0, 1] = -1
+    want_dq, want_dkv = om.sparse_mla_bwd_oracle(q.double().cpu().numpy(), kv.double().cpu().numpy(), idx, d_out.double().cpu().numpy(),
+                                                 sm_scale=D ** -0.5, d_v=d_v)
+    runs = []
+    for _ in range(2):
+        dq, dkv = torch.full((B, S, H, D), 9.0, device=device), torch.full((B, Skv, G, D), 9.0, device=device)
+        ops.sparse_mla_backward(q, kv, d_out, to_dev(idx.astype(np.int32), device), sm_scale=D ** -0.5, d_v=d_v, dq=dq, dkv=dkv)
+        runs.append((dq, dkv))
+    for got, want in zip(runs[0], (want_dq, want_dkv)):
+        err, ref = error_report(got.cpu().numpy(), want)
+        assert err <= 1e-4 * ref, (err, ref)
+    assert torch.equal(runs[0][0], runs[1][0]) and torch.equal(runs[0][1], runs[1][1])   # (atomics would differ now and then)
+
+
+def test_backward_in_several_slabs_matches_its_halves(device):
+    S, H, Skv, topk, D = 1200, 16, 1100, 1024, 64
+    gen = torch.Generator(device=device).manual_seed(3)
+    q, d_out = (torch.randn(1, S, H, D, generator=gen, device=device).bfloat16() for _ in range(2))
+    kv = torch.randn(1, Skv, 1, D, generator=gen, device=device).bfloat16()
+    idx = torch.rand(S, Skv, generator=gen, device=device).topk(topk, dim=1).indices.int().view(1, S, 1, topk)
+    dq, dkv = ops.sparse_mla_backward(q, kv, d_out, idx, sm_scale=0.1, d_v=D, dq=torch.empty_like(q), dkv=torch.empty(kv.shape, device=device))
+    want_dq, want_dkv = torch.empty_like(q), torch.empty(kv.shape, device=device)
+    for part, half in enumerate((slice(0, 500), slice(500, S))):
+        out = torch.empty_like(q[:, half])
+        ops.sparse_mla_backward(q[:, half].contiguous(), kv, d_out[:, half].contiguous(), idx[:, half].contiguous(), sm_scale=0.1, d_v=D,
+                                dq=out, dkv=want_dkv, clear_dkv=part == 0)
+        want_dq[:, half] = out
+    assert torch.equal(dq, want_dq)
+    assert (dkv - want_dkv).abs().max() <= 1e-5 * want_dkv.abs().max()
