@@ -1,9 +1,16 @@
 // Sparse MLA forward over an FP8 latent KV cache on the matrix cores (gfx950), with the
 // wavefronts of a workgroup split into score producers and value consumers.
 //
-// Shapes served: bf16 queries of 576 = 512 latent + 64 rope channels, d_v = 512, keys as e4m3
-// latent [512] with fp32 scales (per 128 / 256 / 512 channels, per row, or none) plus a bf16
-// rope tail [64]; more than 32 heads per KV group.
+// Shapes served, all with d_v = 512:
+//   bf16 queries of 576 = 512 latent + 64 rope channels, keys as e4m3 latent [512] with fp32 scales
+//   (per 128 / 256 / 512 channels, per row, or none) plus a bf16 rope tail [64];
+//   queries and key rows of 576 e4m3 codes with one fp32 scale per (query, head) and per row.
+//
+// Measured against the kernel of sparse_mla_mfma.hip that has the whole tile loop in every wavefront:
+//   code rows, 128 heads x 999 queries x 2048 keys: 1013 -> 445 us (the scores are e4m3 products: the
+//   same work in bf16 at the rate of a large matrix product is 458 us); 64 heads x 1 query x 2048: 58 -> 18 us;
+//   16 heads (three quarters of the chunk idle): latent rows 1 x 2048 of 8192 39 -> 17 us, 2000 x 2048 998 -> 563 us,
+//   code rows 1000 x 2048 443 -> 212 us.  No shape tried (16 .. 128 heads, 1 .. 2000 queries, 256 .. 2048 keys) was slower.
 //
 // Workgroup = (query, KV group, chunk of 64 heads, key split), 8 wavefronts, key tiles of 32
 // rows in a ring of five LDS slots filled by the load unit (global_load_lds) three tiles ahead.
@@ -26,8 +33,8 @@
 //   pipeline  iteration t: barrier; producers: scores and P of tile t+1; consumers: issue tile
 //             t+4, value product of tile t.  One barrier per tile.
 //
-// Key splits write their accumulators (rounded to bf16) to the workspace as the lanes hold them
-// plus (max, sum) per head; sparse_mla_latent_combine_kernel merges them and does the transposition
+// Key splits write their accumulators (rounded to bf16; in fp32 for code rows and for up to 32 heads) to the
+// workspace as the lanes hold them plus (max, sum) per head; sparse_mla_latent_combine_kernel merges them and does the transposition
 // to [head][channel] that the single-split path does in LDS.
 
 #include <type_traits>
@@ -173,8 +180,14 @@ __device__ __forceinline__ float max_rows(float v) {
   return vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-// NBLK: fp32 scales per key row (1, 2 or 4)
-template <int NBLK>
+// Key splits of these keep float32: code rows and single groups of heads have few enough of them.
+__host__ __device__ __forceinline__ bool f32_partials(const MlaParams& p) { return p.q_dtype == CPPMEGA_MI355_E4M3 || p.heads_per_group <= 32; }
+
+// NBLK: fp32 scales per key row (1, 2 or 4).
+// ROWS: key rows and queries of 576 e4m3 codes with one fp32 scale each (NBLK = 1).  The query's codes are the
+// second operand as they are, one plane of them; the tail of 64 codes is two products of 32; a head's query
+// scale joins the softmax scale and a key's scale multiplies the whole sum.
+template <int NBLK, bool ROWS>
 __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = (int)threadIdx.x, lane = tid & 63;
@@ -182,6 +195,8 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   const bool producer = wave < 4;
   const int role = wave & 3;                    // producer p / consumer c
   constexpr int nblk = NBLK;
+  static_assert(!ROWS || NBLK == 1, "one scale per row");
+  constexpr int kRowPitch = ROWS ? kDqk : kLat;     // bytes of a key row in the cache
 
   // ---- which (query, KV group, head chunk, split).  Workgroup ids that are equal modulo 8 run on
   //      the same XCD and share its L2: every workgroup of one (query, KV group) gets such ids, so
@@ -313,42 +328,61 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     // order through the ring slot 1 + role, which holds no tile before the first barrier of the
     // pipeline (rows padded by 16 bytes: the 16 lanes of an operand read fall on distinct banks).
     typedef __attribute__((ext_vector_type(4))) unsigned u4;
-    constexpr int kQPieces = kDqk / 8;              // 72 pieces of 16 bytes per head row
-    constexpr int kQPitch = kDqk * 2 + 16;          // 1168
+    constexpr int kQRow = ROWS ? kDqk : kDqk * 2;   // bytes of a head row
+    constexpr int kQPieces = kQRow / 16;            // pieces of 16 bytes per head row
+    constexpr int kQPitch = kQRow + 16;
+    constexpr int kQLoads = 16 * kQPieces / 64;
     static_assert(16 * kQPitch <= kLatBytes + kRopeBytes, "the query rows fit a slot without touching its scale area");
-    u4 qload[18];
+    u4 qload[kQLoads];
 #pragma unroll
-    for (int t = 0; t < 18; ++t) {
+    for (int t = 0; t < kQLoads; ++t) {
       const int P = lane + 64 * t, hl = P / kQPieces, piece = P - hl * kQPieces;
       const int h = 16 * role + hl;
       // heads past the end of the group repeat head 0: their columns stay finite and are never stored
-      qload[t] = *reinterpret_cast<const u4*>((const unsigned short*)p.q + (bs * p.H + head0 + (h < heads_here ? h : 0)) * (size_t)kDqk + 8 * piece);
+      qload[t] = *reinterpret_cast<const u4*>((const unsigned char*)p.q + (bs * p.H + head0 + (h < heads_here ? h : 0)) * (size_t)kQRow + 16 * piece);
     }
+    float q_scale = 1.0f;                           // of head n
+    if (ROWS) q_scale = ((const float*)p.q_scale)[bs * p.H + head0 + (16 * role + n < heads_here ? 16 * role + n : 0)];
     __builtin_amdgcn_sched_barrier(0);
     stage_keys();
     unsigned char* qstage = smem + (1 + role) * kSlotBytes;
 #pragma unroll
-    for (int t = 0; t < 18; ++t) {
+    for (int t = 0; t < kQLoads; ++t) {
       const int P = lane + 64 * t, hl = P / kQPieces, piece = P - hl * kQPieces;
       *reinterpret_cast<u4*>(qstage + hl * kQPitch + piece * 16) = qload[t];
     }
     uint4 qraw[4][4];
     bf16x8 qr[2];
+    i32x8 qh[4], ql[4];
+    unsigned long long qt[2];                       // ROWS: the tail, codes 512 + 16 kg .. + 7 and + 8 .. + 15
+    if (ROWS) {
 #pragma unroll
-    for (int blk = 0; blk < 4; ++blk)
+      for (int blk = 0; blk < 4; ++blk) {
+        const uint4 c0 = *reinterpret_cast<const uint4*>(qstage + n * kQPitch + 128 * blk + 32 * kg);
+        const uint4 c1 = *reinterpret_cast<const uint4*>(qstage + n * kQPitch + 128 * blk + 32 * kg + 16);
+        qh[blk] = i32x8{(int)c0.x, (int)c0.y, (int)c0.z, (int)c0.w, (int)c1.x, (int)c1.y, (int)c1.z, (int)c1.w};
+      }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) qraw[blk][j] = *reinterpret_cast<const uint4*>(qstage + n * kQPitch + (16 * blk + 4 * kg + j) * 16);
+      for (int r = 0; r < 2; ++r) qt[r] = *reinterpret_cast<const unsigned long long*>(qstage + n * kQPitch + kLat + 16 * kg + 8 * r);
+    } else {
 #pragma unroll
-    for (int r = 0; r < 2; ++r) qr[r] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qstage + n * kQPitch + (64 + 4 * r + kg) * 16));
+      for (int blk = 0; blk < 4; ++blk)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) qraw[blk][j] = *reinterpret_cast<const uint4*>(qstage + n * kQPitch + (16 * blk + 4 * kg + j) * 16);
+#pragma unroll
+      for (int r = 0; r < 2; ++r) qr[r] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qstage + n * kQPitch + (64 + 4 * r + kg) * 16));
+    }
     __syncthreads();                                // keys[] is complete
     const int n_tiles = count_tiles();
-    i32x8 qh[4], ql[4];
     int qexp = 0;
+    if (!ROWS)
 #pragma unroll
-    for (int blk = 0; blk < 4; ++blk) qexp |= split_q32(qraw[blk], qh[blk], ql[blk]) << (8 * blk);
+      for (int blk = 0; blk < 4; ++blk) qexp |= split_q32(qraw[blk], qh[blk], ql[blk]) << (8 * blk);
     float m_run = -INFINITY;                      // base-2 running reference of head n
     float l_run = 0.0f;                           // this lane's share of its denominator
-    const float qk_scale = sm_scale * kLog2e;
+    const float qk_scale = sm_scale * kLog2e * q_scale;
+    // (the plain path takes maxima before scaling)
+    const bool positive = !ROWS || __ballot(!(q_scale > 0.0f)) == 0ull;
 
     // K operands of a tile -> registers: per sub-tile four 32-byte block fragments and two rope
     // fragments.  The first sub-tile is requested one tile ahead, right after the previous tile's
@@ -356,6 +390,7 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     // the first one's products.
     i32x8 kf[2][4];
     bf16x8 rf[2][2];
+    unsigned long long tf[2][2];                    // ROWS: the tails
     // (a tile's slot is passed as its byte offset into the ring, a running value: one address
     // register per slot then reaches every operand of the tile with an immediate offset)
     auto load_k = [&](unsigned slot_off, int sj) {
@@ -369,8 +404,15 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
         const uint4 c1 = *reinterpret_cast<const uint4*>(lat + blk * kPair + kPlane);
         kf[sj][blk] = i32x8{(int)c0.x, (int)c0.y, (int)c0.z, (int)c0.w, (int)c1.x, (int)c1.y, (int)c1.z, (int)c1.w};
       }
-      rf[sj][0] = *reinterpret_cast<const bf16x8*>(rope);
-      rf[sj][1] = *reinterpret_cast<const bf16x8*>(rope + 1024);
+      if (ROWS) {
+        typedef __attribute__((ext_vector_type(2))) unsigned long long u64x2;
+        const u64x2 c = *reinterpret_cast<const u64x2*>(slot + kLatBytes + sj * 1024);
+        tf[sj][0] = c[0];
+        tf[sj][1] = c[1];
+      } else {
+        rf[sj][0] = *reinterpret_cast<const bf16x8*>(rope);
+        rf[sj][1] = *reinterpret_cast<const bf16x8*>(rope + 1024);
+      }
     };
     constexpr int kOne = 0x7f7f7f7f;                // operand exponent bytes of 2^0: the key bytes enter the products unscaled
 
@@ -383,7 +425,7 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
       const unsigned char* slot = smem + slot_off;
       const int spar = tau & 1;
       const float* scl_base = reinterpret_cast<const float*>(slot + kLatBytes + kRopeBytes);
-      const bool all_valid = tvalid[tau] != 0;      // (uniform) no skipped key in this tile
+      const bool all_valid = tvalid[tau] != 0 && positive;      // (uniform) no skipped key in this tile
       // "no head of this tile moves its reference": written first, so that the common tile ends
       // without an LDS write the barrier would have to wait for
       if (lane == 0) flagbuf[spar * 4 + role] = 0;
@@ -416,6 +458,18 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
       f32x4 st[2];
       auto subtile = [&](auto sj_c, const float (&ksc)[4][nblk]) {
         constexpr int sj = decltype(sj_c)::value;
+        if constexpr (ROWS) {                        // one scale for the whole row: two running sums, then the scale
+          f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
+          mfma_s8<0>(a0, kf[sj][0], qh[0], kOne, kOne);
+          mfma_s8<0>(a1, kf[sj][1], qh[1], kOne, kOne);
+          mfma_s8<0>(a0, kf[sj][2], qh[2], kOne, kOne);
+          mfma_s8<0>(a1, kf[sj][3], qh[3], kOne, kOne);
+          a0 = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)tf[sj][0], (long)qt[0], a0, 0, 0, 0);
+          a1 = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)tf[sj][1], (long)qt[1], a1, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) st[sj][i] = ksc[i][0] * (a0[i] + a1[i]);
+          return;
+        }
         st[sj] = f32x4{0.f, 0.f, 0.f, 0.f};
         mfma_s(st[sj], rf[sj][0], qr[0]);
         mfma_s(st[sj], rf[sj][1], qr[1]);
@@ -537,21 +591,28 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   stage_keys();
   __syncthreads();                                // keys[] is complete
   const int n_tiles = count_tiles();
-  // HBM -> LDS.  A skipped key fetches cache row 0 instead (its probability is zero), so every
+  int spare_row = 0;
+  if (ROWS && n_tiles > 0) {
+    int m = -1;
+    for (int w = 0; w < 8; ++w) m = max(m, last_valid[w]);
+    spare_row = __builtin_amdgcn_readfirstlane(keys[m]);
+  }
+  // HBM -> LDS.  A skipped key fetches cache row 0 (ROWS: its list's last valid row) instead (its probability is zero), so every
   // tile is the same six load instructions per wavefront and the in-order load counter can be
   // waited on by count.  The loads are inline assembly (the compiler would otherwise order every
   // later LDS read behind them) with a uniform 64-bit base and a 32-bit byte offset per lane:
   //   latent : block c of both sub-tiles, two planes each: lane (n, kg) of plane j fetches bytes
   //            128 c + 32 kg + 16 j .. + 15 of key 16 sj + n
   //   rope   : plane (sj = c / 2, s = c % 2): lane (n, kq) fetches bytes 64 s + 16 kq .. + 15 of the rope row
+  //            (ROWS: half c % 2 of the plane of sub-tile c / 2: bytes 512 + 16 kq .. + 15 of the row)
   //   scales : elements 8 nblk c .. 8 nblk (c + 1) - 1 of [32 rows][nblk], one per lane (without
   //            scales in memory: a word nobody reads, so that the count stays six)
   const size_t group_row0 = ((size_t)b * p.Skv_pitch) * p.G + g;     // cache row of key 0; key k is G rows further per step
-  const unsigned char* lat_base = (const unsigned char*)p.kv + group_row0 * kLat;
-  const unsigned char* rope_base = (const unsigned char*)p.rope + group_row0 * (kRope * 2);
+  const unsigned char* lat_base = (const unsigned char*)p.kv + group_row0 * kRowPitch;
+  const unsigned char* rope_base = ROWS ? lat_base + kLat : (const unsigned char*)p.rope + group_row0 * (kRope * 2);
   const unsigned char* sc_base = has_scale ? (const unsigned char*)p.kv_scale + group_row0 * nblk * 4 : (const unsigned char*)p.kv;
-  const unsigned lat_step = (unsigned)p.G * kLat, rope_step = (unsigned)p.G * (kRope * 2), sc_step = has_scale ? (unsigned)p.G * nblk * 4 : 0u;
-  const unsigned lat_lane = 128u * role + 32u * (lane >> 4), rope_lane = 64u * (role & 1) + 16u * (lane >> 4);
+  const unsigned lat_step = (unsigned)p.G * kRowPitch, rope_step = ROWS ? lat_step : (unsigned)p.G * (kRope * 2), sc_step = has_scale ? (unsigned)p.G * nblk * 4 : 0u;
+  const unsigned lat_lane = 128u * role + 32u * (lane >> 4), rope_lane = (ROWS ? 0u : 64u * (role & 1)) + 16u * (lane >> 4);
   const int sc_elem = 8 * nblk * role + lane;                         // (lanes below 8 nblk)
   const unsigned sc_lane = has_scale ? 4u * (unsigned)(sc_elem % nblk) : 0u;
   const int sc_row = min(sc_elem / nblk, kTK - 1);
@@ -572,8 +633,9 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   auto dma_prepare = [&](int tau, unsigned slot_off) {
     dma_slot = smem_base + slot_off;
     const int* tk = keys + tau * kTK;
-    const unsigned k0 = (unsigned)max(tk[lane & 15], 0), k1 = (unsigned)max(tk[16 + (lane & 15)], 0);   // this lane's key of sub-tile 0 / 1
-    const unsigned ks = (unsigned)max(tk[sc_row], 0);
+    auto fetched = [&](int k) { return (unsigned)(ROWS ? (k >= 0 ? k : spare_row) : max(k, 0)); };
+    const unsigned k0 = fetched(tk[lane & 15]), k1 = fetched(tk[16 + (lane & 15)]);   // this lane's key of sub-tile 0 / 1
+    const unsigned ks = fetched(tk[sc_row]);
     off_l0 = __umul24(k0, lat_step) + lat_lane;
     off_l1 = __umul24(k1, lat_step) + lat_lane;
     off_r = __umul24((role >> 1) ? k1 : k0, rope_step) + rope_lane;
@@ -584,7 +646,9 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     else if (i == 1) dma16(lat_base, off_l0 + 16u, dma_slot + role * kPair + kPlane);
     else if (i == 2) dma16(lat_base, off_l1, dma_slot + (4 + role) * kPair);
     else if (i == 3) dma16(lat_base, off_l1 + 16u, dma_slot + (4 + role) * kPair + kPlane);
-    else if (i == 4) dma16(rope_base, off_r, dma_slot + kLatBytes + role * 1024);
+    else if (i == 4 && ROWS) {
+      if ((lane >> 5) == (role & 1)) dma16(rope_base, off_r, dma_slot + kLatBytes + (role >> 1) * 1024);
+    } else if (i == 4) dma16(rope_base, off_r, dma_slot + kLatBytes + role * 1024);
     else if (sc_active) dma4(sc_base, off_s, dma_slot + sc_dst);
   };
   auto issue_tile = [&](int tau) {
@@ -727,6 +791,23 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
       // bf16: the values are relative to the split's own maximum, so their range is that of the
       // output times the split's probability mass)
       // (two accumulator rows of a lane per 16-byte store: [consumer][head half][dvb][row pair][lane][8])
+      if (f32_partials(p)) {                        // (uniform)
+        float* blk = (float*)p.workspace + part_block * (size_t)(2 * kPartFloats) + ((size_t)((role * 2 + hb) * 8) * 64 + lane) * 8;
+#pragma unroll
+        for (int dvb = 0; dvb < 4; ++dvb)
+#pragma unroll
+          for (int j4 = 0; j4 < 4; ++j4) {
+            const f32x16& acc = o[dvb][hb];
+            *reinterpret_cast<float4*>(blk + (size_t)(dvb * 2 + (j4 >> 1)) * 512 + (j4 & 1) * 4) =
+                make_float4(acc[4 * j4], acc[4 * j4 + 1], acc[4 * j4 + 2], acc[4 * j4 + 3]);
+          }
+        if (role == 0 && lane < 32) {
+          float* ml = (float*)p.workspace + part_blocks_total * (size_t)(2 * kPartFloats) + (part_block * kHeadsWg + h_local) * 2;
+          ml[0] = m_all;
+          ml[1] = l_all;
+        }
+        continue;
+      }
       unsigned short* blk = (unsigned short*)p.workspace + part_block * (size_t)(2 * kPartFloats) +
                             ((size_t)((role * 2 + hb) * 8) * 64 + lane) * 8;
 #pragma unroll
@@ -807,6 +888,8 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
 // is channel 128w + 32dvb + 8j + 4half + e of head 32hg + hd.  One workgroup per (query, KV group,
 // head chunk, w, hg): coalesced 1 KiB row reads, weights per head, transposition through LDS,
 // coalesced output rows.
+// F32: the partial values are float32 (and twice as long)
+template <bool F32>
 __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const MlaParams p) {
   constexpr int HG = kHeadsWg / 32;
   __shared__ float x[32][kXPitch];
@@ -824,7 +907,7 @@ __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const Ml
   const int hd = lane & 31, half = lane >> 5;
   const int h_local = 32 * hg + hd;
   const size_t blocks_total = (size_t)p.B * p.S * p.G * chunks * p.num_splits;
-  const float* ml = (const float*)((const unsigned short*)p.workspace + blocks_total * (size_t)(HG * kPartFloats));
+  const float* ml = (const float*)((const unsigned short*)p.workspace + blocks_total * (size_t)(HG * kPartFloats) * (F32 ? 2 : 1));
   const size_t block0 = unit * p.num_splits;
   // all (max, sum) pairs first, then the partial rows four splits at a time, so that the loads
   // of a group are in flight together (the split count is at most 16)
@@ -855,27 +938,40 @@ __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const Ml
 #pragma unroll
   for (int s0 = 0; s0 < 16; s0 += 4) {
     if (s0 >= p.num_splits) break;                            // (uniform)
-    uint4 raw[4][2];                                           // two accumulator rows per 16-byte load
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int s = min(s0 + u, p.num_splits - 1);             // a repeated last split gets weight 0
-#pragma unroll
-      for (int i2 = 0; i2 < 2; ++i2) {                          // (read once: non-temporal, 0.7 us of the decode step)
-        typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-        const u32x4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(src0 + (size_t)s * (HG * kPartFloats) + (size_t)i2 * 512));
-        raw[u][i2] = make_uint4(t[0], t[1], t[2], t[3]);
-      }
-    }
     float4 v[4][4];
+    if constexpr (F32) {
+      const float* src = (const float*)p.workspace + (src0 - (const unsigned short*)p.workspace);
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < 4; ++u) {
+        const int s = min(s0 + u, p.num_splits - 1);
 #pragma unroll
-      for (int i2 = 0; i2 < 2; ++i2) {
-        v[u][2 * i2] = make_float4(__uint_as_float(raw[u][i2].x << 16), __uint_as_float(raw[u][i2].x & 0xffff0000u),
-                                   __uint_as_float(raw[u][i2].y << 16), __uint_as_float(raw[u][i2].y & 0xffff0000u));
-        v[u][2 * i2 + 1] = make_float4(__uint_as_float(raw[u][i2].z << 16), __uint_as_float(raw[u][i2].z & 0xffff0000u),
-                                       __uint_as_float(raw[u][i2].w << 16), __uint_as_float(raw[u][i2].w & 0xffff0000u));
+        for (int i = 0; i < 4; ++i) {
+          const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + (size_t)s * (HG * kPartFloats) + (size_t)(i >> 1) * 512 + (i & 1) * 4));
+          v[u][i] = make_float4(t[0], t[1], t[2], t[3]);
+        }
       }
+    } else {
+      uint4 raw[4][2];                                         // two accumulator rows per 16-byte load
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int s = min(s0 + u, p.num_splits - 1);             // a repeated last split gets weight 0
+#pragma unroll
+        for (int i2 = 0; i2 < 2; ++i2) {                          // (read once: non-temporal, 0.7 us of the decode step)
+          typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+          const u32x4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(src0 + (size_t)s * (HG * kPartFloats) + (size_t)i2 * 512));
+          raw[u][i2] = make_uint4(t[0], t[1], t[2], t[3]);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i2 = 0; i2 < 2; ++i2) {
+          v[u][2 * i2] = make_float4(__uint_as_float(raw[u][i2].x << 16), __uint_as_float(raw[u][i2].x & 0xffff0000u),
+                                     __uint_as_float(raw[u][i2].y << 16), __uint_as_float(raw[u][i2].y & 0xffff0000u));
+          v[u][2 * i2 + 1] = make_float4(__uint_as_float(raw[u][i2].z << 16), __uint_as_float(raw[u][i2].z & 0xffff0000u),
+                                         __uint_as_float(raw[u][i2].w << 16), __uint_as_float(raw[u][i2].w & 0xffff0000u));
+        }
+    }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const float f = (s0 + u < p.num_splits && ms[s0 + u] != -INFINITY) ? exp2f(ms[s0 + u] - m_fin) : 0.0f;
@@ -920,7 +1016,14 @@ __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const Ml
 
 }  // namespace
 
-bool sparse_mla_latent_supported(const MlaParams& p) {
+namespace {
+// queries and key rows of 576 e4m3 codes, one scale each
+bool code_rows(const MlaParams& p) {
+  return p.q_dtype == CPPMEGA_MI355_E4M3 && p.kv_dtype == CPPMEGA_MI355_E4M3 && p.q_scale_kind == CPPMEGA_MI355_SCALE_PER_TOKEN &&
+         p.kv_scale_kind == CPPMEGA_MI355_SCALE_PER_TOKEN && p.d_qk == kDqk && p.d_kv == kDqk && p.d_v == kLat && p.rope_dim == 0 &&
+         p.q_scale && p.kv_scale && !((uintptr_t)p.q_scale & 3);
+}
+bool latent_rows(const MlaParams& p) {
   if (p.q_dtype != CPPMEGA_MI355_BF16 || p.q_scale_kind != CPPMEGA_MI355_SCALE_NONE) return false;
   if (p.d_qk != kDqk || p.d_v != kLat || p.d_kv != kLat) return false;
   if (p.kv_dtype != CPPMEGA_MI355_E4M3) return false;
@@ -930,13 +1033,18 @@ bool sparse_mla_latent_supported(const MlaParams& p) {
   } else if (p.kv_scale_kind != CPPMEGA_MI355_SCALE_PER_TOKEN && p.kv_scale_kind != CPPMEGA_MI355_SCALE_NONE) {
     return false;
   }
-  if (p.heads_per_group <= 32) return false;      // a single 32-head group gains nothing from sharing
+  return true;
+}
+}  // namespace
+
+bool sparse_mla_latent_supported(const MlaParams& p) {
+  if (!latent_rows(p) && !code_rows(p)) return false;
   if (p.topk < 1 || (size_t)p.B * p.S == 0) return false;
   if (((uintptr_t)p.q | (uintptr_t)p.kv | (uintptr_t)p.rope) & 15) return false;
   if (p.kv_scale && ((uintptr_t)p.kv_scale & 3)) return false;
   if ((unsigned long long)p.B * p.Skv_pitch * p.G >= 0x7fffffffull) return false;   // cache rows are counted in 32 bits
   // a lane's byte offset from the first row of its batch is a 24-bit row number times a 24-bit step, below 2^31
-  if ((unsigned long long)p.Skv_pitch * p.G * kLat >= (1ull << 31) || p.Skv_pitch >= (1 << 24) || (long long)p.G * kLat >= (1 << 24)) return false;
+  if ((unsigned long long)p.Skv_pitch * p.G * kDqk >= (1ull << 31) || p.Skv_pitch >= (1 << 24) || (long long)p.G * kDqk >= (1 << 24)) return false;
   if (p.topk > 16 * kMaxKeys) return false;       // the combine step merges at most 16 key splits
   return true;
 }
@@ -961,20 +1069,23 @@ int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream) {
     return fail(CPPMEGA_MI355_ERR_UNSUPPORTED, "sparse MLA: launch too large");
   const dim3 grid((unsigned)wgs), block(512);
   const int nblk = p.kv_scale_kind == CPPMEGA_MI355_SCALE_F32_BLOCK ? kLat / p.kv_scale_block : 1;
-#define CM_LAUNCH_PC(NB_)                                                                                          \
+#define CM_LAUNCH_PC(NB_, ROWS_)                                                                                          \
   do {                                                                                                             \
-    CM_HIP_CHECK(hipFuncSetAttribute((const void*)sparse_mla_latent_kernel<NB_>,                                 \
+    CM_HIP_CHECK(hipFuncSetAttribute((const void*)sparse_mla_latent_kernel<NB_, ROWS_>,                                 \
                                      hipFuncAttributeMaxDynamicSharedMemorySize, kSmem));                           \
-    hipLaunchKernelGGL((sparse_mla_latent_kernel<NB_>), grid, block, kSmem, stream, p);                          \
+    hipLaunchKernelGGL((sparse_mla_latent_kernel<NB_, ROWS_>), grid, block, kSmem, stream, p);                          \
   } while (0)
-  if (nblk == 4) CM_LAUNCH_PC(4);
-  else if (nblk == 2) CM_LAUNCH_PC(2);
-  else CM_LAUNCH_PC(1);
+  const bool rows = code_rows(p);
+  if (rows) CM_LAUNCH_PC(1, true);
+  else if (nblk == 4) CM_LAUNCH_PC(4, false);
+  else if (nblk == 2) CM_LAUNCH_PC(2, false);
+  else CM_LAUNCH_PC(1, false);
 #undef CM_LAUNCH_PC
   CM_HIP_CHECK(hipGetLastError());
   if (p.num_splits > 1) {
     const dim3 cgrid((unsigned)((size_t)p.B * p.S * p.G * chunks), (unsigned)(4 * (kHeadsWg / 32)));
-    hipLaunchKernelGGL(sparse_mla_latent_combine_kernel, cgrid, dim3(256), 0, stream, p);
+    if (f32_partials(p)) hipLaunchKernelGGL(sparse_mla_latent_combine_kernel<true>, cgrid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL(sparse_mla_latent_combine_kernel<false>, cgrid, dim3(256), 0, stream, p);
     CM_HIP_CHECK(hipGetLastError());
   }
   return 0;
@@ -984,7 +1095,7 @@ size_t sparse_mla_latent_workspace_bytes(const MlaParams& p) {
   if (p.num_splits <= 1) return 0;
   const int chunks = (p.heads_per_group + kHeadsWg - 1) / kHeadsWg;
   const size_t blocks = (size_t)p.B * p.S * p.G * chunks * p.num_splits;
-  return blocks * ((size_t)2 * kPartFloats * sizeof(unsigned short) + kHeadsWg * 2 * sizeof(float));
+  return blocks * ((size_t)2 * kPartFloats * (f32_partials(p) ? sizeof(float) : sizeof(unsigned short)) + kHeadsWg * 2 * sizeof(float));
 }
 
 }  // namespace cm

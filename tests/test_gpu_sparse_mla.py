@@ -181,6 +181,28 @@ def test_mfma_kernel_per_token_fp8_rows(device, shape, with_sinks):
         assert (out[0, 1] == 0).all() and (lse[0, 1] == 0).all()
 
 
+@pytest.mark.parametrize("S,H,topk", [(3, 16, 33), (1, 65, 300), (2, 128, 1024)], ids=["h16", "h65_splits", "h128_splits"])
+def test_per_token_fp8_rows_with_unusual_scales(device, S, H, topk):
+    """Query scales of zero and below take the masked-key path; a cache row that no list names is never looked at."""
+    rng = np.random.default_rng(topk)
+    Skv = 1200
+    qc, qs = fp8.quantize_per_token(rng.standard_normal((1, S, H, 576)).astype(np.float32))
+    kc, ks = fp8.quantize_per_token(rng.standard_normal((1, Skv, 1, 576)).astype(np.float32))
+    qs[0, 0, 3], qs[0, 0, 5] = 0.0, -qs[0, 0, 5]
+    idx = 1 + sparse_indices(rng, 1, S, 1, Skv - 1, topk)
+    idx[rng.random(idx.shape) < 0.1] = -1
+    want_out, want_lse = om.sparse_mla_oracle(om.dequant_per_token(qc, qs), om.dequant_per_token(kc, ks), idx, sm_scale=0.04, d_v=512)
+    kc[0, 0] = 0x7f                                                  # NaN
+    ks[0, 0] = np.inf
+    out = torch.zeros((1, S, H, 512), dtype=torch.float32, device=device)
+    lse = torch.zeros((1, S, H), dtype=torch.float32, device=device)
+    f8.sparse_mla_fp8_path_c_apply_direct(
+        to_dev(qc, device), to_dev(qs, device), to_dev(kc, device), to_dev(ks, device), to_dev(idx.astype(np.int32), device),
+        sm_scale=0.04, d_v=512, out=out, lse=lse, kernel="mfma")
+    torch.cuda.synchronize()
+    _assert_close(out, lse, want_out, want_lse)
+
+
 @pytest.mark.parametrize("shape", [
     dict(B=1, S=4, H=16, G=1, Skv=255, topk=64),              # an odd number of rows: the last row's scale bytes end the buffer
     dict(B=2, S=3, H=40, G=1, Skv=700, topk=333),
