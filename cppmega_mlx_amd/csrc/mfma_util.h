@@ -100,4 +100,32 @@ __device__ __forceinline__ float xor32(float v) {
   return __uint_as_float((lane_id() & 32) ? r[0] : r[1]);
 }
 
+__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// v_max_f32 as it is (fmaxf first passes every operand through a canonicalising max with itself).
+// Only for operands that ordinary vector instructions produced: never for matrix results, whose
+// read-after-write wait states the compiler pads only for instructions it can see.
+__device__ __forceinline__ float vmax(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+__device__ __forceinline__ float vmax3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// maximum over lanes l, l^16, l^32, l^48 (every lane gets it): a row swap leaves each value next
+// to its partner's
+__device__ __forceinline__ float max_rows(float v) {
+  unsigned u = __float_as_uint(v);
+  u32x2 r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  u = __float_as_uint(v);
+  r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 }  // namespace cm

@@ -26,7 +26,7 @@ struct MlaParams {
   int heads_per_group;
   int num_splits;       // split-KV factor of the MFMA kernel
   int keys_per_split;
-  int heads_per_wg;     // 0: 32-head tile kernel; 64: shared-tile latent kernel (sparse_mla_latent.hip)
+  int heads_per_wg;     // 0: 32-head tile kernel; 32 or 64: a producer/consumer kernel (sparse_mla_latent.hip, sparse_mla_rows16.hip)
   int tile_sharing;     // tile kernel on 16-bit rows: the 4 wavefronts take 4 head groups over one key stream
   float sm_scale;
   const float* sm_scale_dev;     // device copy of the softmax scale; read in place of sm_scale when set
@@ -61,6 +61,22 @@ int sparse_mla_mfma_launch(const MlaParams& p, hipStream_t stream);
 bool sparse_mla_mfma_supported(const MlaParams& p);
 size_t sparse_mla_mfma_workspace_bytes(const MlaParams& p);
 void sparse_mla_mfma_plan(MlaParams& p);
+
+// partial values that a key split keeps of 32 heads: [4 groups of 128 channels][8 row pairs][64 lanes][8]
+constexpr int kMlaPartFloats = 4 * 16 * 64 * 4;
+int sparse_mla_combine_f32(const MlaParams& p, hipStream_t stream);    // merges the key splits' float32 partial values
+
+// Key splits of the producer/consumer kernels, whose workgroups have a CU to themselves: the number (up to 16, up to
+// max_keys each) with the least modelled time - whole rounds of 256 workgroups, each with its workgroups' start and end
+// and tile_us per tile of 32 keys, then, with several splits, the merging kernel and its traffic (partial_bytes per
+// workgroup, written and read).
+void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, double partial_bytes);
+
+// producer/consumer kernel for 16-bit rows (sparse_mla_rows16.hip); dispatched by the *_mfma_* functions
+bool sparse_mla_rows16_supported(const MlaParams& p);
+void sparse_mla_rows16_plan(MlaParams& p);
+int sparse_mla_rows16_launch(const MlaParams& p, hipStream_t stream);   // includes its combine step
+size_t sparse_mla_rows16_workspace_bytes(const MlaParams& p);
 
 // shared-tile kernel for FP8 latent caches (sparse_mla_latent.hip); dispatched by the *_mfma_* functions
 bool sparse_mla_latent_supported(const MlaParams& p);

@@ -75,7 +75,7 @@ constexpr int kMaxKeys = 2048;                  // keys of one split (their rows
 constexpr int kKeyInts = kMaxKeys + kTK;
 constexpr int kHeadsWg = 64;
 constexpr int kXPitch = 132;                    // floats per head row of the output transpose (128 + 4)
-constexpr int kPartFloats = 4 * 16 * 64 * 4;    // partial values of one 32-head group: [4 consumers][8 row pairs][64 lanes][8]
+constexpr int kPartFloats = kMlaPartFloats;
 constexpr float kLazy = 8.0f;                   // move a running maximum only when it grows by > 2^8
 
 constexpr int kPPlane = 2 * 2 * 1024;           // one plane of P of one tile: [k-step][head block][64 lanes x 16 B]
@@ -89,8 +89,6 @@ constexpr int kKeyOff = kValidOff + (kMaxKeys / kTK) * 4;
 constexpr int kSmem = kKeyOff + kKeyInts * 4;
 static_assert(kSmem <= 160 * 1024, "LDS budget");
 static_assert(4 * 32 * kXPitch * 4 <= kRingBytes, "the output transpose reuses the ring");
-
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 __device__ __forceinline__ bf16x8 cvt8(unsigned w0, unsigned w1) {
   const unsigned o0 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, false));
@@ -152,32 +150,6 @@ __device__ __forceinline__ int split_q32(const uint4 (&x)[4], i32x8& hi, i32x8& 
     }
   }
   return e;
-}
-
-// v_max_f32 as it is (fmaxf first passes every operand through a canonicalising max with itself).
-// Only for operands that ordinary vector instructions produced: never for matrix results, whose
-// read-after-write wait states the compiler pads only for instructions it can see.
-__device__ __forceinline__ float vmax(float a, float b) {
-  float r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
-
-__device__ __forceinline__ float vmax3(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-
-// maximum over lanes l, l^16, l^32, l^48 (every lane gets it): a row swap leaves each value next
-// to its partner's
-__device__ __forceinline__ float max_rows(float v) {
-  unsigned u = __float_as_uint(v);
-  u32x2 r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  v = vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  u = __float_as_uint(v);
-  r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
 // Key splits of these keep float32: code rows and single groups of heads have few enough of them.
@@ -888,10 +860,9 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
 // is channel 128w + 32dvb + 8j + 4half + e of head 32hg + hd.  One workgroup per (query, KV group,
 // head chunk, w, hg): coalesced 1 KiB row reads, weights per head, transposition through LDS,
 // coalesced output rows.
-// F32: the partial values are float32 (and twice as long)
-template <bool F32>
+// F32: the partial values are float32 (and twice as long).  HG: 32-head blocks of a chunk.
+template <bool F32, int HG>
 __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const MlaParams p) {
-  constexpr int HG = kHeadsWg / 32;
   __shared__ float x[32][kXPitch];
   const int tid = (int)threadIdx.x, lane = tid & 63, r4 = tid >> 6;
   const int chunks = (p.heads_per_group + 32 * HG - 1) / (32 * HG);
@@ -1049,17 +1020,38 @@ bool sparse_mla_latent_supported(const MlaParams& p) {
   return true;
 }
 
+void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, double partial_bytes) {
+  // (fitted to 216 shapes of 16 and 128 heads, 1 .. 300 queries, 64 .. 2048 keys: 1.2x in the mean against doubling the
+  // splits until 256 workgroups are there, 3x where that ended just above 256 or in splits of four tiles)
+  constexpr double kUnitUs = 7.0, kMergeUs = 5.0, kBytesPerUs = 5e6;
+  const int tiles = (p.topk + kTK - 1) / kTK;
+  double best = 0.0;
+  p.num_splits = 0;
+  for (int s = 1; s <= 16; ++s) {
+    const int per = (tiles + s - 1) / s;
+    if (per * kTK > max_keys || (s > 1 && (per < 2 || per == (tiles + s - 2) / (s - 1)))) continue;
+    const double wgs = (double)units * s;
+    double us = (double)((units * s + 255) / 256) * (kUnitUs + per * tile_us);
+    if (s > 1) us += kMergeUs + 2.0 * wgs * partial_bytes / kBytesPerUs;
+    if (p.num_splits == 0 || us < best) {
+      best = us;
+      p.num_splits = s;
+      p.keys_per_split = per * kTK;
+    }
+  }
+}
+
 void sparse_mla_latent_plan(MlaParams& p) {
   const int chunks = (p.heads_per_group + kHeadsWg - 1) / kHeadsWg;
   const long long base = (long long)p.B * p.S * p.G * chunks;
-  int splits = 1;
-  while (base * splits < 256 && p.topk / (splits * 2) >= 4 * kTK && splits < 16) splits *= 2;
-  while ((p.topk + splits - 1) / splits > kMaxKeys && splits < 16) splits *= 2;
   p.heads_per_wg = kHeadsWg;
-  const int tiles = (p.topk + kTK - 1) / kTK;
-  const int tiles_per_split = (tiles + splits - 1) / splits;
-  p.num_splits = splits;
-  p.keys_per_split = tiles_per_split * kTK;
+  mla_key_splits(p, base, kMaxKeys, 1.1, kHeadsWg * (double)kLat * (f32_partials(p) ? 4 : 2));
+  // a decode step of a batch too large for the fixed scratch of the entry point without allocations is refused there,
+  // and stays so: one split would need no scratch at all (96 sequences x 128 heads x 2048 keys: 85 us instead of 104)
+  if (p.S == 1 && p.num_splits == 1 && base > 128 && base < 256 && !f32_partials(p) && p.topk >= 8 * kTK) {
+    p.num_splits = 2;
+    p.keys_per_split = ((p.topk + kTK - 1) / kTK + 1) / 2 * kTK;
+  }
 }
 
 int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream) {
@@ -1083,11 +1075,20 @@ int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream) {
 #undef CM_LAUNCH_PC
   CM_HIP_CHECK(hipGetLastError());
   if (p.num_splits > 1) {
+    if (f32_partials(p)) return sparse_mla_combine_f32(p, stream);
     const dim3 cgrid((unsigned)((size_t)p.B * p.S * p.G * chunks), (unsigned)(4 * (kHeadsWg / 32)));
-    if (f32_partials(p)) hipLaunchKernelGGL(sparse_mla_latent_combine_kernel<true>, cgrid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL(sparse_mla_latent_combine_kernel<false>, cgrid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((sparse_mla_latent_combine_kernel<false, 2>), cgrid, dim3(256), 0, stream, p);
     CM_HIP_CHECK(hipGetLastError());
   }
+  return 0;
+}
+
+int sparse_mla_combine_f32(const MlaParams& p, hipStream_t stream) {
+  const int chunks = (p.heads_per_group + p.heads_per_wg - 1) / p.heads_per_wg;
+  const dim3 grid((unsigned)((size_t)p.B * p.S * p.G * chunks), (unsigned)(4 * (p.heads_per_wg / 32)));
+  if (p.heads_per_wg == 64) hipLaunchKernelGGL((sparse_mla_latent_combine_kernel<true, 2>), grid, dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((sparse_mla_latent_combine_kernel<true, 1>), grid, dim3(256), 0, stream, p);
+  CM_HIP_CHECK(hipGetLastError());
   return 0;
 }
 

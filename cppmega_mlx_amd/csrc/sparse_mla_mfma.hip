@@ -5,7 +5,9 @@
 // the latent is e4m3 with one fp32 scale per 128 channels (or per row) plus a
 // bf16 rope tail, or a packed bf16 row of 576.  float16 queries with float16
 // rows of 576 run the same kernel on the float16 matrix instructions.
-// Everything else goes to the scalar kernel.
+// Everything else goes to the scalar kernel.  The producer/consumer kernels (sparse_mla_latent.hip,
+// sparse_mla_rows16.hip) come first wherever they can; this one keeps E8M0 rows, scale blocks of 64 channels, lists
+// beyond 32768 keys and caches whose rows need more than 32 bits of offset.
 //
 // Decomposition
 //   workgroup = (batch*query, group of 32 heads, key split); 4 wavefronts.
@@ -834,7 +836,7 @@ __global__ __launch_bounds__(256) void sparse_mla_combine_kernel(const MlaParams
 }  // namespace
 
 bool sparse_mla_mfma_supported(const MlaParams& p) {
-  if (sparse_mla_latent_supported(p)) return true;
+  if (sparse_mla_latent_supported(p) || sparse_mla_rows16_supported(p)) return true;
   if (p.q_dtype == CPPMEGA_MI355_E4M3) {          // FP8 prepared buffers: rows of 576 codes, both sides scaled alike
     const bool tok = p.q_scale_kind == CPPMEGA_MI355_SCALE_PER_TOKEN && p.kv_scale_kind == CPPMEGA_MI355_SCALE_PER_TOKEN &&
                      (((uintptr_t)p.q_scale | (uintptr_t)p.kv_scale) & 3) == 0;
@@ -877,6 +879,10 @@ void sparse_mla_mfma_plan(MlaParams& p) {
     sparse_mla_latent_plan(p);
     return;
   }
+  if (sparse_mla_rows16_supported(p)) {
+    sparse_mla_rows16_plan(p);
+    return;
+  }
   const int groups_per_kv = (p.heads_per_group + kHeads - 1) / kHeads;
   // 16-bit rows with several head groups per KV group: the wavefronts share one key stream
   // (with two head groups two wavefronts only fetch and it still wins: 4.2 ms against 4.7 ms at
@@ -893,13 +899,13 @@ void sparse_mla_mfma_plan(MlaParams& p) {
 }
 
 size_t sparse_mla_mfma_workspace_bytes(const MlaParams& p) {
-  if (p.heads_per_wg != 0) return sparse_mla_latent_workspace_bytes(p);
+  if (p.heads_per_wg != 0) return p.kv_dtype == CPPMEGA_MI355_E4M3 ? sparse_mla_latent_workspace_bytes(p) : sparse_mla_rows16_workspace_bytes(p);
   if (p.num_splits <= 1) return 0;
   return (size_t)p.B * p.S * p.H * p.num_splits * (kLat + 2) * sizeof(float);
 }
 
 int sparse_mla_mfma_launch(const MlaParams& p, hipStream_t stream) {
-  if (p.heads_per_wg != 0) return sparse_mla_latent_launch(p, stream);
+  if (p.heads_per_wg != 0) return p.kv_dtype == CPPMEGA_MI355_E4M3 ? sparse_mla_latent_launch(p, stream) : sparse_mla_rows16_launch(p, stream);
   const int groups_per_kv = (p.heads_per_group + kHeads - 1) / kHeads;
   const int units = p.tile_sharing ? (groups_per_kv + kWaves - 1) / kWaves : groups_per_kv;
   const dim3 grid((unsigned)((size_t)p.B * p.S * p.G * units), (unsigned)p.num_splits), block(kWaves * 64);

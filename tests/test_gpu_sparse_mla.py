@@ -350,6 +350,34 @@ def test_mfma_kernel_float16_rows(device, shape, rope_tail):
     assert (out[0, 1] == 0).all() and (lse[0, 1] == 0).all()
 
 
+@pytest.mark.parametrize("H,G,topk", [(16, 1, 1), (1, 1, 33), (32, 1, 129), (33, 1, 160), (128, 1, 96), (40, 2, 700), (80, 1, 2049)])
+@pytest.mark.parametrize("carrier", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tail", [False, True], ids=["packed576", "latent_plus_rope"])
+def test_rows_of_16_bits_at_tile_edges(device, H, G, topk, carrier, tail):
+    """One key, a tile and one more, the ring's length and one more, several key splits; scores that grow along the list
+    (the running reference moves), skipped keys in every tile and at the end, a query without keys, sinks."""
+    rng = np.random.default_rng(H + topk)
+    B, S, Skv = 1, 3, 2500
+    q = torch.from_numpy(rng.standard_normal((B, S, H, 576)).astype(np.float32)).to(device).to(carrier)
+    kv = rng.standard_normal((B, Skv, G, 576)).astype(np.float32) * np.linspace(0.2, 3.0, Skv).reshape(1, -1, 1, 1).astype(np.float32)
+    kv = torch.from_numpy(kv).to(device).to(carrier)
+    idx = np.sort(sparse_indices(rng, B, S, G, Skv, topk), axis=-1)
+    if topk > 1:
+        idx[rng.random(idx.shape) < 0.1] = -1
+    idx[0, 1] = -1
+    idx[0, 2, :, topk - topk // 3:] = -1
+    sinks = rng.standard_normal(H).astype(np.float32)
+    want_out, want_lse = om.sparse_mla_oracle(q.double().cpu().numpy(), kv.double().cpu().numpy(), idx, sm_scale=0.05, d_v=512, sinks=sinks)
+    out = torch.zeros((B, S, H, 512), dtype=torch.float32, device=device)
+    lse = torch.zeros((B, S, H), dtype=torch.float32, device=device)
+    rows = dict(kv_rope=kv[..., 512:].contiguous()) if tail else {}
+    ops.sparse_mla_forward(q, kv[..., :512].contiguous() if tail else kv, to_dev(idx, device), sm_scale=0.05, d_v=512, out=out, lse=lse,
+                           sinks=to_dev(sinks, device), kernel="mfma", **rows)
+    torch.cuda.synchronize()
+    _assert_close(out, lse, want_out, want_lse, lse_tol=LSE_TOL_MFMA)
+
+
+
 def test_shared_key_stream_int64_indices_and_cache_views(device):
     """128 heads on bf16 rows of 576: int64 indices, and the rows passed as the live prefix of a larger
     cache buffer (batch pitch = capacity), as `update_and_fetch` hands them out."""
