@@ -52,10 +52,11 @@ struct IndexerParams {
   const void* w;
   const void* k;
   const void* mask;
-  float* scores;             // row (b - b_begin) * s_count + (s - s_begin), pitch Skv
-  unsigned short* qw;        // [2][rows of the pass][Dp] bf16: hi plane, then lo plane
+  float* scores;             // row (b - b_begin) * s_count + (s - s_begin), pitch s_pitch
+  unsigned short* qw;        // [2][rows of the pass][Dp] bf16: hi plane, then lo plane; null: a workgroup sums its rows itself
   int q_dtype, w_dtype, k_dtype, mask_dtype;
   int B, Sq, H, D, Skv;
+  int s_pitch;               // floats between score rows: Skv, in whole fours where the rows are not the caller's
   int b_begin, nb, s_begin, s_count;
   int keys_per_wg;           // multiple of kKeysPerIter
   int q_vec, k_vec, s_vec;   // 16-byte accesses allowed for q rows / k rows / score rows
@@ -150,20 +151,13 @@ __device__ __forceinline__ uint4 load_once(const uint4* src) {
 // load sits in a basic block of its own and the sixteen loads of a round are waited for one after
 // the other (11 us for the 32 rows of a decode step, against 3 us).
 template <int WDT>
-__global__ __launch_bounds__(kQwWaves * 64) void indexer_qw_wave_kernel(const IndexerParams p) {
+__device__ __forceinline__ void sum_heads(const IndexerParams& p, size_t row, int lane, int chunks, float (&acc)[8]) {
   const int D = p.D, H = p.H;
-  const int Dp = (D + 31) & ~31;
-  const int chunks = Dp / 8;                      // 4, 8, 16 or 32 lanes per head
   const int hp = 64 / chunks;                     // heads per load instruction
-  const int rows = p.nb * p.s_count;
-  const int lane = (int)threadIdx.x & 63;
-  const int r = (int)blockIdx.x * kQwWaves + ((int)threadIdx.x >> 6);
-  if (r >= rows) return;
   const int c = lane & (chunks - 1), hs = lane / chunks;
-  const size_t row = (size_t)(p.b_begin + r / p.s_count) * p.Sq + (size_t)(p.s_begin + r % p.s_count);
-  const bool live = 8 * c < D;
-  const uint4* src = reinterpret_cast<const uint4*>((const unsigned short*)p.q + row * H * D + 8 * (live ? c : 0));
-  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  const uint4* src = reinterpret_cast<const uint4*>((const unsigned short*)p.q + row * H * D + 8 * (8 * c < D ? c : 0));
+#pragma unroll
+  for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
   auto add = [&](const uint4& t, float wh) {
     const unsigned u[4] = {t.x, t.y, t.z, t.w};
 #pragma unroll
@@ -189,23 +183,43 @@ __global__ __launch_bounds__(kQwWaves * 64) void indexer_qw_wave_kernel(const In
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] += __shfl_xor(acc[i], off, 64);
   }
-  if (lane >= chunks) return;
+}
+// bf16 planes of 8 channels
+__device__ __forceinline__ void split8(const float (&v)[8], uint4& hi4, uint4& lo4) {
   unsigned short hi[8], lo[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) split_bf16(live ? acc[i] : 0.0f, hi[i], lo[i]);
-  const size_t at = (size_t)r * Dp + 8 * c;
-  *reinterpret_cast<uint4*>(p.qw + at) = make_uint4(hi[0] | ((unsigned)hi[1] << 16), hi[2] | ((unsigned)hi[3] << 16),
-                                                    hi[4] | ((unsigned)hi[5] << 16), hi[6] | ((unsigned)hi[7] << 16));
-  *reinterpret_cast<uint4*>(p.qw + (size_t)rows * Dp + at) =
-      make_uint4(lo[0] | ((unsigned)lo[1] << 16), lo[2] | ((unsigned)lo[3] << 16), lo[4] | ((unsigned)lo[5] << 16),
-                 lo[6] | ((unsigned)lo[7] << 16));
+  for (int i = 0; i < 8; ++i) split_bf16(v[i], hi[i], lo[i]);
+  hi4 = make_uint4(hi[0] | ((unsigned)hi[1] << 16), hi[2] | ((unsigned)hi[3] << 16), hi[4] | ((unsigned)hi[5] << 16), hi[6] | ((unsigned)hi[7] << 16));
+  lo4 = make_uint4(lo[0] | ((unsigned)lo[1] << 16), lo[2] | ((unsigned)lo[3] << 16), lo[4] | ((unsigned)lo[5] << 16), lo[6] | ((unsigned)lo[7] << 16));
+}
+
+template <int WDT>
+__global__ __launch_bounds__(kQwWaves * 64) void indexer_qw_wave_kernel(const IndexerParams p) {
+  const int Dp = (p.D + 31) & ~31;
+  const int chunks = Dp / 8;                      // 4, 8, 16 or 32 lanes per head
+  const int rows = p.nb * p.s_count;
+  const int lane = (int)threadIdx.x & 63;
+  const int r = (int)blockIdx.x * kQwWaves + ((int)threadIdx.x >> 6);
+  if (r >= rows) return;
+  const size_t row = (size_t)(p.b_begin + r / p.s_count) * p.Sq + (size_t)(p.s_begin + r % p.s_count);
+  float acc[8];
+  sum_heads<WDT>(p, row, lane, chunks, acc);
+  if (lane >= chunks) return;
+  if (8 * lane >= p.D)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
+  uint4 hi, lo;
+  split8(acc, hi, lo);
+  const size_t at = (size_t)r * Dp + 8 * lane;
+  *reinterpret_cast<uint4*>(p.qw + at) = hi;
+  *reinterpret_cast<uint4*>(p.qw + (size_t)rows * Dp + at) = lo;
 }
 
 // Keys are the MFMA's A rows and 16 queries its B columns: lane (n, kg) holds C rows
 // 4 kg .. 4 kg + 3 of tile j, i.e. four consecutive keys key0 + 16 j + 4 kg + i of query n, and
 // writes them as one 16-byte store; the four lanes of a query cover 64 contiguous bytes.
 // A workgroup holds QT query tiles (16 QT rows): every key fragment it loads is used for all of them.
-// STAGED (bf16 keys whose rows are exactly 32 KSTEPS channels, Skv a multiple of 4): the 64 keys of a
+// STAGED (bf16 keys whose rows are exactly 32 KSTEPS channels, score rows of whole fours): the 64 keys of a
 // wavefront step are one contiguous piece of memory and are fetched as such - neighbouring lanes,
 // neighbouring 16 bytes; loads whose lanes each point into another row move a quarter of the bytes
 // per clock - and pass through a private LDS tile (32 rows at a time, 16-byte slots XOR-swizzled by
@@ -231,7 +245,8 @@ __global__ __launch_bounds__(kThreads, 2) void indexer_scores_kernel(const Index
   unsigned short* q_hi = q_lds;
   unsigned short* q_lo = q_lds + kQRows * QT * pitch;
 
-  {  // the workgroup's qw rows -> LDS
+  const bool own_sums = STAGED && QT == 1 && !p.qw;
+  if (!own_sums) {  // the workgroup's qw rows -> LDS
     const int chunks = Dp / 8;
     const size_t plane = (size_t)p.nb * p.s_count * Dp;
     for (int e = tid; e < kQRows * QT * chunks; e += kThreads) {
@@ -246,7 +261,30 @@ __global__ __launch_bounds__(kThreads, 2) void indexer_scores_kernel(const Index
       *reinterpret_cast<uint4*>(&q_lo[r * pitch + 8 * c]) = l4;
     }
   }
-  __syncthreads();
+  // (own_sums: a wavefront per row, once the first key rows have been requested)
+  auto sum_rows = [&]() {
+    const int chunks = Dp / 8;
+    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+    for (int e = tid; e < kQRows * chunks; e += kThreads) {
+      if (e / chunks < rows_here) continue;
+      *reinterpret_cast<uint4*>(&q_hi[e / chunks * pitch + e % chunks * 8]) = zero;
+      *reinterpret_cast<uint4*>(&q_lo[e / chunks * pitch + e % chunks * 8]) = zero;
+    }
+    for (int r = wave; r < rows_here; r += kThreads / 64) {
+      const size_t row = (size_t)b * p.Sq + (size_t)(p.s_begin + s_off + r);
+      float acc[8];
+      if (p.w_dtype == CPPMEGA_MI355_F32) sum_heads<CPPMEGA_MI355_F32>(p, row, lane, chunks, acc);
+      else sum_heads<CPPMEGA_MI355_BF16>(p, row, lane, chunks, acc);
+      if (lane < chunks) {
+        uint4 hi, lo;
+        split8(acc, hi, lo);
+        *reinterpret_cast<uint4*>(&q_hi[r * pitch + 8 * lane]) = hi;
+        *reinterpret_cast<uint4*>(&q_lo[r * pitch + 8 * lane]) = lo;
+      }
+    }
+    __syncthreads();
+  };
+  if (!own_sums) __syncthreads();
 
   const int n = lane & 15, kg = lane >> 4;
   int key_begin = (int)blockIdx.x * p.keys_per_wg;
@@ -326,6 +364,9 @@ __global__ __launch_bounds__(kThreads, 2) void indexer_scores_kernel(const Index
         }
     }
     if (key_begin + 64 * wave < key_end) fetch_rows(key_begin + 64 * wave, kc);
+    if constexpr (QT == 1) {
+      if (own_sums) sum_rows();
+    }
     for (int key0 = key_begin + 64 * wave; key0 < key_end; key0 += kKeysPerIter) {
       f32x4 acc[QT][4];
 #pragma unroll
@@ -377,13 +418,14 @@ __global__ __launch_bounds__(kThreads, 2) void indexer_scores_kernel(const Index
           const int r = 16 * qt + 4 * u + (lane >> 4), col = 4 * (lane & 15);
           f32x4 v = *reinterpret_cast<const f32x4*>(ctile + (4 * u + (lane >> 4)) * kCPitch + col);
           const int key = key0 + col;
-          if (r < rows_here && key < key_end) {          // (Skv is a multiple of 4: a group of four keys is in or out as a whole)
+          if (r < rows_here && key < key_end) {          // (the pitch is a multiple of 4: what a group of four has past Skv is nobody's)
             if (p.mask) {
               const size_t mrow = ((size_t)b * p.Sq + (size_t)(p.s_begin + s_off + r)) * p.Skv + key;
 #pragma unroll
-              for (int i = 0; i < 4; ++i) v[i] += load_as(p.mask, mrow + i, p.mask_dtype);
+              for (int i = 0; i < 4; ++i)
+                if (key + i < p.Skv) v[i] += load_as(p.mask, mrow + i, p.mask_dtype);
             }
-            *reinterpret_cast<f32x4*>(p.scores + (out_row0 + r) * (size_t)p.Skv + key) = v;
+            *reinterpret_cast<f32x4*>(p.scores + (out_row0 + r) * (size_t)p.s_pitch + key) = v;
           }
         }
       }
@@ -475,7 +517,7 @@ __global__ __launch_bounds__(kThreads, 2) void indexer_scores_kernel(const Index
       const int r = 16 * qt + n;
       if (r >= rows_here) continue;
       const size_t mask_row = ((size_t)b * p.Sq + (size_t)(p.s_begin + s_off + r)) * p.Skv;
-      float* dst = p.scores + (out_row0 + r) * (size_t)p.Skv;
+      float* dst = p.scores + (out_row0 + r) * (size_t)p.s_pitch;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int key = key0 + 16 * j + 4 * kg;
@@ -509,7 +551,7 @@ constexpr size_t kChunkBytes = (size_t)256 << 20;
 
 Plan make_plan(const cppmega_mi355_indexer_args_t& a) {
   Plan pl;
-  const size_t row_bytes = (size_t)a.seq_kv * 4;
+  const size_t row_bytes = (size_t)((a.seq_kv + 3) & ~3) * 4;
   if (a.scores_out) {                 // the caller keeps every score: one pass over everything
     pl.rows_per_pass = a.seq_q;
     pl.batches_per_pass = a.batch;
@@ -530,7 +572,7 @@ Plan make_plan(const cppmega_mi355_indexer_args_t& a) {
   pl.qw_bytes = (rows * (size_t)((a.head_dim + 31) & ~31) * 2 * 2 + 255) & ~(size_t)255;
   cppmega_mi355_topk_args_t t;
   memset(&t, 0, sizeof(t));
-  t.rows = (int)rows; t.width = a.seq_kv; t.row_stride = a.seq_kv; t.k = a.topk;
+  t.rows = (int)rows; t.width = a.seq_kv; t.row_stride = (a.seq_kv + 3) & ~3; t.k = a.topk;
   pl.topk_bytes = 0;
   if (a.topk >= 1 && a.topk <= a.seq_kv) (void)topk_workspace_bytes(t, &pl.topk_bytes);
   return pl;
@@ -566,12 +608,17 @@ int indexer_topk_workspace_bytes(const cppmega_mi355_indexer_args_t& a, size_t* 
   return 0;
 }
 
+// the form of the scores kernel that fetches whole rows of bf16 keys
+static bool scores_staged(const IndexerParams& p) {
+  return p.k_dtype == CPPMEGA_MI355_BF16 && p.k_vec && p.s_vec && (p.D == 32 || p.D == 64 || p.D == 128);
+}
+
 template <bool K_F32, int QT>
 static int launch_scores(const IndexerParams& p, dim3 grid, hipStream_t stream) {
   const size_t q_bytes = (size_t)2 * kQRows * QT * (((p.D + 31) & ~31) + 8) * sizeof(unsigned short);   // (two query tiles are only used up to D = 128: 17 KB)
   const int ks = (p.D + 31) / 32;
   if constexpr (!K_F32) {
-    if (p.k_vec && p.s_vec && p.D % 32 == 0 && (ks == 1 || ks == 2 || ks == 4)) {
+    if (scores_staged(p)) {
       const size_t lds = q_bytes + (size_t)(kThreads / 64) * kStageBytes;
       const void* fn = ks == 1 ? (const void*)indexer_scores_kernel<false, 1, QT, true>
                      : ks == 2 ? (const void*)indexer_scores_kernel<false, 2, QT, true>
@@ -608,13 +655,14 @@ int indexer_topk_launch(const cppmega_mi355_indexer_args_t& a, hipStream_t strea
   IndexerParams p;
   p.q = a.q; p.w = a.weights; p.k = a.k; p.mask = a.mask; p.scores = scores;
   p.starts = nullptr; p.ends = nullptr;
-  p.qw = (unsigned short*)((char*)a.workspace + pl.score_bytes);
+  unsigned short* const qw = (unsigned short*)((char*)a.workspace + pl.score_bytes);
   p.q_dtype = a.q_dtype; p.w_dtype = a.w_dtype; p.k_dtype = a.k_dtype; p.mask_dtype = a.mask_dtype;
   p.B = a.batch; p.Sq = a.seq_q; p.H = a.heads; p.D = a.head_dim; p.Skv = a.seq_kv;
   p.sm_scale = a.sm_scale;
   p.q_vec = a.q_dtype == CPPMEGA_MI355_BF16 && a.head_dim % 8 == 0 && ((uintptr_t)a.q & 15) == 0;
   p.k_vec = a.head_dim % 8 == 0 && ((uintptr_t)a.k & 15) == 0;
-  p.s_vec = a.seq_kv % 4 == 0;
+  p.s_pitch = a.scores_out ? a.seq_kv : (a.seq_kv + 3) & ~3;
+  p.s_vec = p.s_pitch % 4 == 0;
 
   for (int b0 = 0; b0 < a.batch; b0 += pl.batches_per_pass) {
     const int nb = a.batch - b0 < pl.batches_per_pass ? a.batch - b0 : pl.batches_per_pass;
@@ -627,13 +675,19 @@ int indexer_topk_launch(const cppmega_mi355_indexer_args_t& a, hipStream_t strea
         p.ends = a.ends ? a.ends + first : nullptr;
       }
       const int dp8 = ((a.head_dim + 31) & ~31) / 8;
-      if (p.q_vec && (dp8 & (dp8 - 1)) == 0) {
+      const bool waves = p.q_vec && (dp8 & (dp8 - 1)) == 0;
+      // Up to four query rows (decode): a wavefront of every workgroup sums one itself under the first key loads, from
+      // the L2 - 64 heads of 128 channels are 16 KB - and the 5.6 us kernel in front of the scores goes away.
+      const bool own_sums = waves && s_count <= 4 && scores_staged(p);
+      p.qw = own_sums ? nullptr : qw;
+      if (own_sums) {
+      } else if (waves) {
         const dim3 qgrid((unsigned)((nb * s_count + kQwWaves - 1) / kQwWaves)), qblock(kQwWaves * 64);
         if (a.w_dtype == CPPMEGA_MI355_F32) hipLaunchKernelGGL(indexer_qw_wave_kernel<CPPMEGA_MI355_F32>, qgrid, qblock, 0, stream, p);
-        else if (a.w_dtype == CPPMEGA_MI355_BF16) hipLaunchKernelGGL(indexer_qw_wave_kernel<CPPMEGA_MI355_BF16>, qgrid, qblock, 0, stream, p);
-        else hipLaunchKernelGGL(indexer_qw_wave_kernel<CPPMEGA_MI355_F16>, qgrid, qblock, 0, stream, p);
-      } else
+        else hipLaunchKernelGGL(indexer_qw_wave_kernel<CPPMEGA_MI355_BF16>, qgrid, qblock, 0, stream, p);
+      } else {
         hipLaunchKernelGGL(indexer_qw_kernel, dim3((unsigned)(nb * s_count)), dim3(kThreads), 0, stream, p);
+      }
       const int qt = (s_count >= 4 * kQRows && a.head_dim <= 128) ? 2 : 1;     // query tiles per workgroup (prefill: two)
       const int tiles = (s_count + kQRows * qt - 1) / (kQRows * qt);
       const int max_splits = (a.seq_kv + kKeysPerIter - 1) / kKeysPerIter;
@@ -653,7 +707,7 @@ int indexer_topk_launch(const cppmega_mi355_indexer_args_t& a, hipStream_t strea
       t.struct_size = (uint32_t)sizeof(t);
       t.score_dtype = CPPMEGA_MI355_F32;
       t.scores = scores;
-      t.row_stride = a.seq_kv;
+      t.row_stride = p.s_pitch;
       t.rows = nb * s_count;
       t.width = a.seq_kv;
       t.k = a.topk;

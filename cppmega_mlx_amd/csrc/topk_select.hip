@@ -7,12 +7,11 @@
 // In topk_tile_kernel (rows of up to 32768 columns) every thread owns a
 // contiguous run of columns: a thread's selected columns are then a bit mask,
 // one block-wide prefix sum of the popcounts gives every thread its output
-// offset, and the indices come out in ascending order.  Rows whose address and
-// pitch allow 16-byte loads are fetched that way by the owning thread itself,
-// the pieces of a run one load after the other (a wavefront's first load
-// brings in the lines its next ones hit): the histogram can be cleared while
-// the loads travel and no barrier precedes the first pass.  Other rows are
-// loaded a column per lane and reach their owners through an LDS tile.  Wider
+// offset, and the indices come out in ascending order.  The owning thread fetches its run itself,
+// 16 bytes at a time whatever the row's alignment, the pieces of a run one load after the other (a
+// wavefront's first load brings in the lines its next ones hit): the histogram can be cleared while
+// the loads travel and no barrier precedes the first pass.  (Rows whose width or pitch is not a
+// multiple of four took a way through an LDS tile before: 12.6 us instead of 9 for 4 rows of 8191.)  Wider
 // rows (topk_wide_kernel, up to 65536 columns) keep the interleaved ownership
 // of coalesced loads and compact with per-chunk ballots.
 //
@@ -54,7 +53,7 @@ struct TopkParams {
   const int* ends;
   int* out;
   int rows, width, k, order, neg_inf_masked;
-  int sort_len;  // power of two >= k, used by the value-descending order
+  int sort_len;  // power of two >= k, 256 at least, used by the value-descending order
   // Rows too wide for one workgroup's fast path are selected in two stages (tile kernel only):
   // stage 1 launches one workgroup per (row, segment of seg_width columns) and writes the
   // segment's k best as candidates (value, column) in ascending column order; stage 2 selects
@@ -71,31 +70,34 @@ struct BHalf {};
 template <typename T> struct Storage { typedef unsigned short type; };
 template <> struct Storage<float> { typedef float type; };
 
+typedef unsigned u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+// vec4: four columns of a row that may start anywhere
 template <typename T> struct ScoreLoad;
 template <> struct ScoreLoad<float> {
   static __device__ __forceinline__ void vec4(const float* p, float (&o)[4]) {
-    const float4 t = *reinterpret_cast<const float4*>(p);
-    o[0] = t.x; o[1] = t.y; o[2] = t.z; o[3] = t.w;
+    typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+    const f32x4_any t = *reinterpret_cast<const f32x4_any*>(p);
+    o[0] = t[0]; o[1] = t[1]; o[2] = t[2]; o[3] = t[3];
   }
   static __device__ __forceinline__ float one(const float* p) { return *p; }
 };
 template <> struct ScoreLoad<Half> {
   static __device__ __forceinline__ void vec4(const unsigned short* p, float (&o)[4]) {
-    const uint2 t = *reinterpret_cast<const uint2*>(p);
-    o[0] = f16_bits_to_f32((unsigned short)(t.x & 0xffffu));
-    o[1] = f16_bits_to_f32((unsigned short)(t.x >> 16));
-    o[2] = f16_bits_to_f32((unsigned short)(t.y & 0xffffu));
-    o[3] = f16_bits_to_f32((unsigned short)(t.y >> 16));
+    const u32x2_any t = *reinterpret_cast<const u32x2_any*>(p);
+    o[0] = f16_bits_to_f32((unsigned short)(t[0] & 0xffffu));
+    o[1] = f16_bits_to_f32((unsigned short)(t[0] >> 16));
+    o[2] = f16_bits_to_f32((unsigned short)(t[1] & 0xffffu));
+    o[3] = f16_bits_to_f32((unsigned short)(t[1] >> 16));
   }
   static __device__ __forceinline__ float one(const unsigned short* p) { return f16_bits_to_f32(*p); }
 };
 template <> struct ScoreLoad<BHalf> {
   static __device__ __forceinline__ void vec4(const unsigned short* p, float (&o)[4]) {
-    const uint2 t = *reinterpret_cast<const uint2*>(p);
-    o[0] = __uint_as_float(t.x << 16);
-    o[1] = __uint_as_float(t.x & 0xffff0000u);
-    o[2] = __uint_as_float(t.y << 16);
-    o[3] = __uint_as_float(t.y & 0xffff0000u);
+    const u32x2_any t = *reinterpret_cast<const u32x2_any*>(p);
+    o[0] = __uint_as_float(t[0] << 16);
+    o[1] = __uint_as_float(t[0] & 0xffff0000u);
+    o[2] = __uint_as_float(t[1] << 16);
+    o[3] = __uint_as_float(t[1] & 0xffff0000u);
   }
   static __device__ __forceinline__ float one(const unsigned short* p) { return bf16_bits_to_f32(*p); }
 };
@@ -222,37 +224,105 @@ __device__ __forceinline__ unsigned order_key(float x) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
+// The value of lane ^ LX by vector instructions alone.
+template <int LX>
+__device__ __forceinline__ unsigned lane_xor(unsigned v) {
+  if constexpr (LX == 32) {
+    const u32x2 r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return (lane_id() & 32) ? r[0] : r[1];
+  } else if constexpr (LX == 16) {
+    const u32x2 r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return (lane_id() & 16) ? r[0] : r[1];
+  } else if constexpr (LX == 8) {
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, true);              // row_ror:8
+  } else if constexpr (LX == 4) {
+    const int m = __builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true);                 // row_half_mirror: lane ^ 7
+    return (unsigned)__builtin_amdgcn_update_dpp(0, m, 0x1b, 0xf, 0xf, true);                    // quad_perm 3 2 1 0: lane ^ 3
+  } else if constexpr (LX == 2) {
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, true);               // quad_perm 2 3 0 1
+  } else {
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, true);               // quad_perm 1 0 3 2
+  }
+}
+
+// Bitonic sort of P (a power of two from 256 on) keys in LDS, largest first.  A wavefront keeps 256 of them, four to
+// a lane, and exchanges over strides below 256 in registers; only the longer strides go through LDS with a barrier
+// each: 6 of the 66 steps of 2048 keys (with all of them in LDS the best 2048 of a row of 8192 took 28 us in this order,
+// with the exchanges by LDS permutes 21).
+template <int THREADS>
+__device__ __forceinline__ void sort_pairs(unsigned long long* pairs, unsigned P) {
+  const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  // one step of the keys 4 lane .. 4 lane + 3 of a chunk: i & size decides the direction
+  auto in_registers = [&](unsigned base, unsigned first_size, unsigned last_size) {
+    unsigned long long v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = pairs[base + 4 * lane + r];
+    for (unsigned size = first_size; size <= last_size; size <<= 1) {
+      const bool desc_run = ((base + 4 * lane) & size) == 0;
+      auto across = [&](auto lanes) {                  // stride 4 * LX
+        constexpr int LX = decltype(lanes)::value;
+        if (size < 8 * LX) return;                     // (uniform)
+        const bool keep_max = ((lane & LX) == 0) == desc_run;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const unsigned long long other = (unsigned long long)lane_xor<LX>((unsigned)(v[r] >> 32)) << 32 | lane_xor<LX>((unsigned)v[r]);
+          v[r] = (v[r] < other) == keep_max ? other : v[r];
+        }
+      };
+      across(std::integral_constant<int, 32>{});
+      across(std::integral_constant<int, 16>{});
+      across(std::integral_constant<int, 8>{});
+      across(std::integral_constant<int, 4>{});
+      across(std::integral_constant<int, 2>{});
+      across(std::integral_constant<int, 1>{});
+#pragma unroll
+      for (unsigned stride = 2; stride >= 1; stride >>= 1) {
+        if (stride >= size) continue;
+#pragma unroll
+        for (unsigned r = 0; r < 4; ++r) {
+          if (r & stride) continue;
+          const bool desc = ((base + 4 * lane + r) & size) == 0;
+          const unsigned long long a = v[r], b = v[r + stride];
+          const bool swap = (a < b) == desc;
+          v[r] = swap ? b : a;
+          v[r + stride] = swap ? a : b;
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) pairs[base + 4 * lane + r] = v[r];
+  };
+  for (unsigned base = 256 * wave; base < P; base += 4 * THREADS) in_registers(base, 2, 256);
+  __syncthreads();
+  for (unsigned size = 512; size <= P; size <<= 1) {
+    for (unsigned stride = size >> 1; stride >= 256; stride >>= 1) {
+      for (unsigned t = tid; t < P / 2; t += THREADS) {
+        const unsigned i = 2 * t - (t & (stride - 1));
+        const unsigned long long a = pairs[i], b = pairs[i + stride];
+        if ((a < b) == ((i & size) == 0)) { pairs[i] = b; pairs[i + stride] = a; }
+      }
+      __syncthreads();
+    }
+    for (unsigned base = 256 * wave; base < P; base += 4 * THREADS) in_registers(base, size, size);
+    __syncthreads();
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Rows of up to 8192 columns: 256 threads, thread t owns columns [t*E, (t+1)*E).
 // ---------------------------------------------------------------------------
 constexpr int kTileThreads = 256;
 constexpr int kTileScratch = kHistBins + 64;            // words: histogram + scan scratch
-// The row tile is not padded (8192 columns are 32 KiB: four such workgroups fit a CU, and the
-// allocation of a padded tile let only three in).  A thread's run of E columns is E/4 pieces of 16
-// bytes; piece i of thread t sits at position (i + rot(t)) mod E/4 of the run, with rot chosen so
-// that the sixteen lanes of one LDS cycle read sixteen different 16-byte bank groups.
-template <int E>
-__device__ __forceinline__ int tile_piece_slot(int t, int i) {
-  constexpr int PP = E / 4;                               // pieces per thread: 1, 2, 4 or 8
-  if constexpr (PP == 1) return t;
-  constexpr int SH = PP == 2 ? 3 : PP == 4 ? 2 : 1;       // log2(16 / PP)
-  return PP * t + ((i + (t >> SH)) & (PP - 1));
-}
-// both histograms fit the tile's allocation of the widest shape with 64 words to spare
+// the wider shapes have a histogram for each of the first two passes
 __host__ __device__ constexpr bool tile_two_hists(int E, int threads) { return threads * E >= 2 * kHistBins; }
 
 // MODE 0: a row per workgroup.  MODE 1: stage 1 of a wide row (a segment per workgroup, candidates
 // out).  MODE 2: stage 2 (a row of candidates per workgroup, positions translated through index_map).
-// DIRECT: a thread fetches its own run of columns from memory, 16 bytes at a time, the pieces of
-// a run one load after the other (the lines a wavefront touches with its first load serve its
-// next ones from the cache): no trip through an LDS tile and no barriers before the first pass.
-template <typename ScoreT, int E, int VEC, int THREADS = kTileThreads, int MODE = 0, bool DIRECT = false>
+// SORTED: the value-descending order, a kernel of its own (with the sort behind a run-time test the index order of rows
+// of 8193 .. 16384 columns took half as long again).
+template <typename ScoreT, int E, int THREADS, int MODE, bool SORTED>
 __global__ __launch_bounds__(THREADS, E > 16 ? 4 : 8) void topk_tile_kernel(const TopkParams p) {
-  static_assert(!DIRECT || VEC == 4, "direct loads are 16-byte loads");
-  constexpr int ITEMS = E / VEC;                        // loads per thread
-  constexpr int CHUNK = THREADS * VEC;                  // columns covered by one load per thread
   extern __shared__ __align__(16) unsigned smem[];
-  float* tile = reinterpret_cast<float*>(smem);
   unsigned* hist = smem;
   typedef typename Storage<ScoreT>::type St;
 
@@ -273,44 +343,37 @@ __global__ __launch_bounds__(THREADS, E > 16 ? 4 : 8) void topk_tile_kernel(cons
 
   float v[E];
   constexpr int kHist2 = tile_two_hists(E, THREADS) ? kHistBins + 64 : 0;
-  if constexpr (DIRECT) {
-    // (no tile in LDS on this path: the histograms are cleared before the row's bounds have arrived)
+  {
+    // two cleared histograms: pass 1 uses the first, pass 2 the second (no clear + barrier in between);
+    // they are cleared before the row's bounds have arrived
     zero_hist<THREADS>(hist, kHist2 ? kHist2 + kHistBins : kHistBins);
     const int c0 = tid * E;
     const bool any = c0 < end && c0 + E > start;          // (a run with nothing selectable is not read)
+    // The last piece of a row may reach up to three columns past it: into the row's padding or the next row, which is
+    // fine, but behind the last row there may be nothing.
+    const bool past = (T & 3) != 0 && MODE != 2 && row + 1 == p.rows && base + ((T + 3) & ~3) > p.row_stride;     // (uniform)
+    if (!past) {
 #pragma unroll
-    for (int i = 0; i < E / 4; ++i) {
-      float t4[4] = {kNaN, kNaN, kNaN, kNaN};
-      if (any && c0 + 4 * i < T) ScoreLoad<ScoreT>::vec4(src + c0 + 4 * i, t4);
-      v[4 * i] = t4[0]; v[4 * i + 1] = t4[1]; v[4 * i + 2] = t4[2]; v[4 * i + 3] = t4[3];
-    }
-  } else {
-  // ---- HBM -> LDS, coalesced; chunks with nothing selectable are not read ----------
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    const int chunk_lo = j * CHUNK;
-    const int col = chunk_lo + tid * VEC;
-    if (chunk_lo >= end || chunk_lo + CHUNK <= start || col >= T) continue;
-    float* dst = tile + 4 * tile_piece_slot<E>(col / E, (col % E) >> 2) + (col & 3);
-    if constexpr (VEC == 4) {
-      float t4[4];
-      ScoreLoad<ScoreT>::vec4(src + col, t4);
-      *reinterpret_cast<float4*>(dst) = make_float4(t4[0], t4[1], t4[2], t4[3]);
+      for (int i = 0; i < E / 4; ++i) {
+        float t4[4] = {kNaN, kNaN, kNaN, kNaN};
+        if (any && c0 + 4 * i < T) ScoreLoad<ScoreT>::vec4(src + c0 + 4 * i, t4);
+        v[4 * i] = t4[0]; v[4 * i + 1] = t4[1]; v[4 * i + 2] = t4[2]; v[4 * i + 3] = t4[3];
+      }
     } else {
-      *dst = ScoreLoad<ScoreT>::one(src + col);
+#pragma unroll
+      for (int i = 0; i < E / 4; ++i) {
+        float t4[4] = {kNaN, kNaN, kNaN, kNaN};
+        if (any && c0 + 4 * i + 3 < T) {
+          ScoreLoad<ScoreT>::vec4(src + c0 + 4 * i, t4);
+        } else if (any) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            if (c0 + 4 * i + c < T) t4[c] = ScoreLoad<ScoreT>::one(src + c0 + 4 * i + c);
+        }
+        v[4 * i] = t4[0]; v[4 * i + 1] = t4[1]; v[4 * i + 2] = t4[2]; v[4 * i + 3] = t4[3];
+      }
     }
   }
-  __syncthreads();
-  // ---- LDS -> registers: my contiguous run ------------------------------------------
-#pragma unroll
-  for (int i = 0; i < E / 4; ++i) {
-    const float4 t4 = *reinterpret_cast<const float4*>(tile + 4 * tile_piece_slot<E>(tid, i));
-    v[4 * i] = t4.x; v[4 * i + 1] = t4.y; v[4 * i + 2] = t4.z; v[4 * i + 3] = t4.w;
-  }
-  __syncthreads();
-  }
-  // two cleared histograms: pass 1 uses the first, pass 2 the second (no clear + barrier in between)
-  if constexpr (!DIRECT) zero_hist<THREADS>(hist, kHist2 ? kHist2 + kHistBins : kHistBins);
   __syncthreads();
 
   // ---- canonicalise (-0 -> +0, NaN -> quiet NaN, masked -> NaN) + pass 1 -------------
@@ -406,7 +469,7 @@ __global__ __launch_bounds__(THREADS, E > 16 ? 4 : 8) void topk_tile_kernel(cons
   // (the common case - index order, no duplicated threshold - only counts here and compares again
   // when it writes: a compare and an add-with-carry per element instead of building a mask and
   // taking it apart)
-  const bool sorted = p.order == CPPMEGA_MI355_TOPK_ORDER_VALUE;
+  constexpr bool sorted = SORTED;
   const bool plain = !sorted && !tie;
   unsigned gmask = 0, emask = 0, cg = 0, ce = 0;
   if (plain) {
@@ -488,19 +551,7 @@ __global__ __launch_bounds__(THREADS, E > 16 ? 4 : 8) void topk_tile_kernel(cons
   const unsigned P = (unsigned)p.sort_len;
   for (unsigned i = n_sel + tid; i < P; i += THREADS) pairs[i] = 0ull;   // sorts last
   __syncthreads();
-  // bitonic sort, descending: larger value first, then lower index
-  for (unsigned size = 2; size <= P; size <<= 1) {
-    for (unsigned stride = size >> 1; stride > 0; stride >>= 1) {
-      for (unsigned t = tid; t < P / 2; t += THREADS) {
-        const unsigned i = 2 * t - (t & (stride - 1));
-        const unsigned jx = i + stride;
-        const bool desc = (i & size) == 0;
-        const unsigned long long a = pairs[i], b = pairs[jx];
-        if ((a < b) == desc) { pairs[i] = b; pairs[jx] = a; }
-      }
-      __syncthreads();
-    }
-  }
+  sort_pairs<THREADS>(pairs, P);
   for (unsigned i = tid; i < k; i += THREADS) {
     const int pos = (int)(0xffffffffu - (unsigned)(pairs[i] & 0xffffffffull));
     out_row[i] = (i < n_sel) ? (MODE == 2 ? map[pos] : pos) : -1;
@@ -689,18 +740,7 @@ __global__ __launch_bounds__(kWideThreads) void topk_wide_kernel(const TopkParam
   const unsigned P = (unsigned)p.sort_len;
   for (unsigned i = n_sel + tid; i < P; i += THREADS) pairs[i] = 0ull;
   __syncthreads();
-  for (unsigned size = 2; size <= P; size <<= 1) {
-    for (unsigned stride = size >> 1; stride > 0; stride >>= 1) {
-      for (unsigned t = tid; t < P / 2; t += THREADS) {
-        const unsigned i = 2 * t - (t & (stride - 1));
-        const unsigned jx = i + stride;
-        const bool desc = (i & size) == 0;
-        const unsigned long long a = pairs[i], b = pairs[jx];
-        if ((a < b) == desc) { pairs[i] = b; pairs[jx] = a; }
-      }
-      __syncthreads();
-    }
-  }
+  sort_pairs<THREADS>(pairs, P);
   for (unsigned i = tid; i < k; i += THREADS)
     out_row[i] = (i < n_sel) ? (int)(0xffffffffu - (unsigned)(pairs[i] & 0xffffffffull)) : -1;
 }
@@ -721,21 +761,24 @@ int launch_for_type(const TopkParams& p, bool vec4, hipStream_t stream, size_t* 
   const size_t out_words = sorted ? (size_t)p.sort_len * 2 : (size_t)p.k;
   if (T <= 32768) {
     auto tile_smem = [&](int E, int threads) {
-      const size_t tile_words = (size_t)threads * E;
       // (with two histograms the second one's scan scratch, 64 words, lies behind it)
-      const size_t need = (size_t)kTileScratch + (tile_two_hists(E, threads) && out_words < (size_t)kHistBins + 64 ? (size_t)kHistBins + 64 : out_words);
-      return (need > tile_words ? need : tile_words) * 4;
+      return ((size_t)kTileScratch + (tile_two_hists(E, threads) && out_words < (size_t)kHistBins + 64 ? (size_t)kHistBins + 64 : out_words)) * 4;
     };
 #define CM_TOPK_TILE(E, THR)                                                              \
   do {                                                                                    \
     const size_t smem = tile_smem(E, THR);                                                \
     *smem_out = smem;                                                                     \
     if (smem > 160 * 1024) return -3;                                                     \
-    return vec4 ? launch_kernel(topk_tile_kernel<ScoreT, E, 4, THR, MODE, true>, p, THR, smem, stream) \
-                : launch_kernel(topk_tile_kernel<ScoreT, E, 1, THR, MODE, false>, p, THR, smem, stream); \
+    if constexpr (MODE != 1)                                                              \
+      if (sorted) return launch_kernel(topk_tile_kernel<ScoreT, E, THR, MODE, true>, p, THR, smem, stream); \
+    return launch_kernel(topk_tile_kernel<ScoreT, E, THR, MODE, false>, p, THR, smem, stream); \
   } while (0)
     if constexpr (MODE == 1) {                            // a segment is always kSegWidth columns wide
       CM_TOPK_TILE(16, 512);
+    }
+    // sorted: eight wavefronts for their chunks of 256
+    if constexpr (MODE == 0) {
+      if (sorted && p.k > 1024 && T <= 4096) CM_TOPK_TILE(8, 512);
     }
     if (T <= 1024) CM_TOPK_TILE(4, kTileThreads);
     if (T <= 2048) CM_TOPK_TILE(8, kTileThreads);
@@ -751,12 +794,7 @@ int launch_for_type(const TopkParams& p, bool vec4, hipStream_t stream, size_t* 
   const size_t smem = ((size_t)kWideScratch + out_words) * 4;
   *smem_out = smem;
   if (smem > 160 * 1024) return -3;
-  if (vec4) {
-    if (T <= 32768) return launch_kernel(topk_wide_kernel<ScoreT, 8, 4>, p, kWideThreads, smem, stream);
-    if (T <= 65536) return launch_kernel(topk_wide_kernel<ScoreT, 16, 4>, p, kWideThreads, smem, stream);
-  } else {
-    if (T <= 32768) return launch_kernel(topk_wide_kernel<ScoreT, 32, 1>, p, kWideThreads, smem, stream);
-  }
+  if (vec4 && T <= 65536) return launch_kernel(topk_wide_kernel<ScoreT, 16, 4>, p, kWideThreads, smem, stream);
   return -1;
 }
 
@@ -766,9 +804,9 @@ int launch_for_type(const TopkParams& p, bool vec4, hipStream_t stream, size_t* 
 // shape) when the caller supplies a workspace; k must fit a segment and segs * k one stage-2 row.
 constexpr int kSegWidth = 8192;
 static int topk_segments(const cppmega_mi355_topk_args_t& a) {
-  if (a.width <= 16384 || a.k > kSegWidth || a.width % 4 != 0 || a.row_stride % 4 != 0) return 1;
+  if (a.width <= 16384 || a.k > kSegWidth) return 1;
   const int segs = (a.width + kSegWidth - 1) / kSegWidth;
-  if ((long long)segs * a.k > 32768 || ((long long)segs * a.k) % 4 != 0) return 1;
+  if ((long long)segs * a.k > 32768) return 1;
   return segs;
 }
 static size_t topk_workspace_for(const cppmega_mi355_topk_args_t& a, int segs) {
@@ -803,7 +841,7 @@ int topk_select_launch(const cppmega_mi355_topk_args_t& a, hipStream_t stream) {
   TopkParams p;
   p.scores = a.scores; p.row_stride = a.row_stride; p.starts = a.starts; p.ends = a.ends; p.out = a.indices;
   p.rows = a.rows; p.width = a.width; p.k = a.k; p.order = a.order; p.neg_inf_masked = a.neg_inf_is_masked ? 1 : 0;
-  int sort_len = 2;
+  int sort_len = 256;
   while (sort_len < a.k) sort_len <<= 1;
   p.sort_len = sort_len;
   p.segs = 1; p.seg_width = 0; p.cand_val = nullptr; p.cand_idx = nullptr; p.index_map = nullptr;

@@ -221,3 +221,19 @@ def test_argument_errors(device):
         ops.indexer_topk(q.half(), k, w, sm_scale=1.0, topk=4, out=out)
     with pytest.raises(ValueError):
         ops.indexer_topk(q, k, w, sm_scale=1.0, topk=4, out=out.long())
+
+
+@pytest.mark.parametrize("B,Sq,H,D,Skv,topk", [(3, 1, 64, 128, 1023, 64), (2, 4, 7, 64, 517, 30), (1, 3, 100, 32, 2050, 2050), (2, 5, 64, 128, 777, 100)],
+                         ids=["one_row", "four_rows", "all_keys", "five_rows"])
+def test_few_query_rows_over_key_counts_off_four(device, B, Sq, H, D, Skv, topk):
+    """Up to four query rows are summed over their heads by the workgroups that score them; score rows of any length."""
+    rng = np.random.default_rng(Skv)
+    q, k, w = _int_inputs(rng, B, Sq, H, D, Skv)
+    qt, kt = (to_dev(a, device).bfloat16() for a in (q, k))
+    ends = rng.integers(Skv // 2, Skv + 1, B * Sq).astype(np.int32)
+    want = oi.indexer_topk_oracle(q, k, w, sm_scale=0.125, index_topk=topk, ends=ends)
+    for weights in (to_dev(w, device), to_dev(w, device).bfloat16()):
+        out = torch.full((B, Sq, topk), -9, dtype=torch.int32, device=device)
+        ops.indexer_topk(qt, kt, weights, sm_scale=0.125, topk=topk, out=out, ends=to_dev(ends, device))
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy(), want)

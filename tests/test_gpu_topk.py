@@ -155,3 +155,20 @@ def test_wide_rows_two_stage_and_single_workgroup_paths_agree_with_the_oracle(de
     need = C.c_size_t(0)
     assert _lib.load().cppmega_mi355_topk_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK
     assert (need.value > 0) == (width % 4 == 0 and width > 16384)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,width,k,offset", [(3, 1023, 5, 1), (1, 8191, 2048, 3), (2, 4097, 300, 0), (3, 16383, 1000, 1), (2, 30001, 2047, 1), (1, 17, 16, 2)])
+def test_rows_that_start_and_end_anywhere(device, rows, width, k, offset, dtype):
+    """Widths that are no multiple of four, at addresses that are none of 16 bytes; the last row ends its buffer."""
+    rng = np.random.default_rng(width)
+    flat = torch.from_numpy(rng.standard_normal(offset + rows * width).astype(np.float32)).to(device).to(dtype)
+    view = flat[offset:].view(rows, width)
+    assert (_run(view, k, device) == otopk.topk_selector_oracle(view.float().cpu().numpy(), k, order="index")).all()
+
+
+@pytest.mark.parametrize("width,k", [(300, 255), (700, 257), (1500, 1025), (4096, 4096), (8192, 513), (16000, 16000), (40000, 3000)])
+def test_value_order_around_the_chunks_of_the_sort(device, width, k):
+    rng = np.random.default_rng(k)
+    scores = np.round(rng.standard_normal((3, width)) * 50).astype(np.float32)       # many equal values: ties by index
+    assert (_run(to_dev(scores, device), k, device, order="value") == otopk.topk_selector_oracle(scores, k, order="value")).all()
