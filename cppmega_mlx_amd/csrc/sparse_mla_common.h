@@ -27,6 +27,8 @@ struct MlaParams {
   int num_splits;       // split-KV factor of the MFMA kernel
   int keys_per_split;
   int heads_per_wg;     // 0: 32-head tile kernel; 32 or 64: a producer/consumer kernel (sparse_mla_latent.hip, sparse_mla_rows16.hip)
+  int plan_level;       // how the launch is planned: see sparse_mla_mfma_plan_within
+  int rows16;           // with heads_per_wg: the kernel for 16-bit rows
   int tile_sharing;     // tile kernel on 16-bit rows: the 4 wavefronts take 4 head groups over one key stream
   float sm_scale;
   const float* sm_scale_dev;     // device copy of the softmax scale; read in place of sm_scale when set
@@ -61,6 +63,10 @@ int sparse_mla_mfma_launch(const MlaParams& p, hipStream_t stream);
 bool sparse_mla_mfma_supported(const MlaParams& p);
 size_t sparse_mla_mfma_workspace_bytes(const MlaParams& p);
 void sparse_mla_mfma_plan(MlaParams& p);
+// The plan for a caller who brings `have` bytes of workspace, and what it needs: the fastest one (level 0, what the
+// size query answers) if that fits, else key splits only until 256 workgroups are there and no copy of the cache
+// (level 1), else the kernel of sparse_mla_mfma.hip where it serves the shape (level 2).
+size_t sparse_mla_mfma_plan_within(MlaParams& p, size_t have);
 
 // partial values that a key split keeps of 32 heads: [4 groups of 128 channels][8 row pairs][64 lanes][8]
 constexpr int kMlaPartFloats = 4 * 16 * 64 * 4;
@@ -70,6 +76,7 @@ int sparse_mla_combine_f32(const MlaParams& p, hipStream_t stream);    // merges
 // max_keys each) with the least modelled time - whole rounds of 256 workgroups, each with its workgroups' start and end
 // and tile_us per tile of 32 keys, then, with several splits, the merging kernel and its traffic (partial_bytes per
 // workgroup, written and read).
+// At plan level 1: doubled until 256 workgroups are there.
 void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, double partial_bytes);
 
 // producer/consumer kernel for 16-bit rows (sparse_mla_rows16.hip); dispatched by the *_mfma_* functions
@@ -80,6 +87,7 @@ size_t sparse_mla_rows16_workspace_bytes(const MlaParams& p);
 
 // shared-tile kernel for FP8 latent caches (sparse_mla_latent.hip); dispatched by the *_mfma_* functions
 bool sparse_mla_latent_supported(const MlaParams& p);
+bool sparse_mla_latent_f32_partials(const MlaParams& p);
 void sparse_mla_latent_plan(MlaParams& p);
 int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream);   // includes its combine step
 size_t sparse_mla_latent_workspace_bytes(const MlaParams& p);

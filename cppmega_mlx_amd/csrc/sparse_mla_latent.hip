@@ -1020,11 +1020,21 @@ bool sparse_mla_latent_supported(const MlaParams& p) {
   return true;
 }
 
+bool sparse_mla_latent_f32_partials(const MlaParams& p) { return f32_partials(p); }
+
 void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, double partial_bytes) {
   // (fitted to 216 shapes of 16 and 128 heads, 1 .. 300 queries, 64 .. 2048 keys: 1.2x in the mean against doubling the
   // splits until 256 workgroups are there, 3x where that ended just above 256 or in splits of four tiles)
   constexpr double kUnitUs = 7.0, kMergeUs = 5.0, kBytesPerUs = 5e6;
   const int tiles = (p.topk + kTK - 1) / kTK;
+  if (p.plan_level > 0) {
+    int s = 1;
+    while (units * s < 256 && p.topk / (s * 2) >= 4 * kTK && s < 16) s *= 2;
+    while ((p.topk + s - 1) / s > max_keys && s < 16) s *= 2;
+    p.num_splits = s;
+    p.keys_per_split = (tiles + s - 1) / s * kTK;
+    return;
+  }
   double best = 0.0;
   p.num_splits = 0;
   for (int s = 1; s <= 16; ++s) {

@@ -6,8 +6,9 @@
 // bf16 rope tail, or a packed bf16 row of 576.  float16 queries with float16
 // rows of 576 run the same kernel on the float16 matrix instructions.
 // Everything else goes to the scalar kernel.  The producer/consumer kernels (sparse_mla_latent.hip,
-// sparse_mla_rows16.hip) come first wherever they can; this one keeps E8M0 rows, scale blocks of 64 channels, lists
-// beyond 32768 keys and caches whose rows need more than 32 bits of offset.
+// sparse_mla_rows16.hip) come first wherever they can; this one keeps scale blocks of 64 channels, lists beyond
+// 32768 keys, caches whose rows need more than 32 bits of offset, E8M0 rows of which few are selected, and callers whose
+// workspace the others do not fit.
 //
 // Decomposition
 //   workgroup = (batch*query, group of 32 heads, key split); 4 wavefronts.
@@ -835,8 +836,8 @@ __global__ __launch_bounds__(256) void sparse_mla_combine_kernel(const MlaParams
 
 }  // namespace
 
-bool sparse_mla_mfma_supported(const MlaParams& p) {
-  if (sparse_mla_latent_supported(p) || sparse_mla_rows16_supported(p)) return true;
+// what the kernel of this file takes
+static bool tile_kernel_supported(const MlaParams& p) {
   if (p.q_dtype == CPPMEGA_MI355_E4M3) {          // FP8 prepared buffers: rows of 576 codes, both sides scaled alike
     const bool tok = p.q_scale_kind == CPPMEGA_MI355_SCALE_PER_TOKEN && p.kv_scale_kind == CPPMEGA_MI355_SCALE_PER_TOKEN &&
                      (((uintptr_t)p.q_scale | (uintptr_t)p.kv_scale) & 3) == 0;
@@ -871,15 +872,31 @@ bool sparse_mla_mfma_supported(const MlaParams& p) {
   return true;
 }
 
+bool sparse_mla_mfma_supported(const MlaParams& p) {
+  return sparse_mla_latent_supported(p) || sparse_mla_rows16_supported(p) || tile_kernel_supported(p);
+}
+
+size_t sparse_mla_mfma_plan_within(MlaParams& p, size_t have) {
+  size_t need = 0;
+  for (p.plan_level = 0;; ++p.plan_level) {
+    sparse_mla_mfma_plan(p);
+    need = sparse_mla_mfma_workspace_bytes(p);
+    if (need <= have || p.plan_level == 2) return need;
+  }
+}
+
 // Chooses the key-split factor: enough workgroups to cover the 256 CUs, at least 64 keys per wavefront.
 void sparse_mla_mfma_plan(MlaParams& p) {
   p.heads_per_wg = 0;
+  p.rows16 = 0;
   p.tile_sharing = 0;
-  if (sparse_mla_latent_supported(p)) {
+  // (latent caches of more than 32 heads have had the one kernel only: what needs too much scratch there is refused)
+  const bool tiles_only = p.plan_level == 2 && tile_kernel_supported(p);
+  if (sparse_mla_latent_supported(p) && !(tiles_only && sparse_mla_latent_f32_partials(p))) {
     sparse_mla_latent_plan(p);
     return;
   }
-  if (sparse_mla_rows16_supported(p)) {
+  if (sparse_mla_rows16_supported(p) && !tiles_only) {
     sparse_mla_rows16_plan(p);
     return;
   }
@@ -899,13 +916,13 @@ void sparse_mla_mfma_plan(MlaParams& p) {
 }
 
 size_t sparse_mla_mfma_workspace_bytes(const MlaParams& p) {
-  if (p.heads_per_wg != 0) return p.kv_dtype == CPPMEGA_MI355_E4M3 ? sparse_mla_latent_workspace_bytes(p) : sparse_mla_rows16_workspace_bytes(p);
+  if (p.heads_per_wg != 0) return p.rows16 ? sparse_mla_rows16_workspace_bytes(p) : sparse_mla_latent_workspace_bytes(p);
   if (p.num_splits <= 1) return 0;
   return (size_t)p.B * p.S * p.H * p.num_splits * (kLat + 2) * sizeof(float);
 }
 
 int sparse_mla_mfma_launch(const MlaParams& p, hipStream_t stream) {
-  if (p.heads_per_wg != 0) return p.kv_dtype == CPPMEGA_MI355_E4M3 ? sparse_mla_latent_launch(p, stream) : sparse_mla_rows16_launch(p, stream);
+  if (p.heads_per_wg != 0) return p.rows16 ? sparse_mla_rows16_launch(p, stream) : sparse_mla_latent_launch(p, stream);
   const int groups_per_kv = (p.heads_per_group + kHeads - 1) / kHeads;
   const int units = p.tile_sharing ? (groups_per_kv + kWaves - 1) / kWaves : groups_per_kv;
   const dim3 grid((unsigned)((size_t)p.B * p.S * p.G * units), (unsigned)p.num_splits), block(kWaves * 64);

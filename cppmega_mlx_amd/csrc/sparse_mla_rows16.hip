@@ -1,13 +1,16 @@
 // Sparse MLA forward over 16-bit key rows on the matrix cores (gfx950), with the wavefronts of a
 // workgroup split into score producers and value consumers.
 //
-// Shapes served: bf16 or float16 queries of 576 = 512 latent + 64 rope channels over key rows of the same
+// Shapes served: queries and key rows of 576 e4m3 codes with one E8M0 byte per 32 channels, and bf16 or float16 queries of 576 = 512 latent + 64 rope channels over key rows of the same
 // type, packed (576) or as latent rows of 512 plus a rope tail of 64; d_v = 512.
+// A power of two times an e4m3 code is a bfloat16: E8M0 rows become bf16 rows in the workspace first (all of them, about
+// 6 us for 16384), the query's codes on their way to operand order, and nothing is rounded.
 //
 // Measured against the kernel of sparse_mla_mfma.hip, bf16: 64 queries x 16 heads x 64 keys 33 -> 7.8 us (the whole
 // call); 1000 queries x 2048 keys: 16 heads 573 -> 210 us, 64 heads 910 -> 304 us, 128 heads 953 -> 600 us (the
 // products at the rate of a large matrix product: 457 us).  Of 73 shapes (1 .. 1000 queries, 64 .. 2048 keys) none
-// was slower; 2.6x in the mean.  What is left: 1.0 us per tile at 64 heads, where the products of a SIMD are 1088
+// was slower; 2.6x in the mean.  E8M0 rows, 128 heads: 1500 x 2048 of 16384 1726 -> 890 us, 30 x 256 64 -> 25 us; 45 shapes
+// 2.4x in the mean.  What is left: 1.0 us per tile at 64 heads, where the products of a SIMD are 1088
 // clocks, and about 8 us for a workgroup's start and end, which nothing overlaps: the ring fills the LDS of the CU.
 //
 // Workgroup = (query, KV group, chunk of 32 HB heads, key split), 8 wavefronts, key tiles of 32 rows in a
@@ -89,7 +92,8 @@ __device__ __forceinline__ void mfma_o(f32x16& acc, const bf16x8& a, const bf16x
 }
 
 // HB: 32-head blocks of the chunk (1 or 2)
-template <bool F16, int HB>
+// Q_E8: the queries are e4m3 codes with E8M0 scales
+template <bool F16, int HB, bool Q_E8 = false>
 __global__ __launch_bounds__(512, 2) void sparse_mla_rows16_kernel(const MlaParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int kHeadsWg = 32 * HB;
@@ -197,7 +201,19 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_rows16_kernel(const MlaPara
     constexpr int kQPieces = kDqk / 8;              // 72 pieces of 16 bytes per head row
     constexpr int kQRows = 8 * HB;                  // rows of a producer
     constexpr int kQLoads = kQRows * kQPieces / 64; // 9 HB
-    u4 qload[kQLoads];
+    constexpr int kCodePieces = kDqk / 16;          // Q_E8: 36 pieces of 16 codes, two of them to a scale
+    constexpr int kCodeLoads = (kQRows * kCodePieces + 63) / 64;
+    u4 qload[Q_E8 ? kCodeLoads : kQLoads];
+    unsigned char qsc[kCodeLoads];
+    if constexpr (Q_E8) {
+#pragma unroll
+      for (int t = 0; t < kCodeLoads; ++t) {
+        const int P = min(lane + 64 * t, kQRows * kCodePieces - 1), hl = P / kCodePieces, piece = P - hl * kCodePieces, h = kQRows * role + hl;
+        const size_t row = bs * p.H + head0 + (h < heads_here ? h : 0);
+        qload[t] = *reinterpret_cast<const u4*>((const unsigned char*)p.q + row * kDqk + 16 * piece);
+        qsc[t] = ((const unsigned char*)p.q_scale)[row * (kDqk / 32) + (piece >> 1)];
+      }
+    } else
 #pragma unroll
     for (int t = 0; t < kQLoads; ++t) {
       const int P = lane + 64 * t, hl = P / kQPieces, piece = P - hl * kQPieces, h = kQRows * role + hl;
@@ -207,6 +223,16 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_rows16_kernel(const MlaPara
     __builtin_amdgcn_sched_barrier(0);
     stage_keys();
     unsigned char* qstage = smem + kLatSlot;        // (no tile is here before the first barrier of the pipeline)
+    if constexpr (Q_E8) {
+#pragma unroll
+      for (int t = 0; t < kCodeLoads; ++t) {
+        const int P = min(lane + 64 * t, kQRows * kCodePieces - 1), hl = P / kCodePieces, piece = P - hl * kCodePieces;
+        uint4 lo, hi;
+        dequant16<false>(make_uint4(qload[t][0], qload[t][1], qload[t][2], qload[t][3]), e8m0_to_f32(qsc[t]), lo, hi);
+        *reinterpret_cast<uint4*>(qstage + (kQRows * role + hl) * kQPitch + piece * 32) = lo;
+        *reinterpret_cast<uint4*>(qstage + (kQRows * role + hl) * kQPitch + piece * 32 + 16) = hi;
+      }
+    } else
 #pragma unroll
     for (int t = 0; t < kQLoads; ++t) {
       const int P = lane + 64 * t, hl = P / kQPieces, piece = P - hl * kQPieces;
@@ -550,11 +576,44 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_rows16_kernel(const MlaPara
   }
 }
 
+// rows of 576 e4m3 codes and 18 E8M0 bytes -> [B, Skv, G, 576] bf16: 16 codes per thread
+__global__ __launch_bounds__(256) void sparse_mla_e8m0_rows_kernel(const MlaParams p, unsigned short* out) {
+  constexpr unsigned kPieces = kDqk / 16;
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const size_t row = i / kPieces;
+  const unsigned piece = (unsigned)(i - row * kPieces);
+  if (row >= (size_t)p.B * p.Skv * p.G) return;
+  const size_t per_batch = (size_t)p.Skv * p.G, b = row / per_batch;
+  const size_t src = b * ((size_t)p.Skv_pitch * p.G) + (row - b * per_batch);
+  uint4 lo, hi;
+  dequant16<false>(*reinterpret_cast<const uint4*>((const unsigned char*)p.kv + src * kDqk + 16 * piece),
+                   e8m0_to_f32(((const unsigned char*)p.kv_scale)[src * (kDqk / 32) + (piece >> 1)]), lo, hi);
+  uint4* dst = reinterpret_cast<uint4*>(out + row * kDqk + 16 * piece);
+  dst[0] = lo;
+  dst[1] = hi;
+}
+
+bool e8m0_rows(const MlaParams& p) {
+  return p.q_dtype == CPPMEGA_MI355_E4M3 && p.kv_dtype == CPPMEGA_MI355_E4M3 && p.q_scale_kind == CPPMEGA_MI355_SCALE_E8M0 &&
+         p.kv_scale_kind == CPPMEGA_MI355_SCALE_E8M0 && p.q_scale_block == 32 && p.kv_scale_block == 32 && p.q_scale && p.kv_scale;
+}
+size_t e8m0_row_bytes(const MlaParams& p) { return e8m0_rows(p) ? ((size_t)p.B * p.Skv * p.G * kDqk * 2 + 255) & ~(size_t)255 : 0; }
+
+bool rows_of_16_bits(const MlaParams& p) {
+  if (e8m0_rows(p)) {
+    // every row of the cache is converted: where that is more than 65536 of them (25 us), the lists have to name as many
+    const long long rows = (long long)p.B * p.Skv * p.G;
+    return p.plan_level == 0 && p.d_kv == kDqk && p.rope_dim == 0 && (rows <= 65536 || rows <= (long long)p.B * p.S * p.G * p.topk);
+  }
+  if ((p.q_dtype != CPPMEGA_MI355_BF16 && p.q_dtype != CPPMEGA_MI355_F16) || p.kv_dtype != p.q_dtype) return false;
+  if (p.q_scale_kind != CPPMEGA_MI355_SCALE_NONE || p.kv_scale_kind != CPPMEGA_MI355_SCALE_NONE) return false;
+  return true;
+}
+
 }  // namespace
 
 bool sparse_mla_rows16_supported(const MlaParams& p) {
-  if ((p.q_dtype != CPPMEGA_MI355_BF16 && p.q_dtype != CPPMEGA_MI355_F16) || p.kv_dtype != p.q_dtype) return false;
-  if (p.q_scale_kind != CPPMEGA_MI355_SCALE_NONE || p.kv_scale_kind != CPPMEGA_MI355_SCALE_NONE) return false;
+  if (!rows_of_16_bits(p)) return false;
   if (p.d_qk != kDqk || p.d_v != kLat || p.d_kv + p.rope_dim != kDqk) return false;
   if (p.rope_dim != 0 && (p.rope_dim != kRope || p.rope_dtype != p.q_dtype)) return false;
   if (p.topk < 1 || (size_t)p.B * p.S == 0) return false;
@@ -565,19 +624,30 @@ bool sparse_mla_rows16_supported(const MlaParams& p) {
 }
 
 void sparse_mla_rows16_plan(MlaParams& p) {
+  p.rows16 = 1;
   p.heads_per_wg = p.heads_per_group <= 32 ? 32 : 64;
   const int chunks = (p.heads_per_group + p.heads_per_wg - 1) / p.heads_per_wg;
   const long long base = (long long)p.B * p.S * p.G * chunks;
   mla_key_splits(p, base, kMaxKeys, p.heads_per_wg == 64 ? 1.1 : 0.85, p.heads_per_wg * (double)kLat * 4);
 }
 
-int sparse_mla_rows16_launch(const MlaParams& p, hipStream_t stream) {
+int sparse_mla_rows16_launch(const MlaParams& args, hipStream_t stream) {
+  MlaParams p = args;
   const int chunks = (p.heads_per_group + p.heads_per_wg - 1) / p.heads_per_wg;
   const long long wgs = (long long)p.B * p.S * p.G * p.num_splits * chunks;
   if (wgs > 0x7fffffffll || p.keys_per_split > kMaxKeys || p.num_splits > 16)
     return fail(CPPMEGA_MI355_ERR_UNSUPPORTED, "sparse MLA: launch too large");
-  const bool f16 = p.q_dtype == CPPMEGA_MI355_F16;
-  void (*kernel)(MlaParams) = p.heads_per_wg == 64 ? (f16 ? sparse_mla_rows16_kernel<true, 2> : sparse_mla_rows16_kernel<false, 2>)
+  const bool f16 = p.q_dtype == CPPMEGA_MI355_F16, e8 = e8m0_rows(p);
+  if (e8) {
+    const size_t pieces = (size_t)p.B * p.Skv * p.G * (kDqk / 16);
+    hipLaunchKernelGGL(sparse_mla_e8m0_rows_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, args, (unsigned short*)args.workspace);
+    CM_HIP_CHECK(hipGetLastError());
+    p.kv = args.workspace;
+    p.Skv_pitch = p.Skv;
+    p.workspace = (char*)args.workspace + e8m0_row_bytes(args);
+  }
+  void (*kernel)(MlaParams) = e8 ? (p.heads_per_wg == 64 ? sparse_mla_rows16_kernel<false, 2, true> : sparse_mla_rows16_kernel<false, 1, true>)
+                            : p.heads_per_wg == 64 ? (f16 ? sparse_mla_rows16_kernel<true, 2> : sparse_mla_rows16_kernel<false, 2>)
                                                    : (f16 ? sparse_mla_rows16_kernel<true, 1> : sparse_mla_rows16_kernel<false, 1>);
   CM_HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kSmem));
   hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(512), kSmem, stream, p);
@@ -586,10 +656,10 @@ int sparse_mla_rows16_launch(const MlaParams& p, hipStream_t stream) {
 }
 
 size_t sparse_mla_rows16_workspace_bytes(const MlaParams& p) {
-  if (p.num_splits <= 1) return 0;
+  if (p.num_splits <= 1) return e8m0_row_bytes(p);
   const int chunks = (p.heads_per_group + p.heads_per_wg - 1) / p.heads_per_wg;
   const size_t blocks = (size_t)p.B * p.S * p.G * chunks * p.num_splits;
-  return blocks * (size_t)(p.heads_per_wg / 32 * kMlaPartFloats + p.heads_per_wg * 2) * sizeof(float);
+  return e8m0_row_bytes(p) + blocks * (size_t)(p.heads_per_wg / 32 * kMlaPartFloats + p.heads_per_wg * 2) * sizeof(float);
 }
 
 }  // namespace cm

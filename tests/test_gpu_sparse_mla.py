@@ -553,3 +553,58 @@ def test_score_only_entry_points(device):
         f8.fp8_sparse_mla_qk_reduce_path_c(to_dev(a, device), to_dev(a_s.reshape(1), device), to_dev(bm[:, :64].copy(), device), to_dev(b_s, device))
     with pytest.raises(TypeError):
         bs.blockscaled_sparse_mla_qk_reduce_path_c(to_dev(ac, device), to_dev(ab.reshape(-1).astype(np.float32), device), to_dev(bc, device), to_dev(bb, device))
+
+
+@pytest.mark.parametrize("rows", ["bf16", "per_token", "e8m0", "latent"])
+def test_less_workspace_than_asked_for_still_runs(device, rows):
+    """The size query answers for the fastest plan; a caller who brings nothing, or too little for it, gets another one."""
+    import ctypes as C
+
+    from cppmega_mlx_amd import _lib
+    rng = np.random.default_rng(5)
+    B, S, H, Skv, topk = 1, 260, 16, 900, 300
+    idx = sparse_indices(rng, B, S, 1, Skv, topk)
+    q_spec, kv_spec, rope = ops.QuantSpec(), ops.QuantSpec(), None
+    if rows == "bf16":
+        q, kv = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)).to(device).bfloat16() for s in ((B, S, H, 576), (B, Skv, 1, 576)))
+        qf, kf = q.float().cpu().numpy(), kv.float().cpu().numpy()
+    elif rows == "latent":
+        q, qf = bf16_pair(rng.standard_normal((B, S, H, 576)), device)
+        kv, scale, rope, kf = latent_cache(rng, B, Skv, 1, 512, 64, device, pow2=True)
+        kv_spec = ops.QuantSpec(_lib.SCALE_F32_BLOCK, scale, 128)
+    else:
+        quant, dequant, kind, block = (fp8.quantize_per_token, om.dequant_per_token, _lib.SCALE_PER_TOKEN, 0) if rows == "per_token" else (
+            fp8.quantize_mxfp8, om.dequant_e8m0, _lib.SCALE_E8M0, 32)
+        (q, qs), (kv, ks) = (quant(rng.standard_normal(s).astype(np.float32)) for s in ((B, S, H, 576), (B, Skv, 1, 576)))
+        qf, kf = dequant(q, qs), dequant(kv, ks)
+        q, qs, kv, ks = (to_dev(x, device) for x in (q, qs, kv, ks))
+        q_spec, kv_spec = (ops.QuantSpec(kind, s, block) if block else ops.QuantSpec(kind, s) for s in (qs, ks))
+    want_out, want_lse = om.sparse_mla_oracle(qf, kf, idx, sm_scale=0.04, d_v=512)
+    lib, indices = _lib.load(), to_dev(idx, device)
+    for part in (0.0, 0.5, 1.0):
+        out = torch.zeros((B, S, H, 512), dtype=torch.float32, device=device)
+        lse = torch.zeros((B, S, H), dtype=torch.float32, device=device)
+        a = ops._fill_mla_args(q, q_spec, kv, kv_spec, rope, indices, 0.04, 512, sinks=None, out=out, lse=lse, kernel="mfma")
+        need = C.c_size_t(0)
+        assert lib.cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK
+        workspace = torch.empty(max(int(need.value * part), 1), dtype=torch.uint8, device=device)
+        if part and need.value:
+            a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel()
+        assert lib.cppmega_mi355_sparse_mla_fwd(C.byref(a), C.sizeof(a), _lib.current_stream(device)) == _lib.OK, lib.cppmega_mi355_last_error()
+        torch.cuda.synchronize()
+        _assert_close(out, lse, want_out, want_lse, lse_tol=LSE_TOL_MFMA)
+
+
+def test_e8m0_rows_of_a_large_cache_with_few_selected(device):
+    """More than 65536 rows of which a list names few: they are not converted first."""
+    rng = np.random.default_rng(77)
+    S, H, Skv, topk = 2, 40, 70000, 130
+    qc, qb = fp8.quantize_mxfp8(rng.standard_normal((1, S, H, 576)).astype(np.float32))
+    kc, kb = fp8.quantize_mxfp8(rng.standard_normal((1, Skv, 1, 576)).astype(np.float32))
+    idx = sparse_indices(rng, 1, S, 1, Skv, topk)
+    out, lse = torch.zeros((1, S, H, 512), device=device), torch.zeros((1, S, H), device=device)
+    bs.sparse_mla_blockscaled_path_c_apply_direct(to_dev(qc, device), to_dev(qb, device), to_dev(kc, device), to_dev(kb, device),
+                                                  to_dev(idx, device), sm_scale=0.04, d_v=512, out=out, lse=lse, kernel="mfma")
+    torch.cuda.synchronize()
+    want_out, want_lse = om.sparse_mla_oracle(om.dequant_e8m0(qc, qb), om.dequant_e8m0(kc, kb), idx, sm_scale=0.04, d_v=512)
+    _assert_close(out, lse, want_out, want_lse)
