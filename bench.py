@@ -642,7 +642,7 @@ PROFILE_RUNS = {
 # summary file -> (trace run, (fetch run, write run) or None, SQ run or None, kernel-name fragments, workload text
 #                  [, grid size in threads: only dispatches of that size count])
 PROFILE_WORKLOADS = [
-    ("sparse_mla_decode", "trace_main", ("fetch_main", "write_main"), "sq_decode", ("sparse_mla_latent",),
+    ("sparse_mla_decode", "trace_main", ("fetch_main", "write_main"), "sq_decode", ("sparse_mla_latent_kernel<4", "sparse_mla_latent_combine"),
      "decode B=32 S_q=1 H=128 topk=2048 Skv=65536 (e4m3 latent + general fp32/128 scales (amax/448) + bf16 rope)"),
     ("sparse_mla_decode_pow2_scales", "trace_alt", None, None, ("sparse_mla_latent",),
      "decode B=32 S_q=1 H=128 topk=2048 Skv=65536 (e4m3 latent + power-of-two fp32/128 scales + bf16 rope)"),
@@ -660,13 +660,13 @@ PROFILE_WORKLOADS = [
      "W e4m3[7168,16384] + fp32 scale/128, x bf16[16,16384] (one kernel, no K split, no workspace)"),
     ("fp8_vecmat_m32", "trace_main", ("fetch_main", "write_main"), None, ("fp8_gemm_kernel<1, 1, 1, 4", "fp8_gemm_reduce"),
      "W e4m3[7168,16384] + fp32 scale/128, x bf16[32,16384] (32 x 128 tiles, split-K, and the reduce kernel)"),
-    ("topk_selector", "trace_main", ("fetch_main", "write_main"), None, ("topk_tile_kernel<float, 16, 4, 512, 0,",),
+    ("topk_selector", "trace_main", ("fetch_main", "write_main"), None, ("topk_tile_kernel<float, 16, 512, 0, false",),
      "scores fp32[4096 rows,8192] -> int32[4096,2048], indices in ascending order (the dispatches of 4096 workgroups only: "
      "the same kernel also selects for the indexer and for the prefill rows of the same run)", 4096 * 512),
-    ("topk_selector_value_order", "trace_alt", None, None, ("topk_tile_kernel<float, 16, 4, 512, 0,",),
-     "scores fp32[4096 rows,8192] -> int32[4096,2048], indices by descending value (same kernel, sorted in LDS)", 4096 * 512),
+    ("topk_selector_value_order", "trace_alt", None, None, ("topk_tile_kernel<float, 16, 512, 0, true",),
+     "scores fp32[4096 rows,8192] -> int32[4096,2048], indices by descending value (256 pairs per wavefront sorted in registers)", 4096 * 512),
     ("topk_selector_decode_shape", "trace_main", ("fetch_main", "write_main"), None,
-     ("topk_tile_kernel<float, 16, 4, 512, 1,", "topk_tile_kernel<float, 16, 4, 1024, 2,", "topk_wide_kernel"),
+     ("topk_tile_kernel<float, 16, 512, 1,", "topk_tile_kernel<float, 16, 1024, 2,", "topk_wide_kernel"),
      "scores fp32[32,65536] -> int32[32,2048]: the two-stage path (segment kernel, then candidate kernel) and, for "
      "comparison, the one-workgroup-per-row kernel; the indexer's decode row runs the two-stage kernels as well"),
     ("indexer_scores_topk", "trace_main", ("fetch_main", "write_main"), None, ("indexer_scores_kernel", "indexer_qw_"),
@@ -676,14 +676,14 @@ PROFILE_WORKLOADS = [
     ("kv_cache_append", "trace_main", ("fetch_main", "write_main"), None, ("cache_append_kernel",),
      "bf16 latent[B,S,1,512] + rope[..,64] -> e4m3 + fp32/128 scales + bf16 rope in the cache: one dispatch of 8192 rows "
      "(prefill chunk) and one of 32 rows (decode step) per step"),
-    ("sparse_mla_prefill_row_layouts", "trace_main", ("fetch_main", "write_main"), None, ("sparse_mla_mfma_kernel<",),
-     "sparse_mla_fwd q [1,8192,128,576], kv [1,8192,1,576], causal top-2048 indices -> [1,8192,128,512] on the 32-head tile kernel, "
-     "four wavefronts sharing one key stream: <false, true, true, 0> unquantised float16 rows, <true, false, true, 1> e4m3 rows "
-     "with per-token fp32 scales, <true, false, true, 2> e4m3 rows with E8M0 bytes per 32 channels"),
-    ("sparse_mla_backward", "trace_main", ("fetch_main", "write_main"), None, ("sparse_mla_bwd", "fill_zero_kernel"),
+    ("sparse_mla_prefill_row_layouts", "trace_main", ("fetch_main", "write_main"), None, ("sparse_mla_rows16_kernel<", "sparse_mla_e8m0_rows", "sparse_mla_latent_kernel<1, true"),
+     "sparse_mla_fwd q [1,8192,128,576], kv [1,8192,1,576], causal top-2048 indices -> [1,8192,128,512]: "
+     "rows16<true, 2, false> unquantised float16 rows, latent<1, true> e4m3 rows with per-token fp32 scales, "
+     "rows16<false, 2, true> (behind the conversion of the cache) e4m3 rows with E8M0 bytes per 32 channels"),
+    ("sparse_mla_backward", "trace_main", ("fetch_main", "write_main"), None, ("bwd_lists_kernel", "bwd_steps_kernel", "bwd_scores_kernel", "bwd_dq_kernel", "bwd_dkv_kernel", "bwd_sum_kernel"),
      "sparse_mla_bwd q bf16[1,1024,16,576], kv bf16[1,4096,1,576], d_out bf16[1,1024,16,512], topk 256 -> dq bf16, dkv f32 "
-     "(the dkv clear, then the matrix-core kernel with its float32 atomic adds)"),
-    ("dsa_indexer_loss", "trace_main", ("fetch_main", "write_main"), None, ("dsa_indexer_loss",),
+     "(keys by band, steps, scores, dq, dkv added in LDS, the sum of its shares)"),
+    ("dsa_indexer_loss", "trace_main", ("fetch_main", "write_main"), None, ("dsa_loss_", "dsa_indexer_loss"),
      "dsa_indexer_loss query / key bf16[4096,1,8,64], index_scores f32[1,4096,4096]: one dense and one sparse "
      "(topk_indices i32[1,4096,1024]) dispatch per step"),
     ("sparse_index_producers", "trace_main", ("fetch_main", "write_main"), None, ("_indices_",),

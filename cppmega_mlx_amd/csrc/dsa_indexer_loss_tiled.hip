@@ -4,11 +4,11 @@
 // softmaxes going through memory a row's keys are spread over workgroups, so that the causal triangle
 // fills the CUs evenly, and no wavefront waits for another one's reductions:
 //
-//   list_kernel    per row: membership bits of the index list, softmax statistics of the index scores
-//   tile_kernel<.., false>   per tile and head: max and sum of exp of the attention scores, per 64 keys
-//   merge_kernel   per (head, row): log2 of the softmax denominator over all its keys
-//   tile_kernel<.., true>    the scores again, p = mean over heads in registers, sum of p (log p - log q)
-//   sum_kernel     per row: the divergence summed over its 64-key chunks, in order
+//   dsa_loss_list_kernel    per row: membership bits of the index list, softmax statistics of the index scores
+//   dsa_loss_tile_kernel<.., false>   per tile and head: max and sum of exp of the attention scores, per 64 keys
+//   dsa_loss_merge_kernel   per (head, row): log2 of the softmax denominator over all its keys
+//   dsa_loss_tile_kernel<.., true>    the scores again, p = mean over heads in registers, sum of p (log p - log q)
+//   dsa_loss_sum_kernel     per row: the divergence summed over its 64-key chunks, in order
 //
 // In a tile a wavefront has 32 positions (columns of v_mfma_f32_32x32x16, one per lane) and 64 keys (rows);
 // the head's 64 + 128 rows pass through LDS, fetched one head ahead as whole 16-byte pieces.  The masks
@@ -63,7 +63,7 @@ __device__ __forceinline__ float exp2_(float x) { return __builtin_amdgcn_exp2f(
 __device__ __forceinline__ float log2_(float x) { return __builtin_amdgcn_logf(x); }
 
 // One wavefront per row.
-__global__ __launch_bounds__(kThreads) void list_kernel(const LossTiledParams p) {
+__global__ __launch_bounds__(kThreads) void dsa_loss_list_kernel(const LossTiledParams p) {
   extern __shared__ unsigned lds_bits[];
   const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
   const long long row = (long long)blockIdx.x * 4 + wave;
@@ -142,7 +142,7 @@ __host__ __device__ inline long long tiles_before(long long n, long long key_til
 // and enter the first pass as what its products start from, and the second pass leaves keys that do not count
 // out at its end.
 template <bool F16, int AD, bool SECOND, bool GENERAL>
-__global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void tile_kernel(const LossTiledParams p) {
+__global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void dsa_loss_tile_kernel(const LossTiledParams p) {
   constexpr int PIECES = AD / 8;                          // 16-byte pieces of a row of one head
   constexpr int PITCH = PIECES + 1;                       // odd: 16 rows of a piece fall on 16 bank groups
   constexpr int LOADS = (kQ + kK) * PIECES / kThreads;
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void tile_k
 }
 
 // 64 columns by 4 groups of chunks, met in LDS in order
-__global__ __launch_bounds__(kThreads) void merge_kernel(const LossTiledParams p) {
+__global__ __launch_bounds__(kThreads) void dsa_loss_merge_kernel(const LossTiledParams p) {
   __shared__ float2 met[4][64];
   const int lane = lane_id(), group = (int)(threadIdx.x >> 6);
   const long long i = (long long)blockIdx.x * 64 + lane;
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(const LossTiledParams p
   p.norm[i] = d > 0.0f ? m + log2_(d) : 0.0f;
 }
 
-__global__ __launch_bounds__(kThreads) void sum_kernel(const LossTiledParams p) {
+__global__ __launch_bounds__(kThreads) void dsa_loss_sum_kernel(const LossTiledParams p) {
   __shared__ float met[4][64];
   const int lane = lane_id(), group = (int)(threadIdx.x >> 6);
   const long long i = (long long)blockIdx.x * 64 + lane;
@@ -383,12 +383,12 @@ int run(LossTiledParams p, hipStream_t stream) {
     const dim3 grid((unsigned)(tiles_before((end + kQ - 1) / kQ, key_tiles) - tiles_before(p.slab0 / kQ, key_tiles)), (unsigned)p.AB), block(kThreads);
     const long long columns = (long long)p.AB * p.slab_rows / 64;
     const bool general = p.mask || !(p.scale2 > 0.0f);
-    if (general) hipLaunchKernelGGL((tile_kernel<F16, AD, false, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((tile_kernel<F16, AD, false, false>), grid, block, 0, stream, p);
-    hipLaunchKernelGGL(merge_kernel, dim3((unsigned)(columns * p.AH)), block, 0, stream, p);
-    if (general) hipLaunchKernelGGL((tile_kernel<F16, AD, true, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((tile_kernel<F16, AD, true, false>), grid, block, 0, stream, p);
-    hipLaunchKernelGGL(sum_kernel, dim3((unsigned)columns), block, 0, stream, p);
+    if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, false, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, false, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL(dsa_loss_merge_kernel, dim3((unsigned)(columns * p.AH)), block, 0, stream, p);
+    if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, true, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, true, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL(dsa_loss_sum_kernel, dim3((unsigned)columns), block, 0, stream, p);
   }
   CM_HIP_CHECK(hipGetLastError());
   return 0;
@@ -422,7 +422,7 @@ int dsa_indexer_loss_tiled_launch(const cppmega_mi355_dsa_loss_args_t& a, hipStr
   p.slab0 = 0; p.slab_rows = l.slab_rows;
   p.scale2 = a.softmax_scale * kLog2e;
   const size_t rows = (size_t)a.batch * a.seq_q;
-  hipLaunchKernelGGL(list_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads), a.topk_indices ? 16 * (size_t)l.words : 0, stream, p);
+  hipLaunchKernelGGL(dsa_loss_list_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads), a.topk_indices ? 16 * (size_t)l.words : 0, stream, p);
   CM_HIP_CHECK(hipGetLastError());
   if (a.range_event) CM_HIP_CHECK(hipEventRecord((hipEvent_t)a.range_event, stream));
   const bool f16 = a.in_dtype == CPPMEGA_MI355_F16;
