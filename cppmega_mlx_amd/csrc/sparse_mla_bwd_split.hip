@@ -340,7 +340,9 @@ __global__ __launch_bounds__(W * 64, 4) void bwd_scores_kernel(const SplitParams
       s[i][v] = key >= 0 ? sa[v] * scale2 : -INFINITY;
       m[v] = fmaxf(m[v], s[i][v]);
     }
-    dp[i] = da;
+    // (the slots behind a list's last key were fetched from row 0, which may hold anything)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) dp[i][v] = key >= 0 ? da[v] : 0.0f;
   }
   // statistics of head 4 * kg + v: over the row of 16 lanes, then over the wavefronts
 #pragma unroll

@@ -350,3 +350,21 @@ def test_backward_in_several_slabs_matches_its_halves(device):
         want_dq[:, half] = out
     assert torch.equal(dq, want_dq)
     assert (dkv - want_dkv).abs().max() <= 1e-5 * want_dkv.abs().max()
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("topk,D,d_v", [(17, 96, 64), (300, 576, 512), (1030, 64, 32)])
+def test_rows_that_no_list_names_may_hold_anything(device, topk, D, d_v, bad):
+    """Lists that are not whole steps of 16, some with skipped entries, over a cache whose first row is not finite."""
+    B, S, H, Skv = 1, 3, 16, 1100
+    rng = np.random.default_rng(topk)
+    q, kv, d_out = (to_dev(rng.standard_normal(s).astype(np.float32), device).bfloat16() for s in ((B, S, H, D), (B, Skv, 1, D), (B, S, H, d_v)))
+    idx = 1 + sparse_indices(rng, B, S, 1, Skv - 1, topk)
+    idx[:, 1:][rng.random(idx[:, 1:].shape) < 0.1] = -1
+    want = om.sparse_mla_bwd_oracle(q.double().cpu().numpy(), kv.double().cpu().numpy(), idx, d_out.double().cpu().numpy(), sm_scale=D ** -0.5, d_v=d_v)
+    kv[0, 0] = bad
+    dq, dkv = torch.empty((B, S, H, D), device=device), torch.empty((B, Skv, 1, D), device=device)
+    ops.sparse_mla_backward(q, kv, d_out, to_dev(idx.astype(np.int32), device), sm_scale=D ** -0.5, d_v=d_v, dq=dq, dkv=dkv)
+    for got, ref in zip((dq, dkv), want):
+        err, scale = error_report(got.cpu().numpy(), ref)
+        assert err <= 1e-4 * scale, (err, scale)
