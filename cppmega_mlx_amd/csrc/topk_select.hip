@@ -349,9 +349,10 @@ __global__ __launch_bounds__(THREADS, E > 16 ? 4 : 8) void topk_tile_kernel(cons
     zero_hist<THREADS>(hist, kHist2 ? kHist2 + kHistBins : kHistBins);
     const int c0 = tid * E;
     const bool any = c0 < end && c0 + E > start;          // (a run with nothing selectable is not read)
-    // The last piece of a row may reach up to three columns past it: into the row's padding or the next row, which is
-    // fine, but behind the last row there may be nothing.
-    const bool past = (T & 3) != 0 && MODE != 2 && row + 1 == p.rows && base + ((T + 3) & ~3) > p.row_stride;     // (uniform)
+    // The last piece of a row may reach up to three columns past it: into what lies in front of the next row or the next
+    // rows, which is fine, but the buffer may end with the last row's last column, whatever the pitch.
+    const bool past = (T & 3) != 0 && MODE != 2 &&
+                      (long long)row * p.row_stride + base + ((T + 3) & ~3) > (p.rows - 1) * p.row_stride + p.width;     // (uniform)
     if (!past) {
 #pragma unroll
       for (int i = 0; i < E / 4; ++i) {

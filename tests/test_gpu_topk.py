@@ -123,7 +123,7 @@ def test_public_entry_points(device):
     assert tk.topk_selector_path_c_status().available
 
 
-@pytest.mark.parametrize("rows,width,k", [(32, 65536, 2048), (3, 40000, 4000), (2, 24576, 8192), (5, 16388, 100)])
+@pytest.mark.parametrize("rows,width,k", [(32, 65536, 2048), (3, 40000, 4000), (2, 24576, 8192), (5, 16388, 100), (2, 30001, 2000)])
 def test_wide_rows_two_stage_and_single_workgroup_paths_agree_with_the_oracle(device, rows, width, k):
     """Rows wider than 16384 columns: k best of every 8192-column segment, then k of those.  Ties that
     straddle segments, bounds that empty whole segments, -inf and NaN entries."""
@@ -154,7 +154,9 @@ def test_wide_rows_two_stage_and_single_workgroup_paths_agree_with_the_oracle(de
     a.rows, a.width, a.row_stride, a.k = rows, width, width, k
     need = C.c_size_t(0)
     assert _lib.load().cppmega_mi355_topk_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK
-    assert (need.value > 0) == (width % 4 == 0 and width > 16384)
+    assert need.value > 0                                # two stages, whole 16-byte rows or not
+    a.width = a.row_stride = 16384
+    assert _lib.load().cppmega_mi355_topk_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK and need.value == 0
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
@@ -172,3 +174,27 @@ def test_value_order_around_the_chunks_of_the_sort(device, width, k):
     rng = np.random.default_rng(k)
     scores = np.round(rng.standard_normal((3, width)) * 50).astype(np.float32)       # many equal values: ties by index
     assert (_run(to_dev(scores, device), k, device, order="value") == otopk.topk_selector_oracle(scores, k, order="value")).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,width,pitch,k", [(3, 1023, 1024, 5), (2, 1022, 1031, 1022), (3, 8189, 8192, 300), (2, 16381, 16400, 900), (2, 20003, 20010, 77),
+                                                (3, 1, 5, 1), (4, 1, 1, 1), (5, 2, 2, 1), (2, 3, 4, 2)])
+def test_rows_with_a_pitch_whose_buffer_ends_with_the_last_row(device, rows, width, pitch, k, dtype):
+    """The right-hand columns of a wider matrix through the C interface: nothing lies behind the last row's last column."""
+    import ctypes as C
+    from cppmega_mlx_amd import _lib
+    rng = np.random.default_rng(width)
+    whole = torch.from_numpy(rng.standard_normal((rows, pitch)).astype(np.float32)).to(device).to(dtype)
+    view = whole[:, pitch - width:]
+    out = torch.full((rows, k), -7, dtype=torch.int32, device=device)
+    a = _lib.TopkArgs()
+    a.struct_size, a.score_dtype = C.sizeof(a), _lib.F32 if dtype is torch.float32 else _lib.BF16
+    a.scores, a.indices = view.data_ptr(), out.data_ptr()
+    a.rows, a.width, a.row_stride, a.k, a.order = rows, width, pitch, k, _lib.TOPK_ORDER_INDEX
+    need = C.c_size_t(0)
+    lib = _lib.load()
+    assert lib.cppmega_mi355_topk_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK
+    ws = torch.empty(max(need.value, 1), dtype=torch.uint8, device=device)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), need.value
+    assert lib.cppmega_mi355_topk_select(C.byref(a), C.sizeof(a), _lib.current_stream(view.device)) == _lib.OK
+    assert (out.cpu().numpy() == otopk.topk_selector_oracle(view.float().cpu().numpy(), k, order="index")).all()
