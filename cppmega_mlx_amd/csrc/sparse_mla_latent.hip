@@ -564,15 +564,15 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   __syncthreads();                                // keys[] is complete
   const int n_tiles = count_tiles();
   int spare_row = 0;
-  if (ROWS && n_tiles > 0) {
+  if (n_tiles > 0) {
     int m = -1;
     for (int w = 0; w < 8; ++w) m = max(m, last_valid[w]);
     spare_row = __builtin_amdgcn_readfirstlane(keys[m]);
   }
-  // HBM -> LDS.  A skipped key fetches cache row 0 (ROWS: its list's last valid row) instead (its probability is zero), so every
-  // tile is the same six load instructions per wavefront and the in-order load counter can be
-  // waited on by count.  The loads are inline assembly (the compiler would otherwise order every
-  // later LDS read behind them) with a uniform 64-bit base and a 32-bit byte offset per lane:
+  // HBM -> LDS.  A skipped key fetches its split's last valid row instead (its probability is zero, but a row that
+  // nobody selected may hold NaN or infinity), so every tile is the same six load instructions per wavefront and the
+  // in-order load counter can be waited on by count.  The loads are inline assembly (the compiler would otherwise order
+  // every later LDS read behind them) with a uniform 64-bit base and a 32-bit byte offset per lane:
   //   latent : block c of both sub-tiles, two planes each: lane (n, kg) of plane j fetches bytes
   //            128 c + 32 kg + 16 j .. + 15 of key 16 sj + n
   //   rope   : plane (sj = c / 2, s = c % 2): lane (n, kq) fetches bytes 64 s + 16 kq .. + 15 of the rope row
@@ -605,7 +605,7 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   auto dma_prepare = [&](int tau, unsigned slot_off) {
     dma_slot = smem_base + slot_off;
     const int* tk = keys + tau * kTK;
-    auto fetched = [&](int k) { return (unsigned)(ROWS ? (k >= 0 ? k : spare_row) : max(k, 0)); };
+    auto fetched = [&](int k) { return (unsigned)(k >= 0 ? k : spare_row); };
     const unsigned k0 = fetched(tk[lane & 15]), k1 = fetched(tk[16 + (lane & 15)]);   // this lane's key of sub-tile 0 / 1
     const unsigned ks = fetched(tk[sc_row]);
     off_l0 = __umul24(k0, lat_step) + lat_lane;

@@ -608,3 +608,34 @@ def test_e8m0_rows_of_a_large_cache_with_few_selected(device):
     torch.cuda.synchronize()
     want_out, want_lse = om.sparse_mla_oracle(om.dequant_e8m0(qc, qb), om.dequant_e8m0(kc, kb), idx, sm_scale=0.04, d_v=512)
     _assert_close(out, lse, want_out, want_lse)
+
+
+@pytest.mark.parametrize("H,topk", [(16, 33), (16, 300), (40, 70), (128, 1000)])
+@pytest.mark.parametrize("scales", ["block128", "block512", "row", "none"])
+def test_latent_rows_that_no_list_names_may_hold_anything(device, H, topk, scales):
+    """Ragged lists with skipped entries over a latent cache whose first row decodes to NaN and infinity."""
+    from cppmega_mlx_amd import _lib
+    B, S, Skv = 1, 2, 1200
+    rng = np.random.default_rng(topk + H)
+    q, qf = bf16_pair(rng.standard_normal((B, S, H, 576)), device)
+    block = {"block128": 128}.get(scales, 512)
+    codes, scale, rope, rows = latent_cache(rng, B, Skv, 1, 512, 64, device, pow2=False, block=block)
+    if scales == "none":
+        scale = torch.ones_like(scale)
+        rows = om.dequant_block_latent(codes.cpu().numpy(), scale.cpu().numpy(), rope.float().cpu().numpy(), block)
+    idx = 1 + sparse_indices(rng, B, S, 1, Skv - 1, topk)
+    idx[:, 1:][rng.random(idx[:, 1:].shape) < 0.1] = -1
+    sm = 576 ** -0.5 * (0.003 if scales == "none" else 1.0)        # (unscaled codes go up to 448)
+    want_out, want_lse = om.sparse_mla_oracle(qf, rows, idx, sm_scale=sm, d_v=512)
+    codes[0, 0], rope[0, 0] = 0x7f, float("nan")
+    scale[0, 0] = float("inf")
+    if scales == "row":
+        spec = ops.QuantSpec(_lib.SCALE_PER_TOKEN, scale.view(B, Skv, 1), 0)
+    else:
+        spec = ops.QuantSpec() if scales == "none" else ops.QuantSpec(_lib.SCALE_F32_BLOCK, scale, block)
+    out = torch.zeros((B, S, H, 512), dtype=torch.float32, device=device)
+    lse = torch.zeros((B, S, H), dtype=torch.float32, device=device)
+    ops.sparse_mla_forward(q, codes, to_dev(idx.astype(np.int32), device), sm_scale=sm, d_v=512, out=out, lse=lse, kv_spec=spec, kv_rope=rope, kernel="mfma")
+    assert torch.isfinite(out).all()
+    err, ref = error_report(out.cpu().numpy(), want_out)
+    assert err <= REL_TOL * ref and np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_TOL_MFMA
