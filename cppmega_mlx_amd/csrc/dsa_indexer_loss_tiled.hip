@@ -139,8 +139,8 @@ __host__ __device__ inline long long tiles_before(long long n, long long key_til
 }
 
 // GENERAL: an additive mask is given, or the softmax scale is not positive.  Otherwise the masks are 0 or -inf
-// and enter the first pass as what its products start from, and the second pass leaves keys that do not count
-// out at its end.
+// and enter the first pass as what its products start from (a select behind them where a row that does not count
+// turned out not to be finite), and the second pass leaves keys that do not count out at its end.
 template <bool F16, int AD, bool SECOND, bool GENERAL>
 __global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void dsa_loss_tile_kernel(const LossTiledParams p) {
   constexpr int PIECES = AD / 8;                          // 16-byte pieces of a row of one head
@@ -187,6 +187,7 @@ __global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void dsa_lo
       if (GENERAL && p.mask && add[t][v] == 0.0f) {
         const float x = p.mask[row * (size_t)p.Sk + key0 + off];
         add[t][v] = x > -INFINITY ? x * kLog2e : -INFINITY;
+        if (!(x > -INFINITY)) counts[t] &= ~(1u << off);
       }
     }
   }
@@ -242,7 +243,7 @@ __global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void dsa_lo
       for (int t = 0; t < 2; ++t) s[t] = product<F16>(rows[(kQ + wk + t * 32 + l32) * PITCH + 2 * k + half], qf, s[t]);
     }
     // (exponentials first, sums behind them: a sum right behind its exponential waits for it)
-    if (SECOND) {
+    if constexpr (SECOND) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
 #pragma unroll
@@ -251,29 +252,53 @@ __global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void dsa_lo
         for (int v = 0; v < 16; ++v) mean[t][v] += s[t][v];
       }
     } else {
-      float m = -INFINITY;
+      float m, sum;
+      auto statistics = [&]() {
+        m = -INFINITY;
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          if (GENERAL) s[t][v] = fmaf(s[t][v], p.scale2, add[t][v]);
-          m = fmaxf(m, s[t][v]);
+          for (int v = 0; v < 16; ++v) {
+            if (GENERAL) s[t][v] = add[t][v] > -INFINITY ? fmaf(s[t][v], p.scale2, add[t][v]) : -INFINITY;
+            m = fmaxf(m, s[t][v]);
+          }
+        m = fmaxf(m, xor32(m));
+        if (!GENERAL) m *= p.scale2;
+        const float at = m > -INFINITY ? m : 0.0f;
+        float d[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) s[t][v] = exp2_(GENERAL ? s[t][v] - at : fmaf(s[t][v], p.scale2, -at));
+#pragma unroll
+          for (int v = 0; v < 16; ++v) d[v & 3] += s[t][v];
         }
-      m = fmaxf(m, xor32(m));
-      if (!GENERAL) m *= p.scale2;
-      const float at = m > -INFINITY ? m : 0.0f;
-      float d[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        sum = (d[0] + d[1]) + (d[2] + d[3]);
+        sum += xor32(sum);
+      };
+      statistics();
+      // -inf + x is NaN where x is not finite: the row of a key that does not count holds such values, or a row that
+      // counts does.  Only then the masks are applied behind the products.
+      if (!GENERAL && __ballot(!(sum == sum)) != 0ull) {
+        asm volatile("" ::: "memory");                    // (the operands are read again: kept from above, they would not fit)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) s[t][v] = exp2_(GENERAL ? s[t][v] - at : fmaf(s[t][v], p.scale2, -at));
+          for (int v = 0; v < 16; ++v) s[t][v] = 0.0f;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) d[v & 3] += s[t][v];
+        for (int k = 0; k < STEPS; ++k) {
+          const u32x4 qf = rows[(wq + l32) * PITCH + 2 * k + half];
+#pragma unroll
+          for (int t = 0; t < 2; ++t) s[t] = product<F16>(rows[(kQ + wk + t * 32 + l32) * PITCH + 2 * k + half], qf, s[t]);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) s[t][v] = add[t][v] == 0.0f ? s[t][v] : -INFINITY;
+        statistics();
       }
-      d[0] = (d[0] + d[1]) + (d[2] + d[3]);
-      d[0] += xor32(d[0]);
       if (half == 0 && my_q - p.slab0 < p.slab_rows && live_q)
-        p.part[((size_t)(kw / kChunk) * p.AB * p.AH + (size_t)b * p.AH + h) * p.slab_rows + (my_q - p.slab0)] = make_float2(m, d[0]);
+        p.part[((size_t)(kw / kChunk) * p.AB * p.AH + (size_t)b * p.AH + h) * p.slab_rows + (my_q - p.slab0)] = make_float2(m, sum);
     }
   }
   if (!SECOND || !busy) return;

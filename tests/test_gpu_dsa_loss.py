@@ -195,3 +195,36 @@ def test_tiled_kernels_agree_with_the_kernel_without_a_workspace(shape):
     a.seq_q, a.batch, a.heads, a.head_dim, a.seq_k = ASq, AB, AH, AD, Sk
     assert _lib.load().cppmega_mi355_dsa_indexer_loss(C.byref(a), a.struct_size, _lib.current_stream(q.device)) == 0
     torch.testing.assert_close(got, want, atol=2e-5, rtol=2e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["list", "mask", "dense"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+def test_key_rows_that_do_not_count_may_hold_anything(form, bad, dt):
+    """Keys that no position attends to (behind the last position, on no list, masked) and keys that only the positions in
+    front of them name are not finite; the tiles they share with keys that count give what finite rows give."""
+    from cppmega_mlx_amd import ops
+    ASq, AB, AH, AD, Sk, topk = 150, 1, 2, 64 if form == "list" else 96, 203, 40       # (short dense rows of 64 take another kernel)
+    q, k, idx, top = _case(77, ASq, AB, AH, AD, Sk, topk, DTYPES[dt])
+    broken = torch.zeros(Sk, dtype=torch.bool)
+    broken[ASq:] = True                                   # behind the last position
+    if form != "dense":
+        broken[[3, 70, 100]] = True                       # masked where a position could see them
+    mask = None
+    if form == "list":
+        visible = torch.arange(Sk)[None, :] <= torch.arange(ASq)[:, None]
+        top[0] = (torch.rand((ASq, Sk), generator=torch.Generator().manual_seed(1)) - 2.0 * (visible & broken)).topk(topk, dim=-1).indices
+    elif form == "mask":
+        mask = torch.randn((AB, ASq, Sk), generator=torch.Generator().manual_seed(2))
+        mask[:, :, broken] = float("-inf")
+    kb = k.clone()
+    kb[broken] = bad
+    out = torch.empty((AB, ASq), device="cuda")
+    ops.dsa_indexer_loss(q.cuda(), kb.cuda(), idx.cuda(), softmax_scale=AD ** -0.5, out=out, index_mask=None if mask is None else mask.cuda(),
+                         topk_indices=top.cuda() if form == "list" else None)
+    if mask is None:
+        want = _want(q, k, idx, top, AD ** -0.5, form == "list")
+    else:
+        want = od.dsa_indexer_loss_per_position(idx.numpy(), q.float().numpy(), k.float().numpy(), softmax_scale=AD ** -0.5, index_mask=mask.numpy())
+    np.testing.assert_allclose(out.cpu().numpy(), want, atol=2e-5, rtol=2e-4)
