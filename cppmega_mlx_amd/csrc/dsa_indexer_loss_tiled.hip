@@ -48,6 +48,7 @@ struct LossTiledParams {
   float* norm;               // [AB * AH][slab rows]: log2 of the attention softmax's denominator, max included
   float* kl;                 // [chunks][AB][slab rows]
   int* range_flag;           // set to 1 when a list holds an index outside [0, Sk); or NULL
+  unsigned char* outside;    // with range_flag: [rows, in whole workgroups of the list kernel], whether a row's list holds such an index
   int topk, index_dtype, words;
   int ASq, AB, AH, Sk;
   int slab0, slab_rows;      // positions of this slab
@@ -73,8 +74,8 @@ __global__ __launch_bounds__(kThreads) void dsa_loss_list_kernel(const LossTiled
   if (sparse) {
     for (int w = lane; w < p.words; w += 64) bits[w] = 0u;
     __syncthreads();
+    bool outside = false;
     if (live) {
-      bool outside = false;
       for (int t = lane; t < p.topk; t += 64) {
         const size_t at = (size_t)row * p.topk + t;
         const long long c = p.index_dtype == CPPMEGA_MI355_I64 ? static_cast<const long long*>(p.topk_idx)[at]
@@ -84,6 +85,8 @@ __global__ __launch_bounds__(kThreads) void dsa_loss_list_kernel(const LossTiled
       }
       if (outside && p.range_flag) *p.range_flag = 1;
     }
+    const bool any = __ballot(outside) != 0ull;
+    if (p.outside && lane == 0) p.outside[row] = any;
     __syncthreads();
     if (live)
       for (int w = lane; w < p.words; w += 64) p.bits[(size_t)row * p.words + w] = bits[w];
@@ -373,11 +376,15 @@ __global__ __launch_bounds__(kThreads) void dsa_loss_sum_kernel(const LossTiledP
 #pragma unroll 4
   for (int c = group; c < chunks; c += 4) kl += p.kl[(size_t)c * total + i];
   met[group][lane] = kl;
-  __syncthreads();
+  // the caller is told of an index outside the range, and finds the losses as they were
+  int outside = 0;
+  if (p.outside)
+    for (long long w = threadIdx.x; w < ((long long)p.AB * p.ASq + 3) / 4; w += kThreads) outside |= reinterpret_cast<const int*>(p.outside)[w];
+  if (__syncthreads_or(outside)) return;
   if (!group && q < p.ASq) p.loss[(i / p.slab_rows) * p.ASq + q] = (met[0][lane] + met[1][lane]) + (met[2][lane] + met[3][lane]);
 }
 
-struct Layout { size_t bits, index_norm, part, norm, kl, bytes; int words, chunks, slab_rows; };
+struct Layout { size_t bits, outside, index_norm, part, norm, kl, bytes; int words, chunks, slab_rows; };
 
 Layout layout(const cppmega_mi355_dsa_loss_args_t& a) {
   Layout l;
@@ -393,6 +400,7 @@ Layout layout(const cppmega_mi355_dsa_loss_args_t& a) {
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t here = at; at += (bytes + 255) & ~(size_t)255; return here; };
   l.bits = take(a.topk_indices ? rows * l.words * 4 : 0);
+  l.outside = take(a.topk_indices ? (rows + 3) / 4 * 4 : 0);
   l.index_norm = take(rows * 4);
   l.part = take(per_row * l.slab_rows);
   l.norm = take(heads * l.slab_rows * 4);
@@ -442,6 +450,7 @@ int dsa_indexer_loss_tiled_launch(const cppmega_mi355_dsa_loss_args_t& a, hipStr
   p.part = reinterpret_cast<float2*>(ws + l.part); p.norm = reinterpret_cast<float*>(ws + l.norm);
   p.kl = reinterpret_cast<float*>(ws + l.kl);
   p.range_flag = a.range_flag;
+  p.outside = a.range_flag && a.topk_indices ? reinterpret_cast<unsigned char*>(ws + l.outside) : nullptr;
   p.topk = a.topk; p.index_dtype = a.index_dtype; p.words = l.words;
   p.ASq = a.seq_q; p.AB = a.batch; p.AH = a.heads; p.Sk = a.seq_k;
   p.slab0 = 0; p.slab_rows = l.slab_rows;

@@ -269,8 +269,8 @@ def dsa_indexer_loss(query: torch.Tensor, key: torch.Tensor, index_scores: torch
     """Per-position KL(attention || index) into caller-owned float32 ``out`` [AB, ASq];
     ``query`` [ASq, AB, AH, AD], ``key`` [Sk, AB, AH, AD], ``index_scores`` / ``index_mask`` float32 [AB, ASq, Sk];
     ``topk_indices`` int32 / int64 [AB, ASq, topk] restricts both distributions to the listed keys.
-    ``check_range`` raises :class:`IndexRangeError` when a list holds an index outside [0, Sk): the host waits for the
-    kernel that reads the lists, not for the loss."""
+    ``check_range`` raises :class:`IndexRangeError` when a list holds an index outside [0, Sk), and ``out`` stays as it
+    was: the host waits for the kernel that reads the lists, not for the loss."""
     for name, t in (("query", query), ("key", key), ("index_scores", index_scores), ("out", out), ("index_mask", index_mask),
                     ("topk_indices", topk_indices)):
         if t is not None:

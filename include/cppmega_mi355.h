@@ -376,8 +376,8 @@ typedef struct cppmega_mi355_dsa_loss_args {
   /* Optional (callers built against the first layout end here): *_workspace_bytes of scratch switches
    * 16-bit rows to the tiled kernels, the same result several times faster.  With it, an entry of
    * topk_indices outside [0, Sk) also sets *range_flag (device or pinned host memory the caller has
-   * cleared) to 1, and range_event (a hipEvent_t) is recorded on the stream behind the kernel that
-   * reads the lists, in front of the others. */
+   * cleared) to 1 and, where range_flag is given, leaves loss as it was; range_event (a hipEvent_t) is
+   * recorded on the stream behind the kernel that reads the lists, in front of the others. */
   void* workspace;
   size_t workspace_bytes;
   int32_t* range_flag;

@@ -228,3 +228,19 @@ def test_key_rows_that_do_not_count_may_hold_anything(form, bad, dt):
     else:
         want = od.dsa_indexer_loss_per_position(idx.numpy(), q.float().numpy(), k.float().numpy(), softmax_scale=AD ** -0.5, index_mask=mask.numpy())
     np.testing.assert_allclose(out.cpu().numpy(), want, atol=2e-5, rtol=2e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("at", [(0, 0), (1, 149), (1, 70)])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_lists_out_of_range_leave_the_output_as_it_was(dt, at):
+    q, k, idx, top = (t.cuda() for t in _case(8, 150, 2, 4, 64, 150, 20, DTYPES[dt]))
+    out = torch.full((2, 150), 5.0, device="cuda")
+    bad = top.clone()
+    bad[at[0], at[1], 3] = 150
+    with pytest.raises(ValueError, match="out of range"):
+        dsa_splitk_indexer_loss_per_position(idx, bad, q, k, 0.125, True, out=out)
+    torch.cuda.synchronize()
+    assert (out == 5.0).all()
+    dsa_splitk_indexer_loss_per_position(idx, top, q, k, 0.125, True, out=out)       # (and the next call is not held up)
+    assert not (out == 5.0).any()
