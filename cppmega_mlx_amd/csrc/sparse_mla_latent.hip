@@ -33,9 +33,10 @@
 //   pipeline  iteration t: barrier; producers: scores and P of tile t+1; consumers: issue tile
 //             t+4, value product of tile t.  One barrier per tile.
 //
-// Key splits write their accumulators (rounded to bf16; in fp32 for code rows and for up to 32 heads) to the
-// workspace as the lanes hold them plus (max, sum) per head; sparse_mla_latent_combine_kernel merges them and does the transposition
-// to [head][channel] that the single-split path does in LDS.
+// Key splits write their accumulators (in fp32 for code rows, for up to 32 heads and where a launch is split
+// further than 256 workgroups ask for, else rounded to bf16) to the workspace as the lanes hold them plus (max, sum)
+// per head; sparse_mla_latent_combine_kernel merges them and does the transposition to [head][channel] that the
+// single-split path does in LDS.
 
 #include <type_traits>
 
@@ -151,9 +152,6 @@ __device__ __forceinline__ int split_q32(const uint4 (&x)[4], i32x8& hi, i32x8& 
   }
   return e;
 }
-
-// Key splits of these keep float32: code rows and single groups of heads have few enough of them.
-__host__ __device__ __forceinline__ bool f32_partials(const MlaParams& p) { return p.q_dtype == CPPMEGA_MI355_E4M3 || p.heads_per_group <= 32; }
 
 // NBLK: fp32 scales per key row (1, 2 or 4).
 // ROWS: key rows and queries of 576 e4m3 codes with one fp32 scale each (NBLK = 1).  The query's codes are the
@@ -759,11 +757,11 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     const float l_all = stats[((2 * hb + (hd >> 4)) * 16 + (hd & 15)) * 2 + 1];
     const int h_local = 32 * hb + hd;
     if (!direct) {
-      // key split: the unnormalised accumulators leave exactly as the lanes hold them (rounded to
-      // bf16: the values are relative to the split's own maximum, so their range is that of the
+      // key split: the unnormalised accumulators leave exactly as the lanes hold them (where they are
+      // rounded to bf16: the values are relative to the split's own maximum, so their range is that of the
       // output times the split's probability mass)
       // (two accumulator rows of a lane per 16-byte store: [consumer][head half][dvb][row pair][lane][8])
-      if (f32_partials(p)) {                        // (uniform)
+      if (p.f32_partials) {                        // (uniform)
         float* blk = (float*)p.workspace + part_block * (size_t)(2 * kPartFloats) + ((size_t)((role * 2 + hb) * 8) * 64 + lane) * 8;
 #pragma unroll
         for (int dvb = 0; dvb < 4; ++dvb)
@@ -1020,19 +1018,20 @@ bool sparse_mla_latent_supported(const MlaParams& p) {
   return true;
 }
 
-bool sparse_mla_latent_f32_partials(const MlaParams& p) { return f32_partials(p); }
+bool sparse_mla_latent_only(const MlaParams& p) { return latent_rows(p) && p.heads_per_group > 32; }
 
-void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, double partial_bytes) {
+void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, int heads, bool narrow) {
   // (fitted to 216 shapes of 16 and 128 heads, 1 .. 300 queries, 64 .. 2048 keys: 1.2x in the mean against doubling the
   // splits until 256 workgroups are there, 3x where that ended just above 256 or in splits of four tiles)
   constexpr double kUnitUs = 7.0, kMergeUs = 5.0, kBytesPerUs = 5e6;
   const int tiles = (p.topk + kTK - 1) / kTK;
+  int doubled = 1;
+  while (units * doubled < 256 && p.topk / (doubled * 2) >= 4 * kTK && doubled < 16) doubled *= 2;
+  while ((p.topk + doubled - 1) / doubled > max_keys && doubled < 16) doubled *= 2;
   if (p.plan_level > 0) {
-    int s = 1;
-    while (units * s < 256 && p.topk / (s * 2) >= 4 * kTK && s < 16) s *= 2;
-    while ((p.topk + s - 1) / s > max_keys && s < 16) s *= 2;
-    p.num_splits = s;
-    p.keys_per_split = (tiles + s - 1) / s * kTK;
+    p.num_splits = doubled;
+    p.keys_per_split = (tiles + doubled - 1) / doubled * kTK;
+    p.f32_partials = !narrow;
     return;
   }
   double best = 0.0;
@@ -1040,27 +1039,29 @@ void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us,
   for (int s = 1; s <= 16; ++s) {
     const int per = (tiles + s - 1) / s;
     if (per * kTK > max_keys || (s > 1 && (per < 2 || per == (tiles + s - 2) / (s - 1)))) continue;
-    const double wgs = (double)units * s;
+    const bool f32 = !narrow || s > doubled;
     double us = (double)((units * s + 255) / 256) * (kUnitUs + per * tile_us);
-    if (s > 1) us += kMergeUs + 2.0 * wgs * partial_bytes / kBytesPerUs;
+    if (s > 1) us += kMergeUs + 2.0 * (double)units * s * heads * kLat * (f32 ? 4 : 2) / kBytesPerUs;
     if (p.num_splits == 0 || us < best) {
       best = us;
       p.num_splits = s;
       p.keys_per_split = per * kTK;
+      p.f32_partials = f32;
     }
   }
 }
 
 void sparse_mla_latent_plan(MlaParams& p) {
   const int chunks = (p.heads_per_group + kHeadsWg - 1) / kHeadsWg;
-  const long long base = (long long)p.B * p.S * p.G * chunks;
   p.heads_per_wg = kHeadsWg;
-  mla_key_splits(p, base, kMaxKeys, 1.1, kHeadsWg * (double)kLat * (f32_partials(p) ? 4 : 2));
+  const long long base = (long long)p.B * p.S * p.G * chunks;
+  mla_key_splits(p, base, kMaxKeys, 1.1, kHeadsWg, sparse_mla_latent_only(p));
   // a decode step of a batch too large for the fixed scratch of the entry point without allocations is refused there,
   // and stays so: one split would need no scratch at all (96 sequences x 128 heads x 2048 keys: 85 us instead of 104)
-  if (p.S == 1 && p.num_splits == 1 && base > 128 && base < 256 && !f32_partials(p) && p.topk >= 8 * kTK) {
+  if (p.S == 1 && p.num_splits == 1 && base > 128 && base < 256 && sparse_mla_latent_only(p) && p.topk >= 8 * kTK) {
     p.num_splits = 2;
     p.keys_per_split = ((p.topk + kTK - 1) / kTK + 1) / 2 * kTK;
+    p.f32_partials = 0;
   }
 }
 
@@ -1085,7 +1086,7 @@ int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream) {
 #undef CM_LAUNCH_PC
   CM_HIP_CHECK(hipGetLastError());
   if (p.num_splits > 1) {
-    if (f32_partials(p)) return sparse_mla_combine_f32(p, stream);
+    if (p.f32_partials) return sparse_mla_combine_f32(p, stream);
     const dim3 cgrid((unsigned)((size_t)p.B * p.S * p.G * chunks), (unsigned)(4 * (kHeadsWg / 32)));
     hipLaunchKernelGGL((sparse_mla_latent_combine_kernel<false, 2>), cgrid, dim3(256), 0, stream, p);
     CM_HIP_CHECK(hipGetLastError());
@@ -1106,7 +1107,7 @@ size_t sparse_mla_latent_workspace_bytes(const MlaParams& p) {
   if (p.num_splits <= 1) return 0;
   const int chunks = (p.heads_per_group + kHeadsWg - 1) / kHeadsWg;
   const size_t blocks = (size_t)p.B * p.S * p.G * chunks * p.num_splits;
-  return blocks * ((size_t)2 * kPartFloats * (f32_partials(p) ? sizeof(float) : sizeof(unsigned short)) + kHeadsWg * 2 * sizeof(float));
+  return blocks * ((size_t)2 * kPartFloats * (p.f32_partials ? sizeof(float) : sizeof(unsigned short)) + kHeadsWg * 2 * sizeof(float));
 }
 
 }  // namespace cm

@@ -892,7 +892,7 @@ void sparse_mla_mfma_plan(MlaParams& p) {
   p.tile_sharing = 0;
   // (latent caches of more than 32 heads have had the one kernel only: what needs too much scratch there is refused)
   const bool tiles_only = p.plan_level == 2 && tile_kernel_supported(p);
-  if (sparse_mla_latent_supported(p) && !(tiles_only && sparse_mla_latent_f32_partials(p))) {
+  if (sparse_mla_latent_supported(p) && !(tiles_only && !sparse_mla_latent_only(p))) {
     sparse_mla_latent_plan(p);
     return;
   }

@@ -628,7 +628,7 @@ void sparse_mla_rows16_plan(MlaParams& p) {
   p.heads_per_wg = p.heads_per_group <= 32 ? 32 : 64;
   const int chunks = (p.heads_per_group + p.heads_per_wg - 1) / p.heads_per_wg;
   const long long base = (long long)p.B * p.S * p.G * chunks;
-  mla_key_splits(p, base, kMaxKeys, p.heads_per_wg == 64 ? 1.1 : 0.85, p.heads_per_wg * (double)kLat * 4);
+  mla_key_splits(p, base, kMaxKeys, p.heads_per_wg == 64 ? 1.1 : 0.85, p.heads_per_wg, false);
 }
 
 int sparse_mla_rows16_launch(const MlaParams& args, hipStream_t stream) {

@@ -227,3 +227,22 @@ def test_kernel_choice_and_workspace_for_the_latent_cache_layout():
     assert lib.cppmega_mi355_sparse_mla_select_kernel(C.byref(a), C.sizeof(a)) == _lib.MLA_KERNEL_MFMA
     assert lib.cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0
     assert need.value == 2 * 16 * (64 * 512 * 2 + 64 * 2 * 4)
+
+
+@pytest.mark.parametrize("batch,heads,topk,splits,value_bytes", [
+    (1, 128, 2048, 16, 2), (32, 128, 2048, 4, 2), (64, 128, 2048, 2, 2),        # doubled until 256 workgroups are there, or less often
+    (1, 128, 1024, 16, 4), (1, 64, 512, 8, 4), (1, 128, 256, 4, 4),             # split further: float32 sums
+    (1, 16, 2048, 16, 4),                                                       # up to 32 heads: float32 sums
+])
+def test_key_splits_that_doubling_would_not_make_keep_float32_sums(batch, heads, topk, splits, value_bytes):
+    need = C.c_size_t(0)
+    a = _latent_mla_args(batch=batch, heads=heads, topk=topk)
+    assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0
+    assert need.value == batch * ((heads + 63) // 64) * splits * (64 * 512 * value_bytes + 64 * 2 * 4)
+
+
+@pytest.mark.parametrize("queries,heads", [(129, 128), (192, 128), (257, 64), (384, 64)])
+def test_latent_launches_that_fit_without_splits_stay_in_one_piece(queries, heads):
+    need = C.c_size_t(1)
+    a = _latent_mla_args(batch=1, seq_q=queries, heads=heads)
+    assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0 and need.value == 0
