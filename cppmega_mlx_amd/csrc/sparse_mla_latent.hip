@@ -1054,15 +1054,7 @@ void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us,
 void sparse_mla_latent_plan(MlaParams& p) {
   const int chunks = (p.heads_per_group + kHeadsWg - 1) / kHeadsWg;
   p.heads_per_wg = kHeadsWg;
-  const long long base = (long long)p.B * p.S * p.G * chunks;
-  mla_key_splits(p, base, kMaxKeys, 1.1, kHeadsWg, sparse_mla_latent_only(p));
-  // a decode step of a batch too large for the fixed scratch of the entry point without allocations is refused there,
-  // and stays so: one split would need no scratch at all (96 sequences x 128 heads x 2048 keys: 85 us instead of 104)
-  if (p.S == 1 && p.num_splits == 1 && base > 128 && base < 256 && sparse_mla_latent_only(p) && p.topk >= 8 * kTK) {
-    p.num_splits = 2;
-    p.keys_per_split = ((p.topk + kTK - 1) / kTK + 1) / 2 * kTK;
-    p.f32_partials = 0;
-  }
+  mla_key_splits(p, (long long)p.B * p.S * p.G * chunks, kMaxKeys, 1.1, kHeadsWg, sparse_mla_latent_only(p));
 }
 
 int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream) {

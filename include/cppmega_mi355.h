@@ -277,12 +277,13 @@ int cppmega_mi355_sparse_mla_fwd(const cppmega_mi355_sparse_mla_args_t* args, si
 /* cppmega_mi355_sparse_mla_fwd for callers that cannot allocate device memory or
  * carry a workspace around (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It has no counterpart in the reference.
- * Same arguments, kernels and results as cppmega_mi355_sparse_mla_fwd, but the
+ * Same arguments and results as cppmega_mi355_sparse_mla_fwd, but the
  * split-KV partials go to a fixed array of CPPMEGA_MI355_NOALLOC_SCRATCH_BYTES that
  * is part of the library image on every GPU the library runs on; `workspace` and
- * `workspace_bytes` of args are ignored, and the call allocates nothing.  A request
- * whose *_workspace_bytes exceeds the array fails with CPPMEGA_MI355_ERR_WORKSPACE
- * before anything is launched.  All calls on one GPU share that GPU's array, whose
+ * `workspace_bytes` of args are ignored, and the call allocates nothing.  Where
+ * *_workspace_bytes exceeds the array, a plan with fewer key splits (or another kernel)
+ * that fits it runs instead; a request that none fits fails with
+ * CPPMEGA_MI355_ERR_WORKSPACE before anything is launched.  All calls on one GPU share that GPU's array, whose
  * contents are undefined between calls (nothing in it has to start at zero): two
  * calls that overlap in time on one GPU, on different streams, race; calls on one
  * stream, or otherwise ordered, do not. */

@@ -246,3 +246,10 @@ def test_latent_launches_that_fit_without_splits_stay_in_one_piece(queries, head
     need = C.c_size_t(1)
     a = _latent_mla_args(batch=1, seq_q=queries, heads=heads)
     assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0 and need.value == 0
+
+
+@pytest.mark.parametrize("batch", [65, 96, 127])
+def test_decode_steps_that_one_split_serves_fastest_need_no_scratch(batch):
+    need = C.c_size_t(1)
+    a = _latent_mla_args(batch=batch)
+    assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0 and need.value == 0

@@ -79,7 +79,7 @@ def test_noalloc_entry_point_refuses_what_does_not_fit(device):
     a.kernel = _lib.MLA_KERNEL_AUTO
     a.q_dtype, a.kv_dtype, a.kv_scale_kind, a.kv_scale_block = _lib.BF16, _lib.E4M3, _lib.SCALE_F32_BLOCK, 128
     a.rope_dtype, a.rope_dim, a.index_dtype, a.out_dtype = _lib.BF16, 64, _lib.I32, _lib.BF16
-    a.batch, a.seq_q, a.heads, a.kv_groups, a.seq_kv, a.topk, a.d_qk, a.d_v = 96, 1, 128, 1, 65536, 2048, 576, 512
+    a.batch, a.seq_q, a.heads, a.kv_groups, a.seq_kv, a.topk, a.d_qk, a.d_v = 96, 1, 128, 1, 65536, 8192, 576, 512
     a.sm_scale = 576 ** -0.5
     a.q = a.kv = a.kv_scale = a.kv_rope = a.indices = a.out = 0x1000     # 16-byte aligned, never dereferenced
     need = C.c_size_t(0)
