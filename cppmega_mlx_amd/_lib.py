@@ -377,7 +377,7 @@ def library_path() -> Path:
 
 
 def load() -> C.CDLL:
-    """Load the shared library once (thread-safe) and declare its prototypes."""
+    """Load the shared library and the extension in front of it once (thread-safe) and declare the prototypes."""
     global _lib
     with _lock:
         if _lib is not None:
@@ -442,6 +442,7 @@ def load() -> C.CDLL:
         lib.cppmega_mi355_fp8_vecmat_workspace_bytes.argtypes = [
             C.POINTER(VecmatArgs), C.c_size_t, C.POINTER(C.c_size_t)]
         lib.cppmega_mi355_fp8_vecmat_workspace_bytes.restype = C.c_int
+        load_host()
         _lib = lib
         return lib
 

@@ -20,7 +20,22 @@ import torch
 
 from . import _lib
 
-host = _lib.load_host()
+
+class _Host:
+    """The native launch path, loaded at the first call.  Where it cannot be loaded a call is not the plain case: the
+    helpers behind it load the library, which raises the reason."""
+
+    def __getattr__(self, name: str):
+        try:
+            found = getattr(_lib.load_host(), name)
+        except _lib.NativeLibraryError:
+            return lambda *args: None
+        setattr(self, name, found)
+        return found
+
+
+host = _Host()
+
 
 def _workspace(device: torch.device, nbytes: int, stream: int) -> torch.Tensor | None:
     """Per-(device, stream) scratch, grown geometrically up to 1 GiB; a larger request gets a tensor of its own."""

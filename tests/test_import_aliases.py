@@ -26,3 +26,33 @@ def test_v4_import_paths():
     import cppmega_mlx_amd.nn.mla_absorb as ma
     assert LightningIndexer is li.LightningIndexer and LightningIndexerFP8 is li.LightningIndexerFP8
     assert absorbed_mla_decode is ma.absorbed_mla_decode and callable(fused_fp8_gemm)
+
+
+def test_without_the_native_launch_path_modules_import_and_say_why():
+    """The extension missing, or built for another torch: nothing fails before the first use, which names the reason."""
+    import subprocess
+    import sys
+    subprocess.run([sys.executable, "-c", """
+import sys
+sys.modules["cppmega_mlx_amd._host"] = None
+import torch
+from cppmega_mlx_amd import _lib, ops
+import cppmega_mlx_amd.nn.mla_absorb, cppmega_mlx_amd.nn.lightning_indexer, cppmega_mlx_amd.nn.sparse_mla, cppmega_mlx_amd.inference.engine
+from cppmega_mlx_amd.nn._tilelang.dsa_splitk_indexer_loss import dsa_splitk_path_c_status
+from cppmega_mlx_amd.nn._tilelang.fp8_vecmat_path_c import fp8_vecmat_path_c_status
+from cppmega_mlx_amd.nn._tilelang.sparse_mla_blockscaled_path_c import sparse_mla_blockscaled_path_c_status
+from cppmega_mlx_amd.nn._tilelang.sparse_mla_fp8_path_c import sparse_mla_fp8_path_c_status
+from cppmega_mlx_amd.nn._tilelang.topk_selector import topk_selector_path_c_status
+for status in (dsa_splitk_path_c_status, fp8_vecmat_path_c_status, sparse_mla_blockscaled_path_c_status, sparse_mla_fp8_path_c_status,
+               topk_selector_path_c_status):
+    answer = status()
+    assert not answer.available and "cannot load the extension" in answer.reason, answer
+assert ops.host.topk(torch.zeros(1, 4), 1, None, None, None, False, False) is None       # the helper behind it raises
+ops.release_workspaces()
+try:
+    _lib.load()
+except _lib.NativeLibraryError as exc:
+    assert "no fallback" in str(exc)
+else:
+    raise AssertionError("loaded")
+"""], check=True, cwd=__file__.rsplit("/", 2)[0])
