@@ -10,6 +10,8 @@
 // the first loads and the stores of a tile, 10 of 33 us, which a CU with one workgroup does not overlap; a
 // small batch, the weight stream (5 TB/s at M = 32).
 
+#include <stdint.h>
+
 #include "fp8_vecmat.h"
 
 namespace cm {
@@ -305,18 +307,21 @@ constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
 
 struct GemmPlan { const TileShape* shape; int splits; };
 
+size_t split_bytes(int splits, int m, int n) { return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0; }
+
 // The tile shape and K split with the smallest estimate: rounds of workgroups over the CUs, plus, for a
 // split, one more launch and the partial sums written and read (8 bytes per sum).  Fitted to all 33 combinations at
 // 55 shapes of 17..1000 x 512..16384 x 896..16384: the choice is 0.4 % from the best of them in the mean and 7 % at
 // most.  The third workgroup on a CU brings nothing (the weights' stream is what they share).
-GemmPlan gemm_plan(int m, int n, int k) {
+// Splits whose sums need more than `have` bytes are left out; one split needs none.
+GemmPlan gemm_plan(int m, int n, int k, size_t have) {
   const int blocks = k / 128, cus = device_cus();
   GemmPlan best = {&kShapes[0], 1};
   double best_us = 1e30;
   for (const TileShape& s : kShapes) {
     const double tiles = (double)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn);
     for (int splits : kSplits) {
-      if (splits > 1 && splits * 2 > blocks) break;
+      if (splits > 1 && (splits * 2 > blocks || split_bytes(splits, m, n) > have)) break;
       const long long wgs = (long long)tiles * splits, on_cu = (wgs + cus - 1) / cus;
       const double steps = (blocks + splits - 1) / splits;
       const long long rounds = on_cu / s.per_cu, rest = on_cu % s.per_cu;
@@ -345,12 +350,11 @@ bool fp8_gemm_shape(const cppmega_mi355_vecmat_args_t& a) {
 }
 
 size_t fp8_gemm_workspace_bytes(const cppmega_mi355_vecmat_args_t& a) {
-  const GemmPlan g = gemm_plan(a.m, a.n, a.k);
-  return g.splits > 1 ? (size_t)g.splits * a.m * a.n * sizeof(float) : 0;
+  return split_bytes(gemm_plan(a.m, a.n, a.k, SIZE_MAX).splits, a.m, a.n);
 }
 
-int fp8_gemm_launch(VecmatParams p, hipStream_t stream) {
-  const GemmPlan g = gemm_plan(p.m, p.n, p.k);
+int fp8_gemm_launch(VecmatParams p, size_t workspace_bytes, hipStream_t stream) {
+  const GemmPlan g = gemm_plan(p.m, p.n, p.k, workspace_bytes);
   p.k_splits = g.splits;
   const long long tiles = (long long)((p.m + g.shape->bm - 1) / g.shape->bm) * ((p.n + g.shape->bn - 1) / g.shape->bn);
   if (tiles > 0x7fffffffLL) return fail(CPPMEGA_MI355_ERR_SHAPE, "vecmat: M=%d N=%d has too many tiles", p.m, p.n);

@@ -28,7 +28,7 @@ __device__ __forceinline__ float wscale(const VecmatParams& p, int n, int kb) {
 // The tiled GEMM for more activation rows than the streaming kernels are made for (fp8_gemm.hip).
 bool fp8_gemm_shape(const cppmega_mi355_vecmat_args_t& a);
 size_t fp8_gemm_workspace_bytes(const cppmega_mi355_vecmat_args_t& a);
-int fp8_gemm_launch(VecmatParams p, hipStream_t stream);
+int fp8_gemm_launch(VecmatParams p, size_t workspace_bytes, hipStream_t stream);      // with fewer K splits where they do not fit
 int device_cus();
 
 }  // namespace cm

@@ -757,11 +757,8 @@ int fp8_vecmat_launch(const cppmega_mi355_vecmat_args_t& a, hipStream_t stream) 
     rc = stream_pass(p, 0, a.m);
     if (rc) return rc;
   } else if (aligned && fp8_gemm_shape(a)) {
-    const size_t need = fp8_gemm_workspace_bytes(a);
-    if (need > 0 && (!a.workspace || a.workspace_bytes < need))
-      return fail(CPPMEGA_MI355_ERR_WORKSPACE, "vecmat: workspace of %zu bytes needed, %zu given", need, a.workspace ? (size_t)a.workspace_bytes : (size_t)0);
     p.partial = (float*)a.workspace;
-    return fp8_gemm_launch(p, stream);
+    return fp8_gemm_launch(p, a.workspace ? (size_t)a.workspace_bytes : 0, stream);
   } else if (aligned && rows_shape(a)) {
     // about one workgroup per CU, whole MFMA row tiles where that is possible
     int rows = (a.n + device_cus() - 1) / device_cus();

@@ -213,3 +213,31 @@ def test_tiled_gemm_edges(device, M, N, K, dtype):
         vm.fp8_scaled_vecmat_path_c(x.to(device), codes.view(torch.uint8).to(device), scale_x=None, scale_w=scale.to(device), out=out)
         err = (out.double().cpu() - want).abs().max() / want.abs().max()
         assert err <= tol, err
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(17, 257, 1152), (32, 1024, 2048), (100, 300, 4096)])
+def test_tiled_gemm_with_less_workspace_than_asked_for(device, M, N, K, dtype):
+    """Through the C interface: no workspace, one that holds two splits, and the whole one."""
+    import ctypes as C
+    from cppmega_mlx_amd import _lib
+    gen = torch.Generator(device="cpu").manual_seed(M)
+    x = torch.randn((M, K), generator=gen).to(dtype)
+    codes = torch.randn((N, K), generator=gen).to(torch.float8_e4m3fn)
+    scale = torch.rand((N, K // 128), generator=gen) + 0.5
+    want = x.double() @ (codes.double() * scale.double().repeat_interleave(128, dim=1)).T
+    xd, cd, sd = x.to(device), codes.view(torch.uint8).to(device), scale.to(device)
+    a = _lib.VecmatArgs()
+    a.struct_size, a.x_dtype, a.out_dtype, a.scale_w_kind = C.sizeof(a), _lib.dtype_code(xd), _lib.F32, _lib.WSCALE_ROW_BLOCK
+    a.x, a.w, a.scale_w, a.m, a.n, a.k = xd.data_ptr(), cd.data_ptr(), sd.data_ptr(), M, N, K
+    need = C.c_size_t(0)
+    lib = _lib.load()
+    assert lib.cppmega_mi355_fp8_vecmat_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK and need.value > 2 * M * N * 4
+    ws = torch.empty(need.value, dtype=torch.uint8, device=device)
+    for given in (0, 2 * M * N * 4, need.value):
+        ws.fill_(0xff)
+        out = torch.full((M, N), 7.0, device=device)
+        a.out, a.workspace, a.workspace_bytes = out.data_ptr(), ws.data_ptr() if given else None, given
+        assert lib.cppmega_mi355_fp8_vecmat(C.byref(a), C.sizeof(a), _lib.current_stream(xd.device)) == _lib.OK
+        assert (out.double().cpu() - want).abs().max() <= 2e-6 * want.abs().max()
+        assert (ws[given:] == 0xff).all()
