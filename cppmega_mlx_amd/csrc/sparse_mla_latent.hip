@@ -6,11 +6,9 @@
 //   (per 128 / 256 / 512 channels, per row, or none) plus a bf16 rope tail [64];
 //   queries and key rows of 576 e4m3 codes with one fp32 scale per (query, head) and per row.
 //
-// Measured against the kernel of sparse_mla_mfma.hip that has the whole tile loop in every wavefront:
-//   code rows, 128 heads x 999 queries x 2048 keys: 1013 -> 445 us (the scores are e4m3 products: the
-//   same work in bf16 at the rate of a large matrix product is 458 us); 64 heads x 1 query x 2048: 58 -> 18 us;
-//   16 heads (three quarters of the chunk idle): latent rows 1 x 2048 of 8192 39 -> 17 us, 2000 x 2048 998 -> 563 us,
-//   code rows 1000 x 2048 443 -> 212 us.  No shape tried (16 .. 128 heads, 1 .. 2000 queries, 256 .. 2048 keys) was slower.
+// Measured against the kernel of sparse_mla_mfma.hip that has the whole tile loop in every wavefront (us a call, keys
+// of 8192 rows): code rows, 128 heads x 1000 queries x 2048 keys 998 -> 698, 64 x 1 x 2048 55 -> 22, 16 x 1000 x 2048
+// 447 -> 324; latent rows, 16 heads (three quarters of the chunk idle) 1 x 2048 35 -> 23, 2000 x 2048 1013 -> 652.
 //
 // Workgroup = (query, KV group, chunk of 64 heads, key split), 8 wavefronts, key tiles of 32
 // rows in a ring of five LDS slots filled by the load unit (global_load_lds) three tiles ahead.
@@ -18,11 +16,16 @@
 // under the vector instructions of the other.
 //
 //   producers (wavefronts 0..3): producer p owns heads 16p..16p+15 of the chunk.
-//     S^T = K.Q^T on v_mfma_scale_f32_16x16x128_f8f6f4: the key bytes are the A operand as they
-//     lie in the tile (no conversion instructions, operand exponent 2^0); every 128-channel block is
-//     accumulated from zero and enters the score times its keys' fp32 block scales.  Q^T is
-//     split once per workgroup into two e4m3 planes hi + lo (hi + lo = the bf16 value, one
-//     exponent per head and 128 channels), kept in registers.  The rope tail is a bf16 product.
+//     S^T = K.Q^T, every 128-channel block accumulated from zero and entering the score times its
+//     keys' fp32 block scales; the rope tail is a bf16 product.  Latent rows of more than 32 heads:
+//     v_mfma_scale_f32_16x16x128_f8f6f4, the key bytes being the A operand as they lie in the tile (no
+//     conversion instructions, operand exponent 2^0) and Q^T split once per workgroup into two e4m3
+//     planes hi + lo (hi + lo = the bf16 value, one exponent per head and 128 channels), kept in
+//     registers.  Code rows and up to 32 heads: v_mfma_f32_16x16x32_bf16, the key bytes converted
+//     (exactly) on their way.  A sum of e4m3 products, of 32 or of 128 terms, is off by 1.5e-5 of the
+//     result's scale in the mean, one of bf16 products by 2.6e-8 (512 terms): lse of code rows is good
+//     to 4e-7 where it was to 4e-6 (to 1e-6 and 1e-4 with scores of four times the deviation), for
+//     1.25 us a tile instead of 0.95 (128 heads x 1000 x 2048: 536 us with e4m3 products).
 //     Softmax in base 2 with a lazily moved private running maximum per head; P goes to LDS as
 //     bf16 in the B-operand layout of the value product, one plane per scale block: plane b is P
 //     times the keys' scales of block b (one fp32 product, rounded once).
@@ -154,10 +157,10 @@ __device__ __forceinline__ int split_q32(const uint4 (&x)[4], i32x8& hi, i32x8& 
 }
 
 // NBLK: fp32 scales per key row (1, 2 or 4).
-// ROWS: key rows and queries of 576 e4m3 codes with one fp32 scale each (NBLK = 1).  The query's codes are the
-// second operand as they are, one plane of them; the tail of 64 codes is two products of 32; a head's query
-// scale joins the softmax scale and a key's scale multiplies the whole sum.
-template <int NBLK, bool ROWS>
+// ROWS: key rows and queries of 576 e4m3 codes with one fp32 scale each (NBLK = 1): a head's query scale joins the
+// softmax scale and a key's scale multiplies the whole sum.
+// BF16: the scores are bf16 products.
+template <int NBLK, bool ROWS, bool BF16>
 __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = (int)threadIdx.x, lane = tid & 63;
@@ -165,7 +168,7 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   const bool producer = wave < 4;
   const int role = wave & 3;                    // producer p / consumer c
   constexpr int nblk = NBLK;
-  static_assert(!ROWS || NBLK == 1, "one scale per row");
+  static_assert(!ROWS || (NBLK == 1 && BF16), "one scale per row");
   constexpr int kRowPitch = ROWS ? kDqk : kLat;     // bytes of a key row in the cache
 
   // ---- which (query, KV group, head chunk, split).  Workgroup ids that are equal modulo 8 run on
@@ -324,16 +327,19 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     uint4 qraw[4][4];
     bf16x8 qr[2];
     i32x8 qh[4], ql[4];
-    unsigned long long qt[2];                       // ROWS: the tail, codes 512 + 16 kg .. + 7 and + 8 .. + 15
     if (ROWS) {
 #pragma unroll
-      for (int blk = 0; blk < 4; ++blk) {
-        const uint4 c0 = *reinterpret_cast<const uint4*>(qstage + n * kQPitch + 128 * blk + 32 * kg);
-        const uint4 c1 = *reinterpret_cast<const uint4*>(qstage + n * kQPitch + 128 * blk + 32 * kg + 16);
-        qh[blk] = i32x8{(int)c0.x, (int)c0.y, (int)c0.z, (int)c0.w, (int)c1.x, (int)c1.y, (int)c1.z, (int)c1.w};
-      }
+      for (int blk = 0; blk < 4; ++blk)
 #pragma unroll
-      for (int r = 0; r < 2; ++r) qt[r] = *reinterpret_cast<const unsigned long long*>(qstage + n * kQPitch + kLat + 16 * kg + 8 * r);
+        for (int j = 0; j < 4; ++j) {
+          const uint2 c = *reinterpret_cast<const uint2*>(qstage + n * kQPitch + 128 * blk + 32 * kg + 8 * j);
+          qraw[blk][j] = __builtin_bit_cast(uint4, cvt8(c.x, c.y));
+        }
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {                 // the tail: codes 512 + 16 kg + 8 r .. + 7
+        const uint2 c = *reinterpret_cast<const uint2*>(qstage + n * kQPitch + kLat + 16 * kg + 8 * r);
+        qr[r] = cvt8(c.x, c.y);
+      }
     } else {
 #pragma unroll
       for (int blk = 0; blk < 4; ++blk)
@@ -345,7 +351,7 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     __syncthreads();                                // keys[] is complete
     const int n_tiles = count_tiles();
     int qexp = 0;
-    if (!ROWS)
+    if (!BF16)
 #pragma unroll
       for (int blk = 0; blk < 4; ++blk) qexp |= split_q32(qraw[blk], qh[blk], ql[blk]) << (8 * blk);
     float m_run = -INFINITY;                      // base-2 running reference of head n
@@ -360,7 +366,7 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     // the first one's products.
     i32x8 kf[2][4];
     bf16x8 rf[2][2];
-    unsigned long long tf[2][2];                    // ROWS: the tails
+    uint4 tf[2];                                    // ROWS: the tails, 16 codes
     // (a tile's slot is passed as its byte offset into the ring, a running value: one address
     // register per slot then reaches every operand of the tile with an immediate offset)
     auto load_k = [&](unsigned slot_off, int sj) {
@@ -375,10 +381,7 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
         kf[sj][blk] = i32x8{(int)c0.x, (int)c0.y, (int)c0.z, (int)c0.w, (int)c1.x, (int)c1.y, (int)c1.z, (int)c1.w};
       }
       if (ROWS) {
-        typedef __attribute__((ext_vector_type(2))) unsigned long long u64x2;
-        const u64x2 c = *reinterpret_cast<const u64x2*>(slot + kLatBytes + sj * 1024);
-        tf[sj][0] = c[0];
-        tf[sj][1] = c[1];
+        tf[sj] = *reinterpret_cast<const uint4*>(slot + kLatBytes + sj * 1024);
       } else {
         rf[sj][0] = *reinterpret_cast<const bf16x8*>(rope);
         rf[sj][1] = *reinterpret_cast<const bf16x8*>(rope + 1024);
@@ -428,16 +431,22 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
       f32x4 st[2];
       auto subtile = [&](auto sj_c, const float (&ksc)[4][nblk]) {
         constexpr int sj = decltype(sj_c)::value;
-        if constexpr (ROWS) {                        // one scale for the whole row: two running sums, then the scale
-          f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
-          mfma_s8<0>(a0, kf[sj][0], qh[0], kOne, kOne);
-          mfma_s8<0>(a1, kf[sj][1], qh[1], kOne, kOne);
-          mfma_s8<0>(a0, kf[sj][2], qh[2], kOne, kOne);
-          mfma_s8<0>(a1, kf[sj][3], qh[3], kOne, kOne);
-          a0 = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)tf[sj][0], (long)qt[0], a0, 0, 0, 0);
-          a1 = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)tf[sj][1], (long)qt[1], a1, 0, 0, 0);
+        // BF16: a 128-channel block is four products of 32 channels, the lane's codes eight at a time
+        auto part = [&](f32x4& acc, int blk, int j) {
+          mfma_s(acc, cvt8((unsigned)kf[sj][blk][2 * j], (unsigned)kf[sj][blk][2 * j + 1]), __builtin_bit_cast(bf16x8, qraw[blk][j]));
+        };
+        if constexpr (ROWS) {                        // one scale for the whole row: four running sums, then the scale
+          f32x4 a[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) st[sj][i] = ksc[i][0] * (a0[i] + a1[i]);
+          for (int blk = 0; blk < 4; ++blk) a[blk] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int blk = 0; blk < 4; ++blk) part(a[blk], blk, j);
+          mfma_s(a[0], cvt8(tf[sj].x, tf[sj].y), qr[0]);
+          mfma_s(a[1], cvt8(tf[sj].z, tf[sj].w), qr[1]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) st[sj][i] = ksc[i][0] * ((a[0][i] + a[1][i]) + (a[2][i] + a[3][i]));
           return;
         }
         st[sj] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -446,10 +455,18 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
         auto pair = [&](auto b_c) {
           constexpr int b0 = decltype(b_c)::value, b1 = b0 + 1;
           f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
-          mfma_s8<b0>(a0, kf[sj][b0], qh[b0], kOne, qexp);
-          mfma_s8<b1>(a1, kf[sj][b1], qh[b1], kOne, qexp);
-          mfma_s8<b0>(a0, kf[sj][b0], ql[b0], kOne, qexp);
-          mfma_s8<b1>(a1, kf[sj][b1], ql[b1], kOne, qexp);
+          if constexpr (BF16) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              part(a0, b0, j);
+              part(a1, b1, j);
+            }
+          } else {
+            mfma_s8<b0>(a0, kf[sj][b0], qh[b0], kOne, qexp);
+            mfma_s8<b1>(a1, kf[sj][b1], qh[b1], kOne, qexp);
+            mfma_s8<b0>(a0, kf[sj][b0], ql[b0], kOne, qexp);
+            mfma_s8<b1>(a1, kf[sj][b1], ql[b1], kOne, qexp);
+          }
 #pragma unroll
           for (int i = 0; i < 4; ++i) st[sj][i] = __builtin_fmaf(ksc[i][(b0 * nblk) >> 2], a0[i], st[sj][i]);
 #pragma unroll
@@ -1054,7 +1071,7 @@ void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us,
 void sparse_mla_latent_plan(MlaParams& p) {
   const int chunks = (p.heads_per_group + kHeadsWg - 1) / kHeadsWg;
   p.heads_per_wg = kHeadsWg;
-  mla_key_splits(p, (long long)p.B * p.S * p.G * chunks, kMaxKeys, 1.1, kHeadsWg, sparse_mla_latent_only(p));
+  mla_key_splits(p, (long long)p.B * p.S * p.G * chunks, kMaxKeys, code_rows(p) ? 1.25 : 1.1, kHeadsWg, sparse_mla_latent_only(p));
 }
 
 int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream) {
@@ -1064,18 +1081,14 @@ int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream) {
     return fail(CPPMEGA_MI355_ERR_UNSUPPORTED, "sparse MLA: launch too large");
   const dim3 grid((unsigned)wgs), block(512);
   const int nblk = p.kv_scale_kind == CPPMEGA_MI355_SCALE_F32_BLOCK ? kLat / p.kv_scale_block : 1;
-#define CM_LAUNCH_PC(NB_, ROWS_)                                                                                          \
-  do {                                                                                                             \
-    CM_HIP_CHECK(hipFuncSetAttribute((const void*)sparse_mla_latent_kernel<NB_, ROWS_>,                                 \
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, kSmem));                           \
-    hipLaunchKernelGGL((sparse_mla_latent_kernel<NB_, ROWS_>), grid, block, kSmem, stream, p);                          \
-  } while (0)
-  const bool rows = code_rows(p);
-  if (rows) CM_LAUNCH_PC(1, true);
-  else if (nblk == 4) CM_LAUNCH_PC(4, false);
-  else if (nblk == 2) CM_LAUNCH_PC(2, false);
-  else CM_LAUNCH_PC(1, false);
-#undef CM_LAUNCH_PC
+  const bool rows = code_rows(p), bf16 = !sparse_mla_latent_only(p);
+  void (*kernel)(MlaParams) =
+      rows ? sparse_mla_latent_kernel<1, true, true>
+      : nblk == 4 ? (bf16 ? sparse_mla_latent_kernel<4, false, true> : sparse_mla_latent_kernel<4, false, false>)
+      : nblk == 2 ? (bf16 ? sparse_mla_latent_kernel<2, false, true> : sparse_mla_latent_kernel<2, false, false>)
+                  : (bf16 ? sparse_mla_latent_kernel<1, false, true> : sparse_mla_latent_kernel<1, false, false>);
+  CM_HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kSmem));
+  hipLaunchKernelGGL(kernel, grid, block, kSmem, stream, p);
   CM_HIP_CHECK(hipGetLastError());
   if (p.num_splits > 1) {
     if (p.f32_partials) return sparse_mla_combine_f32(p, stream);

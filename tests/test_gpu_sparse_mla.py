@@ -639,3 +639,29 @@ def test_latent_rows_that_no_list_names_may_hold_anything(device, H, topk, scale
     assert torch.isfinite(out).all()
     err, ref = error_report(out.cpu().numpy(), want_out)
     assert err <= REL_TOL * ref and np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_TOL_MFMA
+
+
+@pytest.mark.parametrize("rows,H,topk", [("codes", 16, 64), ("codes", 64, 300), ("codes", 128, 1000), ("latent", 16, 64), ("latent", 32, 300)])
+def test_scores_are_float32_sums(device, rows, H, topk):
+    """Scores of four times the usual deviation.  Every product is exact; a score is 18 partial sums of magnitude up to
+    30 added in float32, off by at most 18 * 30 * 2^-24 = 3.2e-5 and by a few 1e-6 as they come (sums of e4m3
+    products are off by 1e-4 and more)."""
+    from cppmega_mlx_amd import _lib
+    S, Skv, sm = 3, 1200, 4 * 576 ** -0.5
+    rng = np.random.default_rng(H + topk)
+    idx = sparse_indices(rng, 1, S, 1, Skv, topk)
+    out = torch.zeros((1, S, H, 512), dtype=torch.float32, device=device)
+    lse = torch.zeros((1, S, H), dtype=torch.float32, device=device)
+    if rows == "codes":
+        qc, qs = fp8.quantize_per_token(rng.standard_normal((1, S, H, 576)).astype(np.float32))
+        kc, ks = fp8.quantize_per_token(rng.standard_normal((1, Skv, 1, 576)).astype(np.float32))
+        want_out, want_lse = om.sparse_mla_oracle(om.dequant_per_token(qc, qs), om.dequant_per_token(kc, ks), idx, sm_scale=sm, d_v=512)
+        args = (to_dev(qc, device), to_dev(kc, device))
+        kw = dict(q_spec=ops.QuantSpec(_lib.SCALE_PER_TOKEN, to_dev(qs, device)), kv_spec=ops.QuantSpec(_lib.SCALE_PER_TOKEN, to_dev(ks, device)))
+    else:
+        q, qf = bf16_pair(rng.standard_normal((1, S, H, 576)), device)
+        codes, scale, rope, decoded = latent_cache(rng, 1, Skv, 1, 512, 64, device, pow2=True)
+        want_out, want_lse = om.sparse_mla_oracle(qf, decoded, idx, sm_scale=sm, d_v=512)
+        args, kw = (q, codes), dict(kv_spec=ops.QuantSpec(_lib.SCALE_F32_BLOCK, scale, 128), kv_rope=rope)
+    ops.sparse_mla_forward(args[0], args[1], to_dev(idx.astype(np.int32), device), sm_scale=sm, d_v=512, out=out, lse=lse, kernel="mfma", **kw)
+    _assert_close(out, lse, want_out, want_lse, lse_tol=1.6e-5)
