@@ -8,11 +8,12 @@
 // 2048 x 7168 x 16384: 490 = 980 TFLOP/s.  What bounds it: a large product, the issue of MFMAs and of the
 // vector instructions between them (128 per 32 MFMAs: conversions and scaled sums); a short one (K = 1536),
 // the first loads and the stores of a tile, 10 of 33 us, which a CU with one workgroup does not overlap; a
-// small batch, the weight stream (5 TB/s at M = 32).
+// small batch, the weight stream (32 x 7168 x 16384: 37.5 us a call, 3.1 TB/s).
 
 #include <stdint.h>
 
 #include "fp8_vecmat.h"
+#include "mfma_util.h"
 
 namespace cm {
 namespace {
@@ -273,16 +274,29 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void fp8_gemm_kernel(const VecmatP
   else store((float*)p.out, [](float v) { return v; });
 }
 
-// out[m][n] = sum over the K splits of partial[split][m][n], in split order
+// out[m][n] = sum over the K splits of partial[split][m][n], in split order.  Bound by latency (7 MB at 32 x 7168 x 8
+// splits): with the splits' loads one after the other and stores of single values a call took 2 to 3 us longer.
 __global__ __launch_bounds__(256) void fp8_gemm_reduce_kernel(const VecmatParams p) {
   const size_t total = (size_t)p.m * p.n;
   const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= total) return;
   if ((total & 3) == 0) {
-    f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int z = 0; z < p.k_splits; ++z) s += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.partial + (size_t)z * total + i));
+    // (the loads of the up to 16 splits are in flight together)
+    f32x4 part[16], s = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int v = 0; v < 4; ++v) store_as(p.out, i + v, p.out_dtype, s[v]);
+    for (int z = 0; z < 16; ++z)
+      if (z < p.k_splits) part[z] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.partial + (size_t)z * total + i));
+#pragma unroll
+    for (int z = 0; z < 16; ++z)
+      if (z < p.k_splits) s += part[z];
+    if (p.out_dtype != CPPMEGA_MI355_F32 && ((uintptr_t)p.out & 7) == 0) {
+      const bool bf16 = p.out_dtype == CPPMEGA_MI355_BF16;
+      *reinterpret_cast<uint2*>((unsigned short*)p.out + i) = bf16 ? make_uint2(pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3]))
+                                                                   : make_uint2(pack_f16(s[0], s[1]), pack_f16(s[2], s[3]));
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) store_as(p.out, i + v, p.out_dtype, s[v]);
+    }
   } else {
     for (size_t e = i; e < i + 4 && e < total; ++e) {
       float s = 0.0f;
@@ -303,16 +317,17 @@ constexpr TileShape kShapes[] = {
     {64, 128, 2, {0.85, 1.77, 0.0}, 8.35},
     {128, 256, 1, {1.77, 0.0, 0.0}, 9.3},
 };
-constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
+constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 16};
 
 struct GemmPlan { const TileShape* shape; int splits; };
 
 size_t split_bytes(int splits, int m, int n) { return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0; }
 
 // The tile shape and K split with the smallest estimate: rounds of workgroups over the CUs, plus, for a
-// split, one more launch and the partial sums written and read (8 bytes per sum).  Fitted to all 33 combinations at
-// 55 shapes of 17..1000 x 512..16384 x 896..16384: the choice is 0.4 % from the best of them in the mean and 7 % at
-// most.  The third workgroup on a CU brings nothing (the weights' stream is what they share).
+// split, one more launch and the partial sums written and read (8 bytes per sum).  Fitted to all combinations but
+// those of 9 splits at 55 shapes of 17..1000 x 512..16384 x 896..16384: the choice is 0.4 % from the best of them in the
+// mean and 7 % at most.  9 splits give 56 column tiles two workgroups on nearly every CU where 8 leave a quarter of the
+// CUs with one (32 x 7168 x 16384: 41 -> 39 us, the calls of 13 .. 16 splits that finer steps would pick are no faster).  The third workgroup on a CU brings nothing (the weights' stream is what they share).
 // Splits whose sums need more than `have` bytes are left out; one split needs none.
 GemmPlan gemm_plan(int m, int n, int k, size_t have) {
   const int blocks = k / 128, cus = device_cus();

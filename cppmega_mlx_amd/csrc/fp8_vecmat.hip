@@ -629,7 +629,7 @@ static bool stream_k(const cppmega_mi355_vecmat_args_t& a) {
 static bool stream_shape(const cppmega_mi355_vecmat_args_t& a) { return stream_k(a) && a.m <= stream_row_cap(a.x_dtype); }
 // the kernel without a K split: bf16 / fp16 activations, 5 <= M <= 16, whole 128-channel blocks,
 // scales of 32 rows and partial tiles within the LDS
-constexpr int kRowsMaxM = 16;             // more activation rows: the tiled GEMM (M = 32: 31 us against 37 us at 7168 x 16384)
+constexpr int kRowsMaxM = 16;             // more activation rows: the tiled GEMM
 static size_t rows_lds_bytes(int k, int mt) { return (size_t)rows_waves(mt) * (32 * 128 + mt * 16 * 256) + (size_t)(k / 128) * 32 * sizeof(float); }
 static bool rows_shape(const cppmega_mi355_vecmat_args_t& a) {
   return (a.x_dtype == CPPMEGA_MI355_BF16 || a.x_dtype == CPPMEGA_MI355_F16) && a.m >= 5 && a.m <= kRowsMaxM && a.k % 128 == 0 &&
