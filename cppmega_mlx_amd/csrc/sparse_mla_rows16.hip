@@ -601,9 +601,13 @@ size_t e8m0_row_bytes(const MlaParams& p) { return e8m0_rows(p) ? ((size_t)p.B *
 
 bool rows_of_16_bits(const MlaParams& p) {
   if (e8m0_rows(p)) {
-    // every row of the cache is converted: where that is more than 65536 of them (25 us), the lists have to name as many
+    // Every row of the cache is converted, for 1152 bytes of workspace and 0.35 ns each.  Up to 65536 rows (25 us) that is
+    // made up for by short lists too (8 x 256 of 65536: 43 / 48 / 47 us with 16 / 64 / 128 heads, 41 / 68 / 70 on the tile
+    // kernel); beyond, where the lists name two keys for every row (2 M keys of 1 M rows: 715 / 796 / 1058 us against 698 /
+    // 1159 / 1189; 1 M keys: 538 / 571 / 690 against 363 / 583 / 594).  And never for more than the scratch kept between calls.
     const long long rows = (long long)p.B * p.Skv * p.G;
-    return p.plan_level == 0 && p.d_kv == kDqk && p.rope_dim == 0 && (rows <= 65536 || rows <= (long long)p.B * p.S * p.G * p.topk);
+    return p.plan_level == 0 && p.d_kv == kDqk && p.rope_dim == 0 &&
+           (rows <= 65536 || (2 * rows <= (long long)p.B * p.S * p.G * p.topk && e8m0_row_bytes(p) <= ((size_t)1 << 30)));
   }
   if ((p.q_dtype != CPPMEGA_MI355_BF16 && p.q_dtype != CPPMEGA_MI355_F16) || p.kv_dtype != p.q_dtype) return false;
   if (p.q_scale_kind != CPPMEGA_MI355_SCALE_NONE || p.kv_scale_kind != CPPMEGA_MI355_SCALE_NONE) return false;

@@ -253,3 +253,18 @@ def test_decode_steps_that_one_split_serves_fastest_need_no_scratch(batch):
     need = C.c_size_t(1)
     a = _latent_mla_args(batch=batch)
     assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0 and need.value == 0
+
+
+@pytest.mark.parametrize("rows,queries,converted", [
+    (65536, 1, True), (131072, 64, False), (131072, 128, True), (900_000, 1024, True),
+    (1 << 20, 4096, False),                                  # more than the 1 GiB that is kept between calls
+])
+def test_e8m0_rows_are_converted_within_bounds(rows, queries, converted):
+    """Two bytes per code of workspace: up to 65536 rows, then where the lists name two keys for every row, and never more
+    than 1 GiB."""
+    need = C.c_size_t(0)
+    a = _latent_mla_args(batch=1, seq_q=queries, heads=16, seq_kv=rows, topk=2048, rope_dim=0)
+    a.q_dtype, a.q_scale_kind, a.q_scale_block, a.kv_scale_kind, a.kv_scale_block = _lib.E4M3, _lib.SCALE_E8M0, 32, _lib.SCALE_E8M0, 32
+    a.q_scale = a.kv_scale = 0x1000                          # (looked at, not through)
+    assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0
+    assert (need.value >= rows * 1152) == converted
