@@ -596,16 +596,26 @@ __global__ __launch_bounds__(kDkvThreads, 1) void bwd_dkv_kernel(const SplitPara
 #pragma unroll
         for (int v = 0; v < 4; ++v) *at[v] = was[v] + f32x4{add[0][v], add[1][v], add[2][v], add[3][v]};
         if (marked[i]) {                               // (a list that names a key twice)
+          // the lanes of one kg at a time: the others may hold the same key, and the row each has added to is written
+          // before the next one reads it (to a single thread the four rounds are one, hence the fences)
+          auto turn = [] {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+          };
+          turn();
           const int* keys = p.keys + key_at[i] / 4 + kg * 4;
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
             const int slot_of = keys[v], row = (slot_of & ~kAgain) - k0 - wave * p.band_keys;
             const bool again = slot_of >= 0 && (slot_of & kAgain) && row >= 0 && row < p.band_keys;   // (not of a band behind)
-            for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
               if (again && kg == k) {
                 f32x4* once_more = reinterpret_cast<f32x4*>(tile + (row + wave * p.band_keys) * 64) + l16;
                 *once_more += f32x4{add[0][v], add[1][v], add[2][v], add[3][v]};
               }
+              turn();
+            }
           }
         }
         request(i, (ahead + i) & 63);

@@ -368,3 +368,20 @@ def test_rows_that_no_list_names_may_hold_anything(device, topk, D, d_v, bad):
     for got, ref in zip((dq, dkv), want):
         err, scale = error_report(got.cpu().numpy(), ref)
         assert err <= 1e-4 * scale, (err, scale)
+
+
+@pytest.mark.parametrize("times", [3, 9, 16, 40])
+def test_one_key_named_many_times_over(device, times):
+    """More slots of a step of 16 than one lane group holds: their sums meet in one row of dkv."""
+    B, S, H, Skv, topk, D, d_v = 1, 4, 16, 600, 64, 64, 64
+    rng = np.random.default_rng(times)
+    q, kv, d_out = (to_dev(rng.standard_normal(s).astype(np.float32), device).bfloat16() for s in ((B, S, H, D), (B, Skv, 1, D), (B, S, H, d_v)))
+    idx = sparse_indices(rng, B, S, 1, Skv, topk)
+    idx[..., :times] = 7
+    idx = rng.permuted(idx, axis=-1)
+    want = om.sparse_mla_bwd_oracle(q.double().cpu().numpy(), kv.double().cpu().numpy(), idx, d_out.double().cpu().numpy(), sm_scale=D ** -0.5, d_v=d_v)
+    dq, dkv = torch.empty((B, S, H, D), device=device), torch.empty((B, Skv, 1, D), device=device)
+    ops.sparse_mla_backward(q, kv, d_out, to_dev(idx.astype(np.int32), device), sm_scale=D ** -0.5, d_v=d_v, dq=dq, dkv=dkv)
+    for got, ref in zip((dq, dkv), want):
+        err, scale = error_report(got.cpu().numpy(), ref)
+        assert err <= 1e-4 * scale, (err, scale)
