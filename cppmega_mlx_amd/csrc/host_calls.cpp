@@ -3,7 +3,7 @@
 // A Python wrapper of this package checks its arguments, fills an argument struct, asks for the
 // workspace, finds the stream and calls the library: 20 to 40 us a call, as long as the kernels run at
 // decode size.  The functions here do the same for the plain case - tensors of the types and shapes a
-// kernel takes, dense (or a cache view), all on the current device - in 2 to 4 us, launches included.  For
+// kernel takes, dense (or a cache view), all on the current device - in 3 to 7 us, launches included.  For
 // anything else, and whenever the library refuses, they return None without having launched: the wrapper
 // then goes its own way, which knows every other case and says what is wrong with a bad call.
 

@@ -45,7 +45,10 @@ def _workspace(device: torch.device, nbytes: int, stream: int) -> torch.Tensor |
 
 
 def release_workspaces() -> None:
-    """Give the scratch kept between calls back to torch's allocator (the next calls allocate it again)."""
+    """Give the scratch kept between calls back to torch's allocator (the next calls allocate it again).
+
+    A graph captured over calls that use kept scratch holds its address: do not replay it after this, nor after an eager
+    call on the capture's stream that needed more scratch than any before it (the scratch grows by being replaced)."""
     host.release_workspaces()
 
 
