@@ -372,14 +372,17 @@ __global__ __launch_bounds__(kThreads) void dsa_loss_sum_kernel(const LossTiledP
   const long long total = (long long)p.AB * p.slab_rows;
   const int q = p.slab0 + (int)(i % p.slab_rows);
   const int chunks = q < p.ASq ? (min(q + 1, p.Sk) + kChunk - 1) / kChunk : 0;
+  // the caller is told of an index outside the range, and finds the losses as they were
+  int outside = 0;
+  if (p.outside) {
+    const int words = (int)(((long long)p.AB * p.ASq + 3) / 4);
+#pragma unroll 4
+    for (int w = threadIdx.x; w < words; w += kThreads) outside |= reinterpret_cast<const int*>(p.outside)[w];
+  }
   float kl = 0.0f;
 #pragma unroll 4
   for (int c = group; c < chunks; c += 4) kl += p.kl[(size_t)c * total + i];
   met[group][lane] = kl;
-  // the caller is told of an index outside the range, and finds the losses as they were
-  int outside = 0;
-  if (p.outside)
-    for (long long w = threadIdx.x; w < ((long long)p.AB * p.ASq + 3) / 4; w += kThreads) outside |= reinterpret_cast<const int*>(p.outside)[w];
   if (__syncthreads_or(outside)) return;
   if (!group && q < p.ASq) p.loss[(i / p.slab_rows) * p.ASq + q] = (met[0][lane] + met[1][lane]) + (met[2][lane] + met[3][lane]);
 }
