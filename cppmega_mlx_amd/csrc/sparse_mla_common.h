@@ -26,7 +26,6 @@ struct MlaParams {
   int heads_per_group;
   int num_splits;       // split-KV factor of the MFMA kernel
   int keys_per_split;
-  int f32_partials;     // producer/consumer kernels: a key split's sums are kept in float32, not bfloat16
   int heads_per_wg;     // 0: 32-head tile kernel; 32 or 64: a producer/consumer kernel (sparse_mla_latent.hip, sparse_mla_rows16.hip)
   int plan_level;       // how the launch is planned: see sparse_mla_mfma_plan_within
   int rows16;           // with heads_per_wg: the kernel for 16-bit rows
@@ -75,10 +74,9 @@ int sparse_mla_combine_f32(const MlaParams& p, hipStream_t stream);    // merges
 
 // Key splits of the producer/consumer kernels, whose workgroups have a CU to themselves: the number (up to 16, up to
 // max_keys each) with the least modelled time - whole rounds of 256 workgroups, each with its workgroups' start and end
-// and tile_us per tile of 32 keys, then, with several splits, the merging kernel and its traffic (the float32 sums of
-// `heads` heads per workgroup, written and read).
-// `narrow`: as many splits as doubling until 256 workgroups are there gives, and fewer, keep bfloat16 sums; more
-// splits than that are only worth what they cost in float32.
+// and tile_us per tile of 32 keys, then, with several splits, the merging kernel and the traffic of the sums of `heads`
+// heads per workgroup, written and read.
+// `narrow`: the sums are bfloat16, so there are no more splits than doubling until 256 workgroups are there makes.
 // At plan level 1: the doubled number.
 void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, int heads, bool narrow);
 

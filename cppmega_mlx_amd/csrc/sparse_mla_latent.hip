@@ -36,9 +36,8 @@
 //   pipeline  iteration t: barrier; producers: scores and P of tile t+1; consumers: issue tile
 //             t+4, value product of tile t.  One barrier per tile.
 //
-// Key splits write their accumulators (in fp32 for code rows, for up to 32 heads and where a launch is split
-// further than 256 workgroups ask for, else rounded to bf16) to the workspace as the lanes hold them plus (max, sum)
-// per head; sparse_mla_latent_combine_kernel merges them and does the transposition to [head][channel] that the
+// Key splits write their accumulators (in fp32 for code rows and for up to 32 heads, else rounded to bf16) to the
+// workspace as the lanes hold them plus (max, sum) per head; sparse_mla_latent_combine_kernel merges them and does the transposition to [head][channel] that the
 // single-split path does in LDS.
 
 #include <type_traits>
@@ -155,6 +154,9 @@ __device__ __forceinline__ int split_q32(const uint4 (&x)[4], i32x8& hi, i32x8& 
   }
   return e;
 }
+
+// Key splits of these keep float32: code rows and single groups of heads have few enough of them.
+__host__ __device__ __forceinline__ bool f32_partials(const MlaParams& p) { return p.q_dtype == CPPMEGA_MI355_E4M3 || p.heads_per_group <= 32; }
 
 // NBLK: fp32 scales per key row (1, 2 or 4).
 // ROWS: key rows and queries of 576 e4m3 codes with one fp32 scale each (NBLK = 1): a head's query scale joins the
@@ -778,7 +780,7 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
       // rounded to bf16: the values are relative to the split's own maximum, so their range is that of the
       // output times the split's probability mass)
       // (two accumulator rows of a lane per 16-byte store: [consumer][head half][dvb][row pair][lane][8])
-      if (p.f32_partials) {                        // (uniform)
+      if (f32_partials(p)) {                        // (uniform)
         float* blk = (float*)p.workspace + part_block * (size_t)(2 * kPartFloats) + ((size_t)((role * 2 + hb) * 8) * 64 + lane) * 8;
 #pragma unroll
         for (int dvb = 0; dvb < 4; ++dvb)
@@ -1038,9 +1040,13 @@ bool sparse_mla_latent_supported(const MlaParams& p) {
 bool sparse_mla_latent_only(const MlaParams& p) { return latent_rows(p) && p.heads_per_group > 32; }
 
 void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, int heads, bool narrow) {
-  // (fitted to 216 shapes of 16 and 128 heads, 1 .. 300 queries, 64 .. 2048 keys: 1.2x in the mean against doubling the
-  // splits until 256 workgroups are there, 3x where that ended just above 256 or in splits of four tiles)
-  constexpr double kUnitUs = 7.0, kMergeUs = 5.0, kBytesPerUs = 5e6;
+  // float32 sums: fitted to 216 shapes of 16 and 128 heads, 1 .. 300 queries, 64 .. 2048 keys (1.2x in the mean against
+  // doubling the splits until 256 workgroups are there, 3x where that ended just above 256 or in splits of four tiles).
+  // bfloat16 sums: to 24 shapes of 64 and 128 heads, 1 .. 64 queries, 256 .. 2048 keys; the choice is within 1 us of the
+  // best.  More splits than doubling makes would have to keep float32 sums, and gain nothing then: 128 heads x 1 x 1024
+  // keys 16.8 us in 8 splits, 20.3 in 16; 64 x 4 x 512 16.4 in 4, 18.5 in 8.
+  constexpr double kUnitUs = 7.0;
+  const double merge_us = narrow ? 1.0 : 5.0, bytes_per_us = narrow ? 2.8e6 : 5e6;
   const int tiles = (p.topk + kTK - 1) / kTK;
   int doubled = 1;
   while (units * doubled < 256 && p.topk / (doubled * 2) >= 4 * kTK && doubled < 16) doubled *= 2;
@@ -1048,22 +1054,19 @@ void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us,
   if (p.plan_level > 0) {
     p.num_splits = doubled;
     p.keys_per_split = (tiles + doubled - 1) / doubled * kTK;
-    p.f32_partials = !narrow;
     return;
   }
   double best = 0.0;
   p.num_splits = 0;
-  for (int s = 1; s <= 16; ++s) {
+  for (int s = 1; s <= (narrow ? doubled : 16); ++s) {
     const int per = (tiles + s - 1) / s;
     if (per * kTK > max_keys || (s > 1 && (per < 2 || per == (tiles + s - 2) / (s - 1)))) continue;
-    const bool f32 = !narrow || s > doubled;
     double us = (double)((units * s + 255) / 256) * (kUnitUs + per * tile_us);
-    if (s > 1) us += kMergeUs + 2.0 * (double)units * s * heads * kLat * (f32 ? 4 : 2) / kBytesPerUs;
+    if (s > 1) us += merge_us + 2.0 * (double)units * s * heads * kLat * (narrow ? 2 : 4) / bytes_per_us;
     if (p.num_splits == 0 || us < best) {
       best = us;
       p.num_splits = s;
       p.keys_per_split = per * kTK;
-      p.f32_partials = f32;
     }
   }
 }
@@ -1091,7 +1094,7 @@ int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream) {
   hipLaunchKernelGGL(kernel, grid, block, kSmem, stream, p);
   CM_HIP_CHECK(hipGetLastError());
   if (p.num_splits > 1) {
-    if (p.f32_partials) return sparse_mla_combine_f32(p, stream);
+    if (f32_partials(p)) return sparse_mla_combine_f32(p, stream);
     const dim3 cgrid((unsigned)((size_t)p.B * p.S * p.G * chunks), (unsigned)(4 * (kHeadsWg / 32)));
     hipLaunchKernelGGL((sparse_mla_latent_combine_kernel<false, 2>), cgrid, dim3(256), 0, stream, p);
     CM_HIP_CHECK(hipGetLastError());
@@ -1112,7 +1115,7 @@ size_t sparse_mla_latent_workspace_bytes(const MlaParams& p) {
   if (p.num_splits <= 1) return 0;
   const int chunks = (p.heads_per_group + kHeadsWg - 1) / kHeadsWg;
   const size_t blocks = (size_t)p.B * p.S * p.G * chunks * p.num_splits;
-  return blocks * ((size_t)2 * kPartFloats * (p.f32_partials ? sizeof(float) : sizeof(unsigned short)) + kHeadsWg * 2 * sizeof(float));
+  return blocks * ((size_t)2 * kPartFloats * (f32_partials(p) ? sizeof(float) : sizeof(unsigned short)) + kHeadsWg * 2 * sizeof(float));
 }
 
 }  // namespace cm

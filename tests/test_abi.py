@@ -230,11 +230,11 @@ def test_kernel_choice_and_workspace_for_the_latent_cache_layout():
 
 
 @pytest.mark.parametrize("batch,heads,topk,splits,value_bytes", [
-    (1, 128, 2048, 16, 2), (32, 128, 2048, 4, 2), (64, 128, 2048, 2, 2),        # doubled until 256 workgroups are there, or less often
-    (1, 128, 1024, 16, 4), (1, 64, 512, 8, 4), (1, 128, 256, 4, 4),             # split further: float32 sums
+    (1, 128, 2048, 16, 2), (32, 128, 2048, 4, 2), (64, 128, 2048, 2, 2),
+    (1, 128, 1024, 8, 2), (1, 64, 512, 4, 2), (1, 128, 256, 2, 2), (8, 64, 256, 2, 2),
     (1, 16, 2048, 16, 4),                                                       # up to 32 heads: float32 sums
 ])
-def test_key_splits_that_doubling_would_not_make_keep_float32_sums(batch, heads, topk, splits, value_bytes):
+def test_bfloat16_key_splits_are_no_more_than_doubling_makes(batch, heads, topk, splits, value_bytes):
     need = C.c_size_t(0)
     a = _latent_mla_args(batch=batch, heads=heads, topk=topk)
     assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0
