@@ -678,7 +678,7 @@ PROFILE_WORKLOADS = [
      "(prefill chunk) and one of 32 rows (decode step) per step"),
     ("sparse_mla_prefill_row_layouts", "trace_main", ("fetch_main", "write_main"), None, ("sparse_mla_rows16_kernel<", "sparse_mla_e8m0_rows", "sparse_mla_latent_kernel<1, true"),
      "sparse_mla_fwd q [1,8192,128,576], kv [1,8192,1,576], causal top-2048 indices -> [1,8192,128,512]: "
-     "rows16<true, 2, false> unquantised float16 rows, latent<1, true> e4m3 rows with per-token fp32 scales, "
+     "rows16<true, 2, false> unquantised float16 rows, latent<1, true, true> e4m3 rows with per-token fp32 scales, "
      "rows16<false, 2, true> (behind the conversion of the cache) e4m3 rows with E8M0 bytes per 32 channels"),
     ("sparse_mla_backward", "trace_main", ("fetch_main", "write_main"), None, ("bwd_lists_kernel", "bwd_steps_kernel", "bwd_scores_kernel", "bwd_dq_kernel", "bwd_dkv_kernel", "bwd_sum_kernel"),
      "sparse_mla_bwd q bf16[1,1024,16,576], kv bf16[1,4096,1,576], d_out bf16[1,1024,16,512], topk 256 -> dq bf16, dkv f32 "

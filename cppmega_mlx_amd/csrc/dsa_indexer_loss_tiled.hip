@@ -16,8 +16,9 @@
 // and a lane reduces its own keys, so a head costs one lane exchange.
 //
 // Bound by the exponentials and the multiply-adds in front of them (two per pair and head).  Measured at
-// 4096 positions, 8 heads of 64, lists of 1024: 88 us (lists 21, passes 26 and 32), against 274 us with a workgroup of 8 wavefronts per
-// 16 positions (256 workgroups, the longest with twice the mean work, statistics in LDS per step).
+// 4096 positions, 8 heads of 64, lists of 1024: 92 us a call (lists 16, passes 26 and 31, merge and sum 10),
+// against 274 us with a workgroup of 8 wavefronts per 16 positions (256 workgroups, the longest with twice the
+// mean work, statistics in LDS per step).
 
 #include <algorithm>
 

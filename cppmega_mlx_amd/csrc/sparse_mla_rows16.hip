@@ -1,8 +1,9 @@
 // Sparse MLA forward over 16-bit key rows on the matrix cores (gfx950), with the wavefronts of a
 // workgroup split into score producers and value consumers.
 //
-// Shapes served: queries and key rows of 576 e4m3 codes with one E8M0 byte per 32 channels, and bf16 or float16 queries of 576 = 512 latent + 64 rope channels over key rows of the same
-// type, packed (576) or as latent rows of 512 plus a rope tail of 64; d_v = 512.
+// Shapes served: queries and key rows of 576 e4m3 codes with one E8M0 byte per 32 channels, and bf16 or float16
+// queries of 576 = 512 latent + 64 rope channels over key rows of the same type, packed (576) or as latent rows of
+// 512 plus a rope tail of 64; d_v = 512.
 // A power of two times an e4m3 code is a bfloat16: E8M0 rows become bf16 rows in the workspace first (all of them, about
 // 6 us for 16384), the query's codes on their way to operand order, and nothing is rounded.
 //
