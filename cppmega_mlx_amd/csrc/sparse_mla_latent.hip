@@ -1042,11 +1042,11 @@ bool sparse_mla_latent_only(const MlaParams& p) { return latent_rows(p) && p.hea
 void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, int heads, bool narrow) {
   // float32 sums: fitted to 216 shapes of 16 and 128 heads, 1 .. 300 queries, 64 .. 2048 keys (1.2x in the mean against
   // doubling the splits until 256 workgroups are there, 3x where that ended just above 256 or in splits of four tiles).
-  // bfloat16 sums: to 24 shapes of 64 and 128 heads, 1 .. 64 queries, 256 .. 2048 keys; the choice is within 1 us of the
-  // best.  More splits than doubling makes would have to keep float32 sums, and gain nothing then: 128 heads x 1 x 1024
+  // bfloat16 sums: to 24 shapes of 64 and 128 heads, 1 .. 64 queries, 256 .. 2048 keys (the merging kernel takes the
+  // splits four at a time); the choice is within 1 us of the best.  More splits than doubling makes would have to keep float32 sums, and gain nothing then: 128 heads x 1 x 1024
   // keys 16.8 us in 8 splits, 20.3 in 16; 64 x 4 x 512 16.4 in 4, 18.5 in 8.
   constexpr double kUnitUs = 7.0;
-  const double merge_us = narrow ? 1.0 : 5.0, bytes_per_us = narrow ? 2.8e6 : 5e6;
+  const double merge_us = narrow ? 0.7 : 5.0, group_us = narrow ? 0.3 : 0.0, bytes_per_us = narrow ? 2.9e6 : 5e6;
   const int tiles = (p.topk + kTK - 1) / kTK;
   int doubled = 1;
   while (units * doubled < 256 && p.topk / (doubled * 2) >= 4 * kTK && doubled < 16) doubled *= 2;
@@ -1062,7 +1062,7 @@ void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us,
     const int per = (tiles + s - 1) / s;
     if (per * kTK > max_keys || (s > 1 && (per < 2 || per == (tiles + s - 2) / (s - 1)))) continue;
     double us = (double)((units * s + 255) / 256) * (kUnitUs + per * tile_us);
-    if (s > 1) us += merge_us + 2.0 * (double)units * s * heads * kLat * (narrow ? 2 : 4) / bytes_per_us;
+    if (s > 1) us += merge_us + (s + 3) / 4 * group_us + 2.0 * (double)units * s * heads * kLat * (narrow ? 2 : 4) / bytes_per_us;
     if (p.num_splits == 0 || us < best) {
       best = us;
       p.num_splits = s;
