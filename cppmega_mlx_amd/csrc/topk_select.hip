@@ -37,6 +37,7 @@
 // those bins as empty instead of every element being tested.
 
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -53,6 +54,7 @@ struct TopkParams {
   const int* ends;
   int* out;
   int rows, width, k, order, neg_inf_masked;
+  int first_past;  // rows from here on end less than a whole piece of four columns in front of the buffer's end
   int sort_len;  // power of two >= k, 256 at least, used by the value-descending order
   // Rows too wide for one workgroup's fast path are selected in two stages (tile kernel only):
   // stage 1 launches one workgroup per (row, segment of seg_width columns) and writes the
@@ -351,8 +353,7 @@ __global__ __launch_bounds__(THREADS, E > 16 ? 4 : 8) void topk_tile_kernel(cons
     const bool any = c0 < end && c0 + E > start;          // (a run with nothing selectable is not read)
     // The last piece of a row may reach up to three columns past it: into what lies in front of the next row or the next
     // rows, which is fine, but the buffer may end with the last row's last column, whatever the pitch.
-    const bool past = (T & 3) != 0 && MODE != 2 &&
-                      (long long)row * p.row_stride + base + ((T + 3) & ~3) > (p.rows - 1) * p.row_stride + p.width;     // (uniform)
+    const bool past = (T & 3) != 0 && MODE != 2 && row >= p.first_past;     // (uniform)
     if (!past) {
 #pragma unroll
       for (int i = 0; i < E / 4; ++i) {
@@ -842,6 +843,9 @@ int topk_select_launch(const cppmega_mi355_topk_args_t& a, hipStream_t stream) {
   TopkParams p;
   p.scores = a.scores; p.row_stride = a.row_stride; p.starts = a.starts; p.ends = a.ends; p.out = a.indices;
   p.rows = a.rows; p.width = a.width; p.k = a.k; p.order = a.order; p.neg_inf_masked = a.neg_inf_is_masked ? 1 : 0;
+  // (rows - 1 - row) * row_stride < d, the columns that the last piece reaches past the row
+  const int d = -a.width & 3;
+  p.first_past = d ? (int)std::max<long long>(a.rows - 1 - (d - 1) / a.row_stride, 0) : a.rows;
   int sort_len = 256;
   while (sort_len < a.k) sort_len <<= 1;
   p.sort_len = sort_len;
