@@ -74,7 +74,6 @@ constexpr int kRopeBytes = 4 * 1024;            // [sj][s] planes
 constexpr int kScaleBytes = kTK * 4 * 4;        // up to four fp32 scales per row: [row][block]
 constexpr int kSlotBytes = kLatBytes + kRopeBytes + kScaleBytes;   // 23552
 constexpr int kRingBytes = kRing * kSlotBytes;  // 104960
-constexpr int kSkipped = (int)0x80000000u;       // sign bit of a staged key
 constexpr int kMaxKeys = 2048;                  // keys of one split (their rows are staged in LDS)
 constexpr int kKeyInts = kMaxKeys + kTK;
 constexpr int kHeadsWg = 64;
@@ -228,7 +227,7 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     for (int i = tid; i < kRing * kTK; i += 512)
       reinterpret_cast<float*>(smem + (i / kTK) * kSlotBytes + kLatBytes + kRopeBytes)[i % kTK] = 1.0f;
   }
-  // ---- cache rows of this split's keys -> LDS (a skipped one: kSkipped and a row to fetch in its place) ----
+  // ---- cache rows of this split's keys -> LDS (-1 = skipped) ----
   int* last_valid = reinterpret_cast<int*>(stats);          // [8], one per wavefront (the statistics come much later)
   // thread t takes list entries t, t + 512, ..: every index word is requested before the first one
   // is looked at (one memory round trip), unconditionally, with positions clamped to the list.
@@ -253,30 +252,24 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     }
   }
   auto stage_keys = [&]() {
-    int row[kRounds];
-    bool ok[kRounds];
-    int mine = -1, spare = 0;                       // spare: (uniform) a cache row that this wavefront's entries name
+    const int ctid = tid;
+    int* lo = idx_lo; int* hi = idx_hi;
+    int mine = -1;
 #pragma unroll
     for (int r = 0; r < kRounds; ++r) {
-      ok[r] = false;
-      row[r] = 0;
       if (r * 512 < list_tiles * kTK) {
-        const int i = tid + 512 * r;
-        const long long k = wide ? (long long)(((unsigned long long)(unsigned)idx_hi[r] << 32) | (unsigned)idx_lo[r]) : (long long)idx_lo[r];
-        ok[r] = i < n_keys && k >= 0 && k < p.Skv;
-        row[r] = (int)k;
-        if (ok[r]) mine = i;
-        const unsigned long long any = __ballot(ok[r]);
-        if (any) spare = __builtin_amdgcn_readlane(row[r], __ffsll(any) - 1);
+        const int i = ctid + 512 * r;
+        const long long k = wide ? (long long)(((unsigned long long)(unsigned)hi[r] << 32) | (unsigned)lo[r]) : (long long)lo[r];
+        const bool ok = i < n_keys && k >= 0 && k < p.Skv;
+        int row = ok ? (int)k : -1;
+        if (i < list_tiles * kTK) keys[i] = row;
+        if (ok) mine = i;
         // a tile is the 32 consecutive entries of half a wavefront; the masked-key path also serves a
         // non-positive softmax scale (the plain path takes maxima before scaling)
-        const unsigned long long okm = __ballot(ok[r] && sm_scale > 0.0f);
+        const unsigned long long okm = __ballot(ok && sm_scale > 0.0f);
         if ((lane & 31) == 0 && i < list_tiles * kTK) tvalid[i / kTK] = (unsigned)(okm >> (lane & 32)) == 0xffffffffu;
       }
     }
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r)
-      if (r * 512 < list_tiles * kTK && tid + 512 * r < list_tiles * kTK) keys[tid + 512 * r] = ok[r] ? row[r] : spare | kSkipped;
     mine = max(mine, __shfl_xor(mine, 1, 64));
     mine = max(mine, __shfl_xor(mine, 2, 64));
     mine = max(mine, __shfl_xor(mine, 4, 64));
@@ -284,21 +277,6 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     mine = max(mine, __shfl_xor(mine, 16, 64));
     mine = max(mine, __shfl_xor(mine, 32, 64));
     if (lane == 0) last_valid[wave] = mine;
-  };
-  // A wavefront without a valid key has no row for its entries to fetch.  Where the last valid key stands behind them - a
-  // long run of skipped entries inside a list - they take that key's row, behind one more barrier.
-  auto finish_keys = [&]() {
-    int m = -1;
-    bool gap = false;
-#pragma unroll
-    for (int w = 0; w < 8; ++w) m = max(m, last_valid[w]);
-#pragma unroll
-    for (int w = 0; w < 8; ++w) gap |= last_valid[w] < 0 && 64 * w <= m;
-    if (!__builtin_amdgcn_readfirstlane(gap)) return;           // (uniform over the workgroup)
-    const int row = keys[m];
-    if (last_valid[wave] < 0)
-      for (int i = tid; i < list_tiles * kTK; i += 512) keys[i] = row | kSkipped;
-    __syncthreads();
   };
   // causal padding puts the skipped (-1) slots at the end of a list: tiles past the last valid key do nothing
   auto count_tiles = [&]() {
@@ -373,7 +351,6 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
       for (int r = 0; r < 2; ++r) qr[r] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qstage + n * kQPitch + (64 + 4 * r + kg) * 16));
     }
     __syncthreads();                                // keys[] is complete
-    finish_keys();
     const int n_tiles = count_tiles();
     int qexp = 0;
     if (!BF16)
@@ -602,9 +579,14 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   // =======================================================================================
   stage_keys();
   __syncthreads();                                // keys[] is complete
-  finish_keys();
   const int n_tiles = count_tiles();
-  // HBM -> LDS.  A skipped key fetches a row that its split does select (its probability is zero, but a row that
+  int spare_row = 0;
+  if (n_tiles > 0) {
+    int m = -1;
+    for (int w = 0; w < 8; ++w) m = max(m, last_valid[w]);
+    spare_row = __builtin_amdgcn_readfirstlane(keys[m]);
+  }
+  // HBM -> LDS.  A skipped key fetches its split's last valid row instead (its probability is zero, but a row that
   // nobody selected may hold NaN or infinity), so every tile is the same six load instructions per wavefront and the
   // in-order load counter can be waited on by count.  The loads are inline assembly (the compiler would otherwise order
   // every later LDS read behind them) with a uniform 64-bit base and a 32-bit byte offset per lane:
@@ -640,9 +622,9 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   auto dma_prepare = [&](int tau, unsigned slot_off) {
     dma_slot = smem_base + slot_off;
     const int* tk = keys + tau * kTK;
-    // (the products take the lower 24 bits: the rows, without kSkipped)
-    const unsigned k0 = tk[lane & 15], k1 = tk[16 + (lane & 15)];   // this lane's key of sub-tile 0 / 1
-    const unsigned ks = tk[sc_row];
+    auto fetched = [&](int k) { return (unsigned)(k >= 0 ? k : spare_row); };
+    const unsigned k0 = fetched(tk[lane & 15]), k1 = fetched(tk[16 + (lane & 15)]);   // this lane's key of sub-tile 0 / 1
+    const unsigned ks = fetched(tk[sc_row]);
     off_l0 = __umul24(k0, lat_step) + lat_lane;
     off_l1 = __umul24(k1, lat_step) + lat_lane;
     off_r = __umul24((role >> 1) ? k1 : k0, rope_step) + rope_lane;
