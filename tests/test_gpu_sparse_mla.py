@@ -665,3 +665,32 @@ def test_scores_are_float32_sums(device, rows, H, topk):
         args, kw = (q, codes), dict(kv_spec=ops.QuantSpec(_lib.SCALE_F32_BLOCK, scale, 128), kv_rope=rope)
     ops.sparse_mla_forward(args[0], args[1], to_dev(idx.astype(np.int32), device), sm_scale=sm, d_v=512, out=out, lse=lse, kernel="mfma", **kw)
     _assert_close(out, lse, want_out, want_lse, lse_tol=1.6e-5)
+
+
+@pytest.mark.parametrize("valid", [[0], [63], [700], [0, 700], [511, 513], list(range(64, 128)) + [1999], [10, 600, 601, 1300]])
+@pytest.mark.parametrize("rows", ["latent", "codes"])
+def test_long_runs_of_skipped_entries(device, rows, valid):
+    """Wavefronts that stage list entries of which none is valid, in front of, behind and between valid ones; a cache row
+    that no list names is not finite."""
+    from cppmega_mlx_amd import _lib
+    H, Skv, topk = 64, 500, 2000
+    rng = np.random.default_rng(len(valid))
+    idx = np.full((1, 300, 1, topk), -1, dtype=np.int64)               # (one piece: enough queries for no key splits)
+    idx[:, :, :, valid] = 1 + rng.integers(0, Skv - 1, (1, 300, 1, len(valid)))
+    q, qf = bf16_pair(rng.standard_normal((1, 300, H, 576)), device)
+    out = torch.zeros((1, 300, H, 512), dtype=torch.float32, device=device)
+    if rows == "latent":
+        codes, scale, rope, decoded = latent_cache(rng, 1, Skv, 1, 512, 64, device, pow2=True)
+        codes[0, 0], scale[0, 0], rope[0, 0] = 0x7f, float("inf"), float("nan")
+        ops.sparse_mla_forward(q, codes, to_dev(idx.astype(np.int32), device), sm_scale=0.04, d_v=512, out=out, kernel="mfma",
+                               kv_spec=ops.QuantSpec(_lib.SCALE_F32_BLOCK, scale, 128), kv_rope=rope)
+    else:
+        qc, qs = fp8.quantize_per_token(qf)
+        kc, ks = fp8.quantize_per_token(rng.standard_normal((1, Skv, 1, 576)).astype(np.float32))
+        qf, decoded = om.dequant_per_token(qc, qs), om.dequant_per_token(kc, ks)
+        kc[0, 0], ks[0, 0] = 0x7f, np.inf
+        ops.sparse_mla_forward(to_dev(qc, device), to_dev(kc, device), to_dev(idx.astype(np.int32), device), sm_scale=0.04, d_v=512, out=out, kernel="mfma",
+                               q_spec=ops.QuantSpec(_lib.SCALE_PER_TOKEN, to_dev(qs, device)), kv_spec=ops.QuantSpec(_lib.SCALE_PER_TOKEN, to_dev(ks, device)))
+    for s in (0, 7, 299):
+        want, _ = om.sparse_mla_oracle(qf[:, s:s + 1], decoded, idx[:, s:s + 1], sm_scale=0.04, d_v=512)
+        _assert_close(out[:, s:s + 1], None, want, None)
