@@ -22,16 +22,18 @@ from . import _lib
 
 
 class _Host:
-    """The native launch path, loaded at the first call.  Where it cannot be loaded a call is not the plain case: the
-    helpers behind it load the library, which raises the reason."""
+    """Stands in for the native launch path until a first call loads it.  Where it cannot be loaded a call is not the
+    plain case: the helpers behind it load the library, which raises the reason."""
 
     def __getattr__(self, name: str):
+        global host
         try:
-            found = getattr(_lib.load_host(), name)
+            loaded = _lib.load_host()
         except _lib.NativeLibraryError:
             return lambda *args: None
-        setattr(self, name, found)
-        return found
+        if host is self:
+            host = loaded                # (a module's attributes are found faster than those of this class)
+        return getattr(loaded, name)
 
 
 host = _Host()
