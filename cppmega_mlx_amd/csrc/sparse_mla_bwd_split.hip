@@ -12,16 +12,16 @@
 //            16-bit planes each (hi = round(x), lo = round(x - hi), a term is good to 2^-17), and q and d_out by
 //            channel, both as dkv's matrix instructions take them: a load is 1 KB in a row;
 //   dq       per (query, 16 heads, 144 channels): dQ^T = K^T . dS^T over 32-key tiles staged in LDS;
-//   dkv      per (four bands, 64 channels, share of the steps): dS^T . Q + P^T . dO of every step, added to a
+//   dkv      per (band, 64 channels, share of the steps): dS^T . Q + P^T . dO of every step, added to a
 //            float32 tile in LDS, written out once;
 //   sum      over the shares, when there are several.
 //
 // Nothing is added in an order that varies: the same input gives the same bits.
 //
-// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 172 us (561 us with the atomics): lists 8,
-// steps 7, scores 38, dq 31, dkv 89, sum 9.  dkv is bound by the vector cache (27 M accesses of 64 bytes, 51 us if
-// it never waited: 4 KB of q and d_out and about 1 KB of planes for a step's 9 keys of 16) and by the issue of its
-// one wavefront per SIMD; scores and dq by the gather of 302 MB of key rows each.
+// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 167 us (561 us with the atomics): lists 7,
+// steps 7, scores 38, dq 31, dkv 82, sum 9.  dkv is bound by the vector cache (27 M accesses of 64 bytes: 4 KB of q and
+// d_out and about 1 KB of planes for a step's 9 keys of 16) and ends with the CUs whose four bands are all full; scores
+// and dq by the gather of 302 MB of key rows each.
 
 #include <algorithm>
 
@@ -36,9 +36,9 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int kBands = 4;              // bands of keys in a dkv tile
-constexpr int kBandKeys = 150;         // at most: 601 rows of 64 floats (one for nobody) are 154 KB of LDS
-constexpr int kAhead = 4;              // steps on their way in dkv
+constexpr int kBandKeys = 150;         // at most: 151 rows of 64 floats (one for nobody) are 39 KB of LDS, four tiles to a CU
+constexpr int kAhead = 4;              // steps on their way in a wavefront of dkv
+constexpr int kStepGroup = 2 * kAhead; // steps come in whole rounds of dkv's two wavefronts
 constexpr int kAgain = 1 << 30;        // mark of a slot whose key occurs earlier in the same 16 slots
 constexpr int kHeads = 16;             // heads of an item
 constexpr int kRowBytes = 128;         // of planes per key
@@ -55,9 +55,9 @@ struct SplitParams {
   int* keys;                    // [lists][stride] ascending, -1 behind the last
   int* starts;                  // [lists][bands + 2]: first slot of each band, the number of keys, whether one is marked kAgain
   int* step_starts;             // [lists][bands]: each band's first step among the list's
-  int* rows;                    // [lists][list_steps][16]: where in its tile of dkv a slot's key stands, band by band in whole steps
+  unsigned char* rows;          // [lists][list_steps][16]: the row of a slot's key in its tile of dkv, band by band in whole steps
   int* band_steps;              // the number of steps so far, then [B * G * bands][first, number]
-  i32x4* steps;                 // byte offsets of planes, rows (| keys | 32 if one may be marked), by_channel, keys
+  i32x4* steps;                 // byte offset of planes, 64 times the step's place in rows (| keys | 32 if one may be marked), byte offsets of by_channel, keys
   char* planes;                 // [lists][chunks][hi, lo][dS heads 0-7, 8-15, P heads 0-7, 8-15][stride][8]
   unsigned short* by_channel;   // [lists][chunks][D / 64][channel % 4][q heads 0-7, 8-15, d_out heads 0-7, 8-15][16 channels][8]
   float* part;                  // [shares][B, Skv, G, D]
@@ -67,14 +67,15 @@ struct SplitParams {
   int s0, ns;                   // queries of this slab: s0 .. s0 + ns of every sequence; list = (b * ns + s - s0) * G + g
   int chunks;                   // of 16 heads per group
   int stride;                   // key slots per list: topk in whole tiles, and two tiles to read past
-  int tiles, bands, band_keys, shares;                  // bands = tiles * kBands of band_keys keys
+  int bands, band_keys, shares;
   int list_steps;               // at most, of 16 slots of one band
-  unsigned dead_step;           // byte offset in rows of a step of no keys
+  unsigned dead_step;           // 64 times the place in rows of a step of no keys
   int accumulate;               // add to dkv
   float sm_scale;
 };
 
-constexpr int kDeadRow = kBands * kBandKeys;           // of slots of no key
+constexpr int kDeadRow = kBandKeys;                    // of slots of no key
+static_assert(kDeadRow < 256, "rows are bytes");
 
 // ---- lists -----------------------------------------------------------------------------------
 // The valid keys by band in LDS, then each to its rank within the band.
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(kThreads) void bwd_lists_kernel(const SplitParams p
   const int g = (int)(list % p.G), s = (int)((list / p.G) % p.ns), b = (int)(list / ((size_t)p.G * p.ns));
   const size_t src = (((size_t)b * p.S + p.s0 + s) * p.G + g) * (size_t)p.topk;
   if (list == 0 && tid == 0) p.band_steps[0] = 0;
-  if (list == 0 && tid < 16) p.rows[p.dead_step / 4 + tid] = kDeadRow * 256;
+  if (list == 0 && tid < 16) p.rows[p.dead_step / 4 + tid] = kDeadRow;
   for (int r = tid; r < p.bands; r += kThreads) fill[r] = 0;
   if (tid == 0) *again = 0;
   __syncthreads();
@@ -144,17 +145,17 @@ __global__ __launch_bounds__(kThreads) void bwd_lists_kernel(const SplitParams p
   __syncthreads();
   // a key that its step of 16 (from the band's first slot on) holds already is marked, and has no row
   int* out = p.keys + list * (size_t)p.stride;
-  int* rows = p.rows + list * (size_t)p.list_steps * 16;
+  unsigned char* rows = p.rows + list * (size_t)p.list_steps * 16;
   for (int k = tid; k < p.stride; k += kThreads) {
     int v = -1;
     if (k < valid) {
       v = sorted[k];
-      const int of = v / p.band_keys, nth = k - begin[of], row = v - of / kBands * (kBands * p.band_keys);
+      const int of = v / p.band_keys, nth = k - begin[of], row = v - of * p.band_keys;
       const bool marked = (nth & 15) != 0 && sorted[k - 1] == v;
-      int* at = rows + step_of[of] * 16 + nth;
-      *at = (marked ? kDeadRow : row) * 256;
+      unsigned char* at = rows + step_of[of] * 16 + nth;
+      *at = (unsigned char)(marked ? kDeadRow : row);
       if (k + 1 == fill[of])
-        for (int e = nth + 1; e & 15; ++e) *++at = kDeadRow * 256;
+        for (int e = nth + 1; e & 15; ++e) *++at = kDeadRow;
       if (marked) {
         v |= kAgain;
         *again = 1;
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(kStepThreads) void bwd_steps_kernel(const SplitPara
     if (w < wave) at += sums[w];
     all += sums[w];
   }
-  const int padded = (all + kAhead - 1) / kAhead * kAhead;            // with steps whose rows are all dead
+  const int padded = (all + kStepGroup - 1) / kStepGroup * kStepGroup;            // with steps whose rows are all dead
   if (tid == 0) {
     base_of = atomicAdd(p.band_steps, padded);
     p.band_steps[2 + 2 * blockIdx.x] = base_of;
@@ -524,103 +525,133 @@ __global__ __launch_bounds__(64, 3) void bwd_dq_kernel(const SplitParams p) {
 }
 
 // ---- dkv -----------------------------------------------------------------------------------------
-constexpr int kDkvThreads = 256;                       // a wavefront per band
-// A wavefront owns its band of the tile, so it adds with plain reads and writes: ds_add_f32 takes a lane at a time
-// (1160 us for a form of this kernel that took 280 with a plain write in its place).  16 bytes per lane of whole rows
-// meet in no bank.  Two wavefronts per band, 32 channels each, read the planes twice (110 us); one per 16 channels
+// A workgroup is two wavefronts and one band's tile, four workgroups to a CU.  The steps of a band are added one after
+// the other (they may name the same key), with plain reads and writes: ds_add_f32 takes a lane at a time (1160 us for a
+// form of this kernel that took 280 with a plain write in its place).  So the wavefronts take turns: while one reads its
+// step's rows, adds and writes them, the other has its operands arrive and multiplies: 82 us at the shape above and 135
+// with 64 heads (512 queries, 256 of 2048 keys), where one wavefront per band, four bands to a workgroup, took 86 and 160.
+// 16 bytes per lane of whole rows meet in no bank.  Two wavefronts per band with 32 channels each read the planes twice (110 us); one per 16 channels
 // of 600 keys, four times (315 us).
+constexpr int kDkvThreads = 128;
+// A base and 32-bit offsets: a scalar one per step, a lane's own for good.
+struct Slab {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ explicit Slab(const void* base) : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000)) {}
+  template <class T>
+  __device__ T load(int of_lane, int of_all) const { return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(rsrc, of_lane, of_all, 0)); }
+  __device__ unsigned load32(int of_lane, int of_all) const { return __builtin_amdgcn_raw_buffer_load_b32(rsrc, of_lane, of_all, 0); }
+};
 template <bool F16>
-__global__ __launch_bounds__(kDkvThreads, 1) void bwd_dkv_kernel(const SplitParams p) {
+__global__ __launch_bounds__(kDkvThreads, 2) void bwd_dkv_kernel(const SplitParams p) {
   extern __shared__ __align__(16) float tile[];        // [kDeadRow + 1][64], the last row for lanes of no key
   const int tid = (int)threadIdx.x, lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // consecutive tiles read the same planes and rows: an XCD (launches go round them) takes a run of tiles
   const int per_xcd = (int)gridDim.x / 8, work = (int)blockIdx.x % 8 * per_xcd + (int)blockIdx.x / 8;
-  const int cols = (p.D + 63) / 64, range = work % p.tiles, ch0 = work / p.tiles % cols * 64;
-  const int share = work / (p.tiles * cols) % p.shares, bg = work / (p.tiles * cols * p.shares);
+  const int cols = (p.D + 63) / 64, band = work % p.bands, ch0 = work / p.bands % cols * 64;
+  const int share = work / (p.bands * cols) % p.shares, bg = work / (p.bands * cols * p.shares);
   if (bg >= p.B * p.G) return;
   const int g = bg % p.G, b = bg / p.G;
-  const int k0 = range * kBands * p.band_keys, rows = min(kBands * p.band_keys, p.Skv - k0);
+  const int k0 = band * p.band_keys, rows = min(p.band_keys, p.Skv - k0);
   for (int e = tid; e < (kDeadRow + 1) * 16; e += kDkvThreads) reinterpret_cast<f32x4*>(tile)[e] = f32x4{0.f, 0.f, 0.f, 0.f};
-  __syncthreads();
 
-  const int* all = p.band_steps + 2 + 2 * (bg * p.bands + range * kBands + wave);
-  const int groups = __builtin_amdgcn_readfirstlane(all[1]) / kAhead;
-  const int first = (int)((long long)groups * share / p.shares) * kAhead, n = (int)((long long)groups * (share + 1) / p.shares) * kAhead - first;
+  const int* all = p.band_steps + 2 + 2 * (bg * p.bands + band);
+  const int groups = __builtin_amdgcn_readfirstlane(all[1]) / kStepGroup;
+  const int first = (int)((long long)groups * share / p.shares) * kStepGroup;
+  const int n = ((int)((long long)groups * (share + 1) / p.shares) * kStepGroup - first) / 2;      // of this wavefront
   if (n > 0) {
-    const i32x4* steps = p.steps + __builtin_amdgcn_readfirstlane(all[0]) + first;
+    const i32x4* steps = p.steps + __builtin_amdgcn_readfirstlane(all[0]) + first + wave;          // every other one
     const unsigned plane_lane = ((unsigned)kg * p.stride + l16) * 16, lo_plane = (unsigned)p.stride * 64;
-    const unsigned qo_lane = lane * 16;
-    const char* rows_of = reinterpret_cast<const char*>(p.rows);
-    const char* by_channel = reinterpret_cast<const char*>(p.by_channel) + (size_t)ch0 * 64;
+    const Slab planes(p.planes), rows_of(p.rows), by_channel(reinterpret_cast<const char*>(p.by_channel) + (size_t)ch0 * 64);
+    char* const tile_lane = reinterpret_cast<char*>(tile) + l16 * 16;
+    // a step's operands are on their way from its predecessor kAhead before it in the same registers: planes and rows
+    // of q and d_out as soon as that one is multiplied, the places of its keys in the tile as soon as it is added
     bf16x8 hi[kAhead], lo[kAhead], qo[kAhead][4];
-    i32x4 slot[kAhead];
-    int marked[kAhead], key_at[kAhead];
-    i32x4 cur = steps[min(lane, n - 1)], next = steps[min(64 + lane, n - 1)];
+    unsigned slot[kAhead];                             // rows of keys 4 * kg + v in its bytes
+    int row_word[kAhead], key_at[kAhead], row_word_of[kAhead], key_at_of[kAhead];
+    i32x4 cur = steps[2 * min(lane, n - 1)], next = steps[2 * min(64 + lane, n - 1)];
     auto request = [&](int i, int at) {
-      const unsigned plane = __builtin_amdgcn_readlane(cur[0], at), row = __builtin_amdgcn_readlane(cur[1], at);
-      const unsigned operand = __builtin_amdgcn_readlane(cur[2], at);
-      marked[i] = row & 32;
+      const int plane = __builtin_amdgcn_readlane(cur[0], at), operand = __builtin_amdgcn_readlane(cur[2], at);
+      row_word[i] = __builtin_amdgcn_readlane(cur[1], at);
       key_at[i] = __builtin_amdgcn_readlane(cur[3], at);
-      const char *planes = p.planes + plane, *channels = by_channel + operand, *lo_planes = planes + lo_plane;
-      if (l16 < (int)(row & 31)) {                     // (the cache serves the lanes that ask)
-        hi[i] = *reinterpret_cast<const bf16x8*>(planes + plane_lane);
-        lo[i] = *reinterpret_cast<const bf16x8*>(lo_planes + plane_lane);
+      if (l16 < (row_word[i] & 31)) {                  // (the cache serves the lanes that ask)
+        hi[i] = planes.load<bf16x8>(plane_lane, plane);
+        lo[i] = planes.load<bf16x8>(plane_lane, plane + (int)lo_plane);
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) qo[i][j] = *reinterpret_cast<const bf16x8*>(channels + qo_lane + j * 1024);
-      slot[i] = *reinterpret_cast<const i32x4*>(rows_of + (row & ~63u) + kg * 16);
+      for (int j = 0; j < 4; ++j) qo[i][j] = by_channel.load<bf16x8>(lane * 16 + j * 1024, operand);
     };
+    auto request_slots = [&](int i) {
+      slot[i] = rows_of.load32(kg * 4, (int)((unsigned)row_word[i] >> 6) * 16);
+      row_word_of[i] = row_word[i];
+      key_at_of[i] = key_at[i];
+    };
+    f32x4 add[4];
+    auto multiply = [&](int i, int ahead) {            // the step in registers i, which then take the step `ahead`
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) request(i, i);
-    for (int step = 0; step < n; step += kAhead) {
-      const int ahead = step + kAhead;
+      for (int j = 0; j < 4; ++j) add[j] = mm<F16>(hi[i], qo[i][j], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int j = 0; j < 4; ++j) add[j] = mm<F16>(lo[i], qo[i][j], add[j]);
       if ((ahead & 63) == 0) {
         cur = next;
-        next = steps[min(ahead + 64 + lane, n - 1)];
+        next = steps[2 * min(ahead + 64 + lane, n - 1)];
+      }
+      request(i, ahead & 63);
+    };
+    auto add_up = [&](int i) {                         // keys 4 * kg + v, channels 4 * l16 + j
+      f32x4 was[4], *at[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        at[v] = reinterpret_cast<f32x4*>(tile_lane + (slot[i] >> 8 * v & 0xff) * 256);
+        was[v] = *at[v];
       }
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        // keys 4 * kg + v, channels 4 * l16 + j
-        f32x4* at[4];
-        f32x4 was[4], add[4];
+      for (int v = 0; v < 4; ++v) *at[v] = was[v] + f32x4{add[0][v], add[1][v], add[2][v], add[3][v]};
+      if (row_word_of[i] & 32) {                       // (a list that names a key twice)
+        // the lanes of one kg at a time: the others may hold the same key, and the row each has added to is written
+        // before the next one reads it (to a single thread the four rounds are one, hence the fences)
+        auto turn = [] {
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+        };
+        turn();
+        const int* keys = p.keys + key_at_of[i] / 4 + kg * 4;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          at[v] = reinterpret_cast<f32x4*>(reinterpret_cast<char*>(tile) + slot[i][v] + l16 * 16);
-          was[v] = *at[v];
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) add[j] = mm<F16>(hi[i], qo[i][j], f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-        for (int j = 0; j < 4; ++j) add[j] = mm<F16>(lo[i], qo[i][j], add[j]);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) *at[v] = was[v] + f32x4{add[0][v], add[1][v], add[2][v], add[3][v]};
-        if (marked[i]) {                               // (a list that names a key twice)
-          // the lanes of one kg at a time: the others may hold the same key, and the row each has added to is written
-          // before the next one reads it (to a single thread the four rounds are one, hence the fences)
-          auto turn = [] {
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-          };
-          turn();
-          const int* keys = p.keys + key_at[i] / 4 + kg * 4;
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int slot_of = keys[v], row = (slot_of & ~kAgain) - k0 - wave * p.band_keys;
-            const bool again = slot_of >= 0 && (slot_of & kAgain) && row >= 0 && row < p.band_keys;   // (not of a band behind)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              if (again && kg == k) {
-                f32x4* once_more = reinterpret_cast<f32x4*>(tile + (row + wave * p.band_keys) * 64) + l16;
-                *once_more += f32x4{add[0][v], add[1][v], add[2][v], add[3][v]};
-              }
-              turn();
+          const int slot_of = keys[v], row = (slot_of & ~kAgain) - k0;
+          const bool again = slot_of >= 0 && (slot_of & kAgain) && row >= 0 && row < p.band_keys;   // (not of a band behind)
+#pragma unroll 1
+          for (int k = 0; k < 4; ++k) {
+            if (again && kg == k) {
+              f32x4* once_more = reinterpret_cast<f32x4*>(tile + row * 64) + l16;
+              *once_more += f32x4{add[0][v], add[1][v], add[2][v], add[3][v]};
             }
+            turn();
           }
         }
-        request(i, (ahead + i) & 63);
+      }
+      request_slots(i);
+    };
+    // what was added is in LDS before the other wavefront reads it; loads of global memory stay on their way
+    auto pass_on = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      request(i, i);
+      request_slots(i);
+    }
+    pass_on();                                         // the tile is cleared
+    multiply(0, kAhead);
+    if (wave) pass_on();                               // half a turn behind
+    for (int step = 0; step < n; step += kAhead) {
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        add_up(i);
+        pass_on();
+        multiply((i + 1) % kAhead, step + i + 1 + kAhead);             // (behind the last step: one nobody adds)
+        pass_on();
       }
     }
+    if (!wave) pass_on();
   }
   __syncthreads();
   const bool whole = p.shares > 1;
@@ -649,7 +680,7 @@ __global__ __launch_bounds__(kThreads) void bwd_sum_kernel(const SplitParams p) 
 }
 
 struct Plan {
-  int chunks, stride, tiles, band_keys, shares, ns;
+  int chunks, stride, bands, band_keys, shares, ns;
   size_t keys, starts, step_starts, rows, band_steps, steps, list_steps, planes, by_channel, part, slab_bytes, bytes;
 };
 
@@ -657,23 +688,23 @@ Plan make_plan(const cppmega_mi355_sparse_mla_bwd_args_t& a) {
   Plan l;
   l.chunks = (a.heads / a.kv_groups + kHeads - 1) / kHeads;
   l.stride = (a.topk + 15) / 16 * 16 + 32;
-  l.tiles = (a.seq_kv + kBands * kBandKeys - 1) / (kBands * kBandKeys);
-  l.band_keys = (a.seq_kv + l.tiles * kBands - 1) / (l.tiles * kBands);
-  const size_t lists = (size_t)a.batch * a.kv_groups, bands = (size_t)l.tiles * kBands;      // lists per query position
+  l.bands = (a.seq_kv + kBandKeys - 1) / kBandKeys;
+  l.band_keys = (a.seq_kv + l.bands - 1) / l.bands;
+  const size_t lists = (size_t)a.batch * a.kv_groups, bands = (size_t)l.bands;               // lists per query position
   l.list_steps = a.topk / 16 + std::min<size_t>((size_t)a.topk, bands) + 1;
-  const size_t per_s = lists * (l.stride * 4 + (2 * bands + 2) * 4 + l.list_steps * (64 + 16 * l.chunks) + l.chunks * ((size_t)l.stride * kRowBytes + (size_t)(a.d_qk + 63) / 64 * 4096));
+  const size_t per_s = lists * (l.stride * 4 + (2 * bands + 2) * 4 + l.list_steps * (16 + 16 * l.chunks) + l.chunks * ((size_t)l.stride * kRowBytes + (size_t)(a.d_qk + 63) / 64 * 4096));
   l.ns = (int)std::min<size_t>((size_t)a.seq_q, std::max<size_t>(kSlabBytes / per_s, 1));
-  // a tile of dkv has a CU to itself: as many shares of the steps as bring the tiles to the number of CUs, of eight at least
-  const long long tiles = (long long)l.tiles * ((a.d_qk + 63) / 64) * lists;
-  l.shares = (int)std::max<long long>(1, std::min<long long>(256 / tiles, (long long)l.ns * l.chunks * (a.topk / (bands * 16) + 1) / 8));
+  // a CU holds four tiles of dkv: as many shares of the steps as bring the tiles to four times the number of CUs, of eight at least
+  const long long tiles = (long long)l.bands * ((a.d_qk + 63) / 64) * lists;
+  l.shares = (int)std::max<long long>(1, std::min<long long>(1024 / tiles, (long long)l.ns * l.chunks * (a.topk / (bands * 16) + 1) / 8));
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t here = at; at += (bytes + 255) & ~(size_t)255; return here; };
   l.keys = take(lists * l.ns * l.stride * 4);
   l.starts = take(lists * l.ns * (bands + 2) * 4);
   l.band_steps = take((2 + lists * bands * 2) * 4);
   l.step_starts = take(lists * l.ns * bands * 4);
-  l.rows = take((lists * l.ns * l.list_steps + 1) * 64);
-  l.steps = take((lists * l.ns * l.list_steps * l.chunks + lists * bands * kAhead) * 16);
+  l.rows = take((lists * l.ns * l.list_steps + 1) * 16);
+  l.steps = take((lists * l.ns * l.list_steps * l.chunks + lists * bands * kStepGroup) * 16);
   l.planes = take(lists * l.ns * l.chunks * l.stride * kRowBytes);
   l.by_channel = take(lists * l.ns * l.chunks * ((a.d_qk + 63) / 64) * 4096);
   l.slab_bytes = at;
@@ -702,7 +733,7 @@ int run(SplitParams p, const Plan& l, bool clear, hipStream_t stream) {
     else if (p.topk <= 16 * 8 * 4) hipLaunchKernelGGL((bwd_scores_kernel<F16, 8, 4>), of_items, dim3(512), scores_lds(8), stream, p);
     else hipLaunchKernelGGL((bwd_scores_kernel<F16, 16, 8>), of_items, dim3(1024), scores_lds(16), stream, p);
     hipLaunchKernelGGL(bwd_dq_kernel<F16>, dim3((unsigned)(items * dq_parts)), dim3(64), 0, stream, p);
-    const dim3 tiles((unsigned)((p.tiles * ((p.D + 63) / 64) * p.shares * p.B * p.G + 7) / 8 * 8));
+    const dim3 tiles((unsigned)((p.bands * ((p.D + 63) / 64) * p.shares * p.B * p.G + 7) / 8 * 8));
     hipLaunchKernelGGL(bwd_dkv_kernel<F16>, tiles, dim3(kDkvThreads), dkv_lds, stream, p);
     if (p.shares > 1) {
       const size_t n = (size_t)p.B * p.Skv * p.G * p.D / 4;
@@ -726,7 +757,9 @@ bool sparse_mla_bwd_split_supports(const cppmega_mi355_sparse_mla_bwd_args_t& a)
   const long long bands = ((long long)a.seq_kv + kBandKeys - 1) / kBandKeys;
   if (bands * (a.heads / a.kv_groups > kHeads ? 3 : 1) > a.topk) return false;
   if ((long long)a.batch * a.seq_q * a.heads * ((a.d_qk + 143) / 144) > 0x7fffffffLL) return false;
-  return make_plan(a).slab_bytes < 0x7fffffffu;        // (offsets into a slab are 32 bits)
+  const Plan l = make_plan(a);
+  // offsets into a slab are 32 bits, and so are the places of steps times 64
+  return l.slab_bytes < 0x7fffffffu && (unsigned long long)a.batch * a.kv_groups * l.ns * l.list_steps < (1u << 26);
 }
 
 size_t sparse_mla_bwd_split_workspace_bytes(const cppmega_mi355_sparse_mla_bwd_args_t& a) { return make_plan(a).bytes; }
@@ -741,14 +774,14 @@ int sparse_mla_bwd_split_launch(const cppmega_mi355_sparse_mla_bwd_args_t& a, hi
   p.indices = a.indices; p.sm_scale_dev = a.sm_scale_dev; p.dq = a.dq; p.dkv = a.dkv;
   p.keys = reinterpret_cast<int*>(ws + l.keys); p.starts = reinterpret_cast<int*>(ws + l.starts);
   p.band_steps = reinterpret_cast<int*>(ws + l.band_steps); p.steps = reinterpret_cast<i32x4*>(ws + l.steps);
-  p.step_starts = reinterpret_cast<int*>(ws + l.step_starts); p.rows = reinterpret_cast<int*>(ws + l.rows);
+  p.step_starts = reinterpret_cast<int*>(ws + l.step_starts); p.rows = reinterpret_cast<unsigned char*>(ws + l.rows);
   p.list_steps = (int)l.list_steps; p.dead_step = (unsigned)((size_t)a.batch * a.kv_groups * l.ns * l.list_steps * 64);
   p.planes = ws + l.planes; p.by_channel = reinterpret_cast<unsigned short*>(ws + l.by_channel);
   p.part = reinterpret_cast<float*>(ws + l.part);
   p.dq_dtype = a.dq_dtype; p.index_dtype = a.index_dtype;
   p.B = a.batch; p.S = a.seq_q; p.H = a.heads; p.G = a.kv_groups; p.Skv = a.seq_kv; p.topk = a.topk; p.D = a.d_qk; p.d_v = a.d_v;
   p.channels = (a.d_qk + 63) / 64 * 64;
-  p.chunks = l.chunks; p.stride = l.stride; p.tiles = l.tiles; p.bands = l.tiles * kBands; p.band_keys = l.band_keys;
+  p.chunks = l.chunks; p.stride = l.stride; p.bands = l.bands; p.band_keys = l.band_keys;
   p.sm_scale = a.sm_scale;
   return a.q_dtype == CPPMEGA_MI355_F16 ? run<true>(p, l, a.clear_dkv != 0, stream) : run<false>(p, l, a.clear_dkv != 0, stream);
 }
