@@ -11,19 +11,20 @@
 //            softmax statistics and delta across the workgroup, then P and dS = sm_scale P (dP - delta) as two
 //            16-bit planes each (hi = round(x), lo = round(x - hi), a term is good to 2^-17), and q and d_out by
 //            channel, both as dkv's matrix instructions take them: a load is 1 KB in a row;
-//   dq       per (query, 16 heads, 144 channels): dQ^T = K^T . dS^T over 32-key tiles staged in LDS;
+//   dq       per (query, 16 heads, 144 channels): dQ^T = K^T . dS^T over 32-key tiles staged in LDS (rows of 576 = 512 + 64
+//            channels and up to 512 keys: in the kernel of the scores);
 //   dkv      per (band, 64 channels, share of the steps): dS^T . Q + P^T . dO of every step, added to a
 //            float32 tile in LDS, written out once;
-//   sum      over the shares, when there are several.
-//
-// Nothing is added in an order that varies: the same input gives the same bits.
-//
-// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 167 us (561 us with the atomics): lists 7,
-// steps 7, scores 38, dq 31, dkv 82, sum 9.  dkv is bound by the vector cache (27 M accesses of 64 bytes: 4 KB of q and
-// d_out and about 1 KB of planes for a step's 9 keys of 16) and ends with the CUs whose four bands are all full; scores
-// and dq by the gather of 302 MB of key rows each.
+//   sum      over the shares, when there are // Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 165 us (561 us with the atomics): lists 7, steps 7,
+// scores and dq 68, dkv 82, sum 9.  dkv is bound by the vector cache (27 M accesses of 64 bytes: 4 KB of q and d_out and
+// about 1 KB of planes for a step's 9 keys of 16) and ends with the CUs whose four bands are all full; scores and dq by the
+// gather of 302 MB of key rows each.
+
+ssue of its
+// one wavefront per SIMD; scores and dq by the gather of 302 MB of key rows each.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "mfma_util.h"
@@ -89,7 +90,8 @@ __global__ __launch_bounds__(kThreads) void bwd_lists_kernel(const SplitParams p
   int* step_of = again + 1;                            // [bands + 1]: the band's first step
   const int tid = (int)threadIdx.x, lane = tid & 63;
   const size_t list = blockIdx.x;
-  const int g = (int)(list % p.G), s = (int)((list / p.G) % p.ns), b = (int)(list / ((size_t)p.G * p.ns));
+  const unsigned bs = blockIdx.x / (unsigned)p.G;
+  const int g = (int)(blockIdx.x - bs * (unsigned)p.G), b = (int)(bs / (unsigned)p.ns), s = (int)(bs - (unsigned)b * (unsigned)p.ns);
   const size_t src = (((size_t)b * p.S + p.s0 + s) * p.G + g) * (size_t)p.topk;
   if (list == 0 && tid == 0) p.band_steps[0] = 0;
   if (list == 0 && tid < 16) p.rows[p.dead_step / 4 + tid] = kDeadRow;
@@ -231,33 +233,110 @@ __device__ __forceinline__ uint2 pack4(const float (&v)[4]) {
 }
 // hi and lo planes of 4 values
 template <bool F16>
-__device__ __forceinline__ void put_planes(char* at, size_t to_lo, const float (&v)[4]) {
+__device__ __forceinline__ void planes_of(const float (&v)[4], uint2& hi_plane, uint2& lo_plane) {
   float hi[4], lo[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     hi[i] = v[i] * PlaneScale<F16>::up;
     lo[i] = hi[i] - (F16 ? (float)(_Float16)hi[i] : (float)(__bf16)hi[i]);
   }
-  *reinterpret_cast<uint2*>(at) = pack4<F16>(hi);
-  *reinterpret_cast<uint2*>(at + to_lo) = pack4<F16>(lo);
+  hi_plane = pack4<F16>(hi);
+  lo_plane = pack4<F16>(lo);
+}
+template <bool F16>
+__device__ __forceinline__ void put_planes(char* at, size_t to_lo, const float (&v)[4]) {
+  uint2 hi, lo;
+  planes_of<F16>(v, hi, lo);
+  *reinterpret_cast<uint2*>(at) = hi;
+  *reinterpret_cast<uint2*>(at + to_lo) = lo;
 }
 
 struct Item {
   int g, b, chunk, h0, nh;
   size_t list, bs;
 };
-__device__ __forceinline__ Item item_of(const SplitParams& p, size_t i) {
+// (32-bit divisions: there are fewer than 2^31 items, and the 64-bit ones are long scalar chains)
+__device__ __forceinline__ Item item_of(const SplitParams& p, unsigned i) {
   Item it;
-  it.chunk = (int)(i % p.chunks);
-  it.list = i / p.chunks;
-  it.g = (int)(it.list % p.G);
-  const int s = (int)((it.list / p.G) % p.ns);
-  it.b = (int)(it.list / ((size_t)p.G * p.ns));
+  const unsigned list = i / (unsigned)p.chunks, bs = list / (unsigned)p.G;
+  it.chunk = (int)(i - list * (unsigned)p.chunks);
+  it.list = list;
+  it.g = (int)(list - bs * (unsigned)p.G);
+  it.b = (int)(bs / (unsigned)p.ns);
+  const int s = (int)(bs - (unsigned)it.b * (unsigned)p.ns);
   it.bs = (size_t)it.b * p.S + p.s0 + s;
   const int hg = p.H / p.G;
   it.h0 = it.g * hg + it.chunk * kHeads;
   it.nh = min(kHeads, hg - it.chunk * kHeads);
   return it;
+}
+
+// Softmax statistics of heads 4 * kg + v over all keys: the scores of T tiles of a wavefront become exp2(score - maximum).
+struct Stats { float inv_sum[4], delta[4]; };
+template <int W, int T>
+__device__ __forceinline__ Stats row_stats(float* met, f32x4 (&s)[T], const f32x4 (&dp)[T], float (&m)[4], int wave, int l16, int kg, int tiles) {
+  // over the row of 16 lanes, then over the wavefronts
+#pragma unroll
+  for (int v = 0; v < 4; ++v) m[v] = row_max(m[v]);
+  if (l16 == 0)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) met[(wave * 16 + 4 * kg + v) * 3] = m[v];
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    m[v] = -INFINITY;
+    for (int w = 0; w < W; ++w) m[v] = fmaxf(m[v], met[(w * 16 + 4 * kg + v) * 3]);
+    m[v] = m[v] > -INFINITY ? m[v] : 0.0f;
+  }
+  float l[4] = {0.f, 0.f, 0.f, 0.f}, dot[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    if (wave + i * W >= tiles) break;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      s[i][v] = exp2f(s[i][v] - m[v]);
+      l[v] += s[i][v];
+      dot[v] = fmaf(s[i][v], dp[i][v], dot[v]);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    l[v] = row_sum(l[v]);
+    dot[v] = row_sum(dot[v]);
+  }
+  if (l16 == 0)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      met[(wave * 16 + 4 * kg + v) * 3 + 1] = l[v];
+      met[(wave * 16 + 4 * kg + v) * 3 + 2] = dot[v];
+    }
+  __syncthreads();
+  Stats r;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    float sum = 0.0f, d = 0.0f;
+    for (int w = 0; w < W; ++w) {
+      sum += met[(w * 16 + 4 * kg + v) * 3 + 1];
+      d += met[(w * 16 + 4 * kg + v) * 3 + 2];
+    }
+    r.inv_sum[v] = sum > 0.0f ? 1.0f / sum : 0.0f;
+    r.delta[v] = d * r.inv_sum[v];
+  }
+  return r;
+}
+
+// q and d_out by channel: lane (channel l16 of a block, kg): 8 heads of q (kg 0, 1) or of d_out (kg 2, 3)
+template <int W>
+__device__ __forceinline__ void by_channel(const SplitParams& p, const Item& it, const unsigned short* Qs, const unsigned short* Os, int Dp, int Dvp, int wave, int l16, int kg) {
+  const int tr_row = l16 >> 2, tr_col = (l16 & 3) * 4, D = Dp - 8, dv = Dvp - 8;
+  unsigned short* bc = p.by_channel + (it.list * p.chunks + it.chunk) * (size_t)p.channels * 32 + (l16 & 3) * 512 + kg * 128 + (l16 >> 2) * 8;
+  for (int cb = wave; cb < D / 16; cb += W) {
+    const bool has_v = cb * 16 < dv, from_q = kg < 2 || !has_v;      // (every lane issues the transposing read)
+    const unsigned short* src = from_q ? Qs + (8 * (kg & 1) + tr_row) * Dp + cb * 16 + tr_col : Os + (8 * (kg - 2) + tr_row) * Dvp + cb * 16 + tr_col;
+    bf16x8 v = join(lds_tr16(src), lds_tr16(src + 4 * (from_q ? Dp : Dvp)));
+    if (kg >= 2 && !has_v) v = zero8();
+    *reinterpret_cast<bf16x8*>(bc + (size_t)(cb >> 2) * 2048 + (cb & 3) * 32) = v;
+  }
 }
 
 // ---- scores ------------------------------------------------------------------------------------
@@ -345,52 +424,7 @@ __global__ __launch_bounds__(W * 64, 4) void bwd_scores_kernel(const SplitParams
 #pragma unroll
     for (int v = 0; v < 4; ++v) dp[i][v] = key >= 0 ? da[v] : 0.0f;
   }
-  // statistics of head 4 * kg + v: over the row of 16 lanes, then over the wavefronts
-#pragma unroll
-  for (int v = 0; v < 4; ++v) m[v] = row_max(m[v]);
-  if (l16 == 0)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) met[(wave * 16 + 4 * kg + v) * 3] = m[v];
-  __syncthreads();
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    m[v] = -INFINITY;
-    for (int w = 0; w < W; ++w) m[v] = fmaxf(m[v], met[(w * 16 + 4 * kg + v) * 3]);
-    m[v] = m[v] > -INFINITY ? m[v] : 0.0f;
-  }
-  float l[4] = {0.f, 0.f, 0.f, 0.f}, dot[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < T; ++i) {
-    if (wave + i * W >= tiles) break;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      s[i][v] = exp2f(s[i][v] - m[v]);
-      l[v] += s[i][v];
-      dot[v] = fmaf(s[i][v], dp[i][v], dot[v]);
-    }
-  }
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    l[v] = row_sum(l[v]);
-    dot[v] = row_sum(dot[v]);
-  }
-  if (l16 == 0)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      met[(wave * 16 + 4 * kg + v) * 3 + 1] = l[v];
-      met[(wave * 16 + 4 * kg + v) * 3 + 2] = dot[v];
-    }
-  __syncthreads();
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    float sum = 0.0f, d = 0.0f;
-    for (int w = 0; w < W; ++w) {
-      sum += met[(w * 16 + 4 * kg + v) * 3 + 1];
-      d += met[(w * 16 + 4 * kg + v) * 3 + 2];
-    }
-    l[v] = sum > 0.0f ? 1.0f / sum : 0.0f;
-    dot[v] = d * l[v];
-  }
+  const Stats stat = row_stats<W, T>(met, s, dp, m, wave, l16, kg, tiles);
   char* out = p.planes + (it.list * p.chunks + it.chunk) * (size_t)p.stride * kRowBytes + (size_t)(kg >> 1) * p.stride * 16 + 8 * (kg & 1);
 #pragma unroll
   for (int i = 0; i < T; ++i) {
@@ -399,23 +433,14 @@ __global__ __launch_bounds__(W * 64, 4) void bwd_scores_kernel(const SplitParams
     float pv[4], ds[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      pv[v] = s[i][v] * l[v];
-      ds[v] = pv[v] * (dp[i][v] - dot[v]) * sm_scale;
+      pv[v] = s[i][v] * stat.inv_sum[v];
+      ds[v] = pv[v] * (dp[i][v] - stat.delta[v]) * sm_scale;
     }
     char* at = out + (size_t)(t * 16 + l16) * 16;
     put_planes<F16>(at, (size_t)p.stride * 64, ds);
     put_planes<F16>(at + (size_t)p.stride * 32, (size_t)p.stride * 64, pv);
   }
-  // q and d_out by channel: lane (channel l16 of a block, kg): 8 heads of q (kg 0, 1) or of d_out (kg 2, 3)
-  const int tr_row = l16 >> 2, tr_col = (l16 & 3) * 4;
-  unsigned short* bc = p.by_channel + (it.list * p.chunks + it.chunk) * (size_t)p.channels * 32 + (l16 & 3) * 512 + kg * 128 + (l16 >> 2) * 8;
-  for (int cb = wave; cb < D / 16; cb += W) {
-    const bool has_v = cb * 16 < dv, from_q = kg < 2 || !has_v;      // (every lane issues the transposing read)
-    const unsigned short* src = from_q ? Qs + (8 * (kg & 1) + tr_row) * Dp + cb * 16 + tr_col : Os + (8 * (kg - 2) + tr_row) * Dvp + cb * 16 + tr_col;
-    bf16x8 v = join(lds_tr16(src), lds_tr16(src + 4 * (from_q ? Dp : Dvp)));
-    if (kg >= 2 && !has_v) v = zero8();
-    *reinterpret_cast<bf16x8*>(bc + (size_t)(cb >> 2) * 2048 + (cb & 3) * 32) = v;
-  }
+  by_channel<W>(p, it, Qs, Os, Dp, Dvp, wave, l16, kg);
 }
 
 // ---- dq ------------------------------------------------------------------------------------------
@@ -427,6 +452,35 @@ constexpr int kPieces = kStep * kBlocks * 2 / 64;      // 16-byte pieces of a ti
 // Bytes to a row: the rows that one transposing read takes together stand in different banks.
 __device__ __forceinline__ int k_row(int row) { return row * 320 + (row & 8) * 4; }
 constexpr int kKtile = kStep * 320 + 32;
+
+// acc[j][v]: channel 16 * j + 4 * kg + v of head l16, from channel 16 b0 on; `own` is LDS of the wavefront's
+template <bool F16>
+__device__ __forceinline__ void put_dq(const SplitParams& p, const Item& it, char* own, f32x4 (&acc)[kBlocks], int b0, int blocks, int D, int lane, int l16, int kg) {
+#pragma unroll
+  for (int j = 0; j < kBlocks; ++j)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[j][v] *= PlaneScale<F16>::down;
+  const size_t base = (it.bs * p.H + it.h0) * (size_t)D + b0 * 16;
+  if (p.dq_dtype == CPPMEGA_MI355_F32) {
+    if (l16 >= it.nh) return;
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j)
+      if (j < blocks) *reinterpret_cast<f32x4*>((float*)p.dq + base + (size_t)l16 * D + j * 16 + 4 * kg) = acc[j];
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < kBlocks; ++j) {
+    const float v[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
+    *reinterpret_cast<uint2*>(own + l16 * 304 + j * 32 + kg * 8) = p.dq_dtype == CPPMEGA_MI355_F16 ? pack4<true>(v) : pack4<false>(v);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  for (int e = lane; e < it.nh * (kBlocks * 2); e += 64) {
+    const int h = e / (kBlocks * 2), c = e - h * (kBlocks * 2);
+    if (c < blocks * 2)
+      *reinterpret_cast<u32x4*>((unsigned short*)p.dq + base + (size_t)h * D + c * 8) = *reinterpret_cast<const u32x4*>(own + h * 304 + c * 16);
+  }
+}
 
 template <bool F16>
 __global__ __launch_bounds__(64, 3) void bwd_dq_kernel(const SplitParams p) {
@@ -498,30 +552,246 @@ __global__ __launch_bounds__(64, 3) void bwd_dq_kernel(const SplitParams p) {
     }
     __syncthreads();
   }
-  // acc[j][v]: channel 16 * j + 4 * kg + v of head l16
+  put_dq<F16>(p, it, Ks, acc, b0, blocks, D, lane, l16, kg);
+}
+
+// ---- scores and dq of 576 = 512 + 64 channels ---------------------------------------------------
+// The two kernels above in one, for up to 64 W keys: a wavefront scores up to four tiles of 16 keys, two at a time; then it
+// takes a quarter of the channels of all keys for dq, with dS of the other wavefronts out of LDS.  Eight
+// wavefronts: four quarters of the channels by two halves of the tiles of 32 keys, added at the end.
+// Measured against the two kernels: 79 queries x 8 heads x 160 of 7757 keys 25 -> 18 us, 512 x 64 x 256 of 2048 140 ->
+// 123, 1024 x 16 x 256 of 4096 70 -> 68.  Bound by the key rows' way from the L2 (604 MB, of a cache of 4.7 MB that is a
+// little more than an XCD's L2) and by the phases of a workgroup, two of which share a CU (77 KB of LDS each): 5 us until
+// q, d_out and the first keys are there, 8 for the scores, 6 for statistics and planes, 9 for dq.  Neither half the
+// loads in flight nor q and d_out in registers made a difference to the large shape.
+constexpr int kD = 576, kDv = 512, kDp = kD + 8, kDvp = kDv + 8, kStage = 5;
+constexpr int kFusedRows = kHeads * (kDp + kDvp) * 2;  // bytes of q and d_out, then of dS
+template <int W> constexpr int kFusedLds = kFusedRows + W * (kHeads * 3 * 4 + kKtile) + W * 64 * 4;
+static_assert(2 * kStage * 1024 <= kKtile && 4 * kStage >= kD / 32, "a stage of two tiles and 32 keys of dq share a wavefront's LDS");
+
+template <bool F16, int W>
+__global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitParams p) {
+  constexpr int T = 4, kSlots = W * T * 16;
+  static_assert(2 * kSlots * kHeads * 2 <= kFusedRows, "dS takes the place of q and d_out");
+  extern __shared__ __align__(16) unsigned char smem[];
+  unsigned short* Qs = reinterpret_cast<unsigned short*>(smem);       // [16][kDp]
+  unsigned short* Os = Qs + kHeads * kDp;                             // [16][kDvp]
+  float* met = reinterpret_cast<float*>(smem + kFusedRows);           // [W][16][3]
+  const int tid = (int)threadIdx.x, lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  char* own = reinterpret_cast<char*>(met + W * kHeads * 3) + wave * kKtile;
+  int* list_keys = reinterpret_cast<int*>(reinterpret_cast<char*>(met + W * kHeads * 3) + W * kKtile);       // [64 W]
+  const Item it = item_of(p, blockIdx.x);
+  const float sm_scale = p.sm_scale_dev ? *p.sm_scale_dev : p.sm_scale;
+  const float scale2 = sm_scale * kLog2e;
+  const int* keys = p.keys + it.list * (size_t)p.stride;
+  const int valid = p.starts[it.list * (p.bands + 2) + p.bands], tiles = (valid + 15) / 16;
+  const unsigned short* kv = p.kv + ((size_t)it.b * p.Skv * p.G + it.g) * (size_t)kD;
+  const size_t key_step = (size_t)p.G * kD;
+
+  // Two tiles at a time, up to five pieces of 32 channels of each per stage, four lanes to a row: two stages are on
+  // their way in registers while one passes through LDS to operand order.
+  const int row = lane >> 2, col = lane & 3;
+  unsigned short* put = reinterpret_cast<unsigned short*>(own) + row * 32 + ((col ^ (-(row >> 2) & 3)) << 3);
+  const unsigned short* get = reinterpret_cast<const unsigned short*>(own) + l16 * 32 + ((kg ^ (-(l16 >> 2) & 3)) << 3);
+  int slot_row[T], slot_16[T];                         // (tiles behind the list's room are the last one again, and nobody looks)
 #pragma unroll
-  for (int j = 0; j < kBlocks; ++j)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc[j][v] *= PlaneScale<F16>::down;
-  const size_t base = (it.bs * p.H + it.h0) * (size_t)D + b0 * 16;
-  if (p.dq_dtype == CPPMEGA_MI355_F32) {
-    if (l16 >= it.nh) return;
-#pragma unroll
-    for (int j = 0; j < kBlocks; ++j)
-      if (j < blocks) *reinterpret_cast<f32x4*>((float*)p.dq + base + (size_t)l16 * D + j * 16 + 4 * kg) = acc[j];
-    return;
+  for (int i = 0; i < T; ++i) {
+    const int* of_tile = keys + min(wave + i * W, p.stride / 16 - 1) * 16;
+    slot_row[i] = of_tile[row];
+    slot_16[i] = of_tile[l16];
   }
+  const int slot_own = keys[min(tid, p.stride - 1)];
+  // q and d_out, whole rows of neighbouring lanes
+  constexpr int kQLoads = (kHeads * (kD / 8) + W * 64 - 1) / (W * 64), kOLoads = kHeads * (kDv / 8) / (W * 64);
+  u32x4 staged[kQLoads + kOLoads];
 #pragma unroll
-  for (int j = 0; j < kBlocks; ++j) {
-    const float v[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
-    *reinterpret_cast<uint2*>(Ks + l16 * 304 + j * 32 + kg * 8) = p.dq_dtype == CPPMEGA_MI355_F16 ? pack4<true>(v) : pack4<false>(v);
+  for (int i = 0; i < kQLoads + kOLoads; ++i) {
+    const bool of_q = i < kQLoads;
+    const int e = tid + (of_q ? i : i - kQLoads) * W * 64, per = (of_q ? kD : kDv) / 8, h = min(e / per, it.nh - 1), c = e - e / per * per;
+    staged[i] = *reinterpret_cast<const u32x4*>((of_q ? p.q : p.d_out) + (it.bs * p.H + it.h0 + h) * (size_t)(of_q ? kD : kDv) + c * 8);
+  }
+  u32x4 queue[2][2][kStage];
+  const unsigned short* rows_at[T];
+#pragma unroll
+  for (int i = 0; i < T; ++i) rows_at[i] = kv + (size_t)max(plain_key(slot_row[i]), 0) * key_step + col * 8;
+  auto request = [&](auto pair_c, auto stage_c) {      // a stage of tiles 2 * pair and 2 * pair + 1
+    constexpr int pair = decltype(pair_c)::value, stage = decltype(stage_c)::value;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (wave + (2 * pair + j) * W < tiles)           // (uniform)
+#pragma unroll
+        for (int q = 0; q < kStage; ++q)
+          if (stage * kStage + q < kD / 32) queue[stage & 1][j][q] = *reinterpret_cast<const u32x4*>(rows_at[2 * pair + j] + (stage * kStage + q) * 32);
+  };
+  using std::integral_constant;
+  request(integral_constant<int, 0>{}, integral_constant<int, 0>{});
+  request(integral_constant<int, 0>{}, integral_constant<int, 1>{});
+#pragma unroll
+  for (int i = 0; i < kQLoads + kOLoads; ++i) {
+    const bool of_q = i < kQLoads;
+    const int e = tid + (of_q ? i : i - kQLoads) * W * 64, per = (of_q ? kD : kDv) / 8, h = e / per, c = e - h * per;
+    if (i == 0) list_keys[tid] = plain_key(slot_own);
+    if (h < kHeads) *reinterpret_cast<u32x4*>((of_q ? Qs + h * kDp : Os + h * kDvp) + c * 8) = h < it.nh ? staged[i] : u32x4{0u, 0u, 0u, 0u};
   }
   __syncthreads();
-  for (int e = lane; e < it.nh * (kBlocks * 2); e += 64) {
-    const int h = e / (kBlocks * 2), c = e - h * (kBlocks * 2);
-    if (c < blocks * 2)
-      *reinterpret_cast<u32x4*>((unsigned short*)p.dq + base + (size_t)h * D + c * 8) = *reinterpret_cast<const u32x4*>(Ks + h * 304 + c * 16);
+
+  f32x4 s[T], dp[T];
+  float m[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  const unsigned short *qa = Qs + l16 * kDp + 8 * kg, *oa = Os + l16 * kDvp + 8 * kg;
+  auto score_pair = [&](auto pair_c) {
+    constexpr int pair = decltype(pair_c)::value;
+    const bool two = wave + (2 * pair + 1) * W < tiles;               // (uniform)
+    f32x4 sa[2], da[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) sa[j] = da[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto stage_of = [&](auto stage_c) {
+      constexpr int stage = decltype(stage_c)::value;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (j == 0 || two)
+#pragma unroll
+          for (int q = 0; q < kStage; ++q)
+            if (stage * kStage + q < kD / 32) *reinterpret_cast<u32x4*>(put + (j * kStage + q) * 512) = queue[stage & 1][j][q];
+      __builtin_amdgcn_wave_barrier();
+      if constexpr (stage < 2) request(pair_c, integral_constant<int, stage + 2>{});
+      else if constexpr (pair == 0) request(integral_constant<int, 1>{}, integral_constant<int, stage - 2>{});
+#pragma unroll
+      for (int q = 0; q < kStage; ++q) {
+        constexpr int c0 = stage * kStage;
+        const int c = c0 + q;
+        if (c >= kD / 32) continue;
+        const bf16x8 a = lds_b128(qa + c * 32), k0 = lds_b128(get + q * 512);
+        bf16x8 o = a, k1 = k0;
+        if (c < kDv / 32) o = lds_b128(oa + c * 32);
+        sa[0] = mm<F16>(a, k0, sa[0]);
+        if (c < kDv / 32) da[0] = mm<F16>(o, k0, da[0]);
+        if (two) {
+          k1 = lds_b128(get + (kStage + q) * 512);
+          sa[1] = mm<F16>(a, k1, sa[1]);
+          if (c < kDv / 32) da[1] = mm<F16>(o, k1, da[1]);
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    };
+    stage_of(integral_constant<int, 0>{});
+    stage_of(integral_constant<int, 1>{});
+    stage_of(integral_constant<int, 2>{});
+    stage_of(integral_constant<int, 3>{});
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int i = 2 * pair + j;
+      const bool counts = (j == 0 || two) && slot_16[i] >= 0;         // (the slots behind a list's last key were fetched from row 0, which may hold anything)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        s[i][v] = counts ? sa[j][v] * scale2 : -INFINITY;
+        m[v] = fmaxf(m[v], s[i][v]);
+        dp[i][v] = counts ? da[j][v] : 0.0f;
+      }
+    }
+  };
+  if (wave < tiles) score_pair(integral_constant<int, 0>{});
+  if (wave + 2 * W < tiles) score_pair(integral_constant<int, 1>{});
+  const Stats stat = row_stats<W, T>(met, s, dp, m, wave, l16, kg, tiles);
+  by_channel<W>(p, it, Qs, Os, kDp, kDvp, wave, l16, kg);
+  // P and dS: planes for dkv, and dS for the other wavefronts
+  uint2 ds_hi[T], ds_lo[T];
+  char* out = p.planes + (it.list * p.chunks + it.chunk) * (size_t)p.stride * kRowBytes + (size_t)(kg >> 1) * p.stride * 16 + 8 * (kg & 1);
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    const int t = wave + i * W;
+    ds_hi[i] = ds_lo[i] = make_uint2(0u, 0u);
+    if (t < tiles) {
+      float pv[4], ds[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        pv[v] = s[i][v] * stat.inv_sum[v];
+        ds[v] = pv[v] * (dp[i][v] - stat.delta[v]) * sm_scale;
+      }
+      char* at = out + (size_t)(t * 16 + l16) * 16;
+      put_planes<F16>(at + (size_t)p.stride * 32, (size_t)p.stride * 64, pv);
+      uint2 hi, lo;
+      planes_of<F16>(ds, hi, lo);
+      *reinterpret_cast<uint2*>(at) = hi;
+      *reinterpret_cast<uint2*>(at + (size_t)p.stride * 64) = lo;
+      if (t * 16 + l16 < valid) {
+        ds_hi[i] = hi;
+        ds_lo[i] = lo;
+      }
+    }
   }
+
+  // ---- dq: quarter `part` of the channels, tiles of 32 keys first, first + W / 4, .. ----
+  constexpr int kTurns = W / 4;
+  const int part = wave & 3, first = wave >> 2, steps = (valid + kStep - 1) / kStep, b0 = part * kBlocks;
+  const unsigned short* kv_part = kv + b0 * 16;
+  int piece_row[kPieces], piece_col[kPieces];
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) {
+    const int e = lane + i * 64;
+    piece_row[i] = e / (kBlocks * 2);
+    piece_col[i] = e - piece_row[i] * (kBlocks * 2);
+  }
+  // two tiles are on their way
+  u32x4 pre[2][kPieces];
+  auto fetch = [&](int step, u32x4 (&to)[kPieces]) {
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int key = list_keys[min(step * kStep + piece_row[i], valid - 1)];
+      to[i] = *reinterpret_cast<const u32x4*>(kv_part + (size_t)key * key_step + piece_col[i] * 8);
+    }
+  };
+  if (first < steps) {
+    fetch(first, pre[0]);
+    fetch(first + kTurns, pre[1]);
+  }
+  __syncthreads();                                     // q and d_out are read
+  unsigned short* Ss = Qs;                             // [hi, lo][kSlots][16 heads]
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    uint2* at = reinterpret_cast<uint2*>(Ss + ((wave + i * W) * 16 + l16) * kHeads + 4 * kg);
+    at[0] = ds_hi[i];
+    at[kSlots * kHeads / 4] = ds_lo[i];
+  }
+  __syncthreads();
+  f32x4 acc[kBlocks];
+#pragma unroll
+  for (int j = 0; j < kBlocks; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int tr_row = l16 >> 2, tr_col = (l16 & 3) * 4;
+  auto turn = [&](int step, u32x4 (&of)[kPieces]) {
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) *reinterpret_cast<u32x4*>(own + k_row(piece_row[i]) + piece_col[i] * 16) = of[i];
+    __builtin_amdgcn_wave_barrier();
+    fetch(step + 2 * kTurns, of);                      // (behind the last: its last key again)
+    bf16x8 ds[2];
+#pragma unroll
+    for (int pl = 0; pl < 2; ++pl) {
+      const unsigned short* src = Ss + (pl * kSlots + step * kStep + 8 * kg + tr_row) * kHeads + tr_col;
+      ds[pl] = join(lds_tr16(src), lds_tr16(src + 4 * kHeads));
+    }
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j) {
+      const unsigned short* src = reinterpret_cast<const unsigned short*>(own + k_row(8 * kg + tr_row)) + j * 16 + tr_col;
+      const bf16x8 k = join(lds_tr16(src), lds_tr16(src + 4 * 160));
+      acc[j] = mm<F16>(k, ds[0], acc[j]);
+      acc[j] = mm<F16>(k, ds[1], acc[j]);
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  for (int step = first; step < steps; step += 2 * kTurns) {
+    turn(step, pre[0]);
+    if (step + kTurns < steps) turn(step + kTurns, pre[1]);
+  }
+  if (kTurns == 2) {
+    if (first == 1)
+#pragma unroll
+      for (int j = 0; j < kBlocks; ++j) reinterpret_cast<f32x4*>(own)[j * 64 + lane] = acc[j];
+    __syncthreads();
+    if (first == 1) return;
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j) acc[j] += reinterpret_cast<const f32x4*>(own + 4 * kKtile)[j * 64 + lane];
+  }
+  put_dq<F16>(p, it, own, acc, b0, kBlocks, kD, lane, l16, kg);
 }
 
 // ---- dkv -----------------------------------------------------------------------------------------
@@ -721,6 +991,11 @@ int run(SplitParams p, const Plan& l, bool clear, hipStream_t stream) {
   CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_kernel<F16, 8, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scores_lds(8)));
   CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_kernel<F16, 16, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scores_lds(16)));
   CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_dkv_kernel<F16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dkv_lds));
+  const bool fused = p.D == kD && p.d_v == kDv && p.topk <= 512;
+  if (fused) {
+    CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_dq_kernel<F16, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, kFusedLds<4>));
+    CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_dq_kernel<F16, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, kFusedLds<8>));
+  }
   for (p.s0 = 0; p.s0 < p.S; p.s0 += l.ns) {
     p.ns = std::min(l.ns, p.S - p.s0);
     p.shares = l.shares;
@@ -729,10 +1004,13 @@ int run(SplitParams p, const Plan& l, bool clear, hipStream_t stream) {
     hipLaunchKernelGGL(bwd_lists_kernel, dim3((unsigned)lists), dim3(kThreads), (size_t)(3 * p.bands + 2 * p.topk + 2) * 4, stream, p);
     hipLaunchKernelGGL(bwd_steps_kernel, dim3((unsigned)(p.B * p.G * p.bands)), dim3(kStepThreads), 0, stream, p);
     const dim3 of_items((unsigned)items);
-    if (p.topk <= 16 * 4 * 4) hipLaunchKernelGGL((bwd_scores_kernel<F16, 4, 4>), of_items, dim3(256), scores_lds(4), stream, p);
+    if (fused) {
+      if (p.topk <= 256) hipLaunchKernelGGL((bwd_scores_dq_kernel<F16, 4>), of_items, dim3(256), kFusedLds<4>, stream, p);
+      else hipLaunchKernelGGL((bwd_scores_dq_kernel<F16, 8>), of_items, dim3(512), kFusedLds<8>, stream, p);
+    } else if (p.topk <= 16 * 4 * 4) hipLaunchKernelGGL((bwd_scores_kernel<F16, 4, 4>), of_items, dim3(256), scores_lds(4), stream, p);
     else if (p.topk <= 16 * 8 * 4) hipLaunchKernelGGL((bwd_scores_kernel<F16, 8, 4>), of_items, dim3(512), scores_lds(8), stream, p);
     else hipLaunchKernelGGL((bwd_scores_kernel<F16, 16, 8>), of_items, dim3(1024), scores_lds(16), stream, p);
-    hipLaunchKernelGGL(bwd_dq_kernel<F16>, dim3((unsigned)(items * dq_parts)), dim3(64), 0, stream, p);
+    if (!fused) hipLaunchKernelGGL(bwd_dq_kernel<F16>, dim3((unsigned)(items * dq_parts)), dim3(64), 0, stream, p);
     const dim3 tiles((unsigned)((p.bands * ((p.D + 63) / 64) * p.shares * p.B * p.G + 7) / 8 * 8));
     hipLaunchKernelGGL(bwd_dkv_kernel<F16>, tiles, dim3(kDkvThreads), dkv_lds, stream, p);
     if (p.shares > 1) {

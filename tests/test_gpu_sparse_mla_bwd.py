@@ -385,3 +385,20 @@ def test_one_key_named_many_times_over(device, times):
     for got, ref in zip((dq, dkv), want):
         err, scale = error_report(got.cpu().numpy(), ref)
         assert err <= 1e-4 * scale, (err, scale)
+
+
+@pytest.mark.parametrize("heads,topk,valid", [(16, 16, 16), (5, 256, 256), (16, 256, 33), (24, 257, 257), (16, 512, 512), (8, 512, 1), (16, 513, 513)])
+def test_rows_of_576_channels_at_the_edges_of_their_tiles(device, heads, topk, valid):
+    """Up to 256 and up to 512 keys, and one more; whole and single tiles of 16 and 32 keys, and queries with fewer than the others."""
+    B, S, Skv, D, d_v = 2, 3, 700, 576, 512
+    rng = np.random.default_rng(topk + valid)
+    q, kv, d_out = (to_dev(rng.standard_normal(s).astype(np.float32), device).bfloat16() for s in ((B, S, heads, D), (B, Skv, 1, D), (B, S, heads, d_v)))
+    idx = sparse_indices(rng, B, S, 1, Skv, topk)
+    idx[..., valid:] = -1
+    idx[1, 2, :, valid // 2:] = -1
+    want = om.sparse_mla_bwd_oracle(q.double().cpu().numpy(), kv.double().cpu().numpy(), idx, d_out.double().cpu().numpy(), sm_scale=D ** -0.5, d_v=d_v)
+    dq, dkv = torch.full((B, S, heads, D), 9.0, device=device), torch.full((B, Skv, 1, D), 9.0, device=device)
+    ops.sparse_mla_backward(q, kv, d_out, to_dev(idx.astype(np.int32), device), sm_scale=D ** -0.5, d_v=d_v, dq=dq, dkv=dkv)
+    for got, ref in zip((dq, dkv), want):
+        err, scale = error_report(got.cpu().numpy(), ref)
+        assert err <= 1e-4 * scale, (err, scale)                # planes of 2^-17 and float32 sums of up to 1024 terms
