@@ -15,13 +15,14 @@
 //            channels and up to 512 keys: in the kernel of the scores);
 //   dkv      per (band, 64 channels, share of the steps): dS^T . Q + P^T . dO of every step, added to a
 //            float32 tile in LDS, written out once;
-//   sum      over the shares, when there are // Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 165 us (561 us with the atomics): lists 7, steps 7,
+//   sum      over the shares, when there are several.
+//
+// Nothing is added in an order that varies: the same input gives the same bits.
+//
+// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 165 us (561 us with the atomics): lists 7, steps 7,
 // scores and dq 68, dkv 82, sum 9.  dkv is bound by the vector cache (27 M accesses of 64 bytes: 4 KB of q and d_out and
 // about 1 KB of planes for a step's 9 keys of 16) and ends with the CUs whose four bands are all full; scores and dq by the
 // gather of 302 MB of key rows each.
-
-ssue of its
-// one wavefront per SIMD; scores and dq by the gather of 302 MB of key rows each.
 
 #include <algorithm>
 #include <type_traits>
