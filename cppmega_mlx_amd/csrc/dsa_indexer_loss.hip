@@ -184,9 +184,10 @@ static int check_shape(const cppmega_mi355_dsa_loss_args_t& a) {
 int dsa_indexer_loss_workspace_bytes(const cppmega_mi355_dsa_loss_args_t& a, size_t* bytes) {
   const int rc = check_shape(a);
   if (rc) return rc;
-  // A short dense loss is one launch of the kernel without a workspace: 19 us at 256 positions, 8 heads of 64, where
-  // the five tiled launches take 29; they meet at 384 positions (29 us) and, with heads of 128, at 256 (53 / 55 us).
-  const bool one_launch = !a.topk_indices && a.seq_k <= 320 && a.head_dim <= 64 && (long long)a.batch * a.seq_q <= 1024;
+  // A short dense loss is one launch of the kernel without a workspace.  Measured, it against the four tiled launches: 256
+  // positions, 8 heads of 64: 18.8 / 24.1 us (two sequences the same); 16 heads 28.0 / 24.2; 320 positions, 8 heads
+  // 27.9 / 25.0, two sequences of 16 heads 45.6 / 24.7; 128 positions 16.2 / 24.1.
+  const bool one_launch = !a.topk_indices && a.seq_k <= 256 && (long long)a.heads * a.head_dim <= 512 && a.head_dim <= 64 && (long long)a.batch * a.seq_q <= 1024;
   *bytes = dsa_indexer_loss_tiled_supports(a) && !one_launch ? dsa_indexer_loss_tiled_workspace_bytes(a) : 0;
   return 0;
 }

@@ -1,24 +1,26 @@
-// DSA indexer KL loss in tiles of 64 query positions x 128 keys, bfloat16 / float16 query and key (gfx950).
+// DSA indexer KL loss in tiles of 64 query positions x 64 or 128 keys, bfloat16 / float16 query and key (gfx950).
 //
 // Same result as dsa_indexer_loss_mfma.hip, for callers that give a workspace: with the statistics of the
 // softmaxes going through memory a row's keys are spread over workgroups, so that the causal triangle
 // fills the CUs evenly, and no wavefront waits for another one's reductions:
 //
-//   dsa_loss_list_kernel    per row: membership bits of the index list, softmax statistics of the index scores
-//   dsa_loss_tile_kernel<.., false>   per tile and head: max and sum of exp of the attention scores, per 64 keys
+//   dsa_loss_list_kernel    per row: membership bits of the index list, softmax statistics of the index scores (those
+//                           by the first pass where its tiles leave CUs idle)
+//   dsa_loss_tile_kernel<.., false>   per tile and head: sum of exp of the attention scores, per 64 keys
 //   dsa_loss_merge_kernel   per (head, row): log2 of the softmax denominator over all its keys
 //   dsa_loss_tile_kernel<.., true>    the scores again, p = mean over heads in registers, sum of p (log p - log q)
 //   dsa_loss_sum_kernel     per row: the divergence summed over its 64-key chunks, in order
 //
 // In a tile a wavefront has 32 positions (columns of v_mfma_f32_32x32x16, one per lane) and 64 keys (rows);
-// the head's 64 + 128 rows pass through LDS, fetched one head ahead as whole 16-byte pieces.  The masks
+// the heads' rows pass through LDS, fetched a step ahead as whole 16-byte pieces.  The masks
 // (causal, membership, additive) sit in registers as addends of the one multiply-add that scales a score,
 // and a lane reduces its own keys, so a head costs one lane exchange.
 //
 // Bound by the exponentials and the multiply-adds in front of them (two per pair and head).  Measured at
-// 4096 positions, 8 heads of 64, lists of 1024: 92 us a call (lists 16, passes 26 and 31, merge and sum 10),
-// against 274 us with a workgroup of 8 wavefronts per 16 positions (256 workgroups, the longest with twice the
-// mean work, statistics in LDS per step).
+// 4096 positions, 8 heads of 64, lists of 1024: 86 us a call (lists 20: 84 MB read; passes 24 and 29, merge and sum 9), 92
+// with whole tiles only and a maximum taken in the first pass, 274 with a workgroup of 8 wavefronts per 16 positions
+// (256 workgroups, the longest with twice the mean work, statistics in LDS per step).  Short sequences are bound by a
+// workgroup's steps: 2 x 547 positions, 16 heads of 128 70 -> 43 us with split tiles, 943 x 8 x 128 54 -> 38.
 
 #include <algorithm>
 
@@ -29,12 +31,13 @@ namespace cm {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kQ = 64, kK = 128;       // positions and keys of a workgroup
-constexpr int kChunk = 64;             // keys of a wavefront
+constexpr int kQ = 64;                 // positions of a workgroup
+constexpr int kChunk = 64;             // and keys
 constexpr float kEps = 1e-10f;
 constexpr size_t kPartBytes = 64u << 20;   // partial statistics of one slab of positions
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));       // rows of scores begin at any float
 
 struct LossTiledParams {
   const unsigned short* q;   // [ASq, AB, AH, AD]
@@ -48,11 +51,17 @@ struct LossTiledParams {
   float2* part;              // [chunks][AB * AH][slab rows]: max (base 2), sum
   float* norm;               // [AB * AH][slab rows]: log2 of the attention softmax's denominator, max included
   float* kl;                 // [chunks][AB][slab rows]
+  void* range_event;         // recorded behind the kernel that reads the lists; or NULL
   int* range_flag;           // set to 1 when a list holds an index outside [0, Sk); or NULL
   unsigned char* outside;    // with range_flag: [rows, in whole workgroups of the list kernel], whether a row's list holds such an index
   int topk, index_dtype, words;
   int ASq, AB, AH, Sk;
   int slab0, slab_rows;      // positions of this slab
+  int tiles;                 // of 64 positions x 128 keys of this slab and one batch
+  int whole;                 // of all batches' tiles, those from here on are split
+  int stats_rows;            // rows of index statistics that the first pass takes: all, or 0 (the list kernel takes them)
+  int stats_groups;          // its workgroups for them
+  long long first_tile;
   float scale2;              // softmax scale in base 2
 };
 
@@ -61,118 +70,205 @@ __device__ __forceinline__ f32x16 product(const u32x4& a, const u32x4& b, const 
   if (F16) return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
+// Rows from a base on, whose end the load unit checks: what lies behind it reads as zeros.
+struct Rows {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ Rows(const char* base, unsigned bytes) : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, (int)bytes, 0x00020000)) {}
+  __device__ u32x4 load(unsigned of_lane, int of_all) const { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)of_lane, of_all, 0)); }
+};
 __device__ __forceinline__ float exp2_(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float log2_(float x) { return __builtin_amdgcn_logf(x); }
 
-// One wavefront per row.
-__global__ __launch_bounds__(kThreads) void dsa_loss_list_kernel(const LossTiledParams p) {
-  extern __shared__ unsigned lds_bits[];
-  const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
-  const long long row = (long long)blockIdx.x * 4 + wave;
-  const bool live = row < (long long)p.AB * p.ASq;
-  unsigned* bits = lds_bits + wave * p.words;
-  const bool sparse = p.topk_idx != nullptr;
-  if (sparse) {
-    for (int w = lane; w < p.words; w += 64) bits[w] = 0u;
-    __syncthreads();
-    bool outside = false;
-    if (live) {
-      for (int t = lane; t < p.topk; t += 64) {
-        const size_t at = (size_t)row * p.topk + t;
-        const long long c = p.index_dtype == CPPMEGA_MI355_I64 ? static_cast<const long long*>(p.topk_idx)[at]
-                                                               : (long long)static_cast<const int*>(p.topk_idx)[at];
-        if (c >= 0 && c < p.Sk) atomicOr(&bits[(int)(c >> 5)], 1u << (c & 31));
-        else outside = true;
-      }
-      if (outside && p.range_flag) *p.range_flag = 1;
-    }
-    const bool any = __ballot(outside) != 0ull;
-    if (p.outside && lane == 0) p.outside[row] = any;
-    __syncthreads();
-    if (live)
-      for (int w = lane; w < p.words; w += 64) p.bits[(size_t)row * p.words + w] = bits[w];
-  }
-  if (!live) return;
+// Softmax statistics of a row's index scores, by one wavefront; word_of(j): the membership bits from key j on.
+template <class Words>
+__device__ __forceinline__ void index_statistics(const LossTiledParams& p, long long row, Words word_of) {
+  const int lane = lane_id();
   const float* src = p.index_scores + (size_t)row * p.Sk;
   const float* add = p.mask ? p.mask + (size_t)row * p.Sk : nullptr;
   float m = -INFINITY, d = 0.0f;
-  auto take = [&](const float (&v)[4], int n) {              // (NaN scores are skipped)
+  // N quads at a time, all requested before the first is looked at (NaN scores are skipped)
+  constexpr int N = 8;
+  for (int j0 = lane * 4; j0 < p.Sk; j0 += N * 256) {
+    f32x4 v[N];
+    unsigned word[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int j = j0 + n * 256;
+      v[n] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      word[n] = 15u;
+      if (j < p.Sk) {
+        if (j + 3 < p.Sk) v[n] = *reinterpret_cast<const f32x4_any*>(src + j);
+        else
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (j + i < p.Sk) v[n][i] = src[j + i];
+        word[n] = word_of(j);
+      }
+    }
     float top = m;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (i < n && v[i] > top) top = v[i];
-    if (top == -INFINITY) return;
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (add && j0 + n * 256 + i < p.Sk) v[n][i] += add[j0 + n * 256 + i];
+        if (!((word[n] >> i) & 1u)) v[n][i] = -INFINITY;
+        if (v[n][i] > top) top = v[n][i];
+      }
+    if (top == -INFINITY) continue;
     d *= exp2_((m - top) * kLog2e);
     m = top;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (i < n && v[i] > -INFINITY) d += exp2_((v[i] - top) * kLog2e);
-  };
-  if ((p.Sk & 3) == 0 && ((uintptr_t)p.index_scores & 15) == 0) {
-#pragma unroll 4
-    for (int j = lane * 4; j < p.Sk; j += 256) {
-      const f32x4 s = *reinterpret_cast<const f32x4*>(src + j);
-      float v[4] = {s[0], s[1], s[2], s[3]};
-      if (add)
+    for (int n = 0; n < N; ++n)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] += add[j + i];
-      if (sparse) {
-        const unsigned w = bits[j >> 5] >> (j & 31);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = (w >> i) & 1u ? v[i] : -INFINITY;
-      }
-      take(v, 4);
-    }
-  } else {
-    for (int j = lane; j < p.Sk; j += 64) {
-      float v[4] = {src[j] + (add ? add[j] : 0.0f), 0.0f, 0.0f, 0.0f};
-      if (sparse && !((bits[j >> 5] >> (j & 31)) & 1u)) v[0] = -INFINITY;
-      take(v, 1);
-    }
+      for (int i = 0; i < 4; ++i)
+        if (v[n][i] > -INFINITY) d += exp2_((v[n][i] - top) * kLog2e);
   }
   const float top = wave_max(m);
   const float sum = wave_sum(m > -INFINITY ? d * exp2_((m - top) * kLog2e) : 0.0f);
   if (lane == 0) p.index_norm[row] = sum > 0.0f ? fmaf(top, kLog2e, log2_(sum)) : 0.0f;
 }
 
-// Tiles with a visible key in the first n blocks of positions (block i sees the keys of i / 2 + 1 tiles, at
-// most all of them).
+// One wavefront per row: membership bits of the index list, and the statistics of the row where nothing else takes them.
+__global__ __launch_bounds__(kThreads) void dsa_loss_list_kernel(const LossTiledParams p) {
+  extern __shared__ unsigned lds_bits[];
+  const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
+  const long long row = (long long)blockIdx.x * 4 + wave;
+  const bool live = row < (long long)p.AB * p.ASq;
+  if (!p.topk_idx) {
+    if (live) index_statistics(p, row, [](int) { return 15u; });
+    return;
+  }
+  unsigned* bits = lds_bits + wave * p.words;
+  for (int w = lane; w < p.words; w += 64) bits[w] = 0u;
+  __syncthreads();
+  bool outside = false;
+  if (live) {
+#pragma unroll 4
+    for (int t = lane; t < p.topk; t += 64) {
+      const size_t at = (size_t)row * p.topk + t;
+      const long long c = p.index_dtype == CPPMEGA_MI355_I64 ? static_cast<const long long*>(p.topk_idx)[at]
+                                                             : (long long)static_cast<const int*>(p.topk_idx)[at];
+      if (c >= 0 && c < p.Sk) atomicOr(&bits[(int)(c >> 5)], 1u << (c & 31));
+      else outside = true;
+    }
+    if (outside && p.range_flag) *p.range_flag = 1;
+  }
+  const bool any = __ballot(outside) != 0ull;
+  if (p.outside && lane == 0) p.outside[row] = any;
+  __syncthreads();
+  if (!live) return;
+  for (int w = lane; w < p.words; w += 64) p.bits[(size_t)row * p.words + w] = bits[w];
+  if (p.stats_rows == 0) index_statistics(p, row, [&](int j) { return bits[j >> 5] >> (j & 31); });
+}
+
+// Tiles of 64 positions x 128 keys with a visible key in the first n blocks of positions (block i sees the keys of
+// i / 2 + 1 tiles, at most all of them).
 __host__ __device__ inline long long tiles_before(long long n, long long key_tiles) {
   const long long ramp = 2 * key_tiles, m = n < ramp ? n : ramp;
   return (m + 1) * (m + 1) / 4 + (n - m) * key_tiles;
 }
 
+// A tile of 64 positions; a wavefront has 32 positions (columns of v_mfma_f32_32x32x16, one per lane) and 64 keys (rows).
+// Whole tiles of 128 keys: two halves of the positions by two of the keys, a head at a time.  Split ones of 64 keys: two
+// halves of the positions by GROUPS groups of the heads, that many heads at a time.  The CUs hold resident() workgroups
+// each; whole rounds of them take whole tiles (64 + 128 rows per head pass through LDS for 8192 pairs, and the masks are set
+// up once for all heads), the rest, and everything where there is less than a round, go in split ones: what counts there is
+// a workgroup's time, which is its number of steps (1.6 us each, 4 us around them).  Four groups where split tiles have a CU
+// to themselves.
 // GENERAL: an additive mask is given, or the softmax scale is not positive.  Otherwise the masks are 0 or -inf
 // and enter the first pass as what its products start from (a select behind them where a row that does not count
 // turned out not to be finite), and the second pass leaves keys that do not count out at its end.
-template <bool F16, int AD, bool SECOND, bool GENERAL>
-__global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void dsa_loss_tile_kernel(const LossTiledParams p) {
+// Where the tiles leave CUs idle, workgroups of the first pass between those of the tiles take the statistics of the index
+// scores, a row to a wavefront.
+constexpr int resident(int AD, bool general) { return AD <= 64 && !general ? 4 : 2; }
+template <bool F16, int AD, int GROUPS, bool SECOND, bool GENERAL>
+__global__ __launch_bounds__(128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_tile_kernel(const LossTiledParams p) {
+  constexpr int THREADS = 128 * GROUPS;
   constexpr int PIECES = AD / 8;                          // 16-byte pieces of a row of one head
   constexpr int PITCH = PIECES + 1;                       // odd: 16 rows of a piece fall on 16 bank groups
-  constexpr int LOADS = (kQ + kK) * PIECES / kThreads;
+  constexpr int LOADS = 64 * PIECES / THREADS;            // pieces of a thread of 64 rows of one head
   constexpr int STEPS = AD / 16;
-  static_assert(LOADS * kThreads == (kQ + kK) * PIECES, "whole pieces per thread");
-  __shared__ u32x4 rows[(kQ + kK) * PITCH];               // 64 query rows, then 128 key rows
+  static_assert(LOADS * THREADS == 64 * PIECES, "whole pieces per thread");
+  // 64 rows each: queries, keys of the first head, (split: queries,) keys of the second, ..; in the end the wavefronts' sums
+  constexpr int BLOCK = 64 * PITCH, ROWS = 2 * GROUPS * BLOCK, MEET = SECOND ? 2 * GROUPS * 32 * 64 / 4 : 0;
+  __shared__ u32x4 rows[ROWS > MEET ? ROWS : MEET];
 
-  // Tile of this workgroup.  The causal triangle is one row of workgroups; consecutive ones go round the
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int id = (int)blockIdx.x;
+  if (!SECOND && p.stats_rows) {
+    // eights of workgroups (one per XCD) of tiles and of statistics, in proportion
+    const unsigned eight = (unsigned)id >> 3, stats_eights = (unsigned)(p.stats_groups + 7) >> 3, eights = gridDim.x >> 3;
+    const unsigned before = eight * stats_eights / eights;
+    if ((eight + 1) * stats_eights / eights != before) {
+      const int row = ((int)before * 8 + (id & 7)) * (2 * GROUPS) + wave;
+      if (row < p.stats_rows) {
+        const unsigned* bits = p.bits + (size_t)row * p.words;
+        index_statistics(p, row, [&](int j) { return p.topk_idx ? bits[j >> 5] >> (j & 31) : 15u; });
+      }
+      return;
+    }
+    id -= (int)before * 8;
+  }
+  // Tile of this workgroup: the causal triangles of the batches, one after the other.  Consecutive workgroups go round the
   // eight XCDs, and each XCD takes one run of tiles, whose query rows (and the keys) its L2 holds.
-  const int share = (int)gridDim.x >> 3, rest = (int)gridDim.x & 7, xcd = (int)blockIdx.x & 7;
-  const long long key_tiles = (p.Sk + kK - 1) / kK;
-  const long long at_tile = tiles_before(p.slab0 / kQ, key_tiles) + xcd * share + min(xcd, rest) + ((int)blockIdx.x >> 3);
-  int lo = p.slab0 / kQ, hi = (p.ASq + kQ - 1) / kQ;      // tiles_before(lo) <= at_tile < tiles_before(hi)
+  const bool split = GROUPS > 2 || id >= p.whole;
+  int within = id, count = p.whole;
+  if (split) {
+    within = id - p.whole;
+    count = (p.tiles * p.AB - p.whole) * 2;
+  }
+  if (within >= count) return;
+  const int share = count >> 3, rest = count & 7, xcd = within & 7;
+  int at_tile = xcd * share + min(xcd, rest) + (within >> 3);
+  const int key_half = split ? at_tile & 1 : 0;
+  if (split) at_tile = p.whole + (at_tile >> 1);
+  const int b = at_tile / p.tiles, key_tiles = (p.Sk + 127) / 128;
+  const long long of_all = p.first_tile + (at_tile - b * p.tiles);
+  int lo = p.slab0 / kQ, hi = (p.ASq + kQ - 1) / kQ;      // tiles_before(lo) <= of_all < tiles_before(hi)
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
-    if (tiles_before(mid, key_tiles) <= at_tile) lo = mid;
+    if (tiles_before(mid, key_tiles) <= of_all) lo = mid;
     else hi = mid;
   }
-  const int q0 = lo * kQ, k0 = (int)(at_tile - tiles_before(lo, key_tiles)) * kK, b = (int)blockIdx.y;
-  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int q0 = lo * kQ, k0 = (int)(of_all - tiles_before(lo, key_tiles)) * 128 + key_half * 64;
+  if (k0 > q0 + 63 || k0 >= p.Sk) return;                 // (the second half of a tile on the diagonal, or at the end)
   const int l32 = lane & 31, half = lane >> 5;
-  const int wq = (wave & 1) * 32, wk = (wave >> 1) * kChunk;
-  const int my_q = q0 + wq + l32, kw = k0 + wk;           // the lane's position, the wavefront's first key
+  const int wq = (wave & 1) * 32, group = __builtin_amdgcn_readfirstlane(wave >> 1);
+  const int kw = k0 + (split ? 0 : group * 64);          // the wavefront's first key
+  const int my_q = q0 + wq + l32;                         // the lane's position
   const bool live_q = my_q < p.ASq;
   const bool busy = kw <= q0 + wq + 31 && kw < p.Sk;      // the wavefront has a visible key
   const size_t row = (size_t)b * p.ASq + (live_q ? my_q : p.ASq - 1);
+  const int steps = split ? (p.AH + GROUPS - 1) / GROUPS : p.AH;
+
+  // rows of the tile, as far as there are any (the rest reads as zeros)
+  const unsigned pos_bytes = (unsigned)p.AB * p.AH * AD * 2;
+  const Rows q_rows(reinterpret_cast<const char*>(p.q) + (size_t)q0 * pos_bytes + (size_t)b * p.AH * AD * 2, (min(64, p.ASq - q0) - 1) * pos_bytes + p.AH * AD * 2);
+  const Rows k_rows(reinterpret_cast<const char*>(p.k) + (size_t)k0 * pos_bytes + (size_t)b * p.AH * AD * 2, (min(128, p.Sk - k0) - 1) * pos_bytes + p.AH * AD * 2);
+  unsigned src[LOADS];
+  int dst[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int e = tid + i * THREADS, r = e / PIECES, c = e % PIECES;
+    src[i] = (unsigned)r * pos_bytes + (unsigned)c * 16u;
+    dst[i] = r * PITCH + c;
+  }
+  u32x4 piece[2 * GROUPS][LOADS];
+  float norm_next = 0.0f;
+  const float* norm_src = SECOND ? p.norm + (size_t)b * p.AH * p.slab_rows + (live_q ? my_q - p.slab0 : 0) : nullptr;
+  auto fetch = [&](int step) {
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+      const int h = split ? min(step * GROUPS + g, p.AH - 1) : step;
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        if (split || g == 0) piece[2 * g][i] = q_rows.load(src[i], h * AD * 2);
+        piece[2 * g + 1][i] = k_rows.load(src[i] + (split || g == 0 ? 0u : 64u * pos_bytes), h * AD * 2);
+      }
+    }
+    if (SECOND) norm_next = norm_src[(size_t)(split ? min(step * GROUPS + group, p.AH - 1) : step) * p.slab_rows];
+  };
+  fetch(0);
 
   // register v of a 32-key block: key 8 * (v / 4) + 4 * half + v % 4
   float add[2][16];
@@ -196,56 +292,42 @@ __global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void dsa_lo
     }
   }
 
-  const size_t pos_bytes = (size_t)p.AB * p.AH * AD * 2;
-  const char* const q_base = reinterpret_cast<const char*>(p.q) + (size_t)q0 * pos_bytes + (size_t)b * p.AH * AD * 2;
-  const char* const k_base = reinterpret_cast<const char*>(p.k) + (size_t)k0 * pos_bytes + (size_t)b * p.AH * AD * 2;
-  unsigned src[LOADS];
-  int dst[LOADS];
-#pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
-    const int e = tid + i * kThreads, r = e / PIECES, c = e % PIECES;
-    const int at = r < kQ ? min(r, p.ASq - 1 - q0) : min(r - kQ, p.Sk - 1 - k0);
-    src[i] = (unsigned)at * (unsigned)pos_bytes + (unsigned)c * 16u;
-    dst[i] = r * PITCH + c;
-  }
-  u32x4 piece[LOADS];
-  float norm_next = 0.0f;
-  const float* norm_src = SECOND ? p.norm + (size_t)b * p.AH * p.slab_rows + (live_q ? my_q - p.slab0 : 0) : nullptr;
-  auto fetch = [&](int h) {
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {                      // (the first 64 rows are whole pieces of queries for every head size)
-      const char* base = i < kQ * PIECES / kThreads ? q_base : k_base;
-      piece[i] = *reinterpret_cast<const u32x4*>(base + (size_t)h * AD * 2 + src[i]);
-    }
-    if (SECOND) norm_next = norm_src[(size_t)h * p.slab_rows];
-  };
-
+  unsigned any = counts[0] | counts[1];                   // whether the position has a key here (of either half of the lanes)
+  any |= __float_as_uint(xor32(__uint_as_float(any)));
   float mean[2][16];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int v = 0; v < 16; ++v) mean[t][v] = 0.0f;
 
-  fetch(0);
-  for (int h = 0; h < p.AH; ++h) {
-    __syncthreads();                                      // the previous head's rows are read
+  const u32x4* const q_frag = rows + (split ? group : 0) * 2 * BLOCK + (wq + l32) * PITCH + half;
+  const u32x4* const k_frag = rows + (1 + 2 * group) * BLOCK + l32 * PITCH + half;
+  for (int step = 0; step < steps; ++step) {
+    __syncthreads();                                      // the previous heads' rows are read
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) rows[dst[i]] = piece[i];
+    for (int m = 0; m < 2 * GROUPS; ++m)
+      if (m != 2 || split)
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) rows[m * BLOCK + dst[i]] = piece[m][i];
     const float norm = norm_next;
-    fetch(h + 1 < p.AH ? h + 1 : h);
+    fetch(min(step + 1, steps - 1));
     __syncthreads();
-    if (!busy) continue;
+    const int h = split ? step * GROUPS + group : step;
+    if (!busy || h >= p.AH) continue;                     // (uniform)
     f32x16 s[2];
+    auto products = [&](bool masked) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) s[t][v] = SECOND || GENERAL ? 0.0f : add[t][v];
+        for (int v = 0; v < 16; ++v) s[t][v] = masked ? add[t][v] : 0.0f;
 #pragma unroll
-    for (int k = 0; k < STEPS; ++k) {
-      const u32x4 qf = rows[(wq + l32) * PITCH + 2 * k + half];
+      for (int k = 0; k < STEPS; ++k) {
+        const u32x4 qf = q_frag[2 * k];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) s[t] = product<F16>(rows[(kQ + wk + t * 32 + l32) * PITCH + 2 * k + half], qf, s[t]);
-    }
+        for (int t = 0; t < 2; ++t) s[t] = product<F16>(k_frag[t * 32 * PITCH + 2 * k], qf, s[t]);
+      }
+    };
+    products(!SECOND && !GENERAL);
     // (exponentials first, sums behind them: a sum right behind its exponential waits for it)
     if constexpr (SECOND) {
 #pragma unroll
@@ -257,18 +339,8 @@ __global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void dsa_lo
       }
     } else {
       float m, sum;
-      auto statistics = [&]() {
-        m = -INFINITY;
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            if (GENERAL) s[t][v] = add[t][v] > -INFINITY ? fmaf(s[t][v], p.scale2, add[t][v]) : -INFINITY;
-            m = fmaxf(m, s[t][v]);
-          }
-        m = fmaxf(m, xor32(m));
-        if (!GENERAL) m *= p.scale2;
-        const float at = m > -INFINITY ? m : 0.0f;
+      // exponentials relative to `at`, and their sum over the keys
+      auto add_up = [&](float at) {
         float d[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -280,63 +352,112 @@ __global__ __launch_bounds__(kThreads, AD <= 64 && !GENERAL ? 4 : 2) void dsa_lo
         sum = (d[0] + d[1]) + (d[2] + d[3]);
         sum += xor32(sum);
       };
-      statistics();
-      // -inf + x is NaN where x is not finite: the row of a key that does not count holds such values, or a row that
-      // counts does.  Only then the masks are applied behind the products.
-      if (!GENERAL && __ballot(!(sum == sum)) != 0ull) {
-        asm volatile("" ::: "memory");                    // (the operands are read again: kept from above, they would not fit)
+      auto relative_to_maximum = [&]() {
+        m = -INFINITY;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) s[t][v] = 0.0f;
+          for (int v = 0; v < 16; ++v) {
+            if (GENERAL) s[t][v] = add[t][v] > -INFINITY ? fmaf(s[t][v], p.scale2, add[t][v]) : -INFINITY;
+            m = fmaxf(m, s[t][v]);
+          }
+        m = fmaxf(m, xor32(m));
+        if (!GENERAL) m *= p.scale2;
+        add_up(m > -INFINITY ? m : 0.0f);
+      };
+      if (GENERAL) {
+        relative_to_maximum();
+      } else {
+        // Scores of ordinary size need no maximum taken from them (a third of the instructions that are not exponentials):
+        // where the sum lies far from the ends of float32, every term that counts in it is a normal number.
+        add_up(0.0f);
+        m = any ? 0.0f : -INFINITY;
+        // Otherwise, and where -inf + x is NaN because x is not finite (the row of a key that does not count holds such
+        // values, or a row that counts does), the masks are applied behind the products and the maximum is taken.
+        if (__ballot(any ? !(sum > 0x1p-60f && sum < 0x1p+100f) : !(sum == 0.0f)) != 0ull) {
+          asm volatile("" ::: "memory");                  // (the operands are read again: kept from above, they would not fit)
+          products(false);
 #pragma unroll
-        for (int k = 0; k < STEPS; ++k) {
-          const u32x4 qf = rows[(wq + l32) * PITCH + 2 * k + half];
+          for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int t = 0; t < 2; ++t) s[t] = product<F16>(rows[(kQ + wk + t * 32 + l32) * PITCH + 2 * k + half], qf, s[t]);
+            for (int v = 0; v < 16; ++v) s[t][v] = add[t][v] == 0.0f ? s[t][v] : -INFINITY;
+          relative_to_maximum();
         }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) s[t][v] = add[t][v] == 0.0f ? s[t][v] : -INFINITY;
-        statistics();
       }
       if (half == 0 && my_q - p.slab0 < p.slab_rows && live_q)
         p.part[((size_t)(kw / kChunk) * p.AB * p.AH + (size_t)b * p.AH + h) * p.slab_rows + (my_q - p.slab0)] = make_float2(m, sum);
     }
   }
-  if (!SECOND || !busy) return;
+  if (!SECOND) return;
 
-  const bool vec = (p.Sk & 3) == 0 && ((uintptr_t)p.index_scores & 15) == 0;
   const float inv_heads = 1.0f / (float)p.AH, index_norm = p.index_norm[row];
   const float* scores = p.index_scores + row * (size_t)p.Sk;
-  float kl = 0.0f;
+  // keys 8 * g .. + 3 of block t, for which the heads' probabilities add up to `sums`
+  auto divergence = [&](int t, int g, const float (&sums)[4]) {
+    float kl = 0.0f;
+    const int key = kw + t * 32 + 8 * g + 4 * half;
+    if (!live_q || key > my_q || key >= p.Sk) return kl;
+    float iv[4];
+    if (key + 3 < p.Sk) {
+      const f32x4 x = *reinterpret_cast<const f32x4_any*>(scores + key);
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+      for (int i = 0; i < 4; ++i) iv[i] = x[i];
+    } else {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int key = kw + t * 32 + 8 * g + 4 * half;
-      if (!live_q || key > my_q || key >= p.Sk) continue;
-      float iv[4];
-      if (vec) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(scores + key);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) iv[i] = x[i];
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) iv[i] = key + i < p.Sk ? scores[key + i] : 0.0f;
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (key + i > my_q || key + i >= p.Sk) continue;    // masked keys carry p = 0 and q = 0
-        const bool ok = (counts[t] >> (8 * g + i)) & 1u;
-        const float pj = ok ? mean[t][4 * g + i] * inv_heads : 0.0f;
-        const float v = !ok ? -INFINITY : (GENERAL ? fmaf(iv[i], kLog2e, add[t][4 * g + i]) : iv[i] * kLog2e);
-        const float qj = v > -INFINITY ? exp2_(v - index_norm) : 0.0f;
-        kl += pj * (log2_(pj + kEps) - log2_(qj + kEps));
-      }
+      for (int i = 0; i < 4; ++i) iv[i] = key + i < p.Sk ? scores[key + i] : 0.0f;
     }
-  kl += xor32(kl);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (key + i > my_q || key + i >= p.Sk) continue;    // masked keys carry p = 0 and q = 0
+      const bool ok = ((t ? counts[1] : counts[0]) >> (8 * g + i)) & 1u;
+      const float pj = ok ? sums[i] * inv_heads : 0.0f;
+      float v = ok ? iv[i] * kLog2e : -INFINITY;
+      if (GENERAL && ok && p.mask) v = fmaf(iv[i], kLog2e, p.mask[row * (size_t)p.Sk + key + i] * kLog2e);
+      const float qj = v > -INFINITY ? exp2_(v - index_norm) : 0.0f;
+      kl += pj * (log2_(pj + kEps) - log2_(qj + kEps));
+    }
+    return kl;
+  };
+  float kl = 0.0f;
+  if (split) {
+    // the groups of heads meet in LDS, and each finishes its share of the 32 registers
+    constexpr int MINE = 32 / GROUPS;
+    float* const meet = reinterpret_cast<float*>(rows) + lane;               // [wavefront][register][lane]
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) meet[((wave * 2 + t) * 16 + v) * 64] = mean[t][v];
+    __syncthreads();
+    const int t = group * MINE / 16, g0 = group * MINE % 16 / 4;
+#pragma unroll
+    for (int g = 0; g < MINE / 4; ++g) {
+      float sums[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int of = 0; of < GROUPS; ++of)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sums[i] += meet[(((of * 2 + (wave & 1)) * 2 + t) * 16 + 4 * (g0 + g) + i) * 64];
+      kl += divergence(t, g0 + g, sums);
+    }
+    kl += xor32(kl);
+    __syncthreads();
+    float* const ends = reinterpret_cast<float*>(rows) + wq + l32;
+    if (half == 0) ends[group * 64] = kl;
+    __syncthreads();
+    if (group) return;
+#pragma unroll
+    for (int of = 1; of < GROUPS; ++of) kl += ends[of * 64];
+  } else {
+    if (!busy) return;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float sums[4] = {mean[t][4 * g], mean[t][4 * g + 1], mean[t][4 * g + 2], mean[t][4 * g + 3]};
+        kl += divergence(t, g, sums);
+      }
+    kl += xor32(kl);
+  }
   if (half == 0 && live_q && my_q - p.slab0 < p.slab_rows)
     p.kl[((size_t)(kw / kChunk) * p.AB + b) * p.slab_rows + (my_q - p.slab0)] = kl * kLn2;
 }
@@ -413,19 +534,47 @@ Layout layout(const cppmega_mi355_dsa_loss_args_t& a) {
   return l;
 }
 
+template <bool F16, int AD, int GROUPS>
+void passes(LossTiledParams p, long long workgroups, bool general, hipStream_t stream) {
+  p.stats_groups = (p.stats_rows + 2 * GROUPS - 1) / (2 * GROUPS);
+  const dim3 grid((unsigned)workgroups), block(128 * GROUPS), merge(kThreads);
+  const dim3 with_statistics((unsigned)(p.stats_groups ? (workgroups + 7) / 8 * 8 + (p.stats_groups + 7) / 8 * 8 : workgroups));
+  const long long columns = (long long)p.AB * p.slab_rows / 64;
+  if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, false, true>), with_statistics, block, 0, stream, p);
+  else hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, false, false>), with_statistics, block, 0, stream, p);
+  hipLaunchKernelGGL(dsa_loss_merge_kernel, dim3((unsigned)(columns * p.AH)), merge, 0, stream, p);
+  if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, true, true>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, true, false>), grid, block, 0, stream, p);
+  hipLaunchKernelGGL(dsa_loss_sum_kernel, dim3((unsigned)columns), merge, 0, stream, p);
+}
+
 template <bool F16, int AD>
 int run(LossTiledParams p, hipStream_t stream) {
+  const bool general = p.mask || !(p.scale2 > 0.0f);
+  const int key_tiles = (p.Sk + 127) / 128;
+  const long long round = 256 * resident(AD, general);
+  // (the lists' bits come first: the caller may be waiting for what that kernel finds)
+  const size_t rows = (size_t)p.AB * p.ASq;
+  const bool in_tiles = p.slab_rows >= p.ASq && tiles_before((p.ASq + kQ - 1) / kQ, key_tiles) * p.AB < round;
+  p.stats_rows = in_tiles ? (int)rows : 0;
+  if (p.topk_idx || !in_tiles)
+    hipLaunchKernelGGL(dsa_loss_list_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads), p.topk_idx ? 16 * (size_t)p.words : 0, stream, p);
+  CM_HIP_CHECK(hipGetLastError());
+  if (p.range_event) CM_HIP_CHECK(hipEventRecord((hipEvent_t)p.range_event, stream));
   for (p.slab0 = 0; p.slab0 < p.ASq; p.slab0 += p.slab_rows) {
-    const int end = std::min(p.slab0 + p.slab_rows, p.ASq), key_tiles = (p.Sk + kK - 1) / kK;
-    const dim3 grid((unsigned)(tiles_before((end + kQ - 1) / kQ, key_tiles) - tiles_before(p.slab0 / kQ, key_tiles)), (unsigned)p.AB), block(kThreads);
-    const long long columns = (long long)p.AB * p.slab_rows / 64;
-    const bool general = p.mask || !(p.scale2 > 0.0f);
-    if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, false, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, false, false>), grid, block, 0, stream, p);
-    hipLaunchKernelGGL(dsa_loss_merge_kernel, dim3((unsigned)(columns * p.AH)), block, 0, stream, p);
-    if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, true, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, true, false>), grid, block, 0, stream, p);
-    hipLaunchKernelGGL(dsa_loss_sum_kernel, dim3((unsigned)columns), block, 0, stream, p);
+    const int end = std::min(p.slab0 + p.slab_rows, p.ASq);
+    p.first_tile = tiles_before(p.slab0 / kQ, key_tiles);
+    p.tiles = (int)(tiles_before((end + kQ - 1) / kQ, key_tiles) - p.first_tile);
+    const long long all = (long long)p.tiles * p.AB;
+    p.whole = (int)(all / round * round);
+    const long long workgroups = p.whole + (all - p.whole) * 2;
+    if constexpr (AD == 64 || AD == 128) {
+      if (workgroups <= 256 && p.AH > 2) {
+        passes<F16, AD, 4>(p, workgroups, general, stream);
+        continue;
+      }
+    }
+    passes<F16, AD, 2>(p, workgroups, general, stream);
   }
   CM_HIP_CHECK(hipGetLastError());
   return 0;
@@ -437,7 +586,7 @@ int run(LossTiledParams p, hipStream_t stream) {
 bool dsa_indexer_loss_tiled_supports(const cppmega_mi355_dsa_loss_args_t& a) {
   if (a.in_dtype != CPPMEGA_MI355_BF16 && a.in_dtype != CPPMEGA_MI355_F16) return false;
   if (a.head_dim != 32 && a.head_dim != 64 && a.head_dim != 96 && a.head_dim != 128) return false;
-  if ((size_t)a.batch * a.heads * a.head_dim * 2 * kK >= (1ull << 32)) return false;          // a tile's rows within 32-bit offsets
+  if ((size_t)a.batch * a.heads * a.head_dim * 2 * 128 >= (1ull << 32)) return false;         // a tile's rows within 32-bit offsets
   if (a.batch > 65535 || (size_t)a.seq_q * a.batch == 0 || a.heads == 0 || a.seq_k == 0) return false;
   return !a.topk_indices || a.seq_k <= 131072;
 }
@@ -459,10 +608,7 @@ int dsa_indexer_loss_tiled_launch(const cppmega_mi355_dsa_loss_args_t& a, hipStr
   p.ASq = a.seq_q; p.AB = a.batch; p.AH = a.heads; p.Sk = a.seq_k;
   p.slab0 = 0; p.slab_rows = l.slab_rows;
   p.scale2 = a.softmax_scale * kLog2e;
-  const size_t rows = (size_t)a.batch * a.seq_q;
-  hipLaunchKernelGGL(dsa_loss_list_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads), a.topk_indices ? 16 * (size_t)l.words : 0, stream, p);
-  CM_HIP_CHECK(hipGetLastError());
-  if (a.range_event) CM_HIP_CHECK(hipEventRecord((hipEvent_t)a.range_event, stream));
+  p.range_event = a.range_event;
   const bool f16 = a.in_dtype == CPPMEGA_MI355_F16;
   switch (a.head_dim) {
     case 32: return f16 ? run<true, 32>(p, stream) : run<false, 32>(p, stream);

@@ -244,3 +244,16 @@ def test_lists_out_of_range_leave_the_output_as_it_was(dt, at):
     assert (out == 5.0).all()
     dsa_splitk_indexer_loss_per_position(idx, top, q, k, 0.125, True, out=out)       # (and the next call is not held up)
     assert not (out == 5.0).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(150, 1, 3, 64, 170, 40), (330, 2, 6, 128, 330, 50), (340, 1, 5, 64, 340, 30), (70, 1, 2, 128, 70, 9), (1100, 3, 5, 96, 1100, 64)])
+@pytest.mark.parametrize("sparse", [False, True])
+def test_scores_far_from_zero(shape, sparse):
+    """Tiles whose exponentials leave float32 without a maximum taken off beside tiles where they do not; heads that are not
+    whole groups of two or four.  Scores of up to 250 in base 2 are good to 250 * 2^-23 = 3e-5, and so are the shares."""
+    ASq, AB, AH, AD, Sk, topk = shape
+    q, k, idx, top = _case(ASq + AH, ASq, AB, AH, AD, Sk, topk, torch.bfloat16)
+    q[ASq // 3:] *= 32
+    got = dsa_splitk_indexer_loss_per_position(idx.cuda(), top.cuda(), q.cuda(), k.cuda(), AD ** -0.5, sparse).cpu().numpy()
+    np.testing.assert_allclose(got, _want(q, k, idx, top, AD ** -0.5, sparse), atol=2e-5, rtol=2e-4)
