@@ -557,6 +557,9 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     // product of tile t-1 is done.
     unsigned s_cur = 0, s_nxt = kSlotBytes;       // ring offsets of the tile produced in this round and of the next one
     for (int t = -1; t < n_tiles; ++t) {
+      // P and the rescaling factors of the last round are in LDS before a consumer reads them.  (The barrier's own wait is
+      // missing from the code made for this loop: a write at its end and the barrier at its head met without one.)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();
       // (the first barrier only promises tile 0: tile 1's operands are read a round late, once)
       if (t <= 0 && t + 1 < n_tiles) load_k(s_cur, 0);

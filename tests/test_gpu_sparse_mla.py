@@ -694,3 +694,25 @@ def test_long_runs_of_skipped_entries(device, rows, valid):
     for s in (0, 7, 299):
         want, _ = om.sparse_mla_oracle(qf[:, s:s + 1], decoded, idx[:, s:s + 1], sm_scale=0.04, d_v=512)
         _assert_close(out[:, s:s + 1], None, want, None)
+
+
+@pytest.mark.parametrize("heads,topk", [(160, 4096), (64, 1000), (16, 300)])
+def test_code_rows_with_skipped_keys_repeat_bit_for_bit(device, heads, topk):
+    """Tiles that are written the careful way, with rows that arrive at their own pace: inputs in newly mapped memory every time."""
+    rng = np.random.default_rng(heads)
+    B, S, Skv = 1, 2, 9000
+    host = [t for side, n in (("q", heads), ("kv", None)) for t in fp8.quantize_per_token(
+        rng.standard_normal((B, S, n, 576) if side == "q" else (B, Skv, 1, 576)).astype(np.float32) * 3.0)]
+    idx = sparse_indices(rng, B, S, 1, Skv, topk, replace=True)
+    idx[rng.random(idx.shape) < 0.15] = -1
+    first = None
+    for _ in range(40):
+        torch.cuda.empty_cache()
+        ins = [to_dev(t, device) for t in (*host, idx.astype(np.int32))]
+        out = torch.zeros((B, S, heads, 512), dtype=torch.bfloat16, device=device)
+        lse = torch.zeros((B, S, heads), dtype=torch.float32, device=device)
+        f8.sparse_mla_fp8_path_c_apply_direct(*ins, sm_scale=576 ** -0.5, d_v=512, out=out, lse=lse)
+        got = (out.cpu(), lse.cpu())
+        first = first or got
+        assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1])
+        del ins, out, lse
