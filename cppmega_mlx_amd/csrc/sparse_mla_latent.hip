@@ -60,19 +60,21 @@ constexpr int kDqk = kLat + kRope;
 constexpr int kTK = 32;                         // keys per tile
 constexpr int kRing = 5;                        // tile slots
 constexpr int kAhead = kRing - 1;               // tiles issued ahead of the value product
-// A tile slot holds the rows in matrix-operand order.  Latent: for sub-tile sj (16 keys) and
-// 128-channel block blk, two planes j of 64 lanes x 16 bytes: lane (key n = lane % 16, kg = lane / 16)
-// of plane j holds channels 128 blk + 32 kg + 16 j .. + 15 of key 16 sj + n.  A plane is what one
-// load instruction writes (the load unit stores lane after lane) and what one 16-byte-per-lane
-// LDS read of a K operand fetches, contiguously.  Plane 1 starts 128 bytes after the end of plane
-// 0, so that the two neighbouring chunks a V^T read takes from eight rows fall on different banks.
-// Rope: for sub-tile sj and 32-channel step s one plane: lane (n, kq) holds channels 32 s + 8 kq .. + 7.
-constexpr int kPlane = 1024 + 128;              // bytes from plane 0 to plane 1 of a pair
-constexpr int kPair = 2 * kPlane;               // one (sub-tile, block)
-constexpr int kLatBytes = 8 * kPair;            // 18432
-constexpr int kRopeBytes = 4 * 1024;            // [sj][s] planes
+// A tile slot holds, per sub-tile sj (16 keys) and 128-channel block blk, the 16 rows' 128 bytes one after the other: a
+// load instruction (which stores lane after lane) takes 8 rows, 8 lanes to each, so that its quads of lanes read 64
+// contiguous bytes; with the lanes in operand order, every one in another row, it took four times as long (64 clocks for
+// 1 KB, 1400 of the 2000 that a tile has).  Piece c (16 channels) of row r stands at place c ^ fold(r): of the 16
+// lanes that an operand read serves together eight want piece q of rows 0..3 and 12..15 and eight piece q ^ 2 of rows
+// 4..11, and a transposing read takes pieces c and c ^ 1 of eight neighbouring rows; neither meets on a bank.
+// Rope: the same, its reads take q and q ^ 1, hence fold_rope.  Code rows: the 64 bytes of their tails, 16 rows each.
+constexpr int kPair = 16 * 128;                 // one (sub-tile, block)
+constexpr int kLatBytes = 8 * kPair;            // 16384
+constexpr int kRopeBytes = 2 * kPair;           // [sj]
+__host__ __device__ __forceinline__ constexpr int fold(int row) { return ((row >> 1) & 3) << 1 | ((row >> 3) & 1); }
+__host__ __device__ __forceinline__ constexpr int fold_rope(int row) { return (row >> 1) & 7; }
+__host__ __device__ __forceinline__ constexpr int fold_tail(int row) { return -(row >> 2) & 3; }
 constexpr int kScaleBytes = kTK * 4 * 4;        // up to four fp32 scales per row: [row][block]
-constexpr int kSlotBytes = kLatBytes + kRopeBytes + kScaleBytes;   // 23552
+constexpr int kSlotBytes = kLatBytes + kRopeBytes + kScaleBytes;   // 20992, a multiple of 128
 constexpr int kRingBytes = kRing * kSlotBytes;  // 104960
 constexpr int kMaxKeys = 2048;                  // keys of one split (their rows are staged in LDS)
 constexpr int kKeyInts = kMaxKeys + kTK;
@@ -371,22 +373,22 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
     uint4 tf[2];                                    // ROWS: the tails, 16 codes
     // (a tile's slot is passed as its byte offset into the ring, a running value: one address
     // register per slot then reaches every operand of the tile with an immediate offset)
+    const unsigned k_lane = (unsigned)(n * 128 + ((2 * kg) ^ fold(n)) * 16);
+    const unsigned r_lane = (unsigned)(n * 128 + (kg ^ fold_rope(n)) * 16), t_lane = (unsigned)(n * 64 + (kg ^ fold_tail(n)) * 16);
     auto load_k = [&](unsigned slot_off, int sj) {
-      const unsigned char* slot = smem + (slot_off + (unsigned)lane * 16u);
-      // the lane's 32 bytes of a block are its 16 bytes of the block's two planes
-      const unsigned char* lat = slot + sj * (4 * kPair);
-      const unsigned char* rope = slot + kLatBytes + sj * 2048;
+      // the lane's 32 bytes of a block are two neighbouring pieces
+      const unsigned char *lat0 = smem + (slot_off + k_lane) + sj * (4 * kPair), *lat1 = smem + (slot_off + (k_lane ^ 16u)) + sj * (4 * kPair);
 #pragma unroll
       for (int blk = 0; blk < 4; ++blk) {
-        const uint4 c0 = *reinterpret_cast<const uint4*>(lat + blk * kPair);
-        const uint4 c1 = *reinterpret_cast<const uint4*>(lat + blk * kPair + kPlane);
+        const uint4 c0 = *reinterpret_cast<const uint4*>(lat0 + blk * kPair);
+        const uint4 c1 = *reinterpret_cast<const uint4*>(lat1 + blk * kPair);
         kf[sj][blk] = i32x8{(int)c0.x, (int)c0.y, (int)c0.z, (int)c0.w, (int)c1.x, (int)c1.y, (int)c1.z, (int)c1.w};
       }
       if (ROWS) {
-        tf[sj] = *reinterpret_cast<const uint4*>(slot + kLatBytes + sj * 1024);
+        tf[sj] = *reinterpret_cast<const uint4*>(smem + (slot_off + t_lane) + kLatBytes + sj * 1024);
       } else {
-        rf[sj][0] = *reinterpret_cast<const bf16x8*>(rope);
-        rf[sj][1] = *reinterpret_cast<const bf16x8*>(rope + 1024);
+        rf[sj][0] = *reinterpret_cast<const bf16x8*>(smem + (slot_off + r_lane) + kLatBytes + sj * kPair);
+        rf[sj][1] = *reinterpret_cast<const bf16x8*>(smem + (slot_off + (r_lane ^ 64u)) + kLatBytes + sj * kPair);
       }
     };
     constexpr int kOne = 0x7f7f7f7f;                // operand exponent bytes of 2^0: the key bytes enter the products unscaled
@@ -593,10 +595,8 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   // nobody selected may hold NaN or infinity), so every tile is the same six load instructions per wavefront and the
   // in-order load counter can be waited on by count.  The loads are inline assembly (the compiler would otherwise order
   // every later LDS read behind them) with a uniform 64-bit base and a 32-bit byte offset per lane:
-  //   latent : block c of both sub-tiles, two planes each: lane (n, kg) of plane j fetches bytes
-  //            128 c + 32 kg + 16 j .. + 15 of key 16 sj + n
-  //   rope   : plane (sj = c / 2, s = c % 2): lane (n, kq) fetches bytes 64 s + 16 kq .. + 15 of the rope row
-  //            (ROWS: half c % 2 of the plane of sub-tile c / 2: bytes 512 + 16 kq .. + 15 of the row)
+  //   latent : block c of rows 8 h .. 8 h + 7 of the tile, h = 0 .. 3: lane l fetches piece (l % 8) ^ fold of row 8 h + l / 8
+  //   rope   : rows 8 c .. 8 c + 7, likewise (ROWS: the tails, four lanes to a row, half of the lanes of a sub-tile's instruction)
   //   scales : elements 8 nblk c .. 8 nblk (c + 1) - 1 of [32 rows][nblk], one per lane (without
   //            scales in memory: a word nobody reads, so that the count stays six)
   const size_t group_row0 = ((size_t)b * p.Skv_pitch) * p.G + g;     // cache row of key 0; key k is G rows further per step
@@ -604,7 +604,10 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   const unsigned char* rope_base = ROWS ? lat_base + kLat : (const unsigned char*)p.rope + group_row0 * (kRope * 2);
   const unsigned char* sc_base = has_scale ? (const unsigned char*)p.kv_scale + group_row0 * nblk * 4 : (const unsigned char*)p.kv;
   const unsigned lat_step = (unsigned)p.G * kRowPitch, rope_step = ROWS ? lat_step : (unsigned)p.G * (kRope * 2), sc_step = has_scale ? (unsigned)p.G * nblk * 4 : 0u;
-  const unsigned lat_lane = 128u * role + 32u * (lane >> 4), rope_lane = (ROWS ? 0u : 64u * (role & 1)) + 16u * (lane >> 4);
+  const int row8 = lane >> 3;                                         // of the eight rows of an instruction
+  const unsigned lat_even = 128u * role + 16u * (unsigned)((lane & 7) ^ fold(row8)), lat_odd = 128u * role + 16u * (unsigned)((lane & 7) ^ fold(8 + row8));
+  const int tail_row = 16 * (role >> 1) + (lane >> 2);
+  const unsigned rope_lane = 16u * (unsigned)(ROWS ? (lane & 3) ^ fold_tail(lane >> 2) : (lane & 7) ^ fold_rope(8 * (role & 1) + row8));
   const int sc_elem = 8 * nblk * role + lane;                         // (lanes below 8 nblk)
   const unsigned sc_lane = has_scale ? 4u * (unsigned)(sc_elem % nblk) : 0u;
   const int sc_row = min(sc_elem / nblk, kTK - 1);
@@ -621,26 +624,25 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
   // slot at `dma_slot`.  The value product spreads the parts between its matrix instructions:
   // issuing blocks while the load unit's queue is full.
   unsigned dma_slot = 0;                          // (uniform) LDS address of the slot being filled
-  unsigned off_l0 = 0, off_l1 = 0, off_r = 0, off_s = 0;
+  unsigned off_l[4] = {0, 0, 0, 0}, off_r = 0, off_s = 0;
   auto dma_prepare = [&](int tau, unsigned slot_off) {
     dma_slot = smem_base + slot_off;
     const int* tk = keys + tau * kTK;
     auto fetched = [&](int k) { return (unsigned)(k >= 0 ? k : spare_row); };
-    const unsigned k0 = fetched(tk[lane & 15]), k1 = fetched(tk[16 + (lane & 15)]);   // this lane's key of sub-tile 0 / 1
-    const unsigned ks = fetched(tk[sc_row]);
-    off_l0 = __umul24(k0, lat_step) + lat_lane;
-    off_l1 = __umul24(k1, lat_step) + lat_lane;
-    off_r = __umul24((role >> 1) ? k1 : k0, rope_step) + rope_lane;
-    off_s = __umul24(ks, sc_step) + sc_lane;
+    unsigned k[4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      k[h] = fetched(tk[8 * h + row8]);
+      off_l[h] = __umul24(k[h], lat_step) + (h & 1 ? lat_odd : lat_even);
+    }
+    off_r = __umul24(fetched(tk[ROWS ? tail_row : 8 * role + row8]), rope_step) + rope_lane;
+    off_s = __umul24(fetched(tk[sc_row]), sc_step) + sc_lane;
   };
   auto dma_part = [&](int i) {
-    if (i == 0) dma16(lat_base, off_l0, dma_slot + role * kPair);
-    else if (i == 1) dma16(lat_base, off_l0 + 16u, dma_slot + role * kPair + kPlane);
-    else if (i == 2) dma16(lat_base, off_l1, dma_slot + (4 + role) * kPair);
-    else if (i == 3) dma16(lat_base, off_l1 + 16u, dma_slot + (4 + role) * kPair + kPlane);
+    if (i < 4) dma16(lat_base, off_l[i], dma_slot + ((i >> 1) * 4 + role) * kPair + (i & 1) * (kPair / 2));
     else if (i == 4 && ROWS) {
       if ((lane >> 5) == (role & 1)) dma16(rope_base, off_r, dma_slot + kLatBytes + (role >> 1) * 1024);
-    } else if (i == 4) dma16(rope_base, off_r, dma_slot + kLatBytes + role * 1024);
+    } else if (i == 4) dma16(rope_base, off_r, dma_slot + kLatBytes + role * (kPair / 2));
     else if (sc_active) dma4(sc_base, off_s, dma_slot + sc_dst);
   };
   auto issue_tile = [&](int tau) {
@@ -658,21 +660,20 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
 #pragma unroll
       for (int j = 0; j < 16; ++j) o[i][hb][j] = 0.0f;
   const int pvar = (role * nblk) >> 2;                         // scale block of channels 128c..
-  // transposing reads of V^T: lanes t = 0..15 of a group read 8 bytes each from eight consecutive
-  // keys' 16-byte pieces (128 contiguous bytes); half selects the plane, kq2 the upper eight keys of
-  // the step; the four 32-channel blocks are 256 bytes apart
-  const unsigned char* pv_lane;
+  // transposing reads of V^T: lanes t = 0..15 of a group read 8 bytes each from eight consecutive keys' 16-byte
+  // pieces; half selects the piece of a 32-channel block, kq2 the upper eight keys of the step
+  const unsigned char* pv_lane[4];                             // per 32-channel block
   {
     const int t = lane & 15, half = (lane >> 4) & 1, kq2 = lane >> 5;
     const int r = 8 * kq2 + (t >> 1);                          // key within the 16-key step
-    pv_lane = smem + role * kPair + half * kPlane + r * 16 + 8 * (t & 1);
+#pragma unroll
+    for (int dvb = 0; dvb < 4; ++dvb) pv_lane[dvb] = smem + role * kPair + r * 128 + ((2 * dvb + half) ^ fold(r)) * 16 + 8 * (t & 1);
   }
   // V^T fragments of one 16-key step (four 32-channel blocks) of the tile in the slot at `slot_off`, raw
   auto load_v = [&](unsigned slot_off, int kstep, i32x2 (&vr)[4]) {
-    const unsigned char* vslot = pv_lane + slot_off;
 #pragma unroll
     for (int dvb = 0; dvb < 4; ++dvb)
-      vr[dvb] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) i32x2*)(vslot + kstep * (4 * kPair) + dvb * 256));
+      vr[dvb] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) i32x2*)(pv_lane[dvb] + slot_off + kstep * (4 * kPair)));
   };
   const unsigned char* p_lane = smem + kPOff + pvar * kPPlane + lane * 16;
   i32x2 v0[4];                                    // first step of the tile about to be consumed (read ahead of the barrier)
