@@ -207,3 +207,19 @@ def test_decode_layer_step_end_to_end(device):
     want_y = ovm.fused_fp8_gemm_oracle(w_o_codes, w_o_scale, o_h.reshape(B, H * D_v))
     err, ref = error_report(y.float().cpu().numpy(), want_y)
     assert err <= 2e-2 * ref, (err, ref)
+
+
+@pytest.mark.parametrize("shape", [(1, 2, 64, 32), (4, 3, 70, 160), (17, 2, 66, 128), (33, 1, 8, 512), (65, 2, 130, 480), (16, 2, 64, 544)])
+@pytest.mark.parametrize("y_dtype", [torch.bfloat16, torch.float16])
+def test_head_gemm_of_whole_bf16_rows(device, shape, y_dtype):
+    """Contractions that are whole steps of 32, up to 512 and one more, rows and channels that are not whole tiles, rows of a wider result."""
+    M, G, N, K = shape
+    rng = np.random.default_rng(M + K)
+    xt, wt = (to_dev(rng.standard_normal(s).astype(np.float32), device).bfloat16() for s in ((M, G, K), (G, N, K)))
+    want = np.einsum("mgk,gnk->mgn", xt.double().cpu().numpy(), wt.double().cpu().numpy())
+    for pad, at in ((0, 0), (12, 4), (10, 3)):
+        wide = torch.full((M, G, N + pad), 5.0, dtype=y_dtype, device=device)
+        ops.head_gemm(xt, wt, out=wide[..., at:at + N])
+        got = wide[..., at:at + N].double().cpu().numpy()
+        assert np.abs(got - want).max() <= 2.0 ** -8 * np.abs(want).max()            # one rounding to bfloat16
+        assert (wide[..., :at] == 5).all() and (wide[..., at + N:] == 5).all()
