@@ -29,6 +29,7 @@ struct MlaParams {
   int heads_per_wg;     // 0: 32-head tile kernel; 32 or 64: a producer/consumer kernel (sparse_mla_latent.hip, sparse_mla_rows16.hip)
   int plan_level;       // how the launch is planned: see sparse_mla_mfma_plan_within
   int rows16;           // with heads_per_wg: the kernel for 16-bit rows
+  int few;              // with heads_per_wg: the kernel for up to 16 heads per group (sparse_mla_few.hip)
   int tile_sharing;     // tile kernel on 16-bit rows: the 4 wavefronts take 4 head groups over one key stream
   float sm_scale;
   const float* sm_scale_dev;     // device copy of the softmax scale; read in place of sm_scale when set
@@ -85,6 +86,12 @@ bool sparse_mla_rows16_supported(const MlaParams& p);
 void sparse_mla_rows16_plan(MlaParams& p);
 int sparse_mla_rows16_launch(const MlaParams& p, hipStream_t stream);   // includes its combine step
 size_t sparse_mla_rows16_workspace_bytes(const MlaParams& p);
+
+// kernel for up to 16 heads per KV group (sparse_mla_few.hip); dispatched by the *_mfma_* functions
+bool sparse_mla_few_supported(const MlaParams& p);
+void sparse_mla_few_plan(MlaParams& p);
+int sparse_mla_few_launch(const MlaParams& p, hipStream_t stream);     // includes its combine step
+size_t sparse_mla_few_workspace_bytes(const MlaParams& p);
 
 // shared-tile kernel for FP8 latent caches (sparse_mla_latent.hip); dispatched by the *_mfma_* functions
 bool sparse_mla_latent_supported(const MlaParams& p);

@@ -926,7 +926,7 @@ __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const Ml
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
   const unsigned short* src0 = (const unsigned short*)p.workspace + block0 * (size_t)(HG * kPartFloats) +
-                               ((size_t)((w * HG + hg) * 8 + 2 * r4) * 64 + lane) * 8;
+                               ((size_t)((w * HG + hg) * 8 + 2 * r4) * 64 + 32 * half + min(hd, max(heads_here - 32 * hg, 1) - 1)) * 8;   // (no traffic for heads past the end)
 #pragma unroll
   for (int s0 = 0; s0 < 16; s0 += 4) {
     if (s0 >= p.num_splits) break;                            // (uniform)

@@ -889,7 +889,13 @@ size_t sparse_mla_mfma_plan_within(MlaParams& p, size_t have) {
 void sparse_mla_mfma_plan(MlaParams& p) {
   p.heads_per_wg = 0;
   p.rows16 = 0;
+  p.few = 0;
   p.tile_sharing = 0;
+  // (with less scratch than that plan asks for: the kernels and plans that there were before)
+  if (p.plan_level == 0 && sparse_mla_few_supported(p)) {
+    sparse_mla_few_plan(p);
+    return;
+  }
   // (latent caches of more than 32 heads have had the one kernel only: what needs too much scratch there is refused)
   const bool tiles_only = p.plan_level == 2 && tile_kernel_supported(p);
   if (sparse_mla_latent_supported(p) && !(tiles_only && !sparse_mla_latent_only(p))) {
@@ -916,12 +922,14 @@ void sparse_mla_mfma_plan(MlaParams& p) {
 }
 
 size_t sparse_mla_mfma_workspace_bytes(const MlaParams& p) {
+  if (p.few) return sparse_mla_few_workspace_bytes(p);
   if (p.heads_per_wg != 0) return p.rows16 ? sparse_mla_rows16_workspace_bytes(p) : sparse_mla_latent_workspace_bytes(p);
   if (p.num_splits <= 1) return 0;
   return (size_t)p.B * p.S * p.H * p.num_splits * (kLat + 2) * sizeof(float);
 }
 
 int sparse_mla_mfma_launch(const MlaParams& p, hipStream_t stream) {
+  if (p.few) return sparse_mla_few_launch(p, stream);
   if (p.heads_per_wg != 0) return p.rows16 ? sparse_mla_rows16_launch(p, stream) : sparse_mla_latent_launch(p, stream);
   const int groups_per_kv = (p.heads_per_group + kHeads - 1) / kHeads;
   const int units = p.tile_sharing ? (groups_per_kv + kWaves - 1) / kWaves : groups_per_kv;

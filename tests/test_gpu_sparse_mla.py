@@ -716,3 +716,56 @@ def test_code_rows_with_skipped_keys_repeat_bit_for_bit(device, heads, topk):
         first = first or got
         assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1])
         del ins, out, lse
+
+
+@pytest.mark.parametrize("S,H,G,topk", [(2, 1, 1, 1), (3, 16, 1, 32), (2, 10, 2, 33), (3, 16, 1, 129), (2, 32, 2, 640), (40, 16, 1, 527)])
+@pytest.mark.parametrize("rows", ["bf16", "float16_tail", "block128", "block256", "row", "none", "codes"])
+def test_up_to_16_heads_per_group(device, rows, S, H, G, topk):
+    """One key, a tile and one more, a tile for every wavefront and one more, key splits; lists of either index type with
+    skipped entries and an empty one, scores that grow along the list, and a cache row that no list names and is not finite."""
+    from cppmega_mlx_amd import _lib
+    B, Skv, sm = 1, 900, 0.05
+    rng = np.random.default_rng(S * H + topk)
+    idx = 1 + np.sort(sparse_indices(rng, B, S, G, Skv - 1, topk), axis=-1)
+    if topk > 1:
+        idx[rng.random(idx.shape) < 0.1] = -1
+    idx[0, 1] = -1
+    raw = rng.standard_normal((B, Skv, G, 576)).astype(np.float32) * np.linspace(0.2, 3.0, Skv).reshape(1, -1, 1, 1).astype(np.float32)
+    qraw, kw = rng.standard_normal((B, S, H, 576)).astype(np.float32), {}
+    if rows in ("bf16", "float16_tail"):
+        carrier = torch.bfloat16 if rows == "bf16" else torch.float16
+        q, kv = (torch.from_numpy(t).to(device).to(carrier) for t in (qraw, raw))
+        qf, decoded = q.double().cpu().numpy(), kv.double().cpu().numpy()
+        kv[0, 0] = float("nan")
+        if rows == "float16_tail":
+            kv, kw = kv[..., :512].contiguous(), dict(kv_rope=kv[..., 512:].contiguous())
+    elif rows == "codes":
+        (qc, qs), (kc, ks) = fp8.quantize_per_token(qraw), fp8.quantize_per_token(raw)
+        qf, decoded = om.dequant_per_token(qc, qs), om.dequant_per_token(kc, ks)
+        kc[0, 0], ks[0, 0] = 0x7f, np.inf
+        q, kv = to_dev(qc, device), to_dev(kc, device)
+        kw = dict(q_spec=ops.QuantSpec(_lib.SCALE_PER_TOKEN, to_dev(qs, device)), kv_spec=ops.QuantSpec(_lib.SCALE_PER_TOKEN, to_dev(ks, device)))
+    else:
+        q, qf = bf16_pair(qraw, device)
+        block = {"block128": 128, "block256": 256}.get(rows, 512)
+        kv, scale, rope, decoded = latent_cache(rng, B, Skv, G, 512, 64, device, pow2=False, block=block)
+        if rows == "none":
+            scale, sm = torch.ones_like(scale), 0.05 * 0.003           # (unscaled codes go up to 448)
+            decoded = om.dequant_block_latent(kv.cpu().numpy(), scale.cpu().numpy(), rope.float().cpu().numpy(), block)
+        kv[0, 0], rope[0, 0], scale[0, 0] = 0x7f, float("nan"), float("inf")
+        if rows == "row":
+            spec = ops.QuantSpec(_lib.SCALE_PER_TOKEN, scale.view(B, Skv, G), 0)
+        else:
+            spec = ops.QuantSpec() if rows == "none" else ops.QuantSpec(_lib.SCALE_F32_BLOCK, scale, block)
+        kw = dict(kv_spec=spec, kv_rope=rope)
+    sinks = rng.standard_normal(H).astype(np.float32)
+    want_out, want_lse = om.sparse_mla_oracle(qf, decoded, idx, sm_scale=sm, d_v=512, sinks=sinks)
+    for index_type in (np.int32, np.int64):
+        out = torch.zeros((B, S, H, 512), dtype=torch.float32, device=device)
+        lse = torch.zeros((B, S, H), dtype=torch.float32, device=device)
+        ops.sparse_mla_forward(q, kv, to_dev(idx.astype(index_type), device), sm_scale=sm, d_v=512, out=out, lse=lse,
+                               sinks=to_dev(sinks, device), kernel="mfma", **kw)
+        got = out.cpu().numpy()
+        assert np.isfinite(got).all()
+        err, ref = error_report(got, want_out)
+        assert err <= REL_TOL * ref and np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_TOL_MFMA
