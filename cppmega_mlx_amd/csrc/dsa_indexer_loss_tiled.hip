@@ -170,11 +170,11 @@ __host__ __device__ inline long long tiles_before(long long n, long long key_til
 
 // A tile of 64 positions; a wavefront has 32 positions (columns of v_mfma_f32_32x32x16, one per lane) and 64 keys (rows).
 // Whole tiles of 128 keys: two halves of the positions by two of the keys, a head at a time.  Split ones of 64 keys: two
-// halves of the positions by GROUPS groups of the heads, that many heads at a time.  The CUs hold resident() workgroups
-// each; whole rounds of them take whole tiles (64 + 128 rows per head pass through LDS for 8192 pairs, and the masks are set
-// up once for all heads), the rest, and everything where there is less than a round, go in split ones: what counts there is
-// a workgroup's time, which is its number of steps (1.6 us each, 4 us around them).  Four groups where split tiles have a CU
-// to themselves.
+// halves of the positions by GROUPS groups of the heads, that many heads at a time.  Whole tiles pass 64 + 128 rows per head
+// through LDS for 8192 pairs and set the masks up once for all heads; with less than a round of them what counts is a workgroup's
+// time, which is its number of steps (1.6 us each, 4 us around them), and split ones have half as many.  GROUPS == 1: every
+// tile is whole (three blocks of rows in LDS, not four: three workgroups on a CU for 128 channels); 2: the first p.whole
+// are; 4: none is, where split tiles have a CU to themselves.
 // GENERAL: an additive mask is given, or the softmax scale is not positive.  Otherwise the masks are 0 or -inf
 // and enter the first pass as what its products start from (a select behind them where a row that does not count
 // turned out not to be finite), and the second pass leaves keys that do not count out at its end.
@@ -182,15 +182,16 @@ __host__ __device__ inline long long tiles_before(long long n, long long key_til
 // scores, a row to a wavefront.
 constexpr int resident(int AD, bool general) { return AD <= 64 && !general ? 4 : 2; }
 template <bool F16, int AD, int GROUPS, bool SECOND, bool GENERAL>
-__global__ __launch_bounds__(128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_tile_kernel(const LossTiledParams p) {
-  constexpr int THREADS = 128 * GROUPS;
+__global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_tile_kernel(const LossTiledParams p) {
+  constexpr bool WHOLE = GROUPS == 1;                     // whole tiles only
+  constexpr int THREADS = WHOLE ? 256 : 128 * GROUPS, BLOCKS = WHOLE ? 3 : 2 * GROUPS;
   constexpr int PIECES = AD / 8;                          // 16-byte pieces of a row of one head
   constexpr int PITCH = PIECES + 1;                       // odd: 16 rows of a piece fall on 16 bank groups
   constexpr int LOADS = 64 * PIECES / THREADS;            // pieces of a thread of 64 rows of one head
   constexpr int STEPS = AD / 16;
   static_assert(LOADS * THREADS == 64 * PIECES, "whole pieces per thread");
   // 64 rows each: queries, keys of the first head, (split: queries,) keys of the second, ..; in the end the wavefronts' sums
-  constexpr int BLOCK = 64 * PITCH, ROWS = 2 * GROUPS * BLOCK, MEET = SECOND ? 2 * GROUPS * 32 * 64 / 4 : 0;
+  constexpr int BLOCK = 64 * PITCH, ROWS = BLOCKS * BLOCK, MEET = SECOND && !WHOLE ? 2 * GROUPS * 32 * 64 / 4 : 0;
   __shared__ u32x4 rows[ROWS > MEET ? ROWS : MEET];
 
   const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_
     const unsigned eight = (unsigned)id >> 3, stats_eights = (unsigned)(p.stats_groups + 7) >> 3, eights = gridDim.x >> 3;
     const unsigned before = eight * stats_eights / eights;
     if ((eight + 1) * stats_eights / eights != before) {
-      const int row = ((int)before * 8 + (id & 7)) * (2 * GROUPS) + wave;
+      const int row = ((int)before * 8 + (id & 7)) * (THREADS / 64) + wave;
       if (row < p.stats_rows) {
         const unsigned* bits = p.bits + (size_t)row * p.words;
         index_statistics(p, row, [&](int j) { return p.topk_idx ? bits[j >> 5] >> (j & 31) : 15u; });
@@ -211,7 +212,7 @@ __global__ __launch_bounds__(128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_
   }
   // Tile of this workgroup: the causal triangles of the batches, one after the other.  Consecutive workgroups go round the
   // eight XCDs, and each XCD takes one run of tiles, whose query rows (and the keys) its L2 holds.
-  const bool split = GROUPS > 2 || id >= p.whole;
+  const bool split = !WHOLE && (GROUPS > 2 || id >= p.whole);
   int within = id, count = p.whole;
   if (split) {
     within = id - p.whole;
@@ -253,18 +254,27 @@ __global__ __launch_bounds__(128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_
     src[i] = (unsigned)r * pos_bytes + (unsigned)c * 16u;
     dst[i] = r * PITCH + c;
   }
-  u32x4 piece[2 * GROUPS][LOADS];
+  u32x4 piece[BLOCKS][LOADS];
   float norm_next = 0.0f;
   const float* norm_src = SECOND ? p.norm + (size_t)b * p.AH * p.slab_rows + (live_q ? my_q - p.slab0 : 0) : nullptr;
   auto fetch = [&](int step) {
-#pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
-      const int h = split ? min(step * GROUPS + g, p.AH - 1) : step;
+    if constexpr (WHOLE) {
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
+        piece[0][i] = q_rows.load(src[i], step * AD * 2);
+        piece[1][i] = k_rows.load(src[i], step * AD * 2);
+        piece[2][i] = k_rows.load(src[i] + 64u * pos_bytes, step * AD * 2);
+      }
+    } else {
+#pragma unroll
+      for (int g = 0; g < GROUPS; ++g) {
+        const int h = split ? min(step * GROUPS + g, p.AH - 1) : step;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
         if (split || g == 0) piece[2 * g][i] = q_rows.load(src[i], h * AD * 2);
         piece[2 * g + 1][i] = k_rows.load(src[i] + (split || g == 0 ? 0u : 64u * pos_bytes), h * AD * 2);
       }
+    }
     }
     if (SECOND) norm_next = norm_src[(size_t)(split ? min(step * GROUPS + group, p.AH - 1) : step) * p.slab_rows];
   };
@@ -301,12 +311,12 @@ __global__ __launch_bounds__(128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_
     for (int v = 0; v < 16; ++v) mean[t][v] = 0.0f;
 
   const u32x4* const q_frag = rows + (split ? group : 0) * 2 * BLOCK + (wq + l32) * PITCH + half;
-  const u32x4* const k_frag = rows + (1 + 2 * group) * BLOCK + l32 * PITCH + half;
+  const u32x4* const k_frag = rows + (1 + (WHOLE ? group : 2 * group)) * BLOCK + l32 * PITCH + half;
   for (int step = 0; step < steps; ++step) {
     __syncthreads();                                      // the previous heads' rows are read
 #pragma unroll
-    for (int m = 0; m < 2 * GROUPS; ++m)
-      if (m != 2 || split)
+    for (int m = 0; m < BLOCKS; ++m)
+      if (WHOLE || m != 2 || split)
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) rows[m * BLOCK + dst[i]] = piece[m][i];
     const float norm = norm_next;
@@ -420,6 +430,7 @@ __global__ __launch_bounds__(128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_
   };
   float kl = 0.0f;
   if (split) {
+    if constexpr (!WHOLE) {
     // the groups of heads meet in LDS, and each finishes its share of the 32 registers
     constexpr int MINE = 32 / GROUPS;
     float* const meet = reinterpret_cast<float*>(rows) + lane;               // [wavefront][register][lane]
@@ -447,6 +458,7 @@ __global__ __launch_bounds__(128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_
     if (group) return;
 #pragma unroll
     for (int of = 1; of < GROUPS; ++of) kl += ends[of * 64];
+    }
   } else {
     if (!busy) return;
 #pragma unroll
@@ -536,8 +548,9 @@ Layout layout(const cppmega_mi355_dsa_loss_args_t& a) {
 
 template <bool F16, int AD, int GROUPS>
 void passes(LossTiledParams p, long long workgroups, bool general, hipStream_t stream) {
-  p.stats_groups = (p.stats_rows + 2 * GROUPS - 1) / (2 * GROUPS);
-  const dim3 grid((unsigned)workgroups), block(128 * GROUPS), merge(kThreads);
+  constexpr int waves = GROUPS == 1 ? 4 : 2 * GROUPS;
+  p.stats_groups = (p.stats_rows + waves - 1) / waves;
+  const dim3 grid((unsigned)workgroups), block(64 * waves), merge(kThreads);
   const dim3 with_statistics((unsigned)(p.stats_groups ? (workgroups + 7) / 8 * 8 + (p.stats_groups + 7) / 8 * 8 : workgroups));
   const long long columns = (long long)p.AB * p.slab_rows / 64;
   if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, false, true>), with_statistics, block, 0, stream, p);
@@ -555,7 +568,21 @@ int run(LossTiledParams p, hipStream_t stream) {
   const long long round = 256 * resident(AD, general);
   // (the lists' bits come first: the caller may be waiting for what that kernel finds)
   const size_t rows = (size_t)p.AB * p.ASq;
-  const bool in_tiles = p.slab_rows >= p.ASq && tiles_before((p.ASq + kQ - 1) / kQ, key_tiles) * p.AB < round;
+  // Tiles that are taken whole, of `all` ones.  Heads of up to 64 channels: whole rounds, and a rest of up to 9/16 of one is
+  // split (8 heads of 64, whole / split: 156 tiles 32.8 / 27.6 us, 361 39.5 / 37.5, 552 50.4 / 49.8, 702 54.6 / 56.4, 900 63.5 / 67.0; 1024 + 32
+  // 72.0 / 69.5; 16 heads: 47.6 / 36.5, 55.1 / 53.6, 73.5 / 71.0, 78.1 / 83.1, 92.6 / 99.7).  Larger heads, of which three workgroups of
+  // whole tiles fit on a CU and two of split ones: all or none (16 heads of 128: 225 tiles 66.7 / 58.6, 272 80.0 / 80.9, 441
+  // 87.0 / 99.8, 900 153.8 / 181.3; rounds of whole ones and a split rest 175.5).
+  auto whole_of = [&](long long all) {
+    if (AD > 64) return 2 * all > round ? all : 0;
+    const long long rest = all % round;
+    return 16 * rest <= 9 * round ? all - rest : all;
+  };
+  // The statistics go with the tiles where those are split, so that they do not fill the CUs (8 heads of 64, by themselves / with them:
+  // 156 tiles 30.4 / 27.6, 552 52.3 / 49.8; whole tiles, 16 heads: 900 92.2 / 95.5), and a workgroup of the larger heads
+  // keeps a CU or half of one (16 heads of 128: 64 tiles 37.8 / 34.0, 121 41.9 / 46.9, 225 58.6 / 71.2).
+  const long long of_all_rows = tiles_before((p.ASq + kQ - 1) / kQ, key_tiles) * p.AB;
+  const bool in_tiles = p.slab_rows >= p.ASq && whole_of(of_all_rows) == 0 && (AD <= 64 || of_all_rows <= 64);
   p.stats_rows = in_tiles ? (int)rows : 0;
   if (p.topk_idx || !in_tiles)
     hipLaunchKernelGGL(dsa_loss_list_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads), p.topk_idx ? 16 * (size_t)p.words : 0, stream, p);
@@ -566,8 +593,12 @@ int run(LossTiledParams p, hipStream_t stream) {
     p.first_tile = tiles_before(p.slab0 / kQ, key_tiles);
     p.tiles = (int)(tiles_before((end + kQ - 1) / kQ, key_tiles) - p.first_tile);
     const long long all = (long long)p.tiles * p.AB;
-    p.whole = (int)(all / round * round);
+    p.whole = (int)whole_of(all);
     const long long workgroups = p.whole + (all - p.whole) * 2;
+    if (p.whole == all) {
+      passes<F16, AD, 1>(p, workgroups, general, stream);
+      continue;
+    }
     if constexpr (AD == 64 || AD == 128) {
       if (workgroups <= 256 && p.AH > 2) {
         passes<F16, AD, 4>(p, workgroups, general, stream);
