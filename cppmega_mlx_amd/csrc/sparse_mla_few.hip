@@ -500,7 +500,9 @@ int sparse_mla_few_launch(const MlaParams& p, hipStream_t stream) {
 
 size_t sparse_mla_few_workspace_bytes(const MlaParams& p) {
   if (p.num_splits <= 1) return 0;
-  return (size_t)p.B * p.S * p.G * p.num_splits * (size_t)(kMlaPartFloats + 32 * 2) * sizeof(float);
+  // (8-bit rows: as much per split as the kernel for 64 heads asks for, so that scratch for the one serves the other)
+  const size_t blocks = p.kv_dtype == CPPMEGA_MI355_E4M3 ? 2 : 1;
+  return (size_t)p.B * p.S * p.G * p.num_splits * blocks * (size_t)(kMlaPartFloats + 32 * 2) * sizeof(float);
 }
 
 }  // namespace cm
