@@ -12,7 +12,7 @@
 //            16-bit planes each (hi = round(x), lo = round(x - hi), a term is good to 2^-17), and q and d_out by
 //            channel, both as dkv's matrix instructions take them: a load is 1 KB in a row;
 //   dq       per (query, 16 heads, 144 channels): dQ^T = K^T . dS^T over 32-key tiles staged in LDS (rows of 576 = 512 + 64
-//            channels and up to 512 keys: in the kernel of the scores);
+//            channels: in the kernel of the scores up to 256 keys, and up to 512 where there are few queries);
 //   dkv      per (band, 64 channels, share of the steps): dS^T . Q + P^T . dO of every step, added to a
 //            float32 tile in LDS, written out once;
 //   sum      over the shares, when there are several.
@@ -992,8 +992,8 @@ int run(SplitParams p, const Plan& l, bool clear, hipStream_t stream) {
   CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_kernel<F16, 8, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scores_lds(8)));
   CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_kernel<F16, 16, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scores_lds(16)));
   CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_dkv_kernel<F16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dkv_lds));
-  const bool fused = p.D == kD && p.d_v == kDv && p.topk <= 512;
-  if (fused) {
+  const bool rows_of_576 = p.D == kD && p.d_v == kDv && p.topk <= 512;
+  if (rows_of_576) {
     CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_dq_kernel<F16, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, kFusedLds<4>));
     CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_dq_kernel<F16, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, kFusedLds<8>));
   }
@@ -1005,6 +1005,9 @@ int run(SplitParams p, const Plan& l, bool clear, hipStream_t stream) {
     hipLaunchKernelGGL(bwd_lists_kernel, dim3((unsigned)lists), dim3(kThreads), (size_t)(3 * p.bands + 2 * p.topk + 2) * 4, stream, p);
     hipLaunchKernelGGL(bwd_steps_kernel, dim3((unsigned)(p.B * p.G * p.bands)), dim3(kStepThreads), 0, stream, p);
     const dim3 of_items((unsigned)items);
+    // Of eight wavefronts with up to 512 keys a CU holds one workgroup: one kernel while that is one round, else two (rows of 3000 keys, one kernel
+    // / two: 220 items x 350 27.5 / 36.5 us, 250 x 500 33.4 / 45.4, 376 x 438 55.9 / 53.7, 440 x 300 48.2 / 46.4, 2000 x 350 of 4000 215 / 194).
+    const bool fused = rows_of_576 && (p.topk <= 256 || items <= 256);
     if (fused) {
       if (p.topk <= 256) hipLaunchKernelGGL((bwd_scores_dq_kernel<F16, 4>), of_items, dim3(256), kFusedLds<4>, stream, p);
       else hipLaunchKernelGGL((bwd_scores_dq_kernel<F16, 8>), of_items, dim3(512), kFusedLds<8>, stream, p);

@@ -387,10 +387,12 @@ def test_one_key_named_many_times_over(device, times):
         assert err <= 1e-4 * scale, (err, scale)
 
 
-@pytest.mark.parametrize("heads,topk,valid", [(16, 16, 16), (5, 256, 256), (16, 256, 33), (24, 257, 257), (16, 512, 512), (8, 512, 1), (16, 513, 513)])
-def test_rows_of_576_channels_at_the_edges_of_their_tiles(device, heads, topk, valid):
-    """Up to 256 and up to 512 keys, and one more; whole and single tiles of 16 and 32 keys, and queries with fewer than the others."""
-    B, S, Skv, D, d_v = 2, 3, 700, 576, 512
+@pytest.mark.parametrize("S,heads,topk,valid", [(3, 16, 16, 16), (3, 5, 256, 256), (3, 16, 256, 33), (3, 24, 257, 257), (3, 16, 512, 512), (3, 8, 512, 1),
+                                                (3, 16, 513, 513), (128, 4, 300, 290), (129, 4, 300, 290)])
+def test_rows_of_576_channels_at_the_edges_of_their_tiles(device, S, heads, topk, valid):
+    """Up to 256 and up to 512 keys, and one more; whole and single tiles of 16 and 32 keys, queries with fewer than the others, and
+    256 and more queries."""
+    B, Skv, D, d_v = 2, 700, 576, 512
     rng = np.random.default_rng(topk + valid)
     q, kv, d_out = (to_dev(rng.standard_normal(s).astype(np.float32), device).bfloat16() for s in ((B, S, heads, D), (B, Skv, 1, D), (B, S, heads, d_v)))
     idx = sparse_indices(rng, B, S, 1, Skv, topk)
