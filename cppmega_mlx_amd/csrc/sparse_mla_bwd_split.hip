@@ -19,9 +19,9 @@
 //
 // Nothing is added in an order that varies: the same input gives the same bits.
 //
-// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 165 us (561 us with the atomics): lists 7, steps 7,
-// scores and dq 68, dkv 82, sum 9.  dkv is bound by the vector cache (27 M accesses of 64 bytes: 4 KB of q and d_out and
-// about 1 KB of planes for a step's 9 keys of 16) and ends with the CUs whose four bands are all full; scores and dq by the
+// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 158 us (561 us with the atomics; under the profiler lists 8,
+// steps 6, scores and dq 69, dkv 83, sum 9).  dkv is bound by the vector cache (27 M accesses of 64 bytes: 4 KB of q and d_out and
+// about 1 KB of planes for a step's 9 keys of 16) and ends with the CUs whose three bands are all full; scores and dq by the
 // gather of 302 MB of key rows each.
 
 #include <algorithm>
@@ -38,7 +38,11 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int kBandKeys = 150;         // at most: 151 rows of 64 floats (one for nobody) are 39 KB of LDS, four tiles to a CU
+// At most: 205 rows of 64 floats (one for nobody) are 52 KB of LDS, three tiles to a CU.  Four tiles of 150 keys name as many keys in more
+// steps and keep more of the planes in flight than an XCD's L2 holds (whole calls, 150 / 204 keys: 1024 queries x 16 heads x 256
+// of 4096 keys 166 / 161 us, 1000 x 64 x 250 of 8000 885 / 763, 900 x 64 x 500 of 8000 1081 / 950, 1000 x 32 x 400 of 5000 485 / 447,
+// 500 x 64 x 500 of 700 471 / 500).
+constexpr int kBandKeys = 204;
 constexpr int kAhead = 4;              // steps on their way in a wavefront of dkv
 constexpr int kStepGroup = 2 * kAhead; // steps come in whole rounds of dkv's two wavefronts
 constexpr int kAgain = 1 << 30;        // mark of a slot whose key occurs earlier in the same 16 slots
@@ -796,11 +800,11 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
 }
 
 // ---- dkv -----------------------------------------------------------------------------------------
-// A workgroup is two wavefronts and one band's tile, four workgroups to a CU.  The steps of a band are added one after
+// A workgroup is two wavefronts and one band's tile, three workgroups to a CU.  The steps of a band are added one after
 // the other (they may name the same key), with plain reads and writes: ds_add_f32 takes a lane at a time (1160 us for a
 // form of this kernel that took 280 with a plain write in its place).  So the wavefronts take turns: while one reads its
-// step's rows, adds and writes them, the other has its operands arrive and multiplies: 82 us at the shape above and 135
-// with 64 heads (512 queries, 256 of 2048 keys), where one wavefront per band, four bands to a workgroup, took 86 and 160.
+// step's rows, adds and writes them, the other has its operands arrive and multiplies.  Four such workgroups of 150 keys took 82 us at the
+// shape above and 135 with 64 heads (512 queries, 256 of 2048 keys), where one wavefront per band, four bands to a workgroup, took 86 and 160.
 // 16 bytes per lane of whole rows meet in no bank.  Two wavefronts per band with 32 channels each read the planes twice (110 us); one per 16 channels
 // of 600 keys, four times (315 us).
 constexpr int kDkvThreads = 128;
@@ -965,9 +969,9 @@ Plan make_plan(const cppmega_mi355_sparse_mla_bwd_args_t& a) {
   l.list_steps = a.topk / 16 + std::min<size_t>((size_t)a.topk, bands) + 1;
   const size_t per_s = lists * (l.stride * 4 + (2 * bands + 2) * 4 + l.list_steps * (16 + 16 * l.chunks) + l.chunks * ((size_t)l.stride * kRowBytes + (size_t)(a.d_qk + 63) / 64 * 4096));
   l.ns = (int)std::min<size_t>((size_t)a.seq_q, std::max<size_t>(kSlabBytes / per_s, 1));
-  // a CU holds four tiles of dkv: as many shares of the steps as bring the tiles to four times the number of CUs, of eight at least
+  // a CU holds three tiles of dkv: as many shares of the steps as bring the tiles to three times the number of CUs, of eight at least
   const long long tiles = (long long)l.bands * ((a.d_qk + 63) / 64) * lists;
-  l.shares = (int)std::max<long long>(1, std::min<long long>(1024 / tiles, (long long)l.ns * l.chunks * (a.topk / (bands * 16) + 1) / 8));
+  l.shares = (int)std::max<long long>(1, std::min<long long>(768 / tiles, (long long)l.ns * l.chunks * (a.topk / (bands * 16) + 1) / 8));
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t here = at; at += (bytes + 255) & ~(size_t)255; return here; };
   l.keys = take(lists * l.ns * l.stride * 4);
@@ -1035,8 +1039,8 @@ bool sparse_mla_bwd_split_supports(const cppmega_mi355_sparse_mla_bwd_args_t& a)
   // A step costs the same for one key of a band as for sixteen.  Measured at 64 .. 1024 queries against
   // sparse_mla_bwd_mfma.hip: with 16 heads it is as fast at one key per band (1.1 .. 1.3x) and 3.5x faster at nine;
   // with more heads, which that kernel adds up before its atomics, the line is at two to three (32 heads 0.8x at one
-  // key, 1.06x at two; 128 heads 0.9x at two, 1.3x at five).
-  const long long bands = ((long long)a.seq_kv + kBandKeys - 1) / kBandKeys;
+  // key, 1.06x at two; 128 heads 0.9x at two, 1.3x at five); bands of 150 keys there.
+  const long long bands = ((long long)a.seq_kv + 149) / 150;
   if (bands * (a.heads / a.kv_groups > kHeads ? 3 : 1) > a.topk) return false;
   if ((long long)a.batch * a.seq_q * a.heads * ((a.d_qk + 143) / 144) > 0x7fffffffLL) return false;
   const Plan l = make_plan(a);
