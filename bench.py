@@ -671,7 +671,7 @@ PROFILE_WORKLOADS = [
      "comparison, the one-workgroup-per-row kernel; the indexer's decode row runs the two-stage kernels as well"),
     ("indexer_scores_topk", "trace_main", ("fetch_main", "write_main"), None, ("indexer_scores_kernel", "indexer_qw_"),
      "indexer_topk q bf16[B,Sq,64,128], k bf16[B,Skv,128]: prefill (1, 8192, 8192) and decode (32, 1, 65536) dispatches"),
-    ("mla_absorb_head_gemm", "trace_main", ("fetch_main", "write_main"), None, ("head_gemm_kernel",),
+    ("mla_absorb_head_gemm", "trace_main", ("fetch_main", "write_main"), None, ("head_gemm_",),
      "head_gemm x bf16[32,128,128] . W bf16[128,512,128] and x bf16[32,128,512] . W bf16[128,128,512]"),
     ("kv_cache_append", "trace_main", ("fetch_main", "write_main"), None, ("cache_append_kernel",),
      "bf16 latent[B,S,1,512] + rope[..,64] -> e4m3 + fp32/128 scales + bf16 rope in the cache: one dispatch of 8192 rows "
@@ -680,7 +680,7 @@ PROFILE_WORKLOADS = [
      "sparse_mla_fwd q [1,8192,128,576], kv [1,8192,1,576], causal top-2048 indices -> [1,8192,128,512]: "
      "rows16<true, 2, false> unquantised float16 rows, latent<1, true, true> e4m3 rows with per-token fp32 scales, "
      "rows16<false, 2, true> (behind the conversion of the cache) e4m3 rows with E8M0 bytes per 32 channels"),
-    ("sparse_mla_backward", "trace_main", ("fetch_main", "write_main"), None, ("bwd_lists_kernel", "bwd_steps_kernel", "bwd_scores_kernel", "bwd_dq_kernel", "bwd_dkv_kernel", "bwd_sum_kernel"),
+    ("sparse_mla_backward", "trace_main", ("fetch_main", "write_main"), None, ("bwd_lists_kernel", "bwd_steps_kernel", "bwd_scores_", "bwd_dq_kernel", "bwd_dkv_kernel", "bwd_sum_kernel"),
      "sparse_mla_bwd q bf16[1,1024,16,576], kv bf16[1,4096,1,576], d_out bf16[1,1024,16,512], topk 256 -> dq bf16, dkv f32 "
      "(keys by band, steps, scores, dq, dkv added in LDS, the sum of its shares)"),
     ("dsa_indexer_loss", "trace_main", ("fetch_main", "write_main"), None, ("dsa_loss_", "dsa_indexer_loss"),
