@@ -302,8 +302,6 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
     }
   }
 
-  unsigned any = counts[0] | counts[1];                   // whether the position has a key here (of either half of the lanes)
-  any |= __float_as_uint(xor32(__uint_as_float(any)));
   float mean[2][16];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -349,8 +347,20 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
       }
     } else {
       float m, sum;
-      // exponentials relative to `at`, and their sum over the keys
-      auto add_up = [&](float at) {
+      auto statistics = [&]() {
+        m = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            if (GENERAL) s[t][v] = add[t][v] > -INFINITY ? fmaf(s[t][v], p.scale2, add[t][v]) : -INFINITY;
+            m = fmaxf(m, s[t][v]);
+          }
+        m = fmaxf(m, xor32(m));
+        if (!GENERAL) m *= p.scale2;
+        // (the maximum comes off inside the multiply-add: a score rounded to float32 by itself is off by 2^-24 of its size,
+        // which made the loss's error 1.7 times as large for scores of a spread of 1.4 in base 2 and 4 times for one of 8)
+        const float at = m > -INFINITY ? m : 0.0f;
         float d[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -362,37 +372,17 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
         sum = (d[0] + d[1]) + (d[2] + d[3]);
         sum += xor32(sum);
       };
-      auto relative_to_maximum = [&]() {
-        m = -INFINITY;
+      statistics();
+      // -inf + x is NaN where x is not finite: the row of a key that does not count holds such values, or a row that
+      // counts does.  Only then the masks are applied behind the products.
+      if (!GENERAL && __ballot(!(sum == sum)) != 0ull) {
+        asm volatile("" ::: "memory");                    // (the operands are read again: kept from above, they would not fit)
+        products(false);
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            if (GENERAL) s[t][v] = add[t][v] > -INFINITY ? fmaf(s[t][v], p.scale2, add[t][v]) : -INFINITY;
-            m = fmaxf(m, s[t][v]);
-          }
-        m = fmaxf(m, xor32(m));
-        if (!GENERAL) m *= p.scale2;
-        add_up(m > -INFINITY ? m : 0.0f);
-      };
-      if (GENERAL) {
-        relative_to_maximum();
-      } else {
-        // Scores of ordinary size need no maximum taken from them (a third of the instructions that are not exponentials):
-        // where the sum lies far from the ends of float32, every term that counts in it is a normal number.
-        add_up(0.0f);
-        m = any ? 0.0f : -INFINITY;
-        // Otherwise, and where -inf + x is NaN because x is not finite (the row of a key that does not count holds such
-        // values, or a row that counts does), the masks are applied behind the products and the maximum is taken.
-        if (__ballot(any ? !(sum > 0x1p-60f && sum < 0x1p+100f) : !(sum == 0.0f)) != 0ull) {
-          asm volatile("" ::: "memory");                  // (the operands are read again: kept from above, they would not fit)
-          products(false);
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) s[t][v] = add[t][v] == 0.0f ? s[t][v] : -INFINITY;
-          relative_to_maximum();
-        }
+          for (int v = 0; v < 16; ++v) s[t][v] = add[t][v] == 0.0f ? s[t][v] : -INFINITY;
+        statistics();
       }
       if (half == 0 && my_q - p.slab0 < p.slab_rows && live_q)
         p.part[((size_t)(kw / kChunk) * p.AB * p.AH + (size_t)b * p.AH + h) * p.slab_rows + (my_q - p.slab0)] = make_float2(m, sum);

@@ -257,3 +257,19 @@ def test_scores_far_from_zero(shape, sparse):
     q[ASq // 3:] *= 32
     got = dsa_splitk_indexer_loss_per_position(idx.cuda(), top.cuda(), q.cuda(), k.cuda(), AD ** -0.5, sparse).cpu().numpy()
     np.testing.assert_allclose(got, _want(q, k, idx, top, AD ** -0.5, sparse), atol=2e-5, rtol=2e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(420, 1, 8, 64, 420, 100), (420, 1, 8, 128, 420, 100)])
+@pytest.mark.parametrize("sparse", [False, True])
+def test_scores_on_a_common_level_lose_no_digits(shape, sparse):
+    """Scores around 25 in base 2.  A head's log2 of its denominator, in [32, 64), is rounded to float32 once: off by up to
+    2^-19, its share by that times ln 2, 7.6e-7 rms; the mean of 8 heads by 2.7e-7, and a loss of about one by up to twice
+    that.  (3.1e-7 .. 4.3e-7 measured; 1.2e-6 .. 1.8e-6 where the scores themselves are rounded before a maximum is taken off.)"""
+    ASq, AB, AH, AD, Sk, topk = shape
+    q, k, idx, top = _case(5, ASq, AB, AH, AD, Sk, topk, torch.bfloat16)
+    scale = AD ** -0.5
+    q[..., 0], k[..., 0] = 25 / 1.4427 / scale / 4, 4.0
+    got = dsa_splitk_indexer_loss_per_position(idx.cuda(), top.cuda(), q.cuda(), k.cuda(), scale, sparse).cpu().numpy()
+    want = _want(q, k, idx, top, scale, sparse)
+    assert np.sqrt(np.mean(((got - want) / np.maximum(1.0, np.abs(want))) ** 2)) <= 8e-7
