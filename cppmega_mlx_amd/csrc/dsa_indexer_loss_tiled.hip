@@ -329,11 +329,32 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int v = 0; v < 16; ++v) s[t][v] = masked ? add[t][v] : 0.0f;
+      if constexpr (AD > 64) {
+        // Of the larger heads the operands are read a step ahead of their products: a wavefront is alone with one or two others
+        // on its SIMD, and by itself the compiler waits for each (16 heads of 128, second pass, 272 tiles 36.5 -> 32.7 us, 1806
+        // tiles 71.8 -> 67.6; up to 64 channels there are no registers for it: 28.7 -> 36.1).
+        u32x4 qf[2], kf[2][2];
+        auto read = [&](int k) {
+          qf[k & 1] = q_frag[2 * k];
 #pragma unroll
-      for (int k = 0; k < STEPS; ++k) {
-        const u32x4 qf = q_frag[2 * k];
+          for (int t = 0; t < 2; ++t) kf[k & 1][t] = k_frag[t * 32 * PITCH + 2 * k];
+        };
+        read(0);
+        read(1);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) s[t] = product<F16>(k_frag[t * 32 * PITCH + 2 * k], qf, s[t]);
+        for (int k = 0; k < STEPS; ++k) {
+#pragma unroll
+          for (int t = 0; t < 2; ++t) s[t] = product<F16>(kf[k & 1][t], qf[k & 1], s[t]);
+          if (k + 2 < STEPS) read(k + 2);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < STEPS; ++k) {
+          const u32x4 qf = q_frag[2 * k];
+#pragma unroll
+          for (int t = 0; t < 2; ++t) s[t] = product<F16>(k_frag[t * 32 * PITCH + 2 * k], qf, s[t]);
+        }
       }
     };
     products(!SECOND && !GENERAL);
