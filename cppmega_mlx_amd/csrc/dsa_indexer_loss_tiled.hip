@@ -258,28 +258,26 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
   u32x4 piece[BLOCKS][LOADS];
   float norm_next = 0.0f;
   const float* norm_src = SECOND ? p.norm + (size_t)b * p.AH * p.slab_rows + (live_q ? my_q - p.slab0 : 0) : nullptr;
-  auto fetch = [&](int step) {
-    if constexpr (WHOLE) {
+  // (first pass of split tiles, 64 channels: the last 64 rows are requested behind the products, whose operands need the registers)
+  constexpr bool LATE = !SECOND && GROUPS == 2 && AD == 64;
+  auto fetch_rows = [&](int step, int from, int to) {     // rows of the blocks from .. to - 1
+#pragma unroll
+    for (int m = from; m < to; ++m) {
+      const int h = split ? min(step * GROUPS + (m >> 1), p.AH - 1) : step;
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
-        piece[0][i] = q_rows.load(src[i], step * AD * 2);
-        piece[1][i] = k_rows.load(src[i], step * AD * 2);
-        piece[2][i] = k_rows.load(src[i] + 64u * pos_bytes, step * AD * 2);
-      }
-    } else {
-#pragma unroll
-      for (int g = 0; g < GROUPS; ++g) {
-        const int h = split ? min(step * GROUPS + g, p.AH - 1) : step;
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) {
-        if (split || g == 0) piece[2 * g][i] = q_rows.load(src[i], h * AD * 2);
-        piece[2 * g + 1][i] = k_rows.load(src[i] + (split || g == 0 ? 0u : 64u * pos_bytes), h * AD * 2);
+        if (WHOLE) piece[m][i] = m ? k_rows.load(src[i] + (m == 2 ? 64u * pos_bytes : 0u), step * AD * 2) : q_rows.load(src[i], step * AD * 2);
+        else if (m & 1) piece[m][i] = k_rows.load(src[i] + (split || m == 1 ? 0u : 64u * pos_bytes), h * AD * 2);
+        else if (split || m == 0) piece[m][i] = q_rows.load(src[i], h * AD * 2);
       }
     }
-    }
+  };
+  auto fetch = [&](int step) {
+    fetch_rows(step, 0, LATE ? BLOCKS - 1 : BLOCKS);
     if (SECOND) norm_next = norm_src[(size_t)(split ? min(step * GROUPS + group, p.AH - 1) : step) * p.slab_rows];
   };
   fetch(0);
+  if (LATE) fetch_rows(0, BLOCKS - 1, BLOCKS);
 
   // register v of a 32-key block: key 8 * (v / 4) + 4 * half + v % 4
   float add[2][16];
@@ -322,7 +320,10 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
     fetch(min(step + 1, steps - 1));
     __syncthreads();
     const int h = split ? step * GROUPS + group : step;
-    if (!busy || h >= p.AH) continue;                     // (uniform)
+    if (!busy || h >= p.AH) {                             // (uniform)
+      if (LATE) fetch_rows(min(step + 1, steps - 1), BLOCKS - 1, BLOCKS);
+      continue;
+    }
     f32x16 s[2];
     auto products = [&](bool masked) {
 #pragma unroll
@@ -358,6 +359,10 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
       }
     };
     products(!SECOND && !GENERAL);
+    if (LATE) {
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_rows(min(step + 1, steps - 1), BLOCKS - 1, BLOCKS);
+    }
     // (exponentials first, sums behind them: a sum right behind its exponential waits for it)
     if constexpr (SECOND) {
 #pragma unroll
