@@ -585,21 +585,26 @@ int run(LossTiledParams p, hipStream_t stream) {
   const long long round = 256 * resident(AD, general);
   // (the lists' bits come first: the caller may be waiting for what that kernel finds)
   const size_t rows = (size_t)p.AB * p.ASq;
-  // Tiles that are taken whole, of `all` ones.  Heads of up to 64 channels: whole rounds, and a rest of up to 9/16 of one is
-  // split (8 heads of 64, whole / split: 156 tiles 32.8 / 27.6 us, 361 39.5 / 37.5, 552 50.4 / 49.8, 702 54.6 / 56.4, 900 63.5 / 67.0; 1024 + 32
-  // 72.0 / 69.5; 16 heads: 47.6 / 36.5, 55.1 / 53.6, 73.5 / 71.0, 78.1 / 83.1, 92.6 / 99.7).  Larger heads, of which three workgroups of
-  // whole tiles fit on a CU and two of split ones: all or none (16 heads of 128: 225 tiles 66.7 / 58.6, 272 80.0 / 80.9, 441
-  // 87.0 / 99.8, 900 153.8 / 181.3; rounds of whole ones and a split rest 175.5).
+  // Tiles that are taken whole, of `all` ones.  Heads of up to 64 channels: whole rounds, and a rest of up to 9/16 of one (with
+  // lists, whose kernel takes the statistics of the index scores beside them, 7/16) is split (dense, whole / split, 8 heads of
+  // 64: 121 tiles 31.6 / 25.2 us, 361 39.2 / 37.7, 552 49.5 / 48.0, 702 52.4 / 54.8, 900 60.2 / 64.8; 16 heads: 46.5 / 30.8, 54.7 / 50.9, 70.4 /
+  // 69.9, 74.5 / 81.1, 89.8 / 98.3; lists: 361 tiles 49.6 / 47.8 and 64.7 / 60.9, 450 52.3 / 52.8 and 68.0 / 67.6, 544 56.3 / 58.7 and 77.2 / 79.7).
+  // Larger heads, of which three workgroups of whole tiles fit on a CU and two of split ones: all or none (16 heads of 128: 225
+  // tiles 62.7 / 55.2, 272 75.2 / 76.0, 441 81.2 / 95.7, 900 149.8 / 176.2).
   auto whole_of = [&](long long all) {
     if (AD > 64) return 2 * all > round ? all : 0;
     const long long rest = all % round;
-    return 16 * rest <= 9 * round ? all - rest : all;
+    return 16 * rest <= (p.topk_idx ? 7 : 9) * round ? all - rest : all;
   };
-  // The statistics go with the tiles where those are split, so that they do not fill the CUs (8 heads of 64, by themselves / with them:
-  // 156 tiles 30.4 / 27.6, 552 52.3 / 49.8; whole tiles, 16 heads: 900 92.2 / 95.5), and a workgroup of the larger heads
-  // keeps a CU or half of one (16 heads of 128: 64 tiles 37.8 / 34.0, 121 41.9 / 46.9, 225 58.6 / 71.2).
+  // The statistics go with the tiles where those are split, so that they do not fill the CUs, and leave room for them: with
+  // lists, whose kernel is there anyway, up to a fifth of a round of tiles (by themselves / with them, 8 heads of 64: 180 tiles 39.0 /
+  // 36.8 us, 242 40.0 / 41.4, 450 52.8 / 56.1), dense up to 5/16, and where the split ones are more than a round anyway; between, tiles
+  // that would start at once wait for them (272 35.8 / 33.7, 361 37.7 / 38.2, 450 42.1 / 44.0, 552 51.1 / 48.1; 16 heads 48.5 / 46.3, 50.9 /
+  // 52.1, 57.1 / 64.9, 71.9 / 69.9).  A workgroup of the larger heads keeps a CU or half of one (16 heads of 128: 64 tiles 38.8 / 35.1, 121
+  // 42.1 / 47.3, 225 56.3 / 67.2).
   const long long of_all_rows = tiles_before((p.ASq + kQ - 1) / kQ, key_tiles) * p.AB;
-  const bool in_tiles = p.slab_rows >= p.ASq && whole_of(of_all_rows) == 0 && (AD <= 64 || of_all_rows <= 64);
+  const bool room = AD > 64 ? of_all_rows <= 64 : p.topk_idx ? 5 * of_all_rows <= round : 16 * of_all_rows <= 5 * round || 2 * of_all_rows > round;
+  const bool in_tiles = p.slab_rows >= p.ASq && whole_of(of_all_rows) == 0 && room;
   p.stats_rows = in_tiles ? (int)rows : 0;
   if (p.topk_idx || !in_tiles)
     hipLaunchKernelGGL(dsa_loss_list_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads), p.topk_idx ? 16 * (size_t)p.words : 0, stream, p);
