@@ -184,10 +184,14 @@ static int check_shape(const cppmega_mi355_dsa_loss_args_t& a) {
 int dsa_indexer_loss_workspace_bytes(const cppmega_mi355_dsa_loss_args_t& a, size_t* bytes) {
   const int rc = check_shape(a);
   if (rc) return rc;
-  // A short dense loss is one launch of the kernel without a workspace.  Measured, it against the four tiled launches: 256
-  // positions, 8 heads of 64: 18.8 / 24.1 us (two sequences the same); 16 heads 28.0 / 24.2; 320 positions, 8 heads
-  // 27.9 / 25.0, two sequences of 16 heads 45.6 / 24.7; 128 positions 16.2 / 24.1.
-  const bool one_launch = !a.topk_indices && a.seq_k <= 256 && (long long)a.heads * a.head_dim <= 512 && a.head_dim <= 64 && (long long)a.batch * a.seq_q <= 1024;
+  // A short dense loss is one launch of the kernel without a workspace, whose time grows with the heads and in steps of 64 and
+  // 256 keys; the four tiled launches take 24 us up to 16 heads, by the host.  Measured, the one launch / the tiled ones: 128 positions, heads
+  // of 64: 8 16.8 / 24.2 us, 16 25.4 / 24.1 .. 26.6, 20 29.4 / 25.7; of 32: 32 28.9 / 31.7, 128 92.4 / 91.8; 192: 12 of 64 22.7 / 24.4, 14 24.9 /
+  // 24.3, 24 of 32 26.8 / 27.3, 28 29.9 / 29.5; 256: 12 of 64 23.8 / 24.2, 16 of 32 23.8 / 24.2, 20 27.0 / 24.8; 320: 4 of 64 20.0 /
+  // 24.2, 6 24.1 / 24.2, 8 of 32 23.9 / 24.3, 10 26.9 / 24.4 (three sequences the same).
+  const bool narrow = a.head_dim <= 32;
+  const int heads = a.seq_k <= 128 ? (narrow ? 128 : 16) : a.seq_k <= 192 ? (narrow ? 24 : 12) : a.seq_k <= 256 ? (narrow ? 17 : 12) : a.seq_k <= 320 ? (narrow ? 8 : 5) : 0;
+  const bool one_launch = !a.topk_indices && a.heads <= heads && a.head_dim <= 64 && (long long)a.batch * a.seq_q <= 1024;
   *bytes = dsa_indexer_loss_tiled_supports(a) && !one_launch ? dsa_indexer_loss_tiled_workspace_bytes(a) : 0;
   return 0;
 }

@@ -268,3 +268,16 @@ def test_e8m0_rows_are_converted_within_bounds(rows, queries, converted):
     a.q_scale = a.kv_scale = 0x1000                          # (looked at, not through)
     assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0
     assert (need.value >= rows * 1152) == converted
+
+
+@pytest.mark.parametrize("heads,dim,keys,one", [
+    (8, 64, 256, True), (12, 64, 192, True), (16, 64, 128, True), (4, 64, 320, True), (32, 32, 100, True), (8, 32, 320, True),
+    (17, 64, 64, False), (13, 64, 256, False), (8, 64, 320, False), (32, 32, 256, False), (4, 128, 100, False), (4, 64, 321, False),
+])
+def test_short_dense_losses_are_one_launch_where_that_is_faster(heads, dim, keys, one):
+    need = C.c_size_t(1)
+    a = _lib.DsaLossArgs()
+    a.struct_size, a.in_dtype = C.sizeof(a), _lib.BF16
+    a.seq_q, a.batch, a.heads, a.head_dim, a.seq_k = keys, 1, heads, dim, keys
+    assert _lib.load().cppmega_mi355_dsa_indexer_loss_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0
+    assert (need.value == 0) == one

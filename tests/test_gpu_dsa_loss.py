@@ -273,3 +273,12 @@ def test_scores_on_a_common_level_lose_no_digits(shape, sparse):
     got = dsa_splitk_indexer_loss_per_position(idx.cuda(), top.cuda(), q.cuda(), k.cuda(), scale, sparse).cpu().numpy()
     want = _want(q, k, idx, top, scale, sparse)
     assert np.sqrt(np.mean(((got - want) / np.maximum(1.0, np.abs(want))) ** 2)) <= 8e-7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(128, 1, 16, 64, 128, 1), (128, 1, 17, 64, 128, 1), (192, 2, 12, 64, 192, 1), (193, 1, 24, 32, 193, 1), (320, 1, 5, 64, 320, 1), (321, 1, 5, 64, 321, 1), (40, 1, 128, 32, 128, 1)])
+def test_short_dense_losses_on_both_sides_of_the_one_launch_rule(shape):
+    ASq, AB, AH, AD, Sk, topk = shape
+    q, k, idx, top = _case(ASq + AH, ASq, AB, AH, AD, Sk, topk, torch.bfloat16)
+    got = dsa_splitk_indexer_loss_per_position(idx.cuda(), None, q.cuda(), k.cuda(), AD ** -0.5, False).cpu().numpy()
+    np.testing.assert_allclose(got, _want(q, k, idx, top, AD ** -0.5, False), atol=2e-5, rtol=2e-4)
