@@ -421,7 +421,12 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sparse_mla_few_kernel(const Ml
     const size_t off = (bs * p.H + head0 + n) * (size_t)kLat + 128 * wave + 4 * kg;
 #pragma unroll
     for (int i = 0; i < 8; ++i) sums[i] *= out_scale;
-    if (p.out_dtype == CPPMEGA_MI355_F32) {
+    if ((uintptr_t)p.out & 15) {                          // (uniform; not part of the choice of a plan: scratch is asked for before there is an output)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) store_as(p.out, off + 16 * i + e, p.out_dtype, sums[i][e]);
+    } else if (p.out_dtype == CPPMEGA_MI355_F32) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>((float*)p.out + off + 16 * i) = sums[i];
     } else {
@@ -455,7 +460,7 @@ int launch_as(const MlaParams& p, hipStream_t stream) {
 }  // namespace
 
 bool sparse_mla_few_supported(const MlaParams& p) {
-  if (p.heads_per_group > 16 || p.d_qk != kDqk || p.d_v != kLat || (uintptr_t)p.out & 15) return false;
+  if (p.heads_per_group > 16 || p.d_qk != kDqk || p.d_v != kLat) return false;
   const long long units = (long long)p.B * p.S * p.G;
   if (units * 16 > 0x7fffffffll) return false;
   // 8-bit rows: at 64 keys as fast as the kernel for 64 heads (9.3 / 9.1 us latent, 7.9 / 8.2 codes, one query), from there on

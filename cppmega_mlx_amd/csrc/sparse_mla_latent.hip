@@ -993,7 +993,7 @@ __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const Ml
       const float4 t = *reinterpret_cast<const float4*>(&x[row][c0 + 4 * i]);
       v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
     }
-    if (p.out_dtype == CPPMEGA_MI355_BF16) {
+    if (p.out_dtype == CPPMEGA_MI355_BF16 && ((uintptr_t)p.out & 15) == 0) {
       uint4 a, b;
       a = make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
       b = make_uint4(pack_bf16(v[8], v[9]), pack_bf16(v[10], v[11]), pack_bf16(v[12], v[13]), pack_bf16(v[14], v[15]));

@@ -281,3 +281,14 @@ def test_short_dense_losses_are_one_launch_where_that_is_faster(heads, dim, keys
     a.seq_q, a.batch, a.heads, a.head_dim, a.seq_k = keys, 1, heads, dim, keys
     assert _lib.load().cppmega_mi355_dsa_indexer_loss_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0
     assert (need.value == 0) == one
+
+
+@pytest.mark.parametrize("over", [dict(heads=16, batch=1), dict(heads=16, batch=4, topk=512), dict(heads=8, batch=1, seq_q=40, topk=640)])
+def test_the_scratch_asked_for_serves_any_output(over):
+    """The launch chooses its plan as the size query did, which may not know the output yet."""
+    need, known = C.c_size_t(0), C.c_size_t(0)
+    a = _latent_mla_args(**over)
+    assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == 0
+    a.out = 0x1002                                           # (looked at, not through)
+    assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(known)) == 0
+    assert need.value == known.value

@@ -769,3 +769,24 @@ def test_up_to_16_heads_per_group(device, rows, S, H, G, topk):
         assert np.isfinite(got).all()
         err, ref = error_report(got, want_out)
         assert err <= REL_TOL * ref and np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_TOL_MFMA
+
+
+@pytest.mark.parametrize("S,topk", [(300, 64), (2, 700)])          # in one piece; in key splits
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_up_to_16_heads_write_outputs_that_begin_anywhere(device, S, topk, dtype):
+    from cppmega_mlx_amd import _lib
+    H, Skv = 16, 900
+    rng = np.random.default_rng(S)
+    q, qf = bf16_pair(rng.standard_normal((1, S, H, 576)), device)
+    codes, scale, rope, decoded = latent_cache(rng, 1, Skv, 1, 512, 64, device, pow2=True)
+    idx = sparse_indices(rng, 1, S, 1, Skv, topk)
+    room = torch.full((1 + S * H * 512 + 1,), 7.0, dtype=dtype, device=device)
+    out = room[1:-1].view(1, S, H, 512)
+    ops.sparse_mla_forward(q, codes, to_dev(idx.astype(np.int32), device), sm_scale=0.04, d_v=512, out=out, kernel="mfma",
+                           kv_spec=ops.QuantSpec(_lib.SCALE_F32_BLOCK, scale, 128), kv_rope=rope)
+    aligned = torch.empty((1, S, H, 512), dtype=dtype, device=device)
+    ops.sparse_mla_forward(q, codes, to_dev(idx.astype(np.int32), device), sm_scale=0.04, d_v=512, out=aligned, kernel="mfma",
+                           kv_spec=ops.QuantSpec(_lib.SCALE_F32_BLOCK, scale, 128), kv_rope=rope)
+    assert torch.equal(out, aligned) and room[0] == 7.0 and room[-1] == 7.0
+    want, _ = om.sparse_mla_oracle(qf[:, :1], decoded, idx[:, :1], sm_scale=0.04, d_v=512)
+    _assert_close(out[:, :1], None, want, None)
