@@ -790,3 +790,55 @@ def test_up_to_16_heads_write_outputs_that_begin_anywhere(device, S, topk, dtype
     assert torch.equal(out, aligned) and room[0] == 7.0 and room[-1] == 7.0
     want, _ = om.sparse_mla_oracle(qf[:, :1], decoded, idx[:, :1], sm_scale=0.04, d_v=512)
     _assert_close(out[:, :1], None, want, None)
+
+
+# (260 queries: one piece, eight tiles to a wavefront; 40: six splits, three tiles to one)
+@pytest.mark.parametrize("S,topk", [(260, 1000), (40, 2048)])
+@pytest.mark.parametrize("rows,out_dtype", [("bf16", torch.bfloat16), ("float16", torch.float16), ("float16_tail", torch.float32), ("block128", torch.bfloat16),
+                                            ("block512", torch.float16), ("codes", torch.bfloat16), ("codes", torch.float32)])
+def test_up_to_16_heads_over_many_tiles(device, rows, out_dtype, S, topk):
+    """Several tiles of 32 keys to each of the four wavefronts: references that move (scores grow along the list by far more
+    than 2^8), tiles without a valid key in front of, behind and between others, one valid key, none; a cache row that no list
+    names is not finite.  Outputs of 16 bits are rounded once: 2^-8 of a value."""
+    from cppmega_mlx_amd import _lib
+    H, Skv, sm = 16, 2200, 0.1
+    rng = np.random.default_rng(S + topk)
+    idx = 1 + np.sort(np.stack([rng.permutation(Skv - 1)[:topk] for _ in range(S)]), axis=-1).reshape(1, S, 1, topk)
+    skip = rng.random(idx.shape) < 0.1
+    skip[0, :8] = True
+    skip[0, 0] = False                                                   # every entry
+    skip[0, 1, 0, [5 * 32 + 3, 6 * 32, 29 * 32 + 31]] = False            # three tiles of two wavefronts
+    skip[0, 2, 0, 20 * 32:] = False                                      # nothing in the first 20 tiles
+    skip[0, 3, 0, :40] = False                                           # nothing behind the first two
+    skip[0, 4, 0, topk - 1] = False                                      # the last entry alone
+    skip[0, 5, 0] = np.arange(topk) // 32 % 4 != 2                       # one wavefront has all there is
+    skip[0, 6, 0] = np.arange(topk) // 32 % 8 < 4                        # every other tile of each
+    idx[skip] = -1                                                       # (query 7 has none)
+    raw = rng.standard_normal((1, Skv, 1, 576)).astype(np.float32) * np.linspace(0.2, 3.0, Skv).reshape(1, -1, 1, 1).astype(np.float32)
+    qraw, kw = rng.standard_normal((1, S, H, 576)).astype(np.float32), {}
+    if rows in ("bf16", "float16", "float16_tail"):
+        carrier = torch.bfloat16 if rows == "bf16" else torch.float16
+        q, kv = (torch.from_numpy(t).to(device).to(carrier) for t in (qraw, raw))
+        qf, decoded = q.double().cpu().numpy(), kv.double().cpu().numpy()
+        kv[0, 0] = float("nan")
+        if rows == "float16_tail":
+            kv, kw = kv[..., :512].contiguous(), dict(kv_rope=kv[..., 512:].contiguous())
+    elif rows == "codes":
+        (qc, qs), (kc, ks) = fp8.quantize_per_token(qraw), fp8.quantize_per_token(raw)
+        qf, decoded = om.dequant_per_token(qc, qs), om.dequant_per_token(kc, ks)
+        kc[0, 0], ks[0, 0] = 0x7f, np.inf
+        q, kv = to_dev(qc, device), to_dev(kc, device)
+        kw = dict(q_spec=ops.QuantSpec(_lib.SCALE_PER_TOKEN, to_dev(qs, device)), kv_spec=ops.QuantSpec(_lib.SCALE_PER_TOKEN, to_dev(ks, device)))
+    else:
+        q, qf = bf16_pair(qraw, device)
+        block = int(rows[5:])
+        kv, scale, rope, decoded = latent_cache(rng, 1, Skv, 1, 512, 64, device, pow2=False, block=block)
+        kv[0, 0], rope[0, 0], scale[0, 0] = 0x7f, float("nan"), float("inf")
+        kw = dict(kv_spec=ops.QuantSpec(_lib.SCALE_F32_BLOCK, scale, block), kv_rope=rope)
+    out = torch.zeros((1, S, H, 512), dtype=out_dtype, device=device)
+    lse = torch.zeros((1, S, H), dtype=torch.float32, device=device)
+    ops.sparse_mla_forward(q, kv, to_dev(idx.astype(np.int32), device), sm_scale=sm, d_v=512, out=out, lse=lse, kernel="mfma", **kw)
+    assert torch.isfinite(out).all()
+    some = [0, 1, 2, 3, 4, 5, 6, 7, 8, S // 2, S - 1]
+    want_out, want_lse = om.sparse_mla_oracle(qf[:, some], decoded, idx[:, some], sm_scale=sm, d_v=512)
+    _assert_close(out[:, some], lse[:, some], want_out, want_lse, rel=REL_TOL + 2 ** -8, lse_tol=LSE_TOL_MFMA)
