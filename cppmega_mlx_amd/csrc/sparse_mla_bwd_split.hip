@@ -38,11 +38,8 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-// At most: 205 rows of 64 floats (one for nobody) are 52 KB of LDS, three tiles to a CU.  Four tiles of 150 keys name as many keys in more
-// steps and keep more of the planes in flight than an XCD's L2 holds (whole calls, 150 / 204 keys: 1024 queries x 16 heads x 256
-// of 4096 keys 166 / 161 us, 1000 x 64 x 250 of 8000 885 / 763, 900 x 64 x 500 of 8000 1081 / 950, 1000 x 32 x 400 of 5000 485 / 447,
-// 500 x 64 x 500 of 700 471 / 500).
-constexpr int kBandKeys = 204;
+// At most: 210 rows of 64 floats (one for nobody) are 52.5 KB of LDS, three tiles to a CU; how many there are is chosen by make_plan.
+constexpr int kBandKeys = 209;
 constexpr int kAhead = 4;              // steps on their way in a wavefront of dkv
 constexpr int kStepGroup = 2 * kAhead; // steps come in whole rounds of dkv's two wavefronts
 constexpr int kAgain = 1 << 30;        // mark of a slot whose key occurs earlier in the same 16 slots
@@ -80,8 +77,7 @@ struct SplitParams {
   float sm_scale;
 };
 
-constexpr int kDeadRow = kBandKeys;                    // of slots of no key
-static_assert(kDeadRow < 256, "rows are bytes");
+static_assert(kBandKeys < 256, "rows are bytes, and row band_keys is that of slots of no key");
 
 // ---- lists -----------------------------------------------------------------------------------
 // The valid keys by band in LDS, then each to its rank within the band.
@@ -99,7 +95,7 @@ __global__ __launch_bounds__(kThreads) void bwd_lists_kernel(const SplitParams p
   const int g = (int)(blockIdx.x - bs * (unsigned)p.G), b = (int)(bs / (unsigned)p.ns), s = (int)(bs - (unsigned)b * (unsigned)p.ns);
   const size_t src = (((size_t)b * p.S + p.s0 + s) * p.G + g) * (size_t)p.topk;
   if (list == 0 && tid == 0) p.band_steps[0] = 0;
-  if (list == 0 && tid < 16) p.rows[p.dead_step / 4 + tid] = kDeadRow;
+  if (list == 0 && tid < 16) p.rows[p.dead_step / 4 + tid] = (unsigned char)p.band_keys;
   for (int r = tid; r < p.bands; r += kThreads) fill[r] = 0;
   if (tid == 0) *again = 0;
   __syncthreads();
@@ -160,9 +156,9 @@ __global__ __launch_bounds__(kThreads) void bwd_lists_kernel(const SplitParams p
       const int of = v / p.band_keys, nth = k - begin[of], row = v - of * p.band_keys;
       const bool marked = (nth & 15) != 0 && sorted[k - 1] == v;
       unsigned char* at = rows + step_of[of] * 16 + nth;
-      *at = (unsigned char)(marked ? kDeadRow : row);
+      *at = (unsigned char)(marked ? p.band_keys : row);
       if (k + 1 == fill[of])
-        for (int e = nth + 1; e & 15; ++e) *++at = kDeadRow;
+        for (int e = nth + 1; e & 15; ++e) *++at = (unsigned char)p.band_keys;
       if (marked) {
         v |= kAgain;
         *again = 1;
@@ -818,7 +814,7 @@ struct Slab {
 };
 template <bool F16>
 __global__ __launch_bounds__(kDkvThreads, 2) void bwd_dkv_kernel(const SplitParams p) {
-  extern __shared__ __align__(16) float tile[];        // [kDeadRow + 1][64], the last row for lanes of no key
+  extern __shared__ __align__(16) float tile[];        // [band_keys + 1][64], the last row for lanes of no key
   const int tid = (int)threadIdx.x, lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // consecutive tiles read the same planes and rows: an XCD (launches go round them) takes a run of tiles
@@ -828,7 +824,7 @@ __global__ __launch_bounds__(kDkvThreads, 2) void bwd_dkv_kernel(const SplitPara
   if (bg >= p.B * p.G) return;
   const int g = bg % p.G, b = bg / p.G;
   const int k0 = band * p.band_keys, rows = min(p.band_keys, p.Skv - k0);
-  for (int e = tid; e < (kDeadRow + 1) * 16; e += kDkvThreads) reinterpret_cast<f32x4*>(tile)[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int e = tid; e < (p.band_keys + 1) * 16; e += kDkvThreads) reinterpret_cast<f32x4*>(tile)[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int* all = p.band_steps + 2 + 2 * (bg * p.bands + band);
   const int groups = __builtin_amdgcn_readfirstlane(all[1]) / kStepGroup;
@@ -959,19 +955,48 @@ struct Plan {
   size_t keys, starts, step_starts, rows, band_steps, steps, list_steps, planes, by_channel, part, slab_bytes, bytes;
 };
 
+// A CU holds three tiles of dkv: as many shares of the steps as bring the tiles to three times the number of CUs, of eight at least.
+int shares_of(long long tiles, long long items, int topk, int bands) {
+  return (int)std::max<long long>(1, std::min<long long>(768 / tiles, items * (topk / (bands * 16) + 1) / 8));
+}
+
+// Bands of a sequence's keys: the number with the least modelled time of what depends on it.  A list of n keys in a band is
+// n / 16 + 1/2 steps in the mean, 0.266 us each, which the busiest of the 768 places of a tile takes one after the other (with 22
+// bands of 9 columns three shares leave 174 places empty, with 21 four leave 12); the shares' sums cross memory twice; a band
+// more costs the lists and steps 0.3 us.  Measured on 108 shapes (8 .. 64 heads, 64 .. 1024 queries, 64 .. 512 of 512 .. 8192 keys),
+// up to nine numbers of bands each, whole calls: 0.4 % from the best of them in the mean, 1.8 % at most, and 4.4 % faster than bands
+// of 204 keys whatever the shape (1000 queries x 32 heads x 400 of 5000 keys, 25 / 28 bands 442 / 420 us; 394 x 64 x 183 of 4302 22 / 21
+// 231 / 208; 500 x 64 x 500 of 700 4 / 6 500 / 476; 1024 x 16 x 256 of 4096 21 / 22 157 / 171).  Four tiles of 150 keys on a CU keep more of
+// the planes in flight than an XCD's L2 holds (900 x 64 x 500 of 8000 943 / 1080).
+int choose_bands(const cppmega_mi355_sparse_mla_bwd_args_t& a) {
+  const long long columns = (long long)(a.d_qk + 63) / 64 * a.batch * a.kv_groups, items = (long long)a.seq_q * ((a.heads / a.kv_groups + kHeads - 1) / kHeads);
+  const int least = (a.seq_kv + kBandKeys - 1) / kBandKeys, most = std::min((a.seq_kv + 99) / 100, least + 48);
+  const double sum_us = (double)a.batch * a.seq_kv * a.kv_groups * a.d_qk * 8 / 3.5e6;
+  int best = least;
+  double best_us = 0.0;
+  for (int bands = least; bands <= most; ++bands) {
+    const int shares = shares_of(bands * columns, items, a.topk, bands);
+    const double n = (double)a.topk / bands, steps = items * std::min(n, n / 16 + 0.5) / shares;
+    const double us = 0.266 * (double)((bands * columns * shares + 767) / 768) * steps + (shares > 1 ? shares * sum_us : 0.0) + 0.3 * bands;
+    if (bands == least || us < best_us) {
+      best = bands;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 Plan make_plan(const cppmega_mi355_sparse_mla_bwd_args_t& a) {
   Plan l;
   l.chunks = (a.heads / a.kv_groups + kHeads - 1) / kHeads;
   l.stride = (a.topk + 15) / 16 * 16 + 32;
-  l.bands = (a.seq_kv + kBandKeys - 1) / kBandKeys;
+  l.bands = choose_bands(a);
   l.band_keys = (a.seq_kv + l.bands - 1) / l.bands;
   const size_t lists = (size_t)a.batch * a.kv_groups, bands = (size_t)l.bands;               // lists per query position
   l.list_steps = a.topk / 16 + std::min<size_t>((size_t)a.topk, bands) + 1;
   const size_t per_s = lists * (l.stride * 4 + (2 * bands + 2) * 4 + l.list_steps * (16 + 16 * l.chunks) + l.chunks * ((size_t)l.stride * kRowBytes + (size_t)(a.d_qk + 63) / 64 * 4096));
   l.ns = (int)std::min<size_t>((size_t)a.seq_q, std::max<size_t>(kSlabBytes / per_s, 1));
-  // a CU holds three tiles of dkv: as many shares of the steps as bring the tiles to three times the number of CUs, of eight at least
-  const long long tiles = (long long)l.bands * ((a.d_qk + 63) / 64) * lists;
-  l.shares = (int)std::max<long long>(1, std::min<long long>(768 / tiles, (long long)l.ns * l.chunks * (a.topk / (bands * 16) + 1) / 8));
+  l.shares = shares_of((long long)l.bands * ((a.d_qk + 63) / 64) * lists, (long long)l.ns * l.chunks, a.topk, l.bands);
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t here = at; at += (bytes + 255) & ~(size_t)255; return here; };
   l.keys = take(lists * l.ns * l.stride * 4);
@@ -991,7 +1016,7 @@ Plan make_plan(const cppmega_mi355_sparse_mla_bwd_args_t& a) {
 template <bool F16>
 int run(SplitParams p, const Plan& l, bool clear, hipStream_t stream) {
   auto scores_lds = [&](int waves) { return (size_t)2 * kHeads * (p.D + 8 + p.d_v + 8) + waves * (kHeads * 3 * 4 + 1024); };
-  const size_t dkv_lds = (size_t)(kDeadRow + 1) * 64 * 4;
+  const size_t dkv_lds = (size_t)(p.band_keys + 1) * 64 * 4;
   const int dq_parts = (p.D / 16 + kBlocks - 1) / kBlocks;
   CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_kernel<F16, 8, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scores_lds(8)));
   CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_kernel<F16, 16, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scores_lds(16)));
@@ -1036,10 +1061,11 @@ bool sparse_mla_bwd_split_supports(const cppmega_mi355_sparse_mla_bwd_args_t& a)
   const bool half = (a.q_dtype == CPPMEGA_MI355_BF16 || a.q_dtype == CPPMEGA_MI355_F16) && a.kv_dtype == a.q_dtype && a.d_out_dtype == a.q_dtype;
   if (!half || a.d_qk % 32 != 0 || a.d_v % 32 != 0 || a.d_qk > kBlocks * 64 || a.topk < 1 || a.topk > 2048) return false;
   if (a.batch < 1 || a.seq_q < 1 || a.seq_kv < 1 || a.seq_kv > 64 * 1024 || (long long)a.batch * a.kv_groups > 65535) return false;
-  // A step costs the same for one key of a band as for sixteen.  Measured at 64 .. 1024 queries against
-  // sparse_mla_bwd_mfma.hip: with 16 heads it is as fast at one key per band (1.1 .. 1.3x) and 3.5x faster at nine;
-  // with more heads, which that kernel adds up before its atomics, the line is at two to three (32 heads 0.8x at one
-  // key, 1.06x at two; 128 heads 0.9x at two, 1.3x at five); bands of 150 keys there.
+  // A step costs the same for one key of a band as for sixteen, and the atomics the same for each key.  Measured at 64, 300 and 1000
+  // queries over 1500 .. 60000 keys, time with the atomics over this path's by keys per 150 keys of the cache: up to 16 heads half a
+  // key 0.7 .. 1.2, one 0.7 .. 1.4 (below one for 64 queries of up to 8000 keys and for 1000 of 20000), one and a half 0.7 .. 1.6; with more
+  // heads, which that kernel adds up before its atomics, two 0.6 .. 1.6, three 0.7 .. 1.7 (below one for 64 queries of up to 4000 keys and
+  // for 300 and 1000 of 20000), four 0.9 .. 1.7.
   const long long bands = ((long long)a.seq_kv + 149) / 150;
   if (bands * (a.heads / a.kv_groups > kHeads ? 3 : 1) > a.topk) return false;
   if ((long long)a.batch * a.seq_q * a.heads * ((a.d_qk + 143) / 144) > 0x7fffffffLL) return false;

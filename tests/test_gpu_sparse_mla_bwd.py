@@ -404,3 +404,20 @@ def test_rows_of_576_channels_at_the_edges_of_their_tiles(device, S, heads, topk
     for got, ref in zip((dq, dkv), want):
         err, scale = error_report(got.cpu().numpy(), ref)
         assert err <= 1e-4 * scale, (err, scale)                # planes of 2^-17 and float32 sums of up to 1024 terms
+
+
+@pytest.mark.parametrize("Skv,topk", [(5, 4), (100, 90), (101, 64), (209, 100), (210, 100), (418, 33), (419, 200), (1000, 129), (4200, 64)])
+@pytest.mark.parametrize("S,H,G", [(2, 16, 1), (70, 24, 1), (40, 8, 2)])
+def test_bands_of_any_width(device, S, H, G, Skv, topk):
+    """One band and several, of as few and as many keys as there are, and the number of bands that few and many steps lead to."""
+    B, D, d_v = 1, 64, 64
+    rng = np.random.default_rng(Skv + S)
+    q, kv, d_out = (to_dev(rng.standard_normal(s).astype(np.float32), device).bfloat16() for s in ((B, S, H, D), (B, Skv, G, D), (B, S, H, d_v)))
+    idx = sparse_indices(rng, B, S, G, Skv, topk)
+    idx[0, 1, :, topk // 2:] = -1
+    want = om.sparse_mla_bwd_oracle(q.double().cpu().numpy(), kv.double().cpu().numpy(), idx, d_out.double().cpu().numpy(), sm_scale=D ** -0.5, d_v=d_v)
+    dq, dkv = torch.full((B, S, H, D), 9.0, device=device), torch.full((B, Skv, G, D), 9.0, device=device)
+    ops.sparse_mla_backward(q, kv, d_out, to_dev(idx.astype(np.int32), device), sm_scale=D ** -0.5, d_v=d_v, dq=dq, dkv=dkv)
+    for got, ref in zip((dq, dkv), want):
+        err, scale = error_report(got.cpu().numpy(), ref)
+        assert err <= 1e-4 * scale, (err, scale)                # planes of 2^-17 and float32 sums of up to 70 x 24 terms
