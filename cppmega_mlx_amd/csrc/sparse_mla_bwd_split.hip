@@ -1018,13 +1018,11 @@ int run(SplitParams p, const Plan& l, bool clear, hipStream_t stream) {
   auto scores_lds = [&](int waves) { return (size_t)2 * kHeads * (p.D + 8 + p.d_v + 8) + waves * (kHeads * 3 * 4 + 1024); };
   const size_t dkv_lds = (size_t)(p.band_keys + 1) * 64 * 4;
   const int dq_parts = (p.D / 16 + kBlocks - 1) / kBlocks;
-  CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_kernel<F16, 8, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scores_lds(8)));
-  CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_kernel<F16, 16, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scores_lds(16)));
-  CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_dkv_kernel<F16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dkv_lds));
+  // (all but the kernels of scores and dq together stay within the 64 KB that need no asking)
   const bool rows_of_576 = p.D == kD && p.d_v == kDv && p.topk <= 512;
   if (rows_of_576) {
-    CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_dq_kernel<F16, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, kFusedLds<4>));
-    CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_dq_kernel<F16, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, kFusedLds<8>));
+    if (p.topk <= 256) CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_dq_kernel<F16, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, kFusedLds<4>));
+    else CM_HIP_CHECK(hipFuncSetAttribute((const void*)bwd_scores_dq_kernel<F16, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, kFusedLds<8>));
   }
   for (p.s0 = 0; p.s0 < p.S; p.s0 += l.ns) {
     p.ns = std::min(l.ns, p.S - p.s0);
