@@ -842,3 +842,30 @@ def test_up_to_16_heads_over_many_tiles(device, rows, out_dtype, S, topk):
     some = [0, 1, 2, 3, 4, 5, 6, 7, 8, S // 2, S - 1]
     want_out, want_lse = om.sparse_mla_oracle(qf[:, some], decoded, idx[:, some], sm_scale=sm, d_v=512)
     _assert_close(out[:, some], lse[:, some], want_out, want_lse, rel=REL_TOL + 2 ** -8, lse_tol=LSE_TOL_MFMA)
+
+
+@pytest.mark.parametrize("rows", ["block128", "block512", "codes"])
+def test_up_to_16_heads_add_scores_128_channels_at_a_time(device, rows):
+    """Scores of up to about 100, times 0.3.  Rope and four sums of 128 channels, each rounded at its own size: rounding a score
+    five times on its way, 2^-18 / sqrt(3) at its full size, and the sums four times at a quarter of it, is 1.2e-6 rms (1.15e-6 ..
+    1.18e-6 measured); one chain through all channels 1.7e-6 (1.76e-6 and 1.97e-6)."""
+    from cppmega_mlx_amd import _lib
+    S, H, Skv, topk, sm = 64, 16, 4096, 512, 0.3
+    rng = np.random.default_rng(9)
+    idx = np.stack([rng.permutation(Skv)[:topk] for _ in range(S)]).reshape(1, S, 1, topk)
+    raw, qraw = rng.standard_normal((1, Skv, 1, 576)).astype(np.float32), rng.standard_normal((1, S, H, 576)).astype(np.float32)
+    if rows == "codes":
+        (qc, qs), (kc, ks) = fp8.quantize_per_token(qraw), fp8.quantize_per_token(raw)
+        qf, decoded = om.dequant_per_token(qc, qs), om.dequant_per_token(kc, ks)
+        q, kv = to_dev(qc, device), to_dev(kc, device)
+        kw = dict(q_spec=ops.QuantSpec(_lib.SCALE_PER_TOKEN, to_dev(qs, device)), kv_spec=ops.QuantSpec(_lib.SCALE_PER_TOKEN, to_dev(ks, device)))
+    else:
+        q, qf = bf16_pair(qraw, device)
+        block = int(rows[5:])
+        kv, scale, rope, decoded = latent_cache(rng, 1, Skv, 1, 512, 64, device, pow2=False, block=block)
+        kw = dict(kv_spec=ops.QuantSpec(_lib.SCALE_F32_BLOCK, scale, block), kv_rope=rope)
+    out = torch.empty((1, S, H, 512), dtype=torch.float32, device=device)
+    lse = torch.empty((1, S, H), dtype=torch.float32, device=device)
+    ops.sparse_mla_forward(q, kv, to_dev(idx.astype(np.int32), device), sm_scale=sm, d_v=512, out=out, lse=lse, kernel="mfma", **kw)
+    _, want_lse = om.sparse_mla_oracle(qf, decoded, idx, sm_scale=sm, d_v=512)
+    assert np.sqrt(np.mean((lse.cpu().numpy() - want_lse) ** 2)) <= 1.45e-6
