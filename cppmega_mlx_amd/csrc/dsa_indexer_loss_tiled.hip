@@ -36,7 +36,6 @@ constexpr int kChunk = 64;             // and keys
 constexpr float kEps = 1e-10f;
 constexpr size_t kPartBytes = 64u << 20;   // partial statistics of one slab of positions
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));       // rows of scores begin at any float
 
 struct LossTiledParams {
@@ -448,33 +447,33 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
   float kl = 0.0f;
   if (split) {
     if constexpr (!WHOLE) {
-    // the groups of heads meet in LDS, and each finishes its share of the 32 registers
-    constexpr int MINE = 32 / GROUPS;
-    float* const meet = reinterpret_cast<float*>(rows) + lane;               // [wavefront][register][lane]
-    __syncthreads();
+      // the groups of heads meet in LDS, and each finishes its share of the 32 registers
+      constexpr int MINE = 32 / GROUPS;
+      float* const meet = reinterpret_cast<float*>(rows) + lane;               // [wavefront][register][lane]
+      __syncthreads();
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) meet[((wave * 2 + t) * 16 + v) * 64] = mean[t][v];
-    __syncthreads();
-    const int t = group * MINE / 16, g0 = group * MINE % 16 / 4;
+        for (int v = 0; v < 16; ++v) meet[((wave * 2 + t) * 16 + v) * 64] = mean[t][v];
+      __syncthreads();
+      const int t = group * MINE / 16, g0 = group * MINE % 16 / 4;
 #pragma unroll
-    for (int g = 0; g < MINE / 4; ++g) {
-      float sums[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int g = 0; g < MINE / 4; ++g) {
+        float sums[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int of = 0; of < GROUPS; ++of)
+        for (int of = 0; of < GROUPS; ++of)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sums[i] += meet[(((of * 2 + (wave & 1)) * 2 + t) * 16 + 4 * (g0 + g) + i) * 64];
-      kl += divergence(t, g0 + g, sums);
-    }
-    kl += xor32(kl);
-    __syncthreads();
-    float* const ends = reinterpret_cast<float*>(rows) + wq + l32;
-    if (half == 0) ends[group * 64] = kl;
-    __syncthreads();
-    if (group) return;
+          for (int i = 0; i < 4; ++i) sums[i] += meet[(((of * 2 + (wave & 1)) * 2 + t) * 16 + 4 * (g0 + g) + i) * 64];
+        kl += divergence(t, g0 + g, sums);
+      }
+      kl += xor32(kl);
+      __syncthreads();
+      float* const ends = reinterpret_cast<float*>(rows) + wq + l32;
+      if (half == 0) ends[group * 64] = kl;
+      __syncthreads();
+      if (group) return;
 #pragma unroll
-    for (int of = 1; of < GROUPS; ++of) kl += ends[of * 64];
+      for (int of = 1; of < GROUPS; ++of) kl += ends[of * 64];
     }
   } else {
     if (!busy) return;

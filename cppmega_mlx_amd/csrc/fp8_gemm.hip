@@ -18,8 +18,6 @@
 namespace cm {
 namespace {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
 // 8 e4m3 codes -> the bf16 / fp16 values they stand for (exact)
 template <bool F16>
 __device__ __forceinline__ u32x4 codes8(unsigned a, unsigned b) {

@@ -88,6 +88,23 @@ __device__ __forceinline__ void dequant16(const uint4 raw, float scale, uint4& l
   hi = make_uint4(o[4], o[5], o[6], o[7]);
 }
 
+// 8 e4m3 bytes as bfloat16 (exact)
+__device__ __forceinline__ bf16x8 cvt8(unsigned w0, unsigned w1) {
+  const unsigned o0 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, false));
+  const unsigned o1 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, true));
+  const unsigned o2 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, false));
+  const unsigned o3 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, true));
+  return __builtin_bit_cast(bf16x8, make_uint4(o0, o1, o2, o3));
+}
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+// one 16 x 16 x 32 matrix instruction on operands held as 8 x 16 bits: bfloat16, or float16 when F16
+template <bool F16>
+__device__ __forceinline__ f32x4 mm(const bf16x8 a, const bf16x8 b, const f32x4 c) {
+  if (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
 // value of lane (lane ^ 16) / (lane ^ 32), VALU only
 __device__ __forceinline__ float xor16(float v) {
   const unsigned u = __float_as_uint(v);

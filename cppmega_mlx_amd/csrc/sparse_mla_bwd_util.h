@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.h"
+#include "mfma_util.h"
 
 namespace cm {
 
@@ -19,13 +20,6 @@ __device__ __forceinline__ bf16x8 join(const bf16x4 a, const bf16x4 b) {
   r[0] = a[0]; r[1] = a[1]; r[2] = a[2]; r[3] = a[3];
   r[4] = b[0]; r[5] = b[1]; r[6] = b[2]; r[7] = b[3];
   return r;
-}
-typedef _Float16 f16x8b __attribute__((ext_vector_type(8)));
-// one matrix instruction on operands held as 8 x 16 bits: bfloat16, or float16 when F16
-template <bool F16>
-__device__ __forceinline__ f32x4 mm(const bf16x8 a, const bf16x8 b, const f32x4 c) {
-  if (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8b, a), __builtin_bit_cast(f16x8b, b), c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 __device__ __forceinline__ bf16x8 zero8() {
   return __builtin_bit_cast(bf16x8, make_uint4(0u, 0u, 0u, 0u));

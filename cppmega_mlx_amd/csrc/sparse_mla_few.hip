@@ -32,7 +32,6 @@ namespace cm {
 
 namespace {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((ext_vector_type(4))) unsigned u4;
 
@@ -49,18 +48,6 @@ __device__ __forceinline__ int fold16(int r) { return ((r & 3) << 2) | (-(r >> 2
 __device__ __forceinline__ int fold8(int r) { return (r & 15) ^ ((r >> 1) & 8); }
 __device__ __forceinline__ int fold_rope(int r) { return (r >> 1) & 7; }
 __device__ __forceinline__ int fold_tail(int r) { return -(r >> 2) & 3; }
-
-template <bool F16>
-__device__ __forceinline__ f32x4 mm(const bf16x8& a, const bf16x8& b, const f32x4& c) {
-  if (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ bf16x8 cvt8(unsigned w0, unsigned w1) {
-  return __builtin_bit_cast(bf16x8, make_uint4(__builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, false)),
-                                               __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, true)),
-                                               __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, false)),
-                                               __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, true))));
-}
 
 // bytes of a wavefront's tile in LDS: rows, the rope part (code rows: the last 64 codes), scales
 template <int KIND> constexpr int kRowBytes = KIND == kRows16 ? 2 * kLat : kLat;

@@ -95,14 +95,6 @@ constexpr int kSmem = kKeyOff + kKeyInts * 4;
 static_assert(kSmem <= 160 * 1024, "LDS budget");
 static_assert(4 * 32 * kXPitch * 4 <= kRingBytes, "the output transpose reuses the ring");
 
-__device__ __forceinline__ bf16x8 cvt8(unsigned w0, unsigned w1) {
-  const unsigned o0 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, false));
-  const unsigned o1 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, true));
-  const unsigned o2 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, false));
-  const unsigned o3 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, true));
-  return __builtin_bit_cast(bf16x8, make_uint4(o0, o1, o2, o3));
-}
-
 // 16 x 16 x 128 over e4m3 bytes, operands scaled by 2^(byte - 127): the byte is byte SEL of `a_exp`
 // for A and of `b_exp` for B, and must be the same in the four lanes of a row (l, l+16, ..).
 template <int SEL>

@@ -42,8 +42,6 @@ namespace cm {
 
 namespace {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
 constexpr int kLat = 512;
 constexpr int kRope = 64;
 constexpr int kDqk = kLat + kRope;
