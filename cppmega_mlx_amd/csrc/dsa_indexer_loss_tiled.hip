@@ -17,10 +17,10 @@
 // and a lane reduces its own keys, so a head costs one lane exchange.
 //
 // Bound by the exponentials and the multiply-adds in front of them (two per pair and head).  Measured at
-// 4096 positions, 8 heads of 64, lists of 1024: 86 us a call (lists 20: 84 MB read; passes 24 and 29, merge and sum 9), 92
-// with whole tiles only and a maximum taken in the first pass, 274 with a workgroup of 8 wavefronts per 16 positions
+// 4096 positions, 8 heads of 64, lists of 1024: 84 us a call (lists 20: 84 MB read; passes 23 and 27, merge and sum 9), 88
+// with whole tiles only, 274 with a workgroup of 8 wavefronts per 16 positions
 // (256 workgroups, the longest with twice the mean work, statistics in LDS per step).  Short sequences are bound by a
-// workgroup's steps: 2 x 547 positions, 16 heads of 128 70 -> 43 us with split tiles, 943 x 8 x 128 54 -> 38.
+// workgroup's steps: 2 x 547 positions, 16 heads of 128 66 -> 34 us with split tiles, 943 x 8 x 128 44 -> 28.
 
 #include <algorithm>
 

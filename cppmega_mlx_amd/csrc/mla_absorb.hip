@@ -51,7 +51,8 @@ struct HeadGemmParams {
 // bf16 operands whose rows are whole 16-byte pieces, K a multiple of 32 up to 32 KS: every weight of a wavefront is
 // requested before the activations are looked at, so that a launch waits for memory once instead of twice, and the
 // activations come as whole rows.  At decode size a launch is that latency (4 rows, 128 heads: 128 -> 512 channels 6.7 -> 5.3 us,
-// 512 -> 128 7.4 -> 5.4; 16.8 MB of weights each, 3.4 us at the rate of a large copy).
+// 512 -> 128 7.4 -> 5.4; 16.8 MB of weights each, 3.4 us at the rate of a large copy).  No number of rows is slower: whole calls of 16,
+// 64 and 128 heads, 1 .. 4096 rows 1.0 .. 1.8x (1000 rows, 128 heads: 206 -> 117 us and 117 -> 95).
 template <int MT, int KS>
 __global__ __launch_bounds__(kThreads) void head_gemm_rows_kernel(const HeadGemmParams p) {
   extern __shared__ __align__(16) unsigned short x_lds[];       // [16 MT][kPitch]

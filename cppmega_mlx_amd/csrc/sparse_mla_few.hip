@@ -16,12 +16,13 @@
 // registers of a SIMD to itself.  Piece c (16 bytes) of row r stands at place c ^ fold: operand reads (16 rows, one
 // piece) and transposing reads spread over the banks.
 //
-// Bound: the LDS, which every row crosses three times (3300 of the 4600 clocks that four tiles of 16-bit rows take,
-// together); 8-bit rows halve that and spend it on conversions.  Four tiles of 128 keys took 3.4 .. 5 us before.
-// Measured (16 heads over 4096 keys; before -> here): 300 queries x 2048 keys: 16-bit rows 109 -> 86 us, latent 159 -> 92,
-// codes 147 -> 85; 100 x 512: 18.9 -> 17.7, 26.4 -> 18.6, 24.5 -> 17.2; one query x 2048 latent keys (splits) 20.2 -> 15.0.
-// Error against float64 (rms, 64 x 512 .. 8 x 2048): 16-bit rows 0.92 .. 0.95 of theirs, codes 0.98 .. 1.03 +- 0.02, latent 0.97 .. 0.99
-// (scales of the rows' own maxima) and 1.00 .. 1.01 (scales drawn by themselves): the same roundings.
+// Bound: a wavefront's own chain, alone on its SIMD.  Counters, 300 x 2048 16-bit rows / 700 x 1024 latent rows: it issues in 51 /
+// 58 % of its time (vector 23 / 43 %: 8-bit rows are converted), waits for data in 31 / 34 %; the matrix cores are busy for 15 /
+// 13 %, the LDS for 35 / 20 % of a workgroup's time, without a bank conflict.  Four tiles of 128 keys took 3.4 .. 5 us before.
+// Measured (16 heads over 4096 keys; before -> here): 300 queries x 2048 keys: 16-bit rows 104 -> 82 us, latent 159 -> 92,
+// codes 147 -> 85; 100 x 800 of 16 bits 24.7 -> 22.0, 100 x 512 latent 26.4 -> 18.8, codes 23.7 -> 17.0; one query x 2048 latent keys (splits) 20.3 -> 15.5.
+// Error against float64 (rms, here over before, 64 x 512 .. 300 x 1000, scores of a deviation of 1, 2.9 and 7): output of 16-bit rows
+// 0.72 .. 0.96, of 8-bit ones 0.93 .. 1.00; lse 0.92 .. 1.02.
 // Operand reads are requested eight ahead of their products: with a wait for each (as the compiler orders them by itself)
 // 700 queries x 1024 latent keys took 123 us, 84 so.
 
