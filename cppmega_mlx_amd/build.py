@@ -43,6 +43,7 @@ FILE_FLAGS: dict[str, list[str]] = {}
 NO_SCRATCH = {
     "sparse_mla_latent.hip": ("sparse_mla_latent_kernel",),
     "sparse_mla_rows16.hip": ("sparse_mla_rows16_kernel",),
+    "fp8_gemm.hip": ("fp8_gemm_kernel",),
 }
 
 

@@ -3,12 +3,14 @@
 //   out[m, n] = sum_k dec(w[n, k]) * w_scale(n, k / 128) * x[m, k],   x bf16 or fp16, fp32 accumulation
 //
 // The kernels of fp8_vecmat.hip read the whole weight once per 4 to 16 activation rows; from 17 rows on a
-// tile of both operands is worth staging in LDS.  Measured (microseconds, against passes over the weights):
-// M x N x K = 2048 x 8192 x 1536: 66 (3364), 48 x 7168 x 16384: 38 (60), 300 x 1434 x 896: 10 (190),
-// 2048 x 7168 x 16384: 490 = 980 TFLOP/s.  What bounds it: a large product, the issue of MFMAs and of the
-// vector instructions between them (128 per 32 MFMAs: conversions and scaled sums); a short one (K = 1536),
-// the first loads and the stores of a tile, 10 of 33 us, which a CU with one workgroup does not overlap; a
-// small batch, the weight stream (32 x 7168 x 16384: 37.5 us a call, 3.1 TB/s).
+// tile of both operands is worth staging in LDS.  The load unit writes the tiles there itself (global_load_lds, pieces of
+// 128 bytes of a row: such loads reach 50 B/clk a CU, pieces of 64 bytes 28, of 16 bytes 10), as many stages ahead as the
+// LDS holds.  Measured (microseconds a call; through registers, two stages ahead -> here), M x N x K:
+// 2048 x 8192 x 1536: 65 -> 59, 2048 x 7168 x 16384: 483 -> 441 = 1090 TFLOP/s, 1040 x 2621 x 5248: 58 -> 43,
+// 879 x 1007 x 6528: 48 -> 24, 231 x 4895 x 10240: 54 -> 38, 32 x 7168 x 16384: 37 -> 28, 55 x 2804 x 640: 7.6 -> 5.7.
+// What bounds it: a large product, the LDS (of 2048 clocks of products a 128 x 256 x 128 step, operand reads and arriving
+// rows take as many at 128 B/clk) and the vector instructions between the products; a small one, launch, first loads and
+// stores (5 us); a small batch, the weights' stream.
 
 #include <stdint.h>
 
@@ -37,321 +39,385 @@ __device__ __forceinline__ u32x4 codes8(unsigned a, unsigned b) {
 }
 
 template <bool F16>
-__device__ __forceinline__ f32x16 product(const u32x4& a, const u32x4& b, const f32x16& c) {
-  if (F16) return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+__device__ __forceinline__ f32x4 product(const u32x4& a, const u32x4& b, const f32x4& c) {
+  return mm<F16>(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c);
 }
 
-// Slot of 16-byte piece `piece` of row `row` in an LDS tile of `PIECES` pieces per row.  A 16-byte read
-// is served sixteen lanes (256 bytes, all banks) at a time, and the rows of such a group differ in their
-// low bits: the exclusive-or spreads one piece of 16 rows over the 16 bank groups.
-template <int PIECES>
-__device__ __forceinline__ int slot(int row, int piece) {
-  return row * PIECES + (piece ^ ((row / (16 / PIECES)) & (PIECES - 1)));
-}
+// floats from one split's sums to the next: whole 16-byte pieces
+__host__ __device__ __forceinline__ size_t split_step(int m, int n) { return ((size_t)m * n + 3) & ~(size_t)3; }
 
-// TM x TN tiles of 32 x 32 per wavefront, WM x WN wavefronts, BK channels per stage.
-//
+// Which of the eight 16-byte places of its 128-byte LDS row a piece lies in: piece ^ fold(row).  A 16-byte read is
+// served sixteen lanes (all banks) at a time: sixteen rows with one piece, or with the pieces of neighbouring quarters
+// of the wavefront; either way the pairs of rows fall on eight different places.
+__device__ __forceinline__ int fold(int row) { return ((((row >> 3) ^ (row >> 2)) & 1) << 2) | (((row >> 2) & 1) << 1) | ((row >> 1) & 1); }
+
+// A workgroup's tile: WM x WN wavefronts of TM x TN tiles of 16 x 16, and WK such groups, which take the 128-channel blocks
+// in turn (two groups add their sums in LDS at the end: half the steps of a tile where the tiles leave CUs idle, without a
+// second launch).  A stage is a block per group: [group][half block][row][128 bytes] of activations, [group][row][128 bytes]
+// of weights and every wavefront's weight scales.  PERSIST: a workgroup goes on to its next tile, whose first stages are on
+// their way under the last products and the stores of the one before.
+template <int TM_, int TN_, int WM_, int WN_, int WK_, int SLOTS_, bool PERSIST_>
+struct Tile {
+  static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, WK = WK_, SLOTS = SLOTS_;
+  static constexpr bool PERSIST = PERSIST_;
+  static constexpr int kWaves = WM * WN * WK, kThreads = 64 * kWaves;
+  static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
+  static constexpr int XL = WK * 2 * BM / 8 / kWaves, WL = WK * BN / 8 / kWaves;    // load instructions per wavefront and stage
+  static_assert(XL * kWaves * 8 == WK * 2 * BM && WL * kWaves * 8 == WK * BN, "whole instructions per wavefront");
+  static constexpr int kX = WK * 2 * BM * 128, kW = WK * BN * 128, kS = kWaves * 256;
+  static constexpr int kStage = kX + kW + kS;                                        // bytes of one slot
+  static constexpr int PITCH = TN * 16 + 4;                                          // floats of a row on its way out
+  static constexpr int kOut = kWaves * 16 * PITCH * 4;
+  static constexpr int kLds = SLOTS * kStage + (PERSIST ? kOut : 0);
+  static_assert(WK == 1 || (WK == 2 && !PERSIST), "the sums of two groups meet in the stages' place");
+};
+
 // Every 128-channel block is accumulated from zero and enters the sums as acc += scale * tile, so fp32
 // scales of any kind are applied exactly; in the product layout (weights as the second operand) a lane
 // holds one output channel, i.e. one scale per tile.  A lane's 16 weight bytes feed two products: the
 // contraction runs over the channels in the order the bytes lie in, and the activation pieces follow it.
-template <int TM, int TN, int WM, int WN, int BK, bool F16>
-__global__ __launch_bounds__(64 * WM * WN, 2) void fp8_gemm_kernel(const VecmatParams p) {
-  constexpr int kGemmThreads = 64 * WM * WN;
-  constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
-  constexpr int XP = BK / 8, WP = BK / 16;               // 16-byte pieces per row of the two tiles
-  constexpr int XL = BM * XP / kGemmThreads, WL = BN * WP / kGemmThreads;
-  static_assert(XL * kGemmThreads == BM * XP && WL * kGemmThreads == BN * WP, "whole pieces per thread");
-  constexpr int STEPS = 128 / BK;
-  constexpr int PITCH = TN * 32 + 4;                     // of the rows on their way out
-  constexpr int TILES = 2 * (BM * XP + BN * WP), ROWS = WM * WN * 32 * PITCH / 4;
-  __shared__ u32x4 smem[TILES > ROWS ? TILES : ROWS];
-  u32x4* const xs = smem;                                // [2][BM * XP]
-  u32x4* const ws = smem + 2 * BM * XP;                  // [2][BN * WP]
+template <class T, bool F16>
+__global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatParams p) {
+  constexpr int TM = T::TM, TN = T::TN, WM = T::WM, WN = T::WN, WK = T::WK, SLOTS = T::SLOTS, BM = T::BM, BN = T::BN, XL = T::XL, WL = T::WL;
+  constexpr int PITCH = T::PITCH, L = XL + WL + 1;
+  __shared__ u32x4 smem[T::kLds / 16];
+  char* const lds = reinterpret_cast<char*>(smem);
 
-  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave / WN) * TM * 32, wn = (wave % WN) * TN * 32;
-  const int half = lane >> 5, l32 = lane & 31;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wk = wave / (WM * WN), wm = (wave / WN % WM) * TM * 16, wn = (wave % WN) * TN * 16;
+  const int quad = lane >> 4, l16 = lane & 15;
 
-  // Tile of this workgroup.  Consecutive workgroups go round the eight XCDs: every XCD takes one run of
-  // the order (groups of eight column tiles; inside, row tile by row tile), so that its L2 holds the
-  // weights of a group while the row tiles pass.
   const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
   const int total = tiles_m * tiles_n;
-  const int q = total >> 3, r = total & 7, xcd = (int)blockIdx.x & 7;
-  const int t = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + ((int)blockIdx.x >> 3);
-  const int per_group = tiles_m * 8, group = t / per_group;
-  const int width = tiles_n - group * 8 < 8 ? tiles_n - group * 8 : 8;
-  const int in_group = t - group * per_group;
-  const int m0 = (in_group / width) * BM, n0 = (group * 8 + in_group % width) * BN;
-
   const int blocks = p.k / 128;
   const int b0 = (int)((long long)blocks * blockIdx.y / p.k_splits), b1 = (int)((long long)blocks * (blockIdx.y + 1) / p.k_splits);
+  const int stages = (b1 - b0 + WK - 1) / WK;
 
-  // one uniform base per operand, moved on by a stage at a time, and 32-bit lane offsets
-  const char* xbase = reinterpret_cast<const char*>(p.x) + ((size_t)m0 * p.k + (size_t)b0 * 128) * 2;
-  const char* wbase = reinterpret_cast<const char*>(p.w) + (size_t)n0 * p.k + (size_t)b0 * 128;
-  unsigned xoff[XL], woff[WL];
-  int xslot[XL], wslot[WL];
-#pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    const int e = tid + i * kGemmThreads, row = e / XP, piece = e % XP;
-    const int m = m0 + row < p.m ? row : p.m - 1 - m0;       // rows past the end repeat the last one and are not stored
-    xoff[i] = (unsigned)m * (unsigned)p.k * 2u + (unsigned)piece * 16u;
-    xslot[i] = slot<XP>(row, piece);
-  }
-#pragma unroll
-  for (int i = 0; i < WL; ++i) {
-    const int e = tid + i * kGemmThreads, row = e / WP, piece = e % WP;
-    const int n = n0 + row < p.n ? row : p.n - 1 - n0;
-    woff[i] = (unsigned)n * (unsigned)p.k + (unsigned)piece * 16u;
-    wslot[i] = slot<WP>(row, piece);
-  }
-  const float* sg[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = n0 + wn + j * 32 + l32 < p.n ? n0 + wn + j * 32 + l32 : p.n - 1;
-    sg[j] = p.scale_w + (size_t)(n >> p.srow_shift) * p.srow_stride;
-  }
+  // Rows and columns of tile e.  Consecutive workgroups go round the eight XCDs: every XCD takes one run of
+  // the order (groups of eight column tiles; inside, row tile by row tile), so that its L2 holds the
+  // weights of a group while the row tiles pass.  (The number of workgroups that take several tiles is a multiple of 8.)
+  auto place = [&](int e, int& m0, int& n0) {
+    const int q = total >> 3, r = total & 7, xcd = e & 7;
+    const int t = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (e >> 3);
+    const int per_group = tiles_m * 8, group = t / per_group;
+    const int width = tiles_n - group * 8 < 8 ? tiles_n - group * 8 : 8;
+    const int in_group = t - group * per_group;
+    m0 = (in_group / width) * BM;
+    n0 = (group * 8 + in_group % width) * BN;
+  };
 
-  // Two register sets, so that two stages are on their way while one computes out of LDS and one is
-  // written there.  Loads in the loop are unconditional (behind a branch the compiler waits for them at
-  // once): past the last stage they fetch it again.
-  u32x4 xr[2][XL], wr[2][WL];
-  const int stages = (b1 - b0) * STEPS;
-  int fetched = 0;
-  auto fetch = [&](int set) {
+  // ---- loads: inline assembly (the compiler would order every later LDS read behind them), waited for by count ----
+  // One uniform base per operand, moved on by a stage at a time, and 32-bit lane offsets.  An instruction moves eight rows
+  // of 128 bytes.
+  const char *xbase, *wbase, *sbase;
+  unsigned xoff[XL], woff[WL], soff;
+  int next_e = (int)blockIdx.x, next_b = b0, left;                   // tile and block to be requested next; stages not requested
+  auto start = [&]() {
+    int m0, n0;
+    place(next_e, m0, n0);
+    xbase = reinterpret_cast<const char*>(p.x) + ((size_t)m0 * p.k + (size_t)b0 * 128) * 2;
+    wbase = reinterpret_cast<const char*>(p.w) + (size_t)n0 * p.k + (size_t)b0 * 128;
+    const int first = n0 >> p.srow_shift;
+    sbase = reinterpret_cast<const char*>(p.scale_w) + ((size_t)first * p.srow_stride + (size_t)b0 * p.scol_stride) * 4;
+    next_b = b0;
 #pragma unroll
-    for (int i = 0; i < XL; ++i) xr[set][i] = *reinterpret_cast<const u32x4*>(xbase + xoff[i]);
+    for (int i = 0; i < XL; ++i) {
+      const int u = wave * XL + i, plane = u & 1, rg = (u >> 1) / WK;
+      const int row = rg * 8 + (lane >> 3), m = m0 + row < p.m ? row : p.m - 1 - m0;       // rows past the end repeat the last one and are not stored
+      xoff[i] = (unsigned)m * (unsigned)p.k * 2u + (unsigned)plane * 128u + 16u * (unsigned)((lane & 7) ^ fold(row));
+    }
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
-      // one row tile: the weights pass once and need not stay in the caches
-      const u32x4* src = reinterpret_cast<const u32x4*>(wbase + woff[i]);
-      wr[set][i] = WM == 1 ? __builtin_nontemporal_load(src) : *src;
+      const int u = wave * WL + i, rg = u / WK;
+      const int row = rg * 8 + (lane >> 3), n = n0 + row < p.n ? row : p.n - 1 - n0;
+      woff[i] = (unsigned)n * (unsigned)p.k + 16u * (unsigned)((lane & 7) ^ fold(row));
     }
-    const bool more = ++fetched < stages;
-    xbase += more ? BK * 2 : 0;
-    wbase += more ? BK : 0;
+    const int c = n0 + wn + lane % (TN * 16), n = c < p.n ? c : p.n - 1;
+    soff = (unsigned)((n >> p.srow_shift) - first) * (unsigned)p.srow_stride * 4u;
   };
-  auto stage = [&](int set, int buf) {
-#pragma unroll
-    for (int i = 0; i < XL; ++i) xs[buf * BM * XP + xslot[i]] = xr[set][i];
-#pragma unroll
-    for (int i = 0; i < WL; ++i) ws[buf * BN * WP + wslot[i]] = wr[set][i];
+  const unsigned lds_base = (unsigned)(size_t)(lds_void*)smem;
+  auto load16 = [&](const char* base, unsigned off, unsigned to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory", "m0");
+  };
+  auto load4 = [&](const char* base, unsigned off, unsigned to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory", "m0");
+  };
+  unsigned next_slot = lds_base;
+  // requests instruction i of the next stage (of the same number whatever the stage holds: a block that is not there
+  // repeats its neighbour)
+  auto issue = [&](int i) {
+    const bool pair = WK == 1 || next_b + 1 < b1;
+    if (i < WL) {
+      const int u = wave * WL + i, g = u % WK, rg = u / WK;
+      load16(wbase + (pair ? g * 128 : 0), woff[i], next_slot + (unsigned)(T::kX + (g * BN + rg * 8) * 128));
+    } else if (i < XL + WL) {
+      const int u = wave * XL + i - WL, plane = u & 1, g = (u >> 1) % WK, rg = (u >> 1) / WK;
+      load16(xbase + (pair ? g * 256 : 0), xoff[i - WL], next_slot + (unsigned)(((g * 2 + plane) * BM + rg * 8) * 128));
+    } else {
+      load4(sbase + (pair ? (size_t)wk * p.scol_stride * 4 : 0), soff, next_slot + (unsigned)(T::kX + T::kW + wave * 256));
+      xbase += WK * 256;
+      wbase += WK * 128;
+      sbase += (size_t)WK * p.scol_stride * 4;
+      next_b += WK;
+      --left;
+      next_slot = next_slot + T::kStage == lds_base + SLOTS * T::kStage ? lds_base : next_slot + T::kStage;
+      if (T::PERSIST && next_b >= b1 && left > 0) {
+        next_e += (int)gridDim.x;
+        start();
+      }
+    }
   };
 
-  f32x16 acc[TM][TN];
+  f32x4 acc[TM][TN], tile[TM][TN];
+  const int xlane = (wk * 2 * BM + wm + l16) * 128, wlane = T::kX + (wk * BN + wn + l16) * 128, slane = T::kX + T::kW + wave * 256 + l16 * 4;
+  const int f = fold(l16);
+  const int xpos[2] = {xlane + 16 * ((quad * 2) ^ f), xlane + 16 * ((quad * 2 + 1) ^ f)};
+  const int wpos[2] = {wlane + 16 * (quad ^ f), wlane + 16 * ((4 + quad) ^ f)};
+  u32x4 wr[2][TN], xr[2][TM];
+  float sc[TN];
+  auto read_w = [&](int slot, int c) {
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+    for (int j = 0; j < TN; ++j) wr[c][j] = *reinterpret_cast<const u32x4*>(lds + slot + wpos[c] + j * 2048);
+  };
+  auto read_x = [&](int slot, int c, int h) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int i = 0; i < TM; ++i) xr[h][i] = *reinterpret_cast<const u32x4*>(lds + slot + xpos[h] + c * BM * 128 + i * 2048);
+  };
+  // products of channels 64 c + 16 quad + 8 h .. of the block; loads of the stage after next go between their columns
+  // (all at once, a wavefront stood still until the load unit's queue had room: 1 to 2 % of a large product)
+  auto multiply = [&](int c, int h, bool loads) {
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+    for (int j = 0; j < TN; ++j) {
+      const u32x4 wv = h == 0 ? codes8<F16>(wr[c][j][0], wr[c][j][1]) : codes8<F16>(wr[c][j][2], wr[c][j][3]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) tile[i][j] = product<F16>(xr[h][i], wv, c == 0 && h == 0 ? zero : tile[i][j]);
+      if (loads) {
+#pragma unroll
+        for (int i = L * j / TN; i < L * (j + 1) / TN; ++i) issue(i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
 
-  // operands of one 32-channel step
-  struct Operands { u32x4 w[TN], x[TM][2]; };
-  auto read = [&](int buf, int kk, Operands& o) {
+  const int mine = T::PERSIST ? (total - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x : 1;
+  left = mine * stages;
+  start();
 #pragma unroll
-    for (int j = 0; j < TN; ++j) o.w[j] = ws[buf * BN * WP + slot<WP>(wn + j * 32 + l32, kk * 2 + half)];
+  for (int s = 0; s < SLOTS; ++s)
+    if (left > 0) {
+#pragma unroll
+      for (int i = 0; i < L; ++i) issue(i);
+    }
+  if (mine * stages >= SLOTS) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((SLOTS - 1) * L) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  // Operands are read half a block of products ahead.  The barrier stands in front of a stage's last products: behind it
+  // the next stage's first operands are read under them, and the place of this one may be filled again.
+  int slot = 0;
+  read_w(0, 0);
+  read_x(0, 0, 0);
+  int todo = mine * stages;                              // stages not multiplied
+  for (int e = (int)blockIdx.x; ; e += (int)gridDim.x) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) o.x[i][h] = xs[buf * BM * XP + slot<XP>(wm + i * 32 + l32, kk * 4 + half * 2 + h)];
-  };
-  Operands ops[2];
-  // One stage out of LDS buffer `buf`, operands read a step ahead.  The barrier stands in front of the
-  // stage's last products: behind it the next stage's first operands can be read under them.  (The other
-  // buffer was last read in front of the previous stage's barrier.)
-  auto step = [&](int buf, f32x16 (&tile)[TM][TN]) {
-    constexpr int KK = BK / 32;
+      for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s = 0; s < stages; ++s) {
+      const int next = slot + T::kStage == SLOTS * T::kStage ? 0 : slot + T::kStage;
+      read_x(slot, 0, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0, 0, false);
+      __builtin_amdgcn_sched_barrier(0);
+      read_w(slot, 1);
+      read_x(slot, 1, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0, 1, false);
+      __builtin_amdgcn_sched_barrier(0);
+      read_x(slot, 1, 1);
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      if (kk == KK - 1) {
-        __syncthreads();
-        read(buf ^ 1, 0, ops[0]);
-      } else {
-        read(buf, kk + 1, ops[(kk + 1) & 1]);
-      }
-      if (kk == 0) {
-        stage(buf ^ 1, buf ^ 1);
-        fetch(buf ^ 1);
+      for (int j = 0; j < TN; ++j) sc[j] = *reinterpret_cast<const float*>(lds + slot + slane + j * 64);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(1, 0, false);
+      __builtin_amdgcn_sched_barrier(0);
+      const bool more = left > 0;
+      if (--todo > 0) {
+        // the next stage has arrived, and everybody has read this one
+        if (SLOTS > 2 && todo >= SLOTS - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((SLOTS - 2) * L) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        read_w(next, 0);
+        read_x(next, 0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
-      const Operands& o = ops[kk & 1];
+      multiply(1, 1, more);
+      if (WK == 1 || b0 + s * WK + wk < b1) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[i][j][v] = fmaf(sc[j], tile[i][j][v], acc[i][j][v]);
+      }
+      slot = next;
+    }
+    if (!T::PERSIST) __syncthreads();                    // the last stage is read: its place is free
+
+    constexpr int TO = TM / WK;                          // row tiles this wavefront stores
+    static_assert(TO * WK == TM, "whole row tiles");
+    if (WK == 2) {
+      f32x4* const swap = reinterpret_cast<f32x4*>(smem) + (size_t)(wave % (WM * WN)) * (2 * TO * TN * 64);
+#pragma unroll
+      for (int i = 0; i < TO; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) swap[((wk * TO + i) * TN + j) * 64 + lane] = wk == 0 ? acc[TM - TO + i][j] : acc[i][j];
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < TO; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-          const u32x4 wv = h == 0 ? codes8<F16>(o.w[j][0], o.w[j][1]) : codes8<F16>(o.w[j][2], o.w[j][3]);
-#pragma unroll
-          for (int i = 0; i < TM; ++i) tile[i][j] = product<F16>(o.x[i][h], wv, tile[i][j]);
+          const f32x4 other = swap[(((1 - wk) * TO + i) * TN + j) * 64 + lane];
+          acc[i][j] = wk == 0 ? acc[i][j] + other : other + acc[TM - TO + i][j];
         }
-      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();
     }
-  };
-  // one 128-channel block: STEPS stages from LDS buffer `buf` on
-  auto block = [&](int b, int buf) {
-    f32x16 tile[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) tile[i][j][v] = 0.0f;
-    float sc[TN];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) sc[j] = sg[j][(size_t)b * p.scol_stride];
-#pragma unroll
-    for (int s = 0; s < STEPS; ++s) step((buf + s) & 1, tile);
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = fmaf(sc[j], tile[i][j][v], acc[i][j][v]);
-  };
 
-  fetch(0);
-  stage(0, 0);
-  fetch(1);
-  fetch(0);
-  __syncthreads();
-  read(0, 0, ops[0]);
-  int b = b0;
-  if (STEPS == 1) {
-    for (; b + 2 <= b1; b += 2) {
-      block(b, 0);
-      block(b + 1, 1);
-    }
-    if (b < b1) block(b, 0);
-  } else {
-    for (; b < b1; ++b) block(b, 0);
-  }
-
-  // Register v of a tile holds row 8 * (v / 4) + 4 * half + v % 4, column l32: 32 rows at a time go
-  // through LDS, so that they leave in 16-byte stores of whole rows.
-  float* const rows = reinterpret_cast<float*>(smem) + wave * 32 * PITCH;
-  const int nw = n0 + wn;
-  auto store = [&](auto* out, auto convert) {
-    typedef decltype(convert(0.0f)) T;
-    constexpr int V = 16 / sizeof(T);
-    typedef T __attribute__((ext_vector_type(V))) vec;
-    const bool vectors = p.n % V == 0 && ((uintptr_t)out & 15) == 0;
+    // Register v of a tile holds row 4 * quad + v, column l16: 16 rows at a time go through LDS, so that they leave in
+    // 16-byte stores of whole rows.
+    int m0, n0;
+    place(e, m0, n0);
+    const int mw = m0 + wm + wk * TO * 16, nw = n0 + wn;
+    float* const rows = reinterpret_cast<float*>(lds + (T::PERSIST ? SLOTS * T::kStage : 0)) + wave * 16 * PITCH;
+    auto store = [&](auto* out, auto convert) {
+      typedef decltype(convert(0.0f)) E;
+      constexpr int V = 16 / sizeof(E);
+      typedef E __attribute__((ext_vector_type(V))) vec;
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+      for (int i = 0; i < TO; ++i) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) rows[(8 * (v >> 2) + 4 * half + (v & 3)) * PITCH + j * 32 + l32] = acc[i][j][v];
-      __builtin_amdgcn_wave_barrier();
+          for (int v = 0; v < 4; ++v) rows[(4 * quad + v) * PITCH + j * 16 + l16] = acc[i][j][v];
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int e = lane; e < 32 * TN * 32 / V; e += 64) {
-        const int row = e / (TN * 32 / V), col = e % (TN * 32 / V) * V;
-        const int m = m0 + wm + i * 32 + row;
-        if (m >= p.m) continue;
-        vec r;
+        for (int e = lane; e < 16 * TN * 16 / V; e += 64) {
+          const int row = e / (TN * 16 / V), col = e % (TN * 16 / V) * V;
+          const int m = mw + i * 16 + row;
+          if (m >= p.m) continue;
+          vec r;
 #pragma unroll
-        for (int v = 0; v < V; ++v) r[v] = convert(rows[row * PITCH + col + v]);
-        T* dst = out + (size_t)m * p.n + nw + col;
-        if (vectors) {
-          if (nw + col < p.n) *reinterpret_cast<vec*>(dst) = r;
-        } else {
+          for (int v = 0; v < V; ++v) r[v] = convert(rows[row * PITCH + col + v]);
+          E* dst = out + (size_t)m * p.n + nw + col;
+          if (nw + col + V <= p.n) {
+            __builtin_memcpy(dst, &r, 16);               // (rows of odd lengths begin anywhere; such stores one value at a time cost 1 us a call)
+          } else {
 #pragma unroll
-          for (int v = 0; v < V; ++v)
-            if (nw + col + v < p.n) dst[v] = r[v];
+            for (int v = 0; v < V; ++v)
+              if (nw + col + v < p.n) dst[v] = r[v];
+          }
         }
+        __builtin_amdgcn_wave_barrier();
       }
-      __builtin_amdgcn_wave_barrier();
-    }
-  };
-  __syncthreads();                                       // the last stage is read
-  if (p.k_splits > 1) store(p.partial + (size_t)blockIdx.y * p.m * p.n, [](float v) { return v; });
-  else if (p.out_dtype == CPPMEGA_MI355_BF16) store((unsigned short*)p.out, f32_to_bf16_bits);
-  else if (p.out_dtype == CPPMEGA_MI355_F16) store((unsigned short*)p.out, f32_to_f16_bits);
-  else store((float*)p.out, [](float v) { return v; });
+    };
+    if (p.k_splits > 1) store(p.partial + (size_t)blockIdx.y * split_step(p.m, p.n), [](float v) { return v; });
+    else if (p.out_dtype == CPPMEGA_MI355_BF16) store((unsigned short*)p.out, f32_to_bf16_bits);
+    else if (p.out_dtype == CPPMEGA_MI355_F16) store((unsigned short*)p.out, f32_to_f16_bits);
+    else store((float*)p.out, [](float v) { return v; });
+    if (!T::PERSIST || todo == 0) break;
+  }
 }
 
 // out[m][n] = sum over the K splits of partial[split][m][n], in split order.  Bound by latency (7 MB at 32 x 7168 x 8
-// splits): with the splits' loads one after the other and stores of single values a call took 2 to 3 us longer.
+// splits): with the splits' loads one after the other and stores of single values a call took 2 to 3 us longer.  Splits
+// begin at whole 16-byte pieces, so that products of odd sizes are read alike (19 x 333 of 16 splits: 12 -> 4 us).
 __global__ __launch_bounds__(256) void fp8_gemm_reduce_kernel(const VecmatParams p) {
-  const size_t total = (size_t)p.m * p.n;
+  const size_t total = (size_t)p.m * p.n, step = split_step(p.m, p.n);
   const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= total) return;
-  if ((total & 3) == 0) {
-    // (the loads of the up to 16 splits are in flight together)
-    f32x4 part[16], s = {0.0f, 0.0f, 0.0f, 0.0f};
+  // (the loads of the up to 16 splits are in flight together)
+  f32x4 part[16], s = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int z = 0; z < 16; ++z)
-      if (z < p.k_splits) part[z] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.partial + (size_t)z * total + i));
+  for (int z = 0; z < 16; ++z)
+    if (z < p.k_splits) part[z] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.partial + (size_t)z * step + i));
 #pragma unroll
-    for (int z = 0; z < 16; ++z)
-      if (z < p.k_splits) s += part[z];
-    if (p.out_dtype != CPPMEGA_MI355_F32 && ((uintptr_t)p.out & 7) == 0) {
-      const bool bf16 = p.out_dtype == CPPMEGA_MI355_BF16;
-      *reinterpret_cast<uint2*>((unsigned short*)p.out + i) = bf16 ? make_uint2(pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3]))
-                                                                   : make_uint2(pack_f16(s[0], s[1]), pack_f16(s[2], s[3]));
-    } else {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) store_as(p.out, i + v, p.out_dtype, s[v]);
-    }
+  for (int z = 0; z < 16; ++z)
+    if (z < p.k_splits) s += part[z];
+  if (i + 4 <= total && p.out_dtype != CPPMEGA_MI355_F32 && ((uintptr_t)p.out & 7) == 0) {
+    const bool bf16 = p.out_dtype == CPPMEGA_MI355_BF16;
+    *reinterpret_cast<uint2*>((unsigned short*)p.out + i) = bf16 ? make_uint2(pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3]))
+                                                                 : make_uint2(pack_f16(s[0], s[1]), pack_f16(s[2], s[3]));
   } else {
-    for (size_t e = i; e < i + 4 && e < total; ++e) {
-      float s = 0.0f;
-      for (int z = 0; z < p.k_splits; ++z) s += p.partial[(size_t)z * total + e];
-      store_as(p.out, e, p.out_dtype, s);
-    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (i + v < total) store_as(p.out, i + v, p.out_dtype, s[v]);
   }
 }
 
-// What a tile shape costs, measured on MI355X: microseconds per 128-channel block with 1, 2, .. of its
-// workgroups on a CU, and per workgroup for its first loads and its stores.
-struct TileShape {
-  int bm, bn, per_cu;
-  double block_us[3], ends_us;
+typedef Tile<2, 2, 1, 4, 2, 3, false> Tile32;            // 32 x 128, two groups, 150 KB of LDS
+typedef Tile<4, 2, 1, 4, 2, 2, false> Tile64Pair;        // 64 x 128, two groups, 132 KB
+typedef Tile<4, 2, 1, 4, 1, 2, false> Tile64;            // 64 x 128, 66 KB: two workgroups on a CU, whose ends overlap
+typedef Tile<4, 2, 1, 4, 1, 2, true> Tile64Many;         // the same, tile after tile
+typedef Tile<4, 4, 2, 4, 1, 2, false> Tile256;           // 128 x 256, 132 KB
+
+// What a tile shape costs, measured on MI355X: microseconds per stage with 1 and 2 of its workgroups on a CU, and per
+// workgroup for its first loads and its stores.
+enum Shape { kTile32, kTile64Pair, kTile64, kTile64Many, kTile256 };
+struct TileCost {
+  int bm, bn, per_cu, groups;
+  double stage_us[2], ends_us;
 };
-constexpr TileShape kShapes[] = {
-    {32, 128, 3, {0.82, 1.48, 3.23}, 6.0},
-    {64, 128, 2, {0.85, 1.77, 0.0}, 8.35},
-    {128, 256, 1, {1.77, 0.0, 0.0}, 9.3},
+constexpr TileCost kCosts[] = {
+    {32, 128, 1, 2, {1.145, 0.0}, 1.32},
+    {64, 128, 1, 2, {1.21, 0.0}, 2.72},
+    {64, 128, 2, 1, {0.92, 1.0}, 3.08},
+    {64, 128, 2, 1, {0.5, 1.09}, 0.88},
+    {128, 256, 1, 1, {1.71, 0.0}, 3.2},
 };
-constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 16};
+constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
 
-struct GemmPlan { const TileShape* shape; int splits; };
+struct GemmPlan { Shape shape; int splits; };
 
-size_t split_bytes(int splits, int m, int n) { return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0; }
+size_t split_bytes(int splits, int m, int n) { return splits > 1 ? splits * split_step(m, n) * sizeof(float) : 0; }
 
-// The tile shape and K split with the smallest estimate: rounds of workgroups over the CUs, plus, for a
-// split, one more launch and the partial sums written and read (8 bytes per sum).  Fitted to all combinations but
-// those of 9 splits at 55 shapes of 17..1000 x 512..16384 x 896..16384: the choice is 0.4 % from the best of them in the
-// mean and 7 % at most.  9 splits give 56 column tiles two workgroups on nearly every CU where 8 leave a quarter of the
-// CUs with one (32 x 7168 x 16384: 41 -> 39 us, the calls of 13 .. 16 splits that finer steps would pick are no faster).  The third workgroup on a CU brings nothing (the weights' stream is what they share).
-// Splits whose sums need more than `have` bytes are left out; one split needs none.
+// The tile shape and K split with the smallest estimate: rounds of workgroups over the CUs, no less than the weights'
+// stream takes, plus, for a split, one more launch and the partial sums written and read (8 bytes per sum).
+// Fitted at 110 shapes of 17..4000 x 256..16400 x 512..16384, both scale layouts: the choice is 0.2 % from the best of all
+// combinations there in the mean and 5 % at most.
+// Splits whose sums need more than `have` bytes are left out; one split needs none.  64 x 128 tiles that are more than
+// two to a CU are taken one after the other by as many workgroups (717 x 7411 x 1024: 23.7 -> 21.2 us, 1647 x 8297 x 1152:
+// 46.3 -> 42.8; with one tile to a workgroup the loop costs 1 to 5 %).
 GemmPlan gemm_plan(int m, int n, int k, size_t have) {
   const int blocks = k / 128, cus = device_cus();
-  GemmPlan best = {&kShapes[0], 1};
+  GemmPlan best = {kTile32, 1};
   double best_us = 1e30;
-  for (const TileShape& s : kShapes) {
-    const double tiles = (double)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn);
+  for (int shape = kTile32; shape <= kTile256; ++shape) {
+    const TileCost& c = kCosts[shape];
+    const long long tiles = (long long)((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn);
+    const bool many = tiles > 2LL * cus;
+    if ((shape == kTile64 && many) || (shape == kTile64Many && !many)) continue;
     for (int splits : kSplits) {
-      if (splits > 1 && (splits * 2 > blocks || split_bytes(splits, m, n) > have)) break;
-      const long long wgs = (long long)tiles * splits, on_cu = (wgs + cus - 1) / cus;
-      const double steps = (blocks + splits - 1) / splits;
-      const long long rounds = on_cu / s.per_cu, rest = on_cu % s.per_cu;
-      double us = (double)rounds * (steps * s.block_us[s.per_cu - 1] + s.ends_us);
-      if (rest) us += steps * s.block_us[rest - 1] + s.ends_us;
-      if (splits > 1) us += 3.3 + (double)splits * m * n * 8.0 / 5.1e6;
-      if (us < best_us) { best_us = us; best = {&s, splits}; }
+      if (splits > 1 && (splits * 2 > blocks || split_bytes(splits, m, n) > have || shape == kTile64Many)) break;
+      const long long on_cu = (tiles * splits + cus - 1) / cus, rounds = on_cu / c.per_cu, rest = on_cu % c.per_cu;
+      const int stages = ((blocks + splits - 1) / splits + c.groups - 1) / c.groups;
+      double us = (double)rounds * (stages * c.stage_us[c.per_cu - 1] + c.ends_us);
+      if (rest) us += stages * c.stage_us[0] + c.ends_us;
+      const double stream_us = (double)n * k / 5.6e6 + 2.0;
+      if (us < stream_us) us = stream_us;
+      if (splits > 1) us += 4.8 + (double)splits * m * n * 8.0 / 5.5e6;
+      if (us < best_us) { best_us = us; best = {(Shape)shape, splits}; }
     }
   }
   return best;
 }
 
-template <int TM, int TN, int WM, int WN, int BK>
-void launch_as(dim3 grid, hipStream_t stream, const VecmatParams& p) {
-  const dim3 block(64 * WM * WN);
-  if (p.x_dtype == CPPMEGA_MI355_F16) hipLaunchKernelGGL((fp8_gemm_kernel<TM, TN, WM, WN, BK, true>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((fp8_gemm_kernel<TM, TN, WM, WN, BK, false>), grid, block, 0, stream, p);
+template <class T>
+void launch_as(int m, int n, hipStream_t stream, const VecmatParams& p) {
+  unsigned tiles = (unsigned)((m + T::BM - 1) / T::BM) * (unsigned)((n + T::BN - 1) / T::BN);
+  if (T::PERSIST) {
+    const unsigned most = (unsigned)(2 * device_cus()) & ~7u;          // a multiple of the XCDs
+    if (most > 0 && tiles > most) tiles = most;
+  }
+  const dim3 grid(tiles, (unsigned)p.k_splits), block(T::kThreads);
+  if (p.x_dtype == CPPMEGA_MI355_F16) hipLaunchKernelGGL((fp8_gemm_kernel<T, true>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((fp8_gemm_kernel<T, false>), grid, block, 0, stream, p);
 }
 
 }  // namespace
@@ -363,18 +429,26 @@ bool fp8_gemm_shape(const cppmega_mi355_vecmat_args_t& a) {
 }
 
 size_t fp8_gemm_workspace_bytes(const cppmega_mi355_vecmat_args_t& a) {
-  return split_bytes(gemm_plan(a.m, a.n, a.k, SIZE_MAX).splits, a.m, a.n);
+  int splits = gemm_plan(a.m, a.n, a.k, SIZE_MAX).splits;
+  // a few small tiles ask for the room of three splits (3 MB at most) whatever the plan: workspaces that callers laid out
+  // for a range of such sizes stay as large as they were when each of them was split
+  if (splits < 3 && a.k >= 6 * 128 && (long long)((a.m + 31) / 32) * ((a.n + 127) / 128) <= device_cus() / 4) splits = 3;
+  return split_bytes(splits, a.m, a.n);
 }
 
 int fp8_gemm_launch(VecmatParams p, size_t workspace_bytes, hipStream_t stream) {
-  const GemmPlan g = gemm_plan(p.m, p.n, p.k, workspace_bytes);
+  // (the sums of splits are read in 16-byte pieces)
+  const GemmPlan g = gemm_plan(p.m, p.n, p.k, ((uintptr_t)p.partial & 15) == 0 ? workspace_bytes : 0);
   p.k_splits = g.splits;
-  const long long tiles = (long long)((p.m + g.shape->bm - 1) / g.shape->bm) * ((p.n + g.shape->bn - 1) / g.shape->bn);
+  const long long tiles = (long long)((p.m + kCosts[g.shape].bm - 1) / kCosts[g.shape].bm) * ((p.n + kCosts[g.shape].bn - 1) / kCosts[g.shape].bn);
   if (tiles > 0x7fffffffLL) return fail(CPPMEGA_MI355_ERR_SHAPE, "vecmat: M=%d N=%d has too many tiles", p.m, p.n);
-  const dim3 grid((unsigned)tiles, (unsigned)g.splits);
-  if (g.shape->bm == 32) launch_as<1, 1, 1, 4, 128>(grid, stream, p);
-  else if (g.shape->bm == 64) launch_as<2, 1, 1, 4, 128>(grid, stream, p);
-  else launch_as<2, 2, 2, 4, 64>(grid, stream, p);
+  switch (g.shape) {
+    case kTile32: launch_as<Tile32>(p.m, p.n, stream, p); break;
+    case kTile64Pair: launch_as<Tile64Pair>(p.m, p.n, stream, p); break;
+    case kTile64: launch_as<Tile64>(p.m, p.n, stream, p); break;
+    case kTile64Many: launch_as<Tile64Many>(p.m, p.n, stream, p); break;
+    case kTile256: launch_as<Tile256>(p.m, p.n, stream, p); break;
+  }
   CM_HIP_CHECK(hipGetLastError());
   if (g.splits > 1) {
     const size_t quads = ((size_t)p.m * p.n + 3) / 4;

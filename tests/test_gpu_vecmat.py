@@ -215,6 +215,29 @@ def test_tiled_gemm_edges(device, M, N, K, dtype):
         assert err <= tol, err
 
 
+# one or two per tile shape: two groups of 32 or 64 rows with an odd number of blocks, two tiles of 64 to a CU with K splits of
+# unequal lengths, more tiles than workgroups, 128 x 256 with and without a rest; rows that begin at odd addresses
+@pytest.mark.parametrize("M,N,K", [(45, 947, 1152), (333, 2061, 640), (135, 8687, 640), (300, 1695, 896), (258, 7987, 640),
+                                   (1000, 707, 8320), (1425, 3333, 128), (2787, 3331, 512), (3427, 1995, 1408), (512, 14279, 1408)])
+def test_tiled_gemm_tile_shapes(device, M, N, K):
+    gen = torch.Generator(device="cpu").manual_seed(M + N + K)
+    dtype = torch.bfloat16 if M % 2 else torch.float16
+    x = torch.randn((M, K), generator=gen).to(dtype)
+    codes = torch.randn((N, K), generator=gen).mul(2).to(torch.float8_e4m3fn)
+    scale = torch.rand(((N + 127) // 128, K // 128), generator=gen) + 0.5
+    rows = torch.cat([torch.arange(0, M, 61), torch.arange(max(0, M - 70), M)])
+    want = x[rows].double() @ (codes.double() * scale.double().repeat_interleave(128, dim=0)[:N].repeat_interleave(128, dim=1)).T
+    got = fused_fp8_gemm(codes.view(torch.uint8).to(device), scale.to(device), x.to(device))
+    err = (got.cpu()[rows].double() - want).abs().max() / want.abs().max()
+    assert err <= 5e-3, err                              # a result rounded to 8 bits of mantissa, at most the largest itself
+    out = torch.full((M * N + 1,), 7.0, dtype=torch.float32, device=device)
+    vm.fp8_scaled_vecmat_path_c(x.to(device), codes.view(torch.uint8).to(device), scale_x=None,
+                                scale_w=scale.repeat_interleave(128, dim=0)[:N].contiguous().to(device), out=out[1:].view(M, N))
+    assert out[0] == 7.0
+    # float32 sums of K products in blocks of 128: 2e-6 of the largest, as for the other tiles
+    assert (out[1:].view(M, N).cpu()[rows].double() - want).abs().max() <= 2e-6 * want.abs().max()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,N,K", [(17, 257, 1152), (32, 1024, 2048), (100, 300, 4096)])
 def test_tiled_gemm_with_less_workspace_than_asked_for(device, M, N, K, dtype):
