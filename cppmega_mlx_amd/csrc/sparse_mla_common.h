@@ -29,7 +29,8 @@ struct MlaParams {
   int heads_per_wg;     // 0: 32-head tile kernel; 32 or 64: a producer/consumer kernel (sparse_mla_latent.hip, sparse_mla_rows16.hip)
   int plan_level;       // how the launch is planned: see sparse_mla_mfma_plan_within
   int rows16;           // with heads_per_wg: the kernel for 16-bit rows
-  int few;              // with heads_per_wg: the kernel for up to 16 heads per group (sparse_mla_few.hip)
+  int few;              // with heads_per_wg: the kernel of workgroups of 16 heads (sparse_mla_few.hip)
+  int no_few;           // the scratch does not hold that kernel's plan: plans without it
   int tile_sharing;     // tile kernel on 16-bit rows: the 4 wavefronts take 4 head groups over one key stream
   float sm_scale;
   const float* sm_scale_dev;     // device copy of the softmax scale; read in place of sm_scale when set
@@ -65,7 +66,7 @@ bool sparse_mla_mfma_supported(const MlaParams& p);
 size_t sparse_mla_mfma_workspace_bytes(const MlaParams& p);
 void sparse_mla_mfma_plan(MlaParams& p);
 // The plan for a caller who brings `have` bytes of workspace, and what it needs: the fastest one (level 0, what the
-// size query answers) if that fits, else key splits only until 256 workgroups are there and no copy of the cache
+// size query answers) if that fits (first with, then without the kernel of 16 heads where there are more), else key splits only until 256 workgroups are there and no copy of the cache
 // (level 1), else the kernel of sparse_mla_mfma.hip where it serves the shape (level 2).
 size_t sparse_mla_mfma_plan_within(MlaParams& p, size_t have);
 
@@ -79,15 +80,20 @@ int sparse_mla_combine_f32(const MlaParams& p, hipStream_t stream);    // merges
 // heads per workgroup, written and read.
 // `narrow`: the sums are bfloat16, so there are no more splits than doubling until 256 workgroups are there makes.
 // At plan level 1: the doubled number.
-void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, int heads, bool narrow);
+// Returns the modelled microseconds (level 0).
+double mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, int heads, bool narrow);
 
 // producer/consumer kernel for 16-bit rows (sparse_mla_rows16.hip); dispatched by the *_mfma_* functions
 bool sparse_mla_rows16_supported(const MlaParams& p);
-void sparse_mla_rows16_plan(MlaParams& p);
+double sparse_mla_rows16_plan(MlaParams& p);             // modelled microseconds
+// E8M0 rows: room for a bfloat16 copy of the queries and of every cache row (0: not such rows), and the launch that writes it to the
+// workspace and makes p the same call on 16-bit rows, with the workspace behind the copy
+size_t sparse_mla_e8m0_copy_bytes(const MlaParams& p);
+int sparse_mla_e8m0_copy(MlaParams& p, hipStream_t stream);
 int sparse_mla_rows16_launch(const MlaParams& p, hipStream_t stream);   // includes its combine step
 size_t sparse_mla_rows16_workspace_bytes(const MlaParams& p);
 
-// kernel for up to 16 heads per KV group (sparse_mla_few.hip); dispatched by the *_mfma_* functions
+// kernel of workgroups of 16 heads (sparse_mla_few.hip); dispatched by the *_mfma_* functions
 bool sparse_mla_few_supported(const MlaParams& p);
 void sparse_mla_few_plan(MlaParams& p);
 int sparse_mla_few_launch(const MlaParams& p, hipStream_t stream);     // includes its combine step
@@ -96,7 +102,7 @@ size_t sparse_mla_few_workspace_bytes(const MlaParams& p);
 // shared-tile kernel for FP8 latent caches (sparse_mla_latent.hip); dispatched by the *_mfma_* functions
 bool sparse_mla_latent_supported(const MlaParams& p);
 bool sparse_mla_latent_only(const MlaParams& p);         // no other kernel has served these shapes
-void sparse_mla_latent_plan(MlaParams& p);
+double sparse_mla_latent_plan(MlaParams& p);             // modelled microseconds
 int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream);   // includes its combine step
 size_t sparse_mla_latent_workspace_bytes(const MlaParams& p);
 

@@ -1,8 +1,9 @@
-// Sparse MLA forward for up to 16 heads per KV group on the matrix cores (gfx950), d_v = 512.
+// Sparse MLA forward by chunks of 16 heads on the matrix cores (gfx950), d_v = 512: KV groups of up to 16 heads, and few queries of more.
 //
 // Rows served: bf16 or float16 queries of 576 = 512 latent + 64 rope channels over key rows of the same type (packed, or a
 // latent and a rope part); bf16 queries over e4m3 latent rows with fp32 scales (per 128 / 256 / 512 channels, per row, or
-// none) and a bf16 rope tail; queries and key rows of 576 e4m3 codes with one fp32 scale each.
+// none) and a bf16 rope tail; queries and key rows of 576 e4m3 codes with one fp32 scale each, or with E8M0 bytes per 32
+// channels, over a bf16 copy in the workspace.
 //
 // The producer/consumer kernels (sparse_mla_latent.hip, sparse_mla_rows16.hip) share a tile of keys among 64 or 32 heads;
 // with 16 most of their products are for heads that are not there, and a tile still takes 0.85 .. 1.25 us.  Here a
@@ -69,14 +70,22 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sparse_mla_few_kernel(const Ml
   unsigned char* const tile = smem + wave * kTileBytes<KIND>;
   float* const stats = reinterpret_cast<float*>(smem + kSmem<KIND> - kWaves * 16 * 2 * 4);      // [wave][16 heads][max, sum]
 
-  // which (query, KV group, split); several queries per sequence: the last ones, with the longest causal lists, first
-  const unsigned id = p.S > 1 ? gridDim.x - 1u - blockIdx.x : blockIdx.x;
-  const unsigned qg = id / (unsigned)p.num_splits;
-  const int split = (int)(id - qg * (unsigned)p.num_splits);
+  // which (query, KV group, split, 16 heads of the group); several queries per sequence: the last ones, with the longest causal
+  // lists, first
+  const unsigned chunks = (unsigned)(p.heads_per_group + 15) / 16u;
+  unsigned id = p.S > 1 ? gridDim.x - 1u - blockIdx.x : blockIdx.x;
+  if (chunks > 1) {                                       // the workgroups of one list in one XCD (launches go round the eight): each takes a run of them
+    const unsigned q = gridDim.x >> 3, r = gridDim.x & 7, xcd = blockIdx.x & 7;
+    id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (blockIdx.x >> 3);
+  }
+  const unsigned unit = id / chunks;
+  const int chunk = (int)(id - unit * chunks);
+  const unsigned qg = unit / (unsigned)p.num_splits;
+  const int split = (int)(unit - qg * (unsigned)p.num_splits);
   const unsigned bs32 = qg / (unsigned)p.G;
   const int g = (int)(qg - bs32 * (unsigned)p.G), b = (int)(bs32 / (unsigned)p.S);
   const size_t bs = bs32;
-  const int head0 = g * p.heads_per_group, heads_here = p.heads_per_group;
+  const int head0 = g * p.heads_per_group + 16 * chunk, heads_here = min(16, p.heads_per_group - 16 * chunk);
   const size_t idx_base = (bs * p.G + g) * (size_t)p.topk;
   const int key_begin = split * p.keys_per_split, key_end = min(p.topk, key_begin + p.keys_per_split);
   const int n_tiles = max(0, (key_end - key_begin + kTK - 1) / kTK);
@@ -395,7 +404,10 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sparse_mla_few_kernel(const Ml
       out_scale = 0.0f;
     }
   }
-  const size_t part_block = (size_t)qg * p.num_splits + split, part_blocks = (size_t)p.B * p.S * p.G * p.num_splits;
+  // (a partial block holds 32 heads, two workgroups')
+  const unsigned blocks32 = (chunks + 1) / 2;
+  const size_t part_block = ((size_t)qg * blocks32 + chunk / 2) * p.num_splits + split, part_blocks = (size_t)p.B * p.S * p.G * blocks32 * p.num_splits;
+  const int part_head = 16 * (chunk & 1) + n;
   // this wavefront finishes blocks 8 wave .. 8 wave + 7 (128 channels)
   f32x4 sums[8];
 #pragma unroll
@@ -408,7 +420,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sparse_mla_few_kernel(const Ml
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int dvb = i >> 1, j = 2 * (i & 1) + (kg >> 1), half = kg & 1;
-      float* blk = (float*)p.workspace + part_block * (size_t)kMlaPartFloats + ((size_t)(wave * 8) * 64 + half * 32 + n) * 8;
+      float* blk = (float*)p.workspace + part_block * (size_t)kMlaPartFloats + ((size_t)(wave * 8) * 64 + half * 32 + part_head) * 8;
       *reinterpret_cast<f32x4*>(blk + (size_t)(dvb * 2 + (j >> 1)) * 512 + (j & 1) * 4) = sums[i];
     }
   } else if (n < heads_here) {
@@ -433,7 +445,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sparse_mla_few_kernel(const Ml
   }
   if (wave == 0 && lane < 16) {
     if (!direct) {
-      float* ml = (float*)p.workspace + part_blocks * (size_t)kMlaPartFloats + (part_block * 32 + n) * 2;
+      float* ml = (float*)p.workspace + part_blocks * (size_t)kMlaPartFloats + (part_block * 32 + part_head) * 2;
       ml[0] = m_all;
       ml[1] = l_all;
     } else if (n < heads_here && p.lse) {
@@ -446,49 +458,83 @@ template <int KIND, int NBLK, bool F16>
 int launch_as(const MlaParams& p, hipStream_t stream) {
   void (*kernel)(MlaParams) = sparse_mla_few_kernel<KIND, NBLK, F16>;
   CM_HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kSmem<KIND>));
-  hipLaunchKernelGGL(kernel, dim3((unsigned)((size_t)p.B * p.S * p.G * p.num_splits)), dim3(kWaves * 64), kSmem<KIND>, stream, p);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((size_t)p.B * p.S * p.G * ((p.heads_per_group + 15) / 16) * p.num_splits)), dim3(kWaves * 64), kSmem<KIND>, stream, p);
   CM_HIP_CHECK(hipGetLastError());
   return p.num_splits > 1 ? sparse_mla_combine_f32(p, stream) : 0;
 }
 
 }  // namespace
 
+namespace {
+// The number of splits with the least modelled time: rounds of 256 workgroups, each with its start and end and the
+// tiles that one of its four wavefronts has, then the merging kernel and its traffic.  Fitted to 147 shapes (three kinds
+// of rows, 1 .. 300 queries, 128 .. 2048 keys, up to 16 splits): 0.5 % from the best number in the mean, 8 % at most.
+// `units`: queries, KV groups and chunks of 16 heads.
+double few_splits(long long units, int topk, int* splits, int* keys_per_split) {
+  const int tiles = (topk + kTK - 1) / kTK;
+  double best = 0.0;
+  *splits = 0;
+  for (int s = 1; s <= 16; ++s) {
+    const int per = (tiles + s - 1) / s, used = (tiles + per - 1) / per;
+    double us = (double)((units * used + 255) / 256) * (4.0 + 2.1 * ((per + kWaves - 1) / kWaves));
+    if (used > 1) us += 2.0 + 0.2 * used + (double)units * used * kMlaPartFloats * 4 / 4e6;
+    if (*splits == 0 || us < best) {
+      best = us;
+      *splits = used;
+      *keys_per_split = per * kTK;
+    }
+  }
+  return best;
+}
+long long units_of(const MlaParams& p) { return (long long)p.B * p.S * p.G * ((p.heads_per_group + 15) / 16); }
+}  // namespace
+
 bool sparse_mla_few_supported(const MlaParams& p) {
-  if (p.heads_per_group > 16 || p.d_qk != kDqk || p.d_v != kLat) return false;
-  const long long units = (long long)p.B * p.S * p.G;
+  if (p.d_qk != kDqk || p.d_v != kLat) return false;
+  const long long units = units_of(p);
   if (units * 16 > 0x7fffffffll) return false;
+  const bool of_16_bits = sparse_mla_rows16_supported(p);
+  if (of_16_bits && sparse_mla_e8m0_copy_bytes(p) > ((size_t)1 << 30)) return false;
+  if (p.heads_per_group > 16) {
+    // More heads: few queries leave CUs idle where 64 heads share a workgroup, chunks of 16 fill them (4 queries x 128 heads, before /
+    // here: 128 keys of 16-bit rows 12.4 / 10.2 us, 512 19.2 / 15.3, 2048 26.8 / 20.2, codes 26.5 / 20.0, E8M0 rows 32.2 / 27.0; 64 queries x
+    // 64 heads x 512 25.1 / 18.4).  A unit takes about 1.4 times what its model says beside that of the other kernel, 1.5 over the
+    // copy of E8M0 rows, whose queries cost 0.35 ns a row: of 354 shapes (64 and 128 heads, 1 .. 500 queries, 64 .. 2048 keys, three kinds of rows) those that
+    // pass gain 1.17 x in the mean and none loses; one round more of workgroups (96 queries x 128 heads x 512 26.9 / 51.0) and long lists
+    // of 24 queries on (24 x 64 x 2048 26.9 / 32.1) stay where they were.  Latent rows: no gain at 1 or 2 queries, slower from 4 on.
+    if (p.no_few || (!of_16_bits && p.q_dtype != CPPMEGA_MI355_E4M3)) return false;
+    int splits, keys;
+    MlaParams other = p;
+    double other_us;
+    if (of_16_bits) other_us = sparse_mla_rows16_plan(other);
+    else if (sparse_mla_latent_supported(p)) other_us = sparse_mla_latent_plan(other);
+    else return false;
+    const bool copied = of_16_bits && p.q_dtype == CPPMEGA_MI355_E4M3;
+    return (copied ? 1.5 : 1.4) * few_splits(units, p.topk, &splits, &keys) + (copied ? 0.35e-3 * p.B * p.S * p.H : 0.0) < other_us;
+  }
   // 8-bit rows: at 64 keys as fast as the kernel for 64 heads (9.3 / 9.1 us latent, 7.9 / 8.2 codes, one query), from there on
   // faster.  16-bit rows: a wavefront's tile takes 2.1 us from first to last, so short lists and few queries
   // are better off with four wavefronts at one tile (32 x 320: 13.2 us there, 14.3 here; 4 x 2048: 15.9 / 16.1; 32 x 512: 15.2 / 14.9;
-  // 8 x 2048: 17.6 / 16.8; 100 x 800: 26.1 / 23.2).
-  if (sparse_mla_rows16_supported(p)) return p.q_dtype != CPPMEGA_MI355_E4M3 && p.topk >= 512 && units * p.topk >= 16384;
+  // 8 x 2048: 17.6 / 16.8; 100 x 800: 26.1 / 23.2).  E8M0 rows, whose queries are copied too: 13 x 2048 25.5 / 22.4, 500 x 1100 70.5 / 64.5,
+  // 118 x 1100 33.7 / 33.7, 903 x 1161 88.8 / 91.7, 500 x 728 38.1 / 43.2.
+  if (of_16_bits && p.q_dtype == CPPMEGA_MI355_E4M3) return !p.no_few && p.topk >= 1280 && units * p.topk >= 16384;
+  if (of_16_bits) return p.topk >= 512 && units * p.topk >= 16384;
   return sparse_mla_latent_supported(p);
 }
 
 void sparse_mla_few_plan(MlaParams& p) {
   p.few = 1;
   p.heads_per_wg = 32;                                    // (what the merging kernel takes a partial block for)
-  // The number of splits with the least modelled time: rounds of 256 workgroups, each with its start and end and the
-  // tiles that one of its four wavefronts has, then the merging kernel and its traffic.  Fitted to 147 shapes (three kinds
-  // of rows, 1 .. 300 queries, 128 .. 2048 keys, up to 16 splits): 0.5 % from the best number in the mean, 8 % at most.
-  const int tiles = (p.topk + kTK - 1) / kTK;
-  const long long units = (long long)p.B * p.S * p.G;
-  double best = 0.0;
-  p.num_splits = 0;
-  for (int s = 1; s <= 16; ++s) {
-    const int per = (tiles + s - 1) / s, used = (tiles + per - 1) / per;
-    double us = (double)((units * used + 255) / 256) * (4.0 + 2.1 * ((per + kWaves - 1) / kWaves));
-    if (used > 1) us += 2.0 + 0.2 * used + (double)units * used * kMlaPartFloats * 4 / 4e6;
-    if (p.num_splits == 0 || us < best) {
-      best = us;
-      p.num_splits = used;
-      p.keys_per_split = per * kTK;
-    }
-  }
+  few_splits(units_of(p), p.topk, &p.num_splits, &p.keys_per_split);
 }
 
 int sparse_mla_few_launch(const MlaParams& p, hipStream_t stream) {
   if (p.num_splits > 16) return fail(CPPMEGA_MI355_ERR_UNSUPPORTED, "sparse MLA: launch too large");
+  if (sparse_mla_e8m0_copy_bytes(p)) {                      // queries and rows as the bfloat16 values they stand for
+    MlaParams copy = p;
+    const int rc = sparse_mla_e8m0_copy(copy, stream);
+    return rc ? rc : launch_as<kRows16, 0, false>(copy, stream);
+  }
   if (p.kv_dtype != CPPMEGA_MI355_E4M3)
     return p.q_dtype == CPPMEGA_MI355_F16 ? launch_as<kRows16, 0, true>(p, stream) : launch_as<kRows16, 0, false>(p, stream);
   if (p.q_dtype == CPPMEGA_MI355_E4M3) return launch_as<kCodes, 1, false>(p, stream);
@@ -498,10 +544,11 @@ int sparse_mla_few_launch(const MlaParams& p, hipStream_t stream) {
 }
 
 size_t sparse_mla_few_workspace_bytes(const MlaParams& p) {
-  if (p.num_splits <= 1) return 0;
-  // (8-bit rows: as much per split as the kernel for 64 heads asks for, so that scratch for the one serves the other)
-  const size_t blocks = p.kv_dtype == CPPMEGA_MI355_E4M3 ? 2 : 1;
-  return (size_t)p.B * p.S * p.G * p.num_splits * blocks * (size_t)(kMlaPartFloats + 32 * 2) * sizeof(float);
+  const size_t copy = sparse_mla_e8m0_copy_bytes(p);
+  if (p.num_splits <= 1) return copy;
+  // (8-bit rows of up to 16 heads: as much per split as the kernel for 64 heads asks for, so that scratch for the one serves the other)
+  const size_t blocks = p.heads_per_group > 16 ? (p.heads_per_group + 31) / 32 : p.kv_dtype == CPPMEGA_MI355_E4M3 && !copy ? 2 : 1;
+  return copy + (size_t)p.B * p.S * p.G * p.num_splits * blocks * (size_t)(kMlaPartFloats + 32 * 2) * sizeof(float);
 }
 
 }  // namespace cm

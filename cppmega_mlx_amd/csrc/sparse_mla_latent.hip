@@ -1036,7 +1036,7 @@ bool sparse_mla_latent_supported(const MlaParams& p) {
 
 bool sparse_mla_latent_only(const MlaParams& p) { return latent_rows(p) && p.heads_per_group > 32; }
 
-void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, int heads, bool narrow) {
+double mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, int heads, bool narrow) {
   // float32 sums: fitted to 216 shapes of 16 and 128 heads, 1 .. 300 queries, 64 .. 2048 keys (1.2x in the mean against
   // doubling the splits until 256 workgroups are there, 3x where that ended just above 256 or in splits of four tiles).
   // bfloat16 sums: to 24 shapes of 64 and 128 heads, 1 .. 64 queries, 256 .. 2048 keys (the merging kernel takes the
@@ -1051,7 +1051,7 @@ void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us,
   if (p.plan_level > 0) {
     p.num_splits = doubled;
     p.keys_per_split = (tiles + doubled - 1) / doubled * kTK;
-    return;
+    return 0.0;
   }
   double best = 0.0;
   p.num_splits = 0;
@@ -1066,12 +1066,13 @@ void mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us,
       p.keys_per_split = per * kTK;
     }
   }
+  return best;
 }
 
-void sparse_mla_latent_plan(MlaParams& p) {
+double sparse_mla_latent_plan(MlaParams& p) {
   const int chunks = (p.heads_per_group + kHeadsWg - 1) / kHeadsWg;
   p.heads_per_wg = kHeadsWg;
-  mla_key_splits(p, (long long)p.B * p.S * p.G * chunks, kMaxKeys, code_rows(p) ? 1.25 : 1.1, kHeadsWg, sparse_mla_latent_only(p));
+  return mla_key_splits(p, (long long)p.B * p.S * p.G * chunks, kMaxKeys, code_rows(p) ? 1.25 : 1.1, kHeadsWg, sparse_mla_latent_only(p));
 }
 
 int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream) {

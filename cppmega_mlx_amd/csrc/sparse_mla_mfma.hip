@@ -878,9 +878,15 @@ bool sparse_mla_mfma_supported(const MlaParams& p) {
 
 size_t sparse_mla_mfma_plan_within(MlaParams& p, size_t have) {
   size_t need = 0;
+  p.no_few = 0;
   for (p.plan_level = 0;; ++p.plan_level) {
     sparse_mla_mfma_plan(p);
     need = sparse_mla_mfma_workspace_bytes(p);
+    if (need > have && p.few && !p.no_few) {
+      p.no_few = 1;
+      sparse_mla_mfma_plan(p);
+      need = sparse_mla_mfma_workspace_bytes(p);
+    }
     if (need <= have || p.plan_level == 2) return need;
   }
 }

@@ -575,19 +575,21 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_rows16_kernel(const MlaPara
   }
 }
 
-// rows of 576 e4m3 codes and 18 E8M0 bytes -> [B, Skv, G, 576] bf16: 16 codes per thread
-__global__ __launch_bounds__(256) void sparse_mla_e8m0_rows_kernel(const MlaParams p, unsigned short* out) {
+// Rows of 576 e4m3 codes and 18 E8M0 bytes as bf16, 16 codes per thread: the cache, [B, Skv, G, 576], then, for the kernel of 16
+// heads, the queries behind it (q_out), [B, S, H, 576].
+__global__ __launch_bounds__(256) void sparse_mla_e8m0_rows_kernel(const MlaParams p, unsigned short* out, unsigned short* q_out) {
   constexpr unsigned kPieces = kDqk / 16;
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  const size_t row = i / kPieces;
+  const size_t row = i / kPieces, cache_rows = (size_t)p.B * p.Skv * p.G;
   const unsigned piece = (unsigned)(i - row * kPieces);
-  if (row >= (size_t)p.B * p.Skv * p.G) return;
+  const bool of_q = row >= cache_rows;
+  if (of_q && (!q_out || row - cache_rows >= (size_t)p.B * p.S * p.H)) return;
   const size_t per_batch = (size_t)p.Skv * p.G, b = row / per_batch;
-  const size_t src = b * ((size_t)p.Skv_pitch * p.G) + (row - b * per_batch);
+  const size_t src = of_q ? row - cache_rows : b * ((size_t)p.Skv_pitch * p.G) + (row - b * per_batch);
   uint4 lo, hi;
-  dequant16<false>(*reinterpret_cast<const uint4*>((const unsigned char*)p.kv + src * kDqk + 16 * piece),
-                   e8m0_to_f32(((const unsigned char*)p.kv_scale)[src * (kDqk / 32) + (piece >> 1)]), lo, hi);
-  uint4* dst = reinterpret_cast<uint4*>(out + row * kDqk + 16 * piece);
+  dequant16<false>(*reinterpret_cast<const uint4*>((const unsigned char*)(of_q ? p.q : p.kv) + src * kDqk + 16 * piece),
+                   e8m0_to_f32(((const unsigned char*)(of_q ? p.q_scale : p.kv_scale))[src * (kDqk / 32) + (piece >> 1)]), lo, hi);
+  uint4* dst = reinterpret_cast<uint4*>((of_q ? q_out : out) + (of_q ? src : row) * kDqk + 16 * piece);
   dst[0] = lo;
   dst[1] = hi;
 }
@@ -626,12 +628,31 @@ bool sparse_mla_rows16_supported(const MlaParams& p) {
   return p.topk <= 16 * kMaxKeys;                 // the combine step merges at most 16 key splits
 }
 
-void sparse_mla_rows16_plan(MlaParams& p) {
+size_t sparse_mla_e8m0_copy_bytes(const MlaParams& p) {
+  return e8m0_rows(p) ? e8m0_row_bytes(p) + (((size_t)p.B * p.S * p.H * kDqk * 2 + 255) & ~(size_t)255) : 0;
+}
+
+int sparse_mla_e8m0_copy(MlaParams& p, hipStream_t stream) {
+  const size_t cache = e8m0_row_bytes(p), all = sparse_mla_e8m0_copy_bytes(p);
+  const size_t pieces = ((size_t)p.B * p.Skv * p.G + (size_t)p.B * p.S * p.H) * (kDqk / 16);
+  unsigned short *rows = (unsigned short*)p.workspace, *q = (unsigned short*)((char*)p.workspace + cache);
+  hipLaunchKernelGGL(sparse_mla_e8m0_rows_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, p, rows, q);
+  CM_HIP_CHECK(hipGetLastError());
+  p.kv = rows;
+  p.q = q;
+  p.Skv_pitch = p.Skv;
+  p.workspace = (char*)p.workspace + all;
+  p.q_dtype = p.kv_dtype = CPPMEGA_MI355_BF16;
+  p.q_scale_kind = p.kv_scale_kind = CPPMEGA_MI355_SCALE_NONE;
+  return 0;
+}
+
+double sparse_mla_rows16_plan(MlaParams& p) {
   p.rows16 = 1;
   p.heads_per_wg = p.heads_per_group <= 32 ? 32 : 64;
   const int chunks = (p.heads_per_group + p.heads_per_wg - 1) / p.heads_per_wg;
   const long long base = (long long)p.B * p.S * p.G * chunks;
-  mla_key_splits(p, base, kMaxKeys, p.heads_per_wg == 64 ? 1.1 : 0.85, p.heads_per_wg, false);
+  return mla_key_splits(p, base, kMaxKeys, p.heads_per_wg == 64 ? 1.1 : 0.85, p.heads_per_wg, false);
 }
 
 int sparse_mla_rows16_launch(const MlaParams& args, hipStream_t stream) {
@@ -643,7 +664,7 @@ int sparse_mla_rows16_launch(const MlaParams& args, hipStream_t stream) {
   const bool f16 = p.q_dtype == CPPMEGA_MI355_F16, e8 = e8m0_rows(p);
   if (e8) {
     const size_t pieces = (size_t)p.B * p.Skv * p.G * (kDqk / 16);
-    hipLaunchKernelGGL(sparse_mla_e8m0_rows_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, args, (unsigned short*)args.workspace);
+    hipLaunchKernelGGL(sparse_mla_e8m0_rows_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, args, (unsigned short*)args.workspace, (unsigned short*)nullptr);
     CM_HIP_CHECK(hipGetLastError());
     p.kv = args.workspace;
     p.Skv_pitch = p.Skv;

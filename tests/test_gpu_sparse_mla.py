@@ -771,6 +771,47 @@ def test_up_to_16_heads_per_group(device, rows, S, H, G, topk):
         assert err <= REL_TOL * ref and np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_TOL_MFMA
 
 
+# chunks of 16 heads of larger groups: one more than a chunk, a last chunk of 8 in a block of 32 of its own and not, two groups, key splits
+@pytest.mark.parametrize("S,H,G,topk", [(2, 17, 1, 1), (3, 40, 1, 129), (2, 72, 1, 700), (3, 64, 2, 640), (2, 128, 1, 900), (30, 128, 1, 64)])
+@pytest.mark.parametrize("rows", ["bf16", "float16_tail", "codes", "e8m0"])
+def test_few_queries_of_more_than_16_heads(device, rows, S, H, G, topk):
+    """Lists with skipped entries and an empty one, sinks, scores that grow along the list and a cache row that no list names and is not
+    finite."""
+    from cppmega_mlx_amd import _lib
+    B, Skv, sm = 1, 900, 0.05
+    rng = np.random.default_rng(S * H + topk)
+    idx = 1 + np.sort(sparse_indices(rng, B, S, G, Skv - 1, min(topk, Skv - 1)), axis=-1)
+    if topk > 1:
+        idx[rng.random(idx.shape) < 0.1] = -1
+    idx[0, 1] = -1
+    raw = rng.standard_normal((B, Skv, G, 576)).astype(np.float32) * np.linspace(0.2, 3.0, Skv).reshape(1, -1, 1, 1).astype(np.float32)
+    qraw, kw = rng.standard_normal((B, S, H, 576)).astype(np.float32), {}
+    if rows in ("bf16", "float16_tail"):
+        carrier = torch.bfloat16 if rows == "bf16" else torch.float16
+        q, kv = (torch.from_numpy(t).to(device).to(carrier) for t in (qraw, raw))
+        qf, decoded = q.double().cpu().numpy(), kv.double().cpu().numpy()
+        kv[0, 0] = float("nan")
+        if rows == "float16_tail":
+            kv, kw = kv[..., :512].contiguous(), dict(kv_rope=kv[..., 512:].contiguous())
+    else:
+        quantize, decode, kind, block = ((fp8.quantize_per_token, om.dequant_per_token, _lib.SCALE_PER_TOKEN, 0) if rows == "codes"
+                                         else (fp8.quantize_mxfp8, om.dequant_e8m0, _lib.SCALE_E8M0, 32))
+        (qc, qs), (kc, ks) = quantize(qraw), quantize(raw)
+        qf, decoded = decode(qc, qs), decode(kc, ks)
+        kc[0, 0] = 0x7f
+        q, kv = to_dev(qc, device), to_dev(kc, device)
+        kw = dict(q_spec=ops.QuantSpec(kind, to_dev(qs, device), block), kv_spec=ops.QuantSpec(kind, to_dev(ks, device), block))
+    sinks = rng.standard_normal(H).astype(np.float32)
+    want_out, want_lse = om.sparse_mla_oracle(qf, decoded, idx, sm_scale=sm, d_v=512, sinks=sinks)
+    for index_type, out_dtype in ((np.int32, torch.float32), (np.int64, torch.bfloat16)):
+        out = torch.zeros((B, S, H, 512), dtype=out_dtype, device=device)
+        lse = torch.zeros((B, S, H), dtype=torch.float32, device=device)
+        ops.sparse_mla_forward(q, kv, to_dev(idx.astype(index_type), device), sm_scale=sm, d_v=512, out=out, lse=lse,
+                               sinks=to_dev(sinks, device), kernel="mfma", **kw)
+        assert torch.isfinite(out).all()
+        _assert_close(out, lse, want_out, want_lse, rel=REL_TOL + 2 ** -8, lse_tol=LSE_TOL_MFMA)
+
+
 @pytest.mark.parametrize("S,topk", [(300, 64), (2, 700)])          # in one piece; in key splits
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_up_to_16_heads_write_outputs_that_begin_anywhere(device, S, topk, dtype):
