@@ -16,6 +16,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <unordered_map>
@@ -544,6 +545,124 @@ PyObject* cache_append(PyObject*, PyObject* const* arg, Py_ssize_t n) {
   return result;
 }
 
+// ---- training ----------------------------------------------------------------------------------
+// mla_backward(q, kv, d_out, indices, sm_scale or None, d_v or None) -> (dq in q's type, dkv float32) or None
+PyObject* mla_backward(PyObject*, PyObject* const* arg, Py_ssize_t n) {
+  if (n != 6) DECLINE;
+  const Tensor *q = tensor(arg[0]), *kv = tensor(arg[1]), *d_out = tensor(arg[2]), *idx = tensor(arg[3]);
+  if (!q || !kv || !d_out || !idx) DECLINE;
+  if (!(arg[4] == Py_None || PyFloat_CheckExact(arg[4])) || !(arg[5] == Py_None || PyLong_CheckExact(arg[5]))) DECLINE;
+  Place at;
+  if (!at.take(*q) || !at.dense(*q) || !at.dense(*kv) || !at.dense(*d_out) || !at.dense(*idx)) DECLINE;
+  const auto type = q->scalar_type();
+  if (q->dim() != 4 || kv->dim() != 4 || idx->dim() != 4 || !is_index(idx->scalar_type())) DECLINE;
+  if (!is_float(type) || kv->scalar_type() != type || d_out->scalar_type() != type) DECLINE;
+  const int64_t B = q->size(0), S = q->size(1), H = q->size(2), D = q->size(3), T = kv->size(1), G = kv->size(2), topk = idx->size(3);
+  const int64_t d_v = arg[5] == Py_None ? D : as_int(arg[5]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    DECLINE;
+  }
+  if (B < 1 || S < 1 || H < 1 || G < 1 || H % G != 0 || T < 1 || topk < 1 || d_v < 1 || d_v > D) DECLINE;
+  if (!has_shape(*kv, {B, T, G, D}) || !has_shape(*idx, {B, S, G, topk}) || !has_shape(*d_out, {B, S, H, d_v})) DECLINE;
+  for (int64_t x : {B, S, H, T, topk, D})
+    if (!fits_int(x)) DECLINE;
+  cppmega_mi355_sparse_mla_bwd_args_t a;
+  memset(&a, 0, sizeof(a));
+  a.struct_size = sizeof(a);
+  a.q_dtype = a.kv_dtype = a.d_out_dtype = a.dq_dtype = code(type);
+  a.index_dtype = code(idx->scalar_type());
+  a.q = q->data_ptr(); a.kv = kv->data_ptr(); a.d_out = d_out->data_ptr(); a.indices = idx->data_ptr();
+  a.batch = (int32_t)B; a.seq_q = (int32_t)S; a.heads = (int32_t)H; a.kv_groups = (int32_t)G; a.seq_kv = (int32_t)T; a.topk = (int32_t)topk;
+  a.d_qk = (int32_t)D; a.d_v = (int32_t)d_v;
+  a.sm_scale = (float)(arg[4] == Py_None ? std::pow((double)D, -0.5) : PyFloat_AS_DOUBLE(arg[4]));
+  a.clear_dkv = 1;
+  size_t bytes = 0;
+  if (cppmega_mi355_sparse_mla_bwd_workspace_bytes(&a, sizeof(a), &bytes)) DECLINE;
+  Tensor scratch;
+  if (bytes) {
+    scratch = workspace(at.device, at.stream, bytes);
+    a.workspace = scratch.data_ptr();
+    a.workspace_bytes = (size_t)scratch.numel();
+  }
+  Tensor dq = at::empty({B, S, H, D}, q->options()), dkv = at::empty({B, T, G, D}, kv->options().dtype(at::kFloat));
+  a.dq = dq.data_ptr();
+  a.dkv = (float*)dkv.data_ptr();
+  if (unlocked([&] { return cppmega_mi355_sparse_mla_bwd(&a, sizeof(a), at.stream); })) DECLINE;
+  PyObject* result = PyTuple_New(2);
+  if (!result) return nullptr;
+  PyTuple_SET_ITEM(result, 0, wrap(dq));
+  PyTuple_SET_ITEM(result, 1, wrap(dkv));
+  return result;
+}
+
+// indexer_loss(index_scores, topk_indices or None, query, key, softmax_scale, out or None, flag address, event) -> the losses, None, or
+// False: a list names a key that does not exist (out is as it was).  Flag: a word of pinned host memory of this thread's, event: a
+// hipEvent_t; the host waits for the kernel that reads the lists.
+PyObject* indexer_loss(PyObject*, PyObject* const* arg, Py_ssize_t n) {
+  if (n != 8) DECLINE;
+  const Tensor *scores = tensor(arg[0]), *idx = tensor(arg[1]), *query = tensor(arg[2]), *key = tensor(arg[3]), *out = tensor(arg[5]);
+  if (!scores || !query || !key || (!idx && arg[1] != Py_None) || (!out && arg[5] != Py_None) || !PyFloat_CheckExact(arg[4])) DECLINE;
+  Place at;
+  if (!at.take(*query) || !at.dense(*query) || !at.dense(*key) || !at.dense(*scores) || query->dim() != 4 || key->dim() != 4) DECLINE;
+  const auto type = query->scalar_type();
+  if (!is_float(type) || key->scalar_type() != type || scores->scalar_type() != ScalarType::Float) DECLINE;
+  const int64_t Sq = query->size(0), B = query->size(1), H = query->size(2), D = query->size(3), Sk = key->size(0);
+  if (Sq < 1 || B < 1 || H < 1 || H > 128 || D < 1 || Sk < 1) DECLINE;
+  if (!has_shape(*key, {Sk, B, H, D}) || !has_shape(*scores, {B, Sq, Sk})) DECLINE;
+  if (idx && (!at.dense(*idx) || !is_index(idx->scalar_type()) || idx->dim() != 3 || idx->size(2) < 1 || !has_shape(*idx, {B, Sq, idx->size(2)}))) DECLINE;
+  if (out && (!at.dense(*out) || out->scalar_type() != ScalarType::Float || !has_shape(*out, {B, Sq}))) DECLINE;
+  for (int64_t x : {Sq, B, D, Sk, idx ? idx->size(2) : 1})
+    if (!fits_int(x)) DECLINE;
+  cppmega_mi355_dsa_loss_args_t a;
+  memset(&a, 0, sizeof(a));
+  a.struct_size = sizeof(a);
+  a.in_dtype = code(type);
+  a.query = query->data_ptr(); a.key = key->data_ptr(); a.index_scores = (const float*)scores->data_ptr();
+  a.seq_q = (int32_t)Sq; a.batch = (int32_t)B; a.heads = (int32_t)H; a.head_dim = (int32_t)D; a.seq_k = (int32_t)Sk;
+  a.softmax_scale = (float)PyFloat_AS_DOUBLE(arg[4]);
+  if (idx) {
+    a.topk_indices = idx->data_ptr();
+    a.topk = (int32_t)idx->size(2);
+    a.index_dtype = code(idx->scalar_type());
+  }
+  size_t bytes = 0;
+  if (cppmega_mi355_dsa_indexer_loss_workspace_bytes(&a, sizeof(a), &bytes)) DECLINE;
+  Tensor scratch, fresh;
+  volatile int32_t* flag = nullptr;
+  if (idx) {
+    // (without a workspace no kernel reports; a capture cannot be waited for)
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (!bytes || hipStreamIsCapturing((hipStream_t)at.stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) DECLINE;
+    flag = (volatile int32_t*)PyLong_AsVoidPtr(arg[6]);
+    a.range_flag = (int32_t*)flag;
+    a.range_event = PyLong_AsVoidPtr(arg[7]);
+    if (PyErr_Occurred() || !flag || !a.range_event) {
+      PyErr_Clear();
+      DECLINE;
+    }
+    *flag = 0;
+  }
+  if (bytes) {
+    scratch = workspace(at.device, at.stream, bytes);
+    a.workspace = scratch.data_ptr();
+    a.workspace_bytes = (size_t)scratch.numel();
+  }
+  if (!out) fresh = at::empty({B, Sq}, query->options().dtype(at::kFloat));
+  a.loss = (float*)(out ? *out : fresh).data_ptr();
+  if (unlocked([&] { return cppmega_mi355_dsa_indexer_loss(&a, sizeof(a), at.stream); })) DECLINE;
+  if (idx) {
+    const int rc = unlocked([&] { return (int)hipEventSynchronize((hipEvent_t)a.range_event); });
+    if (rc) return PyErr_Format(PyExc_RuntimeError, "indexer loss: waiting for the lists' kernel failed: %s", hipGetErrorString((hipError_t)rc));
+    if (*flag) Py_RETURN_FALSE;
+  }
+  if (out) {
+    Py_INCREF(arg[5]);
+    return arg[5];
+  }
+  return wrap(fresh);
+}
+
 // ---- workspace of the Python launch helpers, release ---------------------------------------------
 // workspace(device, bytes, stream) -> tensor
 PyObject* workspace_of(PyObject*, PyObject* const* arg, Py_ssize_t n) {
@@ -574,6 +693,7 @@ PyMethodDef methods[] = {
     CALL("sparse_mla", sparse_mla),     CALL("topk", topk),         CALL("indexer", indexer),
     CALL("fused_gemm", fused_gemm),     CALL("vecmat", vecmat),     CALL("head_gemm", head_gemm),
     CALL("absorb_query", absorb_query), CALL("cache_append", cache_append), CALL("workspace", workspace_of),
+    CALL("mla_backward", mla_backward), CALL("indexer_loss", indexer_loss),
     {"release_workspaces", release_workspaces, METH_NOARGS, "Give the kept scratch tensors back to torch's allocator."},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Launch path of the per-step calls.", -1, methods};

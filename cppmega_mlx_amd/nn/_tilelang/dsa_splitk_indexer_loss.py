@@ -79,10 +79,22 @@ def _validated_topk(topk_indices: torch.Tensor, query: torch.Tensor, AB: int, AS
     return idx
 
 
+def _raise_out_of_range(idx: torch.Tensor, Sk: int):
+    raise ValueError(f"{_NAME}: topk_indices out of range [0, {Sk}); got [{int(idx.min().item())}, {int(idx.max().item())}].") from None
+
+
 def dsa_splitk_indexer_loss_per_position(index_scores: torch.Tensor, topk_indices: torch.Tensor | None, query: torch.Tensor,
                                          key: torch.Tensor, softmax_scale: float, sparse_loss: bool,
                                          out: torch.Tensor | None = None) -> torch.Tensor:
     """The [AB, ASq] float32 losses the wrapper averages (the reference's ``out_loss``, :1473)."""
+    if query.is_cuda and (topk_indices is not None or not sparse_loss):
+        watch = ops._range_watch(query.device) if sparse_loss else None
+        done = ops.host.indexer_loss(index_scores, topk_indices if sparse_loss else None, query, key, float(softmax_scale), out,
+                                     watch.flag_address if watch else 0, watch.event_handle if watch else 0)
+        if done is False:
+            _raise_out_of_range(topk_indices, int(key.shape[0]))
+        if done is not None:
+            return done
     if query.shape[1] != key.shape[1] or query.shape[2] != key.shape[2] or query.shape[3] != key.shape[3]:
         raise ValueError(f"{_NAME}: query/key shape mismatch: query {tuple(query.shape)}, key {tuple(key.shape)}")
     ASq, AB, AH, AD = (int(v) for v in query.shape)
@@ -103,7 +115,7 @@ def dsa_splitk_indexer_loss_per_position(index_scores: torch.Tensor, topk_indice
         return ops.dsa_indexer_loss(query if query.is_contiguous() else query.contiguous(), key if key.is_contiguous() else key.contiguous(),
                                     scores, softmax_scale=float(softmax_scale), out=out, topk_indices=idx, check_range=True)
     except ops.IndexRangeError:
-        raise ValueError(f"{_NAME}: topk_indices out of range [0, {Sk}); got [{int(idx.min().item())}, {int(idx.max().item())}].") from None
+        _raise_out_of_range(idx, Sk)
 
 
 def dsa_splitk_indexer_loss_tilelang(index_scores: torch.Tensor, topk_indices: torch.Tensor, query: torch.Tensor, key: torch.Tensor,

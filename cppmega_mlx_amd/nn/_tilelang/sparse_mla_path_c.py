@@ -151,6 +151,10 @@ def _sparse_mla_bwd_path_c_direct(q: torch.Tensor, kv: torch.Tensor, d_out: torc
 
 def _backward(q, kv, d_out, indices, sm_scale: torch.Tensor | float, d_v: int | None) -> tuple[torch.Tensor, torch.Tensor]:
     # (a number goes with the call: a buffer made for it would be a copy that the host waits for)
+    if isinstance(sm_scale, float):
+        done = ops.host.mla_backward(q, kv, d_out, indices, sm_scale, d_v)
+        if done is not None:
+            return done
     status = sparse_mla_path_c_status()
     if not status.available:
         raise SparseMLAPathCDirectError(status.reason)
@@ -174,6 +178,9 @@ def _backward(q, kv, d_out, indices, sm_scale: torch.Tensor | float, d_v: int | 
 def sparse_mla_bwd_path_c(q: torch.Tensor, kv: torch.Tensor, d_out: torch.Tensor, indices: torch.Tensor, *,
                           sm_scale: float | None = None, d_v: int | None = None) -> tuple[torch.Tensor, torch.Tensor] | None:
     """``(dq, dkv)`` for the cotangent ``d_out``, or ``None`` when the kernels cannot run."""
+    done = ops.host.mla_backward(q, kv, d_out, indices, sm_scale, d_v)
+    if done is not None:
+        return done
     if not sparse_mla_path_c_status().available:
         return None
     shapes = _resolve_shapes(q, kv, indices, d_v=d_v)

@@ -355,6 +355,7 @@ class _RangeWatch:
         with torch.cuda.device(device):
             self.event = torch.cuda.Event()
             self.event.record()          # creates the handle
+        self.flag_address, self.event_handle = self.flag.data_ptr(), self.event.cuda_event
 
 
 _range_watches = threading.local()       # a call waits for its own report, so one per thread and device is enough

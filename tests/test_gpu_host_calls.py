@@ -10,7 +10,9 @@ from cppmega_mlx_amd.nn import mla_absorb, sparse_mla
 from cppmega_mlx_amd.nn._tilelang import fp8_vecmat_path_c as vm
 from cppmega_mlx_amd.nn._tilelang import sparse_mla_blockscaled_path_c as bs
 from cppmega_mlx_amd.nn._tilelang import sparse_mla_fp8_path_c as f8
+from cppmega_mlx_amd.nn._tilelang.dsa_splitk_indexer_loss import dsa_splitk_indexer_loss_per_position
 from cppmega_mlx_amd.nn._tilelang.fused_fp8_gemm import fused_fp8_gemm
+from cppmega_mlx_amd.nn._tilelang.sparse_mla_path_c import sparse_mla_bwd_path_c
 from cppmega_mlx_amd.nn._tilelang.topk_selector import topk_selector, topk_selector_tilelang_direct
 from cppmega_mlx_amd.nn.lightning_indexer import indexer_scores_topk
 
@@ -98,3 +100,57 @@ def test_cpu_tensors_are_declined():
     x = torch.zeros((4, 8))
     assert ops.host.topk(x, 2, None, None, None, False, False) is None
     assert ops.host.fused_gemm(x, x, x, None) is None and ops.host.topk() is None
+
+
+def _training_calls(device):
+    g = torch.Generator(device=device).manual_seed(9)
+    normal = lambda *s: torch.randn(s, generator=g, device=device)
+    B, S, H, T, k = 2, 5, 16, 90, 24
+    q, kv, d_out = normal(B, S, H, 576).half(), normal(B, T, 1, 576).half(), normal(B, S, H, 512).half()
+    idx = torch.randint(-1, T, (B, S, 1, k), generator=g, device=device, dtype=torch.int32)
+    query, key, scores = normal(300, B, 4, 64).bfloat16(), normal(300, B, 4, 64).bfloat16(), normal(B, 300, 300)
+    lists = scores.topk(40, dim=-1).indices
+    per_position = dsa_splitk_indexer_loss_per_position
+    return {
+        "backward": lambda: sparse_mla_bwd_path_c(q, kv, d_out, idx, d_v=512),
+        "backward_scaled": lambda: sparse_mla_bwd_path_c(q.float(), kv.float(), d_out.float(), idx.long(), sm_scale=0.03, d_v=512),
+        "loss": lambda: per_position(scores, None, query, key, 0.125, False),
+        "loss_lists": lambda: per_position(scores, lists, query, key, 0.125, True, out=torch.empty((B, 300), device=device)),
+        "loss_lists_int32": lambda: per_position(scores, lists.int(), query.float(), key.float(), 0.125, True),
+    }
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["backward", "backward_scaled", "loss", "loss_lists", "loss_lists_int32"])
+def test_training_calls_give_the_results_of_the_python_helpers(device, monkeypatch, name):
+    call = _training_calls(device)[name]
+    native = _flat(call())
+    monkeypatch.setattr(ops, "host", _Declines())
+    for a, b in zip(native, _flat(call()), strict=True):
+        assert a.dtype == b.dtype and a.stride() == b.stride()
+        # (float32 rows of the backward are added with atomics: no order, sums of up to 2 x 5 x 16 terms)
+        assert torch.equal(a, b) if name != "backward_scaled" else torch.allclose(a, b, rtol=1e-4, atol=1e-4 * b.abs().max().item())
+
+
+@pytest.mark.gpu
+def test_training_calls_decline_what_is_not_the_plain_case(device):
+    host = _HOST
+    q, kv, d_out = (torch.zeros(s, device=device, dtype=torch.bfloat16) for s in ((1, 2, 16, 576), (1, 9, 1, 576), (1, 2, 16, 512)))
+    idx = torch.zeros((1, 2, 1, 4), device=device, dtype=torch.int32)
+    assert host.mla_backward(q, kv, d_out, idx, None, 512) is not None
+    for args in ((q.cpu(), kv, d_out, idx, None, 512), (q, kv.half(), d_out, idx, None, 512), (q, kv, d_out[..., :500], idx, None, 500),
+                 (q, kv, d_out, idx, 1, 512), (q, kv, d_out, idx, None, 577), (q, kv, d_out, idx.float(), None, 512), (q[:, :0], kv, d_out[:, :0], idx[:, :0], None, 512)):
+        assert host.mla_backward(*args) is None
+    query, scores = torch.zeros((300, 1, 4, 64), device=device, dtype=torch.bfloat16), torch.zeros((1, 300, 300), device=device)
+    lists = torch.zeros((1, 300, 8), device=device, dtype=torch.int32)
+    watch = ops._range_watch(scores.device)
+    good = (scores, lists, query, query, 0.1, None, watch.flag_address, watch.event_handle)
+    assert host.indexer_loss(*good) is not None
+    for i, bad in ((0, scores.half()), (0, scores[:, :, :299]), (1, lists[:, :, :0]), (1, lists[:, :299]), (2, query.float()), (4, 1), (5, scores), (6, 0), (7, 0)):
+        assert host.indexer_loss(*good[:i], bad, *good[i + 1:]) is None
+    out = torch.full((1, 300), 7.0, device=device)
+    lists[0, 5, 3] = 300
+    assert host.indexer_loss(*good[:5], out, *good[6:]) is False and (out == 7.0).all()
+    assert host.indexer_loss(*good) is False
+    lists[0, 5, 3] = 0
+    assert host.indexer_loss(*good) is not None          # (the report is of one call)
