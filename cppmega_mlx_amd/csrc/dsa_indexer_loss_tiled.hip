@@ -5,7 +5,7 @@
 // fills the CUs evenly, and no wavefront waits for another one's reductions:
 //
 //   dsa_loss_list_kernel    per row: membership bits of the index list, softmax statistics of the index scores (those
-//                           by the first pass where its tiles leave CUs idle)
+//                           by the first pass where there are no lists, or its tiles leave CUs idle)
 //   dsa_loss_tile_kernel<.., false>   per tile and head: sum of exp of the attention scores, per 64 keys
 //   dsa_loss_merge_kernel   per (head, row): log2 of the softmax denominator over all its keys
 //   dsa_loss_tile_kernel<.., true>    the scores again, p = mean over heads in registers, sum of p (log p - log q)
@@ -178,8 +178,8 @@ __host__ __device__ inline long long tiles_before(long long n, long long key_til
 // GENERAL: an additive mask is given, or the softmax scale is not positive.  Otherwise the masks are 0 or -inf
 // and enter the first pass as what its products start from (a select behind them where a row that does not count
 // turned out not to be finite), and the second pass leaves keys that do not count out at its end.
-// Where the tiles leave CUs idle, workgroups of the first pass between those of the tiles take the statistics of the index
-// scores, a row to a wavefront.
+// Workgroups of the first pass between or behind those of the tiles take the statistics of the index scores, a row to a
+// wavefront (where, run() says).
 constexpr int resident(int AD, bool general) { return AD <= 64 && !general ? 4 : 2; }
 template <bool F16, int AD, int GROUPS, bool SECOND, bool GENERAL>
 __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_tile_kernel(const LossTiledParams p) {
@@ -197,10 +197,11 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
   const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int id = (int)blockIdx.x;
   if (!SECOND && p.stats_rows) {
-    // eights of workgroups (one per XCD) of tiles and of statistics, in proportion
+    // eights of workgroups (one per XCD) of tiles and of statistics: with lists in proportion, else all tiles first
     const unsigned eight = (unsigned)id >> 3, stats_eights = (unsigned)(p.stats_groups + 7) >> 3, eights = gridDim.x >> 3;
-    const unsigned before = eight * stats_eights / eights;
-    if ((eight + 1) * stats_eights / eights != before) {
+    const unsigned tile_eights = eights - stats_eights;
+    const unsigned before = p.topk_idx ? eight * stats_eights / eights : eight > tile_eights ? eight - tile_eights : 0;
+    if (p.topk_idx ? (eight + 1) * stats_eights / eights != before : eight >= tile_eights) {
       const int row = ((int)before * 8 + (id & 7)) * (THREADS / 64) + wave;
       if (row < p.stats_rows) {
         const unsigned* bits = p.bits + (size_t)row * p.words;
@@ -595,15 +596,16 @@ int run(LossTiledParams p, hipStream_t stream) {
     const long long rest = all % round;
     return 16 * rest <= (p.topk_idx ? 7 : 9) * round ? all - rest : all;
   };
-  // The statistics go with the tiles where those are split, so that they do not fill the CUs, and leave room for them: with
-  // lists, whose kernel is there anyway, up to a fifth of a round of tiles (by themselves / with them, 8 heads of 64: 180 tiles 39.0 /
-  // 36.8 us, 242 40.0 / 41.4, 450 52.8 / 56.1), dense up to 5/16, and where the split ones are more than a round anyway; between, tiles
-  // that would start at once wait for them (272 35.8 / 33.7, 361 37.7 / 38.2, 450 42.1 / 44.0, 552 51.1 / 48.1; 16 heads 48.5 / 46.3, 50.9 /
-  // 52.1, 57.1 / 64.9, 71.9 / 69.9).  A workgroup of the larger heads keeps a CU or half of one (16 heads of 128: 64 tiles 38.8 / 35.1, 121
-  // 42.1 / 47.3, 225 56.3 / 67.2).
+  // The statistics of the index scores go with the tiles.  Dense: behind them, where they fill what the last round leaves idle, read
+  // memory beside exponentials and need no launch of their own (a kernel in front / between the tiles / behind them: 3300 positions x 16 heads
+  // of 64 74.8 / 76.8 / 69.6 us, 1800 x 2 x 16 of 128 77.2 / 80.9 / 71.9, 2400 x 8 of 128 49.9 / 50.1 / 45.6, 1800 x 8 of 64 29.9 / 29.7 / 26.7, 350
+  // 19.2 / 19.0 / 18.9; of 58 shapes three are slower, by 1 to 2 %).  With lists, whose kernel is there anyway: between the tiles where those are split, so
+  // that they do not fill the CUs, and leave room for them, which they do up to a fifth of a round (by themselves / with them, 8 heads of 64:
+  // 180 tiles 39.0 / 36.8 us, 242 40.0 / 41.4, 450 52.8 / 56.1; behind the tiles 8 heads are up to 6 % slower and 16 up to 5 % faster).  A workgroup of the
+  // larger heads keeps a CU or half of one (16 heads of 128: 64 tiles 38.8 / 35.1, 121 42.1 / 47.3, 225 56.3 / 67.2).
   const long long of_all_rows = tiles_before((p.ASq + kQ - 1) / kQ, key_tiles) * p.AB;
-  const bool room = AD > 64 ? of_all_rows <= 64 : p.topk_idx ? 5 * of_all_rows <= round : 16 * of_all_rows <= 5 * round || 2 * of_all_rows > round;
-  const bool in_tiles = p.slab_rows >= p.ASq && whole_of(of_all_rows) == 0 && room;
+  const bool room = whole_of(of_all_rows) == 0 && (AD > 64 ? of_all_rows <= 64 : 5 * of_all_rows <= round);
+  const bool in_tiles = p.slab_rows >= p.ASq && (room || !p.topk_idx);
   p.stats_rows = in_tiles ? (int)rows : 0;
   if (p.topk_idx || !in_tiles)
     hipLaunchKernelGGL(dsa_loss_list_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads), p.topk_idx ? 16 * (size_t)p.words : 0, stream, p);
