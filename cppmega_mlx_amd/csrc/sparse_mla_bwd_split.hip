@@ -6,7 +6,7 @@
 // at their own occupancy:
 //
 //   lists    per (query, group): its valid keys in order, and where each band of keys begins;
-//   steps    per band: the pieces of up to 16 keys that the queries have in it, one after the other;
+//   steps    per band: the pieces of up to 16 keys that the queries have in it, one after the other (workgroups of the next kernel);
 //   scores   per (query, 16 heads): S = Q . K^T and dP = dO . K^T with the scores of all keys in registers,
 //            softmax statistics and delta across the workgroup, then P and dS = sm_scale P (dP - delta) as two
 //            16-bit planes each (hi = round(x), lo = round(x - hi), a term is good to 2^-17), and q and d_out by
@@ -19,8 +19,8 @@
 //
 // Nothing is added in an order that varies: the same input gives the same bits.
 //
-// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 158 us (561 us with the atomics; under the profiler lists 7,
-// steps 6, scores and dq 68, dkv 71 .. 87, sum 9).  dkv is bound by the vector cache (27 M accesses of 64 bytes: 4 KB of q and d_out and
+// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 150 us (561 us with the atomics; under the profiler lists 6,
+// scores and dq 68, dkv 71 .. 87, sum 9).  dkv is bound by the vector cache (27 M accesses of 64 bytes: 4 KB of q and d_out and
 // about 1 KB of planes for a step's 9 keys of 16) and ends with the CUs whose three bands are all full; scores and dq by the
 // gather of 302 MB of key rows each.
 
@@ -80,70 +80,123 @@ struct SplitParams {
 static_assert(kBandKeys < 256, "rows are bytes, and row band_keys is that of slots of no key");
 
 // ---- lists -----------------------------------------------------------------------------------
-// The valid keys by band in LDS, then each to its rank within the band.
+// A bit per cache row says which are named; what stands below a key's bit is its rank.  A list that names a key twice is
+// sorted by bands and then to each key's rank within its band.  (For every list the latter took 7.4 us at 1024 x 256 of 4096 keys,
+// 11.8 at 600 x 250 of 852, whose bands hold 50 keys of a list; 5.6 and 5.2 here.)
 __global__ __launch_bounds__(kThreads) void bwd_lists_kernel(const SplitParams p) {
   extern __shared__ int smem_lists[];
-  int* begin = smem_lists;                             // [bands]
-  int* fill = begin + p.bands;                         // [bands]
-  int* loose = fill + p.bands;                         // [topk]
+  const int words = (p.Skv + 31) / 32;
+  int* begin = smem_lists;                             // [bands]: the band's first slot
+  int* fill = begin + p.bands;                         // [bands]: behind its last
+  int* step_of = fill + p.bands;                       // [bands]: its first step
+  int* loose = step_of + p.bands;                      // [topk]
   int* sorted = loose + p.topk;                        // [topk]
-  int* again = sorted + p.topk;                        // [1]
-  int* step_of = again + 1;                            // [bands + 1]: the band's first step
-  const int tid = (int)threadIdx.x, lane = tid & 63;
+  unsigned* bits = reinterpret_cast<unsigned*>(sorted + p.topk);       // [words]
+  int* below = reinterpret_cast<int*>(bits + words);   // [words]: keys in the words before
+  __shared__ int sums[kThreads / 64], again;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const size_t list = blockIdx.x;
   const unsigned bs = blockIdx.x / (unsigned)p.G;
   const int g = (int)(blockIdx.x - bs * (unsigned)p.G), b = (int)(bs / (unsigned)p.ns), s = (int)(bs - (unsigned)b * (unsigned)p.ns);
   const size_t src = (((size_t)b * p.S + p.s0 + s) * p.G + g) * (size_t)p.topk;
   if (list == 0 && tid == 0) p.band_steps[0] = 0;
   if (list == 0 && tid < 16) p.rows[p.dead_step / 4 + tid] = (unsigned char)p.band_keys;
-  for (int r = tid; r < p.bands; r += kThreads) fill[r] = 0;
-  if (tid == 0) *again = 0;
-  __syncthreads();
-  int key[8], band[8];                                 // topk <= 2048
+  int key[8];                                          // topk <= 2048
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int k = tid + i * kThreads;
     if (i * kThreads >= p.topk) {                      // (uniform)
-      key[i] = band[i] = -1;
+      key[i] = -1;
       continue;
     }
     long long v = -1;
     if (k < p.topk)
       v = p.index_dtype == CPPMEGA_MI355_I64 ? static_cast<const long long*>(p.indices)[src + k] : (long long)static_cast<const int*>(p.indices)[src + k];
     key[i] = v >= 0 && v < p.Skv ? (int)v : -1;
-    band[i] = key[i] >= 0 ? key[i] / p.band_keys : -1;
-    if (band[i] >= 0) atomicAdd(fill + band[i], 1);
   }
-  __syncthreads();
-  int* starts = p.starts + list * (p.bands + 2);
-  if (tid < 64) {                                      // exclusive prefix, 64 bands at a time
-    int base = 0, step_base = 0;
-    for (int r0 = 0; r0 < p.bands; r0 += 64) {
-      const int r = r0 + lane, n = r < p.bands ? fill[r] : 0, steps = (n + 15) / 16;
-      const int upto = (int)wave_inclusive_sum((unsigned)n), steps_upto = (int)wave_inclusive_sum((unsigned)steps);
-      if (r < p.bands) {
-        starts[r] = begin[r] = fill[r] = base + upto - n;
-        step_of[r] = step_base + steps_upto - steps;
-      }
-      base += __shfl(upto, 63, 64);
-      step_base += __shfl(steps_upto, 63, 64);
-    }
-    if (lane == 0) {
-      starts[p.bands] = base;
-      step_of[p.bands] = step_base;
-    }
-  }
+  for (int w = tid; w < words; w += kThreads) bits[w] = 0u;
+  for (int r = tid; r < p.bands; r += kThreads) fill[r] = 0;
+  if (tid == 0) again = 0;
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    if (band[i] >= 0) loose[atomicAdd(fill + band[i], 1)] = key[i];
+    if (key[i] >= 0) {
+      const unsigned bit = 1u << (key[i] & 31);
+      if (atomicOr(bits + (key[i] >> 5), bit) & bit) again = 1;
+    }
   __syncthreads();
-  const int valid = fill[p.bands - 1];                 // (where its keys end now)
-  for (int e = tid; e < valid; e += kThreads) {
-    const int v = loose[e], first = begin[v / p.band_keys], last = fill[v / p.band_keys];
-    int at = first;
-    for (int o = first; o < last; ++o) at += loose[o] < v || (loose[o] == v && o < e);
-    sorted[at] = v;
+  const bool twice = again != 0;                       // (uniform)
+  int valid;
+  if (!twice) {
+    const int per = (words + kThreads - 1) / kThreads, w0 = min(tid * per, words), w1 = min(w0 + per, words);
+    int mine = 0;
+    for (int w = w0; w < w1; ++w) mine += __popc(bits[w]);
+    const int upto = (int)wave_inclusive_sum_dpp((unsigned)mine);
+    if (lane == 63) sums[wave] = upto;
+    __syncthreads();
+    int at = upto - mine;
+    valid = 0;
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; ++w) {
+      if (w < wave) at += sums[w];
+      valid += sums[w];
+    }
+    for (int w = w0; w < w1; ++w) {
+      below[w] = at;
+      at += __popc(bits[w]);
+    }
+    __syncthreads();
+    auto rank = [&](int k) { return below[k >> 5] + __popc(bits[k >> 5] & ((1u << (k & 31)) - 1u)); };
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (key[i] >= 0) sorted[rank(key[i])] = key[i];
+    for (int r = tid; r < p.bands; r += kThreads) {
+      begin[r] = r * p.band_keys < p.Skv ? rank(r * p.band_keys) : valid;              // (bands behind the end are empty)
+      fill[r] = (r + 1) * p.band_keys < p.Skv ? rank((r + 1) * p.band_keys) : valid;
+    }
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (key[i] >= 0) atomicAdd(fill + key[i] / p.band_keys, 1);
+    __syncthreads();
+    if (tid < 64) {                                    // exclusive prefix, 64 bands at a time
+      int base = 0;
+      for (int r0 = 0; r0 < p.bands; r0 += 64) {
+        const int r = r0 + lane, n = r < p.bands ? fill[r] : 0, upto = (int)wave_inclusive_sum((unsigned)n);
+        if (r < p.bands) begin[r] = fill[r] = base + upto - n;
+        base += __shfl(upto, 63, 64);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (key[i] >= 0) loose[atomicAdd(fill + key[i] / p.band_keys, 1)] = key[i];
+    __syncthreads();
+    valid = fill[p.bands - 1];                         // (where its keys end now)
+    for (int e = tid; e < valid; e += kThreads) {
+      const int v = loose[e], first = begin[v / p.band_keys], last = fill[v / p.band_keys];
+      int at = first;
+      for (int o = first; o < last; ++o) at += loose[o] < v || (loose[o] == v && o < e);
+      sorted[at] = v;
+    }
+    __syncthreads();
+    if (tid == 0) again = 0;                           // (from here on: whether a step of 16 holds a key twice)
+  }
+  int* starts = p.starts + list * (p.bands + 2);
+  if (tid < 64) {
+    int base = 0;
+    for (int r0 = 0; r0 < p.bands; r0 += 64) {
+      const int r = r0 + lane, first = r < p.bands ? begin[r] : 0, steps = r < p.bands ? (fill[r] - first + 15) / 16 : 0;
+      const int upto = (int)wave_inclusive_sum((unsigned)steps);
+      if (r < p.bands) {
+        starts[r] = first;
+        step_of[r] = base + upto - steps;
+        p.step_starts[list * p.bands + r] = base + upto - steps;
+      }
+      base += __shfl(upto, 63, 64);
+    }
+    if (lane == 0) starts[p.bands] = valid;
   }
   __syncthreads();
   // a key that its step of 16 (from the band's first slot on) holds already is marked, and has no row
@@ -154,31 +207,30 @@ __global__ __launch_bounds__(kThreads) void bwd_lists_kernel(const SplitParams p
     if (k < valid) {
       v = sorted[k];
       const int of = v / p.band_keys, nth = k - begin[of], row = v - of * p.band_keys;
-      const bool marked = (nth & 15) != 0 && sorted[k - 1] == v;
+      const bool marked = twice && (nth & 15) != 0 && sorted[k - 1] == v;
       unsigned char* at = rows + step_of[of] * 16 + nth;
       *at = (unsigned char)(marked ? p.band_keys : row);
       if (k + 1 == fill[of])
         for (int e = nth + 1; e & 15; ++e) *++at = (unsigned char)p.band_keys;
       if (marked) {
         v |= kAgain;
-        *again = 1;
+        again = 1;
       }
     }
     out[k] = v;
   }
   __syncthreads();
-  if (tid == 0) starts[p.bands + 1] = *again;
-  for (int r = tid; r < p.bands; r += kThreads) p.step_starts[list * p.bands + r] = step_of[r];
+  if (tid == 0) starts[p.bands + 1] = again;
 }
 
 // ---- steps -----------------------------------------------------------------------------------
-constexpr int kStepThreads = 1024;
-
-__global__ __launch_bounds__(kStepThreads) void bwd_steps_kernel(const SplitParams p) {
-  __shared__ int sums[kStepThreads / 64], base_of;
+// A band to a workgroup, the first workgroups of the kernel of the scores, which needs none of it: 4 to 6 us as a launch of its own.
+template <int THREADS>
+__device__ void steps_of_band(const SplitParams& p, int of) {
+  __shared__ int sums[THREADS / 64], base_of;
   const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int band = (int)blockIdx.x % p.bands, bg = (int)blockIdx.x / p.bands, b = bg / p.G, g = bg - b * p.G;
-  const int per = (p.ns + kStepThreads - 1) / kStepThreads, s0 = min(tid * per, p.ns), s1 = min(s0 + per, p.ns);
+  const int band = of % p.bands, bg = of / p.bands, b = bg / p.G, g = bg - b * p.G;
+  const int per = (p.ns + THREADS - 1) / THREADS, s0 = min(tid * per, p.ns), s1 = min(s0 + per, p.ns);
   auto row = [&](int s) { return p.starts + (((size_t)b * p.ns + s) * p.G + g) * (p.bands + 2); };
   int mine = 0;
   for (int s = s0; s < s1; ++s) mine += (row(s)[band + 1] - row(s)[band] + 15) / 16 * p.chunks;
@@ -186,19 +238,19 @@ __global__ __launch_bounds__(kStepThreads) void bwd_steps_kernel(const SplitPara
   if (lane == 63) sums[wave] = upto;
   __syncthreads();
   int at = upto - mine, all = 0;
-  for (int w = 0; w < kStepThreads / 64; ++w) {
+  for (int w = 0; w < THREADS / 64; ++w) {
     if (w < wave) at += sums[w];
     all += sums[w];
   }
   const int padded = (all + kStepGroup - 1) / kStepGroup * kStepGroup;            // with steps whose rows are all dead
   if (tid == 0) {
     base_of = atomicAdd(p.band_steps, padded);
-    p.band_steps[2 + 2 * blockIdx.x] = base_of;
-    p.band_steps[3 + 2 * blockIdx.x] = padded;
+    p.band_steps[2 + 2 * of] = base_of;
+    p.band_steps[3 + 2 * of] = padded;
   }
   __syncthreads();
   i32x4* out = p.steps + base_of;
-  for (int e = all + tid; e < padded; e += kStepThreads) out[e] = i32x4{0, (int)p.dead_step, 0, 0};
+  for (int e = all + tid; e < padded; e += THREADS) out[e] = i32x4{0, (int)p.dead_step, 0, 0};
   for (int s = s0; s < s1; ++s) {
     const size_t list = ((size_t)b * p.ns + s) * p.G + g;
     const int* st = row(s);
@@ -212,6 +264,10 @@ __global__ __launch_bounds__(kStepThreads) void bwd_steps_kernel(const SplitPara
       }
   }
 }
+
+// Where a 16-byte piece of a row of 64 channels stands in LDS: piece ^ fold_piece(row).  The sixteen rows that an operand read
+// takes together, one piece or those of neighbouring quarter wavefronts, fall on all eight places.
+__device__ __forceinline__ int fold_piece(int row) { return ((((row >> 3) ^ (row >> 2)) & 1) << 2) | (((row >> 2) & 1) << 1) | ((row >> 1) & 1); }
 
 // the key of a slot, -1 for none
 __device__ __forceinline__ int plain_key(int slot) { return slot < 0 ? -1 : slot & ~kAgain; }
@@ -349,6 +405,11 @@ constexpr int kQueue = 6;                              // pieces of 32 channels 
 
 template <bool F16, int W, int T>
 __global__ __launch_bounds__(W * 64, 4) void bwd_scores_kernel(const SplitParams p) {
+  const int step_groups = p.B * p.G * p.bands;
+  if ((int)blockIdx.x < step_groups) {
+    steps_of_band<W * 64>(p, (int)blockIdx.x);
+    return;
+  }
   extern __shared__ __align__(16) unsigned char smem[];
   const int D = p.D, dv = p.d_v, Dp = D + 8, Dvp = dv + 8;
   unsigned short* Qs = reinterpret_cast<unsigned short*>(smem);       // [16][Dp]
@@ -356,7 +417,7 @@ __global__ __launch_bounds__(W * 64, 4) void bwd_scores_kernel(const SplitParams
   float* met = reinterpret_cast<float*>(Os + kHeads * Dvp);           // [W][16][3]
   unsigned short* pieces = reinterpret_cast<unsigned short*>(met + W * kHeads * 3);       // [W][16 keys][32]
   const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, kg = lane >> 4;
-  const Item it = item_of(p, blockIdx.x);
+  const Item it = item_of(p, blockIdx.x - (unsigned)step_groups);
   const float sm_scale = p.sm_scale_dev ? *p.sm_scale_dev : p.sm_scale;
   const float scale2 = sm_scale * kLog2e;
   const int* keys = p.keys + it.list * (size_t)p.stride;
@@ -565,13 +626,18 @@ __global__ __launch_bounds__(64, 3) void bwd_dq_kernel(const SplitParams p) {
 // little more than an XCD's L2) and by the phases of a workgroup, two of which share a CU (77 KB of LDS each): 5 us until
 // q, d_out and the first keys are there, 8 for the scores, 6 for statistics and planes, 9 for dq.  Neither half the
 // loads in flight nor q and d_out in registers made a difference to the large shape.
-constexpr int kD = 576, kDv = 512, kDp = kD + 8, kDvp = kDv + 8, kStage = 5;
+constexpr int kD = 576, kDv = 512, kDp = kD + 8, kDvp = kDv + 8, kStage = 2, kStages = 5;       // pieces of 64 channels of a tile to a stage
 constexpr int kFusedRows = kHeads * (kDp + kDvp) * 2;  // bytes of q and d_out, then of dS
 template <int W> constexpr int kFusedLds = kFusedRows + W * (kHeads * 3 * 4 + kKtile) + W * 64 * 4;
-static_assert(2 * kStage * 1024 <= kKtile && 4 * kStage >= kD / 32, "a stage of two tiles and 32 keys of dq share a wavefront's LDS");
+static_assert(2 * kStage * 2048 <= kKtile && kStages * kStage >= kD / 64, "a stage of two tiles and 32 keys of dq share a wavefront's LDS");
 
 template <bool F16, int W>
 __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitParams p) {
+  const int step_groups = p.B * p.G * p.bands;
+  if ((int)blockIdx.x < step_groups) {
+    steps_of_band<W * 64>(p, (int)blockIdx.x);
+    return;
+  }
   constexpr int T = 4, kSlots = W * T * 16;
   static_assert(2 * kSlots * kHeads * 2 <= kFusedRows, "dS takes the place of q and d_out");
   extern __shared__ __align__(16) unsigned char smem[];
@@ -582,7 +648,7 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   char* own = reinterpret_cast<char*>(met + W * kHeads * 3) + wave * kKtile;
   int* list_keys = reinterpret_cast<int*>(reinterpret_cast<char*>(met + W * kHeads * 3) + W * kKtile);       // [64 W]
-  const Item it = item_of(p, blockIdx.x);
+  const Item it = item_of(p, blockIdx.x - (unsigned)step_groups);
   const float sm_scale = p.sm_scale_dev ? *p.sm_scale_dev : p.sm_scale;
   const float scale2 = sm_scale * kLog2e;
   const int* keys = p.keys + it.list * (size_t)p.stride;
@@ -590,16 +656,21 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
   const unsigned short* kv = p.kv + ((size_t)it.b * p.Skv * p.G + it.g) * (size_t)kD;
   const size_t key_step = (size_t)p.G * kD;
 
-  // Two tiles at a time, up to five pieces of 32 channels of each per stage, four lanes to a row: two stages are on
-  // their way in registers while one passes through LDS to operand order.
-  const int row = lane >> 2, col = lane & 3;
-  unsigned short* put = reinterpret_cast<unsigned short*>(own) + row * 32 + ((col ^ (-(row >> 2) & 3)) << 3);
-  const unsigned short* get = reinterpret_cast<const unsigned short*>(own) + l16 * 32 + ((kg ^ (-(l16 >> 2) & 3)) << 3);
-  int slot_row[T], slot_16[T];                         // (tiles behind the list's room are the last one again, and nobody looks)
+  // Two tiles at a time, two pieces of 64 channels of each per stage, eight lanes to a row (a load serves twice as much from
+  // pieces of 128 bytes as of 64): two stages are on their way in registers while one passes through LDS to operand order.
+  const int row = lane >> 3, col = lane & 7;
+  unsigned short* put[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) put[r] = reinterpret_cast<unsigned short*>(own) + (row + 8 * r) * 64 + ((col ^ fold_piece(row + 8 * r)) << 3);
+  const unsigned short* get[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) get[u] = reinterpret_cast<const unsigned short*>(own) + l16 * 64 + (((4 * u + kg) ^ fold_piece(l16)) << 3);
+  int slot_row[T][2], slot_16[T];                      // (tiles behind the list's room are the last one again, and nobody looks)
 #pragma unroll
   for (int i = 0; i < T; ++i) {
     const int* of_tile = keys + min(wave + i * W, p.stride / 16 - 1) * 16;
-    slot_row[i] = of_tile[row];
+    slot_row[i][0] = of_tile[row];
+    slot_row[i][1] = of_tile[row + 8];
     slot_16[i] = of_tile[l16];
   }
   const int slot_own = keys[min(tid, p.stride - 1)];
@@ -612,10 +683,12 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
     const int e = tid + (of_q ? i : i - kQLoads) * W * 64, per = (of_q ? kD : kDv) / 8, h = min(e / per, it.nh - 1), c = e - e / per * per;
     staged[i] = *reinterpret_cast<const u32x4*>((of_q ? p.q : p.d_out) + (it.bs * p.H + it.h0 + h) * (size_t)(of_q ? kD : kDv) + c * 8);
   }
-  u32x4 queue[2][2][kStage];
-  const unsigned short* rows_at[T];
+  u32x4 queue[2][2][kStage][2];
+  const unsigned short* rows_at[T][2];
 #pragma unroll
-  for (int i = 0; i < T; ++i) rows_at[i] = kv + (size_t)max(plain_key(slot_row[i]), 0) * key_step + col * 8;
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int r = 0; r < 2; ++r) rows_at[i][r] = kv + (size_t)max(plain_key(slot_row[i][r]), 0) * key_step + col * 8;
   auto request = [&](auto pair_c, auto stage_c) {      // a stage of tiles 2 * pair and 2 * pair + 1
     constexpr int pair = decltype(pair_c)::value, stage = decltype(stage_c)::value;
 #pragma unroll
@@ -623,7 +696,9 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
       if (wave + (2 * pair + j) * W < tiles)           // (uniform)
 #pragma unroll
         for (int q = 0; q < kStage; ++q)
-          if (stage * kStage + q < kD / 32) queue[stage & 1][j][q] = *reinterpret_cast<const u32x4*>(rows_at[2 * pair + j] + (stage * kStage + q) * 32);
+          if (stage * kStage + q < kD / 64)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) queue[(pair * kStages + stage) & 1][j][q][r] = *reinterpret_cast<const u32x4*>(rows_at[2 * pair + j][r] + (stage * kStage + q) * 64);
   };
   using std::integral_constant;
   request(integral_constant<int, 0>{}, integral_constant<int, 0>{});
@@ -653,22 +728,24 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
         if (j == 0 || two)
 #pragma unroll
           for (int q = 0; q < kStage; ++q)
-            if (stage * kStage + q < kD / 32) *reinterpret_cast<u32x4*>(put + (j * kStage + q) * 512) = queue[stage & 1][j][q];
-      __builtin_amdgcn_wave_barrier();
-      if constexpr (stage < 2) request(pair_c, integral_constant<int, stage + 2>{});
-      else if constexpr (pair == 0) request(integral_constant<int, 1>{}, integral_constant<int, stage - 2>{});
+            if (stage * kStage + q < kD / 64)
 #pragma unroll
-      for (int q = 0; q < kStage; ++q) {
-        constexpr int c0 = stage * kStage;
-        const int c = c0 + q;
+              for (int r = 0; r < 2; ++r) *reinterpret_cast<u32x4*>(put[r] + (j * kStage + q) * 1024) = queue[(pair * kStages + stage) & 1][j][q][r];
+      __builtin_amdgcn_wave_barrier();
+      if constexpr (stage < kStages - 2) request(pair_c, integral_constant<int, stage + 2>{});
+      else if constexpr (pair == 0) request(integral_constant<int, 1>{}, integral_constant<int, stage + 2 - kStages>{});
+#pragma unroll
+      for (int qu = 0; qu < 2 * kStage; ++qu) {
+        constexpr int c0 = 2 * stage * kStage;
+        const int c = c0 + qu, q = qu >> 1;              // of 32 channels
         if (c >= kD / 32) continue;
-        const bf16x8 a = lds_b128(qa + c * 32), k0 = lds_b128(get + q * 512);
+        const bf16x8 a = lds_b128(qa + c * 32), k0 = lds_b128(get[qu & 1] + q * 1024);
         bf16x8 o = a, k1 = k0;
         if (c < kDv / 32) o = lds_b128(oa + c * 32);
         sa[0] = mm<F16>(a, k0, sa[0]);
         if (c < kDv / 32) da[0] = mm<F16>(o, k0, da[0]);
         if (two) {
-          k1 = lds_b128(get + (kStage + q) * 512);
+          k1 = lds_b128(get[qu & 1] + (kStage + q) * 1024);
           sa[1] = mm<F16>(a, k1, sa[1]);
           if (c < kDv / 32) da[1] = mm<F16>(o, k1, da[1]);
         }
@@ -679,6 +756,7 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
     stage_of(integral_constant<int, 1>{});
     stage_of(integral_constant<int, 2>{});
     stage_of(integral_constant<int, 3>{});
+    stage_of(integral_constant<int, 4>{});
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int i = 2 * pair + j;
@@ -1029,9 +1107,8 @@ int run(SplitParams p, const Plan& l, bool clear, hipStream_t stream) {
     p.shares = l.shares;
     p.accumulate = p.s0 > 0 || !clear;
     const size_t lists = (size_t)p.B * p.ns * p.G, items = lists * p.chunks;
-    hipLaunchKernelGGL(bwd_lists_kernel, dim3((unsigned)lists), dim3(kThreads), (size_t)(3 * p.bands + 2 * p.topk + 2) * 4, stream, p);
-    hipLaunchKernelGGL(bwd_steps_kernel, dim3((unsigned)(p.B * p.G * p.bands)), dim3(kStepThreads), 0, stream, p);
-    const dim3 of_items((unsigned)items);
+    hipLaunchKernelGGL(bwd_lists_kernel, dim3((unsigned)lists), dim3(kThreads), (size_t)(3 * p.bands + 2 * p.topk + 2 * ((p.Skv + 31) / 32)) * 4, stream, p);
+    const dim3 of_items((unsigned)(items + (size_t)p.B * p.G * p.bands));        // (and the bands' steps in front)
     // Of eight wavefronts with up to 512 keys a CU holds one workgroup: one kernel while that is one round, else two (rows of 3000 keys, one kernel
     // / two: 220 items x 350 27.5 / 36.5 us, 250 x 500 33.4 / 45.4, 376 x 438 55.9 / 53.7, 440 x 300 48.2 / 46.4, 2000 x 350 of 4000 215 / 194).
     const bool fused = rows_of_576 && (p.topk <= 256 || items <= 256);

@@ -421,3 +421,28 @@ def test_bands_of_any_width(device, S, H, G, Skv, topk):
     for got, ref in zip((dq, dkv), want):
         err, scale = error_report(got.cpu().numpy(), ref)
         assert err <= 1e-4 * scale, (err, scale)                # planes of 2^-17 and float32 sums of up to 70 x 24 terms
+
+
+@pytest.mark.parametrize("Skv,topk", [(33, 32), (4097, 64), (65536, 700), (65535, 2048)])          # one word of bits and one more; bands behind the last key
+@pytest.mark.parametrize("twice", [False, True])
+def test_lists_by_rank_and_by_sorting(device, Skv, topk, twice):
+    """Lists in any order, of keys named once (their rank comes from bits) or, one list of them, twice; an empty list, the first and the last key."""
+    S, H, D, d_v = 5, 8, 64, 32
+    rng = np.random.default_rng(Skv + topk)
+    idx = np.stack([rng.permutation(Skv)[:topk] for _ in range(S)]).reshape(1, S, 1, topk)
+    idx[rng.random(idx.shape) < 0.2] = -1
+    idx[0, 0, 0, :2] = [Skv - 1, 0]
+    idx[0, 1] = -1
+    if not twice:
+        idx[0, 0, 0, 2:][np.isin(idx[0, 0, 0, 2:], [0, Skv - 1])] = -1
+    else:
+        idx[0, 3, 0, -1] = idx[0, 3, 0, 0] = 7
+    carrier = torch.bfloat16
+    qt, kt, dt = (to_dev(rng.standard_normal(s).astype(np.float32), device).to(carrier) for s in ((1, S, H, D), (1, Skv, 1, D), (1, S, H, d_v)))
+    want_dq, want_dkv = om.sparse_mla_bwd_oracle(*(t.double().cpu().numpy() for t in (qt, kt)), idx, dt.double().cpu().numpy(), sm_scale=0.1, d_v=d_v)
+    for index_type in (np.int32, np.int64):
+        dq, dkv = torch.full_like(qt, 9.0), torch.full((1, Skv, 1, D), 9.0, device=device)
+        ops.sparse_mla_backward(qt, kt, dt, to_dev(idx.astype(index_type), device), sm_scale=0.1, d_v=d_v, dq=dq, dkv=dkv)
+        for got, want, tol in ((dq, want_dq, 2 ** -8), (dkv, want_dkv, 1e-4)):         # dq is rounded to 8 bits once
+            err, ref = error_report(got.float().cpu().numpy(), want)
+            assert err <= tol * ref, (err, ref)
