@@ -894,8 +894,7 @@ __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const Ml
   const size_t blocks_total = (size_t)p.B * p.S * p.G * chunks * p.num_splits;
   const float* ml = (const float*)((const unsigned short*)p.workspace + blocks_total * (size_t)(HG * kPartFloats) * (F32 ? 2 : 1));
   const size_t block0 = unit * p.num_splits;
-  // all (max, sum) pairs first, then the partial rows four splits at a time, so that the loads
-  // of a group are in flight together (the split count is at most 16)
+  // all (max, sum) pairs first, then the partial rows (the split count is at most 16)
   float ms[16], ls[16];
   float m_all = -INFINITY;
 #pragma unroll
@@ -920,53 +919,57 @@ __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const Ml
   for (int i = 0; i < 4; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
   const unsigned short* src0 = (const unsigned short*)p.workspace + block0 * (size_t)(HG * kPartFloats) +
                                ((size_t)((w * HG + hg) * 8 + 2 * r4) * 64 + 32 * half + min(hd, max(heads_here - 32 * hg, 1) - 1)) * 8;   // (no traffic for heads past the end)
+  // Up to eight splits' loads are in flight together, each split's once.  (Four at a time, a last group filled up with repeats
+  // of the last split: 11.1 us where this takes 8.0 at 64 heads x 90 queries in 5 splits, 9.6 and 7.4 at 128 x 20 in 5; 6.1 and
+  // 4.8 at 4 queries x 128 heads in 16.  Tests between the loads instead of a switch make the compiler wait after each: 16 us.)
+  const auto gather = [&](auto group, auto first) {
+    constexpr int kGroup = decltype(group)::value, s0 = decltype(first)::value;
+    f32x4 v32[F32 ? kGroup : 1][4];
+    u32x4 raw[F32 ? 1 : kGroup][2];                           // two accumulator rows per 16-byte load
 #pragma unroll
-  for (int s0 = 0; s0 < 16; s0 += 4) {
-    if (s0 >= p.num_splits) break;                            // (uniform)
-    float4 v[4][4];
-    if constexpr (F32) {
-      const float* src = (const float*)p.workspace + (src0 - (const unsigned short*)p.workspace);
+    for (int u = 0; u < kGroup; ++u) {
+      const size_t at = (size_t)(s0 + u) * (HG * kPartFloats);
+      if constexpr (F32) {
+        const float* src = (const float*)p.workspace + (src0 - (const unsigned short*)p.workspace) + at;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int s = min(s0 + u, p.num_splits - 1);
+        for (int i = 0; i < 4; ++i) v32[u][i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + (size_t)(i >> 1) * 512 + (i & 1) * 4));
+      } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + (size_t)s * (HG * kPartFloats) + (size_t)(i >> 1) * 512 + (i & 1) * 4));
-          v[u][i] = make_float4(t[0], t[1], t[2], t[3]);
-        }
+        for (int i2 = 0; i2 < 2; ++i2)                        // (read once: non-temporal, 0.7 us of the decode step)
+          raw[u][i2] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src0 + at + (size_t)i2 * 512));
       }
-    } else {
-      uint4 raw[4][2];                                         // two accumulator rows per 16-byte load
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int s = min(s0 + u, p.num_splits - 1);             // a repeated last split gets weight 0
-#pragma unroll
-        for (int i2 = 0; i2 < 2; ++i2) {                          // (read once: non-temporal, 0.7 us of the decode step)
-          typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-          const u32x4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(src0 + (size_t)s * (HG * kPartFloats) + (size_t)i2 * 512));
-          raw[u][i2] = make_uint4(t[0], t[1], t[2], t[3]);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int i2 = 0; i2 < 2; ++i2) {
-          v[u][2 * i2] = make_float4(__uint_as_float(raw[u][i2].x << 16), __uint_as_float(raw[u][i2].x & 0xffff0000u),
-                                     __uint_as_float(raw[u][i2].y << 16), __uint_as_float(raw[u][i2].y & 0xffff0000u));
-          v[u][2 * i2 + 1] = make_float4(__uint_as_float(raw[u][i2].z << 16), __uint_as_float(raw[u][i2].z & 0xffff0000u),
-                                         __uint_as_float(raw[u][i2].w << 16), __uint_as_float(raw[u][i2].w & 0xffff0000u));
-        }
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const float f = (s0 + u < p.num_splits && ms[s0 + u] != -INFINITY) ? exp2f(ms[s0 + u] - m_fin) : 0.0f;
+    for (int u = 0; u < kGroup; ++u) {
+      const float f = (ms[s0 + u] != -INFINITY) ? exp2f(ms[s0 + u] - m_fin) : 0.0f;
       l_fin += ls[s0 + u] * f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        acc[i].x += v[u][i].x * f; acc[i].y += v[u][i].y * f; acc[i].z += v[u][i].z * f; acc[i].w += v[u][i].w * f;
+        float4 v;
+        if constexpr (F32) {
+          v = make_float4(v32[u][i][0], v32[u][i][1], v32[u][i][2], v32[u][i][3]);
+        } else {
+          const unsigned lo = raw[u][i >> 1][2 * (i & 1)], hi = raw[u][i >> 1][2 * (i & 1) + 1];
+          v = make_float4(__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u));
+        }
+        acc[i].x += v.x * f; acc[i].y += v.y * f; acc[i].z += v.z * f; acc[i].w += v.w * f;
       }
     }
-  }
+  };
+  const auto gather_of = [&](int n, auto first) {             // (n is uniform)
+    switch (n) {
+      case 1: gather(std::integral_constant<int, 1>{}, first); break;
+      case 2: gather(std::integral_constant<int, 2>{}, first); break;
+      case 3: gather(std::integral_constant<int, 3>{}, first); break;
+      case 4: gather(std::integral_constant<int, 4>{}, first); break;
+      case 5: gather(std::integral_constant<int, 5>{}, first); break;
+      case 6: gather(std::integral_constant<int, 6>{}, first); break;
+      case 7: gather(std::integral_constant<int, 7>{}, first); break;
+      default: gather(std::integral_constant<int, 8>{}, first); break;
+    }
+  };
+  gather_of(min(p.num_splits, 8), std::integral_constant<int, 0>{});
+  if (p.num_splits > 8) gather_of(p.num_splits - 8, std::integral_constant<int, 8>{});
   const float inv = l_fin > 0.0f ? 1.0f / l_fin : 0.0f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {                                // row 4*r4 + i = (dvb = r4, j = i)

@@ -910,3 +910,21 @@ def test_up_to_16_heads_add_scores_128_channels_at_a_time(device, rows):
     ops.sparse_mla_forward(q, kv, to_dev(idx.astype(np.int32), device), sm_scale=sm, d_v=512, out=out, lse=lse, kernel="mfma", **kw)
     _, want_lse = om.sparse_mla_oracle(qf, decoded, idx, sm_scale=sm, d_v=512)
     assert np.sqrt(np.mean((lse.cpu().numpy() - want_lse) ** 2)) <= 1.45e-6
+
+
+# 3 .. 16 splits with float32 sums; 2, 4, 7, 8 and 16 with bfloat16 sums
+@pytest.mark.parametrize("H,topk", [(16, 288 + 128 * i) for i in range(14)] + [(64, topk) for topk in (256, 512, 1056, 1024, 2048)])
+def test_merging_of_key_splits(device, H, topk):
+    """A split left out, taken twice or weighted by another's maximum is off by a share of the result near 1 / splits."""
+    Skv, sm = 2100, 0.1
+    rng = np.random.default_rng(H + topk)
+    q, qf = bf16_pair(rng.standard_normal((1, 1, H, 576)), device)
+    codes, scale, rope, rows = latent_cache(rng, 1, Skv, 1, 512, 64, device, pow2=True)
+    idx = rng.permutation(Skv)[:topk].reshape(1, 1, 1, topk)
+    idx[0, 0, 0, topk // 2] = -1
+    want_out, want_lse = om.sparse_mla_oracle(qf, rows, idx, sm_scale=sm, d_v=512)
+    out = torch.zeros((1, 1, H, 512), dtype=torch.float32, device=device)
+    lse = torch.zeros((1, 1, H), dtype=torch.float32, device=device)
+    bs.sparse_mla_blockscaled_path_c_apply(q, None, codes, scale, to_dev(idx.astype(np.int32), device), sm_scale=sm, d_v=512,
+                                           out=out, lse=lse, kv_rope=rope, kernel="mfma")
+    _assert_close(out, lse, want_out, want_lse, lse_tol=LSE_TOL_MFMA)
