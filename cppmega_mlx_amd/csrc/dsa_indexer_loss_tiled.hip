@@ -5,7 +5,7 @@
 // fills the CUs evenly, and no wavefront waits for another one's reductions:
 //
 //   dsa_loss_list_kernel    per row: membership bits of the index list, softmax statistics of the index scores (those
-//                           by the first pass where there are no lists, or its tiles leave CUs idle)
+//                           by workgroups of the first pass where that is faster)
 //   dsa_loss_tile_kernel<.., false>   per tile and head: sum of exp of the attention scores, per 64 keys
 //   dsa_loss_merge_kernel   per (head, row): log2 of the softmax denominator over all its keys
 //   dsa_loss_tile_kernel<.., true>    the scores again, p = mean over heads in registers, sum of p (log p - log q)
@@ -16,13 +16,14 @@
 // (causal, membership, additive) sit in registers as addends of the one multiply-add that scales a score,
 // and a lane reduces its own keys, so a head costs one lane exchange.
 //
-// Bound by the exponentials and the multiply-adds in front of them (two per pair and head).  Measured at
-// 4096 positions, 8 heads of 64, lists of 1024: 84 us a call (lists 20: 84 MB read; passes 23 and 27, merge and sum 9), 88
-// with whole tiles only, 274 with a workgroup of 8 wavefronts per 16 positions
+// Bound by the exponentials and the multiply-adds in front of them (two per pair and head; vector instructions fill 0.85 of
+// the time in which all CUs have tiles).  Measured at 4096 positions, 8 heads of 64, lists of 1024: 80 us a call (lists 20: 84 MB
+// read; passes 22 and 25, merge and sum 9), 84 with whole tiles only, 274 with a workgroup of 8 wavefronts per 16 positions
 // (256 workgroups, the longest with twice the mean work, statistics in LDS per step).  Short sequences are bound by a
 // workgroup's steps: 2 x 547 positions, 16 heads of 128 66 -> 34 us with split tiles, 943 x 8 x 128 44 -> 28.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "mfma_util.h"
@@ -178,8 +179,8 @@ __host__ __device__ inline long long tiles_before(long long n, long long key_til
 // GENERAL: an additive mask is given, or the softmax scale is not positive.  Otherwise the masks are 0 or -inf
 // and enter the first pass as what its products start from (a select behind them where a row that does not count
 // turned out not to be finite), and the second pass leaves keys that do not count out at its end.
-// Workgroups of the first pass between or behind those of the tiles take the statistics of the index scores, a row to a
-// wavefront (where, run() says).
+// Workgroups of the first pass behind those of the tiles take the statistics of the index scores, a row to a wavefront (when, run()
+// says).
 constexpr int resident(int AD, bool general) { return AD <= 64 && !general ? 4 : 2; }
 template <bool F16, int AD, int GROUPS, bool SECOND, bool GENERAL>
 __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_tile_kernel(const LossTiledParams p) {
@@ -194,22 +195,19 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
   constexpr int BLOCK = 64 * PITCH, ROWS = BLOCKS * BLOCK, MEET = SECOND && !WHOLE ? 2 * GROUPS * 32 * 64 / 4 : 0;
   __shared__ u32x4 rows[ROWS > MEET ? ROWS : MEET];
 
-  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int id = (int)blockIdx.x;
   if (!SECOND && p.stats_rows) {
-    // eights of workgroups (one per XCD) of tiles and of statistics: with lists in proportion, else all tiles first
-    const unsigned eight = (unsigned)id >> 3, stats_eights = (unsigned)(p.stats_groups + 7) >> 3, eights = gridDim.x >> 3;
-    const unsigned tile_eights = eights - stats_eights;
-    const unsigned before = p.topk_idx ? eight * stats_eights / eights : eight > tile_eights ? eight - tile_eights : 0;
-    if (p.topk_idx ? (eight + 1) * stats_eights / eights != before : eight >= tile_eights) {
-      const int row = ((int)before * 8 + (id & 7)) * (THREADS / 64) + wave;
+    // eights of workgroups, one per XCD: those of the tiles first
+    const unsigned eight = (unsigned)id >> 3, tile_eights = (gridDim.x >> 3) - ((unsigned)(p.stats_groups + 7) >> 3);
+    if (eight >= tile_eights) {
+      const int row = ((int)(eight - tile_eights) * 8 + (id & 7)) * (THREADS / 64) + wave;
       if (row < p.stats_rows) {
         const unsigned* bits = p.bits + (size_t)row * p.words;
         index_statistics<8>(p, row, [&](int j) { return p.topk_idx ? bits[j >> 5] >> (j & 31) : 15u; });
       }
       return;
     }
-    id -= (int)before * 8;
   }
   // Tile of this workgroup: the causal triangles of the batches, one after the other.  Consecutive workgroups go round the
   // eight XCDs, and each XCD takes one run of tiles, whose query rows (and the keys) its L2 holds.
@@ -234,10 +232,11 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
   }
   const int q0 = lo * kQ, k0 = (int)(of_all - tiles_before(lo, key_tiles)) * 128 + key_half * 64;
   if (k0 > q0 + 63 || k0 >= p.Sk) return;                 // (the second half of a tile on the diagonal, or at the end)
-  const int l32 = lane & 31, half = lane >> 5;
-  const int wq = (wave & 1) * 32, group = __builtin_amdgcn_readfirstlane(wave >> 1);
+  const int half = lane >> 5;
+  const unsigned l32 = lane & 31;
+  const int wq = (wave & 1) * 32, group = wave >> 1;
   const int kw = k0 + (split ? 0 : group * 64);          // the wavefront's first key
-  const int my_q = q0 + wq + l32;                         // the lane's position
+  const int my_q = q0 + wq + (int)l32;                         // the lane's position
   const bool live_q = my_q < p.ASq;
   const bool busy = kw <= q0 + wq + 31 && kw < p.Sk;      // the wavefront has a visible key
   const size_t row = (size_t)b * p.ASq + (live_q ? my_q : p.ASq - 1);
@@ -253,14 +252,15 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
   for (int i = 0; i < LOADS; ++i) {
     const int e = tid + i * THREADS, r = e / PIECES, c = e % PIECES;
     src[i] = (unsigned)r * pos_bytes + (unsigned)c * 16u;
-    dst[i] = r * PITCH + c;
+    dst[i] = THREADS % PIECES ? r * PITCH + c : tid / PIECES * PITCH + tid % PIECES + i * (THREADS / PIECES * PITCH);
   }
   u32x4 piece[BLOCKS][LOADS];
   float norm_next = 0.0f;
-  const float* norm_src = SECOND ? p.norm + (size_t)b * p.AH * p.slab_rows + (live_q ? my_q - p.slab0 : 0) : nullptr;
+  const int in_slab = q0 + wq - p.slab0;                  // a slab has whole tiles of positions
+  const float* norm_src = SECOND ? p.norm + (size_t)b * p.AH * p.slab_rows + in_slab : nullptr;
   // (first pass of split tiles, 64 channels: the last 64 rows are requested behind the products, whose operands need the registers)
   constexpr bool LATE = !SECOND && GROUPS == 2 && AD == 64;
-  auto fetch_rows = [&](int step, int from, int to) {     // rows of the blocks from .. to - 1
+  auto fetch_rows = [&](auto split, int step, int from, int to) {     // rows of the blocks from .. to - 1
 #pragma unroll
     for (int m = from; m < to; ++m) {
       const int h = split ? min(step * GROUPS + (m >> 1), p.AH - 1) : step;
@@ -272,13 +272,10 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
       }
     }
   };
-  auto fetch = [&](int step) {
-    fetch_rows(step, 0, LATE ? BLOCKS - 1 : BLOCKS);
-    if (SECOND) norm_next = norm_src[(size_t)(split ? min(step * GROUPS + group, p.AH - 1) : step) * p.slab_rows];
+  auto fetch = [&](auto split, int step) {
+    fetch_rows(split, step, 0, LATE ? BLOCKS - 1 : BLOCKS);
+    if (SECOND) norm_next = (norm_src + (size_t)(split ? min(step * GROUPS + group, p.AH - 1) : step) * p.slab_rows)[l32];
   };
-  fetch(0);
-  if (LATE) fetch_rows(0, BLOCKS - 1, BLOCKS);
-
   // register v of a 32-key block: key 8 * (v / 4) + 4 * half + v % 4
   float add[2][16];
   unsigned counts[2];                                     // bit 8 * (v / 4) + v % 4: whether key v counts
@@ -307,141 +304,143 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
 #pragma unroll
     for (int v = 0; v < 16; ++v) mean[t][v] = 0.0f;
 
-  const u32x4* const q_frag = rows + (split ? group : 0) * 2 * BLOCK + (wq + l32) * PITCH + half;
-  const u32x4* const k_frag = rows + (1 + (WHOLE ? group : 2 * group)) * BLOCK + l32 * PITCH + half;
-  for (int step = 0; step < steps; ++step) {
-    __syncthreads();                                      // the previous heads' rows are read
+  // (split is a constant in the loop: as a run-time value its branches met again in front of the products, and all rows of the
+  // step to come were waited for there)
+  auto heads = [&](auto split) {
+    const u32x4* const q_frag = rows + (split ? group : 0) * 2 * BLOCK + (wq + l32) * PITCH + half;
+    const u32x4* const k_frag = rows + (1 + (WHOLE ? group : 2 * group)) * BLOCK + l32 * PITCH + half;
+    fetch(split, 0);
+    if (LATE) fetch_rows(split, 0, BLOCKS - 1, BLOCKS);
+    for (int step = 0; step < steps; ++step) {
+      __syncthreads();                                      // the previous heads' rows are read
 #pragma unroll
-    for (int m = 0; m < BLOCKS; ++m)
-      if (WHOLE || m != 2 || split)
+      for (int m = 0; m < BLOCKS; ++m)
+        if (WHOLE || m != 2 || split)
 #pragma unroll
-        for (int i = 0; i < LOADS; ++i) rows[m * BLOCK + dst[i]] = piece[m][i];
-    const float norm = norm_next;
-    fetch(min(step + 1, steps - 1));
-    __syncthreads();
-    const int h = split ? step * GROUPS + group : step;
-    if (!busy || h >= p.AH) {                             // (uniform)
-      if (LATE) fetch_rows(min(step + 1, steps - 1), BLOCKS - 1, BLOCKS);
-      continue;
-    }
-    f32x16 s[2];
-    auto products = [&](bool masked) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) s[t][v] = masked ? add[t][v] : 0.0f;
-      if constexpr (AD > 64) {
-        // Of the larger heads the operands are read a step ahead of their products: a wavefront is alone with one or two others
-        // on its SIMD, and by itself the compiler waits for each (16 heads of 128, second pass, 272 tiles 36.5 -> 32.7 us, 1806
-        // tiles 71.8 -> 67.6; up to 64 channels there are no registers for it: 28.7 -> 36.1).
-        u32x4 qf[2], kf[2][2];
-        auto read = [&](int k) {
-          qf[k & 1] = q_frag[2 * k];
-#pragma unroll
-          for (int t = 0; t < 2; ++t) kf[k & 1][t] = k_frag[t * 32 * PITCH + 2 * k];
-        };
-        read(0);
-        read(1);
-#pragma unroll
-        for (int k = 0; k < STEPS; ++k) {
-#pragma unroll
-          for (int t = 0; t < 2; ++t) s[t] = product<F16>(kf[k & 1][t], qf[k & 1], s[t]);
-          if (k + 2 < STEPS) read(k + 2);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < STEPS; ++k) {
-          const u32x4 qf = q_frag[2 * k];
-#pragma unroll
-          for (int t = 0; t < 2; ++t) s[t] = product<F16>(k_frag[t * 32 * PITCH + 2 * k], qf, s[t]);
-        }
-      }
-    };
-    products(!SECOND && !GENERAL);
-    if (LATE) {
-      __builtin_amdgcn_sched_barrier(0);
-      fetch_rows(min(step + 1, steps - 1), BLOCKS - 1, BLOCKS);
-    }
-    // (exponentials first, sums behind them: a sum right behind its exponential waits for it)
-    if constexpr (SECOND) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) s[t][v] = exp2_(GENERAL ? fmaf(s[t][v], p.scale2, add[t][v]) - norm : fmaf(s[t][v], p.scale2, -norm));
-#pragma unroll
-        for (int v = 0; v < 16; ++v) mean[t][v] += s[t][v];
-      }
-    } else {
-      float m, sum;
-      auto statistics = [&]() {
-        m = -INFINITY;
+          for (int i = 0; i < LOADS; ++i) rows[m * BLOCK + dst[i]] = piece[m][i];
+      const float norm = norm_next;
+      fetch(split, min(step + 1, steps - 1));
+      __syncthreads();
+      const int h = split ? step * GROUPS + group : step;
+      const bool takes = busy && h < p.AH;                  // (uniform)
+      f32x16 s[2];
+      auto products = [&](bool masked) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            if (GENERAL) s[t][v] = add[t][v] > -INFINITY ? fmaf(s[t][v], p.scale2, add[t][v]) : -INFINITY;
-            m = fmaxf(m, s[t][v]);
+          for (int v = 0; v < 16; ++v) s[t][v] = masked ? add[t][v] : 0.0f;
+        if constexpr (AD > 64) {
+          // Of the larger heads the operands are read a step ahead of their products: a wavefront is alone with one or two others
+          // on its SIMD, and by itself the compiler waits for each (16 heads of 128, second pass, 272 tiles 36.5 -> 32.7 us, 1806
+          // tiles 71.8 -> 67.6; up to 64 channels there are no registers for it: 28.7 -> 36.1).
+          u32x4 qf[2], kf[2][2];
+          auto read = [&](int k) {
+            qf[k & 1] = q_frag[2 * k];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) kf[k & 1][t] = k_frag[t * 32 * PITCH + 2 * k];
+          };
+          read(0);
+          read(1);
+#pragma unroll
+          for (int k = 0; k < STEPS; ++k) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) s[t] = product<F16>(kf[k & 1][t], qf[k & 1], s[t]);
+            if (k + 2 < STEPS) read(k + 2);
+            __builtin_amdgcn_sched_barrier(0);
           }
-        m = fmaxf(m, xor32(m));
-        if (!GENERAL) m *= p.scale2;
-        // (the maximum comes off inside the multiply-add: a score rounded to float32 by itself is off by 2^-24 of its size,
-        // which made the loss's error 1.7 times as large for scores of a spread of 1.4 in base 2 and 4 times for one of 8)
-        const float at = m > -INFINITY ? m : 0.0f;
-        float d[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        } else {
+#pragma unroll
+          for (int k = 0; k < STEPS; ++k) {
+            const u32x4 qf = q_frag[2 * k];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) s[t] = product<F16>(k_frag[t * 32 * PITCH + 2 * k], qf, s[t]);
+          }
+        }
+      };
+      if (takes) products(!SECOND && !GENERAL);
+      if (LATE) {
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_rows(split, min(step + 1, steps - 1), BLOCKS - 1, BLOCKS);
+      }
+      if (!takes) continue;
+      // (exponentials first, sums behind them: a sum right behind its exponential waits for it)
+      if constexpr (SECOND) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
 #pragma unroll
-          for (int v = 0; v < 16; ++v) s[t][v] = exp2_(GENERAL ? s[t][v] - at : fmaf(s[t][v], p.scale2, -at));
+          for (int v = 0; v < 16; ++v) s[t][v] = exp2_(GENERAL ? fmaf(s[t][v], p.scale2, add[t][v]) - norm : fmaf(s[t][v], p.scale2, -norm));
 #pragma unroll
-          for (int v = 0; v < 16; ++v) d[v & 3] += s[t][v];
+          for (int v = 0; v < 16; ++v) mean[t][v] += s[t][v];
         }
-        sum = (d[0] + d[1]) + (d[2] + d[3]);
-        sum += xor32(sum);
-      };
-      statistics();
-      // -inf + x is NaN where x is not finite: the row of a key that does not count holds such values, or a row that
-      // counts does.  Only then the masks are applied behind the products.
-      if (!GENERAL && __ballot(!(sum == sum)) != 0ull) {
-        asm volatile("" ::: "memory");                    // (the operands are read again: kept from above, they would not fit)
-        products(false);
+      } else {
+        float m, sum;
+        auto statistics = [&]() {
+          m = -INFINITY;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+          for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) s[t][v] = add[t][v] == 0.0f ? s[t][v] : -INFINITY;
+            for (int v = 0; v < 16; ++v) {
+              if (GENERAL) s[t][v] = add[t][v] > -INFINITY ? fmaf(s[t][v], p.scale2, add[t][v]) : -INFINITY;
+              m = fmaxf(m, s[t][v]);
+            }
+          m = fmaxf(m, xor32(m));
+          if (!GENERAL) m *= p.scale2;
+          // (the maximum comes off inside the multiply-add: a score rounded to float32 by itself is off by 2^-24 of its size,
+          // which made the loss's error 1.7 times as large for scores of a spread of 1.4 in base 2 and 4 times for one of 8)
+          const float at = m > -INFINITY ? m : 0.0f;
+          float d[4];
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[t][v] = exp2_(GENERAL ? s[t][v] - at : fmaf(s[t][v], p.scale2, -at));
+#pragma unroll
+            for (int v = 0; v < 16; ++v) d[v & 3] = t == 0 && v < 4 ? s[t][v] : d[v & 3] + s[t][v];
+          }
+          sum = (d[0] + d[1]) + (d[2] + d[3]);
+          sum += xor32(sum);
+        };
         statistics();
+        // -inf + x is NaN where x is not finite: the row of a key that does not count holds such values, or a row that
+        // counts does.  Only then the masks are applied behind the products.
+        if (!GENERAL && __ballot(!(sum == sum)) != 0ull) {
+          asm volatile("" ::: "memory");                    // (the operands are read again: kept from above, they would not fit)
+          products(false);
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[t][v] = add[t][v] == 0.0f ? s[t][v] : -INFINITY;
+          statistics();
+          if (LATE) fetch_rows(split, min(step + 1, steps - 1), BLOCKS - 1, BLOCKS);   // (nor would these rows, kept over the above)
+        }
+        if (half == 0 && live_q) (p.part + ((size_t)(kw / kChunk) * p.AB * p.AH + (size_t)b * p.AH + h) * p.slab_rows + in_slab)[l32] = make_float2(m, sum);
       }
-      if (half == 0 && my_q - p.slab0 < p.slab_rows && live_q)
-        p.part[((size_t)(kw / kChunk) * p.AB * p.AH + (size_t)b * p.AH + h) * p.slab_rows + (my_q - p.slab0)] = make_float2(m, sum);
     }
-  }
+  };
+  if constexpr (WHOLE) heads(std::false_type{});
+  else if (GROUPS > 2) heads(std::true_type{});
+  else if (split) heads(std::true_type{});
+  else heads(std::false_type{});
   if (!SECOND) return;
 
   const float inv_heads = 1.0f / (float)p.AH, index_norm = p.index_norm[row];
-  const float* scores = p.index_scores + row * (size_t)p.Sk;
-  // keys 8 * g .. + 3 of block t, for which the heads' probabilities add up to `sums`
-  auto divergence = [&](int t, int g, const float (&sums)[4]) {
+  // Keys 8 * g .. + 3 of block t: their index scores, all requested before the first is looked at (with a branch around each
+  // quad and its loads the second pass took 1709 vector instructions a wavefront, half of them here, for 1365), ..
+  const Rows s_rows(reinterpret_cast<const char*>(p.index_scores + ((size_t)b * p.ASq + q0) * p.Sk), (unsigned)min(64, p.ASq - q0) * (unsigned)p.Sk * 4u);
+  const unsigned s_lane = ((unsigned)(my_q - q0) * (unsigned)p.Sk + (unsigned)(kw + 4 * half)) * 4u;
+  auto scores_of = [&](int t, int g) { return __builtin_bit_cast(f32x4, s_rows.load(s_lane + (t * 32 + 8 * g) * 4u, 0)); };
+  // .. and their divergence, the heads' probabilities adding up to `sums`.  Keys that do not count leave no trace: scores that
+  // are NaN have q = 0 (the maximum of NaN and -inf is -inf).
+  auto divergence = [&](int t, int g, const f32x4& scores, const float (&sums)[4]) {
+    const unsigned of_block = t ? counts[1] : counts[0];
     float kl = 0.0f;
-    const int key = kw + t * 32 + 8 * g + 4 * half;
-    if (!live_q || key > my_q || key >= p.Sk) return kl;
-    float iv[4];
-    if (key + 3 < p.Sk) {
-      const f32x4 x = *reinterpret_cast<const f32x4_any*>(scores + key);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) iv[i] = x[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) iv[i] = key + i < p.Sk ? scores[key + i] : 0.0f;
-    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      if (key + i > my_q || key + i >= p.Sk) continue;    // masked keys carry p = 0 and q = 0
-      const bool ok = ((t ? counts[1] : counts[0]) >> (8 * g + i)) & 1u;
-      const float pj = ok ? sums[i] * inv_heads : 0.0f;
-      float v = ok ? iv[i] * kLog2e : -INFINITY;
-      if (GENERAL && ok && p.mask) v = fmaf(iv[i], kLog2e, p.mask[row * (size_t)p.Sk + key + i] * kLog2e);
-      const float qj = v > -INFINITY ? exp2_(v - index_norm) : 0.0f;
-      kl += pj * (log2_(pj + kEps) - log2_(qj + kEps));
+      const bool ok = (of_block >> (8 * g + i)) & 1u;
+      float shift = -index_norm;
+      if (GENERAL && ok && p.mask) shift = fmaf(p.mask[row * (size_t)p.Sk + kw + t * 32 + 8 * g + 4 * half + i], kLog2e, shift);
+      const float pj = sums[i] * inv_heads, qj = exp2_(fmaxf(fmaf(scores[i], kLog2e, shift), -INFINITY));
+      const float with = fmaf(pj, log2_(pj + kEps) - log2_(qj + kEps), kl);
+      kl = ok ? with : kl;
     }
     return kl;
   };
@@ -450,6 +449,10 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
     if constexpr (!WHOLE) {
       // the groups of heads meet in LDS, and each finishes its share of the 32 registers
       constexpr int MINE = 32 / GROUPS;
+      const int t = group * MINE / 16, g0 = group * MINE % 16 / 4;
+      f32x4 scores[MINE / 4];
+#pragma unroll
+      for (int g = 0; g < MINE / 4; ++g) scores[g] = scores_of(t, g0 + g);
       float* const meet = reinterpret_cast<float*>(rows) + lane;               // [wavefront][register][lane]
       __syncthreads();
 #pragma unroll
@@ -457,7 +460,6 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
 #pragma unroll
         for (int v = 0; v < 16; ++v) meet[((wave * 2 + t) * 16 + v) * 64] = mean[t][v];
       __syncthreads();
-      const int t = group * MINE / 16, g0 = group * MINE % 16 / 4;
 #pragma unroll
       for (int g = 0; g < MINE / 4; ++g) {
         float sums[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -465,7 +467,7 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
         for (int of = 0; of < GROUPS; ++of)
 #pragma unroll
           for (int i = 0; i < 4; ++i) sums[i] += meet[(((of * 2 + (wave & 1)) * 2 + t) * 16 + 4 * (g0 + g) + i) * 64];
-        kl += divergence(t, g0 + g, sums);
+        kl += divergence(t, g0 + g, scores[g], sums);
       }
       kl += xor32(kl);
       __syncthreads();
@@ -478,17 +480,21 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
     }
   } else {
     if (!busy) return;
+    f32x4 scores[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) scores[t][g] = scores_of(t, g);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const float sums[4] = {mean[t][4 * g], mean[t][4 * g + 1], mean[t][4 * g + 2], mean[t][4 * g + 3]};
-        kl += divergence(t, g, sums);
+        kl += divergence(t, g, scores[t][g], sums);
       }
     kl += xor32(kl);
   }
-  if (half == 0 && live_q && my_q - p.slab0 < p.slab_rows)
-    p.kl[((size_t)(kw / kChunk) * p.AB + b) * p.slab_rows + (my_q - p.slab0)] = kl * kLn2;
+  if (half == 0 && live_q) (p.kl + ((size_t)(kw / kChunk) * p.AB + b) * p.slab_rows + in_slab)[l32] = kl * kLn2;
 }
 
 // 64 columns by 4 groups of chunks, met in LDS in order
@@ -596,16 +602,17 @@ int run(LossTiledParams p, hipStream_t stream) {
     const long long rest = all % round;
     return 16 * rest <= (p.topk_idx ? 7 : 9) * round ? all - rest : all;
   };
-  // The statistics of the index scores go with the tiles.  Dense: behind them, where they fill what the last round leaves idle, read
-  // memory beside exponentials and need no launch of their own (a kernel in front / between the tiles / behind them: 3300 positions x 16 heads
-  // of 64 74.8 / 76.8 / 69.6 us, 1800 x 2 x 16 of 128 77.2 / 80.9 / 71.9, 2400 x 8 of 128 49.9 / 50.1 / 45.6, 1800 x 8 of 64 29.9 / 29.7 / 26.7, 350
-  // 19.2 / 19.0 / 18.9; of 58 shapes three are slower, by 1 to 2 %).  With lists, whose kernel is there anyway: between the tiles where those are split, so
-  // that they do not fill the CUs, and leave room for them, which they do up to a fifth of a round (by themselves / with them, 8 heads of 64:
-  // 180 tiles 39.0 / 36.8 us, 242 40.0 / 41.4, 450 52.8 / 56.1; behind the tiles 8 heads are up to 6 % slower and 16 up to 5 % faster).  A workgroup of the
-  // larger heads keeps a CU or half of one (16 heads of 128: 64 tiles 38.8 / 35.1, 121 42.1 / 47.3, 225 56.3 / 67.2).
+  // The statistics of the index scores go behind the tiles, where they fill what the last round leaves idle and read memory beside
+  // exponentials.  Dense, they need no launch of their own then (a kernel in front / behind the tiles: 3300 positions x 16 heads of 64
+  // 74.8 / 69.6 us, 1800 x 2 x 16 of 128 77.2 / 71.9, 2400 x 8 of 128 49.9 / 45.6, 1800 x 8 of 64 29.9 / 26.7, 350 19.2 / 18.9; of
+  // 58 shapes three are slower, by 1 to 2 %).  With lists, whose kernel is there anyway, it takes enough to do beside them: 16 heads of 64 (1250
+  // positions 38.4 / 35.7 us, 1932 48.9 / 45.9, 3171 82.1 / 79.7, 4096 109.6 / 106.8; 22 lengths 1.03x in the mean, none more than 1.5 % slower;
+  // 8 heads 0.95 .. 1.05x), or split tiles that leave room for them, which they do up to a fifth of a round (8 heads of 64: 180 tiles
+  // 39.0 / 36.8 us, 242 40.0 / 41.4, 450 52.8 / 56.1).  A workgroup of the larger heads keeps a CU or half of one (16 heads of 128: 64 tiles
+  // 38.8 / 35.1, 121 42.1 / 47.3, 225 56.3 / 67.2; 300 .. 4096 positions of 8 0.98x in the mean, of 16 1.01x).
   const long long of_all_rows = tiles_before((p.ASq + kQ - 1) / kQ, key_tiles) * p.AB;
   const bool room = whole_of(of_all_rows) == 0 && (AD > 64 ? of_all_rows <= 64 : 5 * of_all_rows <= round);
-  const bool in_tiles = p.slab_rows >= p.ASq && (room || !p.topk_idx);
+  const bool in_tiles = p.slab_rows >= p.ASq && (!p.topk_idx || room || (AD <= 64 && p.AH >= 16));
   p.stats_rows = in_tiles ? (int)rows : 0;
   if (p.topk_idx || !in_tiles)
     hipLaunchKernelGGL(dsa_loss_list_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads), p.topk_idx ? 16 * (size_t)p.words : 0, stream, p);
@@ -642,6 +649,7 @@ bool dsa_indexer_loss_tiled_supports(const cppmega_mi355_dsa_loss_args_t& a) {
   if (a.head_dim != 32 && a.head_dim != 64 && a.head_dim != 96 && a.head_dim != 128) return false;
   if ((size_t)a.batch * a.heads * a.head_dim * 2 * 128 >= (1ull << 32)) return false;         // a tile's rows within 32-bit offsets
   if (a.batch > 65535 || (size_t)a.seq_q * a.batch == 0 || a.heads == 0 || a.seq_k == 0) return false;
+  if (a.seq_k >= 1 << 23) return false;                                                       // 64 rows of scores within 31-bit offsets
   return !a.topk_indices || a.seq_k <= 131072;
 }
 

@@ -282,3 +282,25 @@ def test_short_dense_losses_on_both_sides_of_the_one_launch_rule(shape):
     q, k, idx, top = _case(ASq + AH, ASq, AB, AH, AD, Sk, topk, torch.bfloat16)
     got = dsa_splitk_indexer_loss_per_position(idx.cuda(), None, q.cuda(), k.cuda(), AD ** -0.5, False).cpu().numpy()
     np.testing.assert_allclose(got, _want(q, k, idx, top, AD ** -0.5, False), atol=2e-5, rtol=2e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(330, 2, 6, 64, 330, 50), (330, 1, 16, 64, 341, 50), (330, 1, 3, 128, 330, 50), (2750, 1, 2, 64, 2750, 60)],
+                         ids=["split", "statistics_in_the_first_pass", "large_heads", "whole_tiles"])
+@pytest.mark.parametrize("sparse", [False, True])
+def test_index_scores_that_are_not_finite(shape, sparse):
+    """Scores that count and are -inf or NaN carry no probability; scores that no list names may be anything."""
+    ASq, AB, AH, AD, Sk, topk = shape
+    q, k, idx, top = _case(ASq + AH, ASq, AB, AH, AD, Sk, topk, torch.bfloat16)
+    member = torch.ones(idx.shape, dtype=torch.bool)
+    if sparse:
+        member = torch.zeros(idx.shape, dtype=torch.bool).scatter_(2, top, True)
+    draw = torch.rand(idx.shape, generator=torch.Generator().manual_seed(5))
+    gone = member & (draw < 0.05)
+    gone[..., 0] = False
+    bad = torch.where(gone, torch.where(draw < 0.02, float("nan"), float("-inf")), idx)
+    for i, value in enumerate((float("nan"), float("inf"), float("-inf"))):
+        bad[~member & (draw > 0.9 + 0.03 * i) & (draw <= 0.93 + 0.03 * i)] = value
+    got = dsa_splitk_indexer_loss_per_position(bad.cuda(), top.cuda(), q.cuda(), k.cuda(), AD ** -0.5, sparse).cpu().numpy()
+    clean = torch.where(gone, float("-inf"), idx)
+    np.testing.assert_allclose(got, _want(q, k, clean, top, AD ** -0.5, sparse), atol=2e-5, rtol=2e-4)
