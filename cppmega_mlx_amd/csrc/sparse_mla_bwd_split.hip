@@ -622,7 +622,7 @@ __global__ __launch_bounds__(64, 3) void bwd_dq_kernel(const SplitParams p) {
 // takes a quarter of the channels of all keys for dq, with dS of the other wavefronts out of LDS.  Eight
 // wavefronts: four quarters of the channels by two halves of the tiles of 32 keys, added at the end.
 // Measured against the two kernels: 79 queries x 8 heads x 160 of 7757 keys 25 -> 18 us, 512 x 64 x 256 of 2048 140 ->
-// 123, 1024 x 16 x 256 of 4096 70 -> 68.  Bound by the key rows' way from the L2 (604 MB, of a cache of 4.7 MB that is a
+// 120, 1024 x 16 x 256 of 4096 70 -> 67.  Bound by the key rows' way from the L2 (604 MB, of a cache of 4.7 MB that is a
 // little more than an XCD's L2) and by the phases of a workgroup, two of which share a CU (77 KB of LDS each): 5 us until
 // q, d_out and the first keys are there, 8 for the scores, 6 for statistics and planes, 9 for dq.  Neither half the
 // loads in flight nor q and d_out in registers made a difference to the large shape.
@@ -689,11 +689,11 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
   for (int i = 0; i < T; ++i)
 #pragma unroll
     for (int r = 0; r < 2; ++r) rows_at[i][r] = kv + (size_t)max(plain_key(slot_row[i][r]), 0) * key_step + col * 8;
-  auto request = [&](auto pair_c, auto stage_c) {      // a stage of tiles 2 * pair and 2 * pair + 1
+  auto request = [&](auto pair_c, auto stage_c, bool one, bool two) {      // a stage of tiles 2 * pair and 2 * pair + 1
     constexpr int pair = decltype(pair_c)::value, stage = decltype(stage_c)::value;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      if (wave + (2 * pair + j) * W < tiles)           // (uniform)
+      if (j ? two : one)                               // (uniform)
 #pragma unroll
         for (int q = 0; q < kStage; ++q)
           if (stage * kStage + q < kD / 64)
@@ -701,8 +701,8 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
             for (int r = 0; r < 2; ++r) queue[(pair * kStages + stage) & 1][j][q][r] = *reinterpret_cast<const u32x4*>(rows_at[2 * pair + j][r] + (stage * kStage + q) * 64);
   };
   using std::integral_constant;
-  request(integral_constant<int, 0>{}, integral_constant<int, 0>{});
-  request(integral_constant<int, 0>{}, integral_constant<int, 1>{});
+  request(integral_constant<int, 0>{}, integral_constant<int, 0>{}, wave < tiles, wave + W < tiles);
+  request(integral_constant<int, 0>{}, integral_constant<int, 1>{}, wave < tiles, wave + W < tiles);
 #pragma unroll
   for (int i = 0; i < kQLoads + kOLoads; ++i) {
     const bool of_q = i < kQLoads;
@@ -715,9 +715,9 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
   f32x4 s[T], dp[T];
   float m[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
   const unsigned short *qa = Qs + l16 * kDp + 8 * kg, *oa = Os + l16 * kDvp + 8 * kg;
-  auto score_pair = [&](auto pair_c) {
+  auto score_pair = [&](auto pair_c, auto two_c) {     // two: both of its tiles have keys
     constexpr int pair = decltype(pair_c)::value;
-    const bool two = wave + (2 * pair + 1) * W < tiles;               // (uniform)
+    constexpr bool two = decltype(two_c)::value;
     f32x4 sa[2], da[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) sa[j] = da[j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -732,24 +732,26 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
 #pragma unroll
               for (int r = 0; r < 2; ++r) *reinterpret_cast<u32x4*>(put[r] + (j * kStage + q) * 1024) = queue[(pair * kStages + stage) & 1][j][q][r];
       __builtin_amdgcn_wave_barrier();
-      if constexpr (stage < kStages - 2) request(pair_c, integral_constant<int, stage + 2>{});
-      else if constexpr (pair == 0) request(integral_constant<int, 1>{}, integral_constant<int, stage + 2 - kStages>{});
+      if constexpr (stage < kStages - 2) request(pair_c, integral_constant<int, stage + 2>{}, true, two);
+      else if constexpr (pair == 0 && two) request(integral_constant<int, 1>{}, integral_constant<int, stage + 2 - kStages>{}, wave + 2 * W < tiles, wave + 3 * W < tiles);
+      // (all of a stage's operands are read before its products, and whether there is a second tile is decided outside: with tests between
+      // the products each waited for its own operands; with dq's loop below 41 shapes 1.013x, up to 1.04)
+      constexpr int c0 = 2 * stage * kStage, steps = kD / 32 - c0 < 2 * kStage ? kD / 32 - c0 : 2 * kStage;       // of 32 channels
+      bf16x8 a[steps], o[steps], k[2][steps];
 #pragma unroll
-      for (int qu = 0; qu < 2 * kStage; ++qu) {
-        constexpr int c0 = 2 * stage * kStage;
-        const int c = c0 + qu, q = qu >> 1;              // of 32 channels
-        if (c >= kD / 32) continue;
-        const bf16x8 a = lds_b128(qa + c * 32), k0 = lds_b128(get[qu & 1] + q * 1024);
-        bf16x8 o = a, k1 = k0;
-        if (c < kDv / 32) o = lds_b128(oa + c * 32);
-        sa[0] = mm<F16>(a, k0, sa[0]);
-        if (c < kDv / 32) da[0] = mm<F16>(o, k0, da[0]);
-        if (two) {
-          k1 = lds_b128(get[qu & 1] + (kStage + q) * 1024);
-          sa[1] = mm<F16>(a, k1, sa[1]);
-          if (c < kDv / 32) da[1] = mm<F16>(o, k1, da[1]);
-        }
+      for (int qu = 0; qu < steps; ++qu) {
+        a[qu] = lds_b128(qa + (c0 + qu) * 32);
+        k[0][qu] = lds_b128(get[qu & 1] + (qu >> 1) * 1024);
+        if (two) k[1][qu] = lds_b128(get[qu & 1] + (kStage + (qu >> 1)) * 1024);
+        if (c0 + qu < kDv / 32) o[qu] = lds_b128(oa + (c0 + qu) * 32);
       }
+#pragma unroll
+      for (int qu = 0; qu < steps; ++qu)
+#pragma unroll
+        for (int j = 0; j < (two ? 2 : 1); ++j) {
+          sa[j] = mm<F16>(a[qu], k[j][qu], sa[j]);
+          if (c0 + qu < kDv / 32) da[j] = mm<F16>(o[qu], k[j][qu], da[j]);
+        }
       __builtin_amdgcn_wave_barrier();
     };
     stage_of(integral_constant<int, 0>{});
@@ -769,8 +771,10 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
       }
     }
   };
-  if (wave < tiles) score_pair(integral_constant<int, 0>{});
-  if (wave + 2 * W < tiles) score_pair(integral_constant<int, 1>{});
+  if (wave + W < tiles) score_pair(integral_constant<int, 0>{}, std::true_type{});
+  else if (wave < tiles) score_pair(integral_constant<int, 0>{}, std::false_type{});
+  if (wave + 3 * W < tiles) score_pair(integral_constant<int, 1>{}, std::true_type{});
+  else if (wave + 2 * W < tiles) score_pair(integral_constant<int, 1>{}, std::false_type{});
   const Stats stat = row_stats<W, T>(met, s, dp, m, wave, l16, kg, tiles);
   by_channel<W>(p, it, Qs, Os, kDp, kDvp, wave, l16, kg);
   // P and dS: planes for dkv, and dS for the other wavefronts
@@ -857,10 +861,14 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_scores_dq_kernel(const SplitPar
     }
     __builtin_amdgcn_wave_barrier();
   };
-  for (int step = first; step < steps; step += 2 * kTurns) {
-    turn(step, pre[0]);
-    if (step + kTurns < steps) turn(step + kTurns, pre[1]);
+  // (pairs without a branch between them: where a tile of pre[0] could follow another one the compiler would wait for all that is on
+  // its way)
+  const int turns = first < steps ? (steps - first + kTurns - 1) / kTurns : 0;
+  for (int pair = 0; pair < turns / 2; ++pair) {
+    turn(first + 2 * pair * kTurns, pre[0]);
+    turn(first + (2 * pair + 1) * kTurns, pre[1]);
   }
+  if (turns & 1) turn(first + (turns - 1) * kTurns, pre[0]);
   if (kTurns == 2) {
     if (first == 1)
 #pragma unroll
