@@ -32,6 +32,8 @@
 
 #include <string.h>
 
+#include <algorithm>
+
 #include "common.h"
 
 namespace cm {
@@ -229,10 +231,10 @@ constexpr int kStageBytes = 32 * 2 * kMaxD / 2;    // 8 KB per wavefront: 32 key
 constexpr int kCPitch = 68;                        // floats per row of the score tile in LDS (64 + 4: rows on distinct banks)
 static_assert(16 * kCPitch * 4 <= kStageBytes, "the score tile reuses the key tile");
 
-template <bool K_F32, int KSTEPS, int QT, bool STAGED = false>
+template <bool K_F32, int KSTEPS, int QT, bool STAGED = false, bool MASKED = false>
 __global__ __launch_bounds__(kThreads, 2) void indexer_scores_kernel(const IndexerParams p) {
   extern __shared__ __align__(16) unsigned short q_lds[];     // [2][16 QT][Dp + 8]: hi plane, lo plane; then the staging tiles
-  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bz = (int)blockIdx.z;
   const int b = p.b_begin + bz;
   const int s_off = kQRows * QT * (int)blockIdx.y;            // first query row of the workgroup within the pass
@@ -324,18 +326,17 @@ __global__ __launch_bounds__(kThreads, 2) void indexer_scores_kernel(const Index
     unsigned char* stage = reinterpret_cast<unsigned char*>(q_lds + 2 * kQRows * QT * pitch) + wave * kStageBytes;
     float* ctile = reinterpret_cast<float*>(stage);
     typedef __attribute__((ext_vector_type(4))) unsigned u4;
-    u4 kc[NT], kn[NT];
-    auto fetch_rows = [&](int key0, u4 (&buf)[NT]) {
+    u4 queue[NT];                                        // of a step: two halves of 32 rows
+    // The 64 rows of a step are one run of bytes, whose end the load unit checks: rows behind the last key read as zeros, and
+    // a step that does not exist (from key Skv on) moves nothing.
+    const auto rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>((const unsigned short*)p.k + (size_t)b * p.Skv * (32 * KSTEPS)), 0, p.Skv * (64 * KSTEPS), 0x00020000);
+    auto fetch_rows = [&](int key0, int half) {
+      const int at = key0 * (64 * KSTEPS) + lane * 16;
+      // one query tile per workgroup is the decode-time shape: every key row is read by one workgroup,
+      // once (non-temporal: 132 -> 121 us at 32 x 65536 keys); with more tiles the workgroups of a
+      // batch share the keys through the cache
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int P = lane + 64 * t, row = P / PPR, c = P % PPR;
-        const int key = min(key0 + row, p.Skv - 1);      // clamped: keys past the end are never stored
-        const u4* src = reinterpret_cast<const u4*>((const unsigned short*)p.k + ((size_t)b * p.Skv + (size_t)key) * D + 8 * c);
-        // one query tile per workgroup is the decode-time shape: every key row is read by one workgroup,
-        // once (non-temporal: 132 -> 121 us at 32 x 65536 keys); with more tiles the workgroups of a
-        // batch share the keys through the cache
-        buf[t] = QT == 1 ? __builtin_nontemporal_load(src) : *src;
-      }
+      for (int t = half * (NT / 2); t < (half + 1) * (NT / 2); ++t) queue[t] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rows, at + t * 1024, 0, QT == 1 ? 2 : 0));
     };
     int a_off[2][KSTEPS];                                // operand order inside a 32-row half: tile jj, step ks
 #pragma unroll
@@ -363,25 +364,39 @@ __global__ __launch_bounds__(kThreads, 2) void indexer_scores_kernel(const Index
           bq[qt][ks][1] = *reinterpret_cast<const bf16x8*>(&q_lo[(16 * qt + n) * pitch + d0]);
         }
     }
-    if (key_begin + 64 * wave < key_end) fetch_rows(key_begin + 64 * wave, kc);
+    const int first = __builtin_amdgcn_readfirstlane(key_begin + 64 * wave), last = __builtin_amdgcn_readfirstlane(key_end);
+    const int steps = first < last ? (last - first + kKeysPerIter - 1) / kKeysPerIter : 0;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      fetch_rows(steps > 0 ? first : p.Skv, half);
+      __builtin_amdgcn_sched_barrier(0);               // (in the order in which the loop waits for them)
+    }
     if constexpr (QT == 1) {
       if (own_sums) sum_rows();
     }
-    for (int key0 = key_begin + 64 * wave; key0 < key_end; key0 += kKeysPerIter) {
+    const auto tile_scores = __builtin_amdgcn_make_buffer_rsrc(p.scores + out_row0 * (size_t)p.s_pitch, 0, rows_here * p.s_pitch * 4, 0x00020000);
+    const int lane_score = ((lane >> 4) * p.s_pitch + 4 * (lane & 15)) * 4;
+    // Half a step's rows are requested as soon as its registers are in LDS.  No branch in the loop: behind one around the loads, or around
+    // a store, the compiler waits for all that is on its way.  With both, and a second set of registers for the next step:
+    // 3000 queries x 6000 keys 24.8 us, 21.7 here (18.4 with the plan of scores_keys), 32 batches of 65536 keys 91.9 for 89.7; calls
+    // of 21 batches of 14438 keys, selection included, 30.5 for 24.9.
+    for (int i = 0; i < steps; ++i) {
+      const int key0 = first + i * kKeysPerIter, next = i + 1 < steps ? key0 + kKeysPerIter : p.Skv;
       f32x4 acc[QT][4];
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[qt][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (key0 + kKeysPerIter < key_end) fetch_rows(key0 + kKeysPerIter, kn);
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         // rows 32 half .. 32 half + 31 of the step: registers -> LDS in load order (slot swizzled by the row)
 #pragma unroll
         for (int t = 0; t < NT / 2; ++t) {
           const int P = lane + 64 * t, row = P / PPR, c = P % PPR;      // position within the half
-          *reinterpret_cast<u4*>(stage + (row * PPR + (c ^ ((row / RP) % PPR))) * 16) = kc[half * (NT / 2) + t];
+          *reinterpret_cast<u4*>(stage + (row * PPR + (c ^ ((row / RP) % PPR))) * 16) = queue[half * (NT / 2) + t];
         }
+        fetch_rows(next, half);
+        __builtin_amdgcn_sched_barrier(0);             // (not behind the products)
 #pragma unroll
         for (int jj = 0; jj < 2; ++jj) {
           const int j = 2 * half + jj;
@@ -405,8 +420,6 @@ __global__ __launch_bounds__(kThreads, 2) void indexer_scores_kernel(const Index
           }
         }
       }
-#pragma unroll
-      for (int t = 0; t < NT; ++t) kc[t] = kn[t];
       // score tiles: lane (n, kg) holds query 16 qt + n, keys 16 j + 4 kg + i -> LDS [query][key] -> row segments
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
@@ -418,15 +431,16 @@ __global__ __launch_bounds__(kThreads, 2) void indexer_scores_kernel(const Index
           const int r = 16 * qt + 4 * u + (lane >> 4), col = 4 * (lane & 15);
           f32x4 v = *reinterpret_cast<const f32x4*>(ctile + (4 * u + (lane >> 4)) * kCPitch + col);
           const int key = key0 + col;
-          if (r < rows_here && key < key_end) {          // (the pitch is a multiple of 4: what a group of four has past Skv is nobody's)
-            if (p.mask) {
-              const size_t mrow = ((size_t)b * p.Sq + (size_t)(p.s_begin + s_off + r)) * p.Skv + key;
+          if (MASKED && r < rows_here) {
+            const size_t mrow = ((size_t)b * p.Sq + (size_t)(p.s_begin + s_off + r)) * p.Skv + key;
 #pragma unroll
-              for (int i = 0; i < 4; ++i)
-                if (key + i < p.Skv) v[i] += load_as(p.mask, mrow + i, p.mask_dtype);
-            }
-            *reinterpret_cast<f32x4*>(p.scores + (out_row0 + r) * (size_t)p.s_pitch + key) = v;
+            for (int i = 0; i < 4; ++i)
+              if (key + i < p.Skv) v[i] += load_as(p.mask, mrow + i, p.mask_dtype);
           }
+          // (rows and keys behind the end are out of the descriptor's range; the pitch is a multiple of 4: what a group of four has past Skv
+          // is nobody's)
+          const int at = key < last ? lane_score + ((16 * qt + 4 * u) * p.s_pitch + key0) * 4 : -1;
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), tile_scores, at, 0, 0);
         }
       }
     }
@@ -613,6 +627,29 @@ static bool scores_staged(const IndexerParams& p) {
   return p.k_dtype == CPPMEGA_MI355_BF16 && p.k_vec && p.s_vec && (p.D == 32 || p.D == 64 || p.D == 128);
 }
 
+// Keys of a workgroup.  Staged rows: workgroups come in rounds of 512 of two query tiles, two to a CU, or of 256 of one, which share
+// the key stream however many a CU has; a round lasts its steps and 0.8 or 0.45 of one more until the first rows are there.  Against
+// about 1024 workgroups for every shape (calls, selection included): 26 batches of 16382 keys 32.8 -> 28.9 us, 23 of 9819 24.8 -> 19.6, 19
+// of 21723 39.1 -> 35.2; 3000 queries x 6000 keys 56.4 -> 53.2, 1400 x 9000 52.0 -> 49.0, 3790 x 4210 56.7 -> 58.2; 67 shapes
+// 1.018x in the mean.  Other rows: about 1024 workgroups.
+static int scores_keys(const IndexerParams& p, int qt, int units) {
+  const int all = (p.Skv + kKeysPerIter - 1) / kKeysPerIter;
+  if (!scores_staged(p)) {
+    const int splits = std::min(std::max((1024 + units - 1) / units, 1), all);
+    return ((p.Skv + splits - 1) / splits + kKeysPerIter - 1) / kKeysPerIter * kKeysPerIter;
+  }
+  const int round = qt == 2 ? 512 : 256;
+  int best = 1;
+  float least = 0.0f;
+  for (int steps = 1; steps <= all; ++steps) {
+    const int splits = (all + steps - 1) / steps;
+    const float cost = (float)(((long long)splits * units + round - 1) / round) * ((float)steps + (qt == 2 ? 0.8f : 0.45f));
+    if (steps == 1 || cost < least) least = cost, best = steps;
+    if ((long long)splits * units <= round) break;           // (more steps only last longer)
+  }
+  return best * kKeysPerIter;
+}
+
 template <bool K_F32, int QT>
 static int launch_scores(const IndexerParams& p, dim3 grid, hipStream_t stream) {
   const size_t q_bytes = (size_t)2 * kQRows * QT * (((p.D + 31) & ~31) + 8) * sizeof(unsigned short);   // (two query tiles are only used up to D = 128: 17 KB)
@@ -620,9 +657,13 @@ static int launch_scores(const IndexerParams& p, dim3 grid, hipStream_t stream) 
   if constexpr (!K_F32) {
     if (scores_staged(p)) {
       const size_t lds = q_bytes + (size_t)(kThreads / 64) * kStageBytes;
-      const void* fn = ks == 1 ? (const void*)indexer_scores_kernel<false, 1, QT, true>
-                     : ks == 2 ? (const void*)indexer_scores_kernel<false, 2, QT, true>
-                               : (const void*)indexer_scores_kernel<false, 4, QT, true>;
+      const void* fn;
+      if (p.mask) fn = ks == 1 ? (const void*)indexer_scores_kernel<false, 1, QT, true, true>
+                     : ks == 2 ? (const void*)indexer_scores_kernel<false, 2, QT, true, true>
+                               : (const void*)indexer_scores_kernel<false, 4, QT, true, true>;
+      else fn = ks == 1 ? (const void*)indexer_scores_kernel<false, 1, QT, true>
+              : ks == 2 ? (const void*)indexer_scores_kernel<false, 2, QT, true>
+                        : (const void*)indexer_scores_kernel<false, 4, QT, true>;
       if (lds > 64 * 1024) CM_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
       IndexerParams q = p;
       void* kargs[] = {(void*)&q};
@@ -690,11 +731,7 @@ int indexer_topk_launch(const cppmega_mi355_indexer_args_t& a, hipStream_t strea
       }
       const int qt = (s_count >= 4 * kQRows && a.head_dim <= 128) ? 2 : 1;     // query tiles per workgroup (prefill: two)
       const int tiles = (s_count + kQRows * qt - 1) / (kQRows * qt);
-      const int max_splits = (a.seq_kv + kKeysPerIter - 1) / kKeysPerIter;
-      int splits = (1024 + tiles * nb - 1) / (tiles * nb);
-      splits = splits < 1 ? 1 : (splits > max_splits ? max_splits : splits);
-      const int per = (a.seq_kv + splits - 1) / splits;
-      p.keys_per_wg = (per + kKeysPerIter - 1) / kKeysPerIter * kKeysPerIter;
+      p.keys_per_wg = scores_keys(p, qt, tiles * nb);
       const dim3 grid((unsigned)((a.seq_kv + p.keys_per_wg - 1) / p.keys_per_wg), (unsigned)tiles, (unsigned)nb);
       if (a.k_dtype == CPPMEGA_MI355_F32) rc = qt == 2 ? launch_scores<true, 2>(p, grid, stream) : launch_scores<true, 1>(p, grid, stream);
       else rc = qt == 2 ? launch_scores<false, 2>(p, grid, stream) : launch_scores<false, 1>(p, grid, stream);

@@ -237,3 +237,31 @@ def test_few_query_rows_over_key_counts_off_four(device, B, Sq, H, D, Skv, topk)
         ops.indexer_topk(qt, kt, weights, sm_scale=0.125, topk=topk, out=out, ends=to_dev(ends, device))
         torch.cuda.synchronize()
         np.testing.assert_array_equal(out.cpu().numpy(), want)
+
+
+# bfloat16 keys of 32, 64 and 128 channels, several steps of 64 keys to a wavefront, the last ones short or missing
+@pytest.mark.parametrize("B,Sq,H,D,Skv", [(40, 1, 2, 32, 5003), (9, 20, 1, 64, 4100), (33, 3, 2, 128, 2052), (4, 1000, 1, 32, 2101), (2, 1500, 1, 64, 1600), (3, 700, 1, 128, 1990)])
+@pytest.mark.parametrize("mask", [None, torch.float32, torch.bfloat16, torch.float16], ids=["plain", "mask_f32", "mask_bf16", "mask_f16"])
+def test_many_steps_of_keys(device, B, Sq, H, D, Skv, mask):
+    """Selections, and scores kept in the caller's rows where those are whole fours, equal the oracle's on small integers; the keys
+    behind a batch's last one are another batch's, or nobody's."""
+    topk = 40
+    rng = np.random.default_rng(Skv + D)
+    q, k, w = _int_inputs(rng, B, Sq, H, D, Skv)
+    qt, kt, wt = (to_dev(a, device).bfloat16() for a in (q, k, w))
+    added = None
+    if mask is not None:
+        added = rng.integers(-4, 5, (B, Sq, Skv)).astype(np.float32)
+        added[rng.random(added.shape) < 0.1] = -np.inf
+    want = oi.indexer_scores_oracle(q, k, w, sm_scale=0.125).astype(np.float32)
+    if mask is not None:
+        want = want + added
+    out = torch.full((B, Sq, topk), -9, dtype=torch.int32, device=device)
+    kept = torch.full((B, Sq, Skv), 7.0, device=device) if Skv % 4 == 0 else None
+    ops.indexer_topk(qt, kt, wt, sm_scale=0.125, topk=topk, out=out, mask=None if mask is None else to_dev(added, device).to(mask), scores_out=kept)
+    torch.cuda.synchronize()
+    if kept is not None:
+        np.testing.assert_array_equal(kept.cpu().numpy(), want)
+    # (of equal scores the lower index)
+    chosen = np.sort(np.argsort(-want, axis=-1, kind="stable")[..., :topk], axis=-1)
+    np.testing.assert_array_equal(out.cpu().numpy(), chosen)
