@@ -11,9 +11,9 @@
 //    bytes per instruction and accumulated with v_dot2 (bf16 / fp16) or v_fma (fp32) in fp32 per
 //    128-wide scale block; a row pair's sums are reduced together across the wavefront.
 //  * M == 1, other K or misaligned rows (gemv_kernel): the same shape with bounds tests, fp32 math.
-//  * 5 <= M <= 16 bf16 / fp16 activations, K a multiple of 128 (skinny_rows_kernel): a workgroup owns up to
-//    32 weight rows for the whole K; weights converted to bf16 / fp16 in registers, v_mfma_f32_16x16x32 on
-//    the activations as they are; one kernel, no workspace.
+//  * 5 <= M <= 16 bf16 / fp16 activations, K a multiple of 128 (skinny_rows_kernel; N up to 4096 and K beyond
+//    2048: skinny_rows_long_kernel): a workgroup owns up to 32 or 16 weight rows for the whole K; weights converted
+//    to bf16 / fp16 in registers, v_mfma_f32_16x16x32 on the activations as they are; one kernel, no workspace.
 //  * M >= 17, K a multiple of 128: the tiled GEMM of fp8_gemm.hip.
 //  * anything else (odd K, misaligned rows): rowwise_kernel, one wavefront per
 //    output row, scalar byte loads.
@@ -393,6 +393,24 @@ __host__ __device__ constexpr int rows_waves(int) { return 8; }
 
 typedef _Float16 f16x8v __attribute__((ext_vector_type(8)));
 
+// acc += 8 channels of 16 weight rows, e4m3 codes lo and hi of a lane, by those of 16 activation rows
+template <bool F16>
+__device__ __forceinline__ f32x4 rows_product(unsigned lo, unsigned hi, const uint4& x, const f32x4& acc) {
+  uint4 a;
+  if (F16) {
+    a.x = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, false));
+    a.y = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, true));
+    a.z = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, false));
+    a.w = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, true));
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8v, a), __builtin_bit_cast(f16x8v, x), acc, 0, 0, 0);
+  }
+  a.x = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false));
+  a.y = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true));
+  a.z = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false));
+  a.w = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true));
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, x), acc, 0, 0, 0);
+}
+
 // F16: float16 activations (weights become float16 pairs, exact; v_mfma_f32_16x16x32_f16)
 template <int MT, bool F16 = false>
 __global__ __launch_bounds__(rows_waves(MT) * 64) void skinny_rows_kernel(const VecmatParams p) {
@@ -513,27 +531,8 @@ __global__ __launch_bounds__(rows_waves(MT) * 64) void skinny_rows_kernel(const 
           for (int mt = 0; mt < MT; ++mt) tile[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int s4 = 0; s4 < 4; ++s4) {             // MFMA step s4: channels 32 kg + 8 s4 .. + 7 of the block
-            uint4 a;
-            if (F16) {
-              a.x = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(wd[2 * s4], 1.0f, false));
-              a.y = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(wd[2 * s4], 1.0f, true));
-              a.z = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(wd[2 * s4 + 1], 1.0f, false));
-              a.w = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(wd[2 * s4 + 1], 1.0f, true));
-            } else {
-              a.x = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(wd[2 * s4], 1.0f, false));
-              a.y = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(wd[2 * s4], 1.0f, true));
-              a.z = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(wd[2 * s4 + 1], 1.0f, false));
-              a.w = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(wd[2 * s4 + 1], 1.0f, true));
-            }
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-              if (F16)
-                tile[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8v, a), __builtin_bit_cast(f16x8v, xb[mt][s4]),
-                                                                      tile[rt][mt], 0, 0, 0);
-              else
-                tile[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, xb[mt][s4]),
-                                                                       tile[rt][mt], 0, 0, 0);
-            }
+            for (int mt = 0; mt < MT; ++mt) tile[rt][mt] = rows_product<F16>(wd[2 * s4], wd[2 * s4 + 1], xb[mt][s4], tile[rt][mt]);
           }
         }
         // tile element i: weight row 16 rt + 4 kg + i, activation row 16 mt + r16
@@ -564,6 +563,111 @@ __global__ __launch_bounds__(rows_waves(MT) * 64) void skinny_rows_kernel(const 
       float sum = 0.0f;
 #pragma unroll
       for (int w = 0; w < kRowsWaves; ++w) sum += red[(w * 32 + r) * (16 * MT) + m];
+      store_as(p.out, (size_t)m * p.n + n0 + r, p.out_dtype, sum);
+    }
+  }
+}
+
+// The same for up to 16 weight rows a workgroup (N up to 4096) and K beyond 2048: one MFMA row tile, and 16 wavefronts, as there is
+// nothing else on the CU.  What counts is a wavefront's chain of blocks, so no load stands behind a branch: the compiler
+// waits for all that is on its way where its sides meet, and a block took a memory round trip (16 rows x 16000 channels x
+// 4000 20.0 -> 17.1 us, 5 x 16000 x 300 15.5 -> 11.6, 5 x 4096 x 2000 6.7 -> 5.4; the kernel above, which is
+// bound by the weight stream, is 0.83 .. 1.01 times as fast that way).  Rows that do not exist, of weights or activations, and blocks behind the last
+// one are outside the range of the loads' descriptors and move nothing.
+constexpr int kLongWaves = 16, kLongRows = 16, kLongWaveBytes = kLongRows * 128 + 16 * 256;      // tiles of a wavefront: weights, activations
+template <bool F16>
+__global__ __launch_bounds__(kLongWaves * 64) void skinny_rows_long_kernel(const VecmatParams p) {
+  constexpr int DEPTH = 3;                             // blocks in flight per wavefront (registers)
+  constexpr int kWTile = kLongRows * 128;
+  extern __shared__ __align__(16) unsigned char lds_b[];
+  const int KB = p.k / 128;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  unsigned char* stage = lds_b + wave * kLongWaveBytes;                               // this wavefront's tiles
+  float* sc = reinterpret_cast<float*>(lds_b + kLongWaves * kLongWaveBytes);          // [KB][16] block scales of the rows
+  float* red = reinterpret_cast<float*>(lds_b);                                       // [waves][16][16], reuses the tiles
+  const int r16 = lane & 15, kg = lane >> 4;
+  const int n0 = (int)blockIdx.x * p.rows_per_wg;
+  const int rows_here = min(p.rows_per_wg, p.n - n0);
+  const int per_wave = (KB + kLongWaves - 1) / kLongWaves;
+  const int kb_begin = wave * per_wave, kb_end = min(KB, kb_begin + per_wave);
+  const int nblk = max(kb_end - kb_begin, 0);
+  const int rot = nblk > 0 ? (int)((blockIdx.x * 5u) % (unsigned)nblk) : 0;
+  auto block_at = [&](int i) { const int j = i + rot; return kb_begin + (j >= nblk ? j - nblk : j); };
+
+  const auto w_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(p.w + (size_t)n0 * p.k), 0, rows_here * p.k, 0x00020000);
+  const auto x_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, p.m * p.k * 2, 0x00020000);
+  int woff[2], xoff[4], a_off[2], b_off[4];            // in load order, in operand order (as above)
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int pos = lane + 64 * j, row = pos >> 3, slot = pos & 7;
+    woff[j] = row * p.k + 16 * (slot ^ ((row >> 1) & 7));
+    a_off[j] = r16 * 128 + 16 * ((2 * kg + j) ^ ((r16 >> 1) & 7));
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int pos = lane + 64 * j, row = pos >> 4, slot = pos & 15;
+    xoff[j] = row * p.k * 2 + 16 * (slot ^ row);
+    b_off[j] = kWTile + r16 * 256 + 16 * ((4 * kg + j) ^ r16);
+  }
+  typedef __attribute__((ext_vector_type(4))) unsigned u4;
+  u4 wq[DEPTH][2], xq[DEPTH][4];
+  auto fetch = [&](int slot, int i) {
+    const int kb = i < nblk ? block_at(i) : 1 << 22;   // (behind the last block: 2^29 bytes on, of at most 2^22 that there are)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) wq[slot][j] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(w_rows, woff[j] + kb * 128, 0, 2));   // (non-temporal)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) xq[slot][j] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(x_rows, xoff[j] + kb * 256, 0, 0));
+  };
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) {
+    fetch(d, d);
+    __builtin_amdgcn_sched_barrier(0);                 // (in the order in which the loop waits for them)
+  }
+  // the block scales of this wavefront's run: written and read by this wavefront only
+  for (int e = lane; e < kLongRows * nblk; e += 64) {
+    const int r = e & 15, kb = kb_begin + (e >> 4);
+    sc[kb * kLongRows + r] = r < rows_here ? wscale(p, n0 + r, kb) : 0.0f;
+  }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  auto block = [&](int slot, int i, auto more) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) *reinterpret_cast<u4*>(stage + (lane + 64 * j) * 16) = wq[slot][j];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<u4*>(stage + kWTile + (lane + 64 * j) * 16) = xq[slot][j];
+    if constexpr (decltype(more)::value) {
+      fetch(slot, i + DEPTH);                          // refill the slot just emptied
+      __builtin_amdgcn_sched_barrier(0);               // (not behind the products)
+    }
+    const uint4 w0 = *reinterpret_cast<const uint4*>(stage + a_off[0]), w1 = *reinterpret_cast<const uint4*>(stage + a_off[1]);
+    const unsigned wd[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+    f32x4 tile = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4) {                   // MFMA step s4: channels 32 kg + 8 s4 .. + 7 of the block
+      const uint4 xb = *reinterpret_cast<const uint4*>(stage + b_off[s4]);
+      tile = rows_product<F16>(wd[2 * s4], wd[2 * s4 + 1], xb, tile);
+    }
+    const f32x4 s4v = *reinterpret_cast<const f32x4*>(sc + block_at(i) * kLongRows + 4 * kg);     // tile element e: weight row 4 kg + e
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = fmaf(s4v[e], tile[e], acc[e]);
+  };
+  int i = 0;
+  for (; i + DEPTH <= nblk; i += DEPTH)
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) block(d, i + d, std::true_type{});
+  static_assert(DEPTH == 3, "up to two blocks are left");
+  if (i < nblk) block(0, i, std::false_type{});
+  if (i + 1 < nblk) block(1, i + 1, std::false_type{});
+
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 4; ++e) red[(wave * 16 + 4 * kg + e) * 16 + r16] = acc[e];
+  __syncthreads();
+  if (tid < 256) {
+    const int m = tid >> 4, r = tid & 15;              // consecutive threads: consecutive output columns
+    if (m < p.m && r < rows_here) {
+      float sum = 0.0f;
+#pragma unroll
+      for (int w = 0; w < kLongWaves; ++w) sum += red[(w * 16 + r) * 16 + m];
       store_as(p.out, (size_t)m * p.n + n0 + r, p.out_dtype, sum);
     }
   }
@@ -631,6 +735,7 @@ static bool stream_shape(const cppmega_mi355_vecmat_args_t& a) { return stream_k
 // scales of 32 rows and partial tiles within the LDS
 constexpr int kRowsMaxM = 16;             // more activation rows: the tiled GEMM
 static size_t rows_lds_bytes(int k, int mt) { return (size_t)rows_waves(mt) * (32 * 128 + mt * 16 * 256) + (size_t)(k / 128) * 32 * sizeof(float); }
+static size_t long_lds_bytes(int k) { return (size_t)kLongWaves * kLongWaveBytes + (size_t)(k / 128) * kLongRows * sizeof(float); }      // (fits where the above does)
 static bool rows_shape(const cppmega_mi355_vecmat_args_t& a) {
   return (a.x_dtype == CPPMEGA_MI355_BF16 || a.x_dtype == CPPMEGA_MI355_F16) && a.m >= 5 && a.m <= kRowsMaxM && a.k % 128 == 0 &&
          rows_lds_bytes(a.k, 1) <= 160 * 1024;
@@ -765,12 +870,15 @@ int fp8_vecmat_launch(const cppmega_mi355_vecmat_args_t& a, hipStream_t stream) 
     rows = rows < 16 ? 16 : (rows > kRowsMax ? kRowsMax : rows);
     p.rows_per_wg = rows;
     const dim3 grid((unsigned)((a.n + rows - 1) / rows));
-    const size_t smem = rows_lds_bytes(a.k, 1);
-    const bool f16 = a.x_dtype == CPPMEGA_MI355_F16;
-    const void* fn = f16 ? (const void*)skinny_rows_kernel<1, true> : (const void*)skinny_rows_kernel<1, false>;
+    // (up to 2048 channels a wavefront of the long form has one block: 1200 and 2000 x 2048 as fast, 3100 4.9 us for 5.0; at 2176
+    // channels 1.02 to 1.16x, at 16000 1.17 to 1.43x)
+    const bool f16 = a.x_dtype == CPPMEGA_MI355_F16, lengthy = rows <= kLongRows && a.k > 2048;
+    const size_t smem = lengthy ? long_lds_bytes(a.k) : rows_lds_bytes(a.k, 1);
+    const void* fn = lengthy ? (f16 ? (const void*)skinny_rows_long_kernel<true> : (const void*)skinny_rows_long_kernel<false>)
+                             : (f16 ? (const void*)skinny_rows_kernel<1, true> : (const void*)skinny_rows_kernel<1, false>);
     if (smem > 64 * 1024) CM_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     void* kargs[] = {(void*)&p};
-    CM_HIP_CHECK(hipLaunchKernel(fn, grid, dim3(rows_waves(1) * 64), kargs, smem, stream));
+    CM_HIP_CHECK(hipLaunchKernel(fn, grid, dim3((lengthy ? kLongWaves : rows_waves(1)) * 64), kargs, smem, stream));
   } else if (aligned && stream_k(a)) {
     // more rows than one launch takes: passes over the weights (which the last-level cache may keep)
     const int cap = stream_row_cap(a.x_dtype);

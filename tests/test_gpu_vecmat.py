@@ -264,3 +264,26 @@ def test_tiled_gemm_with_less_workspace_than_asked_for(device, M, N, K, dtype):
         assert lib.cppmega_mi355_fp8_vecmat(C.byref(a), C.sizeof(a), _lib.current_stream(xd.device)) == _lib.OK
         assert (out.double().cpu() - want).abs().max() <= 2e-6 * want.abs().max()
         assert (ws[given:] == 0xff).all()
+
+
+# up to 4096 weight rows take the form with 16 rows to a workgroup: shares of one block, of three (no rest), of four with short and
+# empty ones behind, of seven; one weight row, one more than a workgroup's, the most, one more
+@pytest.mark.parametrize("M,N,K", [(5, 1, 2176), (16, 17, 6144), (9, 4096, 2176), (16, 4097, 2304), (7, 33, 6272), (13, 50, 12416), (6, 16, 98304)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_few_rows_over_long_k(device, M, N, K, dtype):
+    """Products are exact and sums are float32: the bar of the streaming kernels.  The bytes behind the weights and the activations,
+    which no row names, are not finite."""
+    rng = np.random.default_rng(M * N + K)
+    codes, scale = _weights(rng, N, K, pow2=False)
+    w = torch.full((N * K + 4096,), 0x7f, dtype=torch.uint8, device=device)
+    w[:N * K] = to_dev(codes, device).reshape(-1)
+    x = torch.full((M * K + 4096,), float("nan"), dtype=dtype, device=device)
+    x[:M * K] = torch.from_numpy(rng.standard_normal(M * K).astype(np.float32)).to(device).to(dtype)
+    xt = x[:M * K].view(M, K)
+    want = _oracle_blocked(codes, scale, xt.double().cpu().numpy())
+    out = torch.full((M + 1, N), 7.0, dtype=torch.float32, device=device)
+    vm.fp8_scaled_vecmat_path_c(xt, w[:N * K].view(N, K), scale_x=None, scale_w=to_dev(scale, device), out=out[:M])
+    torch.cuda.synchronize()
+    err, ref = error_report(out[:M].cpu().numpy(), want)
+    assert err <= F32_TOL * ref, (err, ref)
+    assert (out[M] == 7.0).all()
