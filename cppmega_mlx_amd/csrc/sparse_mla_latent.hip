@@ -871,16 +871,17 @@ __global__ __launch_bounds__(512, 2) void sparse_mla_latent_kernel(const MlaPara
 // Merges the key splits written by sparse_mla_latent_kernel.  A partial block holds, per
 // (consumer w = 128 value channels, 32-head block hg), 16 rows of 64 lanes x float4 exactly as the
 // accumulator registers held them: row 4*dvb + j, lane (head hd = lane%32, half = lane/32), element e
-// is channel 128w + 32dvb + 8j + 4half + e of head 32hg + hd.  One workgroup per (query, KV group,
-// head chunk, w, hg): coalesced 1 KiB row reads, weights per head, transposition through LDS,
+// is channel 128w + 32dvb + 8j + 4half + e of head 32hg + hd.  A wavefront per (query, KV group,
+// head chunk, w, hg, dvb): coalesced 1 KiB row reads, weights per head, transposition through LDS,
 // coalesced output rows.
-// F32: the partial values are float32 (and twice as long).  HG: 32-head blocks of a chunk.
-template <bool F32, int HG>
-__global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const MlaParams p) {
-  __shared__ float x[32][kXPitch];
-  const int tid = (int)threadIdx.x, lane = tid & 63, r4 = tid >> 6;
+// F32: the partial values are float32 (and twice as long).  HG: 32-head blocks of a chunk.  WAVES: values of dvb to a workgroup.
+template <bool F32, int HG, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void sparse_mla_latent_combine_kernel(const MlaParams p) {
+  __shared__ float x[32][32 * WAVES + 4];
+  constexpr int kParts = 4 / WAVES;
+  const int tid = (int)threadIdx.x, lane = tid & 63, part = (int)blockIdx.y % kParts, r4 = part * WAVES + (tid >> 6);
   const int chunks = (p.heads_per_group + 32 * HG - 1) / (32 * HG);
-  const int w = (int)blockIdx.y / HG, hg = (int)blockIdx.y % HG;
+  const int w = (int)blockIdx.y / (HG * kParts), hg = (int)blockIdx.y / kParts % HG;
   const size_t unit = blockIdx.x;                              // (b*S + s, g, chunk)
   const unsigned qg = blockIdx.x / (unsigned)chunks;           // (32-bit divisions: the 64-bit ones are long scalar chains)
   const int chunk = (int)(blockIdx.x - qg * (unsigned)chunks);
@@ -892,97 +893,87 @@ __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const Ml
   const int hd = lane & 31, half = lane >> 5;
   const int h_local = 32 * hg + hd;
   const size_t blocks_total = (size_t)p.B * p.S * p.G * chunks * p.num_splits;
-  const float* ml = (const float*)((const unsigned short*)p.workspace + blocks_total * (size_t)(HG * kPartFloats) * (F32 ? 2 : 1));
   const size_t block0 = unit * p.num_splits;
-  // all (max, sum) pairs first, then the partial rows (the split count is at most 16)
-  float ms[16], ls[16];
-  float m_all = -INFINITY;
-#pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    ms[s] = -INFINITY;
-    ls[s] = 0.0f;
-    if (s < p.num_splits) {
-      const float2 t = *reinterpret_cast<const float2*>(ml + ((block0 + s) * (32 * HG) + h_local) * 2);
-      ms[s] = t.x;
-      ls[s] = t.y;
-    }
-    m_all = fmaxf(m_all, ms[s]);
-  }
-  float m_fin = m_all, l_fin = 0.0f;
-  if (mla_has_sinks(p) && h_local < heads_here) {
-    const float sk = p.sinks[head0 + h_local] * kLog2e;
-    m_fin = fmaxf(m_all, sk);
-    l_fin = exp2f(sk - m_fin);
-  }
+  const float* ml = (const float*)((const unsigned short*)p.workspace + blocks_total * (size_t)(HG * kPartFloats) * (F32 ? 2 : 1)) +
+                    (block0 * (32 * HG) + h_local) * 2;
+  const unsigned short* src0 = (const unsigned short*)p.workspace + block0 * (size_t)(HG * kPartFloats) * (F32 ? 2 : 1) +
+                               ((size_t)((w * HG + hg) * 8 + 2 * r4) * 64 + 32 * half + min(hd, max(heads_here - 32 * hg, 1) - 1)) * (F32 ? 16 : 8);   // (no traffic for heads past the end)
+  const bool sinks = mla_has_sinks(p) && h_local < heads_here;
+  float sink = 0.0f;
+  if (sinks) sink = p.sinks[head0 + h_local];
   float4 acc[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  const unsigned short* src0 = (const unsigned short*)p.workspace + block0 * (size_t)(HG * kPartFloats) +
-                               ((size_t)((w * HG + hg) * 8 + 2 * r4) * 64 + 32 * half + min(hd, max(heads_here - 32 * hg, 1) - 1)) * 8;   // (no traffic for heads past the end)
-  // Up to eight splits' loads are in flight together, each split's once.  (Four at a time, a last group filled up with repeats
-  // of the last split: 11.1 us where this takes 8.0 at 64 heads x 90 queries in 5 splits, 9.6 and 7.4 at 128 x 20 in 5; 6.1 and
-  // 4.8 at 4 queries x 128 heads in 16.  Tests between the loads instead of a switch make the compiler wait after each: 16 us.)
-  const auto gather = [&](auto group, auto first) {
-    constexpr int kGroup = decltype(group)::value, s0 = decltype(first)::value;
-    f32x4 v32[F32 ? kGroup : 1][4];
-    u32x4 raw[F32 ? 1 : kGroup][2];                           // two accumulator rows per 16-byte load
-#pragma unroll
-    for (int u = 0; u < kGroup; ++u) {
-      const size_t at = (size_t)(s0 + u) * (HG * kPartFloats);
+  float m_fin = -INFINITY, l_fin = 0.0f;
+  // Bound by latency: code of its own for each number of splits, without a branch, so that the (max, sum) pairs and up to kDeep
+  // splits' sums are requested together, and each further split's as one is added.  (The pairs first, then up to eight splits, then the
+  // others, from one workgroup per 128 channels: 2 queries x 64 heads x 1558 codes 16.6 us the call, 13.4 here; 4 x 128 x 2048 latent 19.4 and
+  // 17.9; 20 x 128 x 1558 16-bit rows 30.6 and 29.3.  Four splits at a time: 32.7.)
+  const auto merge = [&](auto splits) {
+    constexpr int N = decltype(splits)::value, kDeep = F32 ? 8 : 16;
+    float2 stat[N];
+    f32x4 v32[F32 ? kDeep : 1][4];
+    u32x4 raw[F32 ? 1 : kDeep][2];                            // two accumulator rows per 16-byte load
+    const auto request = [&](int s) {                         // (read once: non-temporal, 0.7 us of the decode step)
+      const unsigned short* src = src0 + (size_t)s * (HG * kPartFloats) * (F32 ? 2 : 1);
       if constexpr (F32) {
-        const float* src = (const float*)p.workspace + (src0 - (const unsigned short*)p.workspace) + at;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v32[u][i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + (size_t)(i >> 1) * 512 + (i & 1) * 4));
+        for (int i = 0; i < 4; ++i) v32[s % kDeep][i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>((const float*)src + (size_t)(i >> 1) * 512 + (i & 1) * 4));
       } else {
 #pragma unroll
-        for (int i2 = 0; i2 < 2; ++i2)                        // (read once: non-temporal, 0.7 us of the decode step)
-          raw[u][i2] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src0 + at + (size_t)i2 * 512));
+        for (int i2 = 0; i2 < 2; ++i2) raw[s % kDeep][i2] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + (size_t)i2 * 512));
       }
+    };
+#pragma unroll
+    for (int s = 0; s < N; ++s) stat[s] = *reinterpret_cast<const float2*>(ml + s * (32 * HG) * 2);
+#pragma unroll
+    for (int s = 0; s < (N < kDeep ? N : kDeep); ++s) request(s);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < N; ++s) m_fin = fmaxf(m_fin, stat[s].x);
+    if (sinks) {
+      const float sk = sink * kLog2e;
+      m_fin = fmaxf(m_fin, sk);
+      l_fin = exp2f(sk - m_fin);
     }
 #pragma unroll
-    for (int u = 0; u < kGroup; ++u) {
-      const float f = (ms[s0 + u] != -INFINITY) ? exp2f(ms[s0 + u] - m_fin) : 0.0f;
-      l_fin += ls[s0 + u] * f;
+    for (int s = 0; s < N; ++s) {
+      const float f = (stat[s].x != -INFINITY) ? exp2f(stat[s].x - m_fin) : 0.0f;
+      l_fin += stat[s].y * f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float4 v;
         if constexpr (F32) {
-          v = make_float4(v32[u][i][0], v32[u][i][1], v32[u][i][2], v32[u][i][3]);
+          v = make_float4(v32[s % kDeep][i][0], v32[s % kDeep][i][1], v32[s % kDeep][i][2], v32[s % kDeep][i][3]);
         } else {
-          const unsigned lo = raw[u][i >> 1][2 * (i & 1)], hi = raw[u][i >> 1][2 * (i & 1) + 1];
+          const unsigned lo = raw[s % kDeep][i >> 1][2 * (i & 1)], hi = raw[s % kDeep][i >> 1][2 * (i & 1) + 1];
           v = make_float4(__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u));
         }
         acc[i].x += v.x * f; acc[i].y += v.y * f; acc[i].z += v.z * f; acc[i].w += v.w * f;
       }
+      if (s + kDeep < N) request(s + kDeep);
     }
   };
-  const auto gather_of = [&](int n, auto first) {             // (n is uniform)
-    switch (n) {
-      case 1: gather(std::integral_constant<int, 1>{}, first); break;
-      case 2: gather(std::integral_constant<int, 2>{}, first); break;
-      case 3: gather(std::integral_constant<int, 3>{}, first); break;
-      case 4: gather(std::integral_constant<int, 4>{}, first); break;
-      case 5: gather(std::integral_constant<int, 5>{}, first); break;
-      case 6: gather(std::integral_constant<int, 6>{}, first); break;
-      case 7: gather(std::integral_constant<int, 7>{}, first); break;
-      default: gather(std::integral_constant<int, 8>{}, first); break;
-    }
-  };
-  gather_of(min(p.num_splits, 8), std::integral_constant<int, 0>{});
-  if (p.num_splits > 8) gather_of(p.num_splits - 8, std::integral_constant<int, 8>{});
+#define CM_MERGE(n) case n: merge(std::integral_constant<int, n>{}); break;
+  switch (p.num_splits) {                                     // (uniform, at most 16)
+    CM_MERGE(1) CM_MERGE(2) CM_MERGE(3) CM_MERGE(4) CM_MERGE(5) CM_MERGE(6) CM_MERGE(7) CM_MERGE(8)
+    CM_MERGE(9) CM_MERGE(10) CM_MERGE(11) CM_MERGE(12) CM_MERGE(13) CM_MERGE(14) CM_MERGE(15)
+    default: merge(std::integral_constant<int, 16>{});
+  }
+#undef CM_MERGE
   const float inv = l_fin > 0.0f ? 1.0f / l_fin : 0.0f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {                                // row 4*r4 + i = (dvb = r4, j = i)
-    *reinterpret_cast<float4*>(&x[hd][32 * r4 + 8 * i + 4 * half]) =
+    *reinterpret_cast<float4*>(&x[hd][32 * (tid >> 6) + 8 * i + 4 * half]) =
         make_float4(acc[i].x * inv, acc[i].y * inv, acc[i].z * inv, acc[i].w * inv);
   }
   if (p.lse && w == 0 && r4 == 0 && half == 0 && h_local < heads_here)
     p.lse[bs * p.H + head0 + h_local] = l_fin > 0.0f ? (m_fin + log2f(l_fin)) * kLn2 : 0.0f;
   __syncthreads();
-  // thread -> head tid/8, 16 channels (tid%8)*16
-  const int row = tid >> 3, c0 = (tid & 7) * 16;
+  // 16 channels of a head to a thread
+  const int row = tid / (2 * WAVES), c0 = tid % (2 * WAVES) * 16;
   if (32 * hg + row < heads_here) {
-    const size_t off = (bs * p.H + head0 + 32 * hg + row) * (size_t)kLat + 128 * w + c0;
+    const size_t off = (bs * p.H + head0 + 32 * hg + row) * (size_t)kLat + 128 * w + 32 * WAVES * part + c0;
     float v[16];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -1000,6 +991,20 @@ __global__ __launch_bounds__(256) void sparse_mla_latent_combine_kernel(const Ml
       for (int i = 0; i < 16; ++i) store_as(p.out, off + i, p.out_dtype, v[i]);
     }
   }
+}
+
+template <bool F32, int HG>
+int launch_combine(const MlaParams& p, hipStream_t stream) {
+  const size_t units = (size_t)p.B * p.S * p.G * ((p.heads_per_group + 32 * HG - 1) / (32 * HG));
+  // A workgroup of four wavefronts per 128 channels where that fills half of the CUs: below, a CU's loads bound it and one wavefront to a
+  // workgroup gets more of them (1 query x 16 heads x 2048 latent keys in 16 splits 14.9 -> 13.1 us, 2 x 64 x 1558 codes 16.0 -> 13.4, 4 x 128 x 2048
+  // latent 19.1 -> 17.9); above, it is the same or up to 0.6 us slower (60 x 16 x 2048 26.3 -> 26.9).
+  if (units * HG * 4 <= 128)
+    hipLaunchKernelGGL((sparse_mla_latent_combine_kernel<F32, HG, 1>), dim3((unsigned)units, 16 * HG), dim3(64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((sparse_mla_latent_combine_kernel<F32, HG, 4>), dim3((unsigned)units, 4 * HG), dim3(256), 0, stream, p);
+  CM_HIP_CHECK(hipGetLastError());
+  return 0;
 }
 
 }  // namespace
@@ -1096,20 +1101,13 @@ int sparse_mla_latent_launch(const MlaParams& p, hipStream_t stream) {
   CM_HIP_CHECK(hipGetLastError());
   if (p.num_splits > 1) {
     if (f32_partials(p)) return sparse_mla_combine_f32(p, stream);
-    const dim3 cgrid((unsigned)((size_t)p.B * p.S * p.G * chunks), (unsigned)(4 * (kHeadsWg / 32)));
-    hipLaunchKernelGGL((sparse_mla_latent_combine_kernel<false, 2>), cgrid, dim3(256), 0, stream, p);
-    CM_HIP_CHECK(hipGetLastError());
+    return launch_combine<false, 2>(p, stream);
   }
   return 0;
 }
 
 int sparse_mla_combine_f32(const MlaParams& p, hipStream_t stream) {
-  const int chunks = (p.heads_per_group + p.heads_per_wg - 1) / p.heads_per_wg;
-  const dim3 grid((unsigned)((size_t)p.B * p.S * p.G * chunks), (unsigned)(4 * (p.heads_per_wg / 32)));
-  if (p.heads_per_wg == 64) hipLaunchKernelGGL((sparse_mla_latent_combine_kernel<true, 2>), grid, dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL((sparse_mla_latent_combine_kernel<true, 1>), grid, dim3(256), 0, stream, p);
-  CM_HIP_CHECK(hipGetLastError());
-  return 0;
+  return p.heads_per_wg == 64 ? launch_combine<true, 2>(p, stream) : launch_combine<true, 1>(p, stream);
 }
 
 size_t sparse_mla_latent_workspace_bytes(const MlaParams& p) {

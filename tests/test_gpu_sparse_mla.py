@@ -928,3 +928,21 @@ def test_merging_of_key_splits(device, H, topk):
     bs.sparse_mla_blockscaled_path_c_apply(q, None, codes, scale, to_dev(idx.astype(np.int32), device), sm_scale=sm, d_v=512,
                                            out=out, lse=lse, kv_rope=rope, kernel="mfma")
     _assert_close(out, lse, want_out, want_lse, lse_tol=LSE_TOL_MFMA)
+
+
+# one wavefront to a workgroup of the merge up to 128 workgroups of four, four from there on: 16 heads (float32 sums) in 4 pieces of
+# 128 channels, 64 heads (bfloat16 sums) in 8
+@pytest.mark.parametrize("S,H,topk", [(32, 16, 512), (33, 16, 1100), (16, 64, 1024), (17, 64, 1024)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_merging_of_key_splits_of_many_queries(device, S, H, topk, out_dtype):
+    Skv, sm = 1300, 0.1
+    rng = np.random.default_rng(S + H + topk)
+    q, qf = bf16_pair(rng.standard_normal((1, S, H, 576)), device)
+    codes, scale, rope, rows = latent_cache(rng, 1, Skv, 1, 512, 64, device, pow2=True)
+    idx = np.stack([rng.permutation(Skv)[:topk] for _ in range(S)]).reshape(1, S, 1, topk)
+    want_out, want_lse = om.sparse_mla_oracle(qf, rows, idx, sm_scale=sm, d_v=512)
+    out = torch.zeros((1, S, H, 512), dtype=out_dtype, device=device)
+    lse = torch.zeros((1, S, H), dtype=torch.float32, device=device)
+    bs.sparse_mla_blockscaled_path_c_apply(q, None, codes, scale, to_dev(idx.astype(np.int32), device), sm_scale=sm, d_v=512,
+                                           out=out, lse=lse, kv_rope=rope, kernel="mfma")
+    _assert_close(out, lse, want_out, want_lse, lse_tol=LSE_TOL_MFMA)
