@@ -7,7 +7,7 @@
 // 128 bytes of a row: such loads reach 50 B/clk a CU, pieces of 64 bytes 28, of 16 bytes 10), as many stages ahead as the
 // LDS holds.  Measured (microseconds a call; through registers, two stages ahead -> here), M x N x K:
 // 2048 x 8192 x 1536: 65 -> 59, 2048 x 7168 x 16384: 483 -> 441 = 1090 TFLOP/s, 1040 x 2621 x 5248: 58 -> 43,
-// 879 x 1007 x 6528: 48 -> 24, 231 x 4895 x 10240: 54 -> 38, 32 x 7168 x 16384: 37 -> 28, 55 x 2804 x 640: 7.6 -> 5.7.
+// 879 x 1007 x 6528: 48 -> 24, 231 x 4895 x 10240: 54 -> 38, 32 x 7168 x 16384: 29.0 -> 25.8, 55 x 2804 x 640: 7.6 -> 5.7.
 // What bounds it: a large product, the LDS (of 2048 clocks of products a 128 x 256 x 128 step, operand reads and arriving
 // rows take as many at 128 B/clk) and the vector instructions between the products; a small one, launch, first loads and
 // stores (5 us); a small batch, the weights' stream.
@@ -92,6 +92,7 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
   const int blocks = p.k / 128;
   const int b0 = (int)((long long)blocks * blockIdx.y / p.k_splits), b1 = (int)((long long)blocks * (blockIdx.y + 1) / p.k_splits);
   const int stages = (b1 - b0 + WK - 1) / WK;
+  int turned = 0;                                                    // the stage it begins with (two groups)
 
   // Rows and columns of tile e.  Consecutive workgroups go round the eight XCDs: every XCD takes one run of
   // the order (groups of eight column tiles; inside, row tile by row tile), so that its L2 holds the
@@ -115,11 +116,16 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
   auto start = [&]() {
     int m0, n0;
     place(next_e, m0, n0);
-    xbase = reinterpret_cast<const char*>(p.x) + ((size_t)m0 * p.k + (size_t)b0 * 128) * 2;
-    wbase = reinterpret_cast<const char*>(p.w) + (size_t)n0 * p.k + (size_t)b0 * 128;
+    // Column tiles begin at different places of K and go round: where rows are a power of two of bytes apart, workgroups in step
+    // ask the same memory channels (20 x 7168 x 16384 30.5 -> 25.9 us, as the last step of a decode layer 33 -> 28; 30 x 4096 x 14336
+    // 17 -> 15.7).  Only while an XCD's L2 holds the activations, whose tiles are then read at different times: with row
+    // tiles that fetched their weights at different times 1388 x 1098 x 9472 took 60 us for 43.
+    if (WK == 2 && (size_t)p.m * p.k * 2 <= (2u << 20)) turned = (int)((unsigned)(n0 / BN) * 5u % (unsigned)stages);
+    next_b = b0 + turned * WK;
+    xbase = reinterpret_cast<const char*>(p.x) + ((size_t)m0 * p.k + (size_t)next_b * 128) * 2;
+    wbase = reinterpret_cast<const char*>(p.w) + (size_t)n0 * p.k + (size_t)next_b * 128;
     const int first = n0 >> p.srow_shift;
-    sbase = reinterpret_cast<const char*>(p.scale_w) + ((size_t)first * p.srow_stride + (size_t)b0 * p.scol_stride) * 4;
-    next_b = b0;
+    sbase = reinterpret_cast<const char*>(p.scale_w) + ((size_t)first * p.srow_stride + (size_t)next_b * p.scol_stride) * 4;
 #pragma unroll
     for (int i = 0; i < XL; ++i) {
       const int u = wave * XL + i, plane = u & 1, rg = (u >> 1) / WK;
@@ -139,6 +145,13 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
   auto load16 = [&](const char* base, unsigned off, unsigned to) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory", "m0");
   };
+  // Weights that one row tile reads, of a size that the last-level cache (256 MB) does not keep for the next call beside what else a
+  // program runs: non-temporal, so that they push nothing out (20 x 7168 x 16384 25.9 -> 24.4 us, a decode layer of 18 to 32 sequences
+  // 3 to 5 us).  Smaller ones may still be there (three takes in turn of 30 x 4096 x 14336 15.7 / 17.7 us, of 24 x 10000 x 2048 9.9 / 11.6).
+  const bool once = tiles_m == 1 && (size_t)p.n * p.k >= (64u << 20);
+  auto load16_once = [&](const char* base, unsigned off, unsigned to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(to), "v"(off), "s"(base) : "memory", "m0");
+  };
   auto load4 = [&](const char* base, unsigned off, unsigned to) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory", "m0");
   };
@@ -149,7 +162,10 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
     const bool pair = WK == 1 || next_b + 1 < b1;
     if (i < WL) {
       const int u = wave * WL + i, g = u % WK, rg = u / WK;
-      load16(wbase + (pair ? g * 128 : 0), woff[i], next_slot + (unsigned)(T::kX + (g * BN + rg * 8) * 128));
+      const char* const at = wbase + (pair ? g * 128 : 0);
+      const unsigned to = next_slot + (unsigned)(T::kX + (g * BN + rg * 8) * 128);
+      if (BM == 32 && once) load16_once(at, woff[i], to);
+      else load16(at, woff[i], to);
     } else if (i < XL + WL) {
       const int u = wave * XL + i - WL, plane = u & 1, g = (u >> 1) % WK, rg = (u >> 1) / WK;
       load16(xbase + (pair ? g * 256 : 0), xoff[i - WL], next_slot + (unsigned)(((g * 2 + plane) * BM + rg * 8) * 128));
@@ -161,6 +177,12 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
       next_b += WK;
       --left;
       next_slot = next_slot + T::kStage == lds_base + SLOTS * T::kStage ? lds_base : next_slot + T::kStage;
+      if (WK == 2 && next_b >= b1) {
+        next_b = b0;
+        xbase -= (size_t)stages * (WK * 256);
+        wbase -= (size_t)stages * (WK * 128);
+        sbase -= (size_t)stages * WK * p.scol_stride * 4;
+      }
       if (T::PERSIST && next_b >= b1 && left > 0) {
         next_e += (int)gridDim.x;
         start();
@@ -249,7 +271,8 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
       }
       __builtin_amdgcn_sched_barrier(0);
       multiply(1, 1, more);
-      if (WK == 1 || b0 + s * WK + wk < b1) {
+      const int at = s + turned < stages ? s + turned : s + turned - stages;
+      if (WK == 1 || b0 + at * WK + wk < b1) {
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -327,19 +350,18 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
 
 // out[m][n] = sum over the K splits of partial[split][m][n], in split order.  Bound by latency (7 MB at 32 x 7168 x 8
 // splits): with the splits' loads one after the other and stores of single values a call took 2 to 3 us longer.  Splits
-// begin at whole 16-byte pieces, so that products of odd sizes are read alike (19 x 333 of 16 splits: 12 -> 4 us).
+// begin at whole 16-byte pieces, so that products of odd sizes are read alike (19 x 333 of 16 splits: 12 -> 4 us).  Code of
+// its own for each number of splits: with a test in front of each load the first was waited for before the others were asked for.
+template <int SPLITS>
 __global__ __launch_bounds__(256) void fp8_gemm_reduce_kernel(const VecmatParams p) {
   const size_t total = (size_t)p.m * p.n, step = split_step(p.m, p.n);
-  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= total) return;
-  // (the loads of the up to 16 splits are in flight together)
-  f32x4 part[16], s = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 part[SPLITS], s = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int z = 0; z < 16; ++z)
-    if (z < p.k_splits) part[z] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.partial + (size_t)z * step + i));
+  for (int z = 0; z < SPLITS; ++z) part[z] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.partial + (size_t)z * step + i));
 #pragma unroll
-  for (int z = 0; z < 16; ++z)
-    if (z < p.k_splits) s += part[z];
+  for (int z = 0; z < SPLITS; ++z) s += part[z];
   if (i + 4 <= total && p.out_dtype != CPPMEGA_MI355_F32 && ((uintptr_t)p.out & 7) == 0) {
     const bool bf16 = p.out_dtype == CPPMEGA_MI355_BF16;
     *reinterpret_cast<uint2*>((unsigned short*)p.out + i) = bf16 ? make_uint2(pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3]))
@@ -420,6 +442,23 @@ void launch_as(int m, int n, hipStream_t stream, const VecmatParams& p) {
   else hipLaunchKernelGGL((fp8_gemm_kernel<T, false>), grid, block, 0, stream, p);
 }
 
+void launch_reduce(const VecmatParams& p, hipStream_t stream) {
+  const size_t quads = ((size_t)p.m * p.n + 3) / 4;
+  const unsigned threads = quads <= 65536 ? 64 : 256;
+  const dim3 grid((unsigned)((quads + threads - 1) / threads)), block(threads);
+  switch (p.k_splits) {                                         // (one of kSplits)
+    case 2: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<2>, grid, block, 0, stream, p); break;
+    case 3: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<3>, grid, block, 0, stream, p); break;
+    case 4: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<4>, grid, block, 0, stream, p); break;
+    case 5: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<5>, grid, block, 0, stream, p); break;
+    case 6: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<6>, grid, block, 0, stream, p); break;
+    case 8: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<8>, grid, block, 0, stream, p); break;
+    case 10: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<10>, grid, block, 0, stream, p); break;
+    case 12: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<12>, grid, block, 0, stream, p); break;
+    default: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<16>, grid, block, 0, stream, p); break;
+  }
+}
+
 }  // namespace
 
 // bf16 / fp16 activations, whole 128-channel blocks, more rows than the kernels without staging take
@@ -451,8 +490,7 @@ int fp8_gemm_launch(VecmatParams p, size_t workspace_bytes, hipStream_t stream) 
   }
   CM_HIP_CHECK(hipGetLastError());
   if (g.splits > 1) {
-    const size_t quads = ((size_t)p.m * p.n + 3) / 4;
-    hipLaunchKernelGGL(fp8_gemm_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, p);
+    launch_reduce(p, stream);
     CM_HIP_CHECK(hipGetLastError());
   }
   return 0;

@@ -287,3 +287,19 @@ def test_few_rows_over_long_k(device, M, N, K, dtype):
     err, ref = error_report(out[:M].cpu().numpy(), want)
     assert err <= F32_TOL * ref, (err, ref)
     assert (out[M] == 7.0).all()
+
+
+# column tiles begin at different places of K and go round: odd numbers of blocks (the last stage of two holds one, and is anywhere in
+# the order), with and without K splits, one stage; weights of 64 MB and more, which are read past the cache, one column short of it and not
+@pytest.mark.parametrize("M,N,K", [(20, 1030, 1664), (32, 700, 896), (17, 2500, 3200), (64, 520, 6528), (31, 260, 128), (40, 3000, 384),
+                                   (19, 4095, 16384), (19, 4096, 16384), (33, 4100, 16384)])
+def test_tiled_gemm_starts_anywhere_in_k(device, M, N, K):
+    gen = torch.Generator(device=device).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=gen, device=device).to(torch.bfloat16)
+    codes = torch.randn((N, K), generator=gen, device=device).mul(2).to(torch.float8_e4m3fn)
+    scale = torch.rand((N, K // 128), generator=gen, device=device) + 0.5
+    want = x.double() @ (codes.double() * scale.double().repeat_interleave(128, dim=1)).T
+    out = torch.empty((M, N), dtype=torch.float32, device=device)
+    vm.fp8_scaled_vecmat_path_c(x, codes.view(torch.uint8), scale_x=None, scale_w=scale, out=out)
+    # (as for the other tiles)
+    assert (out.double() - want).abs().max() <= 2e-6 * want.abs().max()
