@@ -55,6 +55,7 @@ struct TopkParams {
   int* out;
   int rows, width, k, order, neg_inf_masked;
   int first_past;  // rows from here on end less than a whole piece of four columns in front of the buffer's end
+  bool eager;    // few scores in all: see topk_tile_kernel
   int sort_len;  // power of two >= k, 256 at least, used by the value-descending order
   // Rows too wide for one workgroup's fast path are selected in two stages (tile kernel only):
   // stage 1 launches one workgroup per (row, segment of seg_width columns) and writes the
@@ -247,26 +248,26 @@ __device__ __forceinline__ unsigned lane_xor(unsigned v) {
   }
 }
 
-// Bitonic sort of P (a power of two from 256 on) keys in LDS, largest first.  A wavefront keeps 256 of them, four to
-// a lane, and exchanges over strides below 256 in registers; only the longer strides go through LDS with a barrier
-// each: 6 of the 66 steps of 2048 keys (with all of them in LDS the best 2048 of a row of 8192 took 28 us in this order,
+// Bitonic sort of P (a power of two) keys in LDS, largest first.  A wavefront keeps 64 R of them, R to
+// a lane, and exchanges over strides below 64 R in registers; only the longer strides go through LDS with a barrier
+// each: 6 of the 66 steps of 2048 keys with R = 4 (with all of them in LDS the best 2048 of a row of 8192 took 28 us in this order,
 // with the exchanges by LDS permutes 21).
-template <int THREADS>
-__device__ __forceinline__ void sort_pairs(unsigned long long* pairs, unsigned P) {
+template <int THREADS, int R>
+__device__ __forceinline__ void sort_runs(unsigned long long* pairs, unsigned P) {
   const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  // one step of the keys 4 lane .. 4 lane + 3 of a chunk: i & size decides the direction
+  // one step of the keys R lane .. R lane + R - 1 of a chunk: i & size decides the direction
   auto in_registers = [&](unsigned base, unsigned first_size, unsigned last_size) {
-    unsigned long long v[4];
+    unsigned long long v[R];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = pairs[base + 4 * lane + r];
+    for (int r = 0; r < R; ++r) v[r] = pairs[base + R * lane + r];
     for (unsigned size = first_size; size <= last_size; size <<= 1) {
-      const bool desc_run = ((base + 4 * lane) & size) == 0;
-      auto across = [&](auto lanes) {                  // stride 4 * LX
+      const bool desc_run = ((base + R * lane) & size) == 0;
+      auto across = [&](auto lanes) {                  // stride R * LX
         constexpr int LX = decltype(lanes)::value;
-        if (size < 8 * LX) return;                     // (uniform)
+        if (size < 2 * R * LX) return;                     // (uniform)
         const bool keep_max = ((lane & LX) == 0) == desc_run;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < R; ++r) {
           const unsigned long long other = (unsigned long long)lane_xor<LX>((unsigned)(v[r] >> 32)) << 32 | lane_xor<LX>((unsigned)v[r]);
           v[r] = (v[r] < other) == keep_max ? other : v[r];
         }
@@ -278,12 +279,12 @@ __device__ __forceinline__ void sort_pairs(unsigned long long* pairs, unsigned P
       across(std::integral_constant<int, 2>{});
       across(std::integral_constant<int, 1>{});
 #pragma unroll
-      for (unsigned stride = 2; stride >= 1; stride >>= 1) {
+      for (unsigned stride = R / 2; stride >= 1; stride >>= 1) {
         if (stride >= size) continue;
 #pragma unroll
-        for (unsigned r = 0; r < 4; ++r) {
+        for (unsigned r = 0; r < R; ++r) {
           if (r & stride) continue;
-          const bool desc = ((base + 4 * lane + r) & size) == 0;
+          const bool desc = ((base + R * lane + r) & size) == 0;
           const unsigned long long a = v[r], b = v[r + stride];
           const bool swap = (a < b) == desc;
           v[r] = swap ? b : a;
@@ -292,12 +293,12 @@ __device__ __forceinline__ void sort_pairs(unsigned long long* pairs, unsigned P
       }
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) pairs[base + 4 * lane + r] = v[r];
+    for (int r = 0; r < R; ++r) pairs[base + R * lane + r] = v[r];
   };
-  for (unsigned base = 256 * wave; base < P; base += 4 * THREADS) in_registers(base, 2, 256);
+  for (unsigned base = 64 * R * wave; base < P; base += R * THREADS) in_registers(base, 2, 64 * R);
   __syncthreads();
-  for (unsigned size = 512; size <= P; size <<= 1) {
-    for (unsigned stride = size >> 1; stride >= 256; stride >>= 1) {
+  for (unsigned size = 128 * R; size <= P; size <<= 1) {
+    for (unsigned stride = size >> 1; stride >= 64 * R; stride >>= 1) {
       for (unsigned t = tid; t < P / 2; t += THREADS) {
         const unsigned i = 2 * t - (t & (stride - 1));
         const unsigned long long a = pairs[i], b = pairs[i + stride];
@@ -305,9 +306,18 @@ __device__ __forceinline__ void sort_pairs(unsigned long long* pairs, unsigned P
       }
       __syncthreads();
     }
-    for (unsigned base = 256 * wave; base < P; base += 4 * THREADS) in_registers(base, size, size);
+    for (unsigned base = 64 * R * wave; base < P; base += R * THREADS) in_registers(base, size, size);
     __syncthreads();
   }
+}
+
+// P from 256 on.  A step of a wavefront takes its own instructions, so up to 1024 keys go to four wavefronts, one to a SIMD: 256 of them
+// four to a lane were one wavefront's 36 steps (663 rows of 865, best 229: 9.5 us the call, 8.5 so; 200 x 4000, 512: 12.8 and 11.1).
+template <int THREADS>
+__device__ __forceinline__ void sort_pairs(unsigned long long* pairs, unsigned P) {
+  if (P <= 256) sort_runs<THREADS, 1>(pairs, P);              // (uniform)
+  else if (P <= 512) sort_runs<THREADS, 2>(pairs, P);
+  else sort_runs<THREADS, 4>(pairs, P);
 }
 
 // ---------------------------------------------------------------------------
@@ -322,7 +332,8 @@ __host__ __device__ constexpr bool tile_two_hists(int E, int threads) { return t
 // out).  MODE 2: stage 2 (a row of candidates per workgroup, positions translated through index_map).
 // SORTED: the value-descending order, a kernel of its own (with the sort behind a run-time test the index order of rows
 // of 8193 .. 16384 columns took half as long again).
-template <typename ScoreT, int E, int THREADS, int MODE, bool SORTED>
+// EAGER: the scores are requested before the row's bounds have arrived, and columns outside them are read too.
+template <typename ScoreT, int E, int THREADS, int MODE, bool SORTED, bool EAGER>
 __global__ __launch_bounds__(THREADS, E > 16 ? 4 : 8) void topk_tile_kernel(const TopkParams p) {
   extern __shared__ __align__(16) unsigned smem[];
   unsigned* hist = smem;
@@ -333,10 +344,18 @@ __global__ __launch_bounds__(THREADS, E > 16 ? 4 : 8) void topk_tile_kernel(cons
   const int row = stage1 ? (int)blockIdx.x / p.segs : (int)blockIdx.x;
   const int base = stage1 ? ((int)blockIdx.x % p.segs) * p.seg_width : 0;   // first column of this workgroup's share
   const int T = stage1 ? min(p.seg_width, p.width - base) : p.width;
-  int start = (p.starts ? p.starts[row] : 0) - base;
-  int end = (p.ends ? p.ends[row] : p.width) - base;
-  start = min(max(start, 0), T);
-  end = min(max(end, 0), T);
+  int start, end;
+  auto bounds = [&](int first, int last) {
+    start = min(max(first - base, 0), T);
+    end = min(max(last - base, 0), T);
+  };
+  int start_at = 0, end_at = 0;
+  if constexpr (EAGER) {                                // (no branch around their loads: they are waited for where they are used)
+    start_at = *(p.starts ? p.starts + row : p.out);
+    end_at = *(p.ends ? p.ends + row : p.out);
+  } else {
+    bounds(p.starts ? p.starts[row] : 0, p.ends ? p.ends[row] : p.width);
+  }
   const St* src = reinterpret_cast<const St*>(p.scores) + (long long)row * p.row_stride + base;
   int* out_row = p.out + (long long)row * p.k;
   const float kNaN = __uint_as_float(0x7fc00000u);
@@ -350,11 +369,20 @@ __global__ __launch_bounds__(THREADS, E > 16 ? 4 : 8) void topk_tile_kernel(cons
     // they are cleared before the row's bounds have arrived
     zero_hist<THREADS>(hist, kHist2 ? kHist2 + kHistBins : kHistBins);
     const int c0 = tid * E;
-    const bool any = c0 < end && c0 + E > start;          // (a run with nothing selectable is not read)
     // The last piece of a row may reach up to three columns past it: into what lies in front of the next row or the next
     // rows, which is fine, but the buffer may end with the last row's last column, whatever the pitch.
     const bool past = (T & 3) != 0 && MODE != 2 && row >= p.first_past;     // (uniform)
-    if (!past) {
+    if (EAGER && !past) {
+#pragma unroll
+      for (int i = 0; i < E / 4; ++i) {
+        float t4[4];
+        ScoreLoad<ScoreT>::vec4(src + min(c0 + 4 * i, (T - 1) & ~3), t4);       // (columns behind the row are outside the bounds)
+        v[4 * i] = t4[0]; v[4 * i + 1] = t4[1]; v[4 * i + 2] = t4[2]; v[4 * i + 3] = t4[3];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      bounds(p.starts ? start_at : 0, p.ends ? end_at : p.width);
+    } else if (!past) {
+      const bool any = c0 < end && c0 + E > start;        // (a run with nothing selectable is not read)
 #pragma unroll
       for (int i = 0; i < E / 4; ++i) {
         float t4[4] = {kNaN, kNaN, kNaN, kNaN};
@@ -362,6 +390,8 @@ __global__ __launch_bounds__(THREADS, E > 16 ? 4 : 8) void topk_tile_kernel(cons
         v[4 * i] = t4[0]; v[4 * i + 1] = t4[1]; v[4 * i + 2] = t4[2]; v[4 * i + 3] = t4[3];
       }
     } else {
+      if (EAGER) bounds(p.starts ? start_at : 0, p.ends ? end_at : p.width);
+      const bool any = c0 < end && c0 + E > start;
 #pragma unroll
       for (int i = 0; i < E / 4; ++i) {
         float t4[4] = {kNaN, kNaN, kNaN, kNaN};
@@ -772,8 +802,10 @@ int launch_for_type(const TopkParams& p, bool vec4, hipStream_t stream, size_t* 
     *smem_out = smem;                                                                     \
     if (smem > 160 * 1024) return -3;                                                     \
     if constexpr (MODE != 1)                                                              \
-      if (sorted) return launch_kernel(topk_tile_kernel<ScoreT, E, THR, MODE, true>, p, THR, smem, stream); \
-    return launch_kernel(topk_tile_kernel<ScoreT, E, THR, MODE, false>, p, THR, smem, stream); \
+      if (sorted) return launch_kernel(topk_tile_kernel<ScoreT, E, THR, MODE, true, false>, p, THR, smem, stream); \
+    if constexpr (MODE != 2)                                                              \
+      if (p.eager) return launch_kernel(topk_tile_kernel<ScoreT, E, THR, MODE, false, true>, p, THR, smem, stream); \
+    return launch_kernel(topk_tile_kernel<ScoreT, E, THR, MODE, false, false>, p, THR, smem, stream); \
   } while (0)
     if constexpr (MODE == 1) {                            // a segment is always kSegWidth columns wide
       CM_TOPK_TILE(16, 512);
@@ -849,6 +881,10 @@ int topk_select_launch(const cppmega_mi355_topk_args_t& a, hipStream_t stream) {
   int sort_len = 256;
   while (sort_len < a.k) sort_len <<= 1;
   p.sort_len = sort_len;
+  // Columns outside the bounds are read too while all of them take less time than the bounds' way from memory (41 x 15024 10.05 -> 9.95 us,
+  // 128 x 16000 10.7 -> 10.3, one decode step's 5 x 30000 25.4 -> 24.6).  More of them are left alone: half of a causal prefill's are
+  // outside, though rows that are nearly whole gain there as well (500 x 8000 10.5 -> 10.0).
+  p.eager = (a.starts || a.ends) && (long long)a.rows * a.width * esz <= (8 << 20);
   p.segs = 1; p.seg_width = 0; p.cand_val = nullptr; p.cand_idx = nullptr; p.index_map = nullptr;
 
   int rc;

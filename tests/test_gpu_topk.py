@@ -198,3 +198,24 @@ def test_rows_with_a_pitch_whose_buffer_ends_with_the_last_row(device, rows, wid
     a.workspace, a.workspace_bytes = ws.data_ptr(), need.value
     assert lib.cppmega_mi355_topk_select(C.byref(a), C.sizeof(a), _lib.current_stream(view.device)) == _lib.OK
     assert (out.cpu().numpy() == otopk.topk_selector_oracle(view.float().cpu().numpy(), k, order="index")).all()
+
+
+# one and two keys to a lane of the sort, on 256, 512 and 1024 threads, a key short of a run and not
+@pytest.mark.parametrize("width,k", [(256, 256), (900, 129), (2048, 512), (4096, 400), (8000, 200), (8192, 512), (16000, 256), (20000, 511)])
+def test_value_order_of_short_lists(device, width, k):
+    rng = np.random.default_rng(width + k)
+    scores = np.round(rng.standard_normal((3, width)) * 50).astype(np.float32)       # many equal values: ties by index
+    ends = np.array([width, k // 2, width - 1], np.int32)
+    assert (_run(to_dev(scores, device), k, device, ends=ends, order="value") == otopk.topk_selector_oracle(scores, k, ends=ends, order="value")).all()
+
+
+# scores of 8 MiB, requested before their bounds, and of a row more, of which only columns inside the bounds are read
+@pytest.mark.parametrize("rows,width,k", [(256, 8192, 300), (257, 8192, 300), (2048, 1024, 64), (2049, 1024, 64), (530, 4003, 90), (131, 16384, 700), (60, 40000, 200)])
+def test_bounds_of_many_rows(device, rows, width, k):
+    rng = np.random.default_rng(rows + width)
+    scores = np.round(rng.standard_normal((rows, width)) * 1000).astype(np.float32)
+    starts = rng.integers(-5, width // 2, rows).astype(np.int32)
+    ends = (starts + rng.integers(0, width, rows)).astype(np.int32)
+    ends[0] = starts[0]                                  # an empty interval
+    got = _run(to_dev(scores, device), k, device, starts=starts, ends=ends)
+    assert (got == otopk.topk_selector_oracle(scores, k, starts=starts, ends=ends, order="index")).all()
