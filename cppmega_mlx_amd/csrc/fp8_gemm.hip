@@ -461,9 +461,23 @@ void launch_reduce(const VecmatParams& p, hipStream_t stream) {
 
 }  // namespace
 
+// 5 to 16 rows stay with the kernel without staging while a CU has one workgroup of its 32 weight rows: with two it takes twice as long
+// (16 rows, that kernel / this one: 8192 x 4096 10.3 / 11.4 us, 8500 x 1024 8.0 / 6.8, 8500 x 4096 17.3 / 12.0, 8500 x 16384 47.7 / 29.6, 16384 x
+// 4096 19.3 / 16.1).  Measured at 5 .. 16 rows x 8400 .. 16400 x 512 .. 15900 with either layout of block scales: fewer than 12 rows gain
+// from about 3000 channels on (5 x 8400 x 1024 0.86 x, 6 x 10300 x 2048 0.95, 4096 1.2); where three K splits of the tiles are more
+// than the CUs and two leave some idle, up to 8192 channels (7 x 15814 x 14848 0.92), fewer with a scale per row, whose four
+// bytes take a line of the cache each (6 x 12200 x 8192 0.97, 4096 1.20; 11 x 11467 x 7168 0.92), and any number where neither counts (11 x 14832 x 15872 1.12).
+static bool few_rows_here(const cppmega_mi355_vecmat_args_t& a) {
+  const int cus = device_cus();
+  if (a.m < 5 || a.n <= 32 * cus || (a.m < 12 && a.k < 3072)) return false;
+  const bool row_scales = a.scale_w_kind == CPPMEGA_MI355_WSCALE_ROW_BLOCK;
+  if ((a.n + 127) / 128 * 3 <= cus || (a.m >= 9 && !row_scales)) return true;
+  return a.k <= (row_scales ? 6144 : 8192);
+}
+
 // bf16 / fp16 activations, whole 128-channel blocks, more rows than the kernels without staging take
 bool fp8_gemm_shape(const cppmega_mi355_vecmat_args_t& a) {
-  return (a.x_dtype == CPPMEGA_MI355_BF16 || a.x_dtype == CPPMEGA_MI355_F16) && a.m > 16 && a.k % 128 == 0 &&
+  return (a.x_dtype == CPPMEGA_MI355_BF16 || a.x_dtype == CPPMEGA_MI355_F16) && (a.m > 16 || few_rows_here(a)) && a.k % 128 == 0 &&
          a.k <= (1 << 22);                                      // a tile's rows within 32-bit offsets
 }
 

@@ -14,7 +14,7 @@
 //  * 5 <= M <= 16 bf16 / fp16 activations, K a multiple of 128 (skinny_rows_kernel; N up to 4096 and K beyond
 //    2048: skinny_rows_long_kernel): a workgroup owns up to 32 or 16 weight rows for the whole K; weights converted
 //    to bf16 / fp16 in registers, v_mfma_f32_16x16x32 on the activations as they are; one kernel, no workspace.
-//  * M >= 17, K a multiple of 128: the tiled GEMM of fp8_gemm.hip.
+//  * M >= 17, and mostly 5 <= M <= 16 over more weight rows than 32 a CU, K a multiple of 128: the tiled GEMM of fp8_gemm.hip.
 //  * anything else (odd K, misaligned rows): rowwise_kernel, one wavefront per
 //    output row, scalar byte loads.
 
@@ -733,12 +733,18 @@ static bool stream_k(const cppmega_mi355_vecmat_args_t& a) {
 static bool stream_shape(const cppmega_mi355_vecmat_args_t& a) { return stream_k(a) && a.m <= stream_row_cap(a.x_dtype); }
 // the kernel without a K split: bf16 / fp16 activations, 5 <= M <= 16, whole 128-channel blocks,
 // scales of 32 rows and partial tiles within the LDS
-constexpr int kRowsMaxM = 16;             // more activation rows: the tiled GEMM
+constexpr int kRowsMaxM = 16;             // more activation rows, and some of these over more than 32 weight rows a CU: the tiled GEMM
 static size_t rows_lds_bytes(int k, int mt) { return (size_t)rows_waves(mt) * (32 * 128 + mt * 16 * 256) + (size_t)(k / 128) * 32 * sizeof(float); }
 static size_t long_lds_bytes(int k) { return (size_t)kLongWaves * kLongWaveBytes + (size_t)(k / 128) * kLongRows * sizeof(float); }      // (fits where the above does)
 static bool rows_shape(const cppmega_mi355_vecmat_args_t& a) {
   return (a.x_dtype == CPPMEGA_MI355_BF16 || a.x_dtype == CPPMEGA_MI355_F16) && a.m >= 5 && a.m <= kRowsMaxM && a.k % 128 == 0 &&
          rows_lds_bytes(a.k, 1) <= 160 * 1024;
+}
+
+// up to 16 rows of many weight rows: the tiled GEMM with the workspace that its plan asks for; without it, the kernel that needs none
+static bool wide_scratch(const cppmega_mi355_vecmat_args_t& a) {
+  const size_t need = fp8_gemm_workspace_bytes(a);
+  return need == 0 || (a.workspace && ((uintptr_t)a.workspace & 15) == 0 && (size_t)a.workspace_bytes >= need);
 }
 
 int fp8_vecmat_workspace_bytes(const cppmega_mi355_vecmat_args_t& a, size_t* bytes) {
@@ -861,7 +867,7 @@ int fp8_vecmat_launch(const cppmega_mi355_vecmat_args_t& a, hipStream_t stream) 
   if (aligned && stream_shape(a)) {
     rc = stream_pass(p, 0, a.m);
     if (rc) return rc;
-  } else if (aligned && fp8_gemm_shape(a)) {
+  } else if (aligned && fp8_gemm_shape(a) && (a.m > kRowsMaxM || wide_scratch(a))) {
     p.partial = (float*)a.workspace;
     return fp8_gemm_launch(p, a.workspace ? (size_t)a.workspace_bytes : 0, stream);
   } else if (aligned && rows_shape(a)) {

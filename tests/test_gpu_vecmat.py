@@ -303,3 +303,31 @@ def test_tiled_gemm_starts_anywhere_in_k(device, M, N, K):
     vm.fp8_scaled_vecmat_path_c(x, codes.view(torch.uint8), scale_x=None, scale_w=scale, out=out)
     # (as for the other tiles)
     assert (out.double() - want).abs().max() <= 2e-6 * want.abs().max()
+
+
+# more weight rows than 32 for each of the 256 CUs: the tiled GEMM with the workspace it asks for, the kernel without one otherwise
+@pytest.mark.parametrize("M,N,K", [(5, 8193, 3072), (16, 8192, 640), (16, 8200, 8192), (9, 12001, 6144), (6, 16384, 128), (12, 9001, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_five_to_sixteen_rows_of_many_weight_rows(device, M, N, K, dtype):
+    import ctypes as C
+
+    from cppmega_mlx_amd import _lib
+    gen = torch.Generator(device=device).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=gen, device=device).to(dtype)
+    codes = torch.randn((N, K), generator=gen, device=device).mul(2).to(torch.float8_e4m3fn)
+    scale = torch.rand((N, K // 128), generator=gen, device=device) + 0.5
+    want = x.double() @ (codes.double() * scale.double().repeat_interleave(128, dim=1)).T
+    a = _lib.VecmatArgs()
+    a.struct_size, a.x_dtype, a.out_dtype, a.scale_w_kind = C.sizeof(a), _lib.BF16 if dtype is torch.bfloat16 else _lib.F16, _lib.F32, _lib.WSCALE_ROW_BLOCK
+    a.m, a.n, a.k = M, N, K
+    a.x, a.w, a.scale_w = x.data_ptr(), codes.data_ptr(), scale.data_ptr()
+    need, lib = C.c_size_t(0), _lib.load()
+    assert lib.cppmega_mi355_fp8_vecmat_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK
+    assert (need.value > 0) == (N > 8192 and K >= 3072)  # (K in one piece needs none)
+    ws = torch.empty(need.value + 16, dtype=torch.uint8, device=device)
+    for given in {0, max(need.value - 1, 0), need.value}:
+        out = torch.full((M, N), 7.0, dtype=torch.float32, device=device)
+        a.out, a.workspace, a.workspace_bytes = out.data_ptr(), ws.data_ptr() if given else None, given
+        assert lib.cppmega_mi355_fp8_vecmat(C.byref(a), C.sizeof(a), _lib.current_stream(x.device)) == _lib.OK
+        # (as for the tiles of more rows)
+        assert (out.double() - want).abs().max() <= 2e-6 * want.abs().max()
