@@ -658,7 +658,7 @@ PROFILE_WORKLOADS = [
      "W e4m3[7168,16384] + fp32 scale/128, x bf16[4,16384]"),
     ("fp8_vecmat_m16", "trace_main", ("fetch_main", "write_main"), None, ("skinny_rows_kernel<1",),
      "W e4m3[7168,16384] + fp32 scale/128, x bf16[16,16384] (one kernel, no K split, no workspace)"),
-    ("fp8_vecmat_m32", "trace_main", ("fetch_main", "write_main"), None, ("fp8_gemm_kernel<1, 1, 1, 4", "fp8_gemm_reduce"),
+    ("fp8_vecmat_m32", "trace_main", ("fetch_main", "write_main"), None, ("Tile<2, 2, 1, 4, 2, 3", "fp8_gemm_reduce"),
      "W e4m3[7168,16384] + fp32 scale/128, x bf16[32,16384] (32 x 128 tiles, split-K, and the reduce kernel)"),
     ("topk_selector", "trace_main", ("fetch_main", "write_main"), None, ("topk_tile_kernel<float, 16, 512, 0, false",),
      "scores fp32[4096 rows,8192] -> int32[4096,2048], indices in ascending order (the dispatches of 4096 workgroups only: "
