@@ -19,7 +19,7 @@
 //
 // Nothing is added in an order that varies: the same input gives the same bits.
 //
-// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 150 us (561 us with the atomics; under the profiler lists 6,
+// Measured at q [1, 1024, 16, 576], kv [1, 4096, 1, 576], top-k 256: 150 .. 155 us (561 us with the atomics; under the profiler lists 6,
 // scores and dq 68, dkv 71 .. 87, sum 9).  dkv is bound by the vector cache (27 M accesses of 64 bytes: 4 KB of q and d_out and
 // about 1 KB of planes for a step's 9 keys of 16) and ends with the CUs whose three bands are all full; scores and dq by the
 // gather of 302 MB of key rows each.
