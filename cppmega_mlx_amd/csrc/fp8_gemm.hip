@@ -76,7 +76,12 @@ struct Tile {
 // scales of any kind are applied exactly; in the product layout (weights as the second operand) a lane
 // holds one output channel, i.e. one scale per tile.  A lane's 16 weight bytes feed two products: the
 // contraction runs over the channels in the order the bytes lie in, and the activation pieces follow it.
-template <class T, bool F16>
+//
+// SECTIONS, for float32 results: the error of a sum grows with the number of blocks that are added one after the other, so from six on
+// about sqrt(n) sections of blocks are added up by themselves and then to a second sum.  Without it the plans of few splits lost
+// digits: rms error against float64, one chain / here, 790 x 9331 x 7168 1.37e-7 / 0.80e-7 (two splits of 28 blocks 1.03e-7), 676 x 2255
+// x 6656 1.00e-7 / 0.74e-7 (four splits 0.82e-7).  It costs up to 3 % of a call, and results of 16 bits do not show it.
+template <class T, bool F16, bool SECTIONS>
 __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatParams p) {
   constexpr int TM = T::TM, TN = T::TN, WM = T::WM, WN = T::WN, WK = T::WK, SLOTS = T::SLOTS, BM = T::BM, BN = T::BN, XL = T::XL, WL = T::WL;
   constexpr int PITCH = T::PITCH, L = XL + WL + 1;
@@ -93,6 +98,9 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
   const int b0 = (int)((long long)blocks * blockIdx.y / p.k_splits), b1 = (int)((long long)blocks * (blockIdx.y + 1) / p.k_splits);
   const int stages = (b1 - b0 + WK - 1) / WK;
   int turned = 0;                                                    // the stage it begins with (two groups)
+  // Stages come in sections of `section` or, the last `longer` ones, one more.
+  const int sections = SECTIONS && stages > 5 ? __builtin_amdgcn_readfirstlane((int)__builtin_amdgcn_sqrtf((float)stages - 1.5f)) : 1;
+  const int section = stages / sections, longer = stages - section * sections;
 
   // Rows and columns of tile e.  Consecutive workgroups go round the eight XCDs: every XCD takes one run of
   // the order (groups of eight column tiles; inside, row tile by row tile), so that its L2 holds the
@@ -190,7 +198,7 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
     }
   };
 
-  f32x4 acc[TM][TN], tile[TM][TN];
+  f32x4 acc[TM][TN], tile[TM][TN], sum[SECTIONS ? TM : 1][SECTIONS ? TN : 1];
   const int xlane = (wk * 2 * BM + wm + l16) * 128, wlane = T::kX + (wk * BN + wn + l16) * 128, slane = T::kX + T::kW + wave * 256 + l16 * 4;
   const int f = fold(l16);
   const int xpos[2] = {xlane + 16 * ((quad * 2) ^ f), xlane + 16 * ((quad * 2 + 1) ^ f)};
@@ -244,44 +252,65 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s = 0; s < stages; ++s) {
-      const int next = slot + T::kStage == SLOTS * T::kStage ? 0 : slot + T::kStage;
-      read_x(slot, 0, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(0, 0, false);
-      __builtin_amdgcn_sched_barrier(0);
-      read_w(slot, 1);
-      read_x(slot, 1, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(0, 1, false);
-      __builtin_amdgcn_sched_barrier(0);
-      read_x(slot, 1, 1);
+    if constexpr (SECTIONS)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) sc[j] = *reinterpret_cast<const float*>(lds + slot + slane + j * 64);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(1, 0, false);
-      __builtin_amdgcn_sched_barrier(0);
-      const bool more = left > 0;
-      if (--todo > 0) {
-        // the next stage has arrived, and everybody has read this one
-        if (SLOTS > 2 && todo >= SLOTS - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((SLOTS - 2) * L) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        read_w(next, 0);
-        read_x(next, 0, 0);
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) sum[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s = 0, i = 1; s < stages; ++i) {
+      const int end = SECTIONS ? s + section + (i > sections - longer ? 1 : 0) : stages;
+      for (; s < end; ++s) {
+        const int next = slot + T::kStage == SLOTS * T::kStage ? 0 : slot + T::kStage;
+        read_x(slot, 0, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0, 0, false);
+        __builtin_amdgcn_sched_barrier(0);
+        read_w(slot, 1);
+        read_x(slot, 1, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0, 1, false);
+        __builtin_amdgcn_sched_barrier(0);
+        read_x(slot, 1, 1);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) sc[j] = *reinterpret_cast<const float*>(lds + slot + slane + j * 64);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1, 0, false);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool more = left > 0;
+        if (--todo > 0) {
+          // the next stage has arrived, and everybody has read this one
+          if (SLOTS > 2 && todo >= SLOTS - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((SLOTS - 2) * L) : "memory");
+          else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          read_w(next, 0);
+          read_x(next, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1, 1, more);
+        const int at = s + turned < stages ? s + turned : s + turned - stages;
+        if (WK == 1 || b0 + at * WK + wk < b1) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+              for (int v = 0; v < 4; ++v) acc[i][j][v] = fmaf(sc[j], tile[i][j][v], acc[i][j][v]);
+        }
+        slot = next;
       }
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(1, 1, more);
-      const int at = s + turned < stages ? s + turned : s + turned - stages;
-      if (WK == 1 || b0 + at * WK + wk < b1) {
+      if constexpr (SECTIONS)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[i][j][v] = fmaf(sc[j], tile[i][j][v], acc[i][j][v]);
-      }
-      slot = next;
+          for (int j = 0; j < TN; ++j) {
+            sum[i][j] += acc[i][j];
+            acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+          }
     }
+    if constexpr (SECTIONS)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j];
     if (!T::PERSIST) __syncthreads();                    // the last stage is read: its place is free
 
     constexpr int TO = TM / WK;                          // row tiles this wavefront stores
@@ -348,7 +377,7 @@ __global__ __launch_bounds__(T::kThreads, 2) void fp8_gemm_kernel(const VecmatPa
   }
 }
 
-// out[m][n] = sum over the K splits of partial[split][m][n], in split order.  Bound by latency (7 MB at 32 x 7168 x 8
+// out[m][n] = sum over the K splits of partial[split][m][n], in pairs.  Bound by latency (7 MB at 32 x 7168 x 8
 // splits): with the splits' loads one after the other and stores of single values a call took 2 to 3 us longer.  Splits
 // begin at whole 16-byte pieces, so that products of odd sizes are read alike (19 x 333 of 16 splits: 12 -> 4 us).  Code of
 // its own for each number of splits: with a test in front of each load the first was waited for before the others were asked for.
@@ -357,11 +386,14 @@ __global__ __launch_bounds__(256) void fp8_gemm_reduce_kernel(const VecmatParams
   const size_t total = (size_t)p.m * p.n, step = split_step(p.m, p.n);
   const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= total) return;
-  f32x4 part[SPLITS], s = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 part[SPLITS];
 #pragma unroll
   for (int z = 0; z < SPLITS; ++z) part[z] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.partial + (size_t)z * step + i));
 #pragma unroll
-  for (int z = 0; z < SPLITS; ++z) s += part[z];
+  for (int step_z = 1; step_z < SPLITS; step_z *= 2)
+#pragma unroll
+    for (int z = 0; z + step_z < SPLITS; z += 2 * step_z) part[z] += part[z + step_z];
+  const f32x4 s = part[0];
   if (i + 4 <= total && p.out_dtype != CPPMEGA_MI355_F32 && ((uintptr_t)p.out & 7) == 0) {
     const bool bf16 = p.out_dtype == CPPMEGA_MI355_BF16;
     *reinterpret_cast<uint2*>((unsigned short*)p.out + i) = bf16 ? make_uint2(pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3]))
@@ -374,6 +406,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_reduce_kernel(const VecmatParams
 }
 
 typedef Tile<2, 2, 1, 4, 2, 3, false> Tile32;            // 32 x 128, two groups, 150 KB of LDS
+typedef Tile<2, 2, 1, 4, 1, 4, false> Tile32Short;       // 32 x 128, one group and up to four blocks, all on their way at once, 100 KB
 typedef Tile<4, 2, 1, 4, 2, 2, false> Tile64Pair;        // 64 x 128, two groups, 132 KB
 typedef Tile<4, 2, 1, 4, 1, 2, false> Tile64;            // 64 x 128, 66 KB: two workgroups on a CU, whose ends overlap
 typedef Tile<4, 2, 1, 4, 1, 2, true> Tile64Many;         // the same, tile after tile
@@ -381,19 +414,20 @@ typedef Tile<4, 4, 2, 4, 1, 2, false> Tile256;           // 128 x 256, 132 KB
 
 // What a tile shape costs, measured on MI355X: microseconds per stage with 1 and 2 of its workgroups on a CU, and per
 // workgroup for its first loads and its stores.
-enum Shape { kTile32, kTile64Pair, kTile64, kTile64Many, kTile256 };
+enum Shape { kTile32, kTile32Short, kTile64Pair, kTile64, kTile64Many, kTile256 };
 struct TileCost {
   int bm, bn, per_cu, groups;
   double stage_us[2], ends_us;
 };
 constexpr TileCost kCosts[] = {
     {32, 128, 1, 2, {1.145, 0.0}, 1.32},
+    {32, 128, 1, 1, {0.8, 0.0}, 2.0},
     {64, 128, 1, 2, {1.21, 0.0}, 2.72},
     {64, 128, 2, 1, {0.92, 1.0}, 3.08},
     {64, 128, 2, 1, {0.5, 1.09}, 0.88},
     {128, 256, 1, 1, {1.71, 0.0}, 3.2},
 };
-constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
+constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
 
 struct GemmPlan { Shape shape; int splits; };
 
@@ -403,10 +437,14 @@ size_t split_bytes(int splits, int m, int n) { return splits > 1 ? splits * spli
 // stream takes, plus, for a split, one more launch and the partial sums written and read (8 bytes per sum).
 // Fitted at 110 shapes of 17..4000 x 256..16400 x 512..16384, both scale layouts: the choice is 0.2 % from the best of all
 // combinations there in the mean and 5 % at most.
+// Float32 results over up to four blocks are one chain: the sum of two groups' sums is a rounding more (rms error against float64 1.13 x
+// over 2 blocks, 1.08 x over 3, 1.02 x over 4).  Tiles of 32 rows with all their blocks on their way at once are as fast there (two groups /
+// here: 83 x 763 x 256 4.5 / 4.3 us, 394 x 984 x 512 5.4 / 5.4, 102 x 9598 x 384 6.5 / 6.3, 2698 x 584 x 512 7.2 / 7.7).  Seven splits are for
+// the largest tile, which keeps no second sum: in six its sums were longer (1434 x 719 x 16256 1.03 x the error, 49.7 us for 47.4).
 // Splits whose sums need more than `have` bytes are left out; one split needs none.  64 x 128 tiles that are more than
 // two to a CU are taken one after the other by as many workgroups (717 x 7411 x 1024: 23.7 -> 21.2 us, 1647 x 8297 x 1152:
 // 46.3 -> 42.8; with one tile to a workgroup the loop costs 1 to 5 %).
-GemmPlan gemm_plan(int m, int n, int k, size_t have) {
+GemmPlan gemm_plan(int m, int n, int k, bool f32, size_t have) {
   const int blocks = k / 128, cus = device_cus();
   GemmPlan best = {kTile32, 1};
   double best_us = 1e30;
@@ -415,8 +453,11 @@ GemmPlan gemm_plan(int m, int n, int k, size_t have) {
     const long long tiles = (long long)((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn);
     const bool many = tiles > 2LL * cus;
     if ((shape == kTile64 && many) || (shape == kTile64Many && !many)) continue;
+    const bool one_chain = f32 && blocks <= 4;
+    if (one_chain ? c.groups > 1 : shape == kTile32Short) continue;
     for (int splits : kSplits) {
       if (splits > 1 && (splits * 2 > blocks || split_bytes(splits, m, n) > have || shape == kTile64Many)) break;
+      if (splits == 7 && shape != kTile256) continue;
       const long long on_cu = (tiles * splits + cus - 1) / cus, rounds = on_cu / c.per_cu, rest = on_cu % c.per_cu;
       const int stages = ((blocks + splits - 1) / splits + c.groups - 1) / c.groups;
       double us = (double)rounds * (stages * c.stage_us[c.per_cu - 1] + c.ends_us);
@@ -438,8 +479,16 @@ void launch_as(int m, int n, hipStream_t stream, const VecmatParams& p) {
     if (most > 0 && tiles > most) tiles = most;
   }
   const dim3 grid(tiles, (unsigned)p.k_splits), block(T::kThreads);
-  if (p.x_dtype == CPPMEGA_MI355_F16) hipLaunchKernelGGL((fp8_gemm_kernel<T, true>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((fp8_gemm_kernel<T, false>), grid, block, 0, stream, p);
+  constexpr bool kSections = T::TM * T::TN <= 8 && T::SLOTS < 4;       // (the largest tile has no registers for a second sum, four blocks need none)
+  const bool f16 = p.x_dtype == CPPMEGA_MI355_F16;
+  if (kSections && p.out_dtype == CPPMEGA_MI355_F32) {
+    if (f16) hipLaunchKernelGGL((fp8_gemm_kernel<T, true, kSections>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((fp8_gemm_kernel<T, false, kSections>), grid, block, 0, stream, p);
+  } else if (f16) {
+    hipLaunchKernelGGL((fp8_gemm_kernel<T, true, false>), grid, block, 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((fp8_gemm_kernel<T, false, false>), grid, block, 0, stream, p);
+  }
 }
 
 void launch_reduce(const VecmatParams& p, hipStream_t stream) {
@@ -452,6 +501,7 @@ void launch_reduce(const VecmatParams& p, hipStream_t stream) {
     case 4: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<4>, grid, block, 0, stream, p); break;
     case 5: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<5>, grid, block, 0, stream, p); break;
     case 6: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<6>, grid, block, 0, stream, p); break;
+    case 7: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<7>, grid, block, 0, stream, p); break;
     case 8: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<8>, grid, block, 0, stream, p); break;
     case 10: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<10>, grid, block, 0, stream, p); break;
     case 12: hipLaunchKernelGGL(fp8_gemm_reduce_kernel<12>, grid, block, 0, stream, p); break;
@@ -483,7 +533,7 @@ bool fp8_gemm_shape(const cppmega_mi355_vecmat_args_t& a) {
 }
 
 size_t fp8_gemm_workspace_bytes(const cppmega_mi355_vecmat_args_t& a) {
-  int splits = gemm_plan(a.m, a.n, a.k, SIZE_MAX).splits;
+  int splits = gemm_plan(a.m, a.n, a.k, a.out_dtype == CPPMEGA_MI355_F32, SIZE_MAX).splits;
   // a few small tiles ask for the room of three splits (3 MB at most) whatever the plan: workspaces that callers laid out
   // for a range of such sizes stay as large as they were when each of them was split
   if (splits < 3 && a.k >= 6 * 128 && (long long)((a.m + 31) / 32) * ((a.n + 127) / 128) <= device_cus() / 4) splits = 3;
@@ -492,12 +542,13 @@ size_t fp8_gemm_workspace_bytes(const cppmega_mi355_vecmat_args_t& a) {
 
 int fp8_gemm_launch(VecmatParams p, size_t workspace_bytes, hipStream_t stream) {
   // (the sums of splits are read in 16-byte pieces)
-  const GemmPlan g = gemm_plan(p.m, p.n, p.k, ((uintptr_t)p.partial & 15) == 0 ? workspace_bytes : 0);
+  const GemmPlan g = gemm_plan(p.m, p.n, p.k, p.out_dtype == CPPMEGA_MI355_F32, ((uintptr_t)p.partial & 15) == 0 ? workspace_bytes : 0);
   p.k_splits = g.splits;
   const long long tiles = (long long)((p.m + kCosts[g.shape].bm - 1) / kCosts[g.shape].bm) * ((p.n + kCosts[g.shape].bn - 1) / kCosts[g.shape].bn);
   if (tiles > 0x7fffffffLL) return fail(CPPMEGA_MI355_ERR_SHAPE, "vecmat: M=%d N=%d has too many tiles", p.m, p.n);
   switch (g.shape) {
     case kTile32: launch_as<Tile32>(p.m, p.n, stream, p); break;
+    case kTile32Short: launch_as<Tile32Short>(p.m, p.n, stream, p); break;
     case kTile64Pair: launch_as<Tile64Pair>(p.m, p.n, stream, p); break;
     case kTile64: launch_as<Tile64>(p.m, p.n, stream, p); break;
     case kTile64Many: launch_as<Tile64Many>(p.m, p.n, stream, p); break;

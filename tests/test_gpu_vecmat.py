@@ -335,3 +335,22 @@ def test_five_to_sixteen_rows_of_many_weight_rows(device, M, N, K, dtype):
         assert lib.cppmega_mi355_fp8_vecmat(C.byref(a), C.sizeof(a), _lib.current_stream(x.device)) == _lib.OK
         # float32 sums (2e-6 of the largest, as for the tiles of more rows), rounded once to 8 or 11 bits of mantissa
         assert ((out.double() - want).abs() <= 2e-6 * want.abs().max() + want.abs() * 2.0 ** (-8 if dtype is torch.bfloat16 else -11)).all()
+
+
+# rms error of the kernels that had more K splits (64 and 128 rows to a tile, up to 16 splits, each added up block by block): results of
+# one chain of all blocks, of two groups' chains, of tiles that come one after the other, of the largest tile in splits, of few blocks
+@pytest.mark.parametrize("M,N,K,before", [(3494, 558, 2176, 6.348e-8), (676, 2255, 6656, 8.244e-8), (2038, 869, 7296, 8.474e-8),
+                                          (790, 9331, 7168, 1.0326e-7), (1434, 719, 16256, 9.772e-8), (83, 763, 256, 3.990e-8),
+                                          (394, 984, 512, 4.709e-8)])
+def test_float32_results_of_the_tiled_gemm_are_as_exact_as_split_sums(device, M, N, K, before):
+    """Products are exact, so what is off is the order of the float32 additions.  2 %: what the rms of 60000 results and more varies by
+    with the inputs, four times over."""
+    gen = torch.Generator(device=device).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=gen, device=device).to(torch.bfloat16)
+    codes = torch.randn((N, K), generator=gen, device=device).to(torch.float8_e4m3fn)
+    scale = torch.rand((N, K // 128), generator=gen, device=device) + 0.5
+    want = x.double() @ (codes.double() * scale.double().repeat_interleave(128, dim=1)).T
+    out = torch.empty((M, N), dtype=torch.float32, device=device)
+    vm.fp8_scaled_vecmat_path_c(x, codes.view(torch.uint8), scale_x=None, scale_w=scale, out=out)
+    error = ((out.double() - want).pow(2).mean() / want.pow(2).mean()).sqrt().item()
+    assert error <= 1.02 * before, error
