@@ -665,10 +665,16 @@ __global__ __launch_bounds__(kLongWaves * 64) void skinny_rows_long_kernel(const
   if (tid < 256) {
     const int m = tid >> 4, r = tid & 15;              // consecutive threads: consecutive output columns
     if (m < p.m && r < rows_here) {
-      float sum = 0.0f;
+      // In pairs: one after the other the sums of twice as many wavefronts as above were up to 1.18 x as far off in float32 (16 x 3000 x
+      // 3584, rms error against float64: 8 wavefronts 7.1e-8, 16 one after the other 8.3e-8, in pairs 6.7e-8).
+      float part[kLongWaves];
 #pragma unroll
-      for (int w = 0; w < kLongWaves; ++w) sum += red[(w * 16 + r) * 16 + m];
-      store_as(p.out, (size_t)m * p.n + n0 + r, p.out_dtype, sum);
+      for (int w = 0; w < kLongWaves; ++w) part[w] = red[(w * 16 + r) * 16 + m];
+#pragma unroll
+      for (int step = 1; step < kLongWaves; step *= 2)
+#pragma unroll
+        for (int w = 0; w < kLongWaves; w += 2 * step) part[w] += part[w + step];
+      store_as(p.out, (size_t)m * p.n + n0 + r, p.out_dtype, part[0]);
     }
   }
 }
