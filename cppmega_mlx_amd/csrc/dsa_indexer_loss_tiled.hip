@@ -181,8 +181,11 @@ __host__ __device__ inline long long tiles_before(long long n, long long key_til
 // turned out not to be finite), and the second pass leaves keys that do not count out at its end.
 // Workgroups of the first pass behind those of the tiles take the statistics of the index scores, a row to a wavefront (when, run()
 // says).
+// WIDE: 64 rows of scores are 2 GB and more, beyond the offsets of their descriptor, and are read by address (second pass; 130 positions of
+// 8 heads of 64 over 2^23 keys 11.8 ms, 135 with a workgroup per 16 positions).
+constexpr int kWideKeys = 1 << 23;
 constexpr int resident(int AD, bool general) { return AD <= 64 && !general ? 4 : 2; }
-template <bool F16, int AD, int GROUPS, bool SECOND, bool GENERAL>
+template <bool F16, int AD, int GROUPS, bool SECOND, bool GENERAL, bool WIDE = false>
 __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENERAL)) void dsa_loss_tile_kernel(const LossTiledParams p) {
   constexpr bool WHOLE = GROUPS == 1;                     // whole tiles only
   constexpr int THREADS = WHOLE ? 256 : 128 * GROUPS, BLOCKS = WHOLE ? 3 : 2 * GROUPS;
@@ -427,7 +430,17 @@ __global__ __launch_bounds__(GROUPS == 1 ? 256 : 128 * GROUPS, resident(AD, GENE
   // quad and its loads the second pass took 1709 vector instructions a wavefront, half of them here, for 1365), ..
   const Rows s_rows(reinterpret_cast<const char*>(p.index_scores + ((size_t)b * p.ASq + q0) * p.Sk), (unsigned)min(64, p.ASq - q0) * (unsigned)p.Sk * 4u);
   const unsigned s_lane = ((unsigned)(my_q - q0) * (unsigned)p.Sk + (unsigned)(kw + 4 * half)) * 4u;
-  auto scores_of = [&](int t, int g) { return __builtin_bit_cast(f32x4, s_rows.load(s_lane + (t * 32 + 8 * g) * 4u, 0)); };
+  auto scores_of = [&](int t, int g) {
+    if constexpr (WIDE) {
+      const int key = kw + t * 32 + 8 * g + 4 * half;
+      f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (key + i < p.Sk) v[i] = p.index_scores[row * (size_t)p.Sk + key + i];
+      return v;
+    }
+    return __builtin_bit_cast(f32x4, s_rows.load(s_lane + (t * 32 + 8 * g) * 4u, 0));
+  };
   // .. and their divergence, the heads' probabilities adding up to `sums`.  Keys that do not count leave no trace: scores that
   // are NaN have q = 0 (the maximum of NaN and -inf is -inf).
   auto divergence = [&](int t, int g, const f32x4& scores, const float (&sums)[4]) {
@@ -579,7 +592,10 @@ void passes(LossTiledParams p, long long workgroups, bool general, hipStream_t s
   if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, false, true>), with_statistics, block, 0, stream, p);
   else hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, false, false>), with_statistics, block, 0, stream, p);
   hipLaunchKernelGGL(dsa_loss_merge_kernel, dim3((unsigned)(columns * p.AH)), merge, 0, stream, p);
-  if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, true, true>), grid, block, 0, stream, p);
+  if (p.Sk >= kWideKeys) {
+    if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, true, true, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, true, false, true>), grid, block, 0, stream, p);
+  } else if (general) hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, true, true>), grid, block, 0, stream, p);
   else hipLaunchKernelGGL((dsa_loss_tile_kernel<F16, AD, GROUPS, true, false>), grid, block, 0, stream, p);
   hipLaunchKernelGGL(dsa_loss_sum_kernel, dim3((unsigned)columns), merge, 0, stream, p);
 }
@@ -649,7 +665,6 @@ bool dsa_indexer_loss_tiled_supports(const cppmega_mi355_dsa_loss_args_t& a) {
   if (a.head_dim != 32 && a.head_dim != 64 && a.head_dim != 96 && a.head_dim != 128) return false;
   if ((size_t)a.batch * a.heads * a.head_dim * 2 * 128 >= (1ull << 32)) return false;         // a tile's rows within 32-bit offsets
   if (a.batch > 65535 || (size_t)a.seq_q * a.batch == 0 || a.heads == 0 || a.seq_k == 0) return false;
-  if (a.seq_k >= 1 << 23) return false;                                                       // 64 rows of scores within 31-bit offsets
   return !a.topk_indices || a.seq_k <= 131072;
 }
 

@@ -304,3 +304,44 @@ def test_index_scores_that_are_not_finite(shape, sparse):
     got = dsa_splitk_indexer_loss_per_position(bad.cuda(), top.cuda(), q.cuda(), k.cuda(), AD ** -0.5, sparse).cpu().numpy()
     clean = torch.where(gone, float("-inf"), idx)
     np.testing.assert_allclose(got, _want(q, k, clean, top, AD ** -0.5, sparse), atol=2e-5, rtol=2e-4)
+
+
+def test_scores_of_eight_million_keys_take_the_tiled_path():
+    """The size query is the same function of the positions on both sides of where 64 rows of scores leave 31 bits of offset."""
+    import ctypes as C
+
+    from cppmega_mlx_amd import _lib
+    sizes = []
+    for Sk in ((1 << 23) - 1, 1 << 23, (1 << 24) + 1, (1 << 30) + 1):
+        a = _lib.DsaLossArgs()
+        a.struct_size, a.in_dtype = C.sizeof(a), _lib.BF16
+        a.seq_q, a.batch, a.heads, a.head_dim, a.seq_k = 130, 1, 8, 32, Sk
+        need = C.c_size_t(0)
+        assert _lib.load().cppmega_mi355_dsa_indexer_loss_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK
+        sizes.append(need.value)
+    assert sizes[0] > 0 and sizes == sizes[:1] * 4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("AH,AD,scale", [(2, 32, 0.2), (4, 64, 0.1), (4, 64, -0.1), (3, 128, 0.1)],
+                         ids=["split_in_two", "split_in_four", "masks_behind_the_products", "large_heads"])
+@pytest.mark.parametrize("Sk", [(1 << 23) + 5, (1 << 24) + 2])
+def test_scores_of_eight_million_keys(AH, AD, scale, Sk):
+    """64 rows of scores are 2 and 4 GB: the tolerance of the other shapes, with the softmax over all keys in float64."""
+    ASq = 130
+    g = torch.Generator(device="cuda").manual_seed(AH + AD)
+    q = torch.randn((ASq, 1, AH, AD), generator=g, device="cuda").to(torch.bfloat16)
+    k = torch.zeros((Sk, 1, AH, AD), dtype=torch.bfloat16, device="cuda")
+    k[:ASq] = torch.randn((ASq, 1, AH, AD), generator=g, device="cuda").to(torch.bfloat16)
+    scores = torch.randn((1, ASq, Sk), generator=g, device="cuda")
+    scores[..., :ASq] += 12.0                            # (the visible keys hold a share that the logarithm's offset does not hide)
+    got = dsa_splitk_indexer_loss_per_position(scores, None, q, k, scale, False).double().cpu().numpy()
+    log_sum = torch.stack([torch.logsumexp(scores[0, i].double(), 0) for i in range(ASq)])
+    index = torch.exp(scores[0, :, :ASq].double() - log_sum[:, None])
+    hidden = torch.ones((ASq, ASq), dtype=torch.bool, device="cuda").triu(1)
+    p = torch.zeros((ASq, ASq), dtype=torch.float64, device="cuda")
+    for h in range(AH):
+        s = q[:, 0, h].double() @ k[:ASq, 0, h].double().T * scale
+        p += torch.softmax(s.masked_fill(hidden, float("-inf")), -1) / AH
+    want = (p * (torch.log(p + od.EPS) - torch.log(index + od.EPS))).masked_fill(hidden, 0.0).sum(-1).cpu().numpy()
+    np.testing.assert_allclose(got[0], want, atol=2e-5, rtol=2e-4)
