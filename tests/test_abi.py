@@ -292,3 +292,22 @@ def test_the_scratch_asked_for_serves_any_output(over):
     a.out = 0x1002                                           # (looked at, not through)
     assert _lib.load().cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(known)) == 0
     assert need.value == known.value
+
+
+@pytest.mark.parametrize("S,H,G,topk,splits", [(2, 72, 1, 700, 6), (3, 64, 2, 640, 5), (2, 128, 1, 900, 8), (4, 128, 1, 2048, 8), (16, 64, 1, 512, 1),
+                                               (24, 64, 1, 2048, 8)])
+def test_few_queries_of_many_heads_are_planned_in_chunks_of_16(S, H, G, topk, splits):
+    """The size query tells the plan: partial sums of 32 heads x 512 channels and two statistics each, per split.  Where 64 (groups of 32
+    heads: 32) share a workgroup the first five have 11, 10, 15, 13 and 4 splits; the last one stays there."""
+    lib = _lib.load()
+    a = _lib.SparseMlaArgs()
+    a.struct_size, a.kernel = C.sizeof(a), _lib.MLA_KERNEL_MFMA
+    a.q = a.kv = a.indices = a.out = 0x1000              # (a sizing call: nothing is read)
+    a.q_dtype = a.kv_dtype = a.out_dtype = _lib.BF16
+    a.index_dtype = _lib.I32
+    a.batch, a.seq_q, a.heads, a.kv_groups, a.seq_kv, a.topk, a.d_qk, a.d_v, a.sm_scale = 1, S, H, G, 4096, topk, 576, 512, 0.05
+    need = C.c_size_t(0)
+    assert lib.cppmega_mi355_sparse_mla_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK
+    block = (32 * 512 + 32 * 2) * 4
+    blocks_of_32 = S * G * ((H // G + 31) // 32)
+    assert need.value == (blocks_of_32 * splits * block if splits > 1 else 0)

@@ -946,3 +946,38 @@ def test_merging_of_key_splits_of_many_queries(device, S, H, topk, out_dtype):
     bs.sparse_mla_blockscaled_path_c_apply(q, None, codes, scale, to_dev(idx.astype(np.int32), device), sm_scale=sm, d_v=512,
                                            out=out, lse=lse, kv_rope=rope, kernel="mfma")
     _assert_close(out, lse, want_out, want_lse, lse_tol=LSE_TOL_MFMA)
+
+
+@pytest.mark.parametrize("S,H,G,topk", [(2, 72, 1, 700), (3, 64, 2, 640), (2, 128, 1, 900), (4, 128, 1, 2048), (16, 64, 1, 512)])
+@pytest.mark.parametrize("rows", ["bf16", "codes", "e8m0"])
+def test_few_queries_of_more_than_16_heads_to_the_last_bits(device, rows, S, H, G, topk):
+    """Shapes that the size query shows to be planned in chunks of 16 heads (and the E8M0 rows' own choice).  A weight in bfloat16 is off by
+    2^-8 of itself at most (half of its last place), and so is the root mean square of results in float32; a head, a split or a tile of
+    another one's is off by the whole of it."""
+    from cppmega_mlx_amd import _lib
+    Skv, sm = 2100, 576 ** -0.5
+    gen = torch.Generator(device=device).manual_seed(S + H + topk)
+    idx = torch.stack([torch.randperm(Skv, generator=gen, device=device)[:topk] for _ in range(S * G)]).view(1, S, G, topk).to(torch.int32)
+    q, kv = (torch.randn(shape, generator=gen, device=device) for shape in ((1, S, H, 576), (1, Skv, G, 576)))
+    kw = {}
+    if rows == "bf16":
+        q, kv = q.to(torch.bfloat16), kv.to(torch.bfloat16)
+        qf, kf = q.double(), kv.double()
+    else:
+        quantize, decode, kind, block = ((fp8.quantize_per_token, om.dequant_per_token, _lib.SCALE_PER_TOKEN, 0) if rows == "codes"
+                                         else (fp8.quantize_mxfp8, om.dequant_e8m0, _lib.SCALE_E8M0, 32))
+        (qc, qs), (kc, ks) = quantize(q.cpu().numpy()), quantize(kv.cpu().numpy())
+        qf, kf = (torch.from_numpy(np.asarray(decode(c, s), dtype=np.float64)).to(device) for c, s in ((qc, qs), (kc, ks)))
+        q, kv = to_dev(qc, device), to_dev(kc, device)
+        kw = dict(q_spec=ops.QuantSpec(kind, to_dev(qs, device), block), kv_spec=ops.QuantSpec(kind, to_dev(ks, device), block))
+    out = torch.full((1, S, H, 512), 7.0, device=device)
+    lse = torch.zeros((1, S, H), device=device)
+    ops.sparse_mla_forward(q, kv, idx, sm_scale=sm, d_v=512, out=out, lse=lse, kernel="mfma", **kw)
+    for g in range(G):
+        heads = slice(g * H // G, (g + 1) * H // G)
+        keys = kf[0, :, g][idx[0, :, g].long()]
+        scores = torch.matmul(qf[0, :, heads], keys.transpose(1, 2).contiguous()) * sm
+        want = torch.matmul(torch.softmax(scores, -1), keys[..., :512].contiguous())
+        rms = ((out[0, :, heads].double() - want).pow(2).mean(-1) / want.pow(2).mean(-1)).sqrt()          # of each query and head
+        assert rms.max() <= 2.0 ** -8, rms.max()
+        assert (lse[0, :, heads].double() - torch.logsumexp(scores, -1)).abs().max() <= 1e-5

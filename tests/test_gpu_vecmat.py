@@ -366,3 +366,70 @@ def test_float32_results_of_few_rows_over_long_k_are_as_exact_as_eight_sums(devi
     """(2 %, as above: the rms of 16000 results varies by half a percent.)"""
     error = _rms_error_of_float32_results(device, M, N, K)
     assert error <= 1.02 * before, error
+
+
+# 5 to 16 rows of many weight rows, on both sides of each limit: too few weight rows, too short a K, and where two K splits leave CUs
+# idle and three are a second round (more than 85 column tiles) the longest K, by rows and by whether each row has scales of its own
+@pytest.mark.parametrize("M,N,K,kind,tiled", [(5, 8193, 3072, "grid", True), (5, 8193, 2944, "grid", False), (12, 8193, 2944, "row", True),
+                                              (16, 8192, 8192, "grid", False), (6, 10880, 8320, "grid", True), (6, 10881, 8320, "grid", False),
+                                              (7, 12001, 8192, "grid", True), (8, 12001, 8320, "scalar", False), (9, 12001, 8320, "grid", True),
+                                              (9, 12001, 8320, "per_row", True), (16, 12001, 6272, "row", False), (9, 12001, 6144, "row", True)])
+def test_route_of_five_to_sixteen_rows_by_scales_and_limits(device, M, N, K, kind, tiled):
+    import ctypes as C
+
+    from cppmega_mlx_amd import _lib
+    gen = torch.Generator(device=device).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=gen, device=device).to(torch.bfloat16)
+    codes = torch.randn((N, K), generator=gen, device=device).to(torch.float8_e4m3fn)
+    shape = {"grid": ((N + 127) // 128, K // 128), "row": (N, K // 128), "per_row": (N, 1), "scalar": (1, 1)}[kind]
+    scale = torch.rand(shape, generator=gen, device=device) + 0.5
+    rows = scale.repeat_interleave(128, dim=0)[:N] if kind == "grid" else scale
+    want = x.double() @ (codes.double() * (rows.repeat_interleave(128, dim=1) if rows.shape[1] > 1 else rows).double()).T
+    a = _lib.VecmatArgs()
+    a.struct_size, a.x_dtype, a.out_dtype = C.sizeof(a), _lib.BF16, _lib.BF16
+    a.scale_w_kind = {"grid": _lib.WSCALE_GRID_128, "row": _lib.WSCALE_ROW_BLOCK, "per_row": _lib.WSCALE_PER_ROW, "scalar": _lib.WSCALE_SCALAR}[kind]
+    out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=device)
+    a.m, a.n, a.k = M, N, K
+    a.x, a.w, a.scale_w, a.out = x.data_ptr(), codes.data_ptr(), scale.data_ptr(), out.data_ptr()
+    need, lib = C.c_size_t(0), _lib.load()
+    assert lib.cppmega_mi355_fp8_vecmat_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK
+    assert (need.value > 0) == tiled                     # (each of these is split along K there)
+    ws = torch.empty(need.value + 16, dtype=torch.uint8, device=device)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), need.value
+    assert lib.cppmega_mi355_fp8_vecmat(C.byref(a), C.sizeof(a), _lib.current_stream(x.device)) == _lib.OK
+    # float32 sums (2e-6 of the largest), rounded once to 8 bits of mantissa
+    assert ((out.double() - want).abs() <= 2e-6 * want.abs().max() + want.abs() * 2.0 ** -8).all()
+    if kind in ("grid", "row"):                          # the wrapper brings the workspace itself
+        assert torch.equal(fused_fp8_gemm(codes.view(torch.uint8), scale, x), out)
+
+
+# an odd number of results, whose K splits begin at whole pieces of 16 bytes: the room of two splits is not twice theirs
+@pytest.mark.parametrize("M,N,K", [(17, 257, 3456), (33, 259, 4224)])
+def test_tiled_gemm_of_odd_sizes_with_room_for_fewer_splits(device, M, N, K):
+    import ctypes as C
+
+    from cppmega_mlx_amd import _lib
+    gen = torch.Generator(device=device).manual_seed(M)
+    x = torch.randn((M, K), generator=gen, device=device).to(torch.bfloat16)
+    codes = torch.randn((N, K), generator=gen, device=device).to(torch.float8_e4m3fn)
+    scale = torch.rand((N, K // 128), generator=gen, device=device) + 0.5
+    want = x.double() @ (codes.double() * scale.double().repeat_interleave(128, dim=1)).T
+    a = _lib.VecmatArgs()
+    a.struct_size, a.x_dtype, a.out_dtype, a.scale_w_kind = C.sizeof(a), _lib.BF16, _lib.F32, _lib.WSCALE_ROW_BLOCK
+    a.x, a.w, a.scale_w, a.m, a.n, a.k = x.data_ptr(), codes.data_ptr(), scale.data_ptr(), M, N, K
+    need, lib = C.c_size_t(0), _lib.load()
+    assert lib.cppmega_mi355_fp8_vecmat_workspace_bytes(C.byref(a), C.sizeof(a), C.byref(need)) == _lib.OK
+    one = (M * N + 3) // 4 * 16                          # bytes of a split
+    splits = need.value // one
+    assert splits > 3 and need.value == splits * one
+    ws = torch.empty(need.value, dtype=torch.uint8, device=device)
+    written = []
+    for given in (2 * one - 4, 2 * one, 3 * one, need.value):
+        ws.fill_(0xff)
+        out = torch.full((M, N), 7.0, device=device)
+        a.out, a.workspace, a.workspace_bytes = out.data_ptr(), ws.data_ptr(), given
+        assert lib.cppmega_mi355_fp8_vecmat(C.byref(a), C.sizeof(a), _lib.current_stream(x.device)) == _lib.OK
+        assert (out.double() - want).abs().max() <= 2e-6 * want.abs().max()
+        assert (ws[given:] == 0xff).all()
+        written.append(sum(bool((ws[i * one:i * one + 4 * M * N] != 0xff).any()) for i in range(splits)))
+    assert written == [0, 2, 3, splits]
