@@ -516,8 +516,9 @@ void launch_reduce(const VecmatParams& p, hipStream_t stream) {
 // 4096 19.3 / 16.1).  Measured at 5 .. 16 rows x 8400 .. 16400 x 512 .. 15900 with either layout of block scales: fewer than 12 rows gain
 // from about 3000 channels on (5 x 8400 x 1024 0.86 x, 6 x 10300 x 2048 0.95, 4096 1.2); where three K splits of the tiles are more
 // than the CUs and two leave some idle, up to 8192 channels (7 x 15814 x 14848 0.92), fewer with a scale per row, whose four
-// bytes take a line of the cache each (6 x 12200 x 8192 0.97, 4096 1.20; 11 x 11467 x 7168 0.92), and any number where neither counts (11 x 14832 x 15872 1.12).  Float32 results stay there as well: their
-// error against float64 is 0.93 .. 1.06 of that kernel's here (5.7e-8 .. 1.0e-7), which 16-bit results do not show.
+// bytes take a line of the cache each (6 x 12200 x 8192 0.97, 4096 1.20; 11 x 11467 x 7168 0.92), and any number where neither counts (11 x 14832 x 15872 1.12).  Float32 results stay there:
+// one chain of sums here is up to 1.06 times as far from float64 as that kernel's (0.93 .. 1.06 of 5.7e-8 .. 1.0e-7), which results of 16 bits
+// do not show.
 static bool few_rows_here(const cppmega_mi355_vecmat_args_t& a) {
   const int cus = device_cus();
   if (a.m < 5 || a.n <= 32 * cus || (a.m < 12 && a.k < 3072) || a.out_dtype == CPPMEGA_MI355_F32) return false;
@@ -534,8 +535,8 @@ bool fp8_gemm_shape(const cppmega_mi355_vecmat_args_t& a) {
 
 size_t fp8_gemm_workspace_bytes(const cppmega_mi355_vecmat_args_t& a) {
   int splits = gemm_plan(a.m, a.n, a.k, a.out_dtype == CPPMEGA_MI355_F32, SIZE_MAX).splits;
-  // a few small tiles ask for the room of three splits (3 MB at most) whatever the plan: workspaces that callers laid out
-  // for a range of such sizes stay as large as they were when each of them was split
+  // A few small tiles ask for the room of three splits (3 MB at most) where the plan has one or two: as much as when each of them was
+  // split, so that scratch laid out by asking for one such size goes on serving the others.
   if (splits < 3 && a.k >= 6 * 128 && (long long)((a.m + 31) / 32) * ((a.n + 127) / 128) <= device_cus() / 4) splits = 3;
   return split_bytes(splits, a.m, a.n);
 }

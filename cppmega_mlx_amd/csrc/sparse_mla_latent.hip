@@ -955,8 +955,8 @@ __global__ __launch_bounds__(64 * WAVES) void sparse_mla_latent_combine_kernel(c
     }
   };
 #define CM_MERGE(n) case n: merge(std::integral_constant<int, n>{}); break;
-  switch (p.num_splits) {                                     // (uniform, at most 16)
-    CM_MERGE(1) CM_MERGE(2) CM_MERGE(3) CM_MERGE(4) CM_MERGE(5) CM_MERGE(6) CM_MERGE(7) CM_MERGE(8)
+  switch (p.num_splits) {                                     // (uniform, 2 .. 16)
+    CM_MERGE(2) CM_MERGE(3) CM_MERGE(4) CM_MERGE(5) CM_MERGE(6) CM_MERGE(7) CM_MERGE(8)
     CM_MERGE(9) CM_MERGE(10) CM_MERGE(11) CM_MERGE(12) CM_MERGE(13) CM_MERGE(14) CM_MERGE(15)
     default: merge(std::integral_constant<int, 16>{});
   }
@@ -1047,9 +1047,10 @@ bool sparse_mla_latent_only(const MlaParams& p) { return latent_rows(p) && p.hea
 double mla_key_splits(MlaParams& p, long long units, int max_keys, double tile_us, int heads, bool narrow) {
   // float32 sums: fitted to 216 shapes of 16 and 128 heads, 1 .. 300 queries, 64 .. 2048 keys (1.2x in the mean against
   // doubling the splits until 256 workgroups are there, 3x where that ended just above 256 or in splits of four tiles).
-  // bfloat16 sums: to 24 shapes of 64 and 128 heads, 1 .. 64 queries, 256 .. 2048 keys (the merging kernel takes the
-  // splits four at a time); the choice is within 1 us of the best.  More splits than doubling makes would have to keep float32 sums, and gain nothing then: 128 heads x 1 x 1024
-  // keys 16.8 us in 8 splits, 20.3 in 16; 64 x 4 x 512 16.4 in 4, 18.5 in 8.
+  // bfloat16 sums: to 24 shapes of 64 and 128 heads, 1 .. 64 queries, 256 .. 2048 keys, when the merging kernel took the splits four at
+  // a time (a quarter of them costs group_us). It has all of them on their way at once now: at 56 such shapes the choice is within 0.7 us
+  // of the best number, but for 64 heads x 64 queries x 256 keys (1 split 17.8 us, 2 16.3).  More splits than doubling makes would have to keep
+  // float32 sums, and gain nothing then: 128 heads x 1 x 1024 keys 16.8 us in 8 splits, 20.3 in 16; 64 x 4 x 512 16.4 in 4, 18.5 in 8.
   constexpr double kUnitUs = 7.0;
   const double merge_us = narrow ? 0.7 : 5.0, group_us = narrow ? 0.3 : 0.0, bytes_per_us = narrow ? 2.9e6 : 5e6;
   const int tiles = (p.topk + kTK - 1) / kTK;

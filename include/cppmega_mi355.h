@@ -420,8 +420,9 @@ typedef struct cppmega_mi355_vecmat_args {
   int32_t out_dtype;
   int32_t reserved;
   void* out;
-  void* workspace;            /* split-K partials (M >= 17, or N beyond 32 a CU); with less
-                                 than *_workspace_bytes, or NULL, K is split less */
+  void* workspace;            /* split-K partials. M >= 17: with less than *_workspace_bytes,
+                                 or NULL, K is split less. 5 <= M <= 16 (16-bit results over
+                                 many weight rows): another kernel, which needs none        */
   size_t workspace_bytes;
 } cppmega_mi355_vecmat_args_t;
 
