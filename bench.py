@@ -659,7 +659,7 @@ PROFILE_WORKLOADS = [
     ("fp8_vecmat_m16", "trace_main", ("fetch_main", "write_main"), None, ("skinny_rows_kernel<1",),
      "W e4m3[7168,16384] + fp32 scale/128, x bf16[16,16384] (one kernel, no K split, no workspace)"),
     ("fp8_vecmat_m32", "trace_main", ("fetch_main", "write_main"), None, ("Tile<2, 2, 1, 4, 2, 3", "fp8_gemm_reduce"),
-     "W e4m3[7168,16384] + fp32 scale/128, x bf16[32,16384] (32 x 128 tiles, split-K, and the reduce kernel)"),
+     "W e4m3[7168,16384] + fp32 scale per row and 128 channels, x bf16[32,16384] (32 x 128 tiles, split-K, and the reduce kernel)"),
     ("topk_selector", "trace_main", ("fetch_main", "write_main"), None, ("topk_tile_kernel<float, 16, 512, 0, false",),
      "scores fp32[4096 rows,8192] -> int32[4096,2048], indices in ascending order (the dispatches of 4096 workgroups only: "
      "the same kernel also selects for the indexer and for the prefill rows of the same run)", 4096 * 512),
@@ -680,9 +680,9 @@ PROFILE_WORKLOADS = [
      "sparse_mla_fwd q [1,8192,128,576], kv [1,8192,1,576], causal top-2048 indices -> [1,8192,128,512]: "
      "rows16<true, 2, false> unquantised float16 rows, latent<1, true, true> e4m3 rows with per-token fp32 scales, "
      "rows16<false, 2, true> (behind the conversion of the cache) e4m3 rows with E8M0 bytes per 32 channels"),
-    ("sparse_mla_backward", "trace_main", ("fetch_main", "write_main"), None, ("bwd_lists_kernel", "bwd_steps_kernel", "bwd_scores_", "bwd_dq_kernel", "bwd_dkv_kernel", "bwd_sum_kernel"),
+    ("sparse_mla_backward", "trace_main", ("fetch_main", "write_main"), None, ("bwd_lists_kernel", "bwd_scores_", "bwd_dkv_kernel", "bwd_sum_kernel"),
      "sparse_mla_bwd q bf16[1,1024,16,576], kv bf16[1,4096,1,576], d_out bf16[1,1024,16,512], topk 256 -> dq bf16, dkv f32 "
-     "(keys by band, steps, scores, dq, dkv added in LDS, the sum of its shares)"),
+     "(keys by band, scores and dq behind the bands' steps, dkv added in LDS, the sum of its shares)"),
     ("dsa_indexer_loss", "trace_main", ("fetch_main", "write_main"), None, ("dsa_loss_", "dsa_indexer_loss"),
      "dsa_indexer_loss query / key bf16[4096,1,8,64], index_scores f32[1,4096,4096]: one dense and one sparse "
      "(topk_indices i32[1,4096,1024]) dispatch per step"),

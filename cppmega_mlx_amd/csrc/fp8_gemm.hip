@@ -5,12 +5,16 @@
 // The kernels of fp8_vecmat.hip read the whole weight once per 4 to 16 activation rows; from 17 rows on a
 // tile of both operands is worth staging in LDS.  The load unit writes the tiles there itself (global_load_lds, pieces of
 // 128 bytes of a row: such loads reach 50 B/clk a CU, pieces of 64 bytes 28, of 16 bytes 10), as many stages ahead as the
-// LDS holds.  Measured (microseconds a call; through registers, two stages ahead -> here), M x N x K:
-// 2048 x 8192 x 1536: 65 -> 59, 2048 x 7168 x 16384: 483 -> 441 = 1090 TFLOP/s, 1040 x 2621 x 5248: 58 -> 43,
-// 879 x 1007 x 6528: 48 -> 24, 231 x 4895 x 10240: 54 -> 38, 32 x 7168 x 16384: 29.0 -> 25.8, 55 x 2804 x 640: 7.6 -> 5.7.
-// What bounds it: a large product, the LDS (of 2048 clocks of products a 128 x 256 x 128 step, operand reads and arriving
-// rows take as many at 128 B/clk) and the vector instructions between the products; a small one, launch, first loads and
-// stores (5 us); a small batch, the weights' stream.
+// LDS holds.  Measured (microseconds a call in a row of calls over three weights in turn, bf16 results; through registers, two stages
+// ahead -> here), M x N x K, scales per 128 x 128 / per row and 128 channels:
+//   2048 x 8192 x 1536  64 -> 59 / 65 -> 60            2048 x 7168 x 16384  466 -> 444 = 1080 TFLOP/s / 535 -> 474
+//   1040 x 2621 x 5248  54 -> 41 / 58 -> 43            879 x 1007 x 6528    45 -> 23 / 48 -> 25
+//   231 x 4895 x 10240  52 -> 36 / 56 -> 40            32 x 7168 x 16384    29.1 -> 25.6 / 35.2 -> 33.0
+//   55 x 2804 x 640     7.9 -> 6.1 / 7.9 -> 6.3
+// (Under the profiler, whose calls do not overlap, 32 x 7168 x 16384 with a scale per row is 33 us and 4.6 for the sum of the splits, as before.)
+// What bounds it: a large product, no unit alone: of 5070 clocks a 128 x 256 x 128 stage with its share of a tile's ends (2048 x 8192 x 1536) 2048
+// are products on each SIMD, 1630 other vector instructions, 1770 the LDS (operand reads and, at 128 B/clk, arriving rows), and two
+// wavefronts cover each other's phases in part; a small one, launch, first loads and stores (5 us); a small batch, the weights' stream.
 
 #include <stdint.h>
 
