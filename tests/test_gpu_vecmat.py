@@ -433,3 +433,22 @@ def test_tiled_gemm_of_odd_sizes_with_room_for_fewer_splits(device, M, N, K):
         assert (ws[given:] == 0xff).all()
         written.append(sum(bool((ws[i * one:i * one + 4 * M * N] != 0xff).any()) for i in range(splits)))
     assert written == [0, 2, 3, splits]
+
+
+# float32 results: one to four blocks on 32-row tiles of one group (edges of the tile, a second round of tiles) and on larger ones; sections
+# of blocks: none at five stages, two at six, the last ones longer, with an odd block in one of two groups; tile after tile; seven splits
+@pytest.mark.parametrize("M,N,K", [(17, 1, 128), (32, 128, 256), (33, 129, 384), (70, 300, 512), (130, 7000, 512), (1000, 2000, 512),
+                                   (100, 700, 1280), (100, 700, 1408), (100, 700, 1536), (90, 9000, 1152), (2100, 2000, 768), (700, 7411, 1408),
+                                   (1434, 719, 16256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_float32_results_of_the_tiled_gemm_at_the_edges_of_its_sums(device, M, N, K, dtype):
+    gen = torch.Generator(device=device).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=gen, device=device).to(dtype)
+    codes = torch.randn((N, K), generator=gen, device=device).mul(2).to(torch.float8_e4m3fn)
+    scale = torch.rand((N, K // 128), generator=gen, device=device) + 0.5
+    want = x.double() @ (codes.double() * scale.double().repeat_interleave(128, dim=1)).T
+    out = torch.full((M * N + 8,), 7.0, dtype=torch.float32, device=device)
+    vm.fp8_scaled_vecmat_path_c(x, codes.view(torch.uint8), scale_x=None, scale_w=scale, out=out[4:-4].view(M, N))
+    assert (out[:4] == 7.0).all() and (out[-4:] == 7.0).all()
+    # (as for the other tiles)
+    assert (out[4:-4].view(M, N).double() - want).abs().max() <= 2e-6 * want.abs().max()
